@@ -3,7 +3,8 @@
     python fast-transformers_amd/build.py [--force] [--verbose]
 
 Output: fast_transformers_amd/libftc_causal.so next to the Python package, where
-``fast_transformers_amd._native`` loads it.  hipcc cross-compiles, so no GPU is needed.
+``fast_transformers_amd._native`` loads it, and _ftc_host.so beside it, the Python binding over
+the same C ABI (g++ against torch's headers).  hipcc cross-compiles, so no GPU is needed.
 """
 import argparse
 import glob
@@ -16,6 +17,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT = os.path.join(HERE, "fast_transformers_amd", "libftc_causal.so")
+HOST_SRC = os.path.join(HERE, "host", "ftc_host.cpp")
+HOST_OUT = os.path.join(HERE, "fast_transformers_amd", "_ftc_host.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 # -packed-fp32-ops is switched off on purpose: the compiler must not form
@@ -43,6 +46,22 @@ def headers():
     return sorted(glob.glob(os.path.join(CSRC, "*.h")) + glob.glob(os.path.join(INCLUDE, "*.h")))
 
 
+def host_command():
+    """g++ line of the Python binding: host code only, linked against the library beside it."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+            "-isystem", os.path.join(root, "include"),
+            "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+            "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
+            "-I", INCLUDE, HOST_SRC, "-o", HOST_OUT,
+            "-L" + os.path.dirname(OUT), "-l:" + os.path.basename(OUT),
+            "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+            "-Wl,-rpath,$ORIGIN"]
+
+
 def build(force=False, verbose=False, extra_flags=()):
     hipcc = find_hipcc()
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -65,6 +84,12 @@ def build(force=False, verbose=False, extra_flags=()):
             raise RuntimeError("hipcc failed on %s" % src)
     if procs or force or not os.path.exists(OUT):
         cmd = [hipcc, "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-rdc", "-o", OUT] + objs
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.check_call(cmd)
+    if force or not os.path.exists(HOST_OUT) or os.path.getmtime(HOST_OUT) < max(
+            os.path.getmtime(f) for f in [HOST_SRC] + glob.glob(os.path.join(INCLUDE, "*.h"))):
+        cmd = host_command()
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)

@@ -48,7 +48,26 @@ class Tensor4(ctypes.Structure):
     ]
 
 
+HOST_PATH = os.path.join(_HERE, "_ftc_host.so")
 _lib = None
+_host = None
+
+
+def host():
+    """The compiled binding over the same C ABI that the package's own entry points use
+    (``host/ftc_host.cpp``; the ctypes one below costs a call about 20 us more).  Raises if it has
+    not been built."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(
+                "fast_transformers_amd: %s is missing; build it with "
+                "`python fast-transformers_amd/build.py` (there is no CPU or PyTorch fallback)"
+                % HOST_PATH)
+        load()
+        from . import _ftc_host
+        _host = _ftc_host
+    return _host
 
 
 def load():

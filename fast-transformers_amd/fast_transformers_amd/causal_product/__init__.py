@@ -15,38 +15,9 @@
   product is float32 in both cases (``__init__.py:41`` allocates with the default
   dtype) and the gradients have the dtype of their inputs (``__init__.py:59-61``).
 """
-import os
-import time
-
 import torch
 
 from .. import _native
-
-
-def _prepare(t, name):
-    """The kernels take any N/H/L strides but need unit stride in the last dimension."""
-    if t.dim() != 4:
-        raise RuntimeError("causal_dot_product: %s must be 4-dimensional (N, H, L, X), got %d-d"
-                           % (name, t.dim()))
-    if t.device.type != "cuda":
-        raise RuntimeError("causal_dot_product: %s is on %s, expected a GPU tensor"
-                           % (name, t.device))
-    if t.shape[3] > 1 and t.stride(3) != 1:
-        return t.contiguous()
-    # rows that overlap (an expanded L dimension) would take the slow general path; zero
-    # strides over N or H (one sequence shared by chains) are read as they are
-    if t.shape[2] > 1 and t.stride(2) < t.shape[3]:
-        return t.contiguous()
-    return t
-
-
-def _check_out(t, name):
-    if t.dim() != 4 or t.device.type != "cuda":
-        raise RuntimeError("causal_dot_product: %s must be a 4-dimensional GPU tensor" % name)
-    if t.shape[3] > 1 and t.stride(3) != 1:
-        raise RuntimeError("causal_dot_product: output %s must be contiguous in its last "
-                           "dimension" % name)
-    return t
 
 
 # One scratch buffer per (device, stream), grown on demand.  The library wants the control
@@ -57,41 +28,24 @@ def _check_out(t, name):
 # was cut short.  Reading it means waiting for the GPU, so the wrapper does that only where it
 # is asked for (``check_workspaces()``; after every call when FTC_CHECK=1 is set in the
 # environment) or cheap (before a cached workspace is replaced by a larger one).  Between
-# those it watches without waiting: at most every ``_PROBE_INTERVAL_S`` seconds a call leaves
+# those it watches without waiting: at most every ten milliseconds a call leaves
 # an asynchronous copy of the error word to pinned host memory behind it on its stream, and a
 # later call that finds the copy finished (an event query) reads the word and raises.
 _workspaces = {}
-_ws_bytes = {}            # (query, N, H, L, E, M, dtype code) -> bytes: sizes repeat call after call
-_probes = {}              # workspace key -> [pinned word, event or None, time of the last probe]
-_PROBE_INTERVAL_S = 0.01
+_probes = {}              # workspace key -> [pinned word, event or None]
 
 
-class _NoGuard:
-    def __enter__(self):
-        return self
-
-    def __exit__(self, *exc):
-        return False
+_host_module = None
 
 
-_NO_GUARD = _NoGuard()
-
-
-def _device_guard(device):
-    """Make `device` current for the call -- at no cost when it already is."""
-    index = device.index
-    if index is None or index == torch.cuda.current_device():
-        return _NO_GUARD
-    return torch.cuda.device(index)
-
-
-def _workspace_bytes(query, N, H, L, E, M, code):
-    key = (query, N, H, L, E, M, code)
-    nbytes = _ws_bytes.get(key)
-    if nbytes is None:
-        nbytes = _native.check(getattr(_native.load(), query)(N, H, L, E, M, code), query)
-        _ws_bytes[key] = nbytes
-    return nbytes
+def _host():
+    """The compiled binding, with this module's workspaces behind it."""
+    global _host_module
+    if _host_module is None:
+        host = _native.host()
+        host.setup(_workspaces, _make_workspace, _watch, _probe, _check_if_possible)
+        _host_module = host
+    return _host_module
 
 
 def reload_tuning():
@@ -99,10 +53,11 @@ def reload_tuning():
     use) and forget the workspace sizes asked for under the old values.  A debugging aid: call
     it with no work in flight."""
     _native.check(_native.load().ftc_tuning_reload(), "ftc_tuning_reload")
-    _ws_bytes.clear()
+    _host().forget_sizes()
 
 
 def _workspace(nbytes, device, stream=None):
+    """The workspace of a device and stream (the current one), at least ``nbytes`` large."""
     if nbytes <= 0:
         return None, 0
     if stream is None:
@@ -110,13 +65,17 @@ def _workspace(nbytes, device, stream=None):
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        if ws is not None:
-            check_workspaces()  # the old buffer's last word on the calls made with it
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-        _probes.pop(key, None)
-    _watch(key, ws)
+        ws = _make_workspace(nbytes, key)
     return ws, ws.numel()
+
+
+def _make_workspace(nbytes, key):
+    if key in _workspaces:
+        check_workspaces()  # the old buffer's last word on the calls made with it
+    ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=torch.device("cuda", key[0]))
+    _workspaces[key] = ws
+    _probes.pop(key, None)
+    return ws
 
 
 def _watch(key, ws):
@@ -130,31 +89,25 @@ def _watch(key, ws):
             check_workspaces()   # synchronises, resets the control block and raises
 
 
-def _after_call(ws=None, stream=None):
-    if os.environ.get("FTC_CHECK", "0") not in ("", "0"):
-        # the check synchronises, which a capturing stream does not allow: a captured call is
-        # checked by the first eager call after the replays, or by check_workspaces()
-        if not torch.cuda.is_current_stream_capturing():
-            check_workspaces()
-        return
-    if ws is None:
-        return
-    # leave a probe behind this call when the last one is old enough and has been read
-    now = time.monotonic()
-    if stream is None:
-        stream = torch.cuda.current_stream(ws.device).cuda_stream
-    key = (ws.device.index, stream)
+def _probe(key, ws):
+    """Leave a probe behind the call just made when the last one has been read."""
     probe = _probes.get(key)
-    if probe is not None and (probe[1] is not None or now - probe[2] < _PROBE_INTERVAL_S):
-        return
-    if torch.cuda.is_current_stream_capturing():
+    if (probe is not None and probe[1] is not None) or torch.cuda.is_current_stream_capturing():
         return
     if probe is None:
-        probe = _probes[key] = [torch.zeros(1, dtype=torch.int32).pin_memory(), None, 0.0]
+        probe = _probes[key] = [torch.zeros(1, dtype=torch.int32).pin_memory(), None]
     probe[0].copy_(ws[8:12].view(torch.int32), non_blocking=True)
     ev = torch.cuda.Event()
     ev.record()
-    probe[1], probe[2] = ev, now
+    probe[1] = ev
+
+
+def _check_if_possible():
+    """After every call under FTC_CHECK.  The check synchronises, which a capturing stream does
+    not allow: a captured call is checked by the first eager call after the replays, or by
+    check_workspaces()."""
+    if not torch.cuda.is_current_stream_capturing():
+        check_workspaces()
 
 
 def workspace_error_words():
@@ -191,22 +144,7 @@ def check_workspaces():
 def causal_dot_product_hip(queries, keys, values, product):
     """In-place forward; replaces the reference's native ``causal_dot_product``
     (``causal_product_cuda.cu:1273-1285``).  Enqueued on the current stream."""
-    lib = _native.load()
-    q, k, v = (_prepare(t, n) for t, n in
-               ((queries, "queries"), (keys, "keys"), (values, "values")))
-    out = _check_out(product, "product")
-    N, H, L, E = q.shape
-    M = v.shape[3]
-    with _device_guard(q.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        nbytes = _workspace_bytes("ftc_causal_dot_product_workspace_bytes", N, H, L, E, M,
-                                  _native.dtype_code(q.dtype))
-        ws, nbytes = _workspace(nbytes, q.device, stream)
-        dq, dk, dv, do = (_native.describe(t) for t in (q, k, v, out))
-        rc = lib.ftc_causal_dot_product(dq, dk, dv, do, ws.data_ptr() if ws is not None else None,
-                                        nbytes, stream)
-        _native.check(rc, "ftc_causal_dot_product")
-        _after_call(ws, stream)
+    _host().forward(queries, keys, values, product)
 
 
 def causal_dot_product_with_state(queries, keys, values, initial_state=None,
@@ -220,33 +158,7 @@ def causal_dot_product_with_state(queries, keys, values, initial_state=None,
     (``recurrent/attention/self_attention/linear_attention.py:63-90``), so a prompt processed
     here can be continued there, or by another call on the next piece.  Forward only (no
     autograd); enqueued on the current stream."""
-    lib = _native.load()
-    q, k, v = (_prepare(t, n) for t, n in
-               ((queries, "queries"), (keys, "keys"), (values, "values")))
-    N, H, L, E = q.shape
-    M = v.shape[3]
-    s0 = None
-    if initial_state is not None:
-        s0 = _prepare(initial_state, "initial_state")
-        if s0.dtype != torch.float32 or tuple(s0.shape) != (N, H, E, M):
-            raise RuntimeError("causal_dot_product_with_state: initial_state must be a float32 "
-                               "tensor of shape (N, H, E, M)")
-    out = torch.empty((N, H, L, M), dtype=torch.float32, device=q.device)
-    s1 = torch.empty((N, H, E, M), dtype=torch.float32, device=q.device) if return_state else None
-    with _device_guard(q.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        nbytes = _workspace_bytes("ftc_causal_dot_product_workspace_bytes", N, H, L, E, M,
-                                  _native.dtype_code(q.dtype))
-        ws, nbytes = _workspace(nbytes, q.device, stream)
-        dq, dk, dv, do = (_native.describe(t) for t in (q, k, v, out))
-        d0 = _native.describe(s0) if s0 is not None else None
-        d1 = _native.describe(s1) if s1 is not None else None
-        rc = lib.ftc_causal_dot_product_state(dq, dk, dv, d0, do, d1,
-                                              ws.data_ptr() if ws is not None else None, nbytes,
-                                              stream)
-        _native.check(rc, "ftc_causal_dot_product_state")
-        _after_call(ws, stream)
-    return out, s1
+    return _host().product_with_state(queries, keys, values, initial_state, return_state)
 
 
 def causal_dot_backward_hip(queries, keys, values, grad_out, grad_queries, grad_keys,
@@ -254,27 +166,7 @@ def causal_dot_backward_hip(queries, keys, values, grad_out, grad_queries, grad_
     """In-place backward; replaces the reference's native ``causal_dot_backward``
     (``causal_product_cuda.cu:1438-1467``).  A gradient passed as ``None`` is skipped.
     Enqueued on the current stream."""
-    lib = _native.load()
-    q, k, v, g = (_prepare(t, n) for t, n in
-                  ((queries, "queries"), (keys, "keys"), (values, "values"),
-                   (grad_out, "grad_out")))
-    if g.dtype != torch.float32:
-        g = g.float()
-    gq, gk, gv = (_check_out(t, n) if t is not None else None for t, n in
-                  ((grad_queries, "grad_queries"), (grad_keys, "grad_keys"),
-                   (grad_values, "grad_values")))
-    N, H, L, E = q.shape
-    M = v.shape[3]
-    with _device_guard(q.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        nbytes = _workspace_bytes("ftc_causal_dot_backward_workspace_bytes", N, H, L, E, M,
-                                  _native.dtype_code(q.dtype))
-        ws, nbytes = _workspace(nbytes, q.device, stream)
-        descs = [_native.describe(t) if t is not None else None for t in (q, k, v, g, gq, gk, gv)]
-        rc = lib.ftc_causal_dot_backward(*descs, ws.data_ptr() if ws is not None else None,
-                                         nbytes, stream)
-        _native.check(rc, "ftc_causal_dot_backward")
-        _after_call(ws, stream)
+    _host().backward(queries, keys, values, grad_out, grad_queries, grad_keys, grad_values)
 
 
 FTC_ERR_UNSUPPORTED = -2
@@ -293,14 +185,6 @@ def fused_attention_covers(queries, values, keys=None):
     return queries.shape[3] in (32, 64) and values.shape[3] in (32, 64)
 
 
-def _check_key_lengths(key_lengths, q):
-    if key_lengths is not None:
-        if key_lengths.dtype != torch.int64 or key_lengths.device != q.device or \
-                key_lengths.shape != (q.shape[0],) or not key_lengths.is_contiguous():
-            raise RuntimeError("causal_linear_attention: key_lengths must be a contiguous int64 "
-                               "tensor of N values on the device of the queries")
-
-
 def causal_linear_attention_hip(queries, keys, values, key_lengths, eps, out, denominators=None):
     """In-place fused forward of causally masked linear attention with the feature map
     ``elu(x) + 1``: replaces the body of the reference module's forward
@@ -309,25 +193,7 @@ def causal_linear_attention_hip(queries, keys, values, key_lengths, eps, out, de
     tensor of N lengths on the same device, or None; ``denominators``: None, or a float32
     (N, H, L) tensor that receives the normaliser's denominators (the backward needs them).
     Raises ``RuntimeError`` for sizes without a fused kernel (see ``fused_attention_covers``)."""
-    lib = _native.load()
-    q, k, v = (_prepare(t, n) for t, n in
-               ((queries, "queries"), (keys, "keys"), (values, "values")))
-    o = _check_out(out, "out")
-    N, H, L, E = q.shape
-    M = v.shape[3]
-    _check_key_lengths(key_lengths, q)
-    with _device_guard(q.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        nbytes = _workspace_bytes("ftc_causal_linear_attention_workspace_bytes", N, H, L, E, M,
-                                  _native.dtype_code(q.dtype))
-        ws, nbytes = _workspace(nbytes, q.device, stream)
-        dq, dk, dv, do = (_native.describe(t) for t in (q, k, v, o))
-        dden = _native.describe(denominators.unsqueeze(3)) if denominators is not None else None
-        rc = lib.ftc_causal_linear_attention_forward(
-            dq, dk, dv, key_lengths.data_ptr() if key_lengths is not None else None, float(eps),
-            do, dden, ws.data_ptr() if ws is not None else None, nbytes, stream)
-        _native.check(rc, "ftc_causal_linear_attention_forward")
-        _after_call(ws, stream)
+    _host().attention(queries, keys, values, key_lengths, eps, out, denominators)
 
 
 def causal_linear_attention_backward_hip(queries, keys, values, key_lengths, out, denominators,
@@ -336,29 +202,8 @@ def causal_linear_attention_backward_hip(queries, keys, values, key_lengths, out
     queries, keys and values (any of the three may be None) from ``grad_out``, the forward's
     ``out`` and its ``denominators``.  Replaces what autograd does in the reference for the body
     of ``CausalLinearAttention.forward`` (``attention/causal_linear_attention.py:71-104``)."""
-    lib = _native.load()
-    q, k, v, o, g = (_prepare(t, n) for t, n in
-                     ((queries, "queries"), (keys, "keys"), (values, "values"), (out, "out"),
-                      (grad_out, "grad_out")))
-    gq, gk, gv = (_check_out(t, n) if t is not None else None for t, n in
-                  ((grad_queries, "grad_queries"), (grad_keys, "grad_keys"),
-                   (grad_values, "grad_values")))
-    N, H, L, E = q.shape
-    M = v.shape[3]
-    _check_key_lengths(key_lengths, q)
-    with _device_guard(q.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        nbytes = _workspace_bytes("ftc_causal_linear_attention_backward_workspace_bytes", N, H, L,
-                                  E, M, _native.dtype_code(q.dtype))
-        ws, nbytes = _workspace(nbytes, q.device, stream)
-        descs = [_native.describe(t) if t is not None else None
-                 for t in (q, k, v, o, denominators.unsqueeze(3), g, gq, gk, gv)]
-        rc = lib.ftc_causal_linear_attention_backward(
-            descs[0], descs[1], descs[2],
-            key_lengths.data_ptr() if key_lengths is not None else None, *descs[3:],
-            ws.data_ptr() if ws is not None else None, nbytes, stream)
-        _native.check(rc, "ftc_causal_linear_attention_backward")
-        _after_call(ws, stream)
+    _host().attention_backward(queries, keys, values, key_lengths, out, denominators, grad_out,
+                               grad_queries, grad_keys, grad_values)
 
 
 class CausalLinearAttentionFunction(torch.autograd.Function):
@@ -459,9 +304,9 @@ class CausalDotProduct(torch.autograd.Function):
         product = torch.empty((N, H, L, M), device=device, dtype=torch.float32)
 
         CausalDotProduct.dot[device.type](
-            Q.data,
-            K.data,
-            V.data,
+            Q,
+            K,
+            V,
             product
         )
         return product
@@ -475,9 +320,9 @@ class CausalDotProduct(torch.autograd.Function):
         grad_V = torch.empty_like(V, memory_format=torch.contiguous_format)
 
         CausalDotProduct.dot_backward[Q.device.type](
-            Q.data,
-            K.data,
-            V.data,
+            Q,
+            K,
+            V,
             grad_out,
             grad_Q,
             grad_K,
