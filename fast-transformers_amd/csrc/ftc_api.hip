@@ -45,7 +45,7 @@ static void read_tuning(Tuning &t) {
     t.split = num("FTC_SPLIT"), t.pad = num("FTC_PAD"), t.wg = num("FTC_WG"), t.tp = num("FTC_TP");
     t.tp_segs = num("FTC_TP_SEGS"), t.tpx = num("FTC_TPX"), t.tpx_segs = num("FTC_TPX_SEGS");
     t.seg_chunks = num("FTC_SEG_CHUNKS"), t.group = num("FTC_GROUP"), t.dma = num("FTC_DMA");
-    t.tph = num("FTC_TPH");
+    t.tph = num("FTC_TPH"), t.short_most = num("FTC_SHORT");
     const char *ratio = getenv("FTC_TP_RATIO");
     t.tp_ratio = ratio && *ratio ? atof(ratio) : -1.0;
     t.stamp_ptr = getenv("FTC_STAMP_PTR");
@@ -618,6 +618,7 @@ bool pad_eligible(const ScanDesc &sc, int64_t rows) {
 // types go out in one launch.  Everything else takes the generic path.
 int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, void *workspace,
               size_t workspace_bytes, hipStream_t stream, bool may_pad = true) {
+    if (short_scans_take(scans, n, N, H, L)) return short_scans(scans, n, N, H, L, stream);
     // which scans the matrix-core kernels take as they are
     bool native[kMfmaMaxScans], padded[kMfmaMaxScans], taken[kMfmaMaxScans] = {};
     bool any_padded = false;

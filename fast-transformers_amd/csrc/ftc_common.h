@@ -48,7 +48,7 @@ void note_kernel(const char *name);
 // use), read once when the library is first used and again only by ftc_tuning_reload():
 // -1 stands for "not set".
 struct Tuning {
-    int split, pad, wg, tp, tp_segs, tpx, tpx_segs, seg_chunks, group, dma, tph;
+    int split, pad, wg, tp, tp_segs, tpx, tpx_segs, seg_chunks, group, dma, tph, short_most;
     double tp_ratio;  // < 0: not set
     const char *stamp_ptr;
     uint64_t generation;  // counts the reloads: memoised plans are dropped when it changes
@@ -160,6 +160,11 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
               void *workspace, size_t workspace_bytes, hipStream_t stream,
               const FusedAttention *fused = nullptr, bool may_chain_parallel = true,
               bool forced = false);
+
+// Chains of a few positions (ftc_short.hip): scans of any widths and element types in one launch,
+// on the vector unit, without a workspace.
+bool short_scans_take(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L);
+int short_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, hipStream_t stream);
 
 // Backward of the fused attention (ftc_attention.hip): the kernels around the three scans.
 // prep: Qf = phi(q), Kf = phi(k) [l < key_len] (dense rows of E floats), gz = g / den (dense rows
