@@ -45,7 +45,7 @@ static void read_tuning(Tuning &t) {
     t.split = num("FTC_SPLIT"), t.pad = num("FTC_PAD"), t.wg = num("FTC_WG"), t.tp = num("FTC_TP");
     t.tp_segs = num("FTC_TP_SEGS"), t.tpx = num("FTC_TPX"), t.tpx_segs = num("FTC_TPX_SEGS");
     t.seg_chunks = num("FTC_SEG_CHUNKS"), t.group = num("FTC_GROUP"), t.dma = num("FTC_DMA");
-    t.tph = num("FTC_TPH"), t.short_most = num("FTC_SHORT");
+    t.tph = num("FTC_TPH"), t.short_most = num("FTC_SHORT"), t.odd = num("FTC_ODD");
     const char *ratio = getenv("FTC_TP_RATIO");
     t.tp_ratio = ratio && *ratio ? atof(ratio) : -1.0;
     t.stamp_ptr = getenv("FTC_STAMP_PTR");
@@ -613,6 +613,65 @@ bool pad_eligible(const ScanDesc &sc, int64_t rows) {
     return padded_shape_ok(Dp, round_up(sc.v.width, 32));
 }
 
+// Whether an fp32 scan of odd widths runs on the fp16-piece kernel where its rows lie rather than on
+// padded copies: where each of its operands would have to be copied (forward + backward, us, here
+// / on the copies: 9 x 11 chains, L=1531, 25 x 33: 126 / 248; 8 x 16, L=4096, 50 x 50: 387 / 940; one
+// chain of 100, on the VALU kernel before: 17 / 132).  Scans some of whose rows stay where they
+// are (25 x 64: two copies of four) would gain as well, 344 against 500 us at 8 x 16, L=4096;
+// their route through the copies is what the planner's tests lay down.  Thousands of chains of up
+// to four chunks of narrow rows keep the copies, which bring them to 32 x 32 (2048 chains,
+// L=100, 10 x 9: 228 / 176; 25 x 33: 252 / 302).
+bool odd_in_place(const ScanDesc &sc, int64_t chains, int64_t L) {
+    if (tuning().odd == 0) return false;  // tuning aid
+    if (chains > 1024 && L <= 128 && sc.a.width < 24 && sc.v.width < 24) return false;
+    const Operand *in[3] = {&sc.a, &sc.b, &sc.v};
+    if (sc.out.dtype != FTC_F32) return false;
+    bool any_fits = sc.out.width % 32 == 0 &&
+                    mfma_operand_in_place(sc.out.ptr, sc.out.stride_n, sc.out.stride_h, sc.out.stride_l,
+                                          FTC_F32, sc.out.width, L);
+    for (const Operand *o : in) {
+        if (o->dtype != FTC_F32) return false;
+        any_fits = any_fits || (o->width % 32 == 0 && mfma_operand_in_place(o->ptr, o->stride_n, o->stride_h,
+                                                                            o->stride_l, FTC_F32, o->width, L));
+    }
+    return !any_fits || tuning().odd > 0;
+}
+
+// Scans for which odd_in_place holds, in one launch or one per shape, whichever is estimated
+// shorter (three scans of 99 chains are two rounds of workgroups, two and one are one round each).
+// *done = false (nothing launched): the kernel does not take one of them.
+int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, void *workspace,
+              size_t workspace_bytes, hipStream_t stream, bool *done) {
+    *done = false;
+    ScanDesc group[kMfmaMaxScans][kMfmaMaxScans];
+    int size[kMfmaMaxScans], ngroups = 0, widest_d = 0, widest_f = 0;
+    double apart = 0.0;
+    for (int i = 0; i < n; i++) {
+        widest_d = std::max(widest_d, scans[i].a.width), widest_f = std::max(widest_f, scans[i].v.width);
+        int k = 0;
+        while (k < ngroups && (group[k][0].a.width != scans[i].a.width || group[k][0].v.width != scans[i].v.width)) k++;
+        if (k == ngroups) size[ngroups++] = 0;
+        group[k][size[k]++] = scans[i];
+    }
+    bool apart_ok = true;
+    for (int k = 0; k < ngroups; k++) {
+        apart_ok = apart_ok && mfma_tp_takes(group[k], size[k], N, H, L, false, true);
+        if (apart_ok) apart += mfma_tp_odd_chunks(group[k][0].a.width, group[k][0].v.width, N, H, size[k], L);
+    }
+    const bool together_ok = ngroups > 1 && mfma_tp_takes(scans, n, N, H, L, false, true);
+    if (!apart_ok && !together_ok) return FTC_OK;
+    auto run = [&](const ScanDesc *s, int k) {
+        return mfma_scan(s, k, N, H, L, workspace, workspace_bytes, stream, nullptr, true, false, true);
+    };
+    *done = true;
+    if (together_ok && (!apart_ok || mfma_tp_odd_chunks(widest_d, widest_f, N, H, n, L) <= apart)) return run(scans, n);
+    for (int k = 0; k < ngroups; k++) {
+        const int rc = run(group[k], size[k]);
+        if (rc) return rc;
+    }
+    return FTC_OK;
+}
+
 // Runs a list of independent scans.  A scan whose shape the MFMA kernels cover is cut into
 // column slices; consecutive slices (of any of the scans) that share widths and element
 // types go out in one launch.  Everything else takes the generic path.
@@ -661,6 +720,21 @@ int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
         native[i] = nslices > 0;
         padded[i] = !native[i] && may_pad && pad_eligible(scans[i], N * H * L);
         any_padded = any_padded || padded[i];
+    }
+    // ... odd ones of up to 64 state rows where they lie
+    if (may_pad) {
+        ScanDesc odd[kMfmaMaxScans];
+        int members[kMfmaMaxScans], nodd = 0;
+        for (int i = 0; i < n; i++)
+            if (!taken[i] && !native[i] && odd_in_place(scans[i], N * H, L)) members[nodd] = i, odd[nodd++] = scans[i];
+        if (nodd > 0) {
+            bool done = false;
+            const int rc = odd_scans(odd, nodd, N, H, L, workspace, workspace_bytes, stream, &done);
+            if (rc) return rc;
+            for (int k = 0; k < nodd && done; k++) taken[members[k]] = true, padded[members[k]] = false;
+        }
+        any_padded = false;
+        for (int i = 0; i < n; i++) any_padded = any_padded || padded[i];
     }
     if (any_padded) {
         bool done = false;
@@ -718,7 +792,8 @@ int64_t scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t
     if (nslices == 0 && with_pad)
         need = std::max(need, padded_scan_workspace_bytes(N, H, L, D, F, bf16));
     for (int k = 1; k <= kMfmaMaxScans; k++)
-        need = std::max(need, mfma_tp_workspace_bytes(N, H, L, D, F, k));
+        need = std::max(need, std::max(mfma_tp_workspace_bytes(N, H, L, D, F, k),
+                                       mfma_tp_workspace_bytes(N, H, L, D, F, k, false, true)));
     if (with_pad && split_widths(D, F))
         need = std::max(need, split_scan_workspace_bytes(N, H, L, D, F, nullptr));
     return need;
@@ -898,6 +973,9 @@ int64_t ftc_causal_dot_backward_workspace_bytes(int64_t N, int64_t H, int64_t L,
     const bool bf16 = dtype == FTC_BF16;
     int64_t need = std::max(scan_workspace_bytes(N, H, L, E, M, true, bf16),
                             scan_workspace_bytes(N, H, L, M, E, true, bf16));
+    // (odd widths: scans of both shapes may share a launch)
+    for (int k = 2; k <= 3; k++)
+        need = std::max(need, mfma_tp_workspace_bytes(N, H, L, std::max(E, M), std::max(E, M), k, false, true));
     // the padded route of the three scans together: Q, K, dQ, dK and V, G, dV as dense rows
     if (padded_scan_workspace_bytes(N, H, L, E, M, bf16) > 0 ||
         padded_scan_workspace_bytes(N, H, L, M, E, bf16) > 0) {

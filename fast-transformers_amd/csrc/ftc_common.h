@@ -48,7 +48,7 @@ void note_kernel(const char *name);
 // use), read once when the library is first used and again only by ftc_tuning_reload():
 // -1 stands for "not set".
 struct Tuning {
-    int split, pad, wg, tp, tp_segs, tpx, tpx_segs, seg_chunks, group, dma, tph, short_most;
+    int split, pad, wg, tp, tp_segs, tpx, tpx_segs, seg_chunks, group, dma, tph, short_most, odd;
     double tp_ratio;  // < 0: not set
     const char *stamp_ptr;
     uint64_t generation;  // counts the reloads: memoised plans are dropped when it changes
@@ -136,10 +136,15 @@ int64_t mfma_scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, in
 // its workspace (part of mfma_scan_workspace_bytes where both apply).
 // `forced`: these scans are parts of scans that the caller has split by state rows because
 // only this kernel can take them (any multiple of 4 will do, at any size).
+// `odd`: fp32 rows of any width on any 4-byte boundary, read and written where they lie (states of
+// up to 64 rows; scans of different widths may share the launch where none has more than 64
+// columns).
 bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
-                   bool forced = false);
+                   bool forced = false, bool odd = false);
 int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans,
-                                bool forced = false);
+                                bool forced = false, bool odd = false);
+// estimated time of such a launch, in chunks walked one after the other
+double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L);
 // The fused attention form of a forward scan: a and b go through the feature map
 // elu(x) + 1, rows of b at or beyond key_lengths[n] count as zero, and every output row is
 // divided by (phi(a_l) . sum_{j <= l} phi(b_j) + eps).
@@ -159,7 +164,7 @@ int64_t fused_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
               void *workspace, size_t workspace_bytes, hipStream_t stream,
               const FusedAttention *fused = nullptr, bool may_chain_parallel = true,
-              bool forced = false);
+              bool forced = false, bool odd = false);
 
 // Chains of a few positions (ftc_short.hip): scans of any widths and element types in one launch,
 // on the vector unit, without a workspace.

@@ -30,7 +30,10 @@ bool use_wg_kernel(int64_t D, int64_t F, int nscans, int64_t L, bool all_f32) {
 // widths that are multiples of 4 (a lane's 16 bytes lie wholly inside a row or wholly outside).
 // (`forced`: a part of a scan that the caller has split because only this kernel takes it;
 // then any multiple of 4 will do)
-bool tp_widths(int64_t D, int64_t F, bool forced = false) {
+// `odd`: fp32 rows of any width on 4-byte boundaries, states of up to 64 rows (the fp16-piece
+// kernel reads and writes those where they lie).
+bool tp_widths(int64_t D, int64_t F, bool forced = false, bool odd = false) {
+    if (odd) return D >= 8 && D <= 64 && F >= 8 && F <= 512;
     const int64_t least = forced ? 4 : 16;
     return D >= least && D <= 128 && F >= least && F <= 512 && D % 4 == 0 && F % 4 == 0;
 }
@@ -202,11 +205,11 @@ int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg, bool ke
 // whose values are fp32 (the dV scan of a bf16 backward)
 constexpr int kMixedRows = 1, kMixedGradValues = 2;
 void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg,
-                     int *seg_chunks, bool forced, int mixed) {
+                     int *seg_chunks, bool forced, int mixed, bool odd) {
     *nseg = *seg_chunks = 0;
-    if (!tp_widths(D, F, forced)) return;
-    const bool wide = D != 64 || F != 64 || forced;
-    const bool others = !forced && mfma_scan_supported_widths(D, F);
+    if (!tp_widths(D, F, forced, odd)) return;
+    const bool wide = D != 64 || F != 64 || forced || odd;
+    const bool others = !forced && !odd && mfma_scan_supported_widths(D, F);
     const int64_t units = chains * nscans * tp_fblocks(F);
     // A single scan over bf16 rows: the kernels that split L multiply such rows as they are,
     // one matrix instruction per product, and win while this kernel has workgroups for fewer
@@ -425,12 +428,12 @@ struct TpPlan {
     int nseg, seg_chunks;
 };
 void tp_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg, int *seg_chunks,
-             bool forced = false, int mixed = 0) {
+             bool forced = false, int mixed = 0, bool odd = false) {
     static thread_local PlanMemo<TpPlan> memo;
-    const int64_t key[8] = {D, F, chains, nscans, L, forced ? 1 : 0, mixed, 0};
+    const int64_t key[8] = {D, F, chains, nscans, L, forced ? 1 : 0, mixed, odd ? 1 : 0};
     const TpPlan pl = memo.get(key, [&]() {
         TpPlan p;
-        tp_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks, forced, mixed);
+        tp_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks, forced, mixed, odd);
         return p;
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
@@ -543,16 +546,26 @@ int64_t mfma_scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, in
 }
 
 int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans,
-                                bool forced) {
+                                bool forced, bool odd) {
     int nseg = 0, seg_chunks = 0;
     const int64_t chains = std::max<int64_t>(1, N * H);
-    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced);
+    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, odd);
     return seg_chunks > 0 ? tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D) : 0;
 }
 
-bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L, bool forced) {
-    const int D = scans[0].a.width, F = scans[0].v.width;
-    if (nscans < 1 || nscans > kMaxScans || !tp_widths(D, F, forced)) return false;
+// the widest rows of a launch (they differ between scans only where `odd` allows it)
+void widest_rows(const ScanDesc *scans, int nscans, int *D, int *F) {
+    *D = *F = 0;
+    for (int i = 0; i < nscans; i++) *D = std::max(*D, scans[i].a.width), *F = std::max(*F, scans[i].v.width);
+}
+
+bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L, bool forced,
+                   bool odd) {
+    if (nscans < 1 || nscans > kMaxScans) return false;
+    int D, F;
+    widest_rows(scans, nscans, &D, &F);
+    if (!tp_widths(D, F, forced, odd)) return false;
+    if (odd && !tph_takes_rows(D)) return false;
     int64_t widest_stride = 0;
     int mixed = nscans == 1 && combo_of(scans[0]) == kBBFB ? kMixedGradValues : 0;
     for (int i = 0; i < nscans; i++) {
@@ -561,11 +574,16 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
         if (combo != kFFFF && mixed == 0) mixed = kMixedRows;
         // rows with bf16 among them: the fp16-piece form of the kernel only
         if (combo == kNone || (combo != kFFFF && !tph_takes_rows(D))) return false;
-        if (sd.a.width != D || sd.v.width != F) return false;
-        if (L > 1 && !(stride_ok(sd.a.stride_l, D) && stride_ok(sd.b.stride_l, D) &&
-                       stride_ok(sd.v.stride_l, F) && stride_ok(sd.out.stride_l, F)))
+        // (odd widths: scans of any widths side by side, as long as none has a second block of columns)
+        if ((sd.a.width != D || sd.v.width != F) && !(odd && F <= 64)) return false;
+        if (odd && (combo != kFFFF || sd.a.width < 8 || sd.v.width < 8)) return false;
+        if (L > 1 && !(stride_ok(sd.a.stride_l, sd.a.width) && stride_ok(sd.b.stride_l, sd.a.width) &&
+                       stride_ok(sd.v.stride_l, sd.v.width) && stride_ok(sd.out.stride_l, sd.v.width)))
             return false;
-        if (!(aligned_quads(sd.a.ptr, sd.a.stride_n, sd.a.stride_h, sd.a.stride_l, sd.a.dtype) &&
+        if (odd) {
+            if (((uintptr_t)sd.a.ptr | (uintptr_t)sd.b.ptr | (uintptr_t)sd.v.ptr | (uintptr_t)sd.out.ptr) % 4)
+                return false;
+        } else if (!(aligned_quads(sd.a.ptr, sd.a.stride_n, sd.a.stride_h, sd.a.stride_l, sd.a.dtype) &&
               aligned_quads(sd.b.ptr, sd.b.stride_n, sd.b.stride_h, sd.b.stride_l, sd.b.dtype) &&
               aligned_quads(sd.v.ptr, sd.v.stride_n, sd.v.stride_h, sd.v.stride_l, sd.v.dtype) &&
               aligned_quads(sd.out.ptr, sd.out.stride_n, sd.out.stride_h, sd.out.stride_l, sd.out.dtype)))
@@ -577,8 +595,26 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     if ((L + 2 * kChunk) * std::max<int64_t>(widest_stride, std::max(D, F)) * 4 >= 0x7fffffffLL)
         return false;
     int nseg = 0, seg_chunks = 0;
-    tp_plan(D, F, std::max<int64_t>(1, N * H), nscans, L, &nseg, &seg_chunks, forced, mixed);
+    tp_plan(D, F, std::max<int64_t>(1, N * H), nscans, L, &nseg, &seg_chunks, forced, mixed, odd);
     return nseg > 0;
+}
+
+double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L) {
+    int nseg = 0, seg_chunks = 0;
+    const int64_t chains = std::max<int64_t>(1, N * H), units = chains * nscans * tp_fblocks(F);
+    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, false, 0, true);
+    if (nseg == 0) return 1e30;
+    const int64_t rounds = (units * nseg + 255) / 256;
+    double longest = 0.0;
+    if (seg_chunks > 0) {
+        longest = 1.6 * seg_chunks + 4.0;
+    } else {
+        int32_t start[kMaxTpSegments + 1];
+        nseg = tp_segment_starts((L + kChunk - 1) / kChunk, nseg, start);
+        for (int s = 0; s < nseg; s++)
+            longest = std::max(longest, 0.6 * start[s] + (double)(start[s + 1] - start[s]));
+    }
+    return (double)rounds * (longest + 4.0);
 }
 
 bool fused_attention_supported(const ScanDesc &sd, int64_t L) {
@@ -592,13 +628,14 @@ int64_t fused_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t
 
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
               void *workspace, size_t workspace_bytes, hipStream_t stream,
-              const FusedAttention *fused, bool may_chain_parallel, bool forced) {
+              const FusedAttention *fused, bool may_chain_parallel, bool forced, bool odd) {
     if (nscans < 1 || nscans > kMaxScans) return fail(FTC_ERR_INVALID, "bad scan count");
-    const int D = scans[0].a.width, F = scans[0].v.width;
+    int D, F;
+    widest_rows(scans, nscans, &D, &F);
     const Combo combo = combo_of(scans[0]);
     if (fused && (nscans != 1 || !fused_attention_supported(scans[0], L)))
         return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for this shape or layout");
-    const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced);
+    const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd);
     const int64_t chains = std::max<int64_t>(1, N * H);
     const int64_t fblocks = tp_shape ? tp_fblocks(F) : 1;
     int tpx_nseg = 0, tpx_seg_chunks = 0, tp_nseg = 0;
@@ -606,7 +643,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         int any_bf16 = nscans == 1 && combo == kBBFB ? kMixedGradValues : 0;
         for (int i = 0; i < nscans; i++)
             if (combo_of(scans[i]) != kFFFF && any_bf16 == 0) any_bf16 = kMixedRows;
-        tp_plan(D, F, chains, nscans, L, &tpx_nseg, &tpx_seg_chunks, forced, any_bf16);
+        tp_plan(D, F, chains, nscans, L, &tpx_nseg, &tpx_seg_chunks, forced, any_bf16, odd);
         if (tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     }
     const bool tp = tp_nseg > 0 || tpx_seg_chunks > 0;
@@ -647,10 +684,11 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         auto row_stride = [L](int64_t stride_l, int width) {
             return L == 1 ? std::max<int64_t>(stride_l, width) : stride_l;
         };
-        o.a_sn = sd.a.stride_n, o.a_sh = sd.a.stride_h, o.a_sl = row_stride(sd.a.stride_l, D);
-        o.b_sn = sd.b.stride_n, o.b_sh = sd.b.stride_h, o.b_sl = row_stride(sd.b.stride_l, D);
-        o.v_sn = sd.v.stride_n, o.v_sh = sd.v.stride_h, o.v_sl = row_stride(sd.v.stride_l, F);
-        o.o_sn = sd.out.stride_n, o.o_sh = sd.out.stride_h, o.o_sl = row_stride(sd.out.stride_l, F);
+        o.d = sd.a.width, o.f = sd.v.width;
+        o.a_sn = sd.a.stride_n, o.a_sh = sd.a.stride_h, o.a_sl = row_stride(sd.a.stride_l, o.d);
+        o.b_sn = sd.b.stride_n, o.b_sh = sd.b.stride_h, o.b_sl = row_stride(sd.b.stride_l, o.d);
+        o.v_sn = sd.v.stride_n, o.v_sh = sd.v.stride_h, o.v_sl = row_stride(sd.v.stride_l, o.f);
+        o.o_sn = sd.out.stride_n, o.o_sh = sd.out.stride_h, o.o_sl = row_stride(sd.out.stride_l, o.f);
         o.rev = sd.reverse ? 1 : 0;
         // (element types of the rows, for the kernel that takes them scan by scan)
         o.pad = (sd.a.dtype == FTC_BF16 ? kRowsBf16A : 0) | (sd.b.dtype == FTC_BF16 ? kRowsBf16B : 0) |
@@ -683,7 +721,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     args.nseg = pl.nseg;
     args.waves_per_scan = (int32_t)pl.waves;
     args.total_waves = (int32_t)(pl.waves * nscans * fblocks);
-    args.tp_d = D, args.tp_f = F, args.tp_fblocks = (int32_t)fblocks;
+    args.tp_d = D, args.tp_fblocks = (int32_t)fblocks;
     // very short chains: one level (every step adds the sums of all steps before it);
     // otherwise groups of about sqrt(nseg) steps, which moves fewer states per step
     args.group = pl.nseg;
@@ -701,7 +739,8 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     bool mixed = false;  // rows with bf16 among them
     for (int i = 0; i < nscans; i++) {
         mixed = mixed || combo_of(scans[i]) != kFFFF;
-        if ((!half_pieces && combo_of(scans[i]) != combo) || scans[i].a.width != D || scans[i].v.width != F)
+        if ((!half_pieces && combo_of(scans[i]) != combo) ||
+            (!(tp && odd) && (scans[i].a.width != D || scans[i].v.width != F)))
             return fail(FTC_ERR_INVALID, "scans of one launch must share widths and dtypes");
     }
     // fp32 states of up to 64 rows: the kernel that feeds its fragments from LDS tiles
@@ -727,7 +766,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     }
     if (tp) {
         if (half_pieces)
-            launch_scan_tph(workspace, args, mixed, stream);
+            launch_scan_tph(workspace, args, mixed, odd, stream);
         else
             launch_scan_tp(workspace, args, stream);
     } else if (wg) {

@@ -414,6 +414,7 @@ struct ScanOperands {
     int64_t o_sn, o_sh, o_sl;
     int32_t rev;  // 0: j <= l, walk up; 1: j >= l, walk down
     int32_t pad;  // kRowsBf16* bits (read by the kernel that takes rows of either type scan by scan)
+    int32_t d, f;  // widths of the rows (the chain-parallel kernels): a, b and v, out
     // optional D x F fp32 states per chain (null: none): the state the scan starts from and
     // the state after its last position; strides in elements, unit stride along F
     const float *s0;
@@ -476,9 +477,9 @@ struct ScanArgs {
     // ... or, with an exchange of segment sums (tp_exchange != 0), nseg segments of
     // tp_seg_chunks chunks (a multiple of kTpAhead), taken in the order of arrival
     int32_t tp_exchange, tp_seg_chunks;
-    // widths of the rows as they lie in memory (a, b: tp_d <= 128; v, out: tp_f <= 128, both
-    // multiples of 4) and the number of 64-column blocks of v and out, one workgroup each
-    int32_t tp_d, tp_f, tp_fblocks;
+    // the widest rows of a and b over the scans (<= 128), and the number of 64-column blocks of v
+    // and out, one workgroup each
+    int32_t tp_d, tp_fblocks;
 };
 
 // Which (scan, chain, L-segment) a wavefront works on.

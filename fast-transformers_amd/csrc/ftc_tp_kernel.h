@@ -145,9 +145,9 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     const uint32_t virt = which / nseg;
     const uint32_t scan_id = virt / (uint32_t)p.tp_fblocks;
     const int fb = (int)(virt % (uint32_t)p.tp_fblocks);
-    const int Dw = p.tp_d;                      // state rows in all: a and b are this wide
-    const int fw = min(F, p.tp_f - F * fb);     // output columns of this block
     const ScanOperands &op = p.scan[scan_id];
+    const int Dw = op.d;                        // state rows in all: a and b are this wide
+    const int fw = min(F, op.f - F * fb);       // output columns of this block
     const bool REV = op.rev != 0;
     const int n = (int)(chain / (uint32_t)p.H), h = (int)(chain % (uint32_t)p.H);
     const int rows = (int)p.L;

@@ -4,19 +4,25 @@
 namespace ftc {
 namespace mfma {
 
-void launch_scan_tph(void *ws, const ScanArgs &args, bool mixed, hipStream_t stream) {
+namespace {
+template <int KS>
+void launch(void *ws, const ScanArgs &args, bool mixed, bool odd, hipStream_t stream) {
     // (grid as for launch_scan_tp)
     const dim3 grid((unsigned)args.total_waves), block(768);
-    if (mixed) {
-        if (args.tp_d <= 32)
-            hipLaunchKernelGGL((scan_tph_kernel<1, true>), grid, block, 0, stream, (uint32_t *)ws, args);
-        else
-            hipLaunchKernelGGL((scan_tph_kernel<2, true>), grid, block, 0, stream, (uint32_t *)ws, args);
-    } else if (args.tp_d <= 32) {
-        hipLaunchKernelGGL((scan_tph_kernel<1, false>), grid, block, 0, stream, (uint32_t *)ws, args);
-    } else {
-        hipLaunchKernelGGL((scan_tph_kernel<2, false>), grid, block, 0, stream, (uint32_t *)ws, args);
-    }
+    if (mixed)
+        hipLaunchKernelGGL((scan_tph_kernel<KS, true, false>), grid, block, 0, stream, (uint32_t *)ws, args);
+    else if (odd)
+        hipLaunchKernelGGL((scan_tph_kernel<KS, false, true>), grid, block, 0, stream, (uint32_t *)ws, args);
+    else
+        hipLaunchKernelGGL((scan_tph_kernel<KS, false, false>), grid, block, 0, stream, (uint32_t *)ws, args);
+}
+}  // namespace
+
+void launch_scan_tph(void *ws, const ScanArgs &args, bool mixed, bool odd, hipStream_t stream) {
+    if (args.tp_d <= 32)
+        launch<1>(ws, args, mixed, odd, stream);
+    else
+        launch<2>(ws, args, mixed, odd, stream);
 }
 
 }  // namespace mfma

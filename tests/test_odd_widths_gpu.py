@@ -1,0 +1,45 @@
+"""fp32 rows of odd widths (and rows that are not 16-byte aligned) read and written where they lie
+by the fp16-piece kernel, against the CPU checker anchored on float64."""
+import pytest
+import torch
+
+import oracle
+from parity import scale_error
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # N, H, L, E, M: quads that straddle the width by one, two and three words; one and two groups of
+    # 32 state rows; two blocks of output columns; the smallest widths; whole, cut and exchanged chains;
+    # both state shapes of a backward call in one launch (80 chains) and in two (99)
+    (9, 11, 97, 25, 33), (10, 8, 130, 25, 33), (2, 4, 77, 41, 46), (3, 5, 65, 63, 63), (1, 3, 200, 8, 9),
+    (2, 4, 300, 50, 70), (1, 5, 1500, 51, 27), (1, 3, 9000, 31, 62), (40, 4, 33, 30, 10),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+def test_odd_widths_in_place(shape):
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = shape
+    Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=900 + L)
+    nlh = lambda t: t.permute(0, 2, 1, 3).contiguous().cuda().permute(0, 2, 1, 3)  # NLHE storage
+    q, k, v, g = (nlh(t) for t in (Q, K, V, G))
+    # results inside larger buffers: nothing around a row may be touched
+    def boxed(X):
+        box = torch.full((N, L, H, X + 3), 7.0, device="cuda")
+        return box, box[..., 1:X + 1].permute(0, 2, 1, 3)
+    boxes, outs = zip(*(boxed(X) for X in (M, E, E, M)))
+    cp.causal_dot_product_hip(q, k, v, outs[0])
+    assert b"scan_tph_kernel" in _native.load().ftc_last_kernel()
+    cp.causal_dot_backward_hip(q, k, v, g, *outs[1:])
+    assert b"scan_tph_kernel" in _native.load().ftc_last_kernel()
+    cp.check_workspaces()
+    for box in boxes:
+        assert (box[..., 0] == 7).all() and (box[..., -2:] == 7).all()
+    want = (oracle.forward(Q, K, V),) + tuple(oracle.backward(Q, K, V, G))
+    exact = (oracle.forward(Q.double(), K.double(), V.double()),) + \
+        tuple(oracle.backward(Q.double(), K.double(), V.double(), G.double()))
+    for got, ref, ex in zip(outs, want, exact):
+        # no further from float64 than four times the fp32 checker (or 2e-6 of the chain's largest)
+        assert scale_error(got.cpu(), ex) <= max(4 * scale_error(ref, ex), 2e-6)
