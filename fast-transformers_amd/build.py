@@ -82,7 +82,8 @@ def build(force=False, verbose=False, extra_flags=()):
     for src, p in procs:
         if p.wait() != 0:
             raise RuntimeError("hipcc failed on %s" % src)
-    if procs or force or not os.path.exists(OUT):
+    if procs or force or not os.path.exists(OUT) or \
+            os.path.getmtime(OUT) < max(os.path.getmtime(o) for o in objs):
         cmd = [hipcc, "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-rdc", "-o", OUT] + objs
         if verbose:
             print(" ".join(cmd), flush=True)

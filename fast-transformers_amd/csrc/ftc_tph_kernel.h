@@ -110,9 +110,12 @@ __device__ __forceinline__ float max_abs4(const u32x4 raw, float m) {
     return fmaxf(fmaxf(fabsf(__uint_as_float(raw.z)), fabsf(__uint_as_float(raw.w))), m);
 }
 
-// Exponents travel as E = e + 128 with e clamped to -100 .. 120 (E = 28 .. 248), where 2^e is
-// the ceiling: every value met so far is below it.
-constexpr uint32_t kExpFloor = 28, kExpCeil = 248;
+// Exponents travel as E = e + 128 with e clamped to -99 .. 120 (E = 29 .. 248), where 2^e is
+// the ceiling: every value met so far is below it.  E = 28: nothing but zeros so far.  A state
+// that comes in from elsewhere (another segment, the caller) is kept in units that the rows'
+// ceilings set, so zeros count as 2^-40 there: with units of 2^-200 a state of ones would leave
+// the range of fp32.
+constexpr uint32_t kExpFloor = 28, kExpCeil = 248, kExpOfZeros = 88;
 __device__ __forceinline__ float pow2_field(int field) {  // 2^(field - 127), field clamped
     return __uint_as_float((uint32_t)max(1, min(254, field)) << 23);
 }
@@ -132,7 +135,7 @@ __device__ __forceinline__ uint32_t scalar_min(uint32_t a, uint32_t b) {
 // NaN: the largest)
 __device__ __forceinline__ uint32_t ceiling_of(uint32_t bits) {
     const uint32_t be = (bits >> 23) & 0xffu;  // the value is below 2^(be - 126)
-    return scalar_max(kExpFloor, scalar_min(kExpCeil, be + 2u));
+    return bits == 0 ? kExpFloor : scalar_max(kExpFloor + 1u, scalar_min(kExpCeil, be + 2u));
 }
 // The largest of a non-negative float over the wavefront (wave-uniform): four steps inside
 // the rows of 16 lanes on the data-parallel path, then one lane of every row.
@@ -165,9 +168,15 @@ struct Ceilings {
     __device__ __forceinline__ float scale_a() const { return pow2_field(259 - (int)Ea); }
     __device__ __forceinline__ float scale_b() const { return pow2_field(259 - (int)Eb); }
     __device__ __forceinline__ float scale_v() const { return pow2_field(259 - (int)Ev); }
+    __device__ __forceinline__ uint32_t units_b() const { return Eb == kExpFloor ? kExpOfZeros : Eb; }
+    __device__ __forceinline__ uint32_t units_v() const { return Ev == kExpFloor ? kExpOfZeros : Ev; }
     // exponent of the state's units, and of a chunk's output units (a x state)
-    __device__ __forceinline__ int state_exp() const { return (int)(Eb + Ev) - 264; }
-    __device__ __forceinline__ int out_exp() const { return (int)(Ea + Eb + Ev) - 396; }
+    __device__ __forceinline__ int state_exp() const { return (int)(units_b() + units_v()) - 264; }
+    __device__ __forceinline__ int out_exp() const { return (int)(Ea + units_b() + units_v()) - 396; }
+    // the smallest magnitude that raises a ceiling
+    __device__ __forceinline__ static float raises(uint32_t E) {
+        return E == kExpFloor ? __uint_as_float(1u) : pow2_field((int)E - 1);
+    }
 };
 typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
 // The slot of a position is that of its LDS buffer: words (a, b, v, unused).  The words of b
@@ -192,7 +201,7 @@ __device__ __forceinline__ void raise_slot(lds_u32_t *slots, int k, int pos, con
     if (lane == 0)
         __hip_atomic_fetch_max(s + 0, ((uint32_t)(pos + 1) << 8) | ea, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
-    const bool over = mb >= pow2_field((int)c.Eb - 1) || mv >= pow2_field((int)c.Ev - 1);
+    const bool over = mb >= Ceilings::raises(c.Eb) || mv >= Ceilings::raises(c.Ev);
     if (__builtin_amdgcn_ballot_w64(over) != 0) {
         const uint32_t eb = ceiling_of(wave_max(mb)), ev = ceiling_of(wave_max(mv));
         if (lane == 0) {
@@ -809,6 +818,12 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         ce.Eb = max(ce.Eb, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.y));
         ce.Ev = max(ce.Ev, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.z));
         dU = Ucur - ce.state_exp();
+        if (dU > 0) {  // (rare: small values after nothing but zeros; all of S is up to date)
+            scale_state(dU);
+            s += dU;
+            Ucur -= dU;
+            dU = 0;
+        }
         kappa = pow2_field(127 + dU - s);
         plain_cut = dU - s == 0;
         s_cut = s;

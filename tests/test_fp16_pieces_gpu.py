@@ -175,3 +175,34 @@ def test_state_handed_in_at_another_scale(cp, factor):
     assert _last_kernel() in KERNELS
     _gate("product from a state x%g" % factor, out.cpu(), want, ex)
     _gate("final state x%g" % factor, state.cpu(), want_state, ex_state)
+
+
+@pytest.mark.parametrize("shape", [(1, 16, 16384), (10, 8, 1000), (1, 3, 400)], ids=lambda s: "n%d_h%d_l%d" % s)
+@pytest.mark.parametrize("zeros", ["keys_tail", "values_tail", "both_tail", "all_with_state", "then_small"])
+def test_stretches_of_zeros_next_to_a_state(shape, zeros):
+    """Masked keys or padded values: whole segments of zeros that receive a state from elsewhere
+    (the segments before them, the caller), and small values after nothing but zeros.  Against
+    float64 sums of the same inputs, at the scale gate of the other tests (2e-6 of the chain's
+    largest; four times that for the state's longest sums)."""
+    from fast_transformers_amd import causal_product as cp
+    N, H, L = shape
+    E = M = 64
+    gen = torch.Generator().manual_seed(21)
+    Q, K, V = (torch.rand(N, H, L, w, generator=gen) for w in (E, E, M))
+    S = torch.rand(N, H, E, M, generator=gen) * 100 if zeros in ("all_with_state", "then_small") else None
+    if zeros in ("keys_tail", "both_tail"):
+        K[:, :, L * 3 // 4:] = 0
+    if zeros in ("values_tail", "both_tail"):
+        V[:, :, L * 3 // 4:] = 0
+    if zeros == "all_with_state":
+        K.zero_(), V.zero_()
+    if zeros == "then_small":
+        K[:, :, :L // 2] = 0
+        K[:, :, L // 2:] *= 2.0 ** -70
+    got, state = cp.causal_dot_product_with_state(Q.cuda(), K.cuda(), V.cuda(),
+                                                  S.cuda() if S is not None else None)
+    cp.check_workspaces()
+    want, want_state = oracle.forward_with_state(Q.double(), K.double(), V.double(),
+                                                 S.double() if S is not None else None)
+    assert scale_error(got.cpu(), want) <= 8e-6
+    assert scale_error(state.cpu(), want_state) <= 8e-6
