@@ -116,6 +116,11 @@ __device__ __forceinline__ float max_abs4(const u32x4 raw, float m) {
 // ceilings set, so zeros count as 2^-40 there: with units of 2^-200 a state of ones would leave
 // the range of fp32.
 constexpr uint32_t kExpFloor = 28, kExpCeil = 248, kExpOfZeros = 88;
+// The running ceilings of b and v travel as words that order like the ceilings and whose low half
+// is the exponent to count with: E << 16 | E, and for zeros 0 << 16 | 88.
+__device__ __forceinline__ constexpr uint32_t ceiling_word(uint32_t E) {
+    return E <= kExpFloor ? kExpOfZeros : E << 16 | E;
+}
 __device__ __forceinline__ float pow2_field(int field) {  // 2^(field - 127), field clamped
     return __uint_as_float((uint32_t)max(1, min(254, field)) << 23);
 }
@@ -135,7 +140,7 @@ __device__ __forceinline__ uint32_t scalar_min(uint32_t a, uint32_t b) {
 // NaN: the largest)
 __device__ __forceinline__ uint32_t ceiling_of(uint32_t bits) {
     const uint32_t be = (bits >> 23) & 0xffu;  // the value is below 2^(be - 126)
-    return bits == 0 ? kExpFloor : scalar_max(kExpFloor + 1u, scalar_min(kExpCeil, be + 2u));
+    return scalar_max(kExpFloor, scalar_min(kExpCeil, be + 2u));
 }
 // The largest of a non-negative float over the wavefront (wave-uniform): four steps inside
 // the rows of 16 lanes on the data-parallel path, then one lane of every row.
@@ -164,19 +169,15 @@ __device__ __forceinline__ uint32_t wave_max(float m) {  // (the bits of the lar
 
 // The running ceilings of a, b and v as one wavefront knows them (wave-uniform).
 struct Ceilings {
-    uint32_t Ea, Eb, Ev;
+    uint32_t Ea, Wb, Wv;
+    __device__ __forceinline__ int Eb() const { return (int)(Wb & 0xffffu); }
+    __device__ __forceinline__ int Ev() const { return (int)(Wv & 0xffffu); }
     __device__ __forceinline__ float scale_a() const { return pow2_field(259 - (int)Ea); }
-    __device__ __forceinline__ float scale_b() const { return pow2_field(259 - (int)Eb); }
-    __device__ __forceinline__ float scale_v() const { return pow2_field(259 - (int)Ev); }
-    __device__ __forceinline__ uint32_t units_b() const { return Eb == kExpFloor ? kExpOfZeros : Eb; }
-    __device__ __forceinline__ uint32_t units_v() const { return Ev == kExpFloor ? kExpOfZeros : Ev; }
+    __device__ __forceinline__ float scale_b() const { return pow2_field(259 - Eb()); }
+    __device__ __forceinline__ float scale_v() const { return pow2_field(259 - Ev()); }
     // exponent of the state's units, and of a chunk's output units (a x state)
-    __device__ __forceinline__ int state_exp() const { return (int)(units_b() + units_v()) - 264; }
-    __device__ __forceinline__ int out_exp() const { return (int)(Ea + units_b() + units_v()) - 396; }
-    // the smallest magnitude that raises a ceiling
-    __device__ __forceinline__ static float raises(uint32_t E) {
-        return E == kExpFloor ? __uint_as_float(1u) : pow2_field((int)E - 1);
-    }
+    __device__ __forceinline__ int state_exp() const { return (int)((Wb + Wv) & 0xffffu) - 264; }
+    __device__ __forceinline__ int out_exp() const { return (int)(Ea + ((Wb + Wv) & 0xffffu)) - 396; }
 };
 typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
 // The slot of a position is that of its LDS buffer: words (a, b, v, unused).  The words of b
@@ -187,8 +188,8 @@ typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
 __device__ __forceinline__ void read_slot(const lds_u32_t *slots, int k, Ceilings &c) {
     const u32x4 s = *(const lds_vec4 *)(slots + 4 * k);
     c.Ea = max(kExpFloor, (uint32_t)__builtin_amdgcn_readfirstlane(s.x) & 0xffu);
-    c.Eb = max(c.Eb, (uint32_t)__builtin_amdgcn_readfirstlane(s.y));
-    c.Ev = max(c.Ev, (uint32_t)__builtin_amdgcn_readfirstlane(s.z));
+    c.Wb = max(c.Wb, (uint32_t)__builtin_amdgcn_readfirstlane(s.y));
+    c.Wv = max(c.Wv, (uint32_t)__builtin_amdgcn_readfirstlane(s.z));
 }
 // Lane maxima of the rows of position `pos` (slot k) against the ceilings of the position
 // before it.  a: every row of 16 lanes enters the ceiling of its own values (one lane per row:
@@ -201,12 +202,16 @@ __device__ __forceinline__ void raise_slot(lds_u32_t *slots, int k, int pos, con
     if (lane == 0)
         __hip_atomic_fetch_max(s + 0, ((uint32_t)(pos + 1) << 8) | ea, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
-    const bool over = mb >= Ceilings::raises(c.Eb) || mv >= Ceilings::raises(c.Ev);
+    // (after nothing but zeros: every normal number is at or above 2^-126)
+    const bool over = mb >= pow2_field((int)(c.Wb >> 16) - 1) || mv >= pow2_field((int)(c.Wv >> 16) - 1);
     if (__builtin_amdgcn_ballot_w64(over) != 0) {
-        const uint32_t eb = ceiling_of(wave_max(mb)), ev = ceiling_of(wave_max(mv));
+        auto word_of = [](uint32_t bits) -> uint32_t {
+            return ceiling_word(bits == 0 ? kExpFloor : scalar_max(kExpFloor + 1u, ceiling_of(bits)));
+        };
+        const uint32_t wb = word_of(wave_max(mb)), wv = word_of(wave_max(mv));
         if (lane == 0) {
-            if (eb > c.Eb) __hip_atomic_fetch_max(s + 1, eb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (ev > c.Ev) __hip_atomic_fetch_max(s + 2, ev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (wb > c.Wb) __hip_atomic_fetch_max(s + 1, wb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (wv > c.Wv) __hip_atomic_fetch_max(s + 2, wv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
     }
 }
@@ -306,7 +311,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     constexpr uint32_t kNoRow = 0x80000000u;  // an offset outside every descriptor
     auto chunk_row0 = [&](int c) -> int { return REV ? rows - kChunk * (c + 1) : kChunk * c; };
     if (tid < 16) slot_mem[tid] = 0;
-    Ceilings ce{kExpFloor, kExpFloor, kExpFloor};
+    Ceilings ce{kExpFloor, kExpOfZeros, kExpOfZeros};
     // Position k of the walk goes through LDS buffer (B0 + k) % 3 (pieces, Pt and slot), with B0
     // such that the first chunk of the walk proper has buffer 0: the consumers' loop over
     // those chunks is unrolled three times and addresses LDS with immediate offsets.
@@ -651,7 +656,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         if (op.s0) add_caller_state();
     }
     // ---- the walk proper ----
-    // `ce` holds the ceilings of the chunk at hand, Ucur the units of S.  dU <= 0: the
+    // `ce` holds the ceilings of the chunk at hand, Ucur the units of S.  dU < 0: the
     // state's units rise by -dU with this chunk (S is rescaled once all of it has been cut).
     int dU = Ucur - ce.state_exp();
     int s = 0;  // S is cut as S 2^(dU - s)
@@ -756,7 +761,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         if (dU != 0) {
             scale_state(dU);
             mS = __builtin_amdgcn_ldexpf(mS, dU);
-            s = max(0, s + dU);
+            s = max(0, s + min(dU, 0));
             Ucur -= dU;
         }
         if (B == 0) {
@@ -815,15 +820,11 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         }
         // the ceilings of the next chunk
         ce.Ea = max(kExpFloor, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.x) & 0xffu);
-        ce.Eb = max(ce.Eb, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.y));
-        ce.Ev = max(ce.Ev, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.z));
+        ce.Wb = max(ce.Wb, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.y));
+        ce.Wv = max(ce.Wv, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.z));
+        // (dU > 0: small values after nothing but zeros; the state's units fall, so s rises)
         dU = Ucur - ce.state_exp();
-        if (dU > 0) {  // (rare: small values after nothing but zeros; all of S is up to date)
-            scale_state(dU);
-            s += dU;
-            Ucur -= dU;
-            dU = 0;
-        }
+        s += max(dU, 0);
         kappa = pow2_field(127 + dU - s);
         plain_cut = dU - s == 0;
         s_cut = s;
