@@ -173,6 +173,28 @@ def test_sizes_without_a_fused_kernel_are_refused(lib):
     assert rc == -2 and "fused" in _native.last_error()
 
 
+CHAIN_PARALLEL_SHAPES = [
+    # N, L, H, E, M, key lengths: whole chains, cut chains, an exchange of segment sums (one and two
+    # levels), ragged ends, keys that end before, inside and on a chunk, segments without any key;
+    # one and two groups of 32 feature columns, half of the consumers without value columns
+    (3, 97, 8, 64, 64, [97, 64, 1]), (5, 300, 8, 64, 64, [300, 0, 299, 33, 160]),
+    (2, 1000, 16, 64, 64, [1000, 417]), (3, 520, 8, 64, 32, [520, 100, 40]),
+    (3, 520, 8, 32, 64, [520, 100, 40]), (2, 2500, 8, 64, 64, [2500, 700]),
+    (1, 9000, 16, 64, 64, [4000]),
+]
+
+
+@pytest.mark.parametrize("shape", CHAIN_PARALLEL_SHAPES, ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s[:5])
+def test_chain_parallel_form(lib, shape):
+    """The fused launch on the chain-parallel kernel, against the CPU restatement in float64."""
+    N, L, H, E, M, lens = shape
+    q, k, v = inputs(N, L, H, E, M, seed=70 + L)
+    lengths = torch.tensor(lens)
+    out = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
+    assert lib.ftc_last_kernel().startswith(b"scan_tph_kernel<NORM>"), lib.ftc_last_kernel()
+    gate(out.cpu(), q, k, v, lengths, 1e-6)
+
+
 def _count_backward_calls():
     """Context that counts the calls of the fused backward (autograd runs it on a thread of its
     own, where ftc_last_kernel() of this thread does not see it)."""
