@@ -29,6 +29,9 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option",
     "-I", INCLUDE, "-I", CSRC,
 ]
+# Accumulators in ordinary vector registers: with up to 256 of them in the other file the
+# compiler moves the matrix products' sums back and forth in every k-step.
+FILE_FLAGS = {"ftc_linear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def find_hipcc():
@@ -75,7 +78,8 @@ def build(force=False, verbose=False, extra_flags=()):
                  and os.path.getmtime(obj) >= newest_header)
         if fresh and not force:
             continue
-        cmd = [hipcc, "-c", src, "-o", obj] + HIPCC_FLAGS + list(extra_flags)
+        cmd = [hipcc, "-c", src, "-o", obj] + HIPCC_FLAGS + list(extra_flags) + \
+            FILE_FLAGS.get(os.path.basename(src), [])
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((src, subprocess.Popen(cmd)))

@@ -1,0 +1,521 @@
+// The encoder's matrix products on the fp16 matrix cores at the precision of fp32, and the passes
+// that feed them (include/ftc_causal_product.h: ftc_split_weights, ftc_split_rows,
+// ftc_layer_norm_split, ftc_linear_split).
+//
+//   out[t, f] = sum_k x[t, k] w[f, k] + bias[f]   (+ residual[t, f], or max(., 0))
+//
+// The fp32 matrix rate of this card is 157 TFLOP/s and the library's products of the encoder's
+// sizes reach 111 to 131 of them; fp16 matrix cores do sixteen times that.  As in
+// ftc_tph_kernel.h a row is scaled by a power of two and cut into two fp16 pieces, hi = fp16(x s)
+// and lo = fp16(x s - hi), and a product is hi hi + hi lo + lo hi, each exact in the fp32
+// accumulator.  A row's largest value is scaled to 2^14 .. 2^15, so hi + lo stands for every value
+// down to 2^-17 of that to within one unit in the last place of fp32 (and for smaller ones to
+// 2^-40 of the row's largest); the sums are fp32 sums of 32 products per rounding, where the
+// library rounds after every few: against float64 a product of 40960 x 512 by 512 x 512 is off by
+// 1.9e-7 (2-norm) where the library's is by 2.9e-7, of 1024 columns by 2.6e-7 and 4.1e-7.
+//
+// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 86, 512 -> 1536 475 / 220, 512 -> 1024
+// with relu 310 + 51 / 155, 1024 -> 512 with the residual 305 + 37 / 160; 5000 tokens, 256 -> 512 20 / 17;
+// 300 tokens, 128 -> 260 31 / 10.
+//
+// Rows in pieces take the bytes of fp32 rows: block of 32 columns after block, 64 bytes of hi and 64
+// of lo each, one cache line per row and k-step.  Whoever writes rows that only a product reads
+// writes them in pieces; the scale must be known before the row's first value is cut, so the
+// producer has the whole row (layer norm, ftc_split_rows) or a bound (relu: |y| <= max|x| max_f
+// sum_k |w[f, k]| + max|bias|, four or five bits above the largest value as a rule, which the
+// seventeen bits above leave room for).
+#include <algorithm>
+
+#include "ftc_tp_kernel.h"
+#include "ftc_tph_kernel.h"
+
+namespace ftc {
+namespace {
+using namespace mfma;
+
+constexpr int kStep = 32;                // columns per k-step
+constexpr int kRowBytes = 4 * kStep;     // a row's bytes of a k-step: hi, lo
+
+// the power of two that brings a largest magnitude to 2^14 .. 2^15, and its reciprocal
+__device__ __forceinline__ void scale_of(float largest, float &s, float &inverse) {
+    const int e = (int)((__float_as_uint(largest) >> 23) & 0xffu);  // largest < 2^(e - 126)
+    const int up = e == 0 ? 0 : max(-126, min(126, 141 - e));
+    s = __uint_as_float((uint32_t)(127 + up) << 23);
+    inverse = __uint_as_float((uint32_t)(127 - up) << 23);
+}
+// four consecutive columns of a row in pieces
+__device__ __forceinline__ void store_pieces(char *row, int col, const float4 &x, float s) {
+    uint32_t h0, h1, l0, l1;
+    cut_quad_f16(x.x, x.y, x.z, x.w, s, h0, h1, l0, l1);
+    char *at = row + (col / kStep) * kRowBytes + 2 * (col % kStep);
+    *(uint2 *)at = make_uint2(h0, h1);
+    *(uint2 *)(at + 2 * kStep) = make_uint2(l0, l1);
+}
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1) x += __shfl_xor(x, step);
+    return x;
+}
+__device__ __forceinline__ float wave_largest(float x) {
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1) x = fmaxf(x, __shfl_xor(x, step));
+    return x;
+}
+__device__ __forceinline__ float largest_of(const float4 &x) {
+    return fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
+}
+
+// ---- weights: a wavefront per row of any of the matrices --------------------------------------
+constexpr int kMostWeights = 8;
+struct WeightList {
+    const float *w[kMostWeights], *bias[kMostWeights];
+    int32_t first[kMostWeights + 1];     // rows before each matrix, in all at the end
+    int32_t cols[kMostWeights];
+    char *pieces[kMostWeights];          // of the matrix
+    float *scale[kMostWeights], *bias_out[kMostWeights], *norm[kMostWeights];
+    int32_t count;
+};
+__global__ __launch_bounds__(256) void split_weights_kernel(WeightList list) {
+    const int row = (int)(blockIdx.x * 4 + threadIdx.x / 64), lane = threadIdx.x % 64;
+    if (row >= list.first[list.count]) return;
+    int m = 0;
+    while (row >= list.first[m + 1]) m++;
+    const int r = row - list.first[m], cols = list.cols[m];
+    const float *w = list.w[m] + (int64_t)r * cols;
+    float largest = 0.f, sum = 0.f;
+    for (int c = 4 * lane; c < cols; c += 256) {
+        const float4 x = *(const float4 *)(w + c);
+        largest = fmaxf(largest, largest_of(x));
+        sum += (fabsf(x.x) + fabsf(x.y)) + (fabsf(x.z) + fabsf(x.w));
+    }
+    largest = wave_largest(largest);
+    sum = wave_sum(sum);
+    float s, inverse;
+    scale_of(largest, s, inverse);
+    char *out = list.pieces[m] + (int64_t)r * cols * 4;
+    for (int c = 4 * lane; c < cols; c += 256) store_pieces(out, c, *(const float4 *)(w + c), s);
+    if (lane == 0) {
+        list.scale[m][r] = inverse;
+        list.bias_out[m][r] = list.bias[m] ? list.bias[m][r] : 0.f;
+        list.norm[m][r] = sum;
+    }
+}
+
+// ---- rows: a wavefront per row, which it keeps in registers ------------------------------------
+// NORM: layer norm first (torch's: biased variance, two passes over the row in fp32)
+constexpr int kMostQuads = 16;           // quads of a row per lane: rows of up to 4096 values
+template <int QUADS, bool NORM>
+__global__ __launch_bounds__(256) void rows_kernel(const float *__restrict__ x, const float *__restrict__ gamma,
+                                                   const float *__restrict__ beta, float eps, int64_t rows,
+                                                   int cols, float *__restrict__ out,
+                                                   char *__restrict__ pieces, float *__restrict__ scale) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
+    const int lane = threadIdx.x % 64;
+    if (row >= rows) return;
+    float4 v[QUADS];
+#pragma unroll
+    for (int i = 0; i < QUADS; i++) {
+        const int c = 4 * (lane + 64 * i);
+        v[i] = c < cols ? *(const float4 *)(x + row * cols + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    if (NORM) {
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < QUADS; i++) sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+        const float mean = wave_sum(sum) / (float)cols;
+        float squares = 0.f;
+#pragma unroll
+        for (int i = 0; i < QUADS; i++) {
+            if (4 * (lane + 64 * i) >= cols) continue;
+            v[i].x -= mean, v[i].y -= mean, v[i].z -= mean, v[i].w -= mean;
+            squares += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+        }
+        const float r = 1.0f / sqrtf(wave_sum(squares) / (float)cols + eps);
+#pragma unroll
+        for (int i = 0; i < QUADS; i++) {
+            const int c = 4 * (lane + 64 * i);
+            if (c >= cols) continue;
+            const float4 g = gamma ? *(const float4 *)(gamma + c) : make_float4(1.f, 1.f, 1.f, 1.f);
+            const float4 b = beta ? *(const float4 *)(beta + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[i].x = v[i].x * r * g.x + b.x, v[i].y = v[i].y * r * g.y + b.y;
+            v[i].z = v[i].z * r * g.z + b.z, v[i].w = v[i].w * r * g.w + b.w;
+            *(float4 *)(out + row * cols + c) = v[i];
+        }
+    }
+    if (!pieces) return;
+    float largest = 0.f;
+#pragma unroll
+    for (int i = 0; i < QUADS; i++) largest = fmaxf(largest, largest_of(v[i]));
+    largest = wave_largest(largest);
+    float s, inverse;
+    scale_of(largest, s, inverse);
+#pragma unroll
+    for (int i = 0; i < QUADS; i++) {
+        const int c = 4 * (lane + 64 * i);
+        if (c < cols) store_pieces(pieces + row * cols * 4, c, v[i], s);
+    }
+    if (lane == 0) scale[row] = inverse;
+}
+
+// ---- the product --------------------------------------------------------------------------------
+struct LinearArgs {
+    const char *x, *w;                   // rows in pieces
+    const float *x_scale, *w_scale, *bias, *w_norm;
+    const float *residual;               // kResidual
+    float *out;                          // kPlain, kResidual
+    char *out_pieces;                    // kRelu
+    float *out_scale;
+    int64_t tokens;
+    int32_t features, k, feature_tiles;
+};
+enum { kPlain = 0, kResidual = 1, kRelu = 2 };
+
+// a raw buffer of `bytes` bytes
+__device__ __forceinline__ u32x4 descriptor(const void *base, uint32_t bytes) {
+    const uint64_t a = (uint64_t)base;
+    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), kRsrcFlags};
+}
+// 16 bytes per lane from memory into LDS, lane L to byte `to` + 16 L.  (Written out: the compiler
+// does not follow which of the three buffers a request of its own fills, and would wait for all
+// requests before any read of LDS.  The waits are the k-loop's.)
+__device__ __forceinline__ void load_to_lds(const u32x4 rs, uint32_t to, uint32_t offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :: "s"(to), "v"(offset), "s"(rs) : "memory", "m0");
+}
+
+__device__ __forceinline__ void load_dword_to_lds(const u32x4 rs, uint32_t to, uint32_t offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                 :: "s"(to), "v"(offset), "s"(rs) : "memory", "m0");
+}
+
+// A workgroup of four wavefronts takes tiles of TN tokens by TF features one after the other, a
+// wavefront half of either.  v_mfma_f32_16x16x32_f16 with the features as rows of the result, so
+// that a lane has four consecutive features of one token.  A k-step's rows (128 bytes each) go from
+// memory straight into LDS, two steps ahead, through three buffers; one barrier per step.
+// Split: with 64 x 128 results per wavefront a step reads 24 KB of fragments for 96 matrix
+// instructions (1536 cycles): 768 cycles of the LDS for the four wavefronts and 384 for the
+// rows coming in, three quarters of the time; smaller tiles would be bound by the LDS.  The three
+// buffers leave room for one workgroup per CU, so nothing else runs while a tile begins or ends:
+// the last two steps of a tile request the first two of the next one, and the rows that go out are
+// not waited for.
+template <int TN, int TF, int EPI>
+__global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
+    constexpr int WT = TN / 32, WF = TF / 32;          // tiles of 16 per wavefront
+    constexpr int kBuf = (TN + TF) * kRowBytes;
+    constexpr int kLoadsX = TN * kRowBytes / 4096, kLoadsW = TF * kRowBytes / 4096;  // per lane
+    constexpr int kStores = (EPI == kRelu ? 2 : 1) * WT * WF;                        // per lane
+    __shared__ __align__(16) char tiles_mem[3 * kBuf];
+    // scales and bias of a tile's tokens and features, as each wavefront needs them
+    constexpr int kScales = TN / 2 + TF;
+    __shared__ __align__(16) float scales_mem[2][4][kScales];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ln = lane & 15, g = lane >> 4;
+    const int wt = wave & 1, wf = wave >> 1;
+    const uint32_t row_bytes = (uint32_t)p.k * 4;
+    const int steps = p.k / kStep;
+    // Workgroups go round the eight XCDs: those of one XCD take the feature tiles of a token tile
+    // at the same time, so that its rows are read from memory once.
+    struct Tile {
+        int64_t t0;
+        int f0;
+        bool there;
+        u32x4 x_rs, w_rs, xs_rs, ws_rs, b_rs;
+    };
+    auto tile_of = [&](int round) -> Tile {
+        const int idx = (int)(blockIdx.x / 8) + round * (int)(gridDim.x / 8);
+        Tile t;
+        t.t0 = ((int64_t)(idx / p.feature_tiles) * 8 + blockIdx.x % 8) * TN;
+        t.f0 = (idx % p.feature_tiles) * TF;
+        t.there = t.t0 < p.tokens;
+        const int64_t from = t.there ? t.t0 : 0;
+        const int nt = t.there ? (int)min((int64_t)TN, p.tokens - t.t0) : 0;
+        const int nf = t.there ? min(TF, p.features - t.f0) : 0;
+        t.x_rs = descriptor(p.x + from * row_bytes, (uint32_t)nt * row_bytes);
+        t.w_rs = descriptor(p.w + (int64_t)t.f0 * row_bytes, (uint32_t)nf * row_bytes);
+        t.xs_rs = descriptor(p.x_scale + from, (uint32_t)nt * 4u);
+        t.ws_rs = descriptor(p.w_scale + t.f0, (uint32_t)nf * 4u);
+        t.b_rs = descriptor(p.bias + t.f0, (uint32_t)nf * 4u);
+        return t;
+    };
+    // lane's 16 bytes of a load: slot j of the tile holds piece-and-quarter (j % 8) ^ key of row j / 8
+    uint32_t x_off[kLoadsX], w_off[kLoadsW];
+#pragma unroll
+    for (int i = 0; i < kLoadsX; i++) {
+        const int j = (i * 4 + wave) * 64 + lane, row = j / 8;
+        x_off[i] = (uint32_t)row * row_bytes + 16u * ((j % 8) ^ TpSwizzle<128>::key(row));
+    }
+#pragma unroll
+    for (int i = 0; i < kLoadsW; i++) {
+        const int j = (i * 4 + wave) * 64 + lane, row = j / 8;
+        w_off[i] = (uint32_t)row * row_bytes + 16u * ((j % 8) ^ TpSwizzle<128>::key(row));
+    }
+    lds_char *const tiles = (lds_char *)tiles_mem;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)tiles + 1024u * wave;
+    const uint32_t scales0 = (uint32_t)(uintptr_t)(lds_char *)scales_mem + (uint32_t)(kScales * 4) * wave;
+    // request number i of a step
+    auto fetch = [&](const Tile &t, int buf, int step, int i) {
+        const uint32_t at = (uint32_t)step * kRowBytes, to = lds0 + (uint32_t)buf * kBuf;
+        if (i < kLoadsX)
+            load_to_lds(t.x_rs, to + 4096u * i, x_off[i] + at);
+        else
+            load_to_lds(t.w_rs, to + TN * kRowBytes + 4096u * (i - kLoadsX), w_off[(i - kLoadsX) % kLoadsW] + at);
+    };
+    constexpr int kRequests = kLoadsX + kLoadsW;
+    // (before the first step's, so that whoever waits for its rows waits for the scales too)
+    auto fetch_scales = [&](const Tile &t, int round) {
+        static_assert(TN == 128 && TF % 128 == 0, "64 tokens, TF / 2 features per wavefront");
+        const uint32_t to = scales0 + (uint32_t)(round & 1) * (4 * kScales * 4);
+        load_dword_to_lds(t.xs_rs, to, 4u * (uint32_t)(wt * (TN / 2) + lane));
+#pragma unroll
+        for (int i = 0; i < TF / 128; i++) {
+            const uint32_t from = 4u * (uint32_t)(wf * (TF / 2) + 64 * i + lane);
+            load_dword_to_lds(t.ws_rs, to + 4u * (TN / 2 + 64 * i), from);
+            load_dword_to_lds(t.b_rs, to + 4u * (TN / 2 + TF / 2 + 64 * i), from);
+        }
+    };
+    int x_addr[2], w_addr[2];  // [piece]; further tiles 16 rows of 128 bytes on
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        x_addr[k] = TpSwizzle<128>::addr(wt * (TN / 2) + ln, 64 * k + 16 * g);
+        w_addr[k] = TN * kRowBytes + TpSwizzle<128>::addr(wf * (TF / 2) + ln, 64 * k + 16 * g);
+    }
+    f32x4 acc[WF][WT];
+    // (written out in issue order: fragments of the next feature tile and a request for a later step
+    // under the matrix instructions of this one, instructions that add to one accumulator at least
+    // WT apart)
+    auto compute = [&](const lds_char *buf, auto request) {
+        Frag xf[WT][2], w[2][2];
+        w[0][1] = lds_frag16(buf + w_addr[1]);
+#pragma unroll
+        for (int j = 0; j < WT; j++) xf[j][0] = lds_frag16(buf + x_addr[0] + j * 16 * kRowBytes);
+        w[0][0] = lds_frag16(buf + w_addr[0]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < WF; i++) {
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                if (i == 0 && m == 0) {
+#pragma unroll
+                    for (int j = 0; j < WT; j++) xf[j][1] = lds_frag16(buf + x_addr[1] + j * 16 * kRowBytes);
+                }
+                if (m > 0 && i + 1 < WF)
+                    w[(i + 1) % 2][2 - m] = lds_frag16(buf + w_addr[2 - m] + (i + 1) * 16 * kRowBytes);
+                if (i * 3 + m < kRequests) request(i * 3 + m);
+#pragma unroll
+                for (int j = 0; j < WT; j++)
+                    acc[i][j] = mfma16h(w[i % 2][m == 0 ? 1 : 0], xf[j][m == 1 ? 1 : 0], acc[i][j]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    static_assert(3 * WF >= kRequests, "a request per group of matrix instructions");
+    float bound_w = 0.f, bound_b = 0.f;
+    if (EPI == kRelu) {  // (the same numbers in every workgroup)
+        for (int i = lane; i < p.features; i += 64) {
+            bound_w = fmaxf(bound_w, p.w_norm[i]);
+            bound_b = fmaxf(bound_b, fabsf(p.bias[i]));
+        }
+        bound_w = wave_largest(bound_w), bound_b = wave_largest(bound_b);
+    }
+    Tile t = tile_of(0);
+    if (!t.there) return;
+    fetch_scales(t, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * kRequests; i++) fetch(t, i / kRequests, i / kRequests, i % kRequests);
+    int now = 0;
+    for (int round = 0; t.there; round++) {
+        const Tile next = tile_of(round + 1);
+#pragma unroll
+        for (int i = 0; i < WF; i++)
+#pragma unroll
+            for (int j = 0; j < WT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < steps; s++) {
+            // This step's rows have landed (in flight: the next step's requests and, in the first
+            // two steps of a tile, the rows that the tile before has sent out), and every wavefront
+            // is done with the buffer that the step after the next one goes to.
+            constexpr int kFirst = kRequests + kStores < 63 ? kRequests + kStores : 63;
+            if (s < 2 && round > 0)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFirst) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kRequests) : "memory");
+            const int later = now == 0 ? 2 : now - 1;
+            if (s + 2 < steps) {
+                compute(tiles + now * kBuf, [&](int i) { fetch(t, later, s + 2, i); });
+            } else {
+                if (s + 2 == steps) fetch_scales(next, round + 1);
+                compute(tiles + now * kBuf, [&](int i) { fetch(next, later, s + 2 - steps, i); });
+            }
+            now = now == 2 ? 0 : now + 1;
+        }
+        // ---- rows out: every store is made, those outside the tensor outside the descriptor, so
+        // that their number is known to the waits above ----
+        const int nt = (int)min((int64_t)TN, p.tokens - t.t0);
+        const uint32_t out_row = (uint32_t)p.features * 4u;
+        const __amdgpu_buffer_rsrc_t o_rs = __builtin_amdgcn_make_buffer_rsrc(
+            (EPI == kRelu ? (char *)p.out_pieces : (char *)p.out) + t.t0 * out_row, 0, (uint32_t)nt * out_row,
+            kRsrcFlags);
+        const __amdgpu_buffer_rsrc_t r_rs = __builtin_amdgcn_make_buffer_rsrc(
+            (char *)(EPI == kResidual ? p.residual : p.bias) + (EPI == kResidual ? t.t0 * out_row : 0), 0,
+            (uint32_t)nt * out_row, kRsrcFlags);
+        const float *const scales = scales_mem[round & 1][wave];
+        float xs[WT], s_out[WT];
+        uint32_t at[WT];
+#pragma unroll
+        for (int j = 0; j < WT; j++) {
+            const int tok = 16 * j + ln;
+            xs[j] = scales[tok];
+            at[j] = (uint32_t)(wt * (TN / 2) + tok) * out_row;
+            if (EPI == kRelu) {
+                float inverse;
+                scale_of((32768.f * xs[j]) * bound_w + bound_b, s_out[j], inverse);
+                const int64_t token = t.t0 + wt * (TN / 2) + tok;
+                if (t.f0 == 0 && wf == 0 && g == 0 && token < p.tokens) p.out_scale[token] = inverse;
+            }
+        }
+        // (residual rows two feature tiles ahead: a wait for them then leaves the stores in flight)
+        u32x4 res[3][WT];
+        auto residual = [&](int i) {
+            const int f = t.f0 + wf * (TF / 2) + 16 * i + 4 * g;
+#pragma unroll
+            for (int j = 0; j < WT; j++)
+                res[i % 3][j] = __builtin_amdgcn_raw_buffer_load_b128(
+                    r_rs, f < p.features ? at[j] + 4u * f : 0x80000000u, 0, 0);
+        };
+        if (EPI == kResidual) residual(0), residual(1);
+#pragma unroll
+        for (int i = 0; i < WF; i++) {
+            const int fl = 16 * i + 4 * g, f = t.f0 + wf * (TF / 2) + fl;
+            const bool f_in = f < p.features;
+            const float4 ws = *(const float4 *)(scales + TN / 2 + fl),
+                         b = *(const float4 *)(scales + TN / 2 + TF / 2 + fl);
+            if (EPI == kResidual && i + 2 < WF) residual(i + 2);
+#pragma unroll
+            for (int j = 0; j < WT; j++) {
+                float y0 = fmaf(acc[i][j][0] * xs[j], ws.x, b.x), y1 = fmaf(acc[i][j][1] * xs[j], ws.y, b.y),
+                      y2 = fmaf(acc[i][j][2] * xs[j], ws.z, b.z), y3 = fmaf(acc[i][j][3] * xs[j], ws.w, b.w);
+                if (EPI == kResidual) {
+                    const u32x4 r = res[i % 3][j];
+                    y0 += __uint_as_float(r.x), y1 += __uint_as_float(r.y);
+                    y2 += __uint_as_float(r.z), y3 += __uint_as_float(r.w);
+                }
+                if (EPI == kRelu) {
+                    uint32_t h0, h1, l0, l1;
+                    cut_quad_f16(fmaxf(y0, 0.f), fmaxf(y1, 0.f), fmaxf(y2, 0.f), fmaxf(y3, 0.f), s_out[j], h0, h1, l0, l1);
+                    const uint32_t to = f_in ? at[j] + (uint32_t)(f / kStep * kRowBytes + 2 * (f % kStep)) : 0x80000000u;
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{h0, h1}, o_rs, to, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{l0, l1}, o_rs, to + 2 * kStep, 0, 0);
+                } else {
+                    buffer_store4(o_rs, f_in ? at[j] + 4u * f : 0x80000000u, y0, y1, y2, y3);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        t = next;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the requests of a tile that is not there)
+}
+
+int launched(const char *what) {
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return fail(FTC_ERR_HIP, "%s launch failed: %s", what, hipGetErrorString(err));
+    return FTC_OK;
+}
+bool aligned(const void *p) { return (uintptr_t)p % 16 == 0; }
+
+template <bool NORM>
+int launch_rows(const float *x, const float *gamma, const float *beta, float eps, int64_t rows, int64_t cols,
+                float *out, void *pieces, float *scale, hipStream_t stream) {
+    if (cols % kStep != 0 || cols > 256 * kMostQuads)
+        return fail(FTC_ERR_UNSUPPORTED, "rows of %lld values", (long long)cols);
+    if (!aligned(x) || !aligned(gamma) || !aligned(beta) || !aligned(out) || !aligned(pieces))
+        return fail(FTC_ERR_INVALID, "rows must be 16-byte aligned");
+    if (rows <= 0) return FTC_OK;
+    const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+#define FTC_ROWS(Q)                                                                                   \
+    hipLaunchKernelGGL((rows_kernel<Q, NORM>), grid, block, 0, stream, x, gamma, beta, eps, rows, (int)cols, out, \
+                       (char *)pieces, scale)
+    const int64_t quads = (cols + 255) / 256;
+    if (quads <= 1) FTC_ROWS(1);
+    else if (quads <= 2) FTC_ROWS(2);
+    else if (quads <= 4) FTC_ROWS(4);
+    else FTC_ROWS(16);
+#undef FTC_ROWS
+    return launched("row");
+}
+
+}  // namespace
+}  // namespace ftc
+
+using namespace ftc;
+
+extern "C" {
+
+int ftc_split_weights(const ftc_weight *weights, int32_t count, void *stream) {
+    if (!weights || count < 1 || count > kMostWeights) return fail(FTC_ERR_INVALID, "1 to 8 weights");
+    WeightList list;
+    list.count = count;
+    list.first[0] = 0;
+    for (int i = 0; i < count; i++) {
+        const ftc_weight &w = weights[i];
+        if (!w.w || !w.pieces || !w.scale || !w.bias_out || !w.norm || !aligned(w.w) || !aligned(w.pieces))
+            return fail(FTC_ERR_INVALID, "weight %d: null or misaligned pointer", i);
+        if (w.cols % kStep != 0 || w.cols <= 0 || w.rows <= 0 || w.rows % 4 != 0)
+            return fail(FTC_ERR_UNSUPPORTED, "weight %d: %lld x %lld", i, (long long)w.rows, (long long)w.cols);
+        list.w[i] = w.w, list.bias[i] = w.bias, list.cols[i] = (int32_t)w.cols;
+        list.pieces[i] = (char *)w.pieces, list.scale[i] = w.scale;
+        list.bias_out[i] = w.bias_out, list.norm[i] = w.norm;
+        list.first[i + 1] = list.first[i] + (int32_t)w.rows;
+    }
+    hipLaunchKernelGGL(split_weights_kernel, dim3((unsigned)((list.first[count] + 3) / 4)), dim3(256), 0,
+                       (hipStream_t)stream, list);
+    return launched("weight");
+}
+
+int ftc_split_rows(const float *x, int64_t rows, int64_t cols, void *pieces, float *scale, void *stream) {
+    if (!x || !pieces || !scale) return fail(FTC_ERR_INVALID, "null pointer");
+    return launch_rows<false>(x, nullptr, nullptr, 0.f, rows, cols, nullptr, pieces, scale, (hipStream_t)stream);
+}
+
+int ftc_layer_norm_split(const float *x, const float *gamma, const float *beta, float eps, int64_t rows,
+                         int64_t cols, float *out, void *pieces, float *scale, void *stream) {
+    if (!x || !out || (pieces && !scale)) return fail(FTC_ERR_INVALID, "null pointer");
+    return launch_rows<true>(x, gamma, beta, eps, rows, cols, out, pieces, scale, (hipStream_t)stream);
+}
+
+int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
+                     const float *bias, const float *w_norm, int64_t features, int64_t k,
+                     const float *residual, float *out, void *relu_pieces, float *relu_scale, void *stream) {
+    if (!x || !x_scale || !w || !w_scale || !bias || (!out && !relu_pieces))
+        return fail(FTC_ERR_INVALID, "null pointer");
+    if (relu_pieces && (!relu_scale || !w_norm || residual || out))
+        return fail(FTC_ERR_INVALID, "relu rows leave in pieces, with a scale and without a residual");
+    if (!aligned(x) || !aligned(w) || !aligned(w_scale) || !aligned(bias) || !aligned(residual) || !aligned(out) ||
+        !aligned(relu_pieces))
+        return fail(FTC_ERR_INVALID, "rows must be 16-byte aligned");
+    if (k % kStep != 0 || k < 2 * kStep || k > (1 << 20) || features % 4 != 0 || features <= 0 ||
+        (relu_pieces && features % kStep != 0))
+        return fail(FTC_ERR_UNSUPPORTED, "a product of %lld columns and %lld features", (long long)k, (long long)features);
+    if (tokens <= 0) return FTC_OK;
+    constexpr int TN = 128, TF = 256;
+    LinearArgs a;
+    a.x = (const char *)x, a.w = (const char *)w, a.x_scale = x_scale, a.w_scale = w_scale, a.bias = bias;
+    a.w_norm = w_norm, a.residual = residual, a.out = out, a.out_pieces = (char *)relu_pieces;
+    a.out_scale = relu_scale, a.tokens = tokens, a.features = (int32_t)features, a.k = (int32_t)k;
+    a.feature_tiles = (int32_t)((features + TF - 1) / TF);
+    const int64_t token_tiles = (tokens + TN - 1) / TN;
+    // (one workgroup per CU, a multiple of the eight XCDs)
+    const int64_t tiles = (token_tiles + 7) / 8 * a.feature_tiles;
+    const dim3 grid((unsigned)(8 * std::min<int64_t>(tiles, 32))), block(256);
+    if (relu_pieces)
+        hipLaunchKernelGGL((linear_kernel<TN, TF, kRelu>), grid, block, 0, (hipStream_t)stream, a);
+    else if (residual)
+        hipLaunchKernelGGL((linear_kernel<TN, TF, kResidual>), grid, block, 0, (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL((linear_kernel<TN, TF, kPlain>), grid, block, 0, (hipStream_t)stream, a);
+    return launched("product");
+}
+
+}  // extern "C"

@@ -36,6 +36,10 @@ EXPORTED_SYMBOLS = (
     "ftc_causal_linear_attention_forward",
     "ftc_causal_linear_attention_backward_workspace_bytes",
     "ftc_causal_linear_attention_backward",
+    "ftc_split_weights",
+    "ftc_split_rows",
+    "ftc_layer_norm_split",
+    "ftc_linear_split",
 )
 
 

@@ -4,14 +4,16 @@ Own counterparts of ``fast_transformers/attention/attention_layer.py:44-115`` (Q
 projections around an inner attention) and ``fast_transformers/transformers.py:21-145``
 (post-norm encoder layer, stack with optional final norm).  Parameter names match the
 reference modules so that a reference ``state_dict`` loads unchanged.  Plain ``torch.nn``:
-the only custom kernel is inside the inner attention.
+the custom kernels are inside the inner attention -- and, for a whole encoder of plain layers in
+inference, in its matrix products and norms as well (``TransformerEncoder._fused_forward``).
 """
 import torch
 import torch.nn.functional as F
 from torch.nn import Dropout, LayerNorm, Linear, Module, ModuleList
 
+from ..causal_product import encoder_forward_hip
 from ..masking import FullMask, LengthMask, TriangularCausalMask
-from .causal_linear_attention import CausalLinearAttention
+from .causal_linear_attention import CausalLinearAttention, ActivationFunctionFeatureMap, _elu_plus_one
 
 
 class AttentionLayer(Module):
@@ -71,6 +73,68 @@ class TransformerEncoderLayer(Module):
         return self.norm2(x + y)
 
 
+def _watched(module):
+    return module._forward_hooks or module._forward_pre_hooks
+
+
+def _plain_tensors(x, *tensors):
+    return all(t is None or (t.dtype == torch.float32 and t.device == x.device and t.is_contiguous()
+                             and t.data_ptr() % 16 == 0) for t in tensors)
+
+
+def _plain_linear(module, x):
+    """(weight, bias) of a plain ``Linear`` whose sizes the native products take."""
+    if type(module) is not Linear or _watched(module) or not _plain_tensors(x, module.weight, module.bias):
+        return None
+    rows, cols = module.weight.shape
+    if rows % 32 or cols % 32 or cols < 64:
+        return None
+    return module.weight, module.bias
+
+
+def _plain_norm(module, x):
+    if type(module) is not LayerNorm or _watched(module) or not _plain_tensors(x, module.weight, module.bias):
+        return None
+    if len(module.normalized_shape) != 1 or module.normalized_shape[0] != x.shape[2] or x.shape[2] > 4096:
+        return None
+    return module.weight, module.bias, module.eps
+
+
+def _plain_layer(layer, x):
+    """(sizes of the heads, parameters) of a layer in eval mode that is made of the plain parts
+    (no subclasses, hooks, other activations or feature maps), else None."""
+    d = x.shape[2]
+    if type(layer) is not TransformerEncoderLayer or layer.activation is not F.relu or _watched(layer):
+        return None
+    if layer.dropout.p > 0 and layer.dropout.training or type(layer.dropout) is not Dropout or _watched(layer.dropout):
+        return None
+    outer = layer.attention
+    if type(outer) is not AttentionLayer or _watched(outer):
+        return None
+    inner = outer.inner_attention
+    if type(inner) is not CausalLinearAttention or _watched(inner):
+        return None
+    fm = inner.feature_map
+    if type(fm) is not ActivationFunctionFeatureMap or fm.activation_function is not _elu_plus_one or _watched(fm):
+        return None
+    linears = [_plain_linear(m, x) for m in (outer.query_projection, outer.key_projection, outer.value_projection,
+                                             outer.out_projection, layer.linear1, layer.linear2)]
+    norms = [_plain_norm(m, x) for m in (layer.norm1, layer.norm2)]
+    if any(part is None for part in linears + norms):
+        return None
+    heads = outer.n_heads
+    (q, k, v, o, w1, w2) = (weight for weight, _ in linears)
+    if q.shape[0] % heads or v.shape[0] % heads:
+        return None
+    E, M = q.shape[0] // heads, v.shape[0] // heads
+    if E not in (32, 64) or M not in (32, 64) or k.shape != q.shape or v.shape[0] > 4096:
+        return None
+    if (q.shape[1], v.shape[1], tuple(o.shape), w1.shape[1], tuple(w2.shape)) != \
+            (d, d, (d, v.shape[0]), d, (d, w1.shape[0])):
+        return None
+    return (heads, E, M), (linears, norms, inner.eps)
+
+
 class TransformerEncoder(Module):
     """A stack of encoder layers with an optional final norm (``transformers.py:92-145``)."""
 
@@ -79,7 +143,34 @@ class TransformerEncoder(Module):
         self.layers = ModuleList(layers)
         self.norm = norm_layer
 
+    def _fused_forward(self, x, attn_mask, length_mask):
+        """The whole stack in native code (``encoder_forward_hip``) where nothing has to be
+        differentiated or watched and every part is the plain one; None otherwise."""
+        if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.numel() > 0) or len(self.layers) == 0:
+            return None
+        if attn_mask is None or not attn_mask.lower_triangular or attn_mask.shape[0] != x.shape[1]:
+            return None
+        if torch.is_autocast_enabled() or torch.nn.modules.module._has_any_global_hook():
+            return None
+        lengths = None
+        if length_mask is not None:
+            lengths = getattr(length_mask, "lengths", None)
+            if lengths is None:
+                return None
+            lengths = lengths.to(device=x.device, dtype=torch.int64).contiguous()
+        layers = [_plain_layer(layer, x) for layer in self.layers]
+        if any(layer is None or layer[0] != layers[0][0] for layer in layers):
+            return None
+        norm = _plain_norm(self.norm, x) if self.norm is not None else ()
+        if norm is None or (torch.is_grad_enabled() and (
+                x.requires_grad or any(p.requires_grad for p in self.parameters()))):
+            return None
+        return encoder_forward_hip(x, [layer[1] for layer in layers], norm, layers[0][0], lengths)
+
     def forward(self, x, attn_mask=None, length_mask=None):
+        fused = self._fused_forward(x, attn_mask, length_mask)
+        if fused is not None:
+            return fused
         N, L = x.shape[0], x.shape[1]
         attn_mask = attn_mask or FullMask(L, device=x.device)
         length_mask = length_mask or LengthMask(x.new_full((N,), L, dtype=torch.int64))

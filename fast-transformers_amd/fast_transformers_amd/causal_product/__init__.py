@@ -206,6 +206,20 @@ def causal_linear_attention_backward_hip(queries, keys, values, key_lengths, out
                                grad_queries, grad_keys, grad_values)
 
 
+def encoder_forward_hip(x, layers, final_norm, heads, key_lengths):
+    """A stack of post-norm encoder layers with causal linear attention and ReLU, in eval mode
+    (``transformers.py:76-89,133-145`` with ``attention/attention_layer.py:96-115``): the products
+    at fp32 precision on the fp16 matrix cores (``csrc/ftc_linear.hip``), the attention in its fused
+    launch.  ``layers``: per layer ((weight, bias) of the query, key, value and output projections
+    and of the two feed-forward products, (weight, bias, eps) of the two norms, the attention's
+    eps); ``final_norm``: (weight, bias, eps) or (); ``heads``: (H, E, M)."""
+    host = _host()
+    native = [host.Layer(*(host.Linear(*l) for l in linears), *(host.Norm(*n) for n in norms), eps)
+              for linears, norms, eps in layers]
+    return host.encoder(x.contiguous(), native, host.Norm(*final_norm) if final_norm else None, *heads,
+                        key_lengths)
+
+
 class CausalLinearAttentionFunction(torch.autograd.Function):
     """``out = causal linear attention(queries, keys, values)`` with the feature map
     ``elu(x) + 1``, the key-length mask and the normaliser inside, one fused launch forward

@@ -12,16 +12,20 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <pybind11/stl.h>
+
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdlib>
 #include <map>
 #include <string>
 #include <tuple>
+#include <vector>
 
 #include "ftc_causal_product.h"
 
@@ -260,6 +264,125 @@ void attention_backward(const Tensor &queries, const Tensor &keys, const Tensor 
     call.done();
 }
 
+// ---- the encoder's forward, eval mode ----
+struct Linear {
+    Tensor weight;
+    OptTensor bias;
+};
+struct Norm {
+    OptTensor weight, bias;
+    double eps;
+};
+struct Layer {
+    Linear query, key, value, out, first, second;
+    Norm norm1, norm2;
+    double eps;
+};
+
+// One weight matrix (or several with the same number of columns, their rows one after the other)
+// in pieces.
+struct Pieces {
+    Tensor pieces, scale, bias, norm;
+    int64_t rows, cols;
+    Pieces(std::initializer_list<const Linear *> parts, std::vector<ftc_weight> &list) {
+        rows = 0, cols = (*parts.begin())->weight.size(1);
+        for (const Linear *l : parts) rows += l->weight.size(0);
+        const auto fp32 = (*parts.begin())->weight.options();
+        pieces = at::empty({rows, cols}, fp32);
+        scale = at::empty({rows}, fp32), bias = at::empty({rows}, fp32), norm = at::empty({rows}, fp32);
+        int64_t at_row = 0;
+        for (const Linear *l : parts) {
+            ftc_weight w;
+            w.w = l->weight.const_data_ptr<float>();
+            w.bias = l->bias ? l->bias->const_data_ptr<float>() : nullptr;
+            w.rows = l->weight.size(0), w.cols = cols;
+            w.pieces = pieces.data_ptr<float>() + at_row * cols;
+            w.scale = scale.data_ptr<float>() + at_row, w.bias_out = bias.data_ptr<float>() + at_row;
+            w.norm = norm.data_ptr<float>() + at_row;
+            list.push_back(w);
+            at_row += w.rows;
+        }
+    }
+};
+
+// A stack of post-norm encoder layers (attention/encoder.py) with causal linear attention, and the
+// final norm: every product on the fp16 matrix cores in pieces (csrc/ftc_linear.hip), the norms
+// leaving their rows in pieces as well.  `x`: dense (N, L, d).
+Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::optional<Norm> &final_norm,
+               int64_t H, int64_t E, int64_t M, const OptTensor &key_lengths) {
+    const at::NoGradGuard no_grad;
+    const int64_t N = x.size(0), L = x.size(1), d = x.size(2), T = N * L;
+    const auto fp32 = x.options();
+    const int64_t *lengths = lengths_ptr(key_lengths, x);
+    const int64_t width = H * (2 * E + M);
+    int64_t ff = 0;
+    for (const Layer &l : layers) ff = std::max(ff, l.first.weight.size(0));
+    const Tensor qkv = at::empty({T, width}, fp32), rows = at::empty({T, H * M}, fp32), y = at::empty({T, d}, fp32),
+                 x1 = at::empty({T, d}, fp32), x_pieces = at::empty({T, d}, fp32), x_scale = at::empty({T}, fp32),
+                 r_pieces = at::empty({T, H * M}, fp32), r_scale = at::empty({T}, fp32),
+                 h_pieces = at::empty({T, ff}, fp32), h_scale = at::empty({T}, fp32), out = at::empty_like(x);
+    Tensor now = x;  // the layer's input
+    Tensor next = layers.size() > 1 || final_norm ? at::empty({T, d}, fp32) : out;
+    auto view = [&](const Tensor &t, int64_t column, int64_t row, int64_t X) {
+        ftc_tensor4 v;
+        v.ptr = t.data_ptr<float>() + column, v.dtype = FTC_F32;
+        v.size[0] = N, v.size[1] = H, v.size[2] = L, v.size[3] = X;
+        v.stride[0] = L * row, v.stride[1] = X, v.stride[2] = row, v.stride[3] = 1;
+        return v;
+    };
+    const ftc_tensor4 q = view(qkv, 0, width, E), k = view(qkv, H * E, width, E),
+                      v = view(qkv, 2 * H * E, width, M), o = view(rows, 0, H * M, M);
+    Call call(x, workspace_bytes(ftc_causal_linear_attention_workspace_bytes,
+                                 "ftc_causal_linear_attention_workspace_bytes", N, H, L, E, M, FTC_F32));
+    void *const stream = call.stream;
+    auto f = [](const OptTensor &t) { return t ? t->const_data_ptr<float>() : nullptr; };
+    auto linear = [&](const Tensor &pieces, const Tensor &scale, const Pieces &w, const float *residual,
+                      const Tensor &to) {
+        check(ftc_linear_split(pieces.data_ptr(), scale.const_data_ptr<float>(), T, w.pieces.data_ptr(),
+                               w.scale.const_data_ptr<float>(), w.bias.const_data_ptr<float>(),
+                               w.norm.const_data_ptr<float>(), w.rows, w.cols, residual, to.data_ptr<float>(),
+                               nullptr, nullptr, stream),
+              "ftc_linear_split");
+    };
+    auto norm = [&](const Tensor &in, const Norm &n, const Tensor &to, bool pieces) {
+        check(ftc_layer_norm_split(in.const_data_ptr<float>(), f(n.weight), f(n.bias), (float)n.eps, T, d,
+                                   to.data_ptr<float>(), pieces ? x_pieces.data_ptr() : nullptr,
+                                   pieces ? x_scale.data_ptr<float>() : nullptr, stream),
+              "ftc_layer_norm_split");
+    };
+    check(ftc_split_rows(x.const_data_ptr<float>(), T, d, x_pieces.data_ptr(), x_scale.data_ptr<float>(), stream),
+          "ftc_split_rows");
+    for (size_t i = 0; i < layers.size(); i++) {
+        const Layer &l = layers[i];
+        std::vector<ftc_weight> list;
+        const Pieces in({&l.query, &l.key, &l.value}, list), proj({&l.out}, list), first({&l.first}, list),
+            second({&l.second}, list);
+        check(ftc_split_weights(list.data(), (int32_t)list.size(), stream), "ftc_split_weights");
+        linear(x_pieces, x_scale, in, nullptr, qkv);
+        check(ftc_causal_linear_attention_forward(&q, &k, &v, lengths, (float)l.eps, &o, nullptr, call.ws,
+                                                  call.ws_bytes, stream),
+              "ftc_causal_linear_attention_forward");
+        check(ftc_split_rows(rows.const_data_ptr<float>(), T, H * M, r_pieces.data_ptr(), r_scale.data_ptr<float>(),
+                             stream),
+              "ftc_split_rows");
+        linear(r_pieces, r_scale, proj, now.const_data_ptr<float>(), y);
+        norm(y, l.norm1, x1, true);
+        check(ftc_linear_split(x_pieces.data_ptr(), x_scale.const_data_ptr<float>(), T, first.pieces.data_ptr(),
+                               first.scale.const_data_ptr<float>(), first.bias.const_data_ptr<float>(),
+                               first.norm.const_data_ptr<float>(), first.rows, first.cols, nullptr, nullptr,
+                               h_pieces.data_ptr(), h_scale.data_ptr<float>(), stream),
+              "ftc_linear_split");
+        linear(h_pieces, h_scale, second, x1.const_data_ptr<float>(), y);
+        const bool last = i + 1 == layers.size();
+        if (last && !final_norm) next = out;
+        norm(y, l.norm2, next, !last);
+        now = next;
+    }
+    if (final_norm) norm(now, *final_norm, out, false);
+    call.done();
+    return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_ftc_host, m) {
@@ -270,4 +393,9 @@ PYBIND11_MODULE(_ftc_host, m) {
     m.def("backward", &backward);
     m.def("attention", &attention);
     m.def("attention_backward", &attention_backward);
+    py::class_<Linear>(m, "Linear").def(py::init<Tensor, OptTensor>());
+    py::class_<Norm>(m, "Norm").def(py::init<OptTensor, OptTensor, double>());
+    py::class_<Layer>(m, "Layer").def(
+        py::init<Linear, Linear, Linear, Linear, Linear, Linear, Norm, Norm, double>());
+    m.def("encoder", &encoder);
 }

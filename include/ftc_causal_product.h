@@ -263,6 +263,39 @@ int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_t
                                          const ftc_tensor4 *grad_keys, const ftc_tensor4 *grad_values,
                                          void *workspace, size_t workspace_bytes, void *stream);
 
+/*
+ * The matrix products of an encoder layer around the attention (attention/attention_layer.py:96-115,
+ * transformers.py:76-89) at the precision of fp32 on the fp16 matrix cores: every row is scaled by a
+ * power of two and kept as two fp16 pieces, hi + lo = row x 2^e, and a product is the sum of three
+ * piece products in fp32.  Rows in pieces take 4 bytes per value: for each block of 32 columns 32 hi
+ * and then 32 lo; `scale` holds 2^-e per row.  All pointers are device pointers, 16-byte aligned;
+ * numbers of columns are multiples of 32 (at most 4096 for rows), of features multiples of 4.
+ */
+typedef struct ftc_weight {
+    const float *w;        /* rows x cols, dense (torch.nn.Linear.weight) */
+    const float *bias;     /* rows values, or NULL */
+    int64_t rows, cols;    /* rows: a multiple of 4 */
+    void *pieces;          /* out: rows x cols in pieces */
+    float *scale;          /* out: rows values */
+    float *bias_out;       /* out: bias, or zeros */
+    float *norm;           /* out: sum of |w| along each row */
+} ftc_weight;
+/* Up to eight weight matrices into pieces. */
+int ftc_split_weights(const ftc_weight *weights, int32_t count, void *stream);
+/* Dense fp32 rows into pieces. */
+int ftc_split_rows(const float *x, int64_t rows, int64_t cols, void *pieces, float *scale, void *stream);
+/* out = torch.nn.LayerNorm of dense rows (gamma, beta may be NULL), also in pieces unless NULL. */
+int ftc_layer_norm_split(const float *x, const float *gamma, const float *beta, float eps, int64_t rows,
+                         int64_t cols, float *out, void *pieces, float *scale, void *stream);
+/*
+ * y[t][f] = sum_k x[t][k] w[f][k] + bias[f] for rows in pieces.  Either out = y (+ residual, dense
+ * tokens x features, unless NULL), or max(y, 0) in pieces (relu_pieces, relu_scale; w_norm from
+ * ftc_split_weights bounds the rows).
+ */
+int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
+                     const float *bias, const float *w_norm, int64_t features, int64_t k,
+                     const float *residual, float *out, void *relu_pieces, float *relu_scale, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,136 @@
+"""The encoder's products and norms in pieces (ftc_linear.hip) through the C ABI, against float64;
+the encoder's native forward against the composition of its modules."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+class Weight(ctypes.Structure):
+    _fields_ = [("w", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("rows", ctypes.c_int64),
+                ("cols", ctypes.c_int64), ("pieces", ctypes.c_void_p), ("scale", ctypes.c_void_p),
+                ("bias_out", ctypes.c_void_p), ("norm", ctypes.c_void_p)]
+
+
+def ptr(t):
+    return ctypes.c_void_p(t.data_ptr() if t is not None else None)
+
+
+def stream():
+    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def whole(pieces, scale):
+    rows, cols = pieces.shape
+    h = pieces.view(torch.float16).view(rows, cols // 32, 2, 32).double()
+    return (h[:, :, 0] + h[:, :, 1]).reshape(rows, cols) * scale.double()[:, None]
+
+
+PRODUCTS = [
+    # tokens, columns, features: edges of the 128 x 256 tile, one to many k-steps, more tiles than
+    # workgroups
+    (1, 64, 4), (127, 96, 252), (128, 64, 256), (129, 512, 260), (1000, 160, 1536), (70000, 64, 288),
+    (300, 1024, 512),
+]
+
+
+@pytest.mark.parametrize("shape", PRODUCTS, ids=lambda s: "t%d_k%d_f%d" % s)
+def test_products_in_pieces(shape):
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    T, K, F = shape
+    gen = torch.Generator(device="cuda").manual_seed(T + K + F)
+    x, w, b, r = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, K), (F, K), (F,), (T, F)))
+    # rows far apart in size, and values far apart within a row
+    x *= torch.exp2(torch.randint(-60, 60, (T, 1), device="cuda", generator=gen).float())
+    w *= torch.exp2(torch.randint(-20, 20, (F, 1), device="cuda", generator=gen).float())
+    x[:, ::3] *= 2.0 ** -12
+    new = lambda *s: torch.full(s, float("nan"), device="cuda")
+    xp, xs, wp, ws, bo, wn = new(T, K), new(T), new(F, K), new(F), new(F), new(F)
+    item = Weight(w.data_ptr(), b.data_ptr(), F, K, wp.data_ptr(), ws.data_ptr(), bo.data_ptr(), wn.data_ptr())
+    assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == 0, _native.last_error()
+    assert lib.ftc_split_rows(ptr(x), ctypes.c_int64(T), ctypes.c_int64(K), ptr(xp), ptr(xs), stream()) == 0
+    for whole_rows, rows in ((whole(xp, xs), x), (whole(wp, ws), w)):
+        # one unit in the last place of fp32, or 2^-39 of the row's largest
+        assert ((whole_rows - rows.double()).abs() <= 2.0 ** -23 * rows.double().abs()
+                + 2.0 ** -39 * rows.double().abs().amax(1, keepdim=True)).all()
+    assert torch.equal(bo, b)
+    assert ((wn.double() - w.double().abs().sum(1)).abs() <= 1e-5 * w.double().abs().sum(1)).all()
+
+    def run(residual=None, out=None, pieces=None, scale=None):
+        rc = lib.ftc_linear_split(ptr(xp), ptr(xs), ctypes.c_int64(T), ptr(wp), ptr(ws), ptr(bo), ptr(wn),
+                                  ctypes.c_int64(F), ctypes.c_int64(K), ptr(residual), ptr(out), ptr(pieces),
+                                  ptr(scale), stream())
+        assert rc == 0, _native.last_error()
+    exact = x.double() @ w.double().t()
+    # pieces: 2^-23 per value and 2^-24 for lo lo; sums: 2^-24 per rounding of K / 32 + 3 partial sums
+    bound = (x.double().abs() @ w.double().abs().t()) * (3 * 2.0 ** -23 + (K / 32 + 3) * 2.0 ** -24) \
+        + 2.0 ** -23 * (b.double().abs() + exact.abs())
+    out = new(T, F)
+    run(out=out)
+    assert ((out.double() - (exact + b.double())).abs() <= bound).all()
+    run(residual=r, out=out)
+    assert ((out.double() - (exact + b.double() + r.double())).abs() <= bound + 2.0 ** -23 * r.double().abs()).all()
+    if F % 32 == 0:
+        hp, hs = new(T, F), new(T)
+        run(pieces=hp, scale=hs)
+        # (the row's bound, max|x| max_f sum|w| + max|b|, is at most K + 1 times what the products reach)
+        largest = 2 * (x.double().abs().amax(1, keepdim=True) * w.double().abs().sum(1).max() + b.double().abs().max())
+        want = (exact + b.double()).clamp_min(0)
+        assert ((whole(hp, hs) - want).abs() <= bound + 2.0 ** -22 * want + 2.0 ** -39 * largest).all()
+
+
+@pytest.mark.parametrize("rows_cols", [(1, 32), (5, 96), (130, 512), (33, 1056), (3, 4096)], ids=lambda s: "r%d_c%d" % s)
+def test_layer_norm_in_pieces(rows_cols):
+    from fast_transformers_amd import _native
+    R, C = rows_cols
+    gen = torch.Generator(device="cuda").manual_seed(R + C)
+    x, g, b = (torch.randn(*s, device="cuda", generator=gen) for s in ((R, C), (C,), (C,)))
+    x = x * 3 + 5
+    out, pieces, scale = (torch.full(s, float("nan"), device="cuda") for s in ((R, C), (R, C), (R,)))
+    rc = _native.load().ftc_layer_norm_split(ptr(x), ptr(g), ptr(b), ctypes.c_float(1e-5), ctypes.c_int64(R),
+                                             ctypes.c_int64(C), ptr(out), ptr(pieces), ptr(scale), stream())
+    assert rc == 0, _native.last_error()
+    want = torch.nn.functional.layer_norm(x.double(), (C,), g.double(), b.double(), 1e-5)
+    plain = torch.nn.functional.layer_norm(x, (C,), g, b, 1e-5).double()
+    assert (out.double() - want).abs().max() <= max(4 * (plain - want).abs().max(), 2e-6)
+    assert (whole(pieces, scale) - out.double()).abs().max() <= 2.0 ** -23 * out.double().abs().max()
+
+
+@pytest.mark.parametrize("sizes", [(2, 300, 2, 8, 64, 64, 1024), (3, 129, 3, 4, 32, 32, 512), (1, 7, 1, 4, 64, 32, 96)],
+                         ids=lambda s: "n%d_l%d_x%d_h%d_e%d_m%d_f%d" % s)
+@pytest.mark.parametrize("ragged", [False, True], ids=["full", "ragged"])
+@pytest.mark.parametrize("final", [True, False], ids=["final_norm", "no_norm"])
+def test_encoder_native_forward(sizes, ragged, final):
+    from fast_transformers_amd import attention, masking
+    N, L, layers, H, E, M, ff = sizes
+    torch.manual_seed(L)
+    with torch.device("cuda"):
+        model = attention.build_causal_linear_encoder(layers, H, E, M, ff, final_normalization=final).eval()
+    x = torch.rand(N, L, H * M, device="cuda")
+    mask = masking.TriangularCausalMask(L, device="cuda")
+    lengths = masking.LengthMask(torch.randint(1, L + 1, (N,), device="cuda"), max_len=L) if ragged else None
+    calls = []
+    from fast_transformers_amd.attention import encoder as module
+    native = module.encoder_forward_hip
+    module.encoder_forward_hip = lambda *a: (calls.append(1), native(*a))[1]
+    try:
+        with torch.no_grad():
+            got = model(x, attn_mask=mask, length_mask=lengths)
+            assert calls == [1]
+            # a hook on any part asks for the modules themselves
+            handle = model.layers[0].linear1.register_forward_hook(lambda *a: None)
+            want = model(x, attn_mask=mask, length_mask=lengths)
+            handle.remove()
+        assert calls == [1]
+        # something to differentiate: the modules
+        out = model(x, attn_mask=mask, length_mask=lengths)
+        assert calls == [1] and out.requires_grad
+        with pytest.raises(RuntimeError):
+            model(x, length_mask=lengths)          # not causal: refused as before
+    finally:
+        module.encoder_forward_hip = native
+    # two fp32 evaluations: 1e-6 per layer of the largest value (norms keep rows near one)
+    assert (got - want).abs().max() <= 4e-6 * layers * want.abs().max()
