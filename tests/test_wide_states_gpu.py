@@ -1,0 +1,82 @@
+"""States of 65 to 128 rows on two fp16 pieces (csrc/ftc_tph_wide_kernel.h): chains of 32 chunks or
+more, walked whole, cut, or with an exchange; widths that do not fill either block; rows whose
+scale changes along the chain; a state handed in and out.  Gate: no further from float64 than
+four times the fp32 checker, or 2e-6 of the chain's largest (the gate of the narrower states)."""
+import pytest
+import torch
+
+import oracle
+from parity import scale_error
+
+pytestmark = pytest.mark.gpu
+
+#        N  H  L     E    M
+SHAPES = [(1, 2, 1000, 68, 16),    # one quad in the second block, three consumers without columns
+          (2, 3, 1024, 96, 64),    # the second block half full; whole chunks
+          (1, 3, 1025, 100, 100),  # one row in the last chunk; a second block of columns
+          (1, 2, 1061, 128, 128),
+          (24, 6, 993, 72, 68),    # more chains than half the workgroups
+          (2, 8, 2052, 72, 68)]    # exchange
+
+
+@pytest.fixture(scope="module")
+def cp():
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a GPU (torch.cuda.is_available() is False)")
+    from fast_transformers_amd import causal_product
+    return causal_product
+
+
+def _gate(got, ref, exact):
+    assert torch.isfinite(got).all()
+    assert scale_error(got, exact) <= max(4 * scale_error(ref, exact), 2e-6)
+
+
+def _check(cp, Q, K, V, G):
+    q, k, v, g = (t.cuda() for t in (Q, K, V, G))
+    outs = [torch.full_like(t, float("nan")) for t in (v, q, k, v)]
+    cp.causal_dot_product_hip(q, k, v, outs[0])
+    cp.causal_dot_backward_hip(q, k, v, g, *outs[1:])
+    cp.check_workspaces()
+    wide = [t.double() for t in (Q, K, V, G)]
+    refs = [oracle.forward(Q, K, V)] + list(oracle.backward(Q, K, V, G))
+    exact = [oracle.forward(*wide[:3])] + list(oracle.backward(*wide))
+    for got, ref, ex in zip(outs, refs, exact):
+        _gate(got.cpu(), ref, ex)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+def test_wide_states(cp, shape):
+    _check(cp, *oracle.make_inputs(*shape, seed=70 + shape[2]))
+
+
+@pytest.mark.parametrize("how", ["rising", "zeros", "large"])
+def test_scales_along_the_chain(cp, how):
+    Q, K, V, G = oracle.make_inputs(1, 2, 1050, 128, 72, seed=7)
+    if how == "rising":      # both ceilings rise, the second block's rows first
+        up = torch.logspace(-6, 4, 1050)[:, None]
+        K = K * up
+        K[..., 64:] *= 8
+        V = V * up.sqrt()
+    elif how == "zeros":     # whole chunks of zeros, at the start and in the middle, in one block or both
+        K[:, :, :70] = 0
+        K[:, :, 300:400, 64:] = 0
+        Q[:, :, 500:600, :64] = 0
+        V[:, :, 640:705] = 0
+    else:                    # a state far beyond 2^14 scaled units
+        K = K.abs() + 1
+        V = V.abs() + 1
+    _check(cp, Q, K, V, G)
+
+
+@pytest.mark.parametrize("L", [1000, 1056])
+def test_state_in_and_out(cp, L):
+    N, H, E, M = 2, 3, 104, 84
+    Q, K, V, _ = oracle.make_inputs(N, H, L, E, M, seed=L)
+    S = 50 * torch.randn(N, H, E, M, generator=torch.Generator().manual_seed(1))
+    out, last = cp.causal_dot_product_with_state(Q.cuda(), K.cuda(), V.cuda(), S.cuda())
+    Kd, Vd = K.double(), V.double()
+    exact = oracle.forward(Q.double(), Kd, Vd) + Q.double() @ S.double()
+    ref = oracle.forward(Q, K, V) + Q @ S
+    _gate(out.cpu(), ref, exact)
+    _gate(last.cpu(), S + K.transpose(-1, -2) @ V, S.double() + Kd.transpose(-1, -2) @ Vd)
