@@ -22,7 +22,7 @@
 // of lo each, one cache line per row and k-step.  Whoever writes rows that only a product reads
 // writes them in pieces; the scale must be known before the row's first value is cut, so the
 // producer has the whole row (layer norm, ftc_split_rows) or a bound (relu: |y| <= max|x| max_f
-// sum_k |w[f, k]| + max|bias|, four or five bits above the largest value as a rule, which the
+// sum_k |w[f, k]| + the largest bias, four or five bits above the largest value as a rule, which the
 // seventeen bits above leave room for).
 #include <algorithm>
 
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     if (EPI == kRelu) {  // (the same numbers in every workgroup)
         for (int i = lane; i < p.features; i += 64) {
             bound_w = fmaxf(bound_w, p.w_norm[i]);
-            bound_b = fmaxf(bound_b, fabsf(p.bias[i]));
+            bound_b = fmaxf(bound_b, p.bias[i]);  // (a bias below zero, lowest or -inf, raises nothing)
         }
         bound_w = wave_largest(bound_w), bound_b = wave_largest(bound_b);
     }
@@ -403,7 +403,8 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
                 }
                 if (EPI == kRelu) {
                     uint32_t h0, h1, l0, l1;
-                    cut_quad_f16(fmaxf(y0, 0.f), fmaxf(y1, 0.f), fmaxf(y2, 0.f), fmaxf(y3, 0.f), s_out[j], h0, h1, l0, l1);
+                    auto relu = [](float y) { return y < 0.f ? 0.f : y; };  // (keeps NaN, as torch's does)
+                    cut_quad_f16(relu(y0), relu(y1), relu(y2), relu(y3), s_out[j], h0, h1, l0, l1);
                     const uint32_t to = f_in ? at[j] + (uint32_t)(f / kStep * kRowBytes + 2 * (f % kStep)) : 0x80000000u;
                     __builtin_amdgcn_raw_buffer_store_b64(u32x2{h0, h1}, o_rs, to, 0, 0);
                     __builtin_amdgcn_raw_buffer_store_b64(u32x2{l0, l1}, o_rs, to + 2 * kStep, 0, 0);

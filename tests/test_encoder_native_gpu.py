@@ -82,6 +82,29 @@ def test_products_in_pieces(shape):
         assert ((whole(hp, hs) - want).abs() <= bound + 2.0 ** -22 * want + 2.0 ** -39 * largest).all()
 
 
+def test_relu_keeps_nan_and_takes_any_bias_below_zero():
+    """Features switched off by a bias of the type's lowest value or -inf leave the other features'
+    precision alone; NaN in a weight or a bias comes out as NaN, as from torch's relu."""
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    T, K, F = 130, 64, 288
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    x, w, b = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, K), (F, K), (F,)))
+    b[3], b[200], b[7], w[260, 5] = float("-inf"), torch.finfo(torch.float32).min, float("nan"), float("nan")
+    new = lambda *s: torch.zeros(s, device="cuda")
+    xp, xs, wp, ws, bo, wn, hp, hs = new(T, K), new(T), new(F, K), new(F), new(F), new(F), new(T, F), new(T)
+    item = Weight(w.data_ptr(), b.data_ptr(), F, K, wp.data_ptr(), ws.data_ptr(), bo.data_ptr(), wn.data_ptr())
+    assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == 0, _native.last_error()
+    assert lib.ftc_split_rows(ptr(x), ctypes.c_int64(T), ctypes.c_int64(K), ptr(xp), ptr(xs), stream()) == 0
+    assert lib.ftc_linear_split(ptr(xp), ptr(xs), ctypes.c_int64(T), ptr(wp), ptr(ws), ptr(bo), ptr(wn),
+                                ctypes.c_int64(F), ctypes.c_int64(K), None, None, ptr(hp), ptr(hs), stream()) == 0
+    got, want = whole(hp, hs), torch.relu(x.double() @ w.double().t() + b.double())
+    assert torch.equal(got.isnan(), want.isnan()) and want[:, [7, 260]].isnan().all()
+    assert (got[:, [3, 200]] == 0).all()
+    # K + 1 roundings of sums of absolute products below 200, pieces of the row's bound below 2^-38 of it
+    assert (got - want).nan_to_num().abs().max() <= (K + 1) * 2.0 ** -24 * 200
+
+
 @pytest.mark.parametrize("rows_cols", [(1, 32), (5, 96), (130, 512), (33, 1056), (3, 4096)], ids=lambda s: "r%d_c%d" % s)
 def test_layer_norm_in_pieces(rows_cols):
     from fast_transformers_amd import _native
