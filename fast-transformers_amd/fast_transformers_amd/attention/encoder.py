@@ -9,7 +9,8 @@ inference, in its matrix products and norms as well (``TransformerEncoder._fused
 """
 import torch
 import torch.nn.functional as F
-from torch.nn import Dropout, LayerNorm, Linear, Module, ModuleList
+from torch.nn import Dropout, LayerNorm, Linear, Module, ModuleList, Parameter
+from torch.utils._device import DeviceContext
 
 from ..causal_product import encoder_forward_hip
 from ..masking import FullMask, LengthMask, TriangularCausalMask
@@ -74,11 +75,24 @@ class TransformerEncoderLayer(Module):
 
 
 def _watched(module):
-    return module._forward_hooks or module._forward_pre_hooks
+    # (an instance's own ``forward`` stands in for its class's, as offloading wrappers put it there)
+    return module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+
+
+def _observed():
+    """True where something has to see or rewrite the single operations: a compiler or tracer, a
+    functorch transform, forward-mode differentiation, a dispatch or function mode (apart from the
+    default device's, which only places new tensors)."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0
+            or any(type(mode) is not DeviceContext
+                   for mode in torch.overrides._get_current_function_mode_stack()))
 
 
 def _plain_tensors(x, *tensors):
-    return all(t is None or (t.dtype == torch.float32 and t.device == x.device and t.is_contiguous()
+    return all(t is None or (type(t) in (torch.Tensor, Parameter) and t.dtype == torch.float32 and t.device == x.device and t.is_contiguous()
                              and t.data_ptr() % 16 == 0) for t in tensors)
 
 
@@ -150,8 +164,12 @@ class TransformerEncoder(Module):
             return None
         if attn_mask is None or not attn_mask.lower_triangular or attn_mask.shape[0] != x.shape[1]:
             return None
+        if _observed() or type(x) not in (torch.Tensor, Parameter):
+            return None
         if torch.is_autocast_enabled() or torch.nn.modules.module._has_any_global_hook():
             return None
+        if not x.is_contiguous() or x.data_ptr() % 16:
+            x = x.clone(memory_format=torch.contiguous_format)  # (the rows are read 16 bytes at a time)
         lengths = None
         if length_mask is not None:
             lengths = getattr(length_mask, "lengths", None)

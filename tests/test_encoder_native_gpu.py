@@ -157,3 +157,47 @@ def test_encoder_native_forward(sizes, ragged, final):
         module.encoder_forward_hip = native
     # two fp32 evaluations: 1e-6 per layer of the largest value (norms keep rows near one)
     assert (got - want).abs().max() <= 4e-6 * layers * want.abs().max()
+
+
+def small_encoder(monkeypatch):
+    from fast_transformers_amd import attention, masking
+    from fast_transformers_amd.attention import encoder as module
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        model = attention.build_causal_linear_encoder(2, 2, 32, 32, 64).eval().requires_grad_(False)
+    calls, native = [], module.encoder_forward_hip
+    monkeypatch.setattr(module, "encoder_forward_hip", lambda *a: (calls.append(1), native(*a))[1])
+    return model, masking.TriangularCausalMask(40, device="cuda"), calls
+
+
+@pytest.mark.parametrize("form", ["offset", "permuted", "strided"])
+def test_encoder_takes_any_layout_of_its_input(monkeypatch, form):
+    model, mask, calls = small_encoder(monkeypatch)
+    rows = torch.rand(2, 40, 64, device="cuda")
+    if form == "offset":  # dense, and four bytes off a boundary of sixteen
+        x = torch.empty(2 * 40 * 64 + 1, device="cuda")[1:].view(2, 40, 64).copy_(rows)
+    elif form == "permuted":
+        x = rows.permute(2, 0, 1).contiguous().permute(1, 2, 0)
+    else:
+        x = torch.empty(2, 40, 65, device="cuda")[..., :64].copy_(rows)
+    assert torch.equal(model(x, attn_mask=mask), model(rows, attn_mask=mask)) and len(calls) == 2
+
+
+def test_encoder_keeps_its_modules_where_operations_are_observed(monkeypatch):
+    from torch.utils.flop_counter import FlopCounterMode
+    model, mask, calls = small_encoder(monkeypatch)
+    x = torch.rand(2, 40, 64, device="cuda")
+    with torch.device("cuda"):
+        want = model(x, attn_mask=mask)
+    assert calls == [1]
+    with FlopCounterMode(display=False) as flops:
+        got = [model(x, attn_mask=mask)]
+    assert flops.get_total_flops() > 0
+    with torch.autograd.forward_ad.dual_level():
+        got.append(model(x, attn_mask=mask))
+    inner = model.layers[1].linear2
+    inner.forward = lambda y: type(inner).forward(inner, y)
+    got.append(model(x, attn_mask=mask))
+    assert calls == [1]
+    # two fp32 evaluations, as above
+    assert all((g - want).abs().max() <= 8e-6 * want.abs().max() for g in got)
