@@ -639,7 +639,8 @@ bool odd_in_place(const ScanDesc &sc, int64_t chains, int64_t L) {
 
 // Scans for which odd_in_place holds, in one launch or one per shape, whichever is estimated
 // shorter (three scans of 99 chains are two rounds of workgroups, two and one are one round each).
-// *done = false (nothing launched): the kernel does not take one of them.
+// *done = false (nothing launched): the kernel does not take one of them, or the workspace has no
+// room for an exchange.
 int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, void *workspace,
               size_t workspace_bytes, hipStream_t stream, bool *done) {
     *done = false;
@@ -653,12 +654,19 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
         if (k == ngroups) size[ngroups++] = 0;
         group[k][size[k]++] = scans[i];
     }
+    auto room = [&](int d, int f, int k) {
+        const int64_t need = mfma_tp_workspace_bytes(N, H, L, d, f, k, false, true);
+        return need == 0 || plan_only() ||
+               (workspace && (int64_t)workspace_bytes >= need && (uintptr_t)workspace % 256 == 0);
+    };
     bool apart_ok = true;
     for (int k = 0; k < ngroups; k++) {
-        apart_ok = apart_ok && mfma_tp_takes(group[k], size[k], N, H, L, false, true);
+        apart_ok = apart_ok && mfma_tp_takes(group[k], size[k], N, H, L, false, true) &&
+                   room(group[k][0].a.width, group[k][0].v.width, size[k]);
         if (apart_ok) apart += mfma_tp_odd_chunks(group[k][0].a.width, group[k][0].v.width, N, H, size[k], L);
     }
-    const bool together_ok = ngroups > 1 && mfma_tp_takes(scans, n, N, H, L, false, true);
+    const bool together_ok = ngroups > 1 && mfma_tp_takes(scans, n, N, H, L, false, true) &&
+                             room(widest_d, widest_f, n);
     if (!apart_ok && !together_ok) return FTC_OK;
     auto run = [&](const ScanDesc *s, int k) {
         return mfma_scan(s, k, N, H, L, workspace, workspace_bytes, stream, nullptr, true, false, true);

@@ -43,3 +43,26 @@ def test_odd_widths_in_place(shape):
     for got, ref, ex in zip(outs, want, exact):
         # no further from float64 than four times the fp32 checker (or 2e-6 of the chain's largest)
         assert scale_error(got.cpu(), ex) <= max(4 * scale_error(ref, ex), 2e-6)
+
+
+def test_odd_widths_with_no_room_for_an_exchange():
+    """A long chain whose segments would exchange their sums, with a workspace that has room for
+    the generic kernel only: served as before, and not refused."""
+    import ctypes
+    from fast_transformers_amd import _native
+    N, H, L, E, M = 1, 3, 9000, 9, 9
+    lib = _native.load()
+    plan = _native.plan((N, H, L, E), (N, H, L, M))
+    assert "scan_tph_kernel (exchange)" in plan
+    Q, K, V, _ = oracle.make_inputs(N, H, L, E, M, seed=31)
+    out = torch.full((N, H, L, M), float("nan"), device="cuda")
+    q, k, v = (t.cuda() for t in (Q, K, V))
+    d = [_native.describe(t) for t in (q, k, v, out)]
+    room = int(plan.split("workspace ")[1].split()[0]) - 256
+    ws = torch.zeros(room, dtype=torch.uint8, device="cuda")
+    rc = lib.ftc_causal_dot_product(*(ctypes.byref(t) for t in d), ctypes.c_void_p(ws.data_ptr()),
+                                    ctypes.c_size_t(room), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, _native.last_error()
+    assert lib.ftc_last_kernel() == b"generic_scan_kernel"
+    exact = oracle.forward(Q.double(), K.double(), V.double())
+    assert scale_error(out.cpu(), exact) <= max(4 * scale_error(oracle.forward(Q, K, V), exact), 2e-6)
