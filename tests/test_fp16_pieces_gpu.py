@@ -5,7 +5,7 @@ seeded N(0,1) / elu+1 inputs of the other tests never reach: operands many order
 away from one, ceilings that rise all along a chain, states beyond 2^14 scaled units, all-zero
 chunks, and states handed in that dwarf (or are dwarfed by) the rows.
 
-Everything is compared with the CPU checker (the reference's own fp32 order) and anchored on
+Everything is compared with the CPU oracle (the reference's own fp32 order) and anchored on
 float64: per chain, or per row where rows differ in scale, the HIP result may be at most four
 times as far from float64 as the checker is (or 2e-6 of the scale)."""
 import pytest
@@ -137,7 +137,7 @@ def test_states_beyond_the_range_of_a_piece(cp, shape):
     segments that exchange their sums)."""
     N, H, L, E, M = shape
     Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=74, positive_uniform=True)
-    h = min(H, 3)   # (the CPU checker takes a second per long chain)
+    h = min(H, 3)   # (the CPU oracle takes a second per long chain)
     Qs, Ks, Vs, Gs = (t[:1, :h].contiguous() for t in (Q, K, V, G))
     refs, exact = _references(Qs, Ks, Vs, Gs)
     outs = _run(cp, Q, K, V, G)

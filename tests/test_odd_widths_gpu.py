@@ -1,5 +1,5 @@
 """fp32 rows of odd widths (and rows that are not 16-byte aligned) read and written where they lie
-by the fp16-piece kernel, against the CPU checker anchored on float64."""
+by the fp16-piece kernel, against the CPU oracle anchored on float64."""
 import pytest
 import torch
 
@@ -41,7 +41,7 @@ def test_odd_widths_in_place(shape):
     exact = (oracle.forward(Q.double(), K.double(), V.double()),) + \
         tuple(oracle.backward(Q.double(), K.double(), V.double(), G.double()))
     for got, ref, ex in zip(outs, want, exact):
-        # no further from float64 than four times the fp32 checker (or 2e-6 of the chain's largest)
+        # no further from float64 than four times the fp32 oracle (or 2e-6 of the chain's largest)
         assert scale_error(got.cpu(), ex) <= max(4 * scale_error(ref, ex), 2e-6)
 
 

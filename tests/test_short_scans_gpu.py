@@ -1,5 +1,5 @@
 """Chains of a few positions with a state handed in and out (ftc_short.hip), against the CPU
-checker in float64."""
+oracle in float64."""
 import pytest
 import torch
 

@@ -1,7 +1,7 @@
 """States of 65 to 128 rows on two fp16 pieces (csrc/ftc_tph_wide_kernel.h): chains of 32 chunks or
 more, walked whole, cut, or with an exchange; widths that do not fill either block; rows whose
 scale changes along the chain; a state handed in and out.  Gate: no further from float64 than
-four times the fp32 checker, or 2e-6 of the chain's largest (the gate of the narrower states)."""
+four times the fp32 oracle, or 2e-6 of the chain's largest (the gate of the narrower states)."""
 import pytest
 import torch
 
