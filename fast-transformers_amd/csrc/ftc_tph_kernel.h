@@ -434,7 +434,8 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         // the largest magnitudes of the rows of a position against the ceilings (rows that
         // were not asked for read as zeros); k: that position's slot
         // (NORM: keys at or beyond this row count as zero; phi(0) = 1, so do the rows and columns
-        // that do not exist)
+        // that do not exist.  Their values are cleared as well: a product with zero would drop them,
+        // but not before they had set the scale of the rows that count.)
         int key_rows = rows;
         if (NORM && p.key_len) key_rows = (int)max((int64_t)0, min((int64_t)rows, p.key_len[n]));
         auto features = [&](Raw &r, int pos) {
@@ -447,8 +448,9 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
                 r.b = feature_quad(r.b);
                 // (a scalar test: most chunks lie wholly below the limit)
                 if (KS == 1 || row0 < 0 || row0 + kChunk > key_rows) {
-                    const bool in = ab_in && (uint32_t)(row0 + prow) < (uint32_t)key_rows;
-                    if (!in) r.b = u32x4{0, 0, 0, 0};
+                    const bool counts = (uint32_t)(row0 + prow) < (uint32_t)key_rows;
+                    if (!(ab_in && counts)) r.b = u32x4{0, 0, 0, 0};
+                    if (!counts) r.v = u32x4{0, 0, 0, 0};
                 }
             }
         };

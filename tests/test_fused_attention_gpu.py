@@ -195,6 +195,28 @@ def test_chain_parallel_form(lib, shape):
     gate(out.cpu(), q, k, v, lengths, 1e-6)
 
 
+# whole, cut and exchanged chains (the exchange's first pass walks the segments in which the keys end)
+MASKED_SHAPES = [(3, 97, 8, 64, 64, [97, 64, 1]), (2, 1000, 16, 64, 64, [1000, 417]), (3, 520, 8, 32, 64, [520, 100, 40]),
+                 (1, 9000, 16, 64, 64, [4010])]
+
+
+@pytest.mark.parametrize("padding", [1e8, float("inf")])
+@pytest.mark.parametrize("shape", MASKED_SHAPES, ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s[:5])
+def test_masked_rows_do_not_set_a_scale(lib, shape, padding):
+    """Keys and values at or beyond the length leave every row as it is, bit for bit."""
+    N, L, H, E, M, lens = shape
+    q, k, v = inputs(N, L, H, E, M, seed=170 + L)
+    lengths = torch.tensor(lens)
+    want = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
+    assert lib.ftc_last_kernel().startswith(b"scan_tph_kernel<NORM>"), lib.ftc_last_kernel()
+    for n, length in enumerate(lens):
+        k[n, length:], v[n, length:] = 60.0, padding
+    got = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
+    assert torch.equal(got, want)
+    v[v.isinf()] = 0
+    gate(got.cpu(), q, k, v, lengths, 1e-6)
+
+
 def _count_backward_calls():
     """Context that counts the calls of the fused backward (autograd runs it on a thread of its
     own, where ftc_last_kernel() of this thread does not see it)."""
