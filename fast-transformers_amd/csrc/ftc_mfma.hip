@@ -471,24 +471,10 @@ Combo combo_of(const ScanDesc &sd) {
     return kNone;
 }
 
-// Chain-parallel scans of states of up to 64 rows run on the fp16 matrix path (ftc_tph_kernel.h:
-// two scaled fp16 pieces per value), rows of any type and width.
+// chain-parallel scans of states of up to 64 rows run on the fp16 matrix path
+// (ftc_tph_kernel.h: two scaled fp16 pieces per value), wider ones on three bf16 pieces
 bool tph_takes_rows(int64_t D) {
-    return D <= 64 && tuning().tph != 0;  // (FTC_TPH=0, three bf16 pieces: tuning aid)
-}
-// fp32 states of 65 to 128 rows: the same arithmetic in ftc_tph_wide_kernel.h or three bf16 pieces
-// in ftc_tp_kernel.h, on the same plans and under the same name ("scan_tp_kernel").  The line is
-// where the two-piece form is no further from float64: a walk's fp32 sums round half as often
-// there, the cut itself is coarser, so it loses on short walks.  2-norm errors, 1e-7, two / three
-// pieces, 128 x 128, positive a and b, forward and backward (dQ): 32 chains, L=64 1.27 / 1.13 and
-// 1.71 / 1.49; L=256 1.26 / 1.16 and 2.09 / 2.24; L=512 1.27 / 1.21 and 2.54 / 2.98; 128 x 64, 128
-// chains, L=1000 1.30 / 1.31 and 3.10 / 3.96; with an exchange, segments of 4 chunks, L=2048 1.28 /
-// 1.23 and 2.84 / 3.47; of 8 chunks 1.31 / 1.29 and 4.36 / 5.77; of 16 chunks (100 x 100) 1.36 / 1.56 and
-// 5.95 / 8.22; whole chains, L=4096 1.70 / 2.40 and 5.98 / 8.23.  What the line leaves to three
-// pieces is at most a tenth slower for it (32 chains, L=512: 28 / 26 us).
-bool tph_wide_takes(int64_t D, int64_t L, int seg_chunks) {
-    return D > 64 && D <= 128 && (L + kChunk - 1) / kChunk >= 32 && (seg_chunks == 0 || seg_chunks >= 8) &&
-           tuning().tph != 0;
+    return D <= 64 && tuning().tph != 0;  // (FTC_TPH=0: tuning aid)
 }
 
 // rows must not overlap (the descriptor's end marks the first row outside the segment) and
@@ -821,8 +807,6 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
             launch_scan_tph_norm(workspace, args, stream);
         else if (half_pieces)
             launch_scan_tph(workspace, args, mixed, odd, stream);
-        else if (tph_wide_takes(D, L, tpx_seg_chunks))
-            launch_scan_tph_wide(workspace, args, stream);
         else
             launch_scan_tp(workspace, args, stream);
     } else if (wg) {

@@ -1,7 +1,8 @@
-"""States of 65 to 128 rows on two fp16 pieces (csrc/ftc_tph_wide_kernel.h): chains of 32 chunks or
-more, walked whole, cut, or with an exchange; widths that do not fill either block; rows whose
-scale changes along the chain; a state handed in and out.  Gate: no further from float64 than
-four times the fp32 oracle, or 2e-6 of the chain's largest (the gate of the narrower states)."""
+"""States of 65 to 128 rows: chains of 32 chunks or more, walked whole, cut, or with an exchange;
+widths that do not fill either block; rows whose scale changes along the chain; a state handed in and
+out.  Gate: no further from float64 than four times the fp32 oracle, or 2e-6 of the chain's largest
+(the gate of the narrower states) -- and, where rows or columns of very different size stand side by
+side, the same for every row and every column on its own."""
 import pytest
 import torch
 
@@ -80,3 +81,34 @@ def test_state_in_and_out(cp, L):
     ref = oracle.forward(Q, K, V) + Q @ S
     _gate(out.cpu(), ref, exact)
     _gate(last.cpu(), S + K.transpose(-1, -2) @ V, S.double() + Kd.transpose(-1, -2) @ Vd)
+
+
+def _each(got, exact, dim):
+    """The largest 2-norm error of a row (dim 3) or column (dim 2) over its own 2-norm."""
+    got, exact = got.double(), exact.double()
+    return ((got - exact).norm(dim=dim) / exact.norm(dim=dim)).max().item()
+
+
+@pytest.mark.parametrize("shape", [(1, 8, 1061, 128, 128), (4, 32, 1024, 100, 68)], ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+@pytest.mark.parametrize("small", ["q_rows", "q_columns", "k_columns", "v_columns", "g_rows", "g_columns", "v_early_rows"])
+def test_small_rows_and_columns_beside_large_ones(cp, small, shape):
+    """Every row and column of a result is as close to float64, on its own scale, as the fp32
+    oracle's: no operand's large values set the precision of its small ones."""
+    Q, K, V, G = oracle.make_inputs(*shape, seed=11)
+    if small == "v_early_rows":  # rows 48 and on set no scale for the rows before them
+        V[:, :, 48:] *= 2.0 ** 20
+    else:
+        t = dict(q=Q, k=K, v=V, g=G)[small[0]]
+        t[..., 5::32, :] *= 2.0 ** -20 if small.endswith("rows") else 1
+        t[..., ::2] *= 2.0 ** -20 if small.endswith("columns") else 1
+    q, k, v, g = (t.cuda() for t in (Q, K, V, G))
+    outs = [torch.full_like(t, float("nan")) for t in (v, q, k, v)]
+    cp.causal_dot_product_hip(q, k, v, outs[0])
+    cp.causal_dot_backward_hip(q, k, v, g, *outs[1:])
+    cp.check_workspaces()
+    wide = [t.double() for t in (Q, K, V, G)]
+    refs = [oracle.forward(Q, K, V)] + list(oracle.backward(Q, K, V, G))
+    exact = [oracle.forward(*wide[:3])] + list(oracle.backward(*wide))
+    for got, ref, ex in zip(outs, refs, exact):
+        for dim in (2, 3):
+            assert _each(got.cpu(), ex, dim) <= max(4 * _each(ref, ex, dim), 2e-6)
