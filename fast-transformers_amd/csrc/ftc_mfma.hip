@@ -553,9 +553,6 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
     return seg_chunks > 0 ? tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D) : 0;
 }
 
-// (the exchange of the fused form: a second tile of state for its denominators)
-constexpr int64_t kFusedTpStateRows = 128;
-
 // the widest rows of a launch (they differ between scans only where `odd` allows it)
 void widest_rows(const ScanDesc *scans, int nscans, int *D, int *F) {
     *D = *F = 0;
@@ -625,34 +622,8 @@ bool fused_attention_supported(const ScanDesc &sd, int64_t L) {
            scan_wg_norm_covers(sd.a.width, sd.v.width) && mfma_scan_supported(sd, L);
 }
 
-// The fused attention launch on the chain-parallel kernel: its plan is that of a single 64 x 64
-// scan whatever the widths (a chunk costs the same).  Returns false: the workgroup form, whose
-// units split L and which carries two units of 32 value columns per workgroup.  Measured (us, this
-// way / the workgroup form), 64 x 64: 80 chains, L=1000 36.5 / 48.6, L=4096 109 / 141; 128 chains,
-// L=4096 148 / 200; 512 chains, L=1000 120 / 170; 24 chains, L=500 21.4 / 21.5; but 16 chains, L=500
-// 21.4 / 19.0, L=1500 34 / 29 (L=4096, an exchange: 41.3 / 41.6).  One width of 32: 80 chains, L=1000
-// 36 / 43 and 33.5 / 38; with an exchange 108 / 98 and 100 / 94 (L=4096); 32 x 64, 256 chains of
-// four chunks: 12 / 11.  32 x 32: 80 chains, L=1000 33 / 33, L=4096 99 / 64.
-bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, int *seg_chunks) {
-    *nseg = *seg_chunks = 0;
-    if (!tph_takes_rows(64) || tuning().wg > 0) return false;
-    const int64_t chunks = (L + kChunk - 1) / kChunk;
-    const bool full = D == 64 && F == 64;
-    tp_plan(64, 64, chains, 1, L, nseg, seg_chunks);
-    if (*nseg == 0 || tuning().wg == 0) return *nseg > 0;  // (FTC_WG=0: tuning aid)
-    const bool take = full ? chains >= 24 || (chains >= 16 && *seg_chunks > 0)
-                           : (D == 64 || F == 64) && *seg_chunks == 0 && chains >= 24 && (D == 64 || chunks >= 8);
-    if (!take) *nseg = *seg_chunks = 0;
-    return take;
-}
-
 int64_t fused_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F) {
-    int nseg, seg_chunks;
-    int64_t bytes = make_plan(N, H, L, D, F, 1, true, true).workspace_bytes;
-    const int64_t chains = std::max<int64_t>(1, N * H);
-    if (fused_tp_plan(D, F, chains, L, &nseg, &seg_chunks) && seg_chunks > 0)
-        bytes = std::max(bytes, tp_exchange_workspace_bytes(chains, nseg, kFusedTpStateRows));
-    return bytes;
+    return make_plan(N, H, L, D, F, 1, true, true).workspace_bytes;
 }
 
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
@@ -664,17 +635,10 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     const Combo combo = combo_of(scans[0]);
     if (fused && (nscans != 1 || !fused_attention_supported(scans[0], L)))
         return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for this shape or layout");
-    const int64_t chains = std::max<int64_t>(1, N * H);
-    int tpx_nseg = 0, tpx_seg_chunks = 0, tp_nseg = 0;
-    int64_t widest = 0;
-    for (int64_t s : {scans[0].a.stride_l, scans[0].b.stride_l, scans[0].v.stride_l, scans[0].out.stride_l})
-        widest = std::max(widest, s);
-    // (a whole chain is addressed through one 32-bit descriptor)
-    const bool fused_tp = fused && (L + 2 * kChunk) * std::max<int64_t>(widest, 64) * 4 < 0x7fffffffLL &&
-                          fused_tp_plan(D, F, chains, L, &tpx_nseg, &tpx_seg_chunks);
     const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd);
+    const int64_t chains = std::max<int64_t>(1, N * H);
     const int64_t fblocks = tp_shape ? tp_fblocks(F) : 1;
-    if (fused_tp && tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
+    int tpx_nseg = 0, tpx_seg_chunks = 0, tp_nseg = 0;
     if (tp_shape) {
         int any_bf16 = nscans == 1 && combo == kBBFB ? kMixedGradValues : 0;
         for (int i = 0; i < nscans; i++)
@@ -685,15 +649,14 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     const bool tp = tp_nseg > 0 || tpx_seg_chunks > 0;
     if (!tp && !mfma_scan_supported(scans[0], L))
         return fail(FTC_ERR_UNSUPPORTED, "no MFMA kernel takes a %d x %d state here", D, F);
-    const bool wg = !fused_tp && (fused || use_wg_kernel(D, F, nscans, L, combo == kFFFF));
+    const bool wg = fused || use_wg_kernel(D, F, nscans, L, combo == kFFFF);
     MfmaPlan pl = make_plan(N, H, L, D, F, nscans, wg, fused != nullptr);
     int32_t tp_start[kMaxTpSegments + 1] = {0};
     if (tpx_seg_chunks > 0) {  // one workgroup per chain segment, segment sums exchanged
         pl.nseg = tpx_nseg;
         pl.seg_len = tpx_seg_chunks * kChunk;
         pl.waves = chains * pl.nseg;
-        pl.workspace_bytes = tp_exchange_workspace_bytes(chains * nscans * fblocks, pl.nseg,
-                                                         fused_tp ? kFusedTpStateRows : D);
+        pl.workspace_bytes = tp_exchange_workspace_bytes(chains * nscans * fblocks, pl.nseg, D);
     } else if (tp) {  // one workgroup per chain segment, nothing to exchange
         pl.nseg = tp_segment_starts((L + kChunk - 1) / kChunk, tp_nseg, tp_start);
         pl.seg_len = (int)L;
@@ -746,7 +709,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     args.eps = fused ? fused->eps : 0.f;
     args.key_len = fused ? fused->key_lengths : nullptr;
 #ifdef FTC_TIMELINE
-    if (tp && !fused)  // tuning aid: where the chain-parallel kernel writes its time stamps
+    if (tp)  // tuning aid: where the chain-parallel kernel writes its time stamps
         if (const char *env = getenv("FTC_STAMP_PTR"))  // (a build for measurements only)
             args.key_len = (const int64_t *)(uintptr_t)strtoull(env, nullptr, 0);
 #endif
@@ -783,8 +746,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     // fp32 states of up to 64 rows: the kernel that feeds its fragments from LDS tiles
     bool dma = D <= 64 && combo == kFFFF;
     if (tuning().dma >= 0) dma = dma && tuning().dma != 0;  // tuning aid
-    note_kernel(fused_tp ? (tpx_seg_chunks > 0 ? "scan_tph_kernel<NORM> (exchange)" : "scan_tph_kernel<NORM>")
-                : tp ? (half_pieces ? (tpx_seg_chunks > 0 ? "scan_tph_kernel (exchange)" : "scan_tph_kernel")
+    note_kernel(tp ? (half_pieces ? (tpx_seg_chunks > 0 ? "scan_tph_kernel (exchange)" : "scan_tph_kernel")
                                   : (tpx_seg_chunks > 0 ? "scan_tp_kernel (exchange)" : "scan_tp_kernel"))
                 : wg ? (fused ? "scan_wg_kernel<NORM>" : "scan_wg_kernel")
                 : dma ? "scan_dma_kernel" : "scan_mfma_kernel");
@@ -803,9 +765,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         return FTC_OK;
     }
     if (tp) {
-        if (fused)
-            launch_scan_tph_norm(workspace, args, stream);
-        else if (half_pieces)
+        if (half_pieces)
             launch_scan_tph(workspace, args, mixed, odd, stream);
         else
             launch_scan_tp(workspace, args, stream);

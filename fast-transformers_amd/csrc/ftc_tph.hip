@@ -10,11 +10,11 @@ void launch(void *ws, const ScanArgs &args, bool mixed, bool odd, hipStream_t st
     // (grid as for launch_scan_tp)
     const dim3 grid((unsigned)args.total_waves), block(768);
     if (mixed)
-        hipLaunchKernelGGL((scan_tph_kernel<KS, true, false, false>), grid, block, 0, stream, (uint32_t *)ws, args);
+        hipLaunchKernelGGL((scan_tph_kernel<KS, true, false>), grid, block, 0, stream, (uint32_t *)ws, args);
     else if (odd)
-        hipLaunchKernelGGL((scan_tph_kernel<KS, false, true, false>), grid, block, 0, stream, (uint32_t *)ws, args);
+        hipLaunchKernelGGL((scan_tph_kernel<KS, false, true>), grid, block, 0, stream, (uint32_t *)ws, args);
     else
-        hipLaunchKernelGGL((scan_tph_kernel<KS, false, false, false>), grid, block, 0, stream, (uint32_t *)ws, args);
+        hipLaunchKernelGGL((scan_tph_kernel<KS, false, false>), grid, block, 0, stream, (uint32_t *)ws, args);
 }
 }  // namespace
 

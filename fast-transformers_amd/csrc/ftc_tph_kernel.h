@@ -216,17 +216,6 @@ __device__ __forceinline__ void raise_slot(lds_u32_t *slots, int k, int pos, con
     }
 }
 
-// sum over the four groups of 16 lanes, in every lane: v_permlane16_swap exchanges the odd groups
-// of its first operand with the even groups of its second, v_permlane32_swap the halves
-__device__ __forceinline__ float sum_of_lane_groups(float x) {
-    const uint32_t b = __float_as_uint(x);
-    const auto p16 = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-    const float y = __uint_as_float(p16[0]) + __uint_as_float(p16[1]);
-    const uint32_t c = __float_as_uint(y);
-    const auto p32 = __builtin_amdgcn_permlane32_swap(c, c, false, false);
-    return __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
-}
-
 // four bf16 values in two words -> the same values as fp32 bit patterns
 __device__ __forceinline__ u32x4 widen_bf16_quad(const u32x4 r) {
     return u32x4{r.x << 16, r.x & 0xffff0000u, r.y << 16, r.y & 0xffff0000u};
@@ -241,20 +230,7 @@ __device__ __forceinline__ u32x4 widen_bf16_quad(const u32x4 r) {
 // look-ahead first touches them, and stores such a quad word by word.  Measured against dense
 // zero-padded copies of the operands and results (9 x 11 chains, L=1531, 25 x 33): forward 79 ->
 // 38 us, backward 169 -> 89; a chunk costs what one of 64 x 64 does.
-// NORM: causally masked linear attention in the same walk (fp32, E and M of 32 or 64):
-//
-//   out[c, l, :] = sum_{j <= l} (phi(a_l) . phi'(b_j)) v_j / (phi(a_l) . sum_{j <= l} phi'(b_j) + eps)
-//
-// with phi(x) = elu(x) + 1 and phi'(b_j) = phi(b_j) where j < key_len[n], else 0.  The producers
-// apply phi when the look-ahead first touches the rows and zero the keys at or beyond the key
-// length.  The denominator is what the consumers have at hand: the column sums of the masked
-// quadrants of Pt, and phi(a) times z = sum of phi'(b) over the chunks before.  z is a column of
-// the state whose "values" are ones; consumer w keeps the half of z that belongs to k-step
-// w / 2 (its first one: such consumers swap the two halves of the state's rows) and multiplies
-// it with the 16 positions of its own quadrant: seven matrix instructions, two cuts and a
-// reduction over four lanes per chunk.  The two contributions to a position's denominator meet
-// in LDS behind the chunk's barrier, and the rows are divided as they are stored.
-template <int KS, bool MIX, bool ODD, bool NORM>
+template <int KS, bool MIX, bool ODD>
 __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     constexpr int D = 64, F = 64;              // one block of state rows and of output columns
     constexpr int T = 512;                     // producer lanes (eight wavefronts)
@@ -277,8 +253,6 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     __shared__ __align__(16) char pieces_mem[3 * kBufBytes];
     __shared__ __align__(16) char pt_mem[3 * 2 * kTileP];
     __shared__ __align__(16) uint32_t slot_mem[16];
-    // NORM: the two contributions to the denominators of a chunk's positions
-    __shared__ __align__(16) float den_mem[NORM ? 3 : 1][kChunk][2];
     lds_char *const unit_pc = (lds_char *)pieces_mem;
     lds_char *const pt_pc = (lds_char *)pt_mem;
     lds_u32_t *const slots = (lds_u32_t *)slot_mem;
@@ -433,29 +407,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         };
         // the largest magnitudes of the rows of a position against the ceilings (rows that
         // were not asked for read as zeros); k: that position's slot
-        // (NORM: keys at or beyond this row count as zero; phi(0) = 1, so do the rows and columns
-        // that do not exist.  Their values are cleared as well: a product with zero would drop them,
-        // but not before they had set the scale of the rows that count.)
-        int key_rows = rows;
-        if (NORM && p.key_len) key_rows = (int)max((int64_t)0, min((int64_t)rows, p.key_len[n]));
-        auto features = [&](Raw &r, int pos) {
-            if constexpr (NORM) {
-                const int row0 = pos < nwalk ? chunk_row0(walk_chunk(pos)) : -2 * kChunk;
-                if (pos >= n1) {
-                    r.a = feature_quad(r.a);
-                    if (KS == 1 && !ab_in) r.a = u32x4{0, 0, 0, 0};
-                }
-                r.b = feature_quad(r.b);
-                // (a scalar test: most chunks lie wholly below the limit)
-                if (KS == 1 || row0 < 0 || row0 + kChunk > key_rows) {
-                    const bool counts = (uint32_t)(row0 + prow) < (uint32_t)key_rows;
-                    if (!(ab_in && counts)) r.b = u32x4{0, 0, 0, 0};
-                    if (!counts) r.v = u32x4{0, 0, 0, 0};
-                }
-            }
-        };
         auto look_ahead = [&](Raw &r, int k, int pos) {
-            features(r, pos);
             widen(r.a, a_bf), widen(r.b, b_bf), widen(r.v, v_bf);
             own_words(r.a, ab_own), own_words(r.b, ab_own), own_words(r.v, v_own);
             raise_slot(slots, k, pos, ce, max_abs4(r.a, 0.f), max_abs4(r.b, 0.f), max_abs4(r.v, 0.f), lane);
@@ -523,8 +475,6 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     char *o_seg = (char *)op.out + ((int64_t)n * op.o_sn + (int64_t)h * op.o_sh + F * fb) * o_es;
     const __amdgpu_buffer_rsrc_t o_rs =
         __builtin_amdgcn_make_buffer_rsrc((void *)o_seg, 0, (rows - 1) * o_slb + fw * o_es, kRsrcFlags);
-    // NORM: k-steps of the state's rows in this consumer's order, its own half of z first
-    const int ks0 = NORM && KS == 2 ? w >> 1 : 0;
     // Pt quadrant of this wavefront (see scan_tp_kernel)
     const int jh = w == 0 ? 0 : w == 1 ? 1 : ((w == 2) == REV ? 1 : 0);
     const int ih = w == 0 ? 0 : w == 1 ? 1 : 1 - jh;
@@ -533,11 +483,11 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     for (int ks = 0; ks < 2; ks++) {
 #pragma unroll
         for (int x = 0; x < 2; x++)
-            a_addr[x][ks] = TpSwizzle<RBA>::addr(16 * (x ^ ih) + ln, 2 * (32 * (ks ^ ks0) + 8 * g));
+            a_addr[x][ks] = TpSwizzle<RBA>::addr(16 * (x ^ ih) + ln, 2 * (32 * ks + 8 * g));
 #pragma unroll
         for (int u = 0; u < 2; u++)
             b_addr[ks][u] = kOffB + TpSwizzle<RBA>::addr(
-                                        16 * jh + ln, 2 * b_tile_column(32 * (ks ^ ks0) + 8 * g + 4 * u));
+                                        16 * jh + ln, 2 * b_tile_column(32 * ks + 8 * g + 4 * u));
     }
     int bt_addr[4][2], vt_addr[2];
 #pragma unroll
@@ -546,7 +496,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
 #pragma unroll
         for (int dt = 0; dt < 4; dt++)
             bt_addr[dt][u2] = kOffB + TpSwizzle<RBA>::addr(
-                row, 2 * b_tile_column(32 * ((dt / 2) ^ ks0) + 4 * (dt % 2) + 8 * (ln & 3)));
+                row, 2 * b_tile_column(32 * (dt / 2) + 4 * (dt % 2) + 8 * (ln & 3)));
         vt_addr[u2] = kOffV + TpSwizzle<RBV>::addr(row, 2 * (16 * w + 4 * (ln & 3)));
     }
     const int pt_waddr = TpSwizzle<64>::addr(16 * ih + ln, 2 * (16 * jh + 4 * g));
@@ -577,34 +527,6 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     constexpr int kPa[3] = {1, 0, 0}, kPb[3] = {0, 1, 0};  // piece products, smallest first
     auto state_row = [&](int dt, int r) -> int { return 32 * (dt / 2) + 8 * g + 4 * (dt % 2) + r; };
     const bool st_in = 16 * w + ln < fw;
-    // NORM: this consumer's half of z (tiles 0 and 1 in its order, every column the same), in units
-    // of 2^(Ez - 132)
-    const bool has_z = NORM && (KS == 2 || w < 2);
-    f32x4 Z[2] = {};
-    int Ez = (int)kExpOfZeros;
-    int sz = 0;             // z is cut as Z 2^-sz: |Z| <= 2^(14 + sz)
-    float z_scale = 1.f;
-    const Frag ones = {{0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u}};
-    auto rescale_z = [&](int to) {
-        if (NORM && Ez != to) {
-            const int e = Ez - to;
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) Z[t][r] = __builtin_amdgcn_ldexpf(Z[t][r], e);
-            sz = max(0, sz + e);
-            z_scale = pow2_field(127 - sz);
-            Ez = to;
-        }
-    };
-    // (every third chunk, like s for S: a chunk adds at most 2^9 to an element)
-    auto grow_sz = [&]() {
-        if (!NORM) return;
-        const float m = fmaxf(fmaxf(fmaxf(fabsf(Z[0][0]), fabsf(Z[0][1])), fmaxf(fabsf(Z[0][2]), fabsf(Z[0][3]))),
-                              fmaxf(fmaxf(fabsf(Z[1][0]), fabsf(Z[1][1])), fmaxf(fabsf(Z[1][2]), fabsf(Z[1][3]))));
-        while (sz < 100 && __builtin_amdgcn_ballot_w64(m > pow2_field(127 + 14 + sz)) != 0) sz++;
-        z_scale = pow2_field(127 - sz);
-    };
     auto scale_state = [&](int e) {  // S <- S 2^e
 #pragma unroll
         for (int dt = 0; dt < NT; dt++)
@@ -654,14 +576,12 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     wg_barrier();  // barrier 0: position 0 is cut
     read_slot(slots, B0, ce);
     Ucur = ce.state_exp();
-    Ez = ce.Eb();
-    if (!NORM && op.s0 && !exchange) add_caller_state();
+    if (op.s0 && !exchange) add_caller_state();
     if (n1 > 0) {
         // ---- the first n1 positions of the walk: state update only ----
         // The loop is skewed by one position: while the matrix instructions of position k - 1
         // run, the fragments of position k arrive in the other set of registers.
         int U_prev = Ucur;                 // units of the fragments about to be multiplied
-        int Eb_prev = Ez;
         Frag bt2[4][2] = {}, vf2[2] = {};  // (the first round multiplies zeros)
         for (int c = 0; c < n1; c += PF) {
 #pragma unroll
@@ -671,24 +591,20 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
                 if (U_prev != Ucur) {       // the ceilings rose: the state shrinks
                     scale_state(Ucur - U_prev);
                     Ucur = U_prev;
-                    rescale_z(Eb_prev);
                 }
 #pragma unroll
                 for (int i = 0; i < 12; i++) {
                     const bool rows_exist = (i % 4) / 2 < KS;
                     if (j % 2 == 0) {
                         if (rows_exist) S[i % 4] = mfma16h(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[i % 4]);
-                        if (NORM && i < 8 && i % 4 < 2) Z[i % 2] = mfma16h(bt2[i % 2][1 - i / 4], ones, Z[i % 2]);
                         if (i < 10) tr_frag_into(bt, vf, pc, i);
                     } else {
                         if (rows_exist) S[i % 4] = mfma16h(bt[i % 4][kPa[i / 4]], vf[kPb[i / 4]], S[i % 4]);
-                        if (NORM && i < 8 && i % 4 < 2) Z[i % 2] = mfma16h(bt[i % 2][1 - i / 4], ones, Z[i % 2]);
                         if (i < 10) tr_frag_into(bt2, vf2, pc, i);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 U_prev = ce.state_exp();
-                Eb_prev = ce.Eb();
                 buf = next_buf(buf);
                 wg_barrier();
 #ifdef FTC_TIMELINE
@@ -701,12 +617,10 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         if (U_prev != Ucur) {
             scale_state(Ucur - U_prev);
             Ucur = U_prev;
-            rescale_z(Eb_prev);
         }
 #pragma unroll
         for (int i = 0; i < 12; i++) {
             if ((i % 4) / 2 < KS) S[i % 4] = mfma16h(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[i % 4]);
-            if (NORM && i < 8 && i % 4 < 2) Z[i % 2] = mfma16h(bt2[i % 2][1 - i / 4], ones, Z[i % 2]);
             rm_frag(unit_pc + buf * kBufBytes, i);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -719,17 +633,10 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         // ---- the sum of this segment's rows goes out, the state before the segment comes in ----
         const uint32_t total_units = (uint32_t)p.total_waves;
         gfloat *const sums = (gfloat *)(hdr + kControlBytes / 4);
-        constexpr int FX = NORM ? 2 : 1;  // (z rides along in a second tile)
-        StateExchange<1, FX> xch(flags, sums, 4u * total_units,
+        StateExchange<1, 1> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);
-        f32x16 Sx[1][FX], X[1][FX];
-        if (NORM) {
-            Sx[0][FX - 1] = f32x16{};
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                Sx[0][FX - 1][i] = __builtin_amdgcn_ldexpf(Z[i / 4][i % 4], Ez - 132);
-        }
+        f32x16 Sx[1][1], X[1][1];
 #pragma unroll
         for (int dt = 0; dt < 4; dt++)
 #pragma unroll
@@ -745,13 +652,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         for (int dt = 0; dt < NT; dt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) S[dt][r] = __builtin_amdgcn_ldexpf(X[0][0][4 * dt + r], -Ucur);
-        if (NORM) {
-            Ez = ce.Eb();
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                Z[i / 4][i % 4] = __builtin_amdgcn_ldexpf(X[0][FX - 1][i], 132 - Ez);
-        }
-        if (!NORM && op.s0) add_caller_state();
+        if (op.s0) add_caller_state();
     }
     // ---- the walk proper ----
     // `ce` holds the ceilings of the chunk at hand, Ucur the units of S.  dU < 0: the
@@ -774,9 +675,6 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         const float m = lane_max_state();
         while (s < 100 && __builtin_amdgcn_ballot_w64(m > pow2_field(127 + 14 + s)) != 0) s++;
     }
-    rescale_z(ce.Eb());
-    grow_sz();
-    float r_den[2] = {0.f, 0.f};             // NORM: reciprocals of the denominators of O's rows
     float kappa = pow2_field(127 + dU - s);  // scale of the cut of S
     bool plain_cut = dU - s == 0;            // ... which is one as a rule: a cheaper cut
     int s_cut = s;                            // ... and the s that went into it
@@ -809,9 +707,8 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     int Xo = 0;
     uint32_t o_off = 0x80000000u;
     auto store_rows = [&](int x) {
-        float y0 = __builtin_amdgcn_ldexpf(O[x][0], Xo), y1 = __builtin_amdgcn_ldexpf(O[x][1], Xo),
-              y2 = __builtin_amdgcn_ldexpf(O[x][2], Xo), y3 = __builtin_amdgcn_ldexpf(O[x][3], Xo);
-        if (NORM) y0 *= r_den[x], y1 *= r_den[x], y2 *= r_den[x], y3 *= r_den[x];
+        const float y0 = __builtin_amdgcn_ldexpf(O[x][0], Xo), y1 = __builtin_amdgcn_ldexpf(O[x][1], Xo),
+                    y2 = __builtin_amdgcn_ldexpf(O[x][2], Xo), y3 = __builtin_amdgcn_ldexpf(O[x][3], Xo);
         const uint32_t at = o_in ? o_off + o_lane[x] : kNoRow;
         if (!MIX) {
             buffer_store_out(o_rs, at, y0, y1, y2, y3, (float *)nullptr);
@@ -840,12 +737,8 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         const lds_char *pn = unit_pc + BN * kBufBytes;
         lds_char *const ptc = pt_pc + B * (2 * kTileP);
         Frag pf[2][2];
-        Frag zf[2];  // NORM: z in pieces
-        f32x4 Az;
-        float P_sum = 0.f;
         f32x4 P;  // (cleared by the first matrix instruction of its sum)
         if (c == c0 + 4) FTC_STAMP(0);
-        rescale_z(ce.Eb());
         __builtin_amdgcn_sched_barrier(0);
         // phase 1: (1) the quadrant in turn with (2b) Ot_w = S_w^T a^T for rows 0 .. 31 of
         // the state; underneath: the rows of the chunk before go out, tiles 2, 3 of S_w are
@@ -874,7 +767,6 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
             while (s < 100 && __builtin_amdgcn_ballot_w64(mS > pow2_field(127 + 14 + s)) != 0) s++;
             mS = 0.f;
         }
-        if (NORM && B == 0) grow_sz();
         if (c == c0 + 4) FTC_STAMP(2);
         __builtin_amdgcn_sched_barrier(0);
         // phase 2: (2b) for rows 32 .. 63 in turn with (3) S_w += b^T v_w for tiles 0 and 1;
@@ -884,31 +776,16 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
             const int x = i % 2, m = i / 2;
             if (KS > 1) O[x] = mfma16h(sf[1][kPa[m]], af[x][1][kPb[m]], O[x]);
             S[i % 2] = mfma16h(bt[i % 2][kPa[m]], vf[kPb[m]], S[i % 2]);
-            if (NORM && i < 2) {
-                cut_quad_f16(Z[i][0], Z[i][1], Z[i][2], Z[i][3], z_scale, zf[0].w[2 * i], zf[0].w[2 * i + 1],
-                             zf[1].w[2 * i], zf[1].w[2 * i + 1]);
-            }
-            if (NORM && i >= 2) {
-                Z[i % 2] = mfma16h(bt[i % 2][2 - i / 2], ones, Z[i % 2]);
-                if (i < 5) Az = mfma16h(zf[kPa[i - 2]], af[0][0][kPb[i - 2]], i == 2 ? zero : Az);
-            }
             if (i == 1) {
                 uint32_t h0, l0, h1, l1;
 #pragma unroll
                 for (int r = 0; r < 4; r++) P[r] = keep[r] ? P[r] : 0.f;
-                // (NORM: the quadrant's column sums, over the rows of a lane, then of the lane groups)
-                if (NORM) P_sum = sum_of_lane_groups((P[0] + P[1]) + (P[2] + P[3]));
                 cut_quad_f16_unscaled(P[0], P[1], P[2], P[3], h0, h1, l0, l1);
                 const u32x2 wh = {h0, h1}, wl = {l0, l1};
                 *(lds_vec2 *)(ptc + pt_waddr) = wh;
                 *(lds_vec2 *)(ptc + kTileP + pt_waddr) = wl;
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr (NORM) {
-            const float az = has_z ? __builtin_amdgcn_ldexpf(Az[0], sz) : 0.f;
-            if (g == 0)
-                den_mem[B][16 * ih + ln][w >> 1] = __builtin_amdgcn_ldexpf(az + P_sum, (int)ce.Ea + ce.Eb() - 264);
         }
         if (c == c0 + 4) FTC_STAMP(4);
         wg_barrier();
@@ -923,18 +800,6 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         for (int x = 0; x < 2; x++)
 #pragma unroll
             for (int k = 0; k < 2; k++) pf[x][k] = lds_frag16(ptc + k * kTileP + pt_raddr[x]);
-        if constexpr (NORM) {
-#pragma unroll
-            for (int x = 0; x < 2; x++) {
-                const float *part = den_mem[B][16 * (x ^ ih) + ln];
-                const float den = (part[0] + part[1]) + p.eps;
-                float r = __builtin_amdgcn_rcpf(den);
-                r_den[x] = fmaf(fmaf(-den, r, 1.f), r, r);
-                const int row = chunk_row0(c) + 16 * (x ^ ih) + ln;
-                if (w == 0 && op.s_out && g == 0 && row < rows)
-                    op.s_out[(int64_t)n * op.so_sn + (int64_t)h * op.so_sh + row] = den;
-            }
-        }
         const int Xc = ce.out_exp();
         const u32x4 slot_next = *(const lds_vec4 *)(slots + 4 * BN);
         if (s_cut != 0) {  // (rare: the state has grown beyond 2^14 units)
@@ -989,7 +854,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
 #ifdef FTC_TIMELINE
     if (stamp_on) stamp_base[13] = __builtin_amdgcn_s_memtime();
 #endif
-    if (!NORM && op.s_out && seg == (int)nseg - 1) {
+    if (op.s_out && seg == (int)nseg - 1) {
         float *base =
             op.s_out + (int64_t)n * op.so_sn + (int64_t)h * op.so_sh + F * fb + 16 * w + ln;
 #pragma unroll

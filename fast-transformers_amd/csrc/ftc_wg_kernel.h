@@ -756,8 +756,6 @@ void launch_scan_tp(void *ws, const ScanArgs &args, hipStream_t stream);
 // the same on the fp16 matrix path (ftc_tph_kernel.h): states of up to 64 rows
 // `mixed`: some rows are bf16 (ScanOperands::pad of every scan says which)
 void launch_scan_tph(void *ws, const ScanArgs &args, bool mixed, bool odd, hipStream_t stream);
-// ... in its fused attention form (all rows fp32, 32 or 64 wide)
-void launch_scan_tph_norm(void *ws, const ScanArgs &args, hipStream_t stream);
 
 }  // namespace mfma
 }  // namespace ftc
