@@ -42,6 +42,14 @@ void check(int64_t rc, const char *what) {
         error(std::string(what) + " failed (status " + std::to_string(rc) + "): " + ftc_last_error());
 }
 
+// A call into the library without Python's lock: a launch may block (a full queue), and other
+// threads go on meanwhile.
+template <class F>
+auto native(F f) {
+    const py::gil_scoped_release unlocked;
+    return f();
+}
+
 int32_t dtype_code(const Tensor &t) {
     if (t.scalar_type() == at::kFloat) return FTC_F32;
     if (t.scalar_type() == at::kBFloat16) return FTC_BF16;
@@ -102,7 +110,7 @@ int64_t workspace_bytes(Query query, const char *name, int64_t N, int64_t H, int
     const SizeKey key{query, N, H, L, E, M, code};
     const auto it = g_sizes.find(key);
     if (it != g_sizes.end()) return it->second;
-    const int64_t bytes = query(N, H, L, E, M, code);
+    const int64_t bytes = native([&] { return query(N, H, L, E, M, code); });
     check(bytes, name);
     if (g_sizes.size() >= 4096) g_sizes.clear();
     g_sizes[key] = bytes;
@@ -156,8 +164,9 @@ void forward(const Tensor &queries, const Tensor &keys, const Tensor &values, co
     Call call(q, workspace_bytes(ftc_causal_dot_product_workspace_bytes,
                                  "ftc_causal_dot_product_workspace_bytes", q.size(0), q.size(1), q.size(2),
                                  q.size(3), v.size(3), dq.dtype));
-    check(ftc_causal_dot_product(&dq, &dk, &dv, &dout, call.ws, call.ws_bytes, call.stream),
-          "ftc_causal_dot_product");
+    const int rc = native(
+        [&] { return ftc_causal_dot_product(&dq, &dk, &dv, &dout, call.ws, call.ws_bytes, call.stream); });
+    check(rc, "ftc_causal_dot_product");
     call.done();
 }
 
@@ -184,9 +193,11 @@ std::tuple<Tensor, OptTensor> product_with_state(const Tensor &queries, const Te
     if (s1) d1 = describe(*s1);
     Call call(q, workspace_bytes(ftc_causal_dot_product_workspace_bytes,
                                  "ftc_causal_dot_product_workspace_bytes", N, H, L, E, M, dq.dtype));
-    check(ftc_causal_dot_product_state(&dq, &dk, &dv, s0.defined() ? &d0 : nullptr, &dout,
-                                       s1 ? &d1 : nullptr, call.ws, call.ws_bytes, call.stream),
-          "ftc_causal_dot_product_state");
+    const int rc = native([&] {
+        return ftc_causal_dot_product_state(&dq, &dk, &dv, s0.defined() ? &d0 : nullptr, &dout,
+                                            s1 ? &d1 : nullptr, call.ws, call.ws_bytes, call.stream);
+    });
+    check(rc, "ftc_causal_dot_product_state");
     call.done();
     return {out, s1};
 }
@@ -211,8 +222,11 @@ void backward(const Tensor &queries, const Tensor &keys, const Tensor &values, c
     Call call(q, workspace_bytes(ftc_causal_dot_backward_workspace_bytes,
                                  "ftc_causal_dot_backward_workspace_bytes", q.size(0), q.size(1),
                                  q.size(2), q.size(3), v.size(3), dq.dtype));
-    check(ftc_causal_dot_backward(&dq, &dk, &dv, &dg, gq.p, gk.p, gv.p, call.ws, call.ws_bytes, call.stream),
-          "ftc_causal_dot_backward");
+    const int rc = native([&] {
+        return ftc_causal_dot_backward(&dq, &dk, &dv, &dg, gq.p, gk.p, gv.p, call.ws, call.ws_bytes,
+                                       call.stream);
+    });
+    check(rc, "ftc_causal_dot_backward");
     call.done();
 }
 
@@ -237,10 +251,12 @@ void attention(const Tensor &queries, const Tensor &keys, const Tensor &values, 
     Call call(q, workspace_bytes(ftc_causal_linear_attention_workspace_bytes,
                                  "ftc_causal_linear_attention_workspace_bytes", q.size(0), q.size(1),
                                  q.size(2), q.size(3), v.size(3), dq.dtype));
-    check(ftc_causal_linear_attention_forward(&dq, &dk, &dv, lengths, (float)eps, &dout,
-                                              denominators ? &dden : nullptr, call.ws, call.ws_bytes,
-                                              call.stream),
-          "ftc_causal_linear_attention_forward");
+    const int rc = native([&] {
+        return ftc_causal_linear_attention_forward(&dq, &dk, &dv, lengths, (float)eps, &dout,
+                                                   denominators ? &dden : nullptr, call.ws, call.ws_bytes,
+                                                   call.stream);
+    });
+    check(rc, "ftc_causal_linear_attention_forward");
     call.done();
 }
 
@@ -258,9 +274,11 @@ void attention_backward(const Tensor &queries, const Tensor &keys, const Tensor 
     Call call(q, workspace_bytes(ftc_causal_linear_attention_backward_workspace_bytes,
                                  "ftc_causal_linear_attention_backward_workspace_bytes", q.size(0),
                                  q.size(1), q.size(2), q.size(3), v.size(3), dq.dtype));
-    check(ftc_causal_linear_attention_backward(&dq, &dk, &dv, lengths, &dout, &dden, &dg, gq.p, gk.p, gv.p,
-                                               call.ws, call.ws_bytes, call.stream),
-          "ftc_causal_linear_attention_backward");
+    const int rc = native([&] {
+        return ftc_causal_linear_attention_backward(&dq, &dk, &dv, lengths, &dout, &dden, &dg, gq.p, gk.p,
+                                                    gv.p, call.ws, call.ws_bytes, call.stream);
+    });
+    check(rc, "ftc_causal_linear_attention_backward");
     call.done();
 }
 
@@ -350,35 +368,37 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
                                    pieces ? x_scale.data_ptr<float>() : nullptr, stream),
               "ftc_layer_norm_split");
     };
-    check(ftc_split_rows(x.const_data_ptr<float>(), T, d, x_pieces.data_ptr(), x_scale.data_ptr<float>(), stream),
-          "ftc_split_rows");
-    for (size_t i = 0; i < layers.size(); i++) {
-        const Layer &l = layers[i];
-        std::vector<ftc_weight> list;
-        const Pieces in({&l.query, &l.key, &l.value}, list), proj({&l.out}, list), first({&l.first}, list),
-            second({&l.second}, list);
-        check(ftc_split_weights(list.data(), (int32_t)list.size(), stream), "ftc_split_weights");
-        linear(x_pieces, x_scale, in, nullptr, qkv);
-        check(ftc_causal_linear_attention_forward(&q, &k, &v, lengths, (float)l.eps, &o, nullptr, call.ws,
-                                                  call.ws_bytes, stream),
-              "ftc_causal_linear_attention_forward");
-        check(ftc_split_rows(rows.const_data_ptr<float>(), T, H * M, r_pieces.data_ptr(), r_scale.data_ptr<float>(),
-                             stream),
+    native([&] {
+        check(ftc_split_rows(x.const_data_ptr<float>(), T, d, x_pieces.data_ptr(), x_scale.data_ptr<float>(), stream),
               "ftc_split_rows");
-        linear(r_pieces, r_scale, proj, now.const_data_ptr<float>(), y);
-        norm(y, l.norm1, x1, true);
-        check(ftc_linear_split(x_pieces.data_ptr(), x_scale.const_data_ptr<float>(), T, first.pieces.data_ptr(),
-                               first.scale.const_data_ptr<float>(), first.bias.const_data_ptr<float>(),
-                               first.norm.const_data_ptr<float>(), first.rows, first.cols, nullptr, nullptr,
-                               h_pieces.data_ptr(), h_scale.data_ptr<float>(), stream),
-              "ftc_linear_split");
-        linear(h_pieces, h_scale, second, x1.const_data_ptr<float>(), y);
-        const bool last = i + 1 == layers.size();
-        if (last && !final_norm) next = out;
-        norm(y, l.norm2, next, !last);
-        now = next;
-    }
-    if (final_norm) norm(now, *final_norm, out, false);
+        for (size_t i = 0; i < layers.size(); i++) {
+            const Layer &l = layers[i];
+            std::vector<ftc_weight> list;
+            const Pieces in({&l.query, &l.key, &l.value}, list), proj({&l.out}, list), first({&l.first}, list),
+                second({&l.second}, list);
+            check(ftc_split_weights(list.data(), (int32_t)list.size(), stream), "ftc_split_weights");
+            linear(x_pieces, x_scale, in, nullptr, qkv);
+            check(ftc_causal_linear_attention_forward(&q, &k, &v, lengths, (float)l.eps, &o, nullptr, call.ws,
+                                                      call.ws_bytes, stream),
+                  "ftc_causal_linear_attention_forward");
+            check(ftc_split_rows(rows.const_data_ptr<float>(), T, H * M, r_pieces.data_ptr(), r_scale.data_ptr<float>(),
+                                 stream),
+                  "ftc_split_rows");
+            linear(r_pieces, r_scale, proj, now.const_data_ptr<float>(), y);
+            norm(y, l.norm1, x1, true);
+            check(ftc_linear_split(x_pieces.data_ptr(), x_scale.const_data_ptr<float>(), T, first.pieces.data_ptr(),
+                                   first.scale.const_data_ptr<float>(), first.bias.const_data_ptr<float>(),
+                                   first.norm.const_data_ptr<float>(), first.rows, first.cols, nullptr, nullptr,
+                                   h_pieces.data_ptr(), h_scale.data_ptr<float>(), stream),
+                  "ftc_linear_split");
+            linear(h_pieces, h_scale, second, x1.const_data_ptr<float>(), y);
+            const bool last = i + 1 == layers.size();
+            if (last && !final_norm) next = out;
+            norm(y, l.norm2, next, !last);
+            now = next;
+        }
+        if (final_norm) norm(now, *final_norm, out, false);
+    });
     call.done();
     return out;
 }

@@ -803,6 +803,41 @@ def test_dirty_control_block_is_reported_and_healed(cp, monkeypatch):
     cp.check_workspaces()
 
 
+def test_a_call_lets_other_threads_run(cp):
+    """The launch is made without Python's lock: a thread that waits for the lock gets it while this
+    one does nothing but calls (with a switch interval far beyond the test, only a released lock
+    lets it in)."""
+    import sys
+    import threading
+    import time
+    q, k, v = (torch.rand(1, 1, 64, 64, device="cuda") for _ in range(3))
+    out = torch.empty_like(v)
+    ran = threading.Event()
+
+    def other():
+        time.sleep(0.001)
+        ran.set()
+
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(100)
+    try:
+        time.sleep(0.02)
+        cp.causal_dot_product_hip(q, k, v, out)   # (looks after the error word; not again for 10 ms)
+        end = time.perf_counter() + 0.008
+        thread = threading.Thread(target=other)
+        thread.start()
+        while time.perf_counter() < end - 0.005:  # the other one has slept and wants the lock
+            pass
+        assert not ran.is_set()
+        while time.perf_counter() < end and not ran.is_set():
+            cp.causal_dot_product_hip(q, k, v, out)
+        entered = ran.is_set()
+    finally:
+        sys.setswitchinterval(interval)
+    thread.join()
+    assert entered
+
+
 TP_SHAPES = [
     # N, H, L, E, M: enough chains for one workgroup per chain (and scan), or few enough that
     # a chain is cut into segments whose workgroups rebuild their starting state
