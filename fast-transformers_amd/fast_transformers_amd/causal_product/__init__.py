@@ -29,8 +29,8 @@ from .. import _native
 # is asked for (``check_workspaces()``; after every call when FTC_CHECK=1 is set in the
 # environment) or cheap (before a cached workspace is replaced by a larger one).  Between
 # those it watches without waiting: at most every ten milliseconds a call leaves
-# an asynchronous copy of the error word to pinned host memory behind it on its stream, and a
-# later call that finds the copy finished (an event query) reads the word and raises.
+# an asynchronous copy of the error word to pinned host memory behind it on its stream, and the
+# next call after the copy has arrived finds the word there and raises.
 _workspaces = {}
 _probes = {}              # workspace key -> [pinned word, event or None]
 
@@ -43,7 +43,7 @@ def _host():
     global _host_module
     if _host_module is None:
         host = _native.host()
-        host.setup(_workspaces, _make_workspace, _watch, _probe, _check_if_possible)
+        host.setup(_workspaces, _probes, _make_workspace, _watch, _probe, _check_if_possible)
         _host_module = host
     return _host_module
 

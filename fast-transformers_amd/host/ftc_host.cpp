@@ -8,7 +8,8 @@
 //
 // The workspaces stay Python's (causal_product.__init__: one per device and stream, in a dict that
 // check_workspaces() walks); they are found here through that dict, and Python is called when
-// one has to be made or grown and, every ten milliseconds at most, to look after its error word.
+// one has to be made or grown, when an error word has come back and, every ten milliseconds at
+// most, to send for the next one.
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -90,14 +91,23 @@ const Tensor &check_out(const Tensor &t, const char *name) {
 // ---- workspaces ----
 // (kept for the life of the process: never released, Python may be gone by then)
 struct PythonSide {
-    py::dict workspaces;
+    py::dict workspaces, probes;
     py::function make_workspace, watch, probe, check_all;
 };
 PythonSide *g_python = nullptr;
 
-void setup(py::dict workspaces, py::function make_workspace, py::function watch, py::function probe,
-           py::function check_all) {
-    g_python = new PythonSide{workspaces, make_workspace, watch, probe, check_all};
+void setup(py::dict workspaces, py::dict probes, py::function make_workspace, py::function watch,
+           py::function probe, py::function check_all) {
+    g_python = new PythonSide{workspaces, probes, make_workspace, watch, probe, check_all};
+}
+
+// Whether the last probe of a workspace has brought back an error word.  (Pinned memory that the
+// copy behind an earlier call fills; zero until it arrives.)
+bool failed(const py::object &key) {
+    PyObject *probe = PyDict_GetItem(g_python->probes.ptr(), key.ptr());  // (borrowed)
+    if (!probe) return false;
+    const Tensor &word = THPVariable_Unpack(PyList_GetItem(probe, 0));
+    return *(const volatile int32_t *)word.const_data_ptr() != 0;
 }
 
 // bytes asked for by (query, sizes, dtype): sizes repeat call after call (under Python's lock)
@@ -135,6 +145,7 @@ struct Call {
         if (found) workspace = THPVariable_Unpack(found);
         if (!found || workspace.numel() < bytes)
             workspace = g_python->make_workspace(bytes, key).cast<Tensor>();
+        if (failed(key)) g_python->check_all();
         ws = workspace.data_ptr(), ws_bytes = (size_t)workspace.numel();
         using clock = std::chrono::steady_clock;
         static std::map<std::pair<int, intptr_t>, clock::time_point> last;  // (under Python's lock)

@@ -838,6 +838,30 @@ def test_a_call_lets_other_threads_run(cp):
     assert entered
 
 
+def test_the_next_call_after_a_probe_reads_it(cp, monkeypatch):
+    """An error word that a probe has brought back is reported by the next call, however soon it
+    comes, and not only by one ten milliseconds later."""
+    import time
+    monkeypatch.delenv("FTC_CHECK", raising=False)
+    q, k, v = (torch.rand(2, 2, 1500, 64, device="cuda") for _ in range(3))
+    out = torch.empty_like(v)
+    cp.causal_dot_product_hip(q, k, v, out)
+    torch.cuda.synchronize()
+    cp.check_workspaces()
+    ws = cp._workspaces[(q.device.index, torch.cuda.current_stream().cuda_stream)]
+    time.sleep(0.02)
+    cp.causal_dot_product_hip(q, k, v, out)      # reads the last probe and leaves another
+    torch.cuda.synchronize()
+    time.sleep(0.02)
+    ws[8:12].view(torch.int32).fill_(1)          # (the kernels write the word and do not read it)
+    cp.causal_dot_product_hip(q, k, v, out)      # leaves a probe behind it
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError, match="cut short"):
+        cp.causal_dot_product_hip(q, k, v, out)
+    cp.causal_dot_product_hip(q, k, v, out)
+    cp.check_workspaces()
+
+
 TP_SHAPES = [
     # N, H, L, E, M: enough chains for one workgroup per chain (and scan), or few enough that
     # a chain is cut into segments whose workgroups rebuild their starting state
