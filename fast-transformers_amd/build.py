@@ -65,6 +65,37 @@ def host_command():
             "-Wl,-rpath,$ORIGIN"]
 
 
+def stamp(out):
+    """Where the recipe that a library was built by is kept."""
+    return os.path.join(OBJ_DIR, os.path.basename(out) + ".recipe")
+
+
+def recipe(cmd):
+    """What a library depends on beside its inputs: the command, and for the Python binding the
+    versions of torch and Python whose headers it was compiled against."""
+    import torch
+    versions = [torch.__version__, sys.version] if HOST_OUT in cmd else []
+    return "\n".join(list(cmd) + versions)
+
+
+def stale(out, cmd, inputs):
+    """Whether a library is missing, older than an input or built by another recipe."""
+    if not (os.path.exists(out) and os.path.exists(stamp(out))):
+        return True
+    with open(stamp(out)) as f:
+        if f.read() != recipe(cmd):
+            return True
+    return os.path.getmtime(out) < max(os.path.getmtime(i) for i in inputs)
+
+
+def link(out, cmd, verbose):
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    with open(stamp(out), "w") as f:
+        f.write(recipe(cmd))
+
+
 def build(force=False, verbose=False, extra_flags=()):
     hipcc = find_hipcc()
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -86,18 +117,12 @@ def build(force=False, verbose=False, extra_flags=()):
     for src, p in procs:
         if p.wait() != 0:
             raise RuntimeError("hipcc failed on %s" % src)
-    if procs or force or not os.path.exists(OUT) or \
-            os.path.getmtime(OUT) < max(os.path.getmtime(o) for o in objs):
-        cmd = [hipcc, "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-rdc", "-o", OUT] + objs
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        subprocess.check_call(cmd)
-    if force or not os.path.exists(HOST_OUT) or os.path.getmtime(HOST_OUT) < max(
-            os.path.getmtime(f) for f in [HOST_SRC] + glob.glob(os.path.join(INCLUDE, "*.h"))):
-        cmd = host_command()
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        subprocess.check_call(cmd)
+    cmd = [hipcc, "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-rdc", "-o", OUT] + objs
+    if procs or force or stale(OUT, cmd, objs):
+        link(OUT, cmd, verbose)
+    cmd = host_command()
+    if force or stale(HOST_OUT, cmd, [HOST_SRC] + glob.glob(os.path.join(INCLUDE, "*.h"))):
+        link(HOST_OUT, cmd, verbose)
     return OUT
 
 
