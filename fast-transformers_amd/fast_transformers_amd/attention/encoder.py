@@ -74,9 +74,16 @@ class TransformerEncoderLayer(Module):
         return self.norm2(x + y)
 
 
+# what the native forward restates, as it was when this module was imported
+_FORWARDS = {cls: cls.forward for cls in (Linear, LayerNorm, Dropout, AttentionLayer, TransformerEncoderLayer,
+                                          CausalLinearAttention, ActivationFunctionFeatureMap)}
+
+
 def _watched(module):
-    # (an instance's own ``forward`` stands in for its class's, as offloading wrappers put it there)
-    return module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+    # (another ``forward`` stands in for the class's: an instance's own, as offloading wrappers put it
+    # there, or one that was put on the class)
+    return (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+            or type(module).forward is not _FORWARDS[type(module)])
 
 
 def _observed():

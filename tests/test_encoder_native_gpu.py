@@ -201,3 +201,14 @@ def test_encoder_keeps_its_modules_where_operations_are_observed(monkeypatch):
     assert calls == [1]
     # two fp32 evaluations, as above
     assert all((g - want).abs().max() <= 8e-6 * want.abs().max() for g in got)
+
+
+@pytest.mark.parametrize("cls", ["Linear", "LayerNorm", "Dropout"])
+def test_encoder_keeps_its_modules_where_a_class_has_another_forward(monkeypatch, cls):
+    model, mask, calls = small_encoder(monkeypatch)
+    x = torch.rand(2, 40, 64, device="cuda")
+    cls, seen = getattr(torch.nn, cls), []
+    plain = cls.forward
+    monkeypatch.setattr(cls, "forward", lambda self, y: (seen.append(1), plain(self, y))[1])
+    model(x, attn_mask=mask)
+    assert seen and not calls
