@@ -169,7 +169,10 @@ class TransformerEncoder(Module):
         differentiated or watched and every part is the plain one; None otherwise."""
         if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.numel() > 0) or len(self.layers) == 0:
             return None
-        if attn_mask is None or not attn_mask.lower_triangular or attn_mask.shape[0] != x.shape[1]:
+        if attn_mask is None or not attn_mask.lower_triangular:
+            return None
+        shape = getattr(attn_mask, "shape", None)  # (a mask need not have one)
+        if shape is None or shape[0] != x.shape[1]:
             return None
         if _observed() or type(x) not in (torch.Tensor, Parameter):
             return None

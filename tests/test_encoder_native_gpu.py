@@ -212,3 +212,12 @@ def test_encoder_keeps_its_modules_where_a_class_has_another_forward(monkeypatch
     monkeypatch.setattr(cls, "forward", lambda self, y: (seen.append(1), plain(self, y))[1])
     model(x, attn_mask=mask)
     assert seen and not calls
+
+
+def test_encoder_takes_a_mask_that_only_says_it_is_causal(monkeypatch):
+    from types import SimpleNamespace
+    model, mask, calls = small_encoder(monkeypatch)
+    x = torch.rand(2, 40, 64, device="cuda")
+    got = model(x, attn_mask=SimpleNamespace(lower_triangular=True))
+    want = model(x, attn_mask=mask)
+    assert (got - want).abs().max() <= 8e-6 * want.abs().max()  # (two fp32 evaluations, as above)
