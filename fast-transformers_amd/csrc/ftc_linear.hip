@@ -35,6 +35,9 @@ using namespace mfma;
 
 constexpr int kStep = 32;                // columns per k-step
 constexpr int kRowBytes = 4 * kStep;     // a row's bytes of a k-step: hi, lo
+// Columns or features of a row (128 rows of 2^20 floats stay within a descriptor's 2^31 bytes) and
+// rows of a launch of a wavefront each (HIP takes fewer than 2^32 lanes).
+constexpr int64_t kMostColumns = 1 << 20, kMostRows = 1 << 26;
 
 // the power of two that brings a largest magnitude to 2^14 .. 2^15, and its reciprocal
 __device__ __forceinline__ void scale_of(float largest, float &s, float &inverse) {
@@ -434,6 +437,7 @@ int launch_rows(const float *x, const float *gamma, const float *beta, float eps
     if (!aligned(x) || !aligned(gamma) || !aligned(beta) || !aligned(out) || !aligned(pieces))
         return fail(FTC_ERR_INVALID, "rows must be 16-byte aligned");
     if (rows <= 0) return FTC_OK;
+    if (rows >= kMostRows) return fail(FTC_ERR_UNSUPPORTED, "%lld rows", (long long)rows);
     const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
 #define FTC_ROWS(Q)                                                                                   \
     hipLaunchKernelGGL((rows_kernel<Q, NORM>), grid, block, 0, stream, x, gamma, beta, eps, rows, (int)cols, out, \
@@ -463,7 +467,8 @@ int ftc_split_weights(const ftc_weight *weights, int32_t count, void *stream) {
         const ftc_weight &w = weights[i];
         if (!w.w || !w.pieces || !w.scale || !w.bias_out || !w.norm || !aligned(w.w) || !aligned(w.pieces))
             return fail(FTC_ERR_INVALID, "weight %d: null or misaligned pointer", i);
-        if (w.cols % kStep != 0 || w.cols <= 0 || w.rows <= 0 || w.rows % 4 != 0)
+        if (w.cols % kStep != 0 || w.cols <= 0 || w.cols > kMostColumns || w.rows <= 0 || w.rows > kMostColumns ||
+            w.rows % 4 != 0)
             return fail(FTC_ERR_UNSUPPORTED, "weight %d: %lld x %lld", i, (long long)w.rows, (long long)w.cols);
         list.w[i] = w.w, list.bias[i] = w.bias, list.cols[i] = (int32_t)w.cols;
         list.pieces[i] = (char *)w.pieces, list.scale[i] = w.scale;
@@ -496,8 +501,8 @@ int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const 
     if (!aligned(x) || !aligned(w) || !aligned(w_scale) || !aligned(bias) || !aligned(residual) || !aligned(out) ||
         !aligned(relu_pieces))
         return fail(FTC_ERR_INVALID, "rows must be 16-byte aligned");
-    if (k % kStep != 0 || k < 2 * kStep || k > (1 << 20) || features % 4 != 0 || features <= 0 ||
-        (relu_pieces && features % kStep != 0))
+    if (k % kStep != 0 || k < 2 * kStep || k > kMostColumns || features % 4 != 0 || features <= 0 ||
+        features > kMostColumns || (relu_pieces && features % kStep != 0))
         return fail(FTC_ERR_UNSUPPORTED, "a product of %lld columns and %lld features", (long long)k, (long long)features);
     if (tokens <= 0) return FTC_OK;
     constexpr int TN = 128, TF = 256;

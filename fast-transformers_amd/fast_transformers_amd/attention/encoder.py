@@ -74,6 +74,9 @@ class TransformerEncoderLayer(Module):
         return self.norm2(x + y)
 
 
+# what the native products take (ftc_linear_split, ftc_split_rows): rows, and columns or features
+_MOST_ROWS, _MOST_COLUMNS = 1 << 26, 1 << 20
+
 # what the native forward restates, as it was when this module was imported
 _FORWARDS = {cls: cls.forward for cls in (Linear, LayerNorm, Dropout, AttentionLayer, TransformerEncoderLayer,
                                           CausalLinearAttention, ActivationFunctionFeatureMap)}
@@ -150,6 +153,8 @@ def _plain_layer(layer, x):
     E, M = q.shape[0] // heads, v.shape[0] // heads
     if E not in (32, 64) or M not in (32, 64) or k.shape != q.shape or v.shape[0] > 4096:
         return None
+    if 2 * q.shape[0] + v.shape[0] > _MOST_COLUMNS or w1.shape[0] > _MOST_COLUMNS:
+        return None
     if (q.shape[1], v.shape[1], tuple(o.shape), w1.shape[1], tuple(w2.shape)) != \
             (d, d, (d, v.shape[0]), d, (d, w1.shape[0])):
         return None
@@ -168,6 +173,8 @@ class TransformerEncoder(Module):
         """The whole stack in native code (``encoder_forward_hip``) where nothing has to be
         differentiated or watched and every part is the plain one; None otherwise."""
         if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.numel() > 0) or len(self.layers) == 0:
+            return None
+        if x.shape[0] * x.shape[1] >= _MOST_ROWS:
             return None
         if attn_mask is None or not attn_mask.lower_triangular:
             return None

@@ -269,7 +269,8 @@ int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_t
  * power of two and kept as two fp16 pieces, hi + lo = row x 2^e, and a product is the sum of three
  * piece products in fp32.  Rows in pieces take 4 bytes per value: for each block of 32 columns 32 hi
  * and then 32 lo; `scale` holds 2^-e per row.  All pointers are device pointers, 16-byte aligned;
- * numbers of columns are multiples of 32 (at most 4096 for rows), of features multiples of 4.
+ * numbers of columns are multiples of 32 (at most 4096 for rows), of features multiples of 4, either
+ * at most 2^20; ftc_split_rows and ftc_layer_norm_split take fewer than 2^26 rows.
  */
 typedef struct ftc_weight {
     const float *w;        /* rows x cols, dense (torch.nn.Linear.weight) */

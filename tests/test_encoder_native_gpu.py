@@ -221,3 +221,23 @@ def test_encoder_takes_a_mask_that_only_says_it_is_causal(monkeypatch):
     got = model(x, attn_mask=SimpleNamespace(lower_triangular=True))
     want = model(x, attn_mask=mask)
     assert (got - want).abs().max() <= 8e-6 * want.abs().max()  # (two fp32 evaluations, as above)
+
+
+def test_encoder_keeps_its_modules_beyond_the_native_sizes(monkeypatch):
+    from fast_transformers_amd import attention, masking, _native
+    model, _, calls = small_encoder(monkeypatch)
+    N, L = 1 << 13, 1 << 13   # 2^26 rows, as a view of one (none of them is read)
+    x = torch.rand(1, 1, 64, device="cuda").expand(N, L, 64)
+    assert model._fused_forward(x, masking.TriangularCausalMask(L, device="cuda"), None) is None
+    with torch.device("cuda"):
+        wide = attention.build_causal_linear_encoder(1, 2, 32, 32, (1 << 20) + 32).eval().requires_grad_(False)
+    assert wide(x[:1, :3], attn_mask=masking.TriangularCausalMask(3, device="cuda")).shape == (1, 3, 64) and not calls
+    # the C entries refuse them before they launch anything
+    room = torch.zeros(64, device="cuda")
+    lib, some, big, n = _native.load(), ptr(room), ctypes.c_int64((1 << 20) + 32), ctypes.c_int64(64)
+    assert lib.ftc_linear_split(some, some, n, some, some, some, some, big, n, None, some, None, None, stream()) == -2
+    assert lib.ftc_linear_split(some, some, n, some, some, some, some, n, big, None, some, None, None, stream()) == -2
+    assert lib.ftc_split_rows(some, ctypes.c_int64(1 << 26), n, some, some, stream()) == -2
+    for rows, cols in ((64, big.value), (big.value, 64)):
+        item = Weight(some.value, None, rows, cols, some.value, some.value, some.value, some.value)
+        assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == -2
