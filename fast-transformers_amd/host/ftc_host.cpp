@@ -337,78 +337,89 @@ struct Pieces {
 // A stack of post-norm encoder layers (attention/encoder.py) with causal linear attention, and the
 // final norm: every product on the fp16 matrix cores in pieces (csrc/ftc_linear.hip), the norms
 // leaving their rows in pieces as well.  `x`: dense (N, L, d).
+//
+// Memory: rows are kept only as long as they are read, so that the stack needs no more than its
+// modules did (six times x where the feed-forward layer has at most 3 d features: twelve with a
+// buffer for each of them).  `wide` holds a layer's q, k and v; when the attention has read them, its
+// rows in pieces and, behind them, the output projection; then the feed-forward rows.  `rows` begins a
+// layer with x in pieces and has the attention's rows, the first norm's pieces and the second
+// product in turn; the second norm's pieces go to `other`, and the two change places.  `out` has the
+// first norm's rows and then the layer's.
 Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::optional<Norm> &final_norm,
                int64_t H, int64_t E, int64_t M, const OptTensor &key_lengths) {
     const at::NoGradGuard no_grad;
     const int64_t N = x.size(0), L = x.size(1), d = x.size(2), T = N * L;
     const auto fp32 = x.options();
     const int64_t *lengths = lengths_ptr(key_lengths, x);
-    const int64_t width = H * (2 * E + M);
-    int64_t ff = 0;
-    for (const Layer &l : layers) ff = std::max(ff, l.first.weight.size(0));
-    const Tensor qkv = at::empty({T, width}, fp32), rows = at::empty({T, H * M}, fp32), y = at::empty({T, d}, fp32),
-                 x1 = at::empty({T, d}, fp32), x_pieces = at::empty({T, d}, fp32), x_scale = at::empty({T}, fp32),
-                 r_pieces = at::empty({T, H * M}, fp32), r_scale = at::empty({T}, fp32),
-                 h_pieces = at::empty({T, ff}, fp32), h_scale = at::empty({T}, fp32), out = at::empty_like(x);
-    Tensor now = x;  // the layer's input
-    Tensor next = layers.size() > 1 || final_norm ? at::empty({T, d}, fp32) : out;
-    auto view = [&](const Tensor &t, int64_t column, int64_t row, int64_t X) {
+    const int64_t width = H * (2 * E + M), most_rows = std::max(d, H * M);
+    int64_t most_wide = std::max(width, H * M + d);
+    for (const Layer &l : layers) most_wide = std::max(most_wide, l.first.weight.size(0));
+    const Tensor wide = at::empty({T, most_wide}, fp32), scale_of_rows = at::empty({T}, fp32),
+                 scale_of_wide = at::empty({T}, fp32), out = at::empty_like(x);
+    Tensor rows_buffer = at::empty({T, most_rows}, fp32), other_buffer = at::empty({T, most_rows}, fp32);
+    float *const qkv = wide.data_ptr<float>(), *const projected = qkv + T * H * M;
+    float *rows = rows_buffer.data_ptr<float>(), *other = other_buffer.data_ptr<float>();
+    float *const row_scale = scale_of_rows.data_ptr<float>(), *const wide_scale = scale_of_wide.data_ptr<float>();
+    float *const to = out.data_ptr<float>();
+    auto view = [&](float *base, int64_t column, int64_t row, int64_t X) {
         ftc_tensor4 v;
-        v.ptr = t.data_ptr<float>() + column, v.dtype = FTC_F32;
+        v.ptr = base + column, v.dtype = FTC_F32;
         v.size[0] = N, v.size[1] = H, v.size[2] = L, v.size[3] = X;
         v.stride[0] = L * row, v.stride[1] = X, v.stride[2] = row, v.stride[3] = 1;
         return v;
     };
     const ftc_tensor4 q = view(qkv, 0, width, E), k = view(qkv, H * E, width, E),
-                      v = view(qkv, 2 * H * E, width, M), o = view(rows, 0, H * M, M);
+                      v = view(qkv, 2 * H * E, width, M);
     Call call(x, workspace_bytes(ftc_causal_linear_attention_workspace_bytes,
                                  "ftc_causal_linear_attention_workspace_bytes", N, H, L, E, M, FTC_F32));
     void *const stream = call.stream;
     auto f = [](const OptTensor &t) { return t ? t->const_data_ptr<float>() : nullptr; };
-    auto linear = [&](const Tensor &pieces, const Tensor &scale, const Pieces &w, const float *residual,
-                      const Tensor &to) {
-        check(ftc_linear_split(pieces.data_ptr(), scale.const_data_ptr<float>(), T, w.pieces.data_ptr(),
+    // (either the rows themselves or, behind max(., 0), in pieces with a scale)
+    auto linear = [&](const float *pieces, const float *pieces_scale, const Pieces &w, const float *residual,
+                      float *y, float *relu_pieces, float *relu_scale) {
+        check(ftc_linear_split(pieces, pieces_scale, T, w.pieces.const_data_ptr<float>(),
                                w.scale.const_data_ptr<float>(), w.bias.const_data_ptr<float>(),
-                               w.norm.const_data_ptr<float>(), w.rows, w.cols, residual, to.data_ptr<float>(),
-                               nullptr, nullptr, stream),
+                               w.norm.const_data_ptr<float>(), w.rows, w.cols, residual, y, relu_pieces,
+                               relu_scale, stream),
               "ftc_linear_split");
     };
-    auto norm = [&](const Tensor &in, const Norm &n, const Tensor &to, bool pieces) {
-        check(ftc_layer_norm_split(in.const_data_ptr<float>(), f(n.weight), f(n.bias), (float)n.eps, T, d,
-                                   to.data_ptr<float>(), pieces ? x_pieces.data_ptr() : nullptr,
-                                   pieces ? x_scale.data_ptr<float>() : nullptr, stream),
+    auto split = [&](const float *from, int64_t columns, float *pieces, float *pieces_scale) {
+        check(ftc_split_rows(from, T, columns, pieces, pieces_scale, stream), "ftc_split_rows");
+    };
+    auto norm = [&](const float *from, const Norm &n, float *y, float *pieces) {
+        check(ftc_layer_norm_split(from, f(n.weight), f(n.bias), (float)n.eps, T, d, y, pieces,
+                                   pieces ? row_scale : nullptr, stream),
               "ftc_layer_norm_split");
     };
     native([&] {
-        check(ftc_split_rows(x.const_data_ptr<float>(), T, d, x_pieces.data_ptr(), x_scale.data_ptr<float>(), stream),
-              "ftc_split_rows");
+        split(x.const_data_ptr<float>(), d, rows, row_scale);
         for (size_t i = 0; i < layers.size(); i++) {
             const Layer &l = layers[i];
+            const float *const input = i == 0 ? x.const_data_ptr<float>() : to;
             std::vector<ftc_weight> list;
             const Pieces in({&l.query, &l.key, &l.value}, list), proj({&l.out}, list), first({&l.first}, list),
                 second({&l.second}, list);
             check(ftc_split_weights(list.data(), (int32_t)list.size(), stream), "ftc_split_weights");
-            linear(x_pieces, x_scale, in, nullptr, qkv);
+            linear(rows, row_scale, in, nullptr, qkv, nullptr, nullptr);
+            const ftc_tensor4 o = view(rows, 0, H * M, M);
             check(ftc_causal_linear_attention_forward(&q, &k, &v, lengths, (float)l.eps, &o, nullptr, call.ws,
                                                       call.ws_bytes, stream),
                   "ftc_causal_linear_attention_forward");
-            check(ftc_split_rows(rows.const_data_ptr<float>(), T, H * M, r_pieces.data_ptr(), r_scale.data_ptr<float>(),
-                                 stream),
-                  "ftc_split_rows");
-            linear(r_pieces, r_scale, proj, now.const_data_ptr<float>(), y);
-            norm(y, l.norm1, x1, true);
-            check(ftc_linear_split(x_pieces.data_ptr(), x_scale.const_data_ptr<float>(), T, first.pieces.data_ptr(),
-                                   first.scale.const_data_ptr<float>(), first.bias.const_data_ptr<float>(),
-                                   first.norm.const_data_ptr<float>(), first.rows, first.cols, nullptr, nullptr,
-                                   h_pieces.data_ptr(), h_scale.data_ptr<float>(), stream),
-                  "ftc_linear_split");
-            linear(h_pieces, h_scale, second, x1.const_data_ptr<float>(), y);
-            const bool last = i + 1 == layers.size();
-            if (last && !final_norm) next = out;
-            norm(y, l.norm2, next, !last);
-            now = next;
+            split(rows, H * M, qkv, wide_scale);
+            linear(qkv, wide_scale, proj, input, projected, nullptr, nullptr);
+            norm(projected, l.norm1, to, rows);
+            linear(rows, row_scale, first, nullptr, nullptr, qkv, wide_scale);
+            linear(qkv, wide_scale, second, to, rows, nullptr, nullptr);
+            if (i + 1 < layers.size()) {
+                norm(rows, l.norm2, to, other);
+                std::swap(rows, other);
+            } else if (final_norm) {
+                norm(rows, l.norm2, other, nullptr);
+                norm(other, *final_norm, to, nullptr);
+            } else {
+                norm(rows, l.norm2, to, nullptr);
+            }
         }
-        if (final_norm) norm(now, *final_norm, out, false);
     });
     call.done();
     return out;

@@ -241,3 +241,29 @@ def test_encoder_keeps_its_modules_beyond_the_native_sizes(monkeypatch):
     for rows, cols in ((64, big.value), (big.value, 64)):
         item = Weight(some.value, None, rows, cols, some.value, some.value, some.value, some.value)
         assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == -2
+
+
+@pytest.mark.parametrize("final", [True, False], ids=["final_norm", "no_norm"])
+@pytest.mark.parametrize("ff", [512, 1024, 2048])
+def test_encoder_needs_no_more_memory_than_its_modules(ff, final):
+    from fast_transformers_amd import attention, masking
+    with torch.device("cuda"):
+        model = attention.build_causal_linear_encoder(3, 8, 64, 64, ff, final_normalization=final).eval()
+    model.requires_grad_(False)
+    x, mask = torch.rand(10, 2048, 512, device="cuda"), masking.TriangularCausalMask(2048, device="cuda")
+
+    def peak():
+        model(x, attn_mask=mask)     # (workspaces and library handles stay)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        model(x, attn_mask=mask)
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - before
+    native = peak()
+    handle = model.layers[0].linear1.register_forward_hook(lambda *a: None)
+    modules = peak()
+    handle.remove()
+    # (a layer's weights in pieces and the scales of the rows come on top)
+    weights = 4 * 512 * (4 * 512 + 2 * ff + 16) + 2 * 4 * x.shape[0] * x.shape[1]
+    assert native <= modules + 1.1 * weights
