@@ -613,17 +613,45 @@ bool pad_eligible(const ScanDesc &sc, int64_t rows) {
     return padded_shape_ok(Dp, round_up(sc.v.width, 32));
 }
 
+// Whether the padded copies of scan i (`padded`: the scans that would have them) would run on the
+// fp16-piece kernel: the scans of one padded shape are offered to it together, as run_scans does.
+bool copies_on_pieces(const ScanDesc *scans, int n, const bool *padded, int i, int64_t N, int64_t H, int64_t L) {
+    auto shape = [&](int j, int64_t &D, int64_t &F) {
+        D = padded_rows(scans[j].a.width), F = round_up(scans[j].v.width, 32);
+    };
+    int64_t D, F;
+    shape(i, D, F);
+    if (!padded[i]) return false;
+    ScanDesc group[kMfmaMaxScans];
+    int ngroup = 0;
+    for (int j = 0; j < n; j++) {
+        int64_t Dj, Fj;
+        shape(j, Dj, Fj);
+        if (padded[j] && Dj > 64) return false;  // (that one's copies serve the others as well)
+        if (!padded[j] || Dj != D || Fj != F) continue;
+        ScanDesc &sc = group[ngroup++] = scans[j];
+        Operand *in[3] = {&sc.a, &sc.b, &sc.v};
+        for (int k = 0; k < 3; k++) {
+            const int64_t w = k == 2 ? F : D;
+            *in[k] = Operand{nullptr, H * L * w, L * w, w, in[k]->dtype, (int32_t)w};
+        }
+        sc.out = OperandOut{nullptr, H * L * F, L * F, F, sc.out.dtype, (int32_t)F};
+    }
+    return mfma_tp_takes(group, ngroup, N, H, L);
+}
+
 // Whether an fp32 scan of odd widths runs on the fp16-piece kernel where its rows lie rather than on
-// padded copies: where each of its operands would have to be copied (forward + backward, us, here
-// / on the copies: 9 x 11 chains, L=1531, 25 x 33: 126 / 248; 8 x 16, L=4096, 50 x 50: 387 / 940; one
-// chain of 100, on the VALU kernel before: 17 / 132).  Scans some of whose rows stay where they
-// are (25 x 64: two copies of four) would gain as well, 344 against 500 us at 8 x 16, L=4096;
-// their route through the copies is what the planner's tests lay down.  Thousands of chains of up
-// to four chunks of narrow rows keep the copies, which bring them to 32 x 32 (2048 chains,
-// L=100, 10 x 9: 228 / 176; 25 x 33: 252 / 302).
-bool odd_in_place(const ScanDesc &sc, int64_t chains, int64_t L) {
+// padded copies: where each of its operands would have to be copied and the copies would run on
+// that kernel as well (forward + backward, us, here / on the copies: 8 x 16 chains, L=4096, 50 x 50:
+// 387 / 940).  Where they would not -- few chains of narrow rows, too few rows for copies -- the other
+// kernels hold every fp32 value exactly, and two pieces under a scale shared by a chunk's rows and
+// columns do not (9 x 11 chains, L=1531, 25 x 33, forward: 2-norm error 6.6e-7 here, 5.2e-7 there; with
+// every other column 2^-20 of its neighbours the small ones are off by 8e-2 of their size and by 5e-7).
+// Scans some of whose rows stay where they are (25 x 64: two copies of four) keep the copies, although
+// 8 x 16 chains, L=4096, take 500 us on them and 344 here.
+bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64_t N, int64_t H, int64_t L) {
+    const ScanDesc &sc = scans[i];
     if (tuning().odd == 0) return false;  // tuning aid
-    if (chains > 1024 && L <= 128 && sc.a.width < 24 && sc.v.width < 24) return false;
     const Operand *in[3] = {&sc.a, &sc.b, &sc.v};
     if (sc.out.dtype != FTC_F32) return false;
     bool any_fits = sc.out.width % 32 == 0 &&
@@ -634,7 +662,7 @@ bool odd_in_place(const ScanDesc &sc, int64_t chains, int64_t L) {
         any_fits = any_fits || (o->width % 32 == 0 && mfma_operand_in_place(o->ptr, o->stride_n, o->stride_h,
                                                                             o->stride_l, FTC_F32, o->width, L));
     }
-    return !any_fits || tuning().odd > 0;
+    return tuning().odd > 0 || (!any_fits && copies_on_pieces(scans, n, padded, i, N, H, L));
 }
 
 // Scans for which odd_in_place holds, in one launch or one per shape, whichever is estimated
@@ -734,7 +762,7 @@ int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
         ScanDesc odd[kMfmaMaxScans];
         int members[kMfmaMaxScans], nodd = 0;
         for (int i = 0; i < n; i++)
-            if (!taken[i] && !native[i] && odd_in_place(scans[i], N * H, L)) members[nodd] = i, odd[nodd++] = scans[i];
+            if (!taken[i] && !native[i] && odd_in_place(scans, n, padded, i, N, H, L)) members[nodd] = i, odd[nodd++] = scans[i];
         if (nodd > 0) {
             bool done = false;
             const int rc = odd_scans(odd, nodd, N, H, L, workspace, workspace_bytes, stream, &done);

@@ -18,9 +18,19 @@ SHAPES = [
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
-def test_odd_widths_in_place(shape):
+def test_odd_widths_in_place(shape, monkeypatch):
     from fast_transformers_amd import _native
     import fast_transformers_amd.causal_product as cp
+    monkeypatch.setenv("FTC_ODD", "1")  # (also where the copies would run on another kernel)
+    cp.reload_tuning()
+    try:
+        _odd_widths_in_place(shape, cp, _native)
+    finally:
+        monkeypatch.delenv("FTC_ODD")
+        cp.reload_tuning()
+
+
+def _odd_widths_in_place(shape, cp, _native):
     N, H, L, E, M = shape
     Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=900 + L)
     nlh = lambda t: t.permute(0, 2, 1, 3).contiguous().cuda().permute(0, 2, 1, 3)  # NLHE storage
@@ -50,7 +60,7 @@ def test_odd_widths_with_no_room_for_an_exchange():
     the generic kernel only: served as before, and not refused."""
     import ctypes
     from fast_transformers_amd import _native
-    N, H, L, E, M = 1, 3, 9000, 9, 9
+    N, H, L, E, M = 1, 3, 9000, 50, 50
     lib = _native.load()
     plan = _native.plan((N, H, L, E), (N, H, L, M))
     assert "scan_tph_kernel (exchange)" in plan
@@ -66,3 +76,41 @@ def test_odd_widths_with_no_room_for_an_exchange():
     assert lib.ftc_last_kernel() == b"generic_scan_kernel"
     exact = oracle.forward(Q.double(), K.double(), V.double())
     assert scale_error(out.cpu(), exact) <= max(4 * scale_error(oracle.forward(Q, K, V), exact), 2e-6)
+
+
+def _each(got, exact, dim):
+    """The largest 2-norm error of a row (dim 3) or column (dim 2) over its own 2-norm."""
+    got, exact = got.double(), exact.double()
+    return ((got - exact).norm(dim=dim) / exact.norm(dim=dim)).max().item()
+
+
+# calls whose aligned counterparts run on kernels that hold every fp32 value exactly: too few rows
+# for copies; few chains of narrow rows; of a backward call, some scans only (the results named)
+EXACT = [((1, 1, 100, 25, 33), "oqkv"), ((1, 1, 1356, 18, 18), "oqkv"), ((9, 11, 1531, 25, 33), "ov")]
+
+
+@pytest.mark.parametrize("shape, results", EXACT, ids=lambda s: s if isinstance(s, str) else "n%d_h%d_l%d_e%d_m%d" % s)
+@pytest.mark.parametrize("small", ["q_rows", "q_columns", "k_columns", "v_columns", "g_rows", "g_columns", "v_early_rows"])
+def test_small_rows_and_columns_beside_large_ones(small, shape, results):
+    """Every row and column is as close to float64, on its own scale, as the fp32 oracle's, where
+    the widths' multiples of 32 are."""
+    import fast_transformers_amd.causal_product as cp
+    Q, K, V, G = oracle.make_inputs(*shape, seed=11)
+    if small == "v_early_rows":  # rows 48 and on set no scale for the rows before them
+        V[:, :, 48:] *= 2.0 ** 20
+    else:
+        t = dict(q=Q, k=K, v=V, g=G)[small[0]]
+        t[..., 5::32, :] *= 2.0 ** -20 if small.endswith("rows") else 1
+        t[..., ::2] *= 2.0 ** -20 if small.endswith("columns") else 1
+    q, k, v, g = (t.cuda() for t in (Q, K, V, G))
+    outs = [torch.full_like(t, float("nan")) for t in (v, q, k, v)]
+    cp.causal_dot_product_hip(q, k, v, outs[0])
+    cp.causal_dot_backward_hip(q, k, v, g, *outs[1:])
+    cp.check_workspaces()
+    wide = [t.double() for t in (Q, K, V, G)]
+    refs = [oracle.forward(Q, K, V)] + list(oracle.backward(Q, K, V, G))
+    exact = [oracle.forward(*wide[:3])] + list(oracle.backward(*wide))
+    for name, got, ref, ex in zip("oqkv", outs, refs, exact):
+        for dim in (2, 3):
+            if name in results:
+                assert _each(got.cpu(), ex, dim) <= max(4 * _each(ref, ex, dim), 2e-6)

@@ -312,3 +312,22 @@ def test_rows_of_more_than_512_values_are_cut_into_pieces():
     # bf16 rows of that width: refused, by the queries as by the calls
     assert lib.ftc_causal_dot_product_workspace_bytes(1, 2, 300, 600, 520, _native.FTC_BF16) < 0
     assert b"fp32" in lib.ftc_last_error()
+
+
+def test_odd_widths_lie_in_place_only_where_their_copies_run_on_the_same_kernel():
+    """The padded shape's own plan names the kernel that the copies would run on."""
+    up = lambda w: (w + 31) // 32 * 32
+    seen = set()
+    for N, H, L, E, M in [(1, 1, 100, 25, 33), (1, 1, 1356, 18, 18), (9, 11, 1531, 25, 33), (8, 16, 4096, 50, 50),
+                          (2, 8, 333, 50, 50), (1, 3, 9000, 31, 62), (3, 5, 65, 63, 63), (64, 32, 100, 10, 9),
+                          (1, 16, 24853, 63, 63), (24, 8, 1, 19, 41), (5, 32, 1, 60, 61)]:
+        odd = lines((N, H, L, E), (N, H, L, M))
+        aligned = lines((N, H, L, up(E)), (N, H, L, up(M)))
+        in_place = odd[0].startswith("scan_tph_kernel")
+        assert in_place == (aligned[0].startswith("scan_tph_kernel") and N * H * L >= 512)
+        seen.add(in_place)
+    assert seen == {False, True}
+    # a backward call may have both
+    mixed = lines((9, 11, 1531, 25, 33)[:4], (9, 11, 1531, 33), backward=True)
+    assert mixed[0].startswith("scan_tph_kernel: 2 scans") and mixed[1].startswith("pad_rows_kernel: 3 operands")
+    assert mixed[2].startswith("scan_dma_kernel: 1 scan")
