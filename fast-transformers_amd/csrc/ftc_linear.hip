@@ -22,8 +22,11 @@
 // of lo each, one cache line per row and k-step.  Whoever writes rows that only a product reads
 // writes them in pieces; the scale must be known before the row's first value is cut, so the
 // producer has the whole row (layer norm, ftc_split_rows) or a bound (relu: |y| <= max|x| max_f
-// sum_k |w[f, k]| + the largest bias, four or five bits above the largest value as a rule, which the
-// seventeen bits above leave room for).
+// sum_k |w[f, k]| + the largest bias, six or seven bits above a row's ordinary values, which the
+// seventeen bits above leave room for).  Where the features are too far apart for one bound -- it is
+// more than 2^6 times max|x| sum_k |w[f, k]| of the least of them -- a row leaves the product in fp32
+// and a pass behind it (cut_rows_kernel) cuts it by its own largest value (where no row needs it,
+// 4.6 us for 40960 rows).
 #include <algorithm>
 
 #include "ftc_tp_kernel.h"
@@ -42,7 +45,7 @@ constexpr int64_t kMostColumns = 1 << 20, kMostRows = 1 << 26;
 // the power of two that brings a largest magnitude to 2^14 .. 2^15, and its reciprocal
 __device__ __forceinline__ void scale_of(float largest, float &s, float &inverse) {
     const int e = (int)((__float_as_uint(largest) >> 23) & 0xffu);  // largest < 2^(e - 126)
-    const int up = e == 0 ? 0 : max(-126, min(126, 141 - e));
+    const int up = max(-126, min(126, 141 - e));  // (a row of zeros: 126, so that its scale bounds it)
     s = __uint_as_float((uint32_t)(127 + up) << 23);
     inverse = __uint_as_float((uint32_t)(127 - up) << 23);
 }
@@ -158,6 +161,34 @@ __global__ __launch_bounds__(256) void rows_kernel(const float *__restrict__ x, 
         if (c < cols) store_pieces(pieces + row * cols * 4, c, v[i], s);
     }
     if (lane == 0) scale[row] = inverse;
+}
+
+// Rows that the product left in fp32 (scale < 0, a row's values where its pieces go) in pieces, each
+// in its place: a wavefront reads 256 columns and writes the same 1024 bytes.  A wavefront looks at
+// kCutRows rows.
+constexpr int kCutRows = 8;
+__global__ __launch_bounds__(256) void cut_rows_kernel(char *rows, float *scale, int64_t count, int cols) {
+    const int64_t first = ((int64_t)blockIdx.x * 4 + threadIdx.x / 64) * kCutRows;
+    const int lane = threadIdx.x % 64;
+    const bool here = lane < kCutRows && first + lane < count && scale[first + lane] < 0.f;
+    for (uint64_t left = __ballot(here); left != 0; left &= left - 1) {
+        const int64_t r = first + __builtin_ctzll(left);
+        char *const row = rows + r * cols * 4;
+        float largest = 0.f;
+        for (int c = 4 * lane; c < cols; c += 256) largest = fmaxf(largest, largest_of(*(const float4 *)(row + 4 * c)));
+        largest = wave_largest(largest);
+        float s, inverse;
+        scale_of(largest, s, inverse);
+        for (int c0 = 0; c0 < cols; c0 += 256) {
+            const int c = c0 + 4 * lane;
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (c < cols) x = *(const float4 *)(row + 4 * c);
+            // (every lane's value is here before any lane writes where it was)
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w)::"memory");
+            if (c < cols) store_pieces(row, c, x, s);
+        }
+        if (lane == 0) scale[r] = inverse;
+    }
 }
 
 // ---- the product --------------------------------------------------------------------------------
@@ -315,13 +346,16 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
         }
     };
     static_assert(3 * WF >= kRequests, "a request per group of matrix instructions");
-    float bound_w = 0.f, bound_b = 0.f;
+    float bound_w = 0.f, bound_b = 0.f, least_w = __builtin_inff();
     if (EPI == kRelu) {  // (the same numbers in every workgroup)
         for (int i = lane; i < p.features; i += 64) {
             bound_w = fmaxf(bound_w, p.w_norm[i]);
             bound_b = fmaxf(bound_b, p.bias[i]);  // (a bias below zero, lowest or -inf, raises nothing)
+            // (a feature without weights and with no bias above zero is zero in any row)
+            least_w = fminf(least_w, p.w_norm[i] == 0.f && !(p.bias[i] > 0.f) ? __builtin_inff() : p.w_norm[i]);
         }
         bound_w = wave_largest(bound_w), bound_b = wave_largest(bound_b);
+        least_w = -wave_largest(-least_w);
     }
     Tile t = tile_of(0);
     if (!t.there) return;
@@ -373,7 +407,9 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
             at[j] = (uint32_t)(wt * (TN / 2) + tok) * out_row;
             if (EPI == kRelu) {
                 float inverse;
-                scale_of((32768.f * xs[j]) * bound_w + bound_b, s_out[j], inverse);
+                const float x_most = 32768.f * xs[j], bound = x_most * bound_w + bound_b;
+                scale_of(bound, s_out[j], inverse);
+                if (!(bound <= 64.f * (x_most * least_w))) s_out[j] = 0.f, inverse = -1.f;  // (in fp32)
                 const int64_t token = t.t0 + wt * (TN / 2) + tok;
                 if (t.f0 == 0 && wf == 0 && g == 0 && token < p.tokens) p.out_scale[token] = inverse;
             }
@@ -407,10 +443,18 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
                 if (EPI == kRelu) {
                     uint32_t h0, h1, l0, l1;
                     auto relu = [](float y) { return y < 0.f ? 0.f : y; };  // (keeps NaN, as torch's does)
-                    cut_quad_f16(relu(y0), relu(y1), relu(y2), relu(y3), s_out[j], h0, h1, l0, l1);
-                    const uint32_t to = f_in ? at[j] + (uint32_t)(f / kStep * kRowBytes + 2 * (f % kStep)) : 0x80000000u;
+                    y0 = relu(y0), y1 = relu(y1), y2 = relu(y2), y3 = relu(y3);
+                    cut_quad_f16(y0, y1, y2, y3, s_out[j], h0, h1, l0, l1);
+                    const bool whole = s_out[j] == 0.f;  // the row in fp32, both halves of the quad
+                    if (whole) {
+                        h0 = __float_as_uint(y0), h1 = __float_as_uint(y1);
+                        l0 = __float_as_uint(y2), l1 = __float_as_uint(y3);
+                    }
+                    const uint32_t to = !f_in ? 0x80000000u
+                                        : whole ? at[j] + 4u * f
+                                                : at[j] + (uint32_t)(f / kStep * kRowBytes + 2 * (f % kStep));
                     __builtin_amdgcn_raw_buffer_store_b64(u32x2{h0, h1}, o_rs, to, 0, 0);
-                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{l0, l1}, o_rs, to + 2 * kStep, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{l0, l1}, o_rs, to + (whole ? 8u : 2u * kStep), 0, 0);
                 } else {
                     buffer_store4(o_rs, f_in ? at[j] + 4u * f : 0x80000000u, y0, y1, y2, y3);
                 }
@@ -515,9 +559,12 @@ int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const 
     // (one workgroup per CU, a multiple of the eight XCDs)
     const int64_t tiles = (token_tiles + 7) / 8 * a.feature_tiles;
     const dim3 grid((unsigned)(8 * std::min<int64_t>(tiles, 32))), block(256);
-    if (relu_pieces)
+    if (relu_pieces) {
         hipLaunchKernelGGL((linear_kernel<TN, TF, kRelu>), grid, block, 0, (hipStream_t)stream, a);
-    else if (residual)
+        const dim3 cuts((unsigned)((tokens + 4 * kCutRows - 1) / (4 * kCutRows)));
+        hipLaunchKernelGGL(cut_rows_kernel, cuts, block, 0, (hipStream_t)stream, a.out_pieces, relu_scale, tokens,
+                           (int)features);
+    } else if (residual)
         hipLaunchKernelGGL((linear_kernel<TN, TF, kResidual>), grid, block, 0, (hipStream_t)stream, a);
     else
         hipLaunchKernelGGL((linear_kernel<TN, TF, kPlain>), grid, block, 0, (hipStream_t)stream, a);

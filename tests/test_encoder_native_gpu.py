@@ -105,6 +105,39 @@ def test_relu_keeps_nan_and_takes_any_bias_below_zero():
     assert (got - want).nan_to_num().abs().max() <= (K + 1) * 2.0 ** -24 * 200
 
 
+@pytest.mark.parametrize("shape", [(130, 64, 288), (7, 96, 4160), (1, 64, 32)], ids=lambda s: "t%d_k%d_f%d" % s)
+@pytest.mark.parametrize("large", ["weight", "bias", "zero_rows"])
+def test_relu_features_of_very_different_size(large, shape):
+    """A feature with large weights or a large bias leaves the other features of a row where it is
+    switched off their precision (a row's pieces hold values down to 2^-17 of the row's largest)."""
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    T, K, F = shape
+    gen = torch.Generator(device="cuda").manual_seed(F)
+    x, w, b = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, K), (F, K), (F,)))
+    if large == "weight":       # (off in the rows of odd number)
+        w[F // 2] = 2.0 ** 24
+        x[::2], x[1::2] = x[::2].abs(), -x[1::2].abs()
+    elif large == "bias":       # (off: the row's own product is below minus the bias)
+        w[F // 2], b[F // 2] = -2.0 ** 14, 2.0 ** 14
+        x[1::2] = x[1::2].abs() + 1
+    else:
+        x[1::2] = 0
+    new = lambda *s: torch.full(s, float("nan"), device="cuda")
+    xp, xs, wp, ws, bo, wn, hp, hs = new(T, K), new(T), new(F, K), new(F), new(F), new(F), new(T, F), new(T)
+    item = Weight(w.data_ptr(), b.data_ptr(), F, K, wp.data_ptr(), ws.data_ptr(), bo.data_ptr(), wn.data_ptr())
+    assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == 0, _native.last_error()
+    assert lib.ftc_split_rows(ptr(x), ctypes.c_int64(T), ctypes.c_int64(K), ptr(xp), ptr(xs), stream()) == 0
+    assert lib.ftc_linear_split(ptr(xp), ptr(xs), ctypes.c_int64(T), ptr(wp), ptr(ws), ptr(bo), ptr(wn),
+                                ctypes.c_int64(F), ctypes.c_int64(K), None, None, ptr(hp), ptr(hs), stream()) == 0
+    got, want = whole(hp, hs), torch.relu(x.double() @ w.double().t() + b.double())
+    assert (hs > 0).all()
+    # as in test_products_in_pieces, and 2^-39 of the row's own largest
+    bound = (x.double().abs() @ w.double().abs().t()) * (3 * 2.0 ** -23 + (K / 32 + 3) * 2.0 ** -24) \
+        + 2.0 ** -22 * (b.double().abs() + want) + 2.0 ** -39 * want.amax(1, keepdim=True)
+    assert ((got - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("rows_cols", [(1, 32), (5, 96), (130, 512), (33, 1056), (3, 4096)], ids=lambda s: "r%d_c%d" % s)
 def test_layer_norm_in_pieces(rows_cols):
     from fast_transformers_amd import _native
