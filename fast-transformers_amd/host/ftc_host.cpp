@@ -24,6 +24,7 @@
 #include <chrono>
 #include <cstdlib>
 #include <map>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -44,10 +45,12 @@ void check(int64_t rc, const char *what) {
 }
 
 // A call into the library without Python's lock: a launch may block (a full queue), and other
-// threads go on meanwhile.
+// threads go on meanwhile.  `turn`: held during the call, by one thread at a time.
 template <class F>
-auto native(F f) {
+auto native(F f, std::mutex *turn = nullptr) {
     const py::gil_scoped_release unlocked;
+    std::unique_lock<std::mutex> held;
+    if (turn) held = std::unique_lock<std::mutex>(*turn);
     return f();
 }
 
@@ -136,6 +139,9 @@ struct Call {
     size_t ws_bytes = 0;
     py::object key;
     bool due = false;
+    // A call's launches pass data on through the workspace, which all calls on a stream share:
+    // another thread's must not come between them.
+    std::mutex *turn = nullptr;
 
     Call(const Tensor &q, int64_t bytes) : guard(q.device()) {
         stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
@@ -148,12 +154,17 @@ struct Call {
         if (failed(key)) g_python->check_all();
         ws = workspace.data_ptr(), ws_bytes = (size_t)workspace.numel();
         using clock = std::chrono::steady_clock;
-        static std::map<std::pair<int, intptr_t>, clock::time_point> last;  // (under Python's lock)
-        auto &then = last[{(int)q.device().index(), (intptr_t)stream}];
+        struct Shared {
+            clock::time_point then;
+            std::mutex turn;
+        };
+        static std::map<std::pair<int, intptr_t>, Shared> shared;  // (under Python's lock)
+        Shared &mine = shared[{(int)q.device().index(), (intptr_t)stream}];
+        turn = &mine.turn;
         const auto now = clock::now();
-        due = now - then >= std::chrono::milliseconds(10);
+        due = now - mine.then >= std::chrono::milliseconds(10);
         if (due) {
-            then = now;
+            mine.then = now;
             g_python->watch(key, workspace);
         }
     }
@@ -176,7 +187,7 @@ void forward(const Tensor &queries, const Tensor &keys, const Tensor &values, co
                                  "ftc_causal_dot_product_workspace_bytes", q.size(0), q.size(1), q.size(2),
                                  q.size(3), v.size(3), dq.dtype));
     const int rc = native(
-        [&] { return ftc_causal_dot_product(&dq, &dk, &dv, &dout, call.ws, call.ws_bytes, call.stream); });
+        [&] { return ftc_causal_dot_product(&dq, &dk, &dv, &dout, call.ws, call.ws_bytes, call.stream); }, call.turn);
     check(rc, "ftc_causal_dot_product");
     call.done();
 }
@@ -207,7 +218,7 @@ std::tuple<Tensor, OptTensor> product_with_state(const Tensor &queries, const Te
     const int rc = native([&] {
         return ftc_causal_dot_product_state(&dq, &dk, &dv, s0.defined() ? &d0 : nullptr, &dout,
                                             s1 ? &d1 : nullptr, call.ws, call.ws_bytes, call.stream);
-    });
+    }, call.turn);
     check(rc, "ftc_causal_dot_product_state");
     call.done();
     return {out, s1};
@@ -236,7 +247,7 @@ void backward(const Tensor &queries, const Tensor &keys, const Tensor &values, c
     const int rc = native([&] {
         return ftc_causal_dot_backward(&dq, &dk, &dv, &dg, gq.p, gk.p, gv.p, call.ws, call.ws_bytes,
                                        call.stream);
-    });
+    }, call.turn);
     check(rc, "ftc_causal_dot_backward");
     call.done();
 }
@@ -266,7 +277,7 @@ void attention(const Tensor &queries, const Tensor &keys, const Tensor &values, 
         return ftc_causal_linear_attention_forward(&dq, &dk, &dv, lengths, (float)eps, &dout,
                                                    denominators ? &dden : nullptr, call.ws, call.ws_bytes,
                                                    call.stream);
-    });
+    }, call.turn);
     check(rc, "ftc_causal_linear_attention_forward");
     call.done();
 }
@@ -288,7 +299,7 @@ void attention_backward(const Tensor &queries, const Tensor &keys, const Tensor 
     const int rc = native([&] {
         return ftc_causal_linear_attention_backward(&dq, &dk, &dv, lengths, &dout, &dden, &dg, gq.p, gk.p,
                                                     gv.p, call.ws, call.ws_bytes, call.stream);
-    });
+    }, call.turn);
     check(rc, "ftc_causal_linear_attention_backward");
     call.done();
 }
@@ -420,7 +431,7 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
                 norm(rows, l.norm2, to, nullptr);
             }
         }
-    });
+    }, call.turn);
     call.done();
     return out;
 }

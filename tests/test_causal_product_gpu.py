@@ -862,6 +862,36 @@ def test_the_next_call_after_a_probe_reads_it(cp, monkeypatch):
     cp.check_workspaces()
 
 
+def test_threads_take_turns_on_a_stream(cp):
+    """Calls of several launches that hand data on through the workspace, from two threads on one
+    stream: each has the results that it has alone, bit for bit."""
+    import threading
+    shapes = [(1, 1, 1356, 18, 18), (2, 3, 700, 25, 33)]   # padded copies, segments with an exchange
+    inputs = [[t.cuda() for t in oracle.make_inputs(*shape, seed=60 + i)] for i, shape in enumerate(shapes)]
+
+    def call(q, k, v, g):
+        outs = [torch.empty_like(t) for t in (v, q, k, v)]
+        cp.causal_dot_product_hip(q, k, v, outs[0])
+        cp.causal_dot_backward_hip(q, k, v, g, *outs[1:])
+        return outs
+    alone = [call(*tensors) for tensors in inputs]
+    got, start = [[], []], threading.Barrier(2)
+
+    def work(i):
+        start.wait()
+        got[i] = [call(*inputs[i]) for _ in range(40)]
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    cp.check_workspaces()
+    for i in range(2):
+        assert len(got[i]) == 40
+        for outs in got[i]:
+            assert all(torch.equal(o, want) for o, want in zip(outs, alone[i]))
+
+
 TP_SHAPES = [
     # N, H, L, E, M: enough chains for one workgroup per chain (and scan), or few enough that
     # a chain is cut into segments whose workgroups rebuild their starting state
