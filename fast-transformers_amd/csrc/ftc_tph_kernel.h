@@ -228,8 +228,8 @@ __device__ __forceinline__ u32x4 widen_bf16_quad(const u32x4 r) {
 // hardware asks for 4-byte alignment and checks the descriptor's end word by word); a lane whose
 // quad straddles the end of a row clears the words that belong to the next one when the
 // look-ahead first touches them, and stores such a quad word by word.  Measured against dense
-// zero-padded copies of the operands and results (9 x 11 chains, L=1531, 25 x 33): forward 79 ->
-// 38 us, backward 169 -> 89; a chunk costs what one of 64 x 64 does.
+// zero-padded copies of the operands and results (8 x 16 chains, L=4096, 50 x 50, forward + backward):
+// 940 -> 387 us; a chunk costs what one of 64 x 64 does.
 template <int KS, bool MIX, bool ODD>
 __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     constexpr int D = 64, F = 64;              // one block of state rows and of output columns

@@ -59,7 +59,7 @@ _host = None
 
 def host():
     """The compiled binding over the same C ABI that the package's own entry points use
-    (``host/ftc_host.cpp``; the ctypes one below costs a call about 20 us more).  Raises if it has
+    (``host/ftc_host.cpp``; the ctypes one below costs a call 12 to 17 us more).  Raises if it has
     not been built."""
     global _host
     if _host is None:

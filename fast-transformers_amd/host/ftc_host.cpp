@@ -2,9 +2,10 @@
 // fast_transformers_amd.causal_product take their tensors here.
 //
 // What bounds a small or ordinary call is the host: with the tensors described through ctypes a
-// forward + backward pass of N=10, H=8, L=1000, E=M=64 took the host 165 us where its two kernels
-// take 68.  Here a call checks its tensors, describes them on the stack, looks its workspace up
-// and launches, in about a microsecond and a half; nothing of a tensor is kept.
+// training step took the host 159 us (one chain of 64 positions), where the two kernels of N=10,
+// H=8, L=1000, E=M=64 take 68.  Here a call checks its tensors, describes them on the stack, looks
+// its workspace up and launches: 4.3 to 5.2 us per call where ctypes took 16.6 to 21.7; nothing of a
+// tensor is kept.
 //
 // The workspaces stay Python's (causal_product.__init__: one per device and stream, in a dict that
 // check_workspaces() walks); they are found here through that dict, and Python is called when
