@@ -403,11 +403,12 @@ def attention_training_step(steps=10, warmup=3):
 def encoder_workload(args):
     """Config 4: eval forward of an 8-layer causal-linear encoder (8 heads, query/value
     dims 64, d_model 512, FFN 1024, random-init weights) on rand(10, 4096, 512).  A step is
-    one forward pass; the share of causal_dot_product is timed with events around the
-    native call inside the attention module."""
+    one forward pass; the native calls that it makes (the whole stack in one call or, layer by
+    layer, the attention's) are timed with events around them, the attention launch by itself."""
     import torch
+    from fast_transformers_amd import _native
     from fast_transformers_amd.attention import build_causal_linear_encoder
-    from fast_transformers_amd.attention import causal_linear_attention as cla
+    from fast_transformers_amd.attention import causal_linear_attention as cla, encoder
     from fast_transformers_amd.masking import TriangularCausalMask
 
     torch.cuda.set_device(0)
@@ -417,20 +418,23 @@ def encoder_workload(args):
     x = torch.rand(N, L, D, generator=torch.Generator().manual_seed(4)).cuda()
     mask = TriangularCausalMask(L, device="cuda")
     op_events = []
-    # the native entry points the attention module may call: the fused one (feature map,
-    # mask, product and normaliser in one launch) when it covers the sizes, else the product
-    natives = {name: getattr(cla, name)
-               for name in ("causal_linear_attention_hip", "causal_dot_product_hip")}
+    # the native entry points that the encoder may call: the whole stack, or layer by layer the
+    # fused attention (feature map, mask, product and normaliser in one launch) when it covers the
+    # sizes, else the product
+    modules = {"encoder_forward_hip": encoder, "causal_linear_attention_hip": cla,
+               "causal_dot_product_hip": cla}
+    natives = {name: getattr(module, name) for name, module in modules.items()}
     used = set()
 
     def timed(name):
         def call(*a):
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             e0.record()
-            natives[name](*a)
+            result = natives[name](*a)
             e1.record()
             op_events.append((e0, e1))
             used.add(name)
+            return result
         return call
 
     with torch.no_grad():
@@ -446,15 +450,16 @@ def encoder_workload(args):
             enc(x, attn_mask=mask)
         torch.cuda.synchronize()
         ms = (time.perf_counter() - t0) * 1e3 / args.steps
-        for name in natives:
-            setattr(cla, name, timed(name))
+        for name, module in modules.items():
+            setattr(module, name, timed(name))
         for _ in range(args.steps):
             enc(x, attn_mask=mask)
         torch.cuda.synchronize()
-        for name in natives:
-            setattr(cla, name, natives[name])
+        for name, module in modules.items():
+            setattr(module, name, natives[name])
     op_ms = sum(a.elapsed_time(b) for a, b in op_events) / args.steps
-    fused = used == {"causal_linear_attention_hip"}
+    stack = used == {"encoder_forward_hip"}
+    fused = stack or used == {"causal_linear_attention_hip"}
     # The events above bracket the Python wrapper, so when the GPU has run dry they also see
     # the host preparing the call.  The launch itself: the same native entry on the
     # encoder's (N, L, H, 64) layout, back to back over rotating inputs (> 512 MB, cold).
@@ -479,6 +484,7 @@ def encoder_workload(args):
         e1.record()
         torch.cuda.synchronize()
         launch_ms = e0.elapsed_time(e1) / 60
+        kernel = _native.load().ftc_last_kernel().decode()
         del sets
     TH = N * 8 * L
     # roofline of the operator's launches inside the encoder (8 per forward pass, one per
@@ -511,10 +517,12 @@ def encoder_workload(args):
                    "native_ms_per_forward_bracketed_in_model": round(op_ms, 4),
                    "causal_dot_product_fwd_alg_GBps": round(gbps, 1)},
         "roofline": {"bound": bound,
-                     "kernel": ("scan_wg_kernel<64,64,NORM> (ftc_causal_linear_attention" if fused
-                                else "scan_dma_kernel (ftc_causal_dot_product")
-                               + ": the operator's forward launch, one per layer; the rest of "
-                                 "the encoder is torch's GEMMs and elementwise work)",
+                     "kernel": "%s (%s: the operator's forward launch, one per layer; the rest of "
+                               "the encoder is %s)"
+                               % (kernel, "ftc_causal_linear_attention_forward" if fused
+                                  else "ftc_causal_dot_product",
+                                  "linear_kernel's products on fp16 pieces and the norms between "
+                                  "them" if stack else "torch's GEMMs and elementwise work"),
                      "achieved": binding["achieved"], "peak": binding["peak"],
                      "unit": binding["unit"], "frac": binding["frac"],
                      "hbm": hbm_entry, "mfma": mfma_entry,
