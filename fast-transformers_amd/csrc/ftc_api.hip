@@ -649,7 +649,9 @@ bool copies_on_pieces(const ScanDesc *scans, int n, const bool *padded, int i, i
 // every other column 2^-20 of its neighbours the small ones are off by 8e-2 of their size and by 5e-7).
 // Scans some of whose rows stay where they are (25 x 64: two copies of four) keep the copies, although
 // 8 x 16 chains, L=4096, take 500 us on them and 344 here.
-bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64_t N, int64_t H, int64_t L) {
+// And a workspace without room for copies means the VALU kernel, here as for any width.
+bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64_t N, int64_t H, int64_t L,
+                  size_t workspace_bytes) {
     const ScanDesc &sc = scans[i];
     if (tuning().odd == 0) return false;  // tuning aid
     const Operand *in[3] = {&sc.a, &sc.b, &sc.v};
@@ -662,7 +664,10 @@ bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64
         any_fits = any_fits || (o->width % 32 == 0 && mfma_operand_in_place(o->ptr, o->stride_n, o->stride_h,
                                                                             o->stride_l, FTC_F32, o->width, L));
     }
-    return tuning().odd > 0 || (!any_fits && copies_on_pieces(scans, n, padded, i, N, H, L));
+    if (tuning().odd > 0) return true;
+    const bool room = plan_only() ||
+                      (int64_t)workspace_bytes >= padded_scan_workspace_bytes(N, H, L, sc.a.width, sc.v.width);
+    return !any_fits && room && copies_on_pieces(scans, n, padded, i, N, H, L);
 }
 
 // Scans for which odd_in_place holds, in one launch or one per shape, whichever is estimated
@@ -762,7 +767,7 @@ int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
         ScanDesc odd[kMfmaMaxScans];
         int members[kMfmaMaxScans], nodd = 0;
         for (int i = 0; i < n; i++)
-            if (!taken[i] && !native[i] && odd_in_place(scans, n, padded, i, N, H, L)) members[nodd] = i, odd[nodd++] = scans[i];
+            if (!taken[i] && !native[i] && odd_in_place(scans, n, padded, i, N, H, L, workspace_bytes)) members[nodd] = i, odd[nodd++] = scans[i];
         if (nodd > 0) {
             bool done = false;
             const int rc = odd_scans(odd, nodd, N, H, L, workspace, workspace_bytes, stream, &done);
@@ -827,9 +832,11 @@ int64_t scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t
             need = std::max(need, mfma_scan_workspace_bytes(N, H, L, D, widths[j], k));
     if (nslices == 0 && with_pad)
         need = std::max(need, padded_scan_workspace_bytes(N, H, L, D, F, bf16));
-    for (int k = 1; k <= kMfmaMaxScans; k++)
-        need = std::max(need, std::max(mfma_tp_workspace_bytes(N, H, L, D, F, k),
-                                       mfma_tp_workspace_bytes(N, H, L, D, F, k, false, true)));
+    for (int k = 1; k <= kMfmaMaxScans; k++) need = std::max(need, mfma_tp_workspace_bytes(N, H, L, D, F, k));
+    // (odd widths where they lie, which takes room for their copies: odd_in_place)
+    if (with_pad && !bf16 && padded_scan_workspace_bytes(N, H, L, D, F) > 0)
+        for (int k = 1; k <= kMfmaMaxScans; k++)
+            need = std::max(need, mfma_tp_workspace_bytes(N, H, L, D, F, k, false, true));
     if (with_pad && split_widths(D, F))
         need = std::max(need, split_scan_workspace_bytes(N, H, L, D, F, nullptr));
     return need;
@@ -1009,12 +1016,12 @@ int64_t ftc_causal_dot_backward_workspace_bytes(int64_t N, int64_t H, int64_t L,
     const bool bf16 = dtype == FTC_BF16;
     int64_t need = std::max(scan_workspace_bytes(N, H, L, E, M, true, bf16),
                             scan_workspace_bytes(N, H, L, M, E, true, bf16));
-    // (odd widths: scans of both shapes may share a launch)
-    for (int k = 2; k <= 3; k++)
-        need = std::max(need, mfma_tp_workspace_bytes(N, H, L, std::max(E, M), std::max(E, M), k, false, true));
     // the padded route of the three scans together: Q, K, dQ, dK and V, G, dV as dense rows
     if (padded_scan_workspace_bytes(N, H, L, E, M, bf16) > 0 ||
         padded_scan_workspace_bytes(N, H, L, M, E, bf16) > 0) {
+        // (odd widths: scans of both shapes may share a launch)
+        for (int k = 2; k <= 3 && !bf16; k++)
+            need = std::max(need, mfma_tp_workspace_bytes(N, H, L, std::max(E, M), std::max(E, M), k, false, true));
         int64_t ws = 0;
         if (padded_rows(E)) ws = std::max(ws, scan_workspace_bytes(N, H, L, padded_rows(E), round_up(M, 32)));
         if (padded_rows(M)) ws = std::max(ws, scan_workspace_bytes(N, H, L, padded_rows(M), round_up(E, 32)));

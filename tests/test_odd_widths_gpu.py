@@ -84,6 +84,32 @@ def _each(got, exact, dim):
     return ((got - exact).norm(dim=dim) / exact.norm(dim=dim)).max().item()
 
 
+def test_odd_widths_with_no_room_for_their_copies():
+    """A workspace for the VALU kernel alone has that kernel run, although rows read where they lie
+    would not need more."""
+    import ctypes
+    from fast_transformers_amd import _native
+    N, H, L, E, M = 2, 8, 333, 50, 50
+    lib = _native.load()
+    assert "scan_tph_kernel" in _native.plan((N, H, L, E), (N, H, L, M))
+    Q, K, V, _ = oracle.make_inputs(N, H, L, E, M, seed=32)
+    Q[..., ::2] *= 2.0 ** -20
+    V[..., ::2] *= 2.0 ** -20
+    out = torch.full((N, H, L, M), float("nan"), device="cuda")
+    q, k, v = (t.cuda() for t in (Q, K, V))
+    d = [_native.describe(t) for t in (q, k, v, out)]
+    room = 8 << 20
+    assert room < lib.ftc_causal_dot_product_workspace_bytes(N, H, L, E, M, 0)
+    ws = torch.zeros(room, dtype=torch.uint8, device="cuda")
+    rc = lib.ftc_causal_dot_product(*(ctypes.byref(t) for t in d), ctypes.c_void_p(ws.data_ptr()),
+                                    ctypes.c_size_t(room), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, _native.last_error()
+    assert lib.ftc_last_kernel() == b"generic_scan_kernel"
+    exact, ref = oracle.forward(Q.double(), K.double(), V.double()), oracle.forward(Q, K, V)
+    for dim in (2, 3):
+        assert _each(out.cpu(), exact, dim) <= max(4 * _each(ref, exact, dim), 2e-6)
+
+
 # calls whose aligned counterparts run on kernels that hold every fp32 value exactly: too few rows
 # for copies; few chains of narrow rows; of a backward call, some scans only (the results named)
 EXACT = [((1, 1, 100, 25, 33), "oqkv"), ((1, 1, 1356, 18, 18), "oqkv"), ((9, 11, 1531, 25, 33), "ov")]

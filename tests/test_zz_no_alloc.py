@@ -72,6 +72,27 @@ def test_static_scratch_entry_point_matches_workspace_entry_point():
             assert scale_error(got, oracle.forward(Q, K, V)) <= 1e-4
 
 
+def test_static_scratch_takes_long_narrow_chains():
+    """Sizes whose kernel needs a fraction of the array: routes that these widths never take (rows
+    of odd widths where they lie would exchange 55 MB here) have no say in what is asked for."""
+    from fast_transformers_amd import _native as native
+    lib = native.load()
+    N, H, L, E, M = 1, 17, 127751, 32, 32
+    nbytes = lib.ftc_causal_dot_product_workspace_bytes(N, H, L, E, M, native.FTC_F32)
+    assert 0 < nbytes <= (16 << 20)
+    q, k, v = (torch.rand(N, H, L, E, device="cuda") for _ in range(3))
+    outs = [torch.full((N, H, L, M), float("nan"), device="cuda") for _ in range(2)]
+    descs = [native.describe(t) for t in (q, k, v)]
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+    native.check(lib.ftc_causal_dot_product(*descs, native.describe(outs[0]), ws.data_ptr(), nbytes, stream),
+                 "ftc_causal_dot_product")
+    native.check(lib.ftc_causal_dot_product_static(*descs, native.describe(outs[1]), stream),
+                 "ftc_causal_dot_product_static")
+    torch.cuda.synchronize()
+    assert torch.equal(*outs) and torch.isfinite(outs[0]).all()
+
+
 def test_static_scratch_refuses_sizes_beyond_the_array():
     import os
     from fast_transformers_amd import _native as native
