@@ -58,8 +58,8 @@ auto native(F f, std::mutex *turn = nullptr) {
 int32_t dtype_code(const Tensor &t) {
     if (t.scalar_type() == at::kFloat) return FTC_F32;
     if (t.scalar_type() == at::kBFloat16) return FTC_BF16;
-    error(std::string("causal_dot_product: expected float32 or bfloat16 tensors, got torch.") +
-          at::toString(t.scalar_type()));
+    error("causal_dot_product: expected float32 or bfloat16 tensors, got " +
+          py::str(py::cast(t.scalar_type())).cast<std::string>());
 }
 
 ftc_tensor4 describe(const Tensor &t) {

@@ -862,6 +862,13 @@ def test_the_next_call_after_a_probe_reads_it(cp, monkeypatch):
     cp.check_workspaces()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float64, torch.int64], ids=str)
+def test_an_element_type_that_is_refused_is_named(cp, dtype):
+    q = torch.zeros(1, 2, 8, 16, device="cuda", dtype=dtype)
+    with pytest.raises(RuntimeError, match="got %s$" % dtype):
+        cp.causal_dot_product(q, q, q)
+
+
 def test_threads_take_turns_on_a_stream(cp):
     """Calls of several launches that hand data on through the workspace, from two threads on one
     stream: each has the results that it has alone, bit for bit."""
