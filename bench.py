@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139324950, "52d9cd11b1c5a91c"),
-    "cfg3": (2610766434, "52d9cd11b1c5a91c"),
-    "cfg5": (4973563576, "52d9cd11b1c5a91c"),
-    "wide": (1877389335, "52d9cd11b1c5a91c"),
+    "cfg2": (138957244, "3564befb816f5b16"),
+    "cfg3": (2595580585, "3564befb816f5b16"),
+    "cfg5": (4968379284, "3564befb816f5b16"),
+    "wide": (1877148925, "3564befb816f5b16"),
 }
 
 WORKLOADS = {

@@ -26,8 +26,11 @@
 //    state, every value of that operand met so far in the walk (a ceiling that only rises);
 //    for a, the values of the chunk alone.  Scaled values therefore stay below 16, values
 //    down to 2^-7 of the ceiling keep 22 bits, and the error of smaller ones is below 2^-29 of
-//    the ceiling -- for b and v the way the reference's running fp32 state treats small
-//    contributions, for a within the 32 rows of a chunk.  The ceilings come about without a
+//    the ceiling.  A ceiling is one for all columns and for the 32 rows of a chunk: where columns,
+//    or rows of one chunk, differ by more than 2^7, the small ones lose bits that fp32 sums
+//    would keep (2^-20 beside 1: off by up to 8e-2 of their own size).  Wider states, the fused
+//    attention and odd widths whose copies run elsewhere stay on kernels that hold every fp32
+//    value exactly for that.  The ceilings come about without a
 //    pass of their own: while they cut position k of the walk, the producers look at the rows
 //    of position k + 1, which they already hold in registers, and enter what they find in
 //    that position's slot in LDS with atomic maxima (for b and v only when a value reaches the
