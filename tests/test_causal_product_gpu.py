@@ -140,7 +140,7 @@ def test_wide_rows_with_states_handed_in_and_out(cp):
 
 
 CONFIG_SHAPES = {
-    # BASELINE configs 1 and 2 at full size
+    # the two smaller benchmark workloads at full size
     "cfg1": (2, 4, 512, 64, 64, 1),
     "cfg2": (10, 8, 1000, 64, 64, 2),
     # config 3's length with 2 of its 16 heads (the CPU checker needs ~1 s per head)
