@@ -28,6 +28,7 @@
 // and a pass behind it (cut_rows_kernel) cuts it by its own largest value (where no row needs it,
 // 4.6 us for 40960 rows).
 #include <algorithm>
+#include <type_traits>
 
 #include "ftc_tp_kernel.h"
 #include "ftc_tph_kernel.h"
@@ -212,7 +213,7 @@ __device__ __forceinline__ u32x4 descriptor(const void *base, uint32_t bytes) {
                  (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), kRsrcFlags};
 }
 // 16 bytes per lane from memory into LDS, lane L to byte `to` + 16 L.  (Written out: the compiler
-// does not follow which of the three buffers a request of its own fills, and would wait for all
+// does not follow which of the buffers a request of its own fills, and would wait for all
 // requests before any read of LDS.  The waits are the k-loop's.)
 __device__ __forceinline__ void load_to_lds(const u32x4 rs, uint32_t to, uint32_t offset) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
@@ -227,24 +228,24 @@ __device__ __forceinline__ void load_dword_to_lds(const u32x4 rs, uint32_t to, u
 // A workgroup of four wavefronts takes tiles of TN tokens by TF features one after the other, a
 // wavefront half of either.  v_mfma_f32_16x16x32_f16 with the features as rows of the result, so
 // that a lane has four consecutive features of one token.  A k-step's rows (128 bytes each) go from
-// memory straight into LDS, two steps ahead, through three buffers; one barrier per step.
+// memory straight into LDS through STAGES buffers, one barrier per step, and are requested STAGES
+// steps ahead; a tile's last steps request the first ones of the next tile.
 // Split: with 64 x 128 results per wavefront a step reads 24 KB of fragments for 96 matrix
-// instructions (1536 cycles); smaller tiles read more of the LDS per instruction.  By the counters of
-// 512 -> 1536 the matrix cores are busy for 43 % of the wavefronts' life, 40 % of it passes in the
-// step's wait and barrier, and LDS reads take a tenth of the cycles, without conflicts.  The three
-// buffers leave room for one workgroup per CU, so nothing else runs while a tile begins or ends:
-// the last two steps of a tile request the first two of the next one, and the rows that go out are
-// not waited for.
-template <int TN, int TF, int EPI>
+// instructions (1536 cycles); smaller tiles read more of the LDS per instruction, and are there for
+// products of few tiles (product_tile, below, where both are measured).
+template <int TN, int TF, int STAGES, int EPI>
 __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     constexpr int WT = TN / 32, WF = TF / 32;          // tiles of 16 per wavefront
     constexpr int kBuf = (TN + TF) * kRowBytes;
     constexpr int kLoadsX = TN * kRowBytes / 4096, kLoadsW = TF * kRowBytes / 4096;  // per lane
+    constexpr int kRequests = kLoadsX + kLoadsW;                                     // of a step
     constexpr int kStores = (EPI == kRelu ? 2 : 1) * WT * WF;                        // per lane
-    __shared__ __align__(16) char tiles_mem[3 * kBuf];
-    // scales and bias of a tile's tokens and features, as each wavefront needs them
-    constexpr int kScales = TN / 2 + TF;
-    __shared__ __align__(16) float scales_mem[2][4][kScales];
+    // scales and bias of a tile's tokens and features, as each wavefront needs them (64 to a request)
+    constexpr int kScaleT = TN / 2 < 64 ? 64 : TN / 2, kScaleF = TF / 2 < 64 ? 64 : TF / 2;
+    constexpr int kScales = kScaleT + 2 * kScaleF, kScaleLoads = kScales / 64;
+    static_assert(WF % 2 == 0 && TN / 2 <= 64, "the fragments of w in turn; a wavefront's tokens in a request");
+    __shared__ __align__(16) char tiles_mem[STAGES * kBuf];
+    __shared__ __align__(16) float scales_mem[4][kScales];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ln = lane & 15, g = lane >> 4;
@@ -255,9 +256,9 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     // at the same time, so that its rows are read from memory once.
     struct Tile {
         int64_t t0;
-        int f0;
+        int f0, nt, nf;
         bool there;
-        u32x4 x_rs, w_rs, xs_rs, ws_rs, b_rs;
+        u32x4 x_rs, w_rs;
     };
     auto tile_of = [&](int round) -> Tile {
         const int idx = (int)(blockIdx.x / 8) + round * (int)(gridDim.x / 8);
@@ -266,13 +267,10 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
         t.f0 = (idx % p.feature_tiles) * TF;
         t.there = t.t0 < p.tokens;
         const int64_t from = t.there ? t.t0 : 0;
-        const int nt = t.there ? (int)min((int64_t)TN, p.tokens - t.t0) : 0;
-        const int nf = t.there ? min(TF, p.features - t.f0) : 0;
-        t.x_rs = descriptor(p.x + from * row_bytes, (uint32_t)nt * row_bytes);
-        t.w_rs = descriptor(p.w + (int64_t)t.f0 * row_bytes, (uint32_t)nf * row_bytes);
-        t.xs_rs = descriptor(p.x_scale + from, (uint32_t)nt * 4u);
-        t.ws_rs = descriptor(p.w_scale + t.f0, (uint32_t)nf * 4u);
-        t.b_rs = descriptor(p.bias + t.f0, (uint32_t)nf * 4u);
+        t.nt = t.there ? (int)min((int64_t)TN, p.tokens - t.t0) : 0;
+        t.nf = t.there ? min(TF, p.features - t.f0) : 0;
+        t.x_rs = descriptor(p.x + from * row_bytes, (uint32_t)t.nt * row_bytes);
+        t.w_rs = descriptor(p.w + (int64_t)t.f0 * row_bytes, (uint32_t)t.nf * row_bytes);
         return t;
     };
     // lane's 16 bytes of a load: slot j of the tile holds piece-and-quarter (j % 8) ^ key of row j / 8
@@ -290,25 +288,30 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     lds_char *const tiles = (lds_char *)tiles_mem;
     const uint32_t lds0 = (uint32_t)(uintptr_t)tiles + 1024u * wave;
     const uint32_t scales0 = (uint32_t)(uintptr_t)(lds_char *)scales_mem + (uint32_t)(kScales * 4) * wave;
-    // request number i of a step
-    auto fetch = [&](const Tile &t, int buf, int step, int i) {
-        const uint32_t at = (uint32_t)step * kRowBytes, to = lds0 + (uint32_t)buf * kBuf;
+    // The step whose rows are requested: STAGES steps ahead of the one that is computed, in this
+    // tile or in a later one.
+    Tile ahead = tile_of(0);
+    int ahead_step = 0, ahead_round = 0;
+    auto fetch = [&](uint32_t buf, int i) {  // request number i of that step
+        const uint32_t at = (uint32_t)ahead_step * kRowBytes, to = lds0 + buf;
         if (i < kLoadsX)
-            load_to_lds(t.x_rs, to + 4096u * i, x_off[i] + at);
+            load_to_lds(ahead.x_rs, to + 4096u * i, x_off[i % kLoadsX] + at);
         else
-            load_to_lds(t.w_rs, to + TN * kRowBytes + 4096u * (i - kLoadsX), w_off[(i - kLoadsX) % kLoadsW] + at);
+            load_to_lds(ahead.w_rs, to + TN * kRowBytes + 4096u * (i - kLoadsX), w_off[(i - kLoadsX) % kLoadsW] + at);
     };
-    constexpr int kRequests = kLoadsX + kLoadsW;
-    // (before the first step's, so that whoever waits for its rows waits for the scales too)
-    auto fetch_scales = [&](const Tile &t, int round) {
-        static_assert(TN == 128 && TF % 128 == 0, "64 tokens, TF / 2 features per wavefront");
-        const uint32_t to = scales0 + (uint32_t)(round & 1) * (4 * kScales * 4);
-        load_dword_to_lds(t.xs_rs, to, 4u * (uint32_t)(wt * (TN / 2) + lane));
+    auto advance = [&]() {
+        if (++ahead_step == steps) ahead_step = 0, ahead = tile_of(++ahead_round);
+    };
+    auto fetch_scales = [&](const Tile &t) {
+        const u32x4 xs_rs = descriptor(p.x_scale + t.t0, (uint32_t)t.nt * 4u),
+                    ws_rs = descriptor(p.w_scale + t.f0, (uint32_t)t.nf * 4u),
+                    b_rs = descriptor(p.bias + t.f0, (uint32_t)t.nf * 4u);
+        load_dword_to_lds(xs_rs, scales0, 4u * (uint32_t)(wt * (TN / 2) + lane));
 #pragma unroll
-        for (int i = 0; i < TF / 128; i++) {
+        for (int i = 0; i < kScaleF / 64; i++) {
             const uint32_t from = 4u * (uint32_t)(wf * (TF / 2) + 64 * i + lane);
-            load_dword_to_lds(t.ws_rs, to + 4u * (TN / 2 + 64 * i), from);
-            load_dword_to_lds(t.b_rs, to + 4u * (TN / 2 + TF / 2 + 64 * i), from);
+            load_dword_to_lds(ws_rs, scales0 + 4u * (kScaleT + 64 * i), from);
+            load_dword_to_lds(b_rs, scales0 + 4u * (kScaleT + kScaleF + 64 * i), from);
         }
     };
     int x_addr[2], w_addr[2];  // [piece]; further tiles 16 rows of 128 bytes on
@@ -317,88 +320,139 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
         x_addr[k] = TpSwizzle<128>::addr(wt * (TN / 2) + ln, 64 * k + 16 * g);
         w_addr[k] = TN * kRowBytes + TpSwizzle<128>::addr(wf * (TF / 2) + ln, 64 * k + 16 * g);
     }
+    // requests in flight of later steps than the next one
+    constexpr int kFlying = (STAGES - 2) * kRequests;
     f32x4 acc[WF][WT];
-    // (written out in issue order: fragments of the next feature tile and a request for a later step
-    // under the matrix instructions of this one, instructions that add to one accumulator at least
-    // WT apart)
-    auto compute = [&](const lds_char *buf, auto request) {
-        Frag xf[WT][2], w[2][2];
-        w[0][1] = lds_frag16(buf + w_addr[1]);
+    Frag xh[WT], xl[WT], w[2][2];
+    auto first_frags = [&](const lds_char *buf) {
 #pragma unroll
-        for (int j = 0; j < WT; j++) xf[j][0] = lds_frag16(buf + x_addr[0] + j * 16 * kRowBytes);
-        w[0][0] = lds_frag16(buf + w_addr[0]);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int k = 1; k >= 0; k--) {
+            w[0][k] = lds_frag16(buf + w_addr[k]);
+#pragma unroll
+            for (int j = 0; j < WT; j++) (k ? xh[j] : xl[j]) = lds_frag16(buf + x_addr[1 - k] + j * 16 * kRowBytes);
+        }
+    };
+    // One step, written out in issue order: fragments of the next feature tile and a request for a
+    // later step under the matrix instructions of this one, instructions that add to one
+    // accumulator at least WT apart.  The barrier stands before the last feature tile's
+    // instructions: the wavefront has read all it needs of this step's buffer by then, and under
+    // those instructions the first fragments of the next step arrive, whose rows the wait
+    // before the barrier has seen land.  Of the requests of the step that takes this buffer over,
+    // the first ones run under the same instructions and the others under the next step's; those
+    // of a tile's last step all before the rows go out, so that no later wait for them waits for
+    // the rows.
+    auto compute = [&](const lds_char *buf, const lds_char *next, uint32_t to_now, uint32_t to_before, auto first,
+                       auto last, auto wait) {
+        constexpr int kSlots = 3 * WF;
+        static_assert(kSlots >= kRequests, "a request per group of matrix instructions");
+        auto slot_of = [](int r) -> int { return r * kSlots / kRequests; };
+        Frag xn[WT];
 #pragma unroll
         for (int i = 0; i < WF; i++) {
+            if (i == WF - 1) {
+                wait();
+                advance();
+            }
 #pragma unroll
             for (int m = 0; m < 3; m++) {
-                if (i == 0 && m == 0) {
+                if (i + 1 < WF) {
+                    if (m > 0) w[(i + 1) % 2][2 - m] = lds_frag16(buf + w_addr[2 - m] + (i + 1) * 16 * kRowBytes);
+                } else if (m < 2) {
+                    w[0][1 - m] = lds_frag16(next + w_addr[1 - m]);
+                    if (m == 0) {
 #pragma unroll
-                    for (int j = 0; j < WT; j++) xf[j][1] = lds_frag16(buf + x_addr[1] + j * 16 * kRowBytes);
+                        for (int j = 0; j < WT; j++) xn[j] = lds_frag16(next + x_addr[0] + j * 16 * kRowBytes);
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < WT; j++) xl[j] = lds_frag16(next + x_addr[1] + j * 16 * kRowBytes);
                 }
-                if (m > 0 && i + 1 < WF)
-                    w[(i + 1) % 2][2 - m] = lds_frag16(buf + w_addr[2 - m] + (i + 1) * 16 * kRowBytes);
-                if (i * 3 + m < kRequests) request(i * 3 + m);
+                const int slot = i == WF - 1 ? m : 3 + 3 * i + m;
+#pragma unroll
+                for (int r = 0; r < kRequests; r++) {
+                    if (i == WF - 1 ? (decltype(last)::value ? r * 3 / kRequests == m : slot_of(r) == slot)
+                                    : !decltype(first)::value && slot_of(r) == slot)
+                        fetch(i == WF - 1 ? to_now : to_before, r);
+                }
 #pragma unroll
                 for (int j = 0; j < WT; j++)
-                    acc[i][j] = mfma16h(w[i % 2][m == 0 ? 1 : 0], xf[j][m == 1 ? 1 : 0], acc[i][j]);
+                    acc[i][j] = mfma16h(w[i % 2][m == 0 ? 1 : 0], m == 1 ? xl[j] : xh[j], acc[i][j]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+#pragma unroll
+        for (int j = 0; j < WT; j++) xh[j] = xn[j];
     };
-    static_assert(3 * WF >= kRequests, "a request per group of matrix instructions");
+    if (!ahead.there) return;
+#pragma unroll
+    for (int s = 0; s < STAGES; s++) {
+#pragma unroll
+        for (int i = 0; i < kRequests; i++) fetch((uint32_t)s * kBuf, i);
+        if (s + 1 < STAGES) advance();
+    }
     float bound_w = 0.f, bound_b = 0.f, least_w = __builtin_inff();
     if (EPI == kRelu) {  // (the same numbers in every workgroup)
+#pragma unroll 4
         for (int i = lane; i < p.features; i += 64) {
-            bound_w = fmaxf(bound_w, p.w_norm[i]);
-            bound_b = fmaxf(bound_b, p.bias[i]);  // (a bias below zero, lowest or -inf, raises nothing)
+            const float norm = p.w_norm[i], bias = p.bias[i];
+            bound_w = fmaxf(bound_w, norm);
+            bound_b = fmaxf(bound_b, bias);  // (a bias below zero, lowest or -inf, raises nothing)
             // (a feature without weights and with no bias above zero is zero in any row)
-            least_w = fminf(least_w, p.w_norm[i] == 0.f && !(p.bias[i] > 0.f) ? __builtin_inff() : p.w_norm[i]);
+            least_w = fminf(least_w, norm == 0.f && !(bias > 0.f) ? __builtin_inff() : norm);
         }
         bound_w = wave_largest(bound_w), bound_b = wave_largest(bound_b);
         least_w = -wave_largest(-least_w);
     }
-    Tile t = tile_of(0);
-    if (!t.there) return;
-    fetch_scales(t, 0);
-#pragma unroll
-    for (int i = 0; i < 2 * kRequests; i++) fetch(t, i / kRequests, i / kRequests, i % kRequests);
-    int now = 0;
-    for (int round = 0; t.there; round++) {
-        const Tile next = tile_of(round + 1);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((STAGES - 1) * kRequests) : "memory");
+    first_frags(tiles);
+    uint32_t now = 0;
+    auto after = [&](uint32_t buf) -> uint32_t { return buf == (STAGES - 1) * kBuf ? 0u : buf + kBuf; };
+    for (int round = 0;; round++) {
+        const Tile t = tile_of(round);
+        if (!t.there) break;
+        fetch_scales(t);
 #pragma unroll
         for (int i = 0; i < WF; i++)
 #pragma unroll
             for (int j = 0; j < WT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        uint32_t before = 0;
         for (int s = 0; s < steps; s++) {
-            // This step's rows have landed (in flight: the next step's requests and, in the first
-            // two steps of a tile, the rows that the tile before has sent out), and every wavefront
-            // is done with the buffer that the step after the next one goes to.
-            constexpr int kFirst = kRequests + kStores < 63 ? kRequests + kStores : 63;
-            if (s < 2 && round > 0)
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFirst) : "memory");
+            // The next step's rows have landed (in flight: those of the steps after it and, where
+            // these steps were all requested before the rows of the tile before went out, those
+            // rows and this tile's scales), and every wavefront has what it needs of this
+            // step's buffer.
+            const bool rows_fly = round > 0 && s < STAGES - 1 && steps >= STAGES;
+            auto wait = [&]() {
+                constexpr int kMore = kFlying + kStores + kScaleLoads < 63 ? kFlying + kStores + kScaleLoads : 63;
+                if (rows_fly)
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kMore) : "memory");
+                else
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFlying) : "memory");
+            };
+            const uint32_t later = after(now);
+            constexpr std::true_type yes{};
+            constexpr std::false_type no{};
+            if (s == 0)
+                compute(tiles + now, tiles + later, now, before, yes, no, wait);
+            else if (s + 1 < steps)
+                compute(tiles + now, tiles + later, now, before, no, no, wait);
             else
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kRequests) : "memory");
-            const int later = now == 0 ? 2 : now - 1;
-            if (s + 2 < steps) {
-                compute(tiles + now * kBuf, [&](int i) { fetch(t, later, s + 2, i); });
-            } else {
-                if (s + 2 == steps) fetch_scales(next, round + 1);
-                compute(tiles + now * kBuf, [&](int i) { fetch(next, later, s + 2 - steps, i); });
-            }
-            now = now == 2 ? 0 : now + 1;
+                compute(tiles + now, tiles + later, now, before, no, yes, wait);
+            before = now;
+            now = later;
         }
+        // (this tile's scales: seen to have landed by the steps' waits where there are enough of them)
+        if (steps <= STAGES) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // ---- rows out: every store is made, those outside the tensor outside the descriptor, so
         // that their number is known to the waits above ----
-        const int nt = (int)min((int64_t)TN, p.tokens - t.t0);
         const uint32_t out_row = (uint32_t)p.features * 4u;
         const __amdgpu_buffer_rsrc_t o_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (EPI == kRelu ? (char *)p.out_pieces : (char *)p.out) + t.t0 * out_row, 0, (uint32_t)nt * out_row,
+            (EPI == kRelu ? (char *)p.out_pieces : (char *)p.out) + t.t0 * out_row, 0, (uint32_t)t.nt * out_row,
             kRsrcFlags);
         const __amdgpu_buffer_rsrc_t r_rs = __builtin_amdgcn_make_buffer_rsrc(
             (char *)(EPI == kResidual ? p.residual : p.bias) + (EPI == kResidual ? t.t0 * out_row : 0), 0,
-            (uint32_t)nt * out_row, kRsrcFlags);
-        const float *const scales = scales_mem[round & 1][wave];
+            (uint32_t)t.nt * out_row, kRsrcFlags);
+        const float *const scales = scales_mem[wave];
         float xs[WT], s_out[WT];
         uint32_t at[WT];
 #pragma unroll
@@ -429,8 +483,8 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
         for (int i = 0; i < WF; i++) {
             const int fl = 16 * i + 4 * g, f = t.f0 + wf * (TF / 2) + fl;
             const bool f_in = f < p.features;
-            const float4 ws = *(const float4 *)(scales + TN / 2 + fl),
-                         b = *(const float4 *)(scales + TN / 2 + TF / 2 + fl);
+            const float4 ws = *(const float4 *)(scales + kScaleT + fl),
+                         b = *(const float4 *)(scales + kScaleT + kScaleF + fl);
             if (EPI == kResidual && i + 2 < WF) residual(i + 2);
 #pragma unroll
             for (int j = 0; j < WT; j++) {
@@ -462,9 +516,55 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        t = next;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the requests of a tile that is not there)
+}
+
+template <int TN, int TF, int STAGES, int PER_CU>
+void launch_product(LinearArgs a, hipStream_t stream) {
+    a.feature_tiles = (int32_t)((a.features + TF - 1) / TF);
+    const int64_t token_tiles = (a.tokens + TN - 1) / TN;
+    // (a multiple of the eight XCDs)
+    const int64_t tiles = (token_tiles + 7) / 8 * a.feature_tiles;
+    const dim3 grid((unsigned)(8 * std::min<int64_t>(tiles, 32 * PER_CU))), block(256);
+    if (a.out_pieces)
+        hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kRelu>), grid, block, 0, stream, a);
+    else if (a.residual)
+        hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kResidual>), grid, block, 0, stream, a);
+    else
+        hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kPlain>), grid, block, 0, stream, a);
+}
+
+// Which tile a product runs on.  A workgroup's k-step takes the time below (us; two workgroups on a
+// CU: together, and one alone), a tile's rows out the third number, and the launch lasts as long as
+// its busiest XCD of 32 CUs.  Measured (us, 128 x 256 / 64 x 128 / 64 x 64 / 32 x 64; the library's
+// product is none of these):
+//   40960 tokens, 512 -> 1536   230 / 249 / 289 / 385     1352 tokens, 1024 -> 512  46 / 20 / 15 / 15
+//   40960 tokens, 1024 -> 512   166 / 164 / 200 / 263     169 tokens, 1024 -> 256   46 / 19 / 14 / 11
+//   12000 tokens, 256 -> 768     32 /  23 /  24 /  34     169 tokens, 256 -> 768    16 / 7.1 / 5.7 / 4.8
+// On few tiles a step is the latency of its barrier, its LDS reads and its matrix instructions one
+// after the other, so the smallest tile has the shortest; on many the large tile reads the least of
+// the L2 and the LDS per matrix instruction (its rate there, 0.83 PFLOP/s of fp16 pieces, rises by a
+// fifth on operands of zeros: the clock under that load is part of the bound).
+struct ProductTile {
+    int tokens, features, per_cu;
+    double step, step_alone, rows;
+};
+constexpr ProductTile kProductTiles[] = {
+    {128, 256, 1, 1.65, 1.65, 3.0}, {64, 128, 2, 0.95, 0.50, 1.5}, {64, 64, 2, 0.57, 0.31, 1.0}, {32, 64, 2, 0.40, 0.21, 0.7}};
+int product_tile(int64_t tokens, int64_t features, int64_t steps) {
+    int best = 0;
+    double least = 0;
+    for (int i = 0; i < 4; i++) {
+        const ProductTile &t = kProductTiles[i];
+        const int64_t token_tiles = (tokens + t.tokens - 1) / t.tokens;
+        const int64_t tiles = (token_tiles + 7) / 8 * ((features + t.features - 1) / t.features);
+        const int64_t round = 32 * t.per_cu, left = tiles % round;
+        const double us = (double)(tiles / round + (left > 32)) * ((double)steps * t.step + t.rows) +
+                          (left > 0 && left <= 32 ? (double)steps * t.step_alone + t.rows : 0.);
+        if (i == 0 || us < least) least = us, best = i;
+    }
+    return best;
 }
 
 int launched(const char *what) {
@@ -550,25 +650,22 @@ int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const 
         features > kMostColumns || (relu_pieces && features % kStep != 0))
         return fail(FTC_ERR_UNSUPPORTED, "a product of %lld columns and %lld features", (long long)k, (long long)features);
     if (tokens <= 0) return FTC_OK;
-    constexpr int TN = 128, TF = 256;
     LinearArgs a;
     a.x = (const char *)x, a.w = (const char *)w, a.x_scale = x_scale, a.w_scale = w_scale, a.bias = bias;
     a.w_norm = w_norm, a.residual = residual, a.out = out, a.out_pieces = (char *)relu_pieces;
     a.out_scale = relu_scale, a.tokens = tokens, a.features = (int32_t)features, a.k = (int32_t)k;
-    a.feature_tiles = (int32_t)((features + TF - 1) / TF);
-    const int64_t token_tiles = (tokens + TN - 1) / TN;
-    // (one workgroup per CU, a multiple of the eight XCDs)
-    const int64_t tiles = (token_tiles + 7) / 8 * a.feature_tiles;
-    const dim3 grid((unsigned)(8 * std::min<int64_t>(tiles, 32))), block(256);
+    const hipStream_t on = (hipStream_t)stream;
+    switch (product_tile(tokens, features, k / kStep)) {
+    case 0: launch_product<128, 256, 3, 1>(a, on); break;
+    case 1: launch_product<64, 128, 3, 2>(a, on); break;
+    case 2: launch_product<64, 64, 4, 2>(a, on); break;
+    default: launch_product<32, 64, 4, 2>(a, on); break;
+    }
     if (relu_pieces) {
-        hipLaunchKernelGGL((linear_kernel<TN, TF, kRelu>), grid, block, 0, (hipStream_t)stream, a);
         const dim3 cuts((unsigned)((tokens + 4 * kCutRows - 1) / (4 * kCutRows)));
-        hipLaunchKernelGGL(cut_rows_kernel, cuts, block, 0, (hipStream_t)stream, a.out_pieces, relu_scale, tokens,
+        hipLaunchKernelGGL(cut_rows_kernel, cuts, dim3(256), 0, on, a.out_pieces, relu_scale, tokens,
                            (int)features);
-    } else if (residual)
-        hipLaunchKernelGGL((linear_kernel<TN, TF, kResidual>), grid, block, 0, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL((linear_kernel<TN, TF, kPlain>), grid, block, 0, (hipStream_t)stream, a);
+    }
     return launched("product");
 }
 

@@ -82,6 +82,42 @@ def test_products_in_pieces(shape):
         assert ((whole(hp, hs) - want).abs() <= bound + 2.0 ** -22 * want + 2.0 ** -39 * largest).all()
 
 
+@pytest.mark.parametrize("shape", [
+    # the four tiles a product is cut into: more tiles than workgroups and fewer, rows and features that
+    # end inside a tile, steps fewer and more than a tile's buffers
+    (4990, 512, 1540), (9990, 160, 1536), (4100, 160, 288), (16500, 64, 288), (70001, 96, 260), (129, 96, 544),
+    (33, 64, 64)], ids=lambda s: "t%d_k%d_f%d" % s)
+def test_products_are_the_same_on_every_tile(shape):
+    """A result is a sum in one order whatever tile it lies in: the last rows in a product of their
+    own, on the smallest tile, come out bit for bit as in the whole one."""
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    T, K, F = shape
+    few = min(T, 31)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x, w, b, r = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, K), (F, K), (F,), (T, F)))
+    new = lambda *s: torch.full(s, float("nan"), device="cuda")
+    xp, xs, wp, ws, bo, wn = new(T, K), new(T), new(F, K), new(F), new(F), new(F)
+    item = Weight(w.data_ptr(), b.data_ptr(), F, K, wp.data_ptr(), ws.data_ptr(), bo.data_ptr(), wn.data_ptr())
+    assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == 0, _native.last_error()
+    assert lib.ftc_split_rows(ptr(x), ctypes.c_int64(T), ctypes.c_int64(K), ptr(xp), ptr(xs), stream()) == 0
+
+    def run(first, residual=None, relu=False):
+        out, scale = new(T - first, F), new(T - first)
+        rc = lib.ftc_linear_split(ptr(xp[first:]), ptr(xs[first:]), ctypes.c_int64(T - first), ptr(wp), ptr(ws),
+                                  ptr(bo), ptr(wn), ctypes.c_int64(F), ctypes.c_int64(K),
+                                  ptr(residual[first:]) if residual is not None else None, None if relu else ptr(out),
+                                  ptr(out) if relu else None, ptr(scale) if relu else None, stream())
+        assert rc == 0, _native.last_error()
+        return out, scale
+    for more in ({}, {"residual": r}) + (({"relu": True},) if F % 32 == 0 else ()):
+        (all_rows, all_scales), (rows, scales) = run(0, **more), run(T - few, **more)
+        if "relu" in more:
+            assert torch.equal(all_scales[T - few:], scales) and (all_scales > 0).all()
+            all_rows, rows = whole(all_rows, all_scales), whole(rows, scales)
+        assert not all_rows.isnan().any() and torch.equal(all_rows[T - few:], rows)
+
+
 def test_relu_keeps_nan_and_takes_any_bias_below_zero():
     """Features switched off by a bias of the type's lowest value or -inf leave the other features'
     precision alone; NaN in a weight or a bias comes out as NaN, as from torch's relu."""
