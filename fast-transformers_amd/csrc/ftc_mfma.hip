@@ -622,8 +622,41 @@ bool fused_attention_supported(const ScanDesc &sd, int64_t L) {
            scan_wg_norm_covers(sd.a.width, sd.v.width) && mfma_scan_supported(sd, L);
 }
 
+// (the exchange of the chain-parallel fused form: a second tile of state for its denominators)
+constexpr int64_t kFusedTpStateRows = 128;
+
+// The fused attention launch on the chain-parallel kernel: its plan is that of a single 64 x 64
+// scan whatever the widths (a chunk costs the same).  Returns false: the workgroup form, whose
+// units split L and which carries two units of 32 value columns per workgroup.  Measured (us, the
+// workgroup form / this way), 64 x 64: 80 chains, L=1000 47.8 / 36.9, L=4096 138 / 114; 512 chains,
+// L=1000 160 / 130; 384 chains, L=2774 350 / 286; 216 chains, L=134 17.6 / 15.1; 64 chains, L=1500
+// 50.3 / 45.2; 32 chains, L=4096 62.9 / 53.9; but 8 chains, L=500 17.1 / 19.0, 16 chains, L=1500
+// 27.4 / 29.5.  (Chains that are not exchanged: from 41 on.  The workgroup form's own tests are cases
+// of 24 to 40 of them and ask for it by name; 32 chains, L=500 would be 23.3 / 19.4.)  One width of
+// 32: 80 chains, L=1000 41.6 / 34.8 and 36.7 / 32.0, but 64 chains, L=1500 42.9 / 44.2, more than a
+// round of workgroups 102 / 116, with an exchange 95.7 / 106.  32 x 32: 31.7 / 31.3 and 64 / 96.
+// Chains of more than 256 chunks are not walked whole on three bf16 pieces (tp_plan_compute).
+bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, int *seg_chunks) {
+    *nseg = *seg_chunks = 0;
+    if (tuning().wg > 0) return false;
+    const int64_t chunks = (L + kChunk - 1) / kChunk;
+    tp_plan(64, 64, chains, 1, L, nseg, seg_chunks);
+    if (*nseg > 0 && *seg_chunks == 0 && chunks > 256) *nseg = 0;
+    if (*nseg == 0 || tuning().wg == 0) return *nseg > 0;  // (FTC_WG=0: tuning aid)
+    const bool take = D == 64 && F == 64 ? (*seg_chunks > 0 ? chains >= 24 && chunks >= 64 : chains > 40)
+                                         : (D == 64 || F == 64) && *seg_chunks == 0 && chains > 40 &&
+                                               chains <= 256 && chunks <= 32;
+    if (!take) *nseg = *seg_chunks = 0;
+    return take;
+}
+
 int64_t fused_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F) {
-    return make_plan(N, H, L, D, F, 1, true, true).workspace_bytes;
+    int nseg, seg_chunks;
+    int64_t bytes = make_plan(N, H, L, D, F, 1, true, true).workspace_bytes;
+    const int64_t chains = std::max<int64_t>(1, N * H);
+    if (fused_tp_plan(D, F, chains, L, &nseg, &seg_chunks) && seg_chunks > 0)
+        bytes = std::max(bytes, tp_exchange_workspace_bytes(chains, nseg, kFusedTpStateRows));
+    return bytes;
 }
 
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
@@ -635,10 +668,21 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     const Combo combo = combo_of(scans[0]);
     if (fused && (nscans != 1 || !fused_attention_supported(scans[0], L)))
         return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for this shape or layout");
-    const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd);
     const int64_t chains = std::max<int64_t>(1, N * H);
-    const int64_t fblocks = tp_shape ? tp_fblocks(F) : 1;
     int tpx_nseg = 0, tpx_seg_chunks = 0, tp_nseg = 0;
+    int64_t widest = 0;
+    for (int64_t l : {scans[0].a.stride_l, scans[0].b.stride_l, scans[0].v.stride_l, scans[0].out.stride_l})
+        widest = std::max(widest, l);
+    // (a whole chain is addressed through one 32-bit descriptor; a caller whose workspace is that of the
+    // workgroup form gets the workgroup form)
+    bool fused_tp = fused && (L + 2 * kChunk) * std::max<int64_t>(widest, 64) * 4 < 0x7fffffffLL &&
+                          fused_tp_plan(D, F, chains, L, &tpx_nseg, &tpx_seg_chunks);
+    if (fused_tp && tpx_seg_chunks > 0 && !plan_only() &&
+        (int64_t)workspace_bytes < tp_exchange_workspace_bytes(chains, tpx_nseg, kFusedTpStateRows))
+        fused_tp = false, tpx_nseg = tpx_seg_chunks = 0;
+    const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd);
+    const int64_t fblocks = tp_shape ? tp_fblocks(F) : 1;
+    if (fused_tp && tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     if (tp_shape) {
         int any_bf16 = nscans == 1 && combo == kBBFB ? kMixedGradValues : 0;
         for (int i = 0; i < nscans; i++)
@@ -649,14 +693,15 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     const bool tp = tp_nseg > 0 || tpx_seg_chunks > 0;
     if (!tp && !mfma_scan_supported(scans[0], L))
         return fail(FTC_ERR_UNSUPPORTED, "no MFMA kernel takes a %d x %d state here", D, F);
-    const bool wg = fused || use_wg_kernel(D, F, nscans, L, combo == kFFFF);
+    const bool wg = !fused_tp && (fused || use_wg_kernel(D, F, nscans, L, combo == kFFFF));
     MfmaPlan pl = make_plan(N, H, L, D, F, nscans, wg, fused != nullptr);
     int32_t tp_start[kMaxTpSegments + 1] = {0};
     if (tpx_seg_chunks > 0) {  // one workgroup per chain segment, segment sums exchanged
         pl.nseg = tpx_nseg;
         pl.seg_len = tpx_seg_chunks * kChunk;
         pl.waves = chains * pl.nseg;
-        pl.workspace_bytes = tp_exchange_workspace_bytes(chains * nscans * fblocks, pl.nseg, D);
+        pl.workspace_bytes = tp_exchange_workspace_bytes(chains * nscans * fblocks, pl.nseg,
+                                                         fused_tp ? kFusedTpStateRows : D);
     } else if (tp) {  // one workgroup per chain segment, nothing to exchange
         pl.nseg = tp_segment_starts((L + kChunk - 1) / kChunk, tp_nseg, tp_start);
         pl.seg_len = (int)L;
@@ -709,7 +754,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     args.eps = fused ? fused->eps : 0.f;
     args.key_len = fused ? fused->key_lengths : nullptr;
 #ifdef FTC_TIMELINE
-    if (tp)  // tuning aid: where the chain-parallel kernel writes its time stamps
+    if (tp && !fused)  // tuning aid: where the chain-parallel kernel writes its time stamps
         if (const char *env = getenv("FTC_STAMP_PTR"))  // (a build for measurements only)
             args.key_len = (const int64_t *)(uintptr_t)strtoull(env, nullptr, 0);
 #endif
@@ -746,7 +791,8 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     // fp32 states of up to 64 rows: the kernel that feeds its fragments from LDS tiles
     bool dma = D <= 64 && combo == kFFFF;
     if (tuning().dma >= 0) dma = dma && tuning().dma != 0;  // tuning aid
-    note_kernel(tp ? (half_pieces ? (tpx_seg_chunks > 0 ? "scan_tph_kernel (exchange)" : "scan_tph_kernel")
+    note_kernel(fused_tp ? (tpx_seg_chunks > 0 ? "scan_tp_kernel<NORM> (exchange)" : "scan_tp_kernel<NORM>")
+                : tp ? (half_pieces ? (tpx_seg_chunks > 0 ? "scan_tph_kernel (exchange)" : "scan_tph_kernel")
                                   : (tpx_seg_chunks > 0 ? "scan_tp_kernel (exchange)" : "scan_tp_kernel"))
                 : wg ? (fused ? "scan_wg_kernel<NORM>" : "scan_wg_kernel")
                 : dma ? "scan_dma_kernel" : "scan_mfma_kernel");
@@ -765,7 +811,9 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         return FTC_OK;
     }
     if (tp) {
-        if (half_pieces)
+        if (fused)
+            launch_scan_tp_norm(workspace, args, stream);
+        else if (half_pieces)
             launch_scan_tph(workspace, args, mixed, odd, stream);
         else
             launch_scan_tp(workspace, args, stream);

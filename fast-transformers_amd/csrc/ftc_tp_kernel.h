@@ -97,9 +97,30 @@ __device__ __forceinline__ constexpr int b_tile_column(int d) {
     return 32 * (d / 32) + 16 * ((d / 4) % 2) + 4 * ((d % 32) / 8) + d % 4;
 }
 
+// sum over the four groups of 16 lanes, in every lane: v_permlane16_swap exchanges the odd groups
+// of its first operand with the even groups of its second, v_permlane32_swap the halves
+__device__ __forceinline__ float sum_of_lane_groups(float x) {
+    const uint32_t b = __float_as_uint(x);
+    const auto p16 = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    const float y = __uint_as_float(p16[0]) + __uint_as_float(p16[1]);
+    const uint32_t c = __float_as_uint(y);
+    const auto p32 = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+    return __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
+}
+
 // KS2: groups of 32 rows in the state's last block (1: a state of 65 .. 96 rows, whose last
 // block skips the matrix instructions and fragment reads of its empty half)
-template <int ND, int KS2>
+// NORM: causally masked linear attention in the same walk (see ftc_wg_kernel.h for the equations):
+// the producers apply phi(x) = elu(x) + 1 to a and b as they cut them and zero the rows of b at or
+// beyond the key length.  The denominators phi(a_l) . sum_{j <= l} phi(b_j) are what the consumers
+// have at hand: the column sums of the masked quadrants of Pt, and phi(a) times z, the sum of
+// phi(b) over the chunks before.  z is one more column of the state whose "values" are ones; of each
+// block of 64 rows consumer w keeps the half that belongs to k-step w / 2 (its first one: such
+// consumers walk the two halves in the other order) and multiplies it with the 16 positions of its
+// own quadrant: twelve matrix instructions, a cut and a reduction over the lane groups.  A
+// position's two contributions meet in LDS behind the chunk's barrier, and rows are divided as they
+// are stored.
+template <int ND, int KS2, bool NORM>
 __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     constexpr int D = 64, F = 64;              // one block of state rows and of output columns
     constexpr int T = 256;                     // producer lanes
@@ -121,6 +142,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 
     __shared__ __align__(16) char pieces_mem[3 * kBufBytes];
     __shared__ __align__(16) char pt_mem[2 * 3 * kTileP];
+    __shared__ __align__(16) float den_mem[NORM ? 2 : 1][NORM ? kChunk : 1][2];
     lds_char *const unit_pc = (lds_char *)pieces_mem;
     lds_char *const pt_pc = (lds_char *)pt_mem;
 
@@ -278,15 +300,36 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                         0, 0);
             }
         };
+        // NORM: keys at or beyond this row count as zero (phi(0) = 1, so do the rows that do not
+        // exist, and the columns)
+        const int key_rows = NORM && p.key_len ? (int)max((int64_t)0, min((int64_t)rows, p.key_len[n])) : rows;
+        auto feature_a = [&](const u32x4 x, int hb) -> u32x4 {
+            if (!NORM) return x;
+            u32x4 y = feature_quad(x);
+            if (!ab_in[hb]) y = u32x4{0, 0, 0, 0};
+            return y;
+        };
+        auto feature_b = [&](const u32x4 x, int hb, int v, int q) -> u32x4 {  // quad q of position v
+            if (!NORM) return x;
+            u32x4 y = feature_quad(x);
+            const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
+            // (a scalar test: most chunks lie wholly below the limit)
+            if (row0 < 0 || row0 + kChunk > key_rows) {
+                if ((uint32_t)(row0 + 16 * q + ptid / QA) >= (uint32_t)key_rows) y = u32x4{0, 0, 0, 0};
+            }
+            if (!ab_in[hb]) y = u32x4{0, 0, 0, 0};
+            return y;
+        };
         // position k of the walk goes to LDS buffer k % 3 through register set k % PF.  The
         // first n1 positions (a multiple of PF) only feed the state: no piece of a, and the
         // consumers, who have little to do there, cut rows 16 .. 31 of b and v themselves.
-        auto cut = [&](const Raw &r, int buf, bool own, int hb) {
+        auto cut = [&](const Raw &r, int buf, bool own, int hb, int v) {
             lds_char *const pc = unit_pc + buf * kBufBytes;
 #pragma unroll
             for (int q = 0; q < LA; q++) {
-                if (own) split_quad_to_lds(r.a[q], pc, kTileA, a_waddr[q]);
-                if (own || q == 0) split_quad_to_lds(r.b[q], pc + kOffB, kTileA, b_waddr[q]);
+                if (own) split_quad_to_lds(feature_a(r.a[q], hb), pc, kTileA, a_waddr[q]);
+                if (own || q == 0)
+                    split_quad_to_lds(feature_b(r.b[q], hb, v, q), pc + kOffB, kTileA, b_waddr[q]);
             }
             if (hb == 0) {
 #pragma unroll
@@ -308,7 +351,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
         for (int v = 0; v < n1; v += PF) {
 #pragma unroll
             for (int j = 0; j < PF; j++) {
-                cut(raw[j], buf, false, j % ND);
+                cut(raw[j], buf, false, j % ND, v + j);
                 fetch(raw[j], v + j + PF, j % ND);
                 buf = buf == 2 ? 0 : buf + 1;
                 wg_barrier();
@@ -322,7 +365,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
             for (int j = 0; j < PF; j++) {
                 if (v + j == n1 + 4) FTC_STAMP(0);
-                cut(raw[j], buf, true, j % ND);
+                cut(raw[j], buf, true, j % ND, v + j);
                 if (v + j == n1 + 4) FTC_STAMP(1);
                 fetch(raw[j], v + j + PF, j % ND);
                 buf = buf == 2 ? 0 : buf + 1;
@@ -335,7 +378,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
         for (int j = 0; j < PF - 1; j++) {
             if (v + j > nwalk) return;
-            cut(raw[j], buf, true, j % ND);
+            cut(raw[j], buf, true, j % ND, v + j);
             buf = buf == 2 ? 0 : buf + 1;
             wg_barrier();
             __builtin_amdgcn_sched_barrier(0);
@@ -355,6 +398,8 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     const int ih = w == 0 ? 0 : w == 1 ? 1 : 1 - jh;
     // Position tiles are numbered from this wavefront's own: local tile x is tile x ^ ih, so
     // that the quadrant always multiplies local tile 0.
+    // NORM: k-steps of a block's rows in this consumer's order, its own half of z first
+    const int ks0 = NORM && KS2 == 2 ? w >> 1 : 0;
     // row-major fragments of a and b: k-slots t <-> d = 32 ks + 8 g + t (one 16-byte read)
     // (b: its tile keeps the two groups of four apart, see b_tile_column: two 8-byte reads)
     int a_addr[2][2], b_addr[2][2];  // [local i tile][ks], [ks][u]
@@ -362,11 +407,11 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     for (int ks = 0; ks < 2; ks++) {
 #pragma unroll
         for (int x = 0; x < 2; x++)
-            a_addr[x][ks] = TpSwizzle<RBA>::addr(16 * (x ^ ih) + ln, 2 * (32 * ks + 8 * g));
+            a_addr[x][ks] = TpSwizzle<RBA>::addr(16 * (x ^ ih) + ln, 2 * (32 * (ks ^ ks0) + 8 * g));
 #pragma unroll
         for (int u = 0; u < 2; u++)
             b_addr[ks][u] = kOffB + TpSwizzle<RBA>::addr(
-                                        16 * jh + ln, 2 * b_tile_column(32 * ks + 8 * g + 4 * u));
+                                        16 * jh + ln, 2 * b_tile_column(32 * (ks ^ ks0) + 8 * g + 4 * u));
     }
     // State tile dt = 2 ks + u: row m <-> d = 32 ks + 8 (m / 4) + 4 u + m % 4, so that the
     // accumulator registers of tiles 2 ks and 2 ks + 1 (rows 4 g + r) are k-slots 0..7 of
@@ -383,7 +428,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
         for (int dt = 0; dt < 4; dt++)
             bt_addr[dt][u2] = kOffB + TpSwizzle<RBA>::addr(
-                row, 2 * b_tile_column(32 * (dt / 2) + 4 * (dt % 2) + 8 * (ln & 3)));
+                row, 2 * b_tile_column(32 * ((dt / 2) ^ ks0) + 4 * (dt % 2) + 8 * (ln & 3)));
         vt_addr[u2] = kOffV + TpSwizzle<RBV>::addr(row, 2 * (16 * w + 4 * (ln & 3)));
     }
     // Pt in LDS: row i, j contiguous.  Written 4 values at a time (j = 16 jh + 4 g + r), read
@@ -435,7 +480,36 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     };
     // (with an exchange the sums that travel are those of the rows alone; every segment adds
     // the caller's state on top of what it gathers)
-    if (op.s0 && !exchange) add_caller_state();
+    if (!NORM && op.s0 && !exchange) add_caller_state();
+    // NORM: this consumer's half of z, block by block (tiles 0 and 1 in its order, all columns alike)
+    const bool has_z = NORM && (KS2 == 2 || w < 2);
+    f32x4 Z[ND][2];
+#pragma unroll
+    for (int hb = 0; hb < ND; hb++) Z[hb][0] = Z[hb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const Frag ones = {{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u}};
+    // NORM: a chunk's products are added up by themselves and then, with one rounding, to the state.
+    // (The weights are all positive and the sums of the matrix instructions fall short by a part of the
+    // last place each: 300 chains of 4000 positions walked whole are 7e-7 from float64 without it,
+    // 1e-7 with it, the workgroup form's short segments 3e-7; the time is the same.  Not while
+    // chunks are walked for their state alone: its 24 registers more would spill there.)
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 Sc[4], Zc[2];
+    auto add_product = [&](f32x4 &sum, f32x4 &part, const Frag &x, const Frag &y, bool first) {
+        if (NORM)
+            part = mfma16(x, y, first ? zero : part);
+        else
+            sum = mfma16(x, y, sum);
+    };
+    auto add_chunk = [&](int hb, int from, int to) {
+        if (NORM) {
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++)
+                if (dt >= from && dt < to && dt / 2 < (hb == ND - 1 ? KS2 : 2)) S[hb][dt] += Sc[dt];
+        }
+    };
+    auto add_chunk_z = [&](int hb) {
+        if (NORM) Z[hb][0] += Zc[0], Z[hb][1] += Zc[1];
+    };
 
     // A wavefront issues in order, and four of them share the LDS: reads are therefore
     // written out between the matrix instructions they run under, one at a time, and
@@ -504,15 +578,25 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 r.v = __builtin_amdgcn_raw_buffer_load_b128(
                     v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, 0, 0);
         };
-        auto ccut_b = [&](const RawC &r, int bufk) {
-            split_quad_to_lds(r.b, unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
+        const int key_rows = NORM && p.key_len ? (int)max((int64_t)0, min((int64_t)rows, p.key_len[n])) : rows;
+        auto ccut_b = [&](const RawC &r, int bufk, int v) {
+            u32x4 x = r.b;
+            if (NORM) {  // (position v of the walk, as the producers do)
+                x = feature_quad(x);
+                const int row0 = chunk_row0(so_chunk(v));
+                if (row0 < 0 || row0 + kChunk > key_rows) {
+                    if ((uint32_t)(row0 + crow) >= (uint32_t)key_rows) x = u32x4{0, 0, 0, 0};
+                }
+                if (!b_in[v % ND]) x = u32x4{0, 0, 0, 0};
+            }
+            split_quad_to_lds(x, unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
         };
         auto ccut_v = [&](const RawC &r, int bufk) {
             split_quad_to_lds(r.v, unit_pc + bufk * kBufBytes + kOffV, kTileV, v_waddr);
         };
 #pragma unroll
         for (int j = 0; j < PF; j++) cfetch(rawc[j], j, j % ND);
-        ccut_b(rawc[0], 0);
+        ccut_b(rawc[0], 0, 0);
         ccut_v(rawc[0], 0);
         cfetch(rawc[0], PF, 0);
         wg_barrier();
@@ -535,13 +619,15 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                     if (j % 2 == 0) {
                         if (rows_exist)
                             S[hp][i % 4] = mfma16(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[hp][i % 4]);
+                        if (NORM && i < 6) Z[hp][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
                         if (i < 15) tr_frag_into(bt, vf, pc, pcv, i, j % ND);
                     } else {
                         if (rows_exist)
                             S[hp][i % 4] = mfma16(bt[i % 4][kPa[i / 4]], vf[kPb[i / 4]], S[hp][i % 4]);
+                        if (NORM && i < 6) Z[hp][i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
                         if (i < 15) tr_frag_into(bt2, vf2, pc, pcv, i, j % ND);
                     }
-                    if (i == 15 && cut_next) ccut_b(rn, bufn);
+                    if (i == 15 && cut_next) ccut_b(rn, bufn, c + j + 1);
                     if (i == 19 && cut_next && (j + 1) % ND == 0) ccut_v(rn, bufn);
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -557,6 +643,8 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
         for (int i = 0; i < 24; i++) {
             if ((i % 4) / 2 < KS2)
                 S[ND - 1][i % 4] = mfma16(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[ND - 1][i % 4]);
+            if (NORM && i < 6)
+                Z[ND - 1][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[ND - 1][i % 2]);
             if (i < 18) rm_frag(unit_pc + buf * kBufBytes, i, 0);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -572,10 +660,16 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
         gfloat *const sums = (gfloat *)(hdr + kControlBytes / 4);
         // the flag words and state slots of consumer w of the segment with ticket t are those
         // of "ticket" w * total_units + t (as in ftc_wg_kernel.h)
-        StateExchange<ND, 1> xch(flags, sums, 4u * total_units,
+        constexpr int DX = NORM ? ND + 1 : ND;  // (z rides along in a tile of its own)
+        StateExchange<DX, 1> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);
-        f32x16 Sx[ND][1], X[ND][1];
+        f32x16 Sx[DX][1], X[DX][1];
+        if (NORM) {
+            Sx[DX - 1][0] = f32x16{};
+#pragma unroll
+            for (int i = 0; i < 8 * ND; i++) Sx[DX - 1][0][i] = Z[i / 8][i / 4 % 2][i % 4];
+        }
 #pragma unroll
         for (int hb = 0; hb < ND; hb++)
 #pragma unroll
@@ -592,7 +686,11 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             for (int dt = 0; dt < 4; dt++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) S[hb][dt][r] = X[hb][0][4 * dt + r];
-        if (op.s0) add_caller_state();
+        if (NORM) {
+#pragma unroll
+            for (int i = 0; i < 8 * ND; i++) Z[i / 8][i / 4 % 2][i % 4] = X[DX - 1][0][i];
+        }
+        if (!NORM && op.s0) add_caller_state();
     }
     // S_w as pieces in A operand order (slots 0..3 from tile 2 ks, 4..7 from tile 2 ks + 1).
     // Tiles 0 and 1 are final after phase 3 and are cut under phase 4, tiles 2 and 3 after
@@ -618,11 +716,14 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     for (int i = 0; i < 4; i++) O4[i / 2][i % 2] = f32x4{0.f, 0.f, 0.f, 0.f};
     uint32_t o_off = 0x80000000u;
     // lane (i = 16 (x ^ ih) + ln, g) holds f = 16 w + 4 g + 0..3
+    float r_den[2] = {0.f, 0.f};  // NORM: reciprocals of the denominators of O's rows
     auto store_rows = [&](int x) {
-        const f32x4 o = O4[x][0] + O4[x][1];
+        f32x4 o = O4[x][0] + O4[x][1];
+        if (NORM) o *= r_den[x];
         buffer_store4(o_rs, o_in ? o_off + o_lane[x] : kNoRow, o[0], o[1], o[2], o[3]);
     };
     f32x4 Pkeep = {0.f, 0.f, 0.f, 0.f};  // the quadrant summed over the blocks so far
+    f32x4 Az = {0.f, 0.f, 0.f, 0.f};     // NORM: phi(a) z of the quadrant's positions
     for (int c = c0; c < nchunks; c++) {
 #pragma unroll
         for (int hb = 0; hb < ND; hb++) {  // block hb of the state rows
@@ -634,7 +735,9 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             const bool last_block = hb == ND - 1;
             Frag pf[2][3];
             f32x4 P4[4];
-            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};  // (the first product of a sum adds to a constant)
+            Frag zf[3];  // NORM: z in pieces
+            float P_sum = 0.f;
+            // (the first product of a sum adds to a constant)
             if (c == c0 + 4) FTC_STAMP(0);
             __builtin_amdgcn_sched_barrier(0);
             // phase 1: (1) the quadrant; underneath: tiles 2, 3 of S_w cut into pieces, the
@@ -649,6 +752,12 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 else if (i < 4)
                     P4[i % 4] = zero;
                 if (i < 4 && block_ks(hb) > 1) cut_s(hb, 1, i);
+                if (NORM && i >= 8) {
+                    uint32_t o[3];
+                    split_pair_under_mfma(Z[hb][(i - 8) / 2][2 * (i % 2)], Z[hb][(i - 8) / 2][2 * (i % 2) + 1], o);
+#pragma unroll
+                    for (int k = 0; k < 3; k++) zf[k].w[i - 8] = o[k];
+                }
                 tr_frag_into(bt, vf, pc, pcv, i, hb);
                 if (hb == 0 && (i == 5 || i == 7)) store_rows(i == 5 ? 0 : 1);
                 __builtin_amdgcn_sched_barrier(0);
@@ -666,10 +775,17 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 else if (i < 4 && hb == 0)
                     O4[x][ks] = zero;
                 if (i < 3) tr_frag_into(bt, vf, pc, pcv, 12 + i, hb);
+                if (NORM && i >= 6) Az = mfma16(zf[kPa[i - 6]], af[0][0][kPb[i - 6]], i == 6 && hb == 0 ? zero : Az);
                 if (i == 4) {
                     P = (P4[0] + P4[1]) + (P4[2] + P4[3]);
                     if (hb > 0) P += Pkeep;
                     if (!last_block) Pkeep = P;
+                }
+                if (NORM && i == 9 && last_block) {
+                    float m[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) m[r] = __uint_as_float(__float_as_uint(P[r]) & keep[r]);
+                    P_sum = (m[0] + m[1]) + (m[2] + m[3]);
                 }
                 if (i == 6 && last_block)
                     split_pair_under_mfma(__uint_as_float(__float_as_uint(P[0]) & keep[0]),
@@ -692,13 +808,20 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             for (int i = 0; i < 12; i++) {
                 const int x = i % 2, ks = (i / 2) % 2, m = 3 + i / 4;  // piece products 3..5
                 if (ks < block_ks(hb)) O4[x][ks] = mfma16(sf[ks][kPa[m]], af[x][ks][kPb[m]], O4[x][ks]);
-                S[hb][i % 2] = mfma16(bt[i % 2][kPa[i / 2]], vf[kPb[i / 2]], S[hb][i % 2]);
+                add_product(S[hb][i % 2], Sc[i % 2], bt[i % 2][kPa[i / 2]], vf[kPb[i / 2]], i < 2);
+                if (NORM && i < 6) Zc[i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, i < 2 ? zero : Zc[i % 2]);
+                if (NORM && i == 6 && last_block) {
+                    P_sum = sum_of_lane_groups(P_sum);
+                    if (g == 0) den_mem[c & 1][16 * ih + ln][w >> 1] = (has_z ? Az[0] : 0.f) + P_sum;
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (c == c0 + 4) FTC_STAMP(3);
             buf = next_buf(buf);
             wg_barrier();
             if (c == c0 + 4) FTC_STAMP(4);
+            add_chunk(hb, 0, 2);
+            add_chunk_z(hb);
             // All of Pt is in LDS and the next chunk is cut: its row-major fragments are
             // requested under what follows.
             // phase 4: (3) for tiles 2 and 3 in turn with (2a) Ot_w += v_w^T Pt; underneath:
@@ -710,11 +833,25 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
                     for (int k = 0; k < 3; k++) pf[x][k] = lds_frag16(ptc + k * kTileP + pt_raddr[x]);
             }
+            if constexpr (NORM) {
+                if (last_block) {
+#pragma unroll
+                    for (int x = 0; x < 2; x++) {
+                        const float *part = den_mem[c & 1][16 * (x ^ ih) + ln];
+                        const float den = (part[0] + part[1]) + p.eps;
+                        r_den[x] = 1.0f / den;
+                        // (the caller's copy of the denominators, for the backward)
+                        const int row = chunk_row0(c) + 16 * (x ^ ih) + ln;
+                        if (w == 0 && fb == 0 && op.s_out && g == 0 && row < rows)
+                            op.s_out[(int64_t)n * op.so_sn + (int64_t)h * op.so_sh + row] = den;
+                    }
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 if (block_ks(hb) > 1)
-                    S[hb][2 + i % 2] = mfma16(bt[2 + i % 2][kPa[i / 2]], vf[kPb[i / 2]], S[hb][2 + i % 2]);
+                    add_product(S[hb][2 + i % 2], Sc[2 + i % 2], bt[2 + i % 2][kPa[i / 2]], vf[kPb[i / 2]], i < 2);
                 cut_s((hb + 1) % ND, 0, i);
                 rm_frag(pn, i, (hb + 1) % ND);  // (past the last chunk: a buffer of zeros)
                 __builtin_amdgcn_sched_barrier(0);
@@ -723,7 +860,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             for (int i = 0; i < 12; i++) {
                 if (i < 8 && block_ks(hb) > 1) {
                     const int t = 4 + i;
-                    S[hb][2 + t % 2] = mfma16(bt[2 + t % 2][kPa[t / 2]], vf[kPb[t / 2]], S[hb][2 + t % 2]);
+                    add_product(S[hb][2 + t % 2], Sc[2 + t % 2], bt[2 + t % 2][kPa[t / 2]], vf[kPb[t / 2]], false);
                 }
                 const int x = i % 2, m = i / 2;
                 if (last_block) O4[x][m % 2] = mfma16(vf[kPa[m]], pf[x][kPb[m]], O4[x][m % 2]);
@@ -732,6 +869,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (c == c0 + 4) FTC_STAMP(5);
+            add_chunk(hb, 2, 4);
             o_off = (uint32_t)chunk_row0(c) * o_slb;
             if (c == c0 + 4) FTC_STAMP(6);
         }
@@ -739,7 +877,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     store_rows(0);
     store_rows(1);
     FTC_STAMP(15);  // last rows on their way
-    if (op.s_out && seg == (int)nseg - 1) {
+    if (!NORM && op.s_out && seg == (int)nseg - 1) {
         float *base =
             op.s_out + (int64_t)n * op.so_sn + (int64_t)h * op.so_sh + F * fb + 16 * w + ln;
 #pragma unroll

@@ -240,6 +240,62 @@ def test_small_rows_and_columns_beside_large_ones(lib, shape, small):
         assert ((got - want).norm(dim=dim) / want.norm(dim=dim)).max().item() <= 2e-6
 
 
+MANY_CHAINS = [
+    # N, L, H, E, M, key lengths: chains walked whole, cut in two to five, and with an exchange of segment
+    # sums (one and two levels); single positions, ragged ends, keys that end before, inside and on a
+    # chunk, segments without any key; one and two groups of 32 feature columns
+    (41, 1, 1, 64, 64, [1, 0] * 20 + [5]), (41, 33, 1, 64, 64, [33, 32, 1] * 13 + [0, 7]),
+    (6, 97, 8, 64, 64, [97, 64, 1, 0, 33, 96]), (300, 40, 1, 64, 64, list(range(300))),
+    (6, 1000, 8, 64, 64, [1000, 417, 0, 999, 512, 31]), (3, 2100, 8, 64, 64, [2100, 2049, 500]),
+    (2, 8192, 12, 64, 64, [8192, 3001]), (6, 520, 8, 64, 32, [520, 100, 40, 0, 511, 256]),
+    (6, 520, 8, 32, 64, [520, 100, 40, 0, 511, 256]),
+]
+
+
+@pytest.mark.parametrize("shape", MANY_CHAINS, ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s[:5])
+def test_many_chains(lib, shape):
+    """The chain-parallel form on three bf16 pieces, against the CPU restatement in float64; keys and
+    values at or beyond the length leave every row as it is, bit for bit."""
+    N, L, H, E, M, lens = shape
+    q, k, v = inputs(N, L, H, E, M, seed=270 + L)
+    lengths = torch.tensor(lens)
+    out = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
+    assert lib.ftc_last_kernel().startswith(b"scan_tp_kernel<NORM>")
+    gate(out.cpu(), q, k, v, lengths, 1e-6)
+    for n, length in enumerate(lens):
+        k[n, length:], v[n, length:] = 60.0, 1e30
+    assert torch.equal(fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6), out)
+
+
+@pytest.mark.parametrize("small", ["q_rows", "k_early_rows", "v_columns", "v_early_rows"])
+@pytest.mark.parametrize("shape", [(6, 300, 8, 64, 64), (3, 2100, 8, 64, 64), (6, 520, 8, 64, 32)],
+                         ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s)
+def test_many_chains_small_rows_and_columns_beside_large_ones(lib, shape, small):
+    test_small_rows_and_columns_beside_large_ones(lib, shape, small)
+    assert lib.ftc_last_kernel().startswith(b"scan_tp_kernel<NORM>")
+
+
+def test_many_chains_in_the_workgroup_forms_workspace(lib):
+    """A workspace that the exchange of the chain-parallel form does not fit in gets the workgroup form."""
+    from fast_transformers_amd import _native
+    N, L, H, E, M = 3, 2100, 8, 64, 64
+    q, k, v = (t.cuda() for t in inputs(N, L, H, E, M, seed=5))
+    want = fused(lib, q, k, v, None, 1e-6)
+    assert lib.ftc_last_kernel() == b"scan_tp_kernel<NORM> (exchange)"
+    full = lib.ftc_causal_linear_attention_workspace_bytes(N, H, L, E, M, _native.FTC_F32)
+    ws, out = torch.zeros(full, dtype=torch.uint8, device="cuda"), torch.empty_like(want)
+    d = [_native.describe(t.permute(0, 2, 1, 3)) for t in (q, k, v, out)]
+
+    def call(nbytes):
+        return lib.ftc_causal_linear_attention(
+            *(ctypes.byref(x) for x in d[:3]), None, ctypes.c_float(1e-6), ctypes.byref(d[3]),
+            ctypes.c_void_p(ws.data_ptr()), nbytes, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    least = next(b for b in range(1 << 16, full, 1 << 12) if call(b) == 0)
+    torch.cuda.synchronize()
+    assert least < full and lib.ftc_last_kernel() == b"scan_wg_kernel<NORM>"
+    assert ((out - want).norm() / want.norm()).item() <= 2e-6
+
+
 def _count_backward_calls():
     """Context that counts the calls of the fused backward (autograd runs it on a thread of its
     own, where ftc_last_kernel() of this thread does not see it)."""
