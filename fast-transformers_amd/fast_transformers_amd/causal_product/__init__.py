@@ -113,7 +113,8 @@ def _check_if_possible():
 def workspace_error_words():
     """Error word of every cached workspace (synchronises).  All zero unless a wavefront
     gave up waiting for another one, which a correct launch never does."""
-    return {key: int(ws[8:12].view(torch.int32).item()) for key, ws in _workspaces.items()}
+    # (a copy: reading a word waits, and another thread may add its workspace meanwhile)
+    return {key: int(ws[8:12].view(torch.int32).item()) for key, ws in _workspaces.copy().items()}
 
 
 def check_workspaces():

@@ -84,3 +84,18 @@ def test_cpu_entry_matches_the_checker():
     assert scale_error(out.detach(), oracle.forward(Q, K, V)) <= 1e-5
     for got, ref in zip((Qg.grad, Kg.grad, Vg.grad), oracle.backward(Q, K, V, G)):
         assert scale_error(got, ref) <= 1e-5
+
+
+def test_error_words_are_read_while_another_thread_adds_its_workspace(monkeypatch):
+    import torch
+    from fast_transformers_amd import causal_product as cp
+    workspaces = {}
+
+    class Workspace:  # (reading its word lets the other thread run)
+        def __getitem__(self, words):
+            workspaces[(0, len(workspaces))] = self
+            return torch.zeros(4, dtype=torch.uint8)
+    workspaces[(0, 0)], workspaces[(0, 1)] = Workspace(), Workspace()
+    monkeypatch.setattr(cp, "_workspaces", workspaces)
+    assert cp.workspace_error_words() == {(0, 0): 0, (0, 1): 0}
+    cp.check_workspaces()
