@@ -25,6 +25,7 @@ above, whose pieces autograd differentiates.
 import torch
 from torch.nn import Module
 
+from .. import causal_product
 from ..causal_product import causal_dot_product_hip, causal_dot_backward_hip, \
     causal_linear_attention_hip, fused_attention_covers, CausalLinearAttentionFunction
 
@@ -57,6 +58,10 @@ class ActivationFunctionFeatureMap(Module):
         def inner(query_dims):
             return cls(query_dims, *args, **kwargs)
         return inner
+
+
+_as_defined = (causal_linear_attention_hip, causal_product.causal_linear_attention_backward_hip,
+               CausalLinearAttentionFunction.forward, CausalLinearAttentionFunction.backward)
 
 
 def _elu_plus_one(x):
@@ -156,12 +161,20 @@ class CausalLinearAttention(Module):
         if not (isinstance(fm, ActivationFunctionFeatureMap)
                 and fm.activation_function is _elu_plus_one):
             return None
+        lengths = getattr(key_lengths, "lengths", None)
+        host = causal_product._host_module
+        if host is not None and not torch.compiler.is_compiling() and _as_defined == (
+                causal_linear_attention_hip, causal_product.causal_linear_attention_backward_hip,
+                CausalLinearAttentionFunction.forward, CausalLinearAttentionFunction.backward):
+            # plain tensors: the same in the C++ engine, which costs the host less
+            out = host.attention_module(queries, keys, values, lengths, self.eps)
+            if out is not None:
+                return out
         if queries.shape[1] != keys.shape[1] or keys.shape[1] != values.shape[1]:
             return None
         qv, kv, vv = (t.permute(0, 2, 1, 3) for t in (queries, keys, values))
         if not fused_attention_covers(qv, vv, kv):
             return None
-        lengths = getattr(key_lengths, "lengths", None)
         if lengths is None:  # not a length mask: the composition multiplies by its matrix
             return None
         lengths = lengths.to(device=queries.device, dtype=torch.int64).contiguous()

@@ -346,5 +346,18 @@ class CausalDotProduct(torch.autograd.Function):
         return grad_Q, grad_K, grad_V
 
 
-# Alias the autograd functions to python style snake case naming
-causal_dot_product = CausalDotProduct.apply
+_as_defined = (CausalDotProduct.forward, CausalDotProduct.backward, causal_dot_product_hip, causal_dot_backward_hip)
+
+
+def causal_dot_product(*inputs):
+    """``CausalDotProduct.apply`` (the reference's alias, ``__init__.py:77-78``).  Plain tensors on the
+    GPU take the same function in the C++ engine (``host/ftc_host.cpp``), which costs the host less;
+    the first call, calls that are watched or transformed, and a class or tables that have been
+    changed take the class."""
+    if _host_module is not None and len(inputs) == 3 and not torch.compiler.is_compiling() and _as_defined == (
+            CausalDotProduct.forward, CausalDotProduct.backward, CausalDotProduct.dot.get("cuda"),
+            CausalDotProduct.dot_backward.get("cuda")):
+        product = _host_module.dot(*inputs)
+        if product is not None:
+            return product
+    return CausalDotProduct.apply(*inputs)

@@ -1,0 +1,101 @@
+"""The differentiable entry points on plain tensors run as functions of the C++ engine
+(host/ftc_host.cpp); calls that are watched or transformed run the Python functions.  Both give the
+same bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def cp():
+    from fast_transformers_amd import causal_product
+    causal_product._host()   # (a process's first call goes through Python)
+    return causal_product
+
+
+def operator(cp, dtype, seed=0):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return [torch.rand(2, 3, 70, w, device="cuda", generator=gen).to(dtype) for w in (64, 64, 32)]
+
+
+def attention(seed=0):
+    from fast_transformers_amd.attention import CausalLinearAttention
+    from fast_transformers_amd.masking import LengthMask, TriangularCausalMask
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    lengths = LengthMask(torch.tensor([70, 33], device="cuda"), max_len=70)
+    module, mask = CausalLinearAttention(64), TriangularCausalMask(70, device="cuda")
+    inputs = [torch.randn(2, 70, 3, w, device="cuda", generator=gen) for w in (64, 64, 32)]
+    return inputs, lambda *t: module(*t, mask, lengths, lengths)
+
+
+def in_engine(out):
+    return "CppNode" in out.grad_fn.name()
+
+
+@pytest.mark.parametrize("need", [(1, 1, 1), (1, 0, 0), (0, 1, 1), (0, 0, 0)], ids=str)
+@pytest.mark.parametrize("way", ["fp32", "bf16", "attention"])
+def test_same_bits_as_the_python_functions(cp, way, need):
+    if way == "attention":
+        inputs, call = attention()
+        nhl = lambda t: t.permute(0, 2, 1, 3)
+        lengths = torch.tensor([70, 33], device="cuda")
+        python = lambda *t: nhl(cp.CausalLinearAttentionFunction.apply(*map(nhl, t), lengths, 1e-6))
+    else:
+        inputs, call = operator(cp, {"fp32": torch.float32, "bf16": torch.bfloat16}[way]), cp.causal_dot_product
+        python = cp.CausalDotProduct.apply
+    results = []
+    for f in (call, python):
+        t = [x.clone().requires_grad_(bool(n)) for x, n in zip(inputs, need)]
+        out = f(*t)
+        wanted = [x for x in t if x.requires_grad]
+        if wanted:
+            assert in_engine(out) == (f is call)
+        grads = torch.autograd.grad(out.square().sum(), wanted) if wanted else ()
+        results.append((out,) + grads)
+        assert out.requires_grad == bool(wanted)
+    for a, b in zip(*results):
+        assert torch.equal(a, b) and a.dtype == b.dtype and a.stride() == b.stride()
+
+
+def test_watched_calls_keep_the_python_functions(cp):
+    class Mine(torch.Tensor):
+        pass
+    for inputs, call in ((operator(cp, torch.float32), cp.causal_dot_product), attention()):
+        t = [x.clone().requires_grad_(True) for x in inputs]
+        assert in_engine(call(*t))
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: (seen.append(1), x)[1], lambda x: x):
+            out = call(*t)
+        assert seen and not in_engine(out)
+        assert not in_engine(call(t[0].as_subclass(Mine), *t[1:]).as_subclass(torch.Tensor))
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(call)(*(x[None] for x in inputs))
+    table = cp.CausalDotProduct.dot
+    own = table["cuda"]
+    table["cuda"] = lambda *a: (seen.append(2), own(*a))[1]
+    try:
+        cp.causal_dot_product(*operator(cp, torch.float32))
+    finally:
+        table["cuda"] = own
+    assert seen[-1] == 2
+
+
+def test_python_errors_in_the_engine_reach_the_caller(cp):
+    host = cp._host()
+    # (a few long chains: segment sums are exchanged through a workspace)
+    q, k, v = (torch.rand(1, 2, 4096, 64, device="cuda").requires_grad_(True) for _ in range(3))
+    out = cp.causal_dot_product(q, k, v)
+
+    def broken(nbytes, key):
+        raise ValueError("no workspace")
+    host.setup({}, {}, broken, cp._watch, cp._probe, cp._check_if_possible)
+    host.forget_sizes()
+    try:
+        with pytest.raises(ValueError, match="no workspace"):
+            out.sum().backward()
+    finally:
+        host.setup(cp._workspaces, cp._probes, cp._make_workspace, cp._watch, cp._probe, cp._check_if_possible)
+    again = cp.causal_dot_product(q, k, v)
+    grads = torch.autograd.grad(again.sum(), (q, k, v))
+    assert all(torch.isfinite(g).all() for g in grads)
