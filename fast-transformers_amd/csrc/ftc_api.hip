@@ -344,7 +344,7 @@ int64_t padded_scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, 
     const int64_t Dp = padded_rows(D), Fp = round_up(F, 32), rows = N * H * L;
     const bool copies = Dp != D || Fp != F || (bf16 && Dp > 128);
     if (Dp == 0 || !copies || rows < kPadMinRows || !padded_shape_ok(Dp, Fp)) return 0;
-    return std::max<int64_t>(round_up(scan_workspace_bytes(N, H, L, Dp, Fp), 256),
+    return std::max<int64_t>(round_up(scan_workspace_bytes(N, H, L, Dp, Fp, true, bf16 && Dp <= 128), 256),
                              FTC_WORKSPACE_CONTROL_BYTES) +
            2 * round_up(rows * Dp * 4, 256) + 2 * round_up(rows * Fp * 4, 256) +
            2 * round_up(N * H * Dp * Fp * 4, 256);  // (the states handed in and out)
@@ -405,7 +405,8 @@ int padded_scans(const ScanDesc *scans, int n, const bool *take, int64_t N, int6
             if (sc.final_.ptr)
                 states[nstates++] = StateCopy{sc.final_, sc.a.width, sc.v.width, Dp, Fp, nwork, true, nullptr};
         }
-        ws_scan = std::max(ws_scan, round_up(scan_workspace_bytes(N, H, L, Dp, Fp), 256));
+        const bool bf16 = Dp <= 128 && (sc.a.dtype != FTC_F32 || sc.b.dtype != FTC_F32);
+        ws_scan = std::max(ws_scan, round_up(scan_workspace_bytes(N, H, L, Dp, Fp, true, bf16), 256));
         // states beyond 128 rows run on the fp32 kernels only: bf16 tensors of such a scan are
         // converted on the way
         const bool to_f32 = Dp > 128;
@@ -747,6 +748,11 @@ int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
             continue;
         }
         if (!mfma_tp_takes(group, ngroup, N, H, L)) continue;
+        // (bf16 rows: an exchange that the workspace has no room for is left to the other kernels)
+        if (group[0].a.dtype != FTC_F32 || group[0].b.dtype != FTC_F32) {
+            const int64_t need = mfma_tp_mixed_workspace_bytes(N, H, L, group[0].a.width, group[0].v.width, ngroup);
+            if (need > 0 && !plan_only() && (int64_t)workspace_bytes < need) continue;
+        }
         const int rc = mfma_scan(group, ngroup, N, H, L, workspace, workspace_bytes, stream);
         if (rc) return rc;
         for (int k = 0; k < ngroup; k++) taken[members[k]] = true;
@@ -833,6 +839,7 @@ int64_t scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t
     if (nslices == 0 && with_pad)
         need = std::max(need, padded_scan_workspace_bytes(N, H, L, D, F, bf16));
     for (int k = 1; k <= kMfmaMaxScans; k++) need = std::max(need, mfma_tp_workspace_bytes(N, H, L, D, F, k));
+    for (int k = 1; k <= 3 && bf16; k++) need = std::max(need, mfma_tp_mixed_workspace_bytes(N, H, L, D, F, k));
     // (odd widths where they lie, which takes room for their copies: odd_in_place)
     if (with_pad && !bf16 && padded_scan_workspace_bytes(N, H, L, D, F) > 0)
         for (int k = 1; k <= kMfmaMaxScans; k++)
@@ -1023,8 +1030,8 @@ int64_t ftc_causal_dot_backward_workspace_bytes(int64_t N, int64_t H, int64_t L,
         for (int k = 2; k <= 3 && !bf16; k++)
             need = std::max(need, mfma_tp_workspace_bytes(N, H, L, std::max(E, M), std::max(E, M), k, false, true));
         int64_t ws = 0;
-        if (padded_rows(E)) ws = std::max(ws, scan_workspace_bytes(N, H, L, padded_rows(E), round_up(M, 32)));
-        if (padded_rows(M)) ws = std::max(ws, scan_workspace_bytes(N, H, L, padded_rows(M), round_up(E, 32)));
+        if (padded_rows(E)) ws = std::max(ws, scan_workspace_bytes(N, H, L, padded_rows(E), round_up(M, 32), true, bf16 && padded_rows(E) <= 128));
+        if (padded_rows(M)) ws = std::max(ws, scan_workspace_bytes(N, H, L, padded_rows(M), round_up(E, 32), true, bf16 && padded_rows(M) <= 128));
         int64_t copies = 4 * round_up(N * H * L * round_up(E, 32) * 4, 256) +
                          3 * round_up(N * H * L * round_up(M, 32) * 4, 256);
         // bf16 rows whose two state shapes lie on either side of 128 rows: the scans of the

@@ -143,6 +143,8 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
                    bool forced = false, bool odd = false);
 int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans,
                                 bool forced = false, bool odd = false);
+// ... and of scans with bf16 rows among them
+int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans);
 // estimated time of such a launch, in chunks walked one after the other
 double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L);
 // The fused attention form of a forward scan: a and b go through the feature map

@@ -329,6 +329,66 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
         *nseg = tp_kernel_segments(units, L, wide, others, long_chains, narrow, most_units, brief_chunks);
 }
 
+// Launches of bf16 rows that the rules above leave to the kernels that split L: on the chain-parallel
+// kernel as well (three pieces for the state and fp32 rows, bf16 rows multiplied as they are,
+// scan_mfma_kernel_tp), in whichever is estimated shorter of whole or cut chains and an exchange of
+// segment sums.  A chunk takes a workgroup 0.63 us (a single scan, a state of up to 64 rows), 0.79 (the
+// scans of a backward call), 1.07 and 1.38 (wider states), a first pass over it about 0.7 of that, the
+// exchange 14 us and half a microsecond for every segment up to 16.  Measured over 1 to 1024 chains of
+// 64 to 16384 positions (us, before / here): 128 x 128 forward, 128 chains, L=4096 366 / 169, backward
+// 1213 / 629; 80 chains, L=1000 68 + 228 / 40 + 107; 4 chains, L=64, backward 28.6 / 8.1; 64 x 64
+// forward, 80 chains, L=1000 26.6 / 19.1, 128 chains, L=4096 114 / 81; 32 x 32 backward, 16 chains, L=256
+// 30 / 8.8.  What stays: more than a thousand chains of a few chunks (64 x 64 forward, 1024 chains, L=64 12.7 /
+// 18.1, L=256 equal; backward, L=128 63 / 79; 64 x 128 forward, 384 chains, L=128 16 / 20), single scans
+// of wide states on a few chains (128 x 128, 1 chain, L=1000 15.9 / 23.7, 4 chains equal; 96 x 96, 24
+// chains, L=2048 36 / 40), and of narrow ones (32 rows or columns) long chains (32 x 128 forward, 48 chains, L=16384 218 / 251), few chains
+// (128 x 32 forward, 4 chains, L=1000 16.0 / 23.8), many chains (32 x 32 backward, 1024 chains, L=1000
+// 216 / 273; 64 x 32 forward, 384 chains, L=128 9.7 / 12.4) and single scans of 32 x 32 (16 chains, L=4096
+// 20.5 / 26.1).
+void mixed_rest_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg,
+                             int *seg_chunks) {
+    *nseg = *seg_chunks = 0;
+    if (!tp_widths(D, F) || tuning().tp == 0) return;
+    const int64_t units = chains * nscans * tp_fblocks(F), chunks = (L + kChunk - 1) / kChunk;
+    const bool narrow = D <= 32 || F <= 32, single = nscans == 1;
+    if (narrow) {
+        if ((single && D <= 32 && F <= 32) || chunks > 128 || units > (single ? 768 : 1536) ||
+            (chunks <= 4 && units >= 320) || (chunks <= 8 && units >= (single ? 512 : 1024)) ||
+            (single && (chunks <= 2 || units < (chunks <= 8 ? 1 : chunks <= 32 ? 32 : 128))))
+            return;
+    } else if (D > 64 && F > 64) {
+        if (D <= 96 && ((chunks <= 4 && units >= 320) || (chunks <= 8 && units >= 4096) ||
+                        (single && chunks > 48 && units < 128) || (chunks > 256 && units < 192)))
+            return;
+    } else if ((chunks <= 4 && units >= (single ? 768 : 1024)) || (chunks <= 8 && units >= (single ? 1024 : 2048))) {
+        return;
+    }
+    if (single && D > 64 && ((units < 16 && chunks > 8 && chunks < (units < 8 ? 256 : 96)) || (units >= 320 && chunks <= 2))) return;
+    const double chunk_us = D <= 64 ? (single ? 0.63 : 0.79) : (single ? 1.07 : 1.38);
+    double least = 1e30;
+    // whole chains, or cut ones whose workgroups rebuild the state before their segment (results in
+    // bf16 make the rounding of a long running state a non-issue)
+    if (chunks <= (single ? 256 : 1024)) {
+        int32_t start[kMaxTpSegments + 1];
+        int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), chunks)) : 1;
+        n = tp_segment_starts(chunks, n, start);
+        double longest = (double)chunks;
+        if (n > 1) {
+            longest = 0;
+            for (int i = 0; i < n; i++) longest = std::max(longest, 0.6 * start[i] + (double)(start[i + 1] - start[i]));
+        }
+        least = (double)((units * n + 255) / 256) * (longest * chunk_us + 4.0);
+        *nseg = n;
+    }
+    for (int64_t n = 2; n <= 64 && n <= chunks / 4; n++) {
+        const int64_t c = ((chunks + n - 1) / n + kTpAhead - 1) / kTpAhead * kTpAhead, segs = (chunks + c - 1) / c;
+        if (c > 256 || segs < 2 || 4 * units * segs > kMaxWaves) continue;
+        const double us = (double)((units * segs + 255) / 256) *
+                          (1.7 * (double)c * chunk_us + 14.0 + 0.5 * (double)std::min<int64_t>(segs, 16));
+        if (us < least - 1e-9) least = us, *nseg = (int)segs, *seg_chunks = (int)c;
+    }
+}
+
 // workspace of the exchange: control block, then two state slots (own sum, group total) of
 // D x 16 floats (D rounded up to whole blocks of 64 rows) per consumer, four consumers per segment
 int64_t tp_exchange_workspace_bytes(int64_t units, int nseg, int64_t D) {
@@ -434,6 +494,22 @@ void tp_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *n
     const TpPlan pl = memo.get(key, [&]() {
         TpPlan p;
         tp_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks, forced, mixed, odd);
+        return p;
+    });
+    *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
+}
+// (mixed rows: as_before says whether the rules above have taken the launch)
+void mixed_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int mixed, int *nseg, int *seg_chunks,
+                bool *as_before) {
+    *nseg = *seg_chunks = 0;
+    if (D <= 64) tp_plan(D, F, chains, nscans, L, nseg, seg_chunks, false, mixed);
+    *as_before = *nseg > 0;
+    if (*as_before) return;
+    static thread_local PlanMemo<TpPlan> memo;
+    const int64_t key[8] = {D, F, chains, nscans, L, 0, 0, 0};
+    const TpPlan pl = memo.get(key, [&]() {
+        TpPlan p;
+        mixed_rest_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks);
         return p;
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
@@ -572,8 +648,8 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
         const ScanDesc &sd = scans[i];
         const Combo combo = combo_of(sd);
         if (combo != kFFFF && mixed == 0) mixed = kMixedRows;
-        // rows with bf16 among them: the fp16-piece form of the kernel only
-        if (combo == kNone || (combo != kFFFF && !tph_takes_rows(D))) return false;
+        // (rows with bf16 among them: not as parts of wider scans, whose results are added up in fp32)
+        if (combo == kNone || (combo != kFFFF && (forced || tuning().tph == 0))) return false;
         // (odd widths: scans of any widths side by side, as long as none has a second block of columns)
         if ((sd.a.width != D || sd.v.width != F) && !(odd && F <= 64)) return false;
         if (odd && (combo != kFFFF || sd.a.width < 8 || sd.v.width < 8)) return false;
@@ -595,8 +671,26 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     if ((L + 2 * kChunk) * std::max<int64_t>(widest_stride, std::max(D, F)) * 4 >= 0x7fffffffLL)
         return false;
     int nseg = 0, seg_chunks = 0;
-    tp_plan(D, F, std::max<int64_t>(1, N * H), nscans, L, &nseg, &seg_chunks, forced, mixed, odd);
+    bool as_before;
+    const int64_t chains = std::max<int64_t>(1, N * H);
+    if (mixed)
+        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks, &as_before);
+    else
+        tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, odd);
     return nseg > 0;
+}
+
+int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans) {
+    const int64_t chains = std::max<int64_t>(1, N * H);
+    int64_t bytes = 0;
+    for (const int mixed : {kMixedRows, kMixedGradValues}) {
+        int nseg = 0, seg_chunks = 0;
+        bool as_before;
+        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks, &as_before);
+        if (seg_chunks > 0)
+            bytes = std::max(bytes, tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D));
+    }
+    return bytes;
 }
 
 double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L) {
@@ -670,6 +764,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for this shape or layout");
     const int64_t chains = std::max<int64_t>(1, N * H);
     int tpx_nseg = 0, tpx_seg_chunks = 0, tp_nseg = 0;
+    bool as_before = true;
     int64_t widest = 0;
     for (int64_t l : {scans[0].a.stride_l, scans[0].b.stride_l, scans[0].v.stride_l, scans[0].out.stride_l})
         widest = std::max(widest, l);
@@ -687,7 +782,10 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         int any_bf16 = nscans == 1 && combo == kBBFB ? kMixedGradValues : 0;
         for (int i = 0; i < nscans; i++)
             if (combo_of(scans[i]) != kFFFF && any_bf16 == 0) any_bf16 = kMixedRows;
-        tp_plan(D, F, chains, nscans, L, &tpx_nseg, &tpx_seg_chunks, forced, any_bf16, odd);
+        if (any_bf16)
+            mixed_plan(D, F, chains, nscans, L, any_bf16, &tpx_nseg, &tpx_seg_chunks, &as_before);
+        else
+            tp_plan(D, F, chains, nscans, L, &tpx_nseg, &tpx_seg_chunks, forced, 0, odd);
         if (tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     }
     const bool tp = tp_nseg > 0 || tpx_seg_chunks > 0;
@@ -782,9 +880,10 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
 
     const bool half_pieces = tp && tph_takes_rows(D);
     bool mixed = false;  // rows with bf16 among them
+    const bool rows_as_they_are = tp && combo != kFFFF;
     for (int i = 0; i < nscans; i++) {
         mixed = mixed || combo_of(scans[i]) != kFFFF;
-        if ((!half_pieces && combo_of(scans[i]) != combo) ||
+        if ((!rows_as_they_are && combo_of(scans[i]) != combo) ||
             (!(tp && odd) && (scans[i].a.width != D || scans[i].v.width != F)))
             return fail(FTC_ERR_INVALID, "scans of one launch must share widths and dtypes");
     }
@@ -792,6 +891,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     bool dma = D <= 64 && combo == kFFFF;
     if (tuning().dma >= 0) dma = dma && tuning().dma != 0;  // tuning aid
     note_kernel(fused_tp ? (tpx_seg_chunks > 0 ? "scan_tp_kernel<NORM> (exchange)" : "scan_tp_kernel<NORM>")
+                : rows_as_they_are && !as_before ? (tpx_seg_chunks > 0 ? "scan_mfma_kernel_tp (exchange)" : "scan_mfma_kernel_tp")
                 : tp ? (half_pieces ? (tpx_seg_chunks > 0 ? "scan_tph_kernel (exchange)" : "scan_tph_kernel")
                                   : (tpx_seg_chunks > 0 ? "scan_tp_kernel (exchange)" : "scan_tp_kernel"))
                 : wg ? (fused ? "scan_wg_kernel<NORM>" : "scan_wg_kernel")
@@ -813,8 +913,10 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     if (tp) {
         if (fused)
             launch_scan_tp_norm(workspace, args, stream);
+        else if (mixed)
+            launch_scan_tp_mixed(workspace, args, as_before, stream);
         else if (half_pieces)
-            launch_scan_tph(workspace, args, mixed, odd, stream);
+            launch_scan_tph(workspace, args, odd, stream);
         else
             launch_scan_tp(workspace, args, stream);
     } else if (wg) {

@@ -108,6 +108,67 @@ __device__ __forceinline__ float sum_of_lane_groups(float x) {
     return __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
 }
 
+// Piece products of an X operand in PX pieces and a Y operand in PY (three for fp32 values, one for
+// bf16 ones), smallest first: all but those below the last place of fp32.
+template <int PX, int PY>
+struct Products {
+    static constexpr int count = PX == 3 && PY == 3 ? 6 : PX * PY;
+    __device__ static constexpr int x(int m) {
+        constexpr int all[6] = {0, 1, 2, 0, 1, 0};
+        return PX == 1 ? 0 : PY == 1 ? 2 - m : all[m];
+    }
+    __device__ static constexpr int y(int m) {
+        constexpr int all[6] = {2, 1, 0, 1, 0, 0};
+        return PY == 1 ? 0 : PX == 1 ? 2 - m : all[m];
+    }
+};
+// four consecutive values of a row in memory: fp32 (three pieces) or bf16 (one)
+template <int P>
+struct RowQuad {
+    typedef u32x4 raw;
+    static constexpr int bytes = 4;  // per value
+    __device__ static __forceinline__ raw load(__amdgpu_buffer_rsrc_t rs, uint32_t at) {
+        return __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0);
+    }
+    __device__ static __forceinline__ void to_lds(const raw r, lds_char *tile, int piece_bytes, int addr) {
+        split_quad_to_lds(r, tile, piece_bytes, addr);
+    }
+};
+template <>
+struct RowQuad<1> {
+    typedef u32x2 raw;
+    static constexpr int bytes = 2;
+    __device__ static __forceinline__ raw load(__amdgpu_buffer_rsrc_t rs, uint32_t at) {
+        return __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0);
+    }
+    __device__ static __forceinline__ void to_lds(const raw r, lds_char *tile, int, int addr) {
+        *(lds_vec2 *)(tile + addr) = r;
+    }
+};
+
+// which scan (and block of columns and segment: `which`) and which chain a workgroup takes:
+// workgroups of one scan in groups of 8 (one per XCD), the groups of the scans of a launch side by
+// side, so that scans reading the same rows share an L2 (also the segments of a chain, which read the
+// same early rows)
+__device__ __forceinline__ void tp_workgroup(const ScanArgs &p, uint32_t &which, uint32_t &chain) {
+    const uint32_t chains = (uint32_t)p.waves_per_scan / (uint32_t)p.nseg;
+    const uint32_t per_chain = (uint32_t)p.total_waves / chains;  // scans x segments
+    const uint32_t full = (chains / 8u) * 8u;
+    if (blockIdx.x < full * per_chain) {
+        const uint32_t grp = blockIdx.x / (8u * per_chain), r = blockIdx.x % (8u * per_chain);
+        which = r / 8u;
+        chain = grp * 8u + r % 8u;
+    } else {
+        const uint32_t t = blockIdx.x - full * per_chain;
+        which = t / (chains - full);
+        chain = full + t % (chains - full);
+    }
+}
+// LDS of a workgroup: bytes of the three buffers of a, b and v in pieces, and of Pt's two
+template <int PA, int PB, int PV>
+constexpr int kTpPieceBytes = 3 * (PA + PB + PV) * kChunk * 128;
+constexpr int kTpPtBytes = 2 * 3 * kChunk * 64;
+
 // KS2: groups of 32 rows in the state's last block (1: a state of 65 .. 96 rows, whose last
 // block skips the matrix instructions and fragment reads of its empty half)
 // NORM: causally masked linear attention in the same walk (see ftc_wg_kernel.h for the equations):
@@ -120,15 +181,26 @@ __device__ __forceinline__ float sum_of_lane_groups(float x) {
 // own quadrant: twelve matrix instructions, a cut and a reduction over the lane groups.  A
 // position's two contributions meet in LDS behind the chunk's barrier, and rows are divided as they
 // are stored.
-template <int ND, int KS2, bool NORM>
-__global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
+// PA, PB, PV: pieces of the values of a, b and v: three for fp32 rows, one for bf16 rows, which are
+// multiplied as they are; TO: the type of the result's rows
+template <int ND, int KS2, bool NORM, int PA, int PB, int PV, typename TO>
+__device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, const ScanArgs &p, uint32_t which,
+                                             uint32_t chain, lds_char *unit_pc, lds_char *pt_pc,
+                                             float (*den_mem)[NORM ? kChunk : 1][2], uint32_t *order_sh) {
     constexpr int D = 64, F = 64;              // one block of state rows and of output columns
     constexpr int T = 256;                     // producer lanes
     constexpr int PF = kTpAhead;               // chunks requested ahead
     constexpr int RBA = D * 2, RBV = F * 2;    // bytes per row of a bf16 piece tile
     constexpr int kTileA = kChunk * RBA, kTileV = kChunk * RBV;
-    constexpr int kOffB = 3 * kTileA, kOffV = 6 * kTileA;
-    constexpr int kBufBytes = 6 * kTileA + 3 * kTileV;
+    constexpr int kOffB = PA * kTileA, kOffV = (PA + PB) * kTileA;
+    constexpr int kBufBytes = (PA + PB) * kTileA + PV * kTileV;
+    typedef Products<PB, PA> OfP;   // the quadrant of Pt
+    typedef Products<3, PA> OfO;    // S^T a^T
+    typedef Products<PB, PV> OfS;   // b^T v
+    typedef Products<PV, 3> OfV;    // v^T Pt
+    typedef RowQuad<PA> QuadA;
+    typedef RowQuad<PB> QuadB;
+    typedef RowQuad<PV> QuadV;
     constexpr int kTileP = kChunk * 64;        // Pt pieces: 32 rows (i) of 32 j
     constexpr int QA = D / 4, QV = F / 4;
     constexpr int LA = kChunk * QA / T, LV = kChunk * QV / T;
@@ -140,29 +212,8 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     const bool producer = wave >= 4;
     const int w = wave & 3;
 
-    __shared__ __align__(16) char pieces_mem[3 * kBufBytes];
-    __shared__ __align__(16) char pt_mem[2 * 3 * kTileP];
-    __shared__ __align__(16) float den_mem[NORM ? 2 : 1][NORM ? kChunk : 1][2];
-    lds_char *const unit_pc = (lds_char *)pieces_mem;
-    lds_char *const pt_pc = (lds_char *)pt_mem;
-
-    // ---- which chain: workgroups of one scan in groups of 8 (one per XCD), the groups of
-    // the scans of a launch side by side, so that scans reading the same rows share an L2 ----
-    // (also the segments of a chain, which read the same early rows)
     const uint32_t nseg = (uint32_t)p.nseg;
     const uint32_t chains = (uint32_t)p.waves_per_scan / nseg;
-    const uint32_t per_chain = (uint32_t)p.total_waves / chains;  // scans x segments
-    const uint32_t full = (chains / 8u) * 8u;
-    uint32_t which, chain;
-    if (blockIdx.x < full * per_chain) {
-        const uint32_t grp = blockIdx.x / (8u * per_chain), r = blockIdx.x % (8u * per_chain);
-        which = r / 8u;
-        chain = grp * 8u + r % 8u;
-    } else {
-        const uint32_t t = blockIdx.x - full * per_chain;
-        which = t / (chains - full);
-        chain = full + t % (chains - full);
-    }
     // (a scan with more than 64 output columns counts as two, one per block of columns)
     const uint32_t virt = which / nseg;
     const uint32_t scan_id = virt / (uint32_t)p.tp_fblocks;
@@ -188,13 +239,12 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     gu32 *const flags = hdr + kHdrWords;
     const uint32_t chain_id = virt * chains + chain;  // over all scans of the launch
     int seg = (int)(which % nseg);
-    __shared__ uint32_t order_sh;
     if (exchange) {
         if (tid == 0)
-            order_sh = __hip_atomic_fetch_add(flags + kMaxWaves + chain_id, 1u, __ATOMIC_RELAXED,
+            *order_sh = __hip_atomic_fetch_add(flags + kMaxWaves + chain_id, 1u, __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
-        seg = (int)__builtin_amdgcn_readfirstlane(order_sh);
+        seg = (int)__builtin_amdgcn_readfirstlane(*order_sh);
         if ((uint32_t)seg >= nseg) {  // the control block was not zero when the launch began
             if (tid == 0)
                 __hip_atomic_store(hdr + kHdrError, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -233,18 +283,18 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     if (producer) {
         // =========================== producers ===========================
         const int ptid = w * 64 + lane;
-        const uint32_t a_slb = (uint32_t)op.a_sl * 4, b_slb = (uint32_t)op.b_sl * 4,
-                       v_slb = (uint32_t)op.v_sl * 4;
-        const char *a_seg = (const char *)op.a + ((int64_t)n * op.a_sn + (int64_t)h * op.a_sh) * 4;
-        const char *b_seg = (const char *)op.b + ((int64_t)n * op.b_sn + (int64_t)h * op.b_sh) * 4;
+        const uint32_t a_slb = (uint32_t)op.a_sl * QuadA::bytes, b_slb = (uint32_t)op.b_sl * QuadB::bytes,
+                       v_slb = (uint32_t)op.v_sl * QuadV::bytes;
+        const char *a_seg = (const char *)op.a + ((int64_t)n * op.a_sn + (int64_t)h * op.a_sh) * QuadA::bytes;
+        const char *b_seg = (const char *)op.b + ((int64_t)n * op.b_sn + (int64_t)h * op.b_sh) * QuadB::bytes;
         const char *v_seg = (const char *)op.v +
-                            ((int64_t)n * op.v_sn + (int64_t)h * op.v_sh + F * fb) * 4;
+                            ((int64_t)n * op.v_sn + (int64_t)h * op.v_sh + F * fb) * QuadV::bytes;
         const __amdgpu_buffer_rsrc_t a_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)a_seg, 0, (rows - 1) * a_slb + Dw * 4, kRsrcFlags);
+            (void *)a_seg, 0, (rows - 1) * a_slb + Dw * QuadA::bytes, kRsrcFlags);
         const __amdgpu_buffer_rsrc_t b_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)b_seg, 0, (rows - 1) * b_slb + Dw * 4, kRsrcFlags);
+            (void *)b_seg, 0, (rows - 1) * b_slb + Dw * QuadB::bytes, kRsrcFlags);
         const __amdgpu_buffer_rsrc_t v_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)v_seg, 0, (rows - 1) * v_slb + fw * 4, kRsrcFlags);
+            (void *)v_seg, 0, (rows - 1) * v_slb + fw * QuadV::bytes, kRsrcFlags);
         // Widths that do not fill their last block of 64: a lane whose four columns lie
         // beyond the width asks outside the descriptor and cuts zeros (widths are multiples
         // of 4).  A lane has the same columns in both of its quads.
@@ -257,19 +307,21 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
         for (int q = 0; q < LA; q++) {
             const int u = q * T + ptid, row = u / QA, c4 = u % QA;
-            a_goff[q] = (uint32_t)row * a_slb + 16u * c4;
-            b_goff[q] = (uint32_t)row * b_slb + 16u * c4;
+            a_goff[q] = (uint32_t)row * a_slb + 4u * QuadA::bytes * c4;
+            b_goff[q] = (uint32_t)row * b_slb + 4u * QuadB::bytes * c4;
             a_waddr[q] = TpSwizzle<RBA>::addr(row, 8 * c4);
             b_waddr[q] = TpSwizzle<RBA>::addr(row, 2 * b_tile_column(4 * c4));
         }
 #pragma unroll
         for (int q = 0; q < LV; q++) {
             const int u = q * T + ptid, row = u / QV, c4 = u % QV;
-            v_goff[q] = (uint32_t)row * v_slb + 16u * c4;
+            v_goff[q] = (uint32_t)row * v_slb + 4u * QuadV::bytes * c4;
             v_waddr[q] = TpSwizzle<RBV>::addr(row, 8 * c4);
         }
         struct Raw {
-            u32x4 a[LA], b[LA], v[LV];
+            typename QuadA::raw a[LA];
+            typename QuadB::raw b[LA];
+            typename QuadV::raw v[LV];
         };
         Raw raw[PF];
         // Every request is made every time, whether its rows exist or not (of a chunk walked
@@ -282,43 +334,45 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
         auto fetch = [&](Raw &r, int v, int hb) {  // v: position of the walk, hb = v % ND
             const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
             const int row0_x = v >= n1 ? row0 : -2 * kChunk;
-            const uint32_t col = (uint32_t)(D * 4 * hb);
+            const uint32_t col_a = (uint32_t)(D * QuadA::bytes * hb), col_b = (uint32_t)(D * QuadB::bytes * hb);
 #pragma unroll
             for (int q = 0; q < LA; q++) {
-                r.a[q] = __builtin_amdgcn_raw_buffer_load_b128(
-                    a_rs, ab_in[hb] ? a_goff[q] + col + (uint32_t)row0_x * a_slb : kNoRow, 0, 0);
-                r.b[q] = __builtin_amdgcn_raw_buffer_load_b128(
-                    b_rs, ab_in[hb] ? b_goff[q] + col + (uint32_t)(q == 0 ? row0 : row0_x) * b_slb
-                                    : kNoRow, 0, 0);
+                r.a[q] = QuadA::load(a_rs, ab_in[hb] ? a_goff[q] + col_a + (uint32_t)row0_x * a_slb : kNoRow);
+                r.b[q] = QuadB::load(b_rs, ab_in[hb] ? b_goff[q] + col_b + (uint32_t)(q == 0 ? row0 : row0_x) * b_slb
+                                                     : kNoRow);
             }
             // (the second block of a chunk multiplies the v tile of the first: no second copy)
             if (hb == 0) {
 #pragma unroll
                 for (int q = 0; q < LV; q++)
-                    r.v[q] = __builtin_amdgcn_raw_buffer_load_b128(
-                        v_rs, v_in ? v_goff[q] + (uint32_t)(q == 0 ? row0 : row0_x) * v_slb : kNoRow,
-                        0, 0);
+                    r.v[q] = QuadV::load(v_rs, v_in ? v_goff[q] + (uint32_t)(q == 0 ? row0 : row0_x) * v_slb : kNoRow);
             }
         };
         // NORM: keys at or beyond this row count as zero (phi(0) = 1, so do the rows that do not
         // exist, and the columns)
         const int key_rows = NORM && p.key_len ? (int)max((int64_t)0, min((int64_t)rows, p.key_len[n])) : rows;
-        auto feature_a = [&](const u32x4 x, int hb) -> u32x4 {
-            if (!NORM) return x;
-            u32x4 y = feature_quad(x);
-            if (!ab_in[hb]) y = u32x4{0, 0, 0, 0};
-            return y;
-        };
-        auto feature_b = [&](const u32x4 x, int hb, int v, int q) -> u32x4 {  // quad q of position v
-            if (!NORM) return x;
-            u32x4 y = feature_quad(x);
-            const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
-            // (a scalar test: most chunks lie wholly below the limit)
-            if (row0 < 0 || row0 + kChunk > key_rows) {
-                if ((uint32_t)(row0 + 16 * q + ptid / QA) >= (uint32_t)key_rows) y = u32x4{0, 0, 0, 0};
+        auto feature_a = [&](const auto x, int hb) {
+            if constexpr (NORM) {
+                u32x4 y = feature_quad(x);
+                if (!ab_in[hb]) y = u32x4{0, 0, 0, 0};
+                return y;
+            } else {
+                return x;
             }
-            if (!ab_in[hb]) y = u32x4{0, 0, 0, 0};
-            return y;
+        };
+        auto feature_b = [&](const auto x, int hb, int v, int q) {  // quad q of position v
+            if constexpr (NORM) {
+                u32x4 y = feature_quad(x);
+                const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
+                // (a scalar test: most chunks lie wholly below the limit)
+                if (row0 < 0 || row0 + kChunk > key_rows) {
+                    if ((uint32_t)(row0 + 16 * q + ptid / QA) >= (uint32_t)key_rows) y = u32x4{0, 0, 0, 0};
+                }
+                if (!ab_in[hb]) y = u32x4{0, 0, 0, 0};
+                return y;
+            } else {
+                return x;
+            }
         };
         // position k of the walk goes to LDS buffer k % 3 through register set k % PF.  The
         // first n1 positions (a multiple of PF) only feed the state: no piece of a, and the
@@ -327,14 +381,14 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             lds_char *const pc = unit_pc + buf * kBufBytes;
 #pragma unroll
             for (int q = 0; q < LA; q++) {
-                if (own) split_quad_to_lds(feature_a(r.a[q], hb), pc, kTileA, a_waddr[q]);
+                if (own) QuadA::to_lds(feature_a(r.a[q], hb), pc, kTileA, a_waddr[q]);
                 if (own || q == 0)
-                    split_quad_to_lds(feature_b(r.b[q], hb, v, q), pc + kOffB, kTileA, b_waddr[q]);
+                    QuadB::to_lds(feature_b(r.b[q], hb, v, q), pc + kOffB, kTileA, b_waddr[q]);
             }
             if (hb == 0) {
 #pragma unroll
                 for (int q = 0; q < LV; q++)
-                    if (own || q == 0) split_quad_to_lds(r.v[q], pc + kOffV, kTileV, v_waddr[q]);
+                    if (own || q == 0) QuadV::to_lds(r.v[q], pc + kOffV, kTileV, v_waddr[q]);
             }
             // (a request whose answer is not used would be moved out of the loop: the waits
             // are the same either way)
@@ -388,10 +442,11 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 
     // =========================== consumers ===========================
     const int ln = lane & 15, g = lane >> 4;
-    const uint32_t o_slb = (uint32_t)op.o_sl * 4;
-    char *o_seg = (char *)op.out + ((int64_t)n * op.o_sn + (int64_t)h * op.o_sh + F * fb) * 4;
+    constexpr int kOutBytes = sizeof(TO);
+    const uint32_t o_slb = (uint32_t)op.o_sl * kOutBytes;
+    char *o_seg = (char *)op.out + ((int64_t)n * op.o_sn + (int64_t)h * op.o_sh + F * fb) * kOutBytes;
     const __amdgpu_buffer_rsrc_t o_rs =
-        __builtin_amdgcn_make_buffer_rsrc((void *)o_seg, 0, (rows - 1) * o_slb + fw * 4, kRsrcFlags);
+        __builtin_amdgcn_make_buffer_rsrc((void *)o_seg, 0, (rows - 1) * o_slb + fw * kOutBytes, kRsrcFlags);
     // Pt quadrant of this wavefront: the two on the diagonal, the one inside the mask, and
     // (consumer 3, so that all four run the same instructions) the one outside it: zeros
     const int jh = w == 0 ? 0 : w == 1 ? 1 : ((w == 2) == REV ? 1 : 0);
@@ -447,7 +502,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     uint32_t o_lane[2];
 #pragma unroll
     for (int x = 0; x < 2; x++)
-        o_lane[x] = (uint32_t)(16 * (x ^ ih) + ln) * o_slb + 4u * (16 * w + 4 * g);
+        o_lane[x] = (uint32_t)(16 * (x ^ ih) + ln) * o_slb + (uint32_t)kOutBytes * (16 * w + 4 * g);
     const bool o_in = 16 * w + 4 * g < fw;  // (columns beyond the width are not stored)
 
     f32x4 S[ND][4];  // the slab's rows, block by block
@@ -455,7 +510,6 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     for (int hb = 0; hb < ND; hb++)
 #pragma unroll
         for (int dt = 0; dt < 4; dt++) S[hb][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int kPa[6] = {0, 1, 2, 0, 1, 0}, kPb[6] = {2, 1, 0, 1, 0, 0};  // piece products
     // the caller's state: lane (f = 16 w + ln, g), tile dt, register r <-> row d below
     auto state_row = [&](int dt, int r) -> int { return 32 * (dt / 2) + 8 * g + 4 * (dt % 2) + r; };
     const bool st_in = 16 * w + ln < fw;
@@ -487,52 +541,73 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
     for (int hb = 0; hb < ND; hb++) Z[hb][0] = Z[hb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     const Frag ones = {{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u}};
-    // NORM: a chunk's products are added up by themselves and then, with one rounding, to the state.
-    // (The weights are all positive and the sums of the matrix instructions fall short by a part of the
-    // last place each: 300 chains of 4000 positions walked whole are 7e-7 from float64 without it,
-    // 1e-7 with it, the workgroup form's short segments 3e-7; the time is the same.  Not while
-    // chunks are walked for their state alone: its 24 registers more would spill there.)
+    // The products of up to eight chunks are added up by themselves (R) before they are added to the
+    // state, where there are registers for it; the state in use is S + R.  (The sums of the matrix
+    // instructions fall short by a part of the last place of the sum each, which keys and weights that
+    // are all positive add up.  NORM: 300 chains of 4000 positions walked whole were 7e-7 from float64
+    // without it, the workgroup form's short segments are 3e-7; the time is the same.  Not there while
+    // chunks are walked for their state alone: its registers would spill.  bf16 rows: the state handed
+    // out after 1000 positions was 2.7e-7 off without it, 1.0e-7 on the kernels that split L.)
+    constexpr bool kMixed = PA + PB + PV < 9, kApart = NORM || kMixed;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 Sc[4], Zc[2];
-    auto add_product = [&](f32x4 &sum, f32x4 &part, const Frag &x, const Frag &y, bool first) {
-        if (NORM)
-            part = mfma16(x, y, first ? zero : part);
+    f32x4 R[ND][4], Zr[ND][2];
+    auto add_product = [&](int hb, int dt, const Frag &x, const Frag &y) {
+        if (kApart)
+            R[hb][dt] = mfma16(x, y, R[hb][dt]);
         else
-            sum = mfma16(x, y, sum);
+            S[hb][dt] = mfma16(x, y, S[hb][dt]);
     };
-    auto add_chunk = [&](int hb, int from, int to) {
-        if (NORM) {
+    auto state = [&](int hb, int dt, int r) -> float { return kApart ? S[hb][dt][r] + R[hb][dt][r] : S[hb][dt][r]; };
+    auto clear_apart = [&]() {
 #pragma unroll
-            for (int dt = 0; dt < 4; dt++)
-                if (dt >= from && dt < to && dt / 2 < (hb == ND - 1 ? KS2 : 2)) S[hb][dt] += Sc[dt];
-        }
+        for (int hb = 0; hb < ND; hb++)
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++) {
+                if (kApart) R[hb][dt] = zero;
+                if (NORM) Zr[hb][dt % 2] = zero;
+            }
     };
-    auto add_chunk_z = [&](int hb) {
-        if (NORM) Z[hb][0] += Zc[0], Z[hb][1] += Zc[1];
+    auto add_apart = [&]() {
+        if (kApart) {
+#pragma unroll
+            for (int hb = 0; hb < ND; hb++)
+#pragma unroll
+                for (int dt = 0; dt < 4; dt++) {
+                    if (dt / 2 < (hb == ND - 1 ? KS2 : 2)) S[hb][dt] += R[hb][dt];
+                    if (NORM && dt < 2) Z[hb][dt] += Zr[hb][dt];
+                }
+            clear_apart();
+        }
     };
 
     // A wavefront issues in order, and four of them share the LDS: reads are therefore
     // written out between the matrix instructions they run under, one at a time, and
     // scheduling barriers keep the compiler from regrouping them.
-    Frag af[2][2][3], bfr[2][3], bt[4][3], vf[3];
-    // row-major fragment number i of a chunk (18: b for the quadrant first, then a)
+    Frag af[2][2][PA], bfr[2][PB], bt[4][PB], vf[PV];
+    // row-major fragment number i of a chunk (18 of fp32 rows: b for the quadrant first, then a)
+    constexpr int kRowFrags = 2 * PB + 4 * PA;
     auto rm_frag = [&](const lds_char *pc, int i, int hb) {  // hb: the block of that position
-        const int k = i % 3, ks = (i / 3) % 2, x = i / 6;
-        if (ks >= block_ks(hb)) return;
-        if (x == 0)
-            bfr[ks][k] = lds_frag8x2(pc + k * kTileA + b_addr[ks][0], pc + k * kTileA + b_addr[ks][1]);
-        else
-            af[x - 1][ks][k] = lds_frag16(pc + k * kTileA + a_addr[x - 1][ks]);
+        if (i >= kRowFrags) return;
+        if (i < 2 * PB) {
+            const int k = i % PB, ks = i / PB;
+            if (ks < block_ks(hb))
+                bfr[ks][k] = lds_frag8x2(pc + k * kTileA + b_addr[ks][0], pc + k * kTileA + b_addr[ks][1]);
+        } else {
+            const int k = (i - 2 * PB) % PA, ks = ((i - 2 * PB) / PA) % 2, x = (i - 2 * PB) / (2 * PA);
+            if (ks < block_ks(hb)) af[x][ks][k] = lds_frag16(pc + k * kTileA + a_addr[x][ks]);
+        }
     };
-    // position-major fragment number i of a chunk (15: v first, then b^T tile by tile)
+    // position-major fragment number i of a chunk (15 of fp32 rows: v first, then b^T tile by tile)
     // (pcv: the buffer that holds the chunk's v tile, which is the one of its first block)
-    auto tr_frag_into = [&](Frag (&btx)[4][3], Frag (&vfx)[3], const lds_char *pc,
+    constexpr int kTrFrags = PV + 4 * PB;
+    auto tr_frag_into = [&](Frag (&btx)[4][PB], Frag (&vfx)[PV], const lds_char *pc,
                             const lds_char *pcv, int i, int hb) {
-        if (i >= 3 && (i - 3) / 6 >= block_ks(hb)) return;  // tiles 2, 3: rows 32 .. 63
-        if (i < 3)
+        if (i >= kTrFrags) return;
+        if (i < PV)
             vfx[i] = lds_frag_tr(pcv + i * kTileV + vt_addr[0], pcv + i * kTileV + vt_addr[1]);
         else {
-            const int dt = (i - 3) / 3, k = (i - 3) % 3;
+            const int dt = (i - PV) / PB, k = (i - PV) % PB;
+            if (dt / 2 >= block_ks(hb)) return;  // tiles 2, 3: rows 32 .. 63
             btx[dt][k] = lds_frag_tr(pc + k * kTileA + bt_addr[dt][0], pc + k * kTileA + bt_addr[dt][1]);
         }
     };
@@ -542,46 +617,52 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     int buf = 0;  // LDS buffer of the chunk at hand
     if (n1 > 0) {
         // ---- the first n1 positions of the walk: state update only ----
+        if (kMixed) clear_apart();
+        auto add_first = [&](int hb, int dt, const Frag &x, const Frag &y) {
+            if (kMixed)
+                R[hb][dt] = mfma16(x, y, R[hb][dt]);
+            else
+                S[hb][dt] = mfma16(x, y, S[hb][dt]);
+        };
         // The consumers have little to do here, so they share the producers' work: rows
         // 16 .. 31 of b and v of these chunks are fetched and cut by the consumers (lane
         // 64 w + lane takes the quad that producer lane of the same number would take).
         // The loop is skewed by one chunk: while the matrix instructions of chunk k - 1 run,
         // the fragments of chunk k arrive in the other set of registers.
         const int cid = w * 64 + lane, crow = (T + cid) / QA, cc4 = (T + cid) % QA;
-        const uint32_t b_slb = (uint32_t)op.b_sl * 4, v_slb = (uint32_t)op.v_sl * 4;
-        const char *b_seg = (const char *)op.b + ((int64_t)n * op.b_sn + (int64_t)h * op.b_sh) * 4;
+        const uint32_t b_slb = (uint32_t)op.b_sl * QuadB::bytes, v_slb = (uint32_t)op.v_sl * QuadV::bytes;
+        const char *b_seg = (const char *)op.b + ((int64_t)n * op.b_sn + (int64_t)h * op.b_sh) * QuadB::bytes;
         const char *v_seg = (const char *)op.v +
-                            ((int64_t)n * op.v_sn + (int64_t)h * op.v_sh + F * fb) * 4;
+                            ((int64_t)n * op.v_sn + (int64_t)h * op.v_sh + F * fb) * QuadV::bytes;
         const __amdgpu_buffer_rsrc_t b_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)b_seg, 0, (rows - 1) * b_slb + Dw * 4, kRsrcFlags);
+            (void *)b_seg, 0, (rows - 1) * b_slb + Dw * QuadB::bytes, kRsrcFlags);
         const __amdgpu_buffer_rsrc_t v_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)v_seg, 0, (rows - 1) * v_slb + fw * 4, kRsrcFlags);
+            (void *)v_seg, 0, (rows - 1) * v_slb + fw * QuadV::bytes, kRsrcFlags);
         bool b_in[ND];
 #pragma unroll
         for (int hb = 0; hb < ND; hb++) b_in[hb] = 4 * cc4 + D * hb < Dw;
         const bool v_in = 4 * cc4 < fw;
-        const uint32_t b_goff = (uint32_t)crow * b_slb + 16u * cc4,
-                       v_goff = (uint32_t)crow * v_slb + 16u * cc4;
+        const uint32_t b_goff = (uint32_t)crow * b_slb + 4u * QuadB::bytes * cc4,
+                       v_goff = (uint32_t)crow * v_slb + 4u * QuadV::bytes * cc4;
         const int b_waddr = TpSwizzle<RBA>::addr(crow, 2 * b_tile_column(4 * cc4)),
                   v_waddr = TpSwizzle<RBV>::addr(crow, 8 * cc4);
         struct RawC {
-            u32x4 b, v;
+            typename QuadB::raw b;
+            typename QuadV::raw v;
         };
         RawC rawc[PF];
         // (every request every time, as the producers do: from position n1 on outside the
         // descriptor)
         auto cfetch = [&](RawC &r, int v, int hb) {  // hb = v % ND
             const int row0 = v < n1 ? chunk_row0(so_chunk(v)) : -2 * kChunk;
-            r.b = __builtin_amdgcn_raw_buffer_load_b128(
-                b_rs, b_in[hb] ? b_goff + (uint32_t)(D * 4 * hb) + (uint32_t)row0 * b_slb : kNoRow, 0, 0);
-            if (hb == 0)
-                r.v = __builtin_amdgcn_raw_buffer_load_b128(
-                    v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, 0, 0);
+            r.b = QuadB::load(b_rs, b_in[hb] ? b_goff + (uint32_t)(D * QuadB::bytes * hb) + (uint32_t)row0 * b_slb
+                                             : kNoRow);
+            if (hb == 0) r.v = QuadV::load(v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow);
         };
         const int key_rows = NORM && p.key_len ? (int)max((int64_t)0, min((int64_t)rows, p.key_len[n])) : rows;
         auto ccut_b = [&](const RawC &r, int bufk, int v) {
-            u32x4 x = r.b;
-            if (NORM) {  // (position v of the walk, as the producers do)
+            typename QuadB::raw x = r.b;
+            if constexpr (NORM) {  // (position v of the walk, as the producers do)
                 x = feature_quad(x);
                 const int row0 = chunk_row0(so_chunk(v));
                 if (row0 < 0 || row0 + kChunk > key_rows) {
@@ -589,10 +670,10 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 }
                 if (!b_in[v % ND]) x = u32x4{0, 0, 0, 0};
             }
-            split_quad_to_lds(x, unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
+            QuadB::to_lds(x, unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
         };
         auto ccut_v = [&](const RawC &r, int bufk) {
-            split_quad_to_lds(r.v, unit_pc + bufk * kBufBytes + kOffV, kTileV, v_waddr);
+            QuadV::to_lds(r.v, unit_pc + bufk * kBufBytes + kOffV, kTileV, v_waddr);
         };
 #pragma unroll
         for (int j = 0; j < PF; j++) cfetch(rawc[j], j, j % ND);
@@ -601,7 +682,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
         cfetch(rawc[0], PF, 0);
         wg_barrier();
         FTC_STAMP(13);  // first chunk cut
-        Frag bt2[4][3] = {}, vf2[3] = {};  // (the first round multiplies zeros)
+        Frag bt2[4][PB] = {}, vf2[PV] = {};  // (the first round multiplies zeros)
         int bufn = 1;                      // LDS buffer of the chunk after the one at hand
         for (int c = 0; c < n1; c += PF) {
 #pragma unroll
@@ -617,15 +698,17 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 for (int i = 0; i < 24; i++) {
                     const bool rows_exist = (i % 4) / 2 < block_ks(hp);
                     if (j % 2 == 0) {
-                        if (rows_exist)
-                            S[hp][i % 4] = mfma16(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[hp][i % 4]);
-                        if (NORM && i < 6) Z[hp][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
-                        if (i < 15) tr_frag_into(bt, vf, pc, pcv, i, j % ND);
+                        if (rows_exist && i < 4 * OfS::count)
+                            add_first(hp, i % 4, bt2[i % 4][OfS::x(i / 4)], vf2[OfS::y(i / 4)]);
+                        if constexpr (NORM)
+                            if (i < 6) Z[hp][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
+                        tr_frag_into(bt, vf, pc, pcv, i, j % ND);
                     } else {
-                        if (rows_exist)
-                            S[hp][i % 4] = mfma16(bt[i % 4][kPa[i / 4]], vf[kPb[i / 4]], S[hp][i % 4]);
-                        if (NORM && i < 6) Z[hp][i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
-                        if (i < 15) tr_frag_into(bt2, vf2, pc, pcv, i, j % ND);
+                        if (rows_exist && i < 4 * OfS::count)
+                            add_first(hp, i % 4, bt[i % 4][OfS::x(i / 4)], vf[OfS::y(i / 4)]);
+                        if constexpr (NORM)
+                            if (i < 6) Z[hp][i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
+                        tr_frag_into(bt2, vf2, pc, pcv, i, j % ND);
                     }
                     if (i == 15 && cut_next) ccut_b(rn, bufn, c + j + 1);
                     if (i == 19 && cut_next && (j + 1) % ND == 0) ccut_v(rn, bufn);
@@ -637,22 +720,23 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 wg_barrier();
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if (kMixed && c % 8 == 0) add_apart();
         }
         // the last of these positions (n1 is even: its fragments are in the second set)
 #pragma unroll
         for (int i = 0; i < 24; i++) {
-            if ((i % 4) / 2 < KS2)
-                S[ND - 1][i % 4] = mfma16(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[ND - 1][i % 4]);
-            if (NORM && i < 6)
-                Z[ND - 1][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[ND - 1][i % 2]);
-            if (i < 18) rm_frag(unit_pc + buf * kBufBytes, i, 0);  // our own first chunk is cut
+            if ((i % 4) / 2 < KS2 && i < 4 * OfS::count)
+                add_first(ND - 1, i % 4, bt2[i % 4][OfS::x(i / 4)], vf2[OfS::y(i / 4)]);
+            if constexpr (NORM)
+                if (i < 6) Z[ND - 1][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[ND - 1][i % 2]);
+            rm_frag(unit_pc + buf * kBufBytes, i, 0);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
     } else {
         wg_barrier();
         FTC_STAMP(13);  // first chunk cut
 #pragma unroll
-        for (int i = 0; i < 18; i++) rm_frag(unit_pc, i, 0);
+        for (int i = 0; i < kRowFrags; i++) rm_frag(unit_pc, i, 0);
     }
     if (exchange) {
         // ---- the sum of this segment's rows goes out, the state before the segment comes in ----
@@ -664,6 +748,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
         StateExchange<DX, 1> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);
+        if (kMixed && n1 > 0) add_apart();
         f32x16 Sx[DX][1], X[DX][1];
         if (NORM) {
             Sx[DX - 1][0] = f32x16{};
@@ -692,13 +777,15 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
         }
         if (!NORM && op.s0) add_caller_state();
     }
+    if (kMixed && n1 > 0 && !exchange) add_apart();
+    clear_apart();
     // S_w as pieces in A operand order (slots 0..3 from tile 2 ks, 4..7 from tile 2 ks + 1).
     // Tiles 0 and 1 are final after phase 3 and are cut under phase 4, tiles 2 and 3 after
     // phase 4 and are cut under phase 1 of the next chunk.
     Frag sf[2][3];
     auto cut_s = [&](int hb, int ks, int q) {
         uint32_t o[3];
-        split_pair_under_mfma(S[hb][2 * ks + q / 2][2 * (q % 2)], S[hb][2 * ks + q / 2][2 * (q % 2) + 1], o);
+        split_pair_under_mfma(state(hb, 2 * ks + q / 2, 2 * (q % 2)), state(hb, 2 * ks + q / 2, 2 * (q % 2) + 1), o);
 #pragma unroll
         for (int k = 0; k < 3; k++) sf[ks][k].w[q] = o[k];
     };
@@ -720,7 +807,7 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     auto store_rows = [&](int x) {
         f32x4 o = O4[x][0] + O4[x][1];
         if (NORM) o *= r_den[x];
-        buffer_store4(o_rs, o_in ? o_off + o_lane[x] : kNoRow, o[0], o[1], o[2], o[3]);
+        buffer_store_out(o_rs, o_in ? o_off + o_lane[x] : kNoRow, o[0], o[1], o[2], o[3], (TO *)nullptr);
     };
     f32x4 Pkeep = {0.f, 0.f, 0.f, 0.f};  // the quadrant summed over the blocks so far
     f32x4 Az = {0.f, 0.f, 0.f, 0.f};     // NORM: phi(a) z of the quadrant's positions
@@ -747,14 +834,15 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
             for (int i = 0; i < 12; i++) {
                 const int ks = i % 2, m = i / 2;
-                if (ks < block_ks(hb))
-                    P4[i % 4] = mfma16(bfr[ks][kPa[m]], af[0][ks][kPb[m]], i < 4 ? zero : P4[i % 4]);
+                if (ks < block_ks(hb) && m < OfP::count)
+                    P4[i % 4] = mfma16(bfr[ks][OfP::x(m)], af[0][ks][OfP::y(m)], i < 4 ? zero : P4[i % 4]);
                 else if (i < 4)
                     P4[i % 4] = zero;
                 if (i < 4 && block_ks(hb) > 1) cut_s(hb, 1, i);
-                if (NORM && i >= 8) {
+                if (NORM && i >= 8) {  // z in pieces
                     uint32_t o[3];
-                    split_pair_under_mfma(Z[hb][(i - 8) / 2][2 * (i % 2)], Z[hb][(i - 8) / 2][2 * (i % 2) + 1], o);
+                    split_pair_under_mfma(Z[hb][(i - 8) / 2][2 * (i % 2)] + Zr[hb][(i - 8) / 2][2 * (i % 2)],
+                                          Z[hb][(i - 8) / 2][2 * (i % 2) + 1] + Zr[hb][(i - 8) / 2][2 * (i % 2) + 1], o);
 #pragma unroll
                     for (int k = 0; k < 3; k++) zf[k].w[i - 8] = o[k];
                 }
@@ -771,11 +859,12 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             for (int i = 0; i < 12; i++) {
                 const int x = i % 2, ks = (i / 2) % 2, m = i / 4;  // piece products 0..2
                 if (ks < block_ks(hb))
-                    O4[x][ks] = mfma16(sf[ks][kPa[m]], af[x][ks][kPb[m]], i < 4 && hb == 0 ? zero : O4[x][ks]);
+                    O4[x][ks] = mfma16(sf[ks][OfO::x(m)], af[x][ks][OfO::y(m)], i < 4 && hb == 0 ? zero : O4[x][ks]);
                 else if (i < 4 && hb == 0)
                     O4[x][ks] = zero;
                 if (i < 3) tr_frag_into(bt, vf, pc, pcv, 12 + i, hb);
-                if (NORM && i >= 6) Az = mfma16(zf[kPa[i - 6]], af[0][0][kPb[i - 6]], i == 6 && hb == 0 ? zero : Az);
+                if constexpr (NORM)
+                    if (i >= 6) Az = mfma16(zf[OfO::x(i - 6)], af[0][0][OfO::y(i - 6)], i == 6 && hb == 0 ? zero : Az);
                 if (i == 4) {
                     P = (P4[0] + P4[1]) + (P4[2] + P4[3]);
                     if (hb > 0) P += Pkeep;
@@ -807,9 +896,12 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
 #pragma unroll
             for (int i = 0; i < 12; i++) {
                 const int x = i % 2, ks = (i / 2) % 2, m = 3 + i / 4;  // piece products 3..5
-                if (ks < block_ks(hb)) O4[x][ks] = mfma16(sf[ks][kPa[m]], af[x][ks][kPb[m]], O4[x][ks]);
-                add_product(S[hb][i % 2], Sc[i % 2], bt[i % 2][kPa[i / 2]], vf[kPb[i / 2]], i < 2);
-                if (NORM && i < 6) Zc[i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, i < 2 ? zero : Zc[i % 2]);
+                if (ks < block_ks(hb) && m < OfO::count)
+                    O4[x][ks] = mfma16(sf[ks][OfO::x(m)], af[x][ks][OfO::y(m)], O4[x][ks]);
+                if (i < 2 * OfS::count)
+                    add_product(hb, i % 2, bt[i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)]);
+                if constexpr (NORM)
+                    if (i < 6) Zr[hb][i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, Zr[hb][i % 2]);
                 if (NORM && i == 6 && last_block) {
                     P_sum = sum_of_lane_groups(P_sum);
                     if (g == 0) den_mem[c & 1][16 * ih + ln][w >> 1] = (has_z ? Az[0] : 0.f) + P_sum;
@@ -820,8 +912,6 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             buf = next_buf(buf);
             wg_barrier();
             if (c == c0 + 4) FTC_STAMP(4);
-            add_chunk(hb, 0, 2);
-            add_chunk_z(hb);
             // All of Pt is in LDS and the next chunk is cut: its row-major fragments are
             // requested under what follows.
             // phase 4: (3) for tiles 2 and 3 in turn with (2a) Ot_w += v_w^T Pt; underneath:
@@ -850,30 +940,32 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                if (block_ks(hb) > 1)
-                    add_product(S[hb][2 + i % 2], Sc[2 + i % 2], bt[2 + i % 2][kPa[i / 2]], vf[kPb[i / 2]], i < 2);
+                if (block_ks(hb) > 1 && i < 2 * OfS::count)
+                    add_product(hb, 2 + i % 2, bt[2 + i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)]);
                 cut_s((hb + 1) % ND, 0, i);
                 rm_frag(pn, i, (hb + 1) % ND);  // (past the last chunk: a buffer of zeros)
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int i = 0; i < 12; i++) {
-                if (i < 8 && block_ks(hb) > 1) {
+                if (4 + i < 2 * OfS::count && block_ks(hb) > 1) {
                     const int t = 4 + i;
-                    add_product(S[hb][2 + t % 2], Sc[2 + t % 2], bt[2 + t % 2][kPa[t / 2]], vf[kPb[t / 2]], false);
+                    add_product(hb, 2 + t % 2, bt[2 + t % 2][OfS::x(t / 2)], vf[OfS::y(t / 2)]);
                 }
                 const int x = i % 2, m = i / 2;
-                if (last_block) O4[x][m % 2] = mfma16(vf[kPa[m]], pf[x][kPb[m]], O4[x][m % 2]);
+                if (last_block && m < OfV::count)
+                    O4[x][m % 2] = mfma16(vf[OfV::x(m)], pf[x][OfV::y(m)], O4[x][m % 2]);
                 rm_frag(pn, 4 + i, (hb + 1) % ND);
                 if (i < 2) rm_frag(pn, 16 + i, (hb + 1) % ND);
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (c == c0 + 4) FTC_STAMP(5);
-            add_chunk(hb, 2, 4);
+            if (kApart && last_block && (c - c0) % 8 == 7) add_apart();
             o_off = (uint32_t)chunk_row0(c) * o_slb;
             if (c == c0 + 4) FTC_STAMP(6);
         }
     }
+    add_apart();
     store_rows(0);
     store_rows(1);
     FTC_STAMP(15);  // last rows on their way
@@ -909,6 +1001,18 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
                 __hip_atomic_store(hdr + kHdrDone, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+}
+
+template <int ND, int KS2, bool NORM>
+__global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
+    __shared__ __align__(16) char pieces_mem[kTpPieceBytes<3, 3, 3>];
+    __shared__ __align__(16) char pt_mem[kTpPtBytes];
+    __shared__ __align__(16) float den_mem[NORM ? 2 : 1][NORM ? kChunk : 1][2];
+    __shared__ uint32_t order_sh;
+    uint32_t which, chain;
+    tp_workgroup(p, which, chain);
+    scan_tp_body<ND, KS2, NORM, 3, 3, 3, float>(ws_ptr, p, which, chain, (lds_char *)pieces_mem, (lds_char *)pt_mem,
+                                                den_mem, &order_sh);
 }
 
 }  // namespace mfma

@@ -6,23 +6,21 @@ namespace mfma {
 
 namespace {
 template <int KS>
-void launch(void *ws, const ScanArgs &args, bool mixed, bool odd, hipStream_t stream) {
+void launch(void *ws, const ScanArgs &args, bool odd, hipStream_t stream) {
     // (grid as for launch_scan_tp)
     const dim3 grid((unsigned)args.total_waves), block(768);
-    if (mixed)
-        hipLaunchKernelGGL((scan_tph_kernel<KS, true, false>), grid, block, 0, stream, (uint32_t *)ws, args);
-    else if (odd)
-        hipLaunchKernelGGL((scan_tph_kernel<KS, false, true>), grid, block, 0, stream, (uint32_t *)ws, args);
+    if (odd)
+        hipLaunchKernelGGL((scan_tph_kernel<KS, true>), grid, block, 0, stream, (uint32_t *)ws, args);
     else
-        hipLaunchKernelGGL((scan_tph_kernel<KS, false, false>), grid, block, 0, stream, (uint32_t *)ws, args);
+        hipLaunchKernelGGL((scan_tph_kernel<KS, false>), grid, block, 0, stream, (uint32_t *)ws, args);
 }
 }  // namespace
 
-void launch_scan_tph(void *ws, const ScanArgs &args, bool mixed, bool odd, hipStream_t stream) {
+void launch_scan_tph(void *ws, const ScanArgs &args, bool odd, hipStream_t stream) {
     if (args.tp_d <= 32)
-        launch<1>(ws, args, mixed, odd, stream);
+        launch<1>(ws, args, odd, stream);
     else
-        launch<2>(ws, args, mixed, odd, stream);
+        launch<2>(ws, args, odd, stream);
 }
 
 }  // namespace mfma

@@ -1,7 +1,5 @@
-// Chain-parallel form of the MFMA causal scan for gfx950 on the fp16 matrix path: fp32 rows
-// (or, in the MIX form of the kernel, any operand in bf16: such rows are widened as they arrive
-// and rounded to nearest even as they leave; their low pieces are zero), states of up to
-// 64 x 64 per workgroup (output columns beyond 64 have a workgroup of their own, widths that do
+// Chain-parallel form of the MFMA causal scan for gfx950 on the fp16 matrix path: fp32 rows, states of
+// up to 64 x 64 per workgroup (output columns beyond 64 have a workgroup of their own, widths that do
 // not fill the block are clipped).
 //
 //   out[c, l, f] = sum_{j <= l} (a[c,l,:] . b[c,j,:]) * v[c,j,f]      (REV: j >= l)
@@ -219,21 +217,15 @@ __device__ __forceinline__ void raise_slot(lds_u32_t *slots, int k, int pos, con
     }
 }
 
-// four bf16 values in two words -> the same values as fp32 bit patterns
-__device__ __forceinline__ u32x4 widen_bf16_quad(const u32x4 r) {
-    return u32x4{r.x << 16, r.x & 0xffff0000u, r.y << 16, r.y & 0xffff0000u};
-}
-
 // KS: groups of 32 rows of the state (1: a state of up to 32 rows, which skips the matrix
-// instructions and fragment reads of the empty half).  MIX: rows of either element type, as
-// ScanOperands::pad says scan by scan (false: all rows fp32).
+// instructions and fragment reads of the empty half).
 // ODD: fp32 rows of any width on 4-byte boundaries.  The requests stay 16 bytes per lane (the
 // hardware asks for 4-byte alignment and checks the descriptor's end word by word); a lane whose
 // quad straddles the end of a row clears the words that belong to the next one when the
 // look-ahead first touches them, and stores such a quad word by word.  Measured against dense
 // zero-padded copies of the operands and results (8 x 16 chains, L=4096, 50 x 50, forward + backward):
 // 940 -> 387 us; a chunk costs what one of 64 x 64 does.
-template <int KS, bool MIX, bool ODD>
+template <int KS, bool ODD>
 __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     constexpr int D = 64, F = 64;              // one block of state rows and of output columns
     constexpr int T = 512;                     // producer lanes (eight wavefronts)
@@ -339,21 +331,18 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     if (producer) {
         // =========================== producers ===========================
         const int ptid = (wave - 4) * 64 + lane;
-        const bool a_bf = MIX && (op.pad & kRowsBf16A), b_bf = MIX && (op.pad & kRowsBf16B),
-                   v_bf = MIX && (op.pad & kRowsBf16V);
-        const uint32_t a_es = a_bf ? 2 : 4, b_es = b_bf ? 2 : 4, v_es = v_bf ? 2 : 4;  // bytes
-        const uint32_t a_slb = (uint32_t)op.a_sl * a_es, b_slb = (uint32_t)op.b_sl * b_es,
-                       v_slb = (uint32_t)op.v_sl * v_es;
-        const char *a_seg = (const char *)op.a + ((int64_t)n * op.a_sn + (int64_t)h * op.a_sh) * a_es;
-        const char *b_seg = (const char *)op.b + ((int64_t)n * op.b_sn + (int64_t)h * op.b_sh) * b_es;
+        const uint32_t a_slb = (uint32_t)op.a_sl * 4, b_slb = (uint32_t)op.b_sl * 4,
+                       v_slb = (uint32_t)op.v_sl * 4;
+        const char *a_seg = (const char *)op.a + ((int64_t)n * op.a_sn + (int64_t)h * op.a_sh) * 4;
+        const char *b_seg = (const char *)op.b + ((int64_t)n * op.b_sn + (int64_t)h * op.b_sh) * 4;
         const char *v_seg = (const char *)op.v +
-                            ((int64_t)n * op.v_sn + (int64_t)h * op.v_sh + F * fb) * v_es;
+                            ((int64_t)n * op.v_sn + (int64_t)h * op.v_sh + F * fb) * 4;
         const __amdgpu_buffer_rsrc_t a_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)a_seg, 0, (rows - 1) * a_slb + Dw * a_es, kRsrcFlags);
+            (void *)a_seg, 0, (rows - 1) * a_slb + Dw * 4, kRsrcFlags);
         const __amdgpu_buffer_rsrc_t b_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)b_seg, 0, (rows - 1) * b_slb + Dw * b_es, kRsrcFlags);
+            (void *)b_seg, 0, (rows - 1) * b_slb + Dw * 4, kRsrcFlags);
         const __amdgpu_buffer_rsrc_t v_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)v_seg, 0, (rows - 1) * v_slb + fw * v_es, kRsrcFlags);
+            (void *)v_seg, 0, (rows - 1) * v_slb + fw * 4, kRsrcFlags);
         // One quad (four columns of one row) of every operand per lane and position.  Widths
         // that do not fill the block: a lane whose four columns lie beyond the width asks
         // outside the descriptor and cuts zeros (widths are multiples of 4).
@@ -361,9 +350,9 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         const int prow = ptid / QA, pc4 = ptid % QA;
         const bool ab_in = 4 * pc4 < Dw;
         const bool v_in = 4 * pc4 < fw;
-        const uint32_t a_goff = (uint32_t)prow * a_slb + 4u * a_es * pc4,
-                       b_goff = (uint32_t)prow * b_slb + 4u * b_es * pc4,
-                       v_goff = (uint32_t)prow * v_slb + 4u * v_es * pc4;
+        const uint32_t a_goff = (uint32_t)prow * a_slb + 16u * pc4,
+                       b_goff = (uint32_t)prow * b_slb + 16u * pc4,
+                       v_goff = (uint32_t)prow * v_slb + 16u * pc4;
         const int a_waddr = TpSwizzle<RBA>::addr(prow, 8 * pc4),
                   b_waddr = TpSwizzle<RBA>::addr(prow, 2 * b_tile_column(4 * pc4)),
                   v_waddr = TpSwizzle<RBV>::addr(prow, 8 * pc4);
@@ -377,24 +366,10 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         auto own_words = [&](u32x4 &r, const uint32_t (&m)[3]) {
             if (ODD) r = u32x4{r.x, r.y & m[0], r.z & m[1], r.w & m[2]};
         };
-        struct Raw {  // (bf16 rows: the quad in the first two words)
+        struct Raw {
             u32x4 a, b, v;
         };
         Raw raw[PF];
-        // (MIX: the same two 8-byte requests whatever the type -- no branch around a request,
-        // which would end the run of requests in flight; the second one of a bf16 quad asks
-        // outside the descriptor)
-        auto load_quad = [&](const __amdgpu_buffer_rsrc_t rs, uint32_t off, bool bf) -> u32x4 {
-            if (!MIX) return __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
-            const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
-            const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(rs, bf ? kNoRow : off + 8u, 0, 0);
-            return u32x4{lo.x, lo.y, hi.x, hi.y};
-        };
-        // (bf16 quads are widened in place, once, when the look-ahead first touches them: one
-        // position later the cut finds fp32 bit patterns whatever the rows held)
-        auto widen = [&](u32x4 &r, bool bf) {
-            if (MIX && bf) r = widen_bf16_quad(r);
-        };
         // Every request is made every time, whether its rows exist or not (a chunk walked for
         // its state alone needs no rows of a; positions past the end of the walk have no
         // rows): a request outside the descriptor costs no memory traffic and reads as zero,
@@ -404,14 +379,13 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
             const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
             const int row0_x = v >= n1 ? row0 : -2 * kChunk;
             // (the sums wrap: a chunk that starts before the first row has its later rows in place)
-            r.a = load_quad(a_rs, ab_in ? a_goff + (uint32_t)row0_x * a_slb : kNoRow, a_bf);
-            r.b = load_quad(b_rs, ab_in ? b_goff + (uint32_t)row0 * b_slb : kNoRow, b_bf);
-            r.v = load_quad(v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, v_bf);
+            r.a = __builtin_amdgcn_raw_buffer_load_b128(a_rs, ab_in ? a_goff + (uint32_t)row0_x * a_slb : kNoRow, 0, 0);
+            r.b = __builtin_amdgcn_raw_buffer_load_b128(b_rs, ab_in ? b_goff + (uint32_t)row0 * b_slb : kNoRow, 0, 0);
+            r.v = __builtin_amdgcn_raw_buffer_load_b128(v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, 0, 0);
         };
         // the largest magnitudes of the rows of a position against the ceilings (rows that
         // were not asked for read as zeros); k: that position's slot
         auto look_ahead = [&](Raw &r, int k, int pos) {
-            widen(r.a, a_bf), widen(r.b, b_bf), widen(r.v, v_bf);
             own_words(r.a, ab_own), own_words(r.b, ab_own), own_words(r.v, v_own);
             raise_slot(slots, k, pos, ce, max_abs4(r.a, 0.f), max_abs4(r.b, 0.f), max_abs4(r.v, 0.f), lane);
         };
@@ -472,12 +446,10 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
 
     // =========================== consumers ===========================
     const int ln = lane & 15, g = lane >> 4;
-    const bool o_bf = MIX && (op.pad & kRowsBf16Out);
-    const uint32_t o_es = o_bf ? 2 : 4;  // bytes
-    const uint32_t o_slb = (uint32_t)op.o_sl * o_es;
-    char *o_seg = (char *)op.out + ((int64_t)n * op.o_sn + (int64_t)h * op.o_sh + F * fb) * o_es;
+    const uint32_t o_slb = (uint32_t)op.o_sl * 4;
+    char *o_seg = (char *)op.out + ((int64_t)n * op.o_sn + (int64_t)h * op.o_sh + F * fb) * 4;
     const __amdgpu_buffer_rsrc_t o_rs =
-        __builtin_amdgcn_make_buffer_rsrc((void *)o_seg, 0, (rows - 1) * o_slb + fw * o_es, kRsrcFlags);
+        __builtin_amdgcn_make_buffer_rsrc((void *)o_seg, 0, (rows - 1) * o_slb + fw * 4, kRsrcFlags);
     // Pt quadrant of this wavefront (see scan_tp_kernel)
     const int jh = w == 0 ? 0 : w == 1 ? 1 : ((w == 2) == REV ? 1 : 0);
     const int ih = w == 0 ? 0 : w == 1 ? 1 : 1 - jh;
@@ -515,7 +487,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     uint32_t o_lane[2];
 #pragma unroll
     for (int x = 0; x < 2; x++)
-        o_lane[x] = (uint32_t)(16 * (x ^ ih) + ln) * o_slb + o_es * (16 * w + 4 * g);
+        o_lane[x] = (uint32_t)(16 * (x ^ ih) + ln) * o_slb + 4u * (16 * w + 4 * g);
     // (columns beyond the width are not stored; ODD: a quad that straddles the width is stored
     // word by word, by the one wavefront that has such a quad)
     const int o_cols = fw - (16 * w + 4 * g);
@@ -713,20 +685,13 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         const float y0 = __builtin_amdgcn_ldexpf(O[x][0], Xo), y1 = __builtin_amdgcn_ldexpf(O[x][1], Xo),
                     y2 = __builtin_amdgcn_ldexpf(O[x][2], Xo), y3 = __builtin_amdgcn_ldexpf(O[x][3], Xo);
         const uint32_t at = o_in ? o_off + o_lane[x] : kNoRow;
-        if (!MIX) {
-            buffer_store_out(o_rs, at, y0, y1, y2, y3, (float *)nullptr);
-            if (o_straddles) {
-                const uint32_t first = o_off + o_lane[x];
-                const bool some = o_cols < 4;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y0), o_rs, some && o_cols > 0 ? first : kNoRow, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y1), o_rs, some && o_cols > 1 ? first + 4u : kNoRow, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y2), o_rs, some && o_cols > 2 ? first + 8u : kNoRow, 0, 0);
-            }
-        } else if (o_bf) {  // (a branch that the whole launch takes one way: no request hangs on it)
-            const u32x2 packed = {pack_bf16_rne(y0, y1), pack_bf16_rne(y2, y3)};
-            __builtin_amdgcn_raw_buffer_store_b64(packed, o_rs, at, 0, 0);
-        } else {
-            buffer_store_out(o_rs, at, y0, y1, y2, y3, (float *)nullptr);
+        buffer_store_out(o_rs, at, y0, y1, y2, y3, (float *)nullptr);
+        if (o_straddles) {
+            const uint32_t first = o_off + o_lane[x];
+            const bool some = o_cols < 4;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y0), o_rs, some && o_cols > 0 ? first : kNoRow, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y1), o_rs, some && o_cols > 1 ? first + 4u : kNoRow, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y2), o_rs, some && o_cols > 2 ? first + 8u : kNoRow, 0, 0);
         }
     };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
