@@ -1129,15 +1129,33 @@ int ftc_causal_dot_plan(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
     return rc;
 }
 
-int64_t ftc_causal_linear_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E,
-                                                    int64_t M, int32_t dtype) {
+// rows of the fused attention: 32 or 64 values, and 128 for the functions that take those
+static bool attention_widths(int64_t E, int64_t M, bool wide) {
+    auto one = [wide](int64_t w) { return w == 32 || w == 64 || (wide && w == 128); };
+    return one(E) && one(M);
+}
+static const char *attention_sizes(bool wide) { return wide ? "{32, 64, 128}" : "{32, 64}"; }
+
+static int64_t attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E, int64_t M, int32_t dtype,
+                                         bool wide) {
     if (N < 0 || H < 0 || L < 0 || E < 0 || M < 0) return fail(FTC_ERR_INVALID, "negative size");
     if (dtype != FTC_F32 && dtype != FTC_BF16) return fail(FTC_ERR_INVALID, "unknown dtype");
-    if (dtype != FTC_F32 || !(E == 32 || E == 64) || !(M == 32 || M == 64))
-        return fail(FTC_ERR_UNSUPPORTED,
-                    "the fused attention kernel takes fp32 rows with E, M in {32, 64}");
+    if (dtype != FTC_F32 || !attention_widths(E, M, wide))
+        return fail(FTC_ERR_UNSUPPORTED, "the fused attention kernel takes fp32 rows with E, M in %s",
+                    attention_sizes(wide));
     if (N * H * L == 0) return 0;
+    if ((E > 64 || M > 64) && !fused_attention_wide_covers(N, H, L, E, M))
+        return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for these sizes");
     return fused_attention_workspace_bytes(N, H, L, E, M);
+}
+
+int64_t ftc_causal_linear_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E,
+                                                    int64_t M, int32_t dtype) {
+    return attention_workspace_bytes(N, H, L, E, M, dtype, false);
+}
+int64_t ftc_causal_linear_attention_wide_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E,
+                                                         int64_t M, int32_t dtype) {
+    return attention_workspace_bytes(N, H, L, E, M, dtype, true);
 }
 
 static int check_denominators(const ftc_tensor4 *den, const Dims &d) {
@@ -1148,11 +1166,10 @@ static int check_denominators(const ftc_tensor4 *den, const Dims &d) {
     return FTC_OK;
 }
 
-int ftc_causal_linear_attention_forward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
-                                        const ftc_tensor4 *values, const int64_t *key_lengths,
-                                        float eps, const ftc_tensor4 *out,
-                                        const ftc_tensor4 *denominators, void *workspace,
-                                        size_t workspace_bytes, void *stream) {
+static int attention_forward(const ftc_tensor4 *queries, const ftc_tensor4 *keys, const ftc_tensor4 *values,
+                             const int64_t *key_lengths, float eps, const ftc_tensor4 *out,
+                             const ftc_tensor4 *denominators, void *workspace, size_t workspace_bytes,
+                             void *stream, bool wide) {
     Dims d;
     int rc = read_dims(queries, values, &d);
     if (rc) return rc;
@@ -1162,9 +1179,9 @@ int ftc_causal_linear_attention_forward(const ftc_tensor4 *queries, const ftc_te
     if ((rc = check_tensor(out, "out", d.N, d.H, d.L, d.M, FTC_F32, FTC_F32))) return rc;
     if (denominators && (rc = check_denominators(denominators, d))) return rc;
     if (!(eps == eps)) return fail(FTC_ERR_INVALID, "eps is not a number");
-    if (!(d.E == 32 || d.E == 64) || !(d.M == 32 || d.M == 64))
-        return fail(FTC_ERR_UNSUPPORTED,
-                    "the fused attention kernel takes fp32 rows with E, M in {32, 64}");
+    if (!attention_widths(d.E, d.M, wide))
+        return fail(FTC_ERR_UNSUPPORTED, "the fused attention kernel takes fp32 rows with E, M in %s",
+                    attention_sizes(wide));
     if (d.N * d.H * d.L == 0) return FTC_OK;
     const ScanDesc fwd = {as_operand(queries), as_operand(keys), as_operand(values),
                           as_operand_out(out), false};
@@ -1181,6 +1198,23 @@ int ftc_causal_linear_attention_forward(const ftc_tensor4 *queries, const ftc_te
     }
     return mfma_scan(&fwd, 1, d.N, d.H, d.L, workspace, workspace_bytes, (hipStream_t)stream,
                      &fused);
+}
+
+int ftc_causal_linear_attention_forward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
+                                        const ftc_tensor4 *values, const int64_t *key_lengths,
+                                        float eps, const ftc_tensor4 *out,
+                                        const ftc_tensor4 *denominators, void *workspace,
+                                        size_t workspace_bytes, void *stream) {
+    return attention_forward(queries, keys, values, key_lengths, eps, out, denominators, workspace, workspace_bytes,
+                             stream, false);
+}
+int ftc_causal_linear_attention_wide_forward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
+                                             const ftc_tensor4 *values, const int64_t *key_lengths,
+                                             float eps, const ftc_tensor4 *out,
+                                             const ftc_tensor4 *denominators, void *workspace,
+                                             size_t workspace_bytes, void *stream) {
+    return attention_forward(queries, keys, values, key_lengths, eps, out, denominators, workspace, workspace_bytes,
+                             stream, true);
 }
 
 int ftc_causal_linear_attention(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
@@ -1207,23 +1241,32 @@ static int64_t attention_backward_layout(int64_t N, int64_t H, int64_t L, int64_
     return at;
 }
 
-int64_t ftc_causal_linear_attention_backward_workspace_bytes(int64_t N, int64_t H, int64_t L,
-                                                             int64_t E, int64_t M, int32_t dtype) {
+static int64_t attention_backward_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E, int64_t M,
+                                                  int32_t dtype, bool wide) {
     if (N < 0 || H < 0 || L < 0 || E < 0 || M < 0) return fail(FTC_ERR_INVALID, "negative size");
-    if (dtype != FTC_F32 || !(E == 32 || E == 64) || !(M == 32 || M == 64))
-        return fail(FTC_ERR_UNSUPPORTED,
-                    "the fused attention backward takes fp32 rows with E, M in {32, 64}");
+    if (dtype != FTC_F32 || !attention_widths(E, M, wide))
+        return fail(FTC_ERR_UNSUPPORTED, "the fused attention backward takes fp32 rows with E, M in %s",
+                    attention_sizes(wide));
     if (N * H * L == 0) return 0;
     int64_t offset[6];
     return attention_backward_layout(N, H, L, E, M, offset);
 }
 
-int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
-                                         const ftc_tensor4 *values, const int64_t *key_lengths,
-                                         const ftc_tensor4 *out, const ftc_tensor4 *denominators,
-                                         const ftc_tensor4 *grad_out, const ftc_tensor4 *grad_queries,
-                                         const ftc_tensor4 *grad_keys, const ftc_tensor4 *grad_values,
-                                         void *workspace, size_t workspace_bytes, void *stream) {
+int64_t ftc_causal_linear_attention_backward_workspace_bytes(int64_t N, int64_t H, int64_t L,
+                                                             int64_t E, int64_t M, int32_t dtype) {
+    return attention_backward_workspace_bytes(N, H, L, E, M, dtype, false);
+}
+int64_t ftc_causal_linear_attention_wide_backward_workspace_bytes(int64_t N, int64_t H, int64_t L,
+                                                                  int64_t E, int64_t M, int32_t dtype) {
+    return attention_backward_workspace_bytes(N, H, L, E, M, dtype, true);
+}
+
+static int attention_backward(const ftc_tensor4 *queries, const ftc_tensor4 *keys, const ftc_tensor4 *values,
+                              const int64_t *key_lengths, const ftc_tensor4 *out,
+                              const ftc_tensor4 *denominators, const ftc_tensor4 *grad_out,
+                              const ftc_tensor4 *grad_queries, const ftc_tensor4 *grad_keys,
+                              const ftc_tensor4 *grad_values, void *workspace, size_t workspace_bytes,
+                              void *stream, bool wide) {
     Dims d;
     int rc = read_dims(queries, values, &d);
     if (rc) return rc;
@@ -1240,9 +1283,9 @@ int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_t
         return rc;
     if (grad_values && (rc = check_tensor(grad_values, "grad_values", d.N, d.H, d.L, d.M, FTC_F32, FTC_F32)))
         return rc;
-    if (!(d.E == 32 || d.E == 64) || !(d.M == 32 || d.M == 64))
-        return fail(FTC_ERR_UNSUPPORTED,
-                    "the fused attention backward takes fp32 rows with E, M in {32, 64}");
+    if (!attention_widths(d.E, d.M, wide))
+        return fail(FTC_ERR_UNSUPPORTED, "the fused attention backward takes fp32 rows with E, M in %s",
+                    attention_sizes(wide));
     if (d.N * d.H * d.L == 0) return FTC_OK;
     for (const ftc_tensor4 *t : {queries, keys, values, out, grad_out, grad_queries, grad_keys})
         if (t && ((uintptr_t)t->ptr % 16 || t->stride[0] % 4 || t->stride[1] % 4 || t->stride[2] % 4))
@@ -1284,6 +1327,25 @@ int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_t
     if (err != hipSuccess) return fail(FTC_ERR_HIP, "attention backward launch failed: %s", hipGetErrorString(err));
     note_kernel("attention backward: prep, three scans, prefix sums");
     return FTC_OK;
+}
+
+int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
+                                         const ftc_tensor4 *values, const int64_t *key_lengths,
+                                         const ftc_tensor4 *out, const ftc_tensor4 *denominators,
+                                         const ftc_tensor4 *grad_out, const ftc_tensor4 *grad_queries,
+                                         const ftc_tensor4 *grad_keys, const ftc_tensor4 *grad_values,
+                                         void *workspace, size_t workspace_bytes, void *stream) {
+    return attention_backward(queries, keys, values, key_lengths, out, denominators, grad_out, grad_queries,
+                              grad_keys, grad_values, workspace, workspace_bytes, stream, false);
+}
+int ftc_causal_linear_attention_wide_backward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
+                                              const ftc_tensor4 *values, const int64_t *key_lengths,
+                                              const ftc_tensor4 *out, const ftc_tensor4 *denominators,
+                                              const ftc_tensor4 *grad_out, const ftc_tensor4 *grad_queries,
+                                              const ftc_tensor4 *grad_keys, const ftc_tensor4 *grad_values,
+                                              void *workspace, size_t workspace_bytes, void *stream) {
+    return attention_backward(queries, keys, values, key_lengths, out, denominators, grad_out, grad_queries,
+                              grad_keys, grad_values, workspace, workspace_bytes, stream, true);
 }
 
 }  // extern "C"

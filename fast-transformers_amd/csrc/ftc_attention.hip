@@ -28,8 +28,11 @@ namespace ftc {
 namespace {
 
 constexpr int kRun = 4;                    // consecutive positions per thread of the finish kernel
-constexpr int kGroups = 32;                // ... whose workgroup has this many groups of 16 lanes
+constexpr int kGroups = 32;                // ... whose workgroup has this many groups of lanes
 constexpr int kSegment = kGroups * kRun;   // positions per workgroup
+// (LANES: lanes of a group, which hold a row of up to 4 LANES values: 16, or 32 for rows of 128.
+// Measured, forward and backward at 128 x 128, us, autograd through two scans and the element-wise
+// passes / the fused calls: 32 chains, L=161 372 / 90; 128 chains, L=1000 824 / 475.)
 
 __device__ __forceinline__ float phi(float x) {
     return x > 0.f ? x + 1.f : __builtin_amdgcn_exp2f(x * 1.44269502f);
@@ -61,28 +64,30 @@ struct RowsOut {
     int64_t sn, sh, sl;
 };
 
-// One workgroup per (chain, segment); 16 lanes per position, lane c of a group takes columns
-// 4 c .. 4 c + 3, and the 16 groups walk the segment 16 positions at a time.
+// One workgroup per (chain, segment); LANES lanes per position, lane c of a group takes columns
+// 4 c .. 4 c + 3, and the groups walk the segment one position each at a time.
 //   Qf, Kf (dense rows of E floats), gz (dense rows of M floats), dd (one float per position)
 //   sums[(chain nseg + seg) 2 E + e]     = sum_{l in segment} Kf[l][e]
 //   sums[(chain nseg + seg) 2 E + E + e] = sum_{l in segment} dd[l] Qf[l][e]
+template <int LANES>
 __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(
     Rows q, Rows k, Rows g, Rows out, Rows den, const int64_t *__restrict__ key_len, int H, int L,
     int E, int M, int nseg, float *__restrict__ Qf, float *__restrict__ Kf, float *__restrict__ gz,
     float *__restrict__ dd, float *__restrict__ sums) {
-    __shared__ float4 part[2][16][16];
+    constexpr int kRows = 256 / LANES;  // positions at a time
+    __shared__ float4 part[2][kRows][LANES];
     // (the heads of one batch entry and segment in neighbouring workgroups: with heads
     // interleaved in memory their rows lie side by side)
     const int h = blockIdx.x % H, seg = (blockIdx.x / H) % nseg, n = blockIdx.x / (H * nseg);
     const int64_t chain = (int64_t)n * H + h;
-    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+    const int r = threadIdx.x / LANES, c = threadIdx.x % LANES;
     const int len = key_len ? (int)min<int64_t>(key_len[n], L) : L;
     const bool has_e = 4 * c < E, has_m = 4 * c < M;
     const int ce = has_e ? 4 * c : 0, cm = has_m ? 4 * c : 0;
     float4 sk = zero4(), sq = zero4();
 #pragma unroll 4
-    for (int p = 0; p < kSegment / 16; p++) {
-        const int l = seg * kSegment + p * 16 + r;
+    for (int p = 0; p < kSegment / kRows; p++) {
+        const int l = seg * kSegment + p * kRows + r;
         const bool live = l < L;
         const int lc = live ? l : L - 1;
         const int64_t pos = chain * L + lc;
@@ -92,9 +97,9 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(
         const float4 o = *(const float4 *)(out.ptr + n * out.sn + h * out.sh + lc * out.sl + cm);
         const float z = 1.0f / den.ptr[n * den.sn + h * den.sh + lc * den.sl];
         float dot = has_m ? (gg.x * o.x + gg.y * o.y) + (gg.z * o.z + gg.w * o.w) : 0.f;
-        // sum over the 16 lanes of the position
+        // sum over the lanes of the position
 #pragma unroll
-        for (int off = 8; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 16);
+        for (int off = LANES / 2; off > 0; off >>= 1) dot += __shfl_xor(dot, off, LANES);
         const float d = -dot * z;
         const float4 xf = phi(x), yf = lc < len ? phi(y) : zero4();
         if (live) {
@@ -111,10 +116,10 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(
     part[0][r][c] = sk;
     part[1][r][c] = sq;
     __syncthreads();
-    if (threadIdx.x < 32) {  // 16 lanes per kind of sum, the groups added in a fixed order
-        const int which = threadIdx.x >> 4;
+    if (threadIdx.x < 2 * LANES) {  // LANES lanes per kind of sum, the groups added in a fixed order
+        const int which = threadIdx.x / LANES;
         float4 t = part[which][0][c];
-        for (int i = 1; i < 16; i++) t = t + part[which][i][c];
+        for (int i = 1; i < kRows; i++) t = t + part[which][i][c];
         if (has_e) *(float4 *)(sums + ((chain * nseg + seg) * 2 + which) * E + ce) = t;
     }
 }
@@ -123,8 +128,9 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(
 // in place, each sum in the fixed order that a walk along the chain would take (ascending for
 // the first kind, descending for the second).  One workgroup per chain, one lane per kind and
 // column; eight totals are in flight at a time.
-__global__ __launch_bounds__(128) void attn_bwd_totals_kernel(float *__restrict__ sums, int E, int nseg) {
-    const int which = threadIdx.x >> 6, col = threadIdx.x & 63;
+template <int LANES>
+__global__ __launch_bounds__(8 * LANES) void attn_bwd_totals_kernel(float *__restrict__ sums, int E, int nseg) {
+    const int which = threadIdx.x / (4 * LANES), col = threadIdx.x % (4 * LANES);
     if (col >= E) return;
     float *s = sums + ((int64_t)blockIdx.x * nseg * 2 + which) * E + col;
     const int64_t step = 2 * (int64_t)E;
@@ -145,20 +151,21 @@ __global__ __launch_bounds__(128) void attn_bwd_totals_kernel(float *__restrict_
     }
 }
 
-// One workgroup of 32 groups per (chain, segment); 16 lanes per position as above, and group r takes the
-// run of kRun consecutive positions seg kSegment + r kRun ...  dq and dk hold the scans'
+// One workgroup of 32 groups per (chain, segment); LANES lanes per position as above, and
+// group r takes the run of kRun consecutive positions seg kSegment + r kRun ...  dq and dk hold the scans'
 // results on entry:
 //   dq[l] = (dq[l] + dd[l] sum_{j <= l} Kf[j]) phi'(q[l])
 //   dk[j] = (dk[j] + sum_{l >= j} dd[l] Qf[l]) phi'(k[j]) [j < key_len]
-__global__ __launch_bounds__(16 * kGroups) void attn_bwd_finish_kernel(
+template <int LANES>
+__global__ __launch_bounds__(LANES * kGroups) void attn_bwd_finish_kernel(
     Rows q, Rows k, const int64_t *__restrict__ key_len, const float *__restrict__ dd,
     const float *__restrict__ sums, int H, int L, int E, int nseg, RowsOut dq, RowsOut dk) {
-    __shared__ float4 total[2][kGroups][16];
+    __shared__ float4 total[2][kGroups][LANES];
     // (the heads of one batch entry and segment in neighbouring workgroups: with heads
     // interleaved in memory their rows lie side by side)
     const int h = blockIdx.x % H, seg = (blockIdx.x / H) % nseg, n = blockIdx.x / (H * nseg);
     const int64_t chain = (int64_t)n * H + h;
-    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+    const int r = threadIdx.x / LANES, c = threadIdx.x % LANES;
     const int len = key_len ? (int)min<int64_t>(key_len[n], L) : L;
     const bool has_e = 4 * c < E;
     const int ce = has_e ? 4 * c : 0;
@@ -234,7 +241,8 @@ void launch_attention_backward_prep(const Operand &q, const Operand &k, const Op
                                     float *Kf, float *gz, float *dd, float *sums,
                                     hipStream_t stream) {
     const int nseg = (int)attention_backward_segments(L);
-    hipLaunchKernelGGL(attn_bwd_prep_kernel, dim3((unsigned)(N * H * nseg)), dim3(256), 0, stream,
+    const auto kernel = E > 64 || M > 64 ? attn_bwd_prep_kernel<32> : attn_bwd_prep_kernel<16>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(N * H * nseg)), dim3(256), 0, stream,
                        rows_of(q), rows_of(k), rows_of(g), rows_of(out), rows_of(den), key_len, (int)H,
                        (int)L, E, M, nseg, Qf, Kf, gz, dd, sums);
 }
@@ -244,8 +252,11 @@ void launch_attention_backward_finish(const Operand &q, const Operand &k, const 
                                       int64_t L, int E, const OperandOut &dq, const OperandOut &dk,
                                       hipStream_t stream) {
     const int nseg = (int)attention_backward_segments(L);
-    hipLaunchKernelGGL(attn_bwd_totals_kernel, dim3((unsigned)(N * H)), dim3(128), 0, stream, sums, E, nseg);
-    hipLaunchKernelGGL(attn_bwd_finish_kernel, dim3((unsigned)(N * H * nseg)), dim3(16 * kGroups), 0, stream,
+    const bool wide = E > 64;
+    hipLaunchKernelGGL((wide ? attn_bwd_totals_kernel<32> : attn_bwd_totals_kernel<16>), dim3((unsigned)(N * H)),
+                       dim3(wide ? 256 : 128), 0, stream, sums, E, nseg);
+    hipLaunchKernelGGL((wide ? attn_bwd_finish_kernel<32> : attn_bwd_finish_kernel<16>),
+                       dim3((unsigned)(N * H * nseg)), dim3((wide ? 32 : 16) * kGroups), 0, stream,
                        rows_of(q), rows_of(k), key_len, dd, (const float *)sums, (int)H, (int)L, E, nseg,
                        rows_of(dq), rows_of(dk));
 }

@@ -159,6 +159,8 @@ struct FusedAttention {
     int64_t den_sn = 0, den_sh = 0;
 };
 bool fused_attention_supported(const ScanDesc &scan, int64_t L);
+// rows of 128: whether a plan exists for the sizes (no workspace needed: 0 bytes)
+bool fused_attention_wide_covers(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F);
 int64_t fused_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F);
 // Runs scans[0..nscans) (all of the same row widths) in one launch.  `fused`: a single
 // forward scan in its fused attention form.  `may_chain_parallel` = false keeps the launch

@@ -711,13 +711,21 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
     return (double)rounds * (longest + 4.0);
 }
 
+// (rows of 128 values: the chain-parallel kernel alone)
+bool fused_wide(int64_t D, int64_t F) { return D > 64 || F > 64; }
+
 bool fused_attention_supported(const ScanDesc &sd, int64_t L) {
-    return combo_of(sd) == kFFFF && !sd.reverse && !sd.initial.ptr && !sd.final_.ptr &&
-           scan_wg_norm_covers(sd.a.width, sd.v.width) && mfma_scan_supported(sd, L);
+    if (combo_of(sd) != kFFFF || sd.reverse || sd.initial.ptr || sd.final_.ptr) return false;
+    if (!fused_wide(sd.a.width, sd.v.width))
+        return scan_wg_norm_covers(sd.a.width, sd.v.width) && mfma_scan_supported(sd, L);
+    for (const Operand *t : {&sd.a, &sd.b, &sd.v})
+        if (!mfma_operand_in_place(t->ptr, t->stride_n, t->stride_h, t->stride_l, t->dtype, t->width, L)) return false;
+    const OperandOut &o = sd.out;
+    return mfma_operand_in_place(o.ptr, o.stride_n, o.stride_h, o.stride_l, o.dtype, o.width, L);
 }
 
-// (the exchange of the chain-parallel fused form: a second tile of state for its denominators)
-constexpr int64_t kFusedTpStateRows = 128;
+// (the exchange of the chain-parallel fused form: another tile of state for its denominators)
+int64_t fused_tp_state_rows(int64_t D) { return (D + 63) / 64 * 64 + 64; }
 
 // The fused attention launch on the chain-parallel kernel: its plan is that of a single 64 x 64
 // scan whatever the widths (a chunk costs the same).  Returns false: the workgroup form, whose
@@ -730,8 +738,17 @@ constexpr int64_t kFusedTpStateRows = 128;
 // 32: 80 chains, L=1000 41.6 / 34.8 and 36.7 / 32.0, but 64 chains, L=1500 42.9 / 44.2, more than a
 // round of workgroups 102 / 116, with an exchange 95.7 / 106.  32 x 32: 31.7 / 31.3 and 64 / 96.
 // Chains of more than 256 chunks are not walked whole on three bf16 pieces (tp_plan_compute).
+//
+// Rows of 128 have no other fused form: the plan is that of such a scan where the chain-parallel kernel
+// has to take it.  Measured, 128 x 128 (us, two scans with the element-wise passes around them / this
+// way): 8 chains, L=2000 122 / 47; 80 chains, L=300 102 / 34; 128 chains, L=856 260 / 90; 256 chains,
+// L=1000 476 / 208; 70 chains, L=8192 1335 / 715.
 bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, int *seg_chunks) {
     *nseg = *seg_chunks = 0;
+    if (fused_wide(D, F)) {
+        tp_plan(D, F, chains, 1, L, nseg, seg_chunks, true);
+        return *nseg > 0;
+    }
     if (tuning().wg > 0) return false;
     const int64_t chunks = (L + kChunk - 1) / kChunk;
     tp_plan(64, 64, chains, 1, L, nseg, seg_chunks);
@@ -746,11 +763,16 @@ bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, i
 
 int64_t fused_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F) {
     int nseg, seg_chunks;
-    int64_t bytes = make_plan(N, H, L, D, F, 1, true, true).workspace_bytes;
+    int64_t bytes = fused_wide(D, F) ? 0 : make_plan(N, H, L, D, F, 1, true, true).workspace_bytes;
     const int64_t chains = std::max<int64_t>(1, N * H);
     if (fused_tp_plan(D, F, chains, L, &nseg, &seg_chunks) && seg_chunks > 0)
-        bytes = std::max(bytes, tp_exchange_workspace_bytes(chains, nseg, kFusedTpStateRows));
+        bytes = std::max(bytes, tp_exchange_workspace_bytes(chains * tp_fblocks(F), nseg, fused_tp_state_rows(D)));
     return bytes;
+}
+
+bool fused_attention_wide_covers(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F) {
+    int nseg, seg_chunks;
+    return fused_tp_plan(D, F, std::max<int64_t>(1, N * H), L, &nseg, &seg_chunks);
 }
 
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
@@ -772,11 +794,14 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     // workgroup form gets the workgroup form)
     bool fused_tp = fused && (L + 2 * kChunk) * std::max<int64_t>(widest, 64) * 4 < 0x7fffffffLL &&
                           fused_tp_plan(D, F, chains, L, &tpx_nseg, &tpx_seg_chunks);
-    if (fused_tp && tpx_seg_chunks > 0 && !plan_only() &&
-        (int64_t)workspace_bytes < tp_exchange_workspace_bytes(chains, tpx_nseg, kFusedTpStateRows))
+    const bool wide_rows = fused && fused_wide(D, F);
+    if (wide_rows && !fused_tp)
+        return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for this shape or layout");
+    if (fused_tp && !wide_rows && tpx_seg_chunks > 0 && !plan_only() &&
+        (int64_t)workspace_bytes < tp_exchange_workspace_bytes(chains, tpx_nseg, fused_tp_state_rows(D)))
         fused_tp = false, tpx_nseg = tpx_seg_chunks = 0;
     const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd);
-    const int64_t fblocks = tp_shape ? tp_fblocks(F) : 1;
+    const int64_t fblocks = tp_shape || wide_rows ? tp_fblocks(F) : 1;
     if (fused_tp && tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     if (tp_shape) {
         int any_bf16 = nscans == 1 && combo == kBBFB ? kMixedGradValues : 0;
@@ -792,14 +817,14 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     if (!tp && !mfma_scan_supported(scans[0], L))
         return fail(FTC_ERR_UNSUPPORTED, "no MFMA kernel takes a %d x %d state here", D, F);
     const bool wg = !fused_tp && (fused || use_wg_kernel(D, F, nscans, L, combo == kFFFF));
-    MfmaPlan pl = make_plan(N, H, L, D, F, nscans, wg, fused != nullptr);
+    MfmaPlan pl = wide_rows ? MfmaPlan{} : make_plan(N, H, L, D, F, nscans, wg, fused != nullptr);
     int32_t tp_start[kMaxTpSegments + 1] = {0};
     if (tpx_seg_chunks > 0) {  // one workgroup per chain segment, segment sums exchanged
         pl.nseg = tpx_nseg;
         pl.seg_len = tpx_seg_chunks * kChunk;
         pl.waves = chains * pl.nseg;
         pl.workspace_bytes = tp_exchange_workspace_bytes(chains * nscans * fblocks, pl.nseg,
-                                                         fused_tp ? kFusedTpStateRows : D);
+                                                         fused_tp ? fused_tp_state_rows(D) : D);
     } else if (tp) {  // one workgroup per chain segment, nothing to exchange
         pl.nseg = tp_segment_starts((L + kChunk - 1) / kChunk, tp_nseg, tp_start);
         pl.seg_len = (int)L;

@@ -168,6 +168,7 @@ __device__ __forceinline__ void tp_workgroup(const ScanArgs &p, uint32_t &which,
 template <int PA, int PB, int PV>
 constexpr int kTpPieceBytes = 3 * (PA + PB + PV) * kChunk * 128;
 constexpr int kTpPtBytes = 2 * 3 * kChunk * 64;
+constexpr int kTpZBytes = 4 * 2 * 2 * 64;  // z of the four consumers, fused attention with two blocks
 
 // KS2: groups of 32 rows in the state's last block (1: a state of 65 .. 96 rows, whose last
 // block skips the matrix instructions and fragment reads of its empty half)
@@ -537,18 +538,29 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     if (!NORM && op.s0 && !exchange) add_caller_state();
     // NORM: this consumer's half of z, block by block (tiles 0 and 1 in its order, all columns alike)
     const bool has_z = NORM && (KS2 == 2 || w < 2);
+    // (two blocks: z is in LDS, one copy per consumer that only it uses, and a chunk's sum is added to it
+    // as a whole.  Accumulated in registers by the matrix instructions 130 chains of 4000 positions were
+    // 5.2e-7 from float64, this way 1.2e-7; added as a whole in registers 21 of them spilled, and 128
+    // chains of 856 took 128 us against 90.)
     f32x4 Z[ND][2];
+    typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+    lds_f32x4 *const z_mem = (lds_f32x4 *)(pt_pc + kTpPtBytes) + 8 * ND * w + g;
 #pragma unroll
-    for (int hb = 0; hb < ND; hb++) Z[hb][0] = Z[hb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int hb = 0; hb < ND; hb++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            Z[hb][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (NORM && ND > 1) z_mem[8 * hb + 4 * t] = Z[hb][t];
+        }
     const Frag ones = {{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u}};
     // The products of up to eight chunks are added up by themselves (R) before they are added to the
     // state, where there are registers for it; the state in use is S + R.  (The sums of the matrix
     // instructions fall short by a part of the last place of the sum each, which keys and weights that
     // are all positive add up.  NORM: 300 chains of 4000 positions walked whole were 7e-7 from float64
     // without it, the workgroup form's short segments are 3e-7; the time is the same.  Not there while
-    // chunks are walked for their state alone: its registers would spill.  bf16 rows: the state handed
+    // chunks are walked for their state alone, nor with two blocks: its registers would spill.  bf16 rows: the state handed
     // out after 1000 positions was 2.7e-7 off without it, 1.0e-7 on the kernels that split L.)
-    constexpr bool kMixed = PA + PB + PV < 9, kApart = NORM || kMixed;
+    constexpr bool kMixed = PA + PB + PV < 9, kApart = (NORM && ND == 1) || kMixed;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 R[ND][4], Zr[ND][2];
     auto add_product = [&](int hb, int dt, const Frag &x, const Frag &y) {
@@ -558,13 +570,14 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             S[hb][dt] = mfma16(x, y, S[hb][dt]);
     };
     auto state = [&](int hb, int dt, int r) -> float { return kApart ? S[hb][dt][r] + R[hb][dt][r] : S[hb][dt][r]; };
+    auto sum_of_keys = [&](int hb, int t, int r) -> float { return Z[hb][t][r] + Zr[hb][t][r]; };
     auto clear_apart = [&]() {
 #pragma unroll
         for (int hb = 0; hb < ND; hb++)
 #pragma unroll
             for (int dt = 0; dt < 4; dt++) {
                 if (kApart) R[hb][dt] = zero;
-                if (NORM) Zr[hb][dt % 2] = zero;
+                if (NORM && kApart) Zr[hb][dt % 2] = zero;
             }
     };
     auto add_apart = [&]() {
@@ -623,6 +636,15 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 R[hb][dt] = mfma16(x, y, R[hb][dt]);
             else
                 S[hb][dt] = mfma16(x, y, S[hb][dt]);
+        };
+        auto add_keys = [&](int hb, int i, const Frag (&btx)[4][PB]) {
+            if (ND == 1) {
+                if (i < 6) Z[hb][i % 2] = mfma16(btx[i % 2][2 - i / 2], ones, Z[hb][i % 2]);
+            } else {
+                if (i < 6) Zr[0][i % 2] = mfma16(btx[i % 2][2 - i / 2], ones, i < 2 ? zero : Zr[0][i % 2]);
+                if (i == 7 || i == 8) Z[0][i - 7] = z_mem[8 * hb + 4 * (i - 7)];
+                if (i == 12 || i == 13) z_mem[8 * hb + 4 * (i - 12)] = Z[0][i - 12] + Zr[0][i - 12];
+            }
         };
         // The consumers have little to do here, so they share the producers' work: rows
         // 16 .. 31 of b and v of these chunks are fetched and cut by the consumers (lane
@@ -701,13 +723,13 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                         if (rows_exist && i < 4 * OfS::count)
                             add_first(hp, i % 4, bt2[i % 4][OfS::x(i / 4)], vf2[OfS::y(i / 4)]);
                         if constexpr (NORM)
-                            if (i < 6) Z[hp][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
+                            add_keys(hp, i, bt2);
                         tr_frag_into(bt, vf, pc, pcv, i, j % ND);
                     } else {
                         if (rows_exist && i < 4 * OfS::count)
                             add_first(hp, i % 4, bt[i % 4][OfS::x(i / 4)], vf[OfS::y(i / 4)]);
                         if constexpr (NORM)
-                            if (i < 6) Z[hp][i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, Z[hp][i % 2]);
+                            add_keys(hp, i, bt);
                         tr_frag_into(bt2, vf2, pc, pcv, i, j % ND);
                     }
                     if (i == 15 && cut_next) ccut_b(rn, bufn, c + j + 1);
@@ -728,7 +750,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             if ((i % 4) / 2 < KS2 && i < 4 * OfS::count)
                 add_first(ND - 1, i % 4, bt2[i % 4][OfS::x(i / 4)], vf2[OfS::y(i / 4)]);
             if constexpr (NORM)
-                if (i < 6) Z[ND - 1][i % 2] = mfma16(bt2[i % 2][2 - i / 2], ones, Z[ND - 1][i % 2]);
+                add_keys(ND - 1, i, bt2);
             rm_frag(unit_pc + buf * kBufBytes, i, 0);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -753,7 +775,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         if (NORM) {
             Sx[DX - 1][0] = f32x16{};
 #pragma unroll
-            for (int i = 0; i < 8 * ND; i++) Sx[DX - 1][0][i] = Z[i / 8][i / 4 % 2][i % 4];
+            for (int i = 0; i < 8 * ND; i++) Sx[DX - 1][0][i] = ND == 1 ? Z[i / 8][i / 4 % 2][i % 4] : z_mem[8 * (i / 8) + 4 * (i / 4 % 2)][i % 4];
         }
 #pragma unroll
         for (int hb = 0; hb < ND; hb++)
@@ -773,7 +795,12 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 for (int r = 0; r < 4; r++) S[hb][dt][r] = X[hb][0][4 * dt + r];
         if (NORM) {
 #pragma unroll
-            for (int i = 0; i < 8 * ND; i++) Z[i / 8][i / 4 % 2][i % 4] = X[DX - 1][0][i];
+            for (int i = 0; i < 2 * ND; i++) {
+                const f32x4 z = {X[DX - 1][0][4 * i], X[DX - 1][0][4 * i + 1], X[DX - 1][0][4 * i + 2],
+                                 X[DX - 1][0][4 * i + 3]};
+                Z[i / 2][i % 2] = z;
+                if (ND > 1) z_mem[4 * i] = z;
+            }
         }
         if (!NORM && op.s0) add_caller_state();
     }
@@ -839,10 +866,14 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 else if (i < 4)
                     P4[i % 4] = zero;
                 if (i < 4 && block_ks(hb) > 1) cut_s(hb, 1, i);
+                if (NORM && ND > 1 && (i == 5 || i == 7)) Z[0][i / 2 - 2] = z_mem[8 * hb + 4 * (i / 2 - 2)];
                 if (NORM && i >= 8) {  // z in pieces
                     uint32_t o[3];
-                    split_pair_under_mfma(Z[hb][(i - 8) / 2][2 * (i % 2)] + Zr[hb][(i - 8) / 2][2 * (i % 2)],
-                                          Z[hb][(i - 8) / 2][2 * (i % 2) + 1] + Zr[hb][(i - 8) / 2][2 * (i % 2) + 1], o);
+                    if (ND > 1)
+                        split_pair_under_mfma(Z[0][(i - 8) / 2][2 * (i % 2)], Z[0][(i - 8) / 2][2 * (i % 2) + 1], o);
+                    else
+                        split_pair_under_mfma(sum_of_keys(hb, (i - 8) / 2, 2 * (i % 2)),
+                                              sum_of_keys(hb, (i - 8) / 2, 2 * (i % 2) + 1), o);
 #pragma unroll
                     for (int k = 0; k < 3; k++) zf[k].w[i - 8] = o[k];
                 }
@@ -901,7 +932,14 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 if (i < 2 * OfS::count)
                     add_product(hb, i % 2, bt[i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)]);
                 if constexpr (NORM)
-                    if (i < 6) Zr[hb][i % 2] = mfma16(bt[i % 2][2 - i / 2], ones, Zr[hb][i % 2]);
+                    if (i < 6) {
+                        f32x4 &sum = kApart ? Zr[hb][i % 2] : Zr[0][i % 2];
+                        sum = mfma16(bt[i % 2][2 - i / 2], ones, kApart || i >= 2 ? sum : zero);
+                    }
+                if (NORM && ND > 1) {
+                    if (i == 7 || i == 8) Z[0][i - 7] = z_mem[8 * hb + 4 * (i - 7)];
+                    if (i == 10 || i == 11) z_mem[8 * hb + 4 * (i - 10)] = Z[0][i - 10] + Zr[0][i - 10];
+                }
                 if (NORM && i == 6 && last_block) {
                     P_sum = sum_of_lane_groups(P_sum);
                     if (g == 0) den_mem[c & 1][16 * ih + ln][w >> 1] = (has_z ? Az[0] : 0.f) + P_sum;
@@ -1006,7 +1044,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 template <int ND, int KS2, bool NORM>
 __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     __shared__ __align__(16) char pieces_mem[kTpPieceBytes<3, 3, 3>];
-    __shared__ __align__(16) char pt_mem[kTpPtBytes];
+    __shared__ __align__(16) char pt_mem[kTpPtBytes + (NORM && ND > 1 ? kTpZBytes : 0)];
     __shared__ __align__(16) float den_mem[NORM ? 2 : 1][NORM ? kChunk : 1][2];
     __shared__ uint32_t order_sh;
     uint32_t which, chain;

@@ -36,6 +36,10 @@ EXPORTED_SYMBOLS = (
     "ftc_causal_linear_attention_forward",
     "ftc_causal_linear_attention_backward_workspace_bytes",
     "ftc_causal_linear_attention_backward",
+    "ftc_causal_linear_attention_wide_workspace_bytes",
+    "ftc_causal_linear_attention_wide_forward",
+    "ftc_causal_linear_attention_wide_backward_workspace_bytes",
+    "ftc_causal_linear_attention_wide_backward",
     "ftc_split_weights",
     "ftc_split_rows",
     "ftc_layer_norm_split",
@@ -97,7 +101,9 @@ def load():
     for name in ("ftc_causal_dot_product_workspace_bytes",
                  "ftc_causal_dot_backward_workspace_bytes",
                  "ftc_causal_linear_attention_workspace_bytes",
-                 "ftc_causal_linear_attention_backward_workspace_bytes"):
+                 "ftc_causal_linear_attention_backward_workspace_bytes",
+                 "ftc_causal_linear_attention_wide_workspace_bytes",
+                 "ftc_causal_linear_attention_wide_backward_workspace_bytes"):
         f = getattr(lib, name)
         f.restype = ctypes.c_int64
         f.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int32]
@@ -122,8 +128,15 @@ def load():
     lib.ftc_causal_linear_attention_forward.argtypes = [t4] * 3 + [ctypes.c_void_p, ctypes.c_float, t4,
                                                                    t4, ctypes.c_void_p,
                                                                    ctypes.c_size_t, ctypes.c_void_p]
+    lib.ftc_causal_linear_attention_wide_forward.restype = ctypes.c_int
+    lib.ftc_causal_linear_attention_wide_forward.argtypes = [t4] * 3 + [ctypes.c_void_p, ctypes.c_float, t4,
+                                                                   t4, ctypes.c_void_p,
+                                                                   ctypes.c_size_t, ctypes.c_void_p]
     lib.ftc_causal_linear_attention_backward.restype = ctypes.c_int
     lib.ftc_causal_linear_attention_backward.argtypes = [t4] * 3 + [ctypes.c_void_p] + [t4] * 6 + [
+        ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    lib.ftc_causal_linear_attention_wide_backward.restype = ctypes.c_int
+    lib.ftc_causal_linear_attention_wide_backward.argtypes = [t4] * 3 + [ctypes.c_void_p] + [t4] * 6 + [
         ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
     lib.ftc_causal_dot_plan.restype = ctypes.c_int
     lib.ftc_causal_dot_plan.argtypes = [t4] * 3 + [ctypes.c_int, ctypes.c_char_p, ctypes.c_size_t]

@@ -19,13 +19,15 @@ default one, the whole body of ``forward`` -- both feature maps, the key-length 
 product, the normaliser and the final scale -- is one launch of
 ``ftc_causal_linear_attention`` (head dimensions 32 or 64, float32), and training on
 ``CausalLinearAttentionFunction``, whose backward is one launch sequence of its own
-(``ftc_causal_linear_attention_backward``).  Other sizes and feature maps keep the composition
+(``ftc_causal_linear_attention_backward``); plain calls have the same for head dimensions of 128
+(``ftc_causal_linear_attention_wide_forward``).  Other sizes and feature maps keep the composition
 above, whose pieces autograd differentiates.
 """
 import torch
 from torch.nn import Module
 
 from .. import causal_product
+from ..masking import LengthMask
 from ..causal_product import causal_dot_product_hip, causal_dot_backward_hip, \
     causal_linear_attention_hip, fused_attention_covers, CausalLinearAttentionFunction
 
@@ -162,12 +164,13 @@ class CausalLinearAttention(Module):
                 and fm.activation_function is _elu_plus_one):
             return None
         lengths = getattr(key_lengths, "lengths", None)
-        host = causal_product._host_module
-        if host is not None and not torch.compiler.is_compiling() and _as_defined == (
+        if not torch.compiler.is_compiling() and torch.cuda.is_initialized() and _as_defined == (
                 causal_linear_attention_hip, causal_product.causal_linear_attention_backward_hip,
                 CausalLinearAttentionFunction.forward, CausalLinearAttentionFunction.backward):
-            # plain tensors: the same in the C++ engine, which costs the host less
-            out = host.attention_module(queries, keys, values, lengths, self.eps)
+            # plain tensors: the same in the C++ engine, which costs the host less and has the
+            # kernels for rows of 128 values (watched calls of those keep the composition)
+            mask_length = key_lengths.max_len if type(key_lengths) is LengthMask else -1
+            out = causal_product._host().attention_module(queries, keys, values, lengths, mask_length, self.eps)
             if out is not None:
                 return out
         if queries.shape[1] != keys.shape[1] or keys.shape[1] != values.shape[1]:

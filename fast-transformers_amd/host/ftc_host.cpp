@@ -269,8 +269,9 @@ const int64_t *lengths_ptr(const OptTensor &lengths, const Tensor &q) {
     return lengths->const_data_ptr<int64_t>();
 }
 
-void attention(const Tensor &queries, const Tensor &keys, const Tensor &values, const OptTensor &key_lengths,
-               double eps, const Tensor &out, const OptTensor &denominators) {
+// (`wide`: rows of 128 values too)
+void fused_attention(const Tensor &queries, const Tensor &keys, const Tensor &values, const OptTensor &key_lengths,
+                     double eps, const Tensor &out, const OptTensor &denominators, bool wide) {
     const at::NoGradGuard no_grad;
     const Tensor q = prepare(queries, "queries"), k = prepare(keys, "keys"), v = prepare(values, "values");
     const int64_t *lengths = lengths_ptr(key_lengths, q);
@@ -278,22 +279,27 @@ void attention(const Tensor &queries, const Tensor &keys, const Tensor &values, 
                       dout = describe(check_out(out, "out"));
     ftc_tensor4 dden;
     if (denominators) dden = describe(denominators->unsqueeze(3));
-    Call call(q, workspace_bytes(ftc_causal_linear_attention_workspace_bytes,
+    Call call(q, workspace_bytes(wide ? ftc_causal_linear_attention_wide_workspace_bytes
+                                      : ftc_causal_linear_attention_workspace_bytes,
                                  "ftc_causal_linear_attention_workspace_bytes", q.size(0), q.size(1),
                                  q.size(2), q.size(3), v.size(3), dq.dtype));
+    const auto run = wide ? ftc_causal_linear_attention_wide_forward : ftc_causal_linear_attention_forward;
     const int rc = native([&] {
-        return ftc_causal_linear_attention_forward(&dq, &dk, &dv, lengths, (float)eps, &dout,
-                                                   denominators ? &dden : nullptr, call.ws, call.ws_bytes,
-                                                   call.stream);
+        return run(&dq, &dk, &dv, lengths, (float)eps, &dout, denominators ? &dden : nullptr, call.ws, call.ws_bytes,
+                   call.stream);
     }, call.turn);
     check(rc, "ftc_causal_linear_attention_forward");
     call.done();
 }
+void attention(const Tensor &queries, const Tensor &keys, const Tensor &values, const OptTensor &key_lengths,
+               double eps, const Tensor &out, const OptTensor &denominators) {
+    fused_attention(queries, keys, values, key_lengths, eps, out, denominators, false);
+}
 
-void attention_backward(const Tensor &queries, const Tensor &keys, const Tensor &values,
-                        const OptTensor &key_lengths, const Tensor &out, const Tensor &denominators,
-                        const Tensor &grad_out, const OptTensor &grad_queries, const OptTensor &grad_keys,
-                        const OptTensor &grad_values) {
+void fused_attention_backward(const Tensor &queries, const Tensor &keys, const Tensor &values,
+                              const OptTensor &key_lengths, const Tensor &out, const Tensor &denominators,
+                              const Tensor &grad_out, const OptTensor &grad_queries, const OptTensor &grad_keys,
+                              const OptTensor &grad_values, bool wide) {
     const at::NoGradGuard no_grad;
     const Tensor q = prepare(queries, "queries"), k = prepare(keys, "keys"), v = prepare(values, "values"),
                  o = prepare(out, "out"), g = prepare(grad_out, "grad_out");
@@ -301,15 +307,23 @@ void attention_backward(const Tensor &queries, const Tensor &keys, const Tensor 
     const ftc_tensor4 dq = describe(q), dk = describe(k), dv = describe(v), dout = describe(o),
                       dden = describe(denominators.unsqueeze(3)), dg = describe(g);
     const Out gq(grad_queries, "grad_queries"), gk(grad_keys, "grad_keys"), gv(grad_values, "grad_values");
-    Call call(q, workspace_bytes(ftc_causal_linear_attention_backward_workspace_bytes,
+    Call call(q, workspace_bytes(wide ? ftc_causal_linear_attention_wide_backward_workspace_bytes
+                                      : ftc_causal_linear_attention_backward_workspace_bytes,
                                  "ftc_causal_linear_attention_backward_workspace_bytes", q.size(0),
                                  q.size(1), q.size(2), q.size(3), v.size(3), dq.dtype));
+    const auto run = wide ? ftc_causal_linear_attention_wide_backward : ftc_causal_linear_attention_backward;
     const int rc = native([&] {
-        return ftc_causal_linear_attention_backward(&dq, &dk, &dv, lengths, &dout, &dden, &dg, gq.p, gk.p,
-                                                    gv.p, call.ws, call.ws_bytes, call.stream);
+        return run(&dq, &dk, &dv, lengths, &dout, &dden, &dg, gq.p, gk.p, gv.p, call.ws, call.ws_bytes, call.stream);
     }, call.turn);
     check(rc, "ftc_causal_linear_attention_backward");
     call.done();
+}
+void attention_backward(const Tensor &queries, const Tensor &keys, const Tensor &values,
+                        const OptTensor &key_lengths, const Tensor &out, const Tensor &denominators,
+                        const Tensor &grad_out, const OptTensor &grad_queries, const OptTensor &grad_keys,
+                        const OptTensor &grad_values) {
+    fused_attention_backward(queries, keys, values, key_lengths, out, denominators, grad_out, grad_queries, grad_keys,
+                             grad_values, false);
 }
 
 // ---- the differentiable entry points ----
@@ -398,12 +412,22 @@ py::object dot(py::handle queries, py::handle keys, py::handle values) {
 
 Tensor swapped(const Tensor &t) { return t.permute({0, 2, 1, 3}); }
 
+// rows of 128 values
+bool wide_rows(const Tensor &q, const Tensor &v) { return q.size(-1) > 64 || v.size(-1) > 64; }
+// ... are read where 16-byte loads reach them in chains within 2 GiB (t as the module has it)
+bool reads_in_place(const Tensor &t) {
+    const int64_t row = std::max(t.stride(1), t.size(2) * t.size(3));
+    return (uintptr_t)t.const_data_ptr() % 16 == 0 && t.stride(3) == 1 && t.stride(0) % 4 == 0 &&
+           t.stride(1) % 4 == 0 && t.stride(2) % 4 == 0 && t.stride(1) >= t.size(3) && row <= (1 << 16) &&
+           (t.size(1) + 64) * row * 4 < 0x7fffffff;
+}
+
 // tensors as the attention module has them, (N, L, H, X)
 struct CausalAttention : torch::autograd::Function<CausalAttention> {
     static Tensor run(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &lengths, double eps,
                       const OptTensor &denominators) {
         const Tensor out = at::empty({q.size(0), q.size(1), q.size(2), v.size(3)}, q.options());
-        ::attention(swapped(q), swapped(k), swapped(v), lengths, eps, swapped(out), denominators);
+        ::fused_attention(swapped(q), swapped(k), swapped(v), lengths, eps, swapped(out), denominators, wide_rows(q, v));
         return out;
     }
     static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v,
@@ -422,24 +446,36 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
         for (int i = 0; i < 3; i++)
             if (ctx->needs_input_grad(i)) out[i] = at::empty_like(saved[i]), to[i] = swapped(out[i]);
         from_engine([&] {
-            ::attention_backward(swapped(saved[0]), swapped(saved[1]), swapped(saved[2]), lengths, swapped(saved[3]),
-                                 saved[4], swapped(grads[0]), to[0], to[1], to[2]);
+            const bool wide = wide_rows(saved[0], saved[2]);
+            const Tensor g = wide && !reads_in_place(grads[0]) ? grads[0].clone(at::MemoryFormat::Contiguous) : grads[0];
+            ::fused_attention_backward(swapped(saved[0]), swapped(saved[1]), swapped(saved[2]), lengths,
+                                       swapped(saved[3]), saved[4], swapped(g), to[0], to[1], to[2], wide);
         });
         return out;
     }
 };
 
 // The fused forward of the attention module; None: not a plain call, or sizes without a fused kernel
-py::object attention_module(py::handle queries, py::handle keys, py::handle values, py::handle key_lengths, double eps) {
+// (mask_length: how many positions the mask of the lengths has, -1 if unknown)
+py::object attention_module(py::handle queries, py::handle keys, py::handle values, py::handle key_lengths,
+                            int64_t mask_length, double eps) {
     const Tensor *q = plain(queries), *k = plain(keys), *v = plain(values);
     if (!q || !k || !v || !THPVariable_CheckExact(key_lengths.ptr()) || !nothing_watches()) return py::none();
     const Tensor &lengths = THPVariable_Unpack(key_lengths.ptr());
-    auto width = [](int64_t w) { return w == 32 || w == 64; };
+    auto width = [](int64_t w) { return w == 32 || w == 64 || w == 128; };
     for (const Tensor *t : {q, k, v})
         if (t->scalar_type() != at::kFloat || t->device() != q->device() || t->size(1) != q->size(1)) return py::none();
     if (k->size(3) != q->size(3) || !width(q->size(3)) || !width(v->size(3)) || lengths.device() != q->device() ||
         lengths.scalar_type() != at::kLong || !lengths.is_contiguous() || lengths.requires_grad())
         return py::none();
+    if (wide_rows(*q, *v)) {  // (what the composition would broadcast or refuse is left to it)
+        if (lengths.dim() != 1 || lengths.size(0) != q->size(0) || mask_length != q->size(1)) return py::none();
+        for (const Tensor *t : {q, k, v})
+            if (!reads_in_place(*t) || t->size(0) != q->size(0) || t->size(2) != q->size(2)) return py::none();
+        if (ftc_causal_linear_attention_wide_workspace_bytes(q->size(0), q->size(2), q->size(1), q->size(3), v->size(3),
+                                                             FTC_F32) < 0)
+            return py::none();
+    }
     return py::cast(differentiated({q, k, v}) ? CausalAttention::apply(*q, *k, *v, lengths, eps)
                                               : CausalAttention::run(*q, *k, *v, lengths, eps, std::nullopt));
 }

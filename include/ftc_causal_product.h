@@ -264,6 +264,28 @@ int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_t
                                          void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * ftc_causal_linear_attention_forward, ..._backward and their workspaces for E, M in {32, 64, 128},
+ * with the same arguments and results (the functions above keep refusing rows of 128 values, as their
+ * callers may rely on).  Rows of 128 need 16-byte aligned rows whose chains lie within 2 GiB; the
+ * workspace queries and the calls return FTC_ERR_UNSUPPORTED for what no kernel takes.
+ */
+int64_t ftc_causal_linear_attention_wide_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E,
+                                                         int64_t M, int32_t dtype);
+int ftc_causal_linear_attention_wide_forward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
+                                             const ftc_tensor4 *values, const int64_t *key_lengths,
+                                             float eps, const ftc_tensor4 *out,
+                                             const ftc_tensor4 *denominators, void *workspace,
+                                             size_t workspace_bytes, void *stream);
+int64_t ftc_causal_linear_attention_wide_backward_workspace_bytes(int64_t N, int64_t H, int64_t L,
+                                                                  int64_t E, int64_t M, int32_t dtype);
+int ftc_causal_linear_attention_wide_backward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
+                                              const ftc_tensor4 *values, const int64_t *key_lengths,
+                                              const ftc_tensor4 *out, const ftc_tensor4 *denominators,
+                                              const ftc_tensor4 *grad_out, const ftc_tensor4 *grad_queries,
+                                              const ftc_tensor4 *grad_keys, const ftc_tensor4 *grad_values,
+                                              void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * The matrix products of an encoder layer around the attention (attention/attention_layer.py:96-115,
  * transformers.py:76-89) at the precision of fp32 on the fp16 matrix cores: every row is scaled by a
  * power of two and kept as two fp16 pieces, hi + lo = row x 2^e, and a product is the sum of three

@@ -418,6 +418,64 @@ def test_backward_against_autograd_in_float64(lib, shape):
         assert (got[2][n_, len_:] == 0).all()
 
 
+WIDE_SHAPES = [
+    # N, L, H, E, M, key lengths: single positions, ragged ends, keys that end before, inside and on a
+    # chunk; cut chains, whole ones of a round and more of workgroups, exchanges of segment sums; one and
+    # two blocks of state rows and of value columns
+    (2, 1, 2, 128, 128, [1, 0]), (2, 33, 3, 128, 128, [33, 7]), (3, 129, 2, 128, 64, [129, 0, 64]),
+    (1, 1100, 4, 128, 128, [900]), (70, 97, 2, 128, 128, [97, 32, 0, 65, 96] * 14), (2, 300, 3, 64, 128, [300, 117]),
+    (2, 257, 2, 32, 128, [257, 40]), (2, 260, 2, 128, 32, [224, 260]), (1, 2500, 1, 128, 128, [2500]),
+]
+
+
+@pytest.mark.parametrize("shape", WIDE_SHAPES, ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s[:5])
+def test_module_at_rows_of_128(lib, shape):
+    """The module's fused calls at widths of 128, forward and backward, against the dense closed form in
+    float64, with the bounds of the narrower widths (above); masked keys and values do not matter; a
+    gradient that 16-byte loads do not reach is copied; rows that they do not reach are composed."""
+    from fast_transformers_amd import attention, causal_product as cp
+    from fast_transformers_amd.masking import LengthMask, TriangularCausalMask
+    N, L, H, E, M, lens = shape
+    assert not cp.fused_attention_covers(torch.empty(1, 1, 1, E, device="cuda"), torch.empty(1, 1, 1, M, device="cuda"))
+    q, k, v = inputs(N, L, H, E, M, seed=41 + L)
+    g = torch.randn(N, L, H, M, generator=torch.Generator().manual_seed(42 + L))
+    lengths, eps = torch.tensor(lens), 1e-6
+    module, mask = attention.CausalLinearAttention(E), TriangularCausalMask(L, device="cuda")
+    keys = LengthMask(lengths.cuda(), max_len=L)
+
+    def grads(f, dtype, *t):
+        t = [x.to(device="cuda", dtype=dtype).requires_grad_(True) for x in t]
+        out = f(*t)
+        return [out.detach()] + list(torch.autograd.grad(out, t, g.to(device="cuda", dtype=dtype)))
+    dense = lambda a, b, c: _dense_attention(a, b, c, lengths.cuda(), eps)
+    fused_module = lambda a, b, c: module(a, b, c, mask, keys, keys)
+    exact, plain = grads(dense, torch.float64, q, k, v), grads(dense, torch.float32, q, k, v)
+    got = grads(fused_module, torch.float32, q, k, v)
+    torch.cuda.synchronize()
+    for name, a, b, c in zip(("out", "grad_queries", "grad_keys", "grad_values"), got, plain, exact):
+        assert torch.isfinite(a).all(), name
+        nlhx = lambda t: t.permute(0, 2, 1, 3).double().cpu()
+        e_hip, e_plain = scale_error(nlhx(a), nlhx(c)), scale_error(nlhx(b), nlhx(c))
+        assert e_hip <= max(4 * e_plain, 5e-6), name
+    masked_k, masked_v = k.cuda(), v.cuda()
+    for n, length in enumerate(lens):
+        assert (got[2][n, length:] == 0).all()
+        masked_k[n, length:], masked_v[n, length:] = 60.0, 1e30
+    with torch.no_grad():
+        again = fused_module(q.cuda(), masked_k, masked_v)
+    assert lib.ftc_last_kernel().startswith(b"scan_tp_kernel<NORM>") and torch.equal(again, got[0])
+    # the same call with its gradient, and then with its queries, one value off the 16-byte boundary
+    off = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    t = [x.cuda().requires_grad_(True) for x in (q, k, v)]
+    out = fused_module(*t)
+    assert "CppNode" in out.grad_fn.name()
+    for a, b in zip(torch.autograd.grad(out, t, off(g.cuda())), got[1:]):
+        assert torch.equal(a, b)
+    out = fused_module(off(q.cuda()).requires_grad_(True), *t[1:])
+    assert "CppNode" not in out.grad_fn.name()
+    assert scale_error(out.detach().permute(0, 2, 1, 3).cpu(), got[0].permute(0, 2, 1, 3).cpu()) <= 5e-6
+
+
 def test_backward_finite_differences(lib):
     """Directional derivatives of sum(out * w) along random directions, by central differences
     of the float64 closed form, against the fused backward's gradients."""
