@@ -641,6 +641,20 @@ bool copies_on_pieces(const ScanDesc *scans, int n, const bool *padded, int i, i
     return mfma_tp_takes(group, ngroup, N, H, L);
 }
 
+// whether all rows of a scan are fp32, and whether any need no copy
+bool fp32_rows(const ScanDesc &sc, int64_t L, bool *any_fits) {
+    if (sc.out.dtype != FTC_F32) return false;
+    *any_fits = sc.out.width % 32 == 0 &&
+                mfma_operand_in_place(sc.out.ptr, sc.out.stride_n, sc.out.stride_h, sc.out.stride_l,
+                                      FTC_F32, sc.out.width, L);
+    for (const Operand *o : {&sc.a, &sc.b, &sc.v}) {
+        if (o->dtype != FTC_F32) return false;
+        *any_fits = *any_fits || (o->width % 32 == 0 && mfma_operand_in_place(o->ptr, o->stride_n, o->stride_h,
+                                                                              o->stride_l, FTC_F32, o->width, L));
+    }
+    return true;
+}
+
 // Whether an fp32 scan of odd widths runs on the fp16-piece kernel where its rows lie rather than on
 // padded copies: where each of its operands would have to be copied and the copies would run on
 // that kernel as well (forward + backward, us, here / on the copies: 8 x 16 chains, L=4096, 50 x 50:
@@ -655,20 +669,42 @@ bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64
                   size_t workspace_bytes) {
     const ScanDesc &sc = scans[i];
     if (tuning().odd == 0) return false;  // tuning aid
-    const Operand *in[3] = {&sc.a, &sc.b, &sc.v};
-    if (sc.out.dtype != FTC_F32) return false;
-    bool any_fits = sc.out.width % 32 == 0 &&
-                    mfma_operand_in_place(sc.out.ptr, sc.out.stride_n, sc.out.stride_h, sc.out.stride_l,
-                                          FTC_F32, sc.out.width, L);
-    for (const Operand *o : in) {
-        if (o->dtype != FTC_F32) return false;
-        any_fits = any_fits || (o->width % 32 == 0 && mfma_operand_in_place(o->ptr, o->stride_n, o->stride_h,
-                                                                            o->stride_l, FTC_F32, o->width, L));
-    }
-    if (tuning().odd > 0) return true;
+    bool any_fits;
+    if (!fp32_rows(sc, L, &any_fits)) return false;
+    if (tuning().odd > 0) return tuning().odd == 1;
     const bool room = plan_only() ||
                       (int64_t)workspace_bytes >= padded_scan_workspace_bytes(N, H, L, sc.a.width, sc.v.width);
     return !any_fits && room && copies_on_pieces(scans, n, padded, i, N, H, L);
+}
+
+// Whether the scans of a call that would all run on padded copies run on three bf16 pieces where their
+// rows lie instead (scan_tp_kernel, ODD: as exact as the copies, whose own passes over the rows are what
+// it saves, and faster than the kernels that split L, which narrow ones would go to).  Measured over
+// 170 calls (us, on copies / here): 25 x 33 forward, 99 chains, L=1531 77 / 33, 2000 chains, L=300 255 / 96;
+// 10 x 9, 214 chains, L=197 39 / 11; 70 x 33, 80 chains, L=1688 130 / 65; 127 x 127, 300 chains, L=2000 838 /
+// 446, backward, 24 chains, L=177 42 / 18; 99 x 101 backward, 2 chains, L=5038 71 / 44.  What keeps them:
+// single scans of more than 64 rows on up to three workgroups' worth of chains too short for an exchange
+// there (75 x 10, 1 chain, L=1942 28 / 67), thousands of workgroups with two chunks each (30 x 50 backward,
+// 3000 chains, L=40 161 / 198), and calls of several scans on more than two rounds of workgroups and
+// 128 chunks or more (99 x 101 backward, 128 chains, L=4096 1494 / 922: faster here, but such a call's plan has the
+// copies in its name and size).  Rows of which some fit stay as in odd_in_place, and so does a workspace without room.
+bool odd_on_three_pieces(const ScanDesc *scans, int n, const bool *padded, int64_t N, int64_t H, int64_t L,
+                         size_t workspace_bytes) {
+    if (tuning().odd == 0 || tuning().tp == 0) return false;  // tuning aids
+    const int64_t chunks = (L + 31) / 32;
+    int64_t units = 0, widest = 0;
+    for (int i = 0; i < n; i++) {
+        const int64_t D = scans[i].a.width, F = scans[i].v.width;
+        bool any_fits;
+        if (!padded[i] || !fp32_rows(scans[i], L, &any_fits) || any_fits) return false;
+        if (!plan_only() && (int64_t)workspace_bytes < padded_scan_workspace_bytes(N, H, L, D, F)) return false;
+        units += N * H * ((F + 63) / 64);
+        widest = std::max(widest, std::max(D, F));
+    }
+    if (tuning().odd == 2) return true;
+    if (n == 1 && scans[0].a.width > 64 && units <= 3 && chunks > 24 && chunks <= 64) return false;
+    if (widest <= 64 && chunks <= 2 && units > 4096) return false;
+    return n == 1 || units <= 512 || chunks < 128;
 }
 
 // Scans for which odd_in_place holds, in one launch or one per shape, whichever is estimated
@@ -676,7 +712,7 @@ bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64
 // *done = false (nothing launched): the kernel does not take one of them, or the workspace has no
 // room for an exchange.
 int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, void *workspace,
-              size_t workspace_bytes, hipStream_t stream, bool *done) {
+              size_t workspace_bytes, hipStream_t stream, bool *done, bool forced = false) {
     *done = false;
     ScanDesc group[kMfmaMaxScans][kMfmaMaxScans];
     int size[kMfmaMaxScans], ngroups = 0, widest_d = 0, widest_f = 0;
@@ -689,24 +725,24 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
         group[k][size[k]++] = scans[i];
     }
     auto room = [&](int d, int f, int k) {
-        const int64_t need = mfma_tp_workspace_bytes(N, H, L, d, f, k, false, true);
+        const int64_t need = mfma_tp_workspace_bytes(N, H, L, d, f, k, forced, true);
         return need == 0 || plan_only() ||
                (workspace && (int64_t)workspace_bytes >= need && (uintptr_t)workspace % 256 == 0);
     };
     bool apart_ok = true;
     for (int k = 0; k < ngroups; k++) {
-        apart_ok = apart_ok && mfma_tp_takes(group[k], size[k], N, H, L, false, true) &&
+        apart_ok = apart_ok && mfma_tp_takes(group[k], size[k], N, H, L, forced, true) &&
                    room(group[k][0].a.width, group[k][0].v.width, size[k]);
-        if (apart_ok) apart += mfma_tp_odd_chunks(group[k][0].a.width, group[k][0].v.width, N, H, size[k], L);
+        if (apart_ok) apart += mfma_tp_odd_chunks(group[k][0].a.width, group[k][0].v.width, N, H, size[k], L, forced);
     }
-    const bool together_ok = ngroups > 1 && mfma_tp_takes(scans, n, N, H, L, false, true) &&
+    const bool together_ok = ngroups > 1 && mfma_tp_takes(scans, n, N, H, L, forced, true) &&
                              room(widest_d, widest_f, n);
     if (!apart_ok && !together_ok) return FTC_OK;
     auto run = [&](const ScanDesc *s, int k) {
-        return mfma_scan(s, k, N, H, L, workspace, workspace_bytes, stream, nullptr, true, false, true);
+        return mfma_scan(s, k, N, H, L, workspace, workspace_bytes, stream, nullptr, true, forced, true);
     };
     *done = true;
-    if (together_ok && (!apart_ok || mfma_tp_odd_chunks(widest_d, widest_f, N, H, n, L) <= apart)) return run(scans, n);
+    if (together_ok && (!apart_ok || mfma_tp_odd_chunks(widest_d, widest_f, N, H, n, L, forced) <= apart)) return run(scans, n);
     for (int k = 0; k < ngroups; k++) {
         const int rc = run(group[k], size[k]);
         if (rc) return rc;
@@ -779,6 +815,12 @@ int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
             const int rc = odd_scans(odd, nodd, N, H, L, workspace, workspace_bytes, stream, &done);
             if (rc) return rc;
             for (int k = 0; k < nodd && done; k++) taken[members[k]] = true, padded[members[k]] = false;
+        }
+        if (nodd == 0 && odd_on_three_pieces(scans, n, padded, N, H, L, workspace_bytes)) {
+            bool done = false;
+            const int rc = odd_scans(scans, n, N, H, L, workspace, workspace_bytes, stream, &done, true);
+            if (rc) return rc;
+            for (int i = 0; i < n && done; i++) taken[i] = true, padded[i] = false;
         }
         any_padded = false;
         for (int i = 0; i < n; i++) any_padded = any_padded || padded[i];

@@ -146,7 +146,7 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
 // ... and of scans with bf16 rows among them
 int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans);
 // estimated time of such a launch, in chunks walked one after the other
-double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L);
+double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L, bool forced);
 // The fused attention form of a forward scan: a and b go through the feature map
 // elu(x) + 1, rows of b at or beyond key_lengths[n] count as zero, and every output row is
 // divided by (phi(a_l) . sum_{j <= l} phi(b_j) + eps).

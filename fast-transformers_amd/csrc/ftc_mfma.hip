@@ -33,7 +33,7 @@ bool use_wg_kernel(int64_t D, int64_t F, int nscans, int64_t L, bool all_f32) {
 // `odd`: fp32 rows of any width on 4-byte boundaries, states of up to 64 rows (the fp16-piece
 // kernel reads and writes those where they lie).
 bool tp_widths(int64_t D, int64_t F, bool forced = false, bool odd = false) {
-    if (odd) return D >= 8 && D <= 64 && F >= 8 && F <= 512;
+    if (odd) return D >= 8 && D <= (forced ? 128 : 64) && F >= 8 && F <= 512;
     const int64_t least = forced ? 4 : 16;
     return D >= least && D <= 128 && F >= least && F <= 512 && D % 4 == 0 && F % 4 == 0;
 }
@@ -285,7 +285,7 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // bf16 anyway, from 192 workgroups on (64 chains, L=16384: 634 against 783 us; 256 chains:
     // 1783 against 2430; 43 chains: 512 against 483)
     const bool mixed_backward = mixed == kMixedRows && nscans == 3;
-    const bool walk_long = (!mixed || mixed_backward) && D <= 64 && L > 256 * kChunk &&
+    const bool walk_long = (!mixed || mixed_backward) && D <= 64 && !(odd && forced) && L > 256 * kChunk &&
                            L <= 1024 * kChunk &&
                            units >= (mixed_backward ? 192 : !wide ? 112 : L > 512 * kChunk ? 128 : 192);
     if (!narrow && !walk_long) *seg_chunks = tp_exchange_segments(units, L, wide, nseg, lone_mixed);
@@ -641,7 +641,7 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     int D, F;
     widest_rows(scans, nscans, &D, &F);
     if (!tp_widths(D, F, forced, odd)) return false;
-    if (odd && !tph_takes_rows(D)) return false;
+    if (odd && !forced && !tph_takes_rows(D)) return false;
     int64_t widest_stride = 0;
     int mixed = nscans == 1 && combo_of(scans[0]) == kBBFB ? kMixedGradValues : 0;
     for (int i = 0; i < nscans; i++) {
@@ -650,8 +650,11 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
         if (combo != kFFFF && mixed == 0) mixed = kMixedRows;
         // (rows with bf16 among them: not as parts of wider scans, whose results are added up in fp32)
         if (combo == kNone || (combo != kFFFF && (forced || tuning().tph == 0))) return false;
-        // (odd widths: scans of any widths side by side, as long as none has a second block of columns)
-        if ((sd.a.width != D || sd.v.width != F) && !(odd && F <= 64)) return false;
+        // (odd widths: scans of any widths side by side, as long as they have as many blocks of columns:
+        // one, where pieces are scaled)
+        if ((sd.a.width != D || sd.v.width != F) &&
+            !(odd && (F <= 64 || (forced && tp_fblocks(sd.v.width) == tp_fblocks(F)))))
+            return false;
         if (odd && (combo != kFFFF || sd.a.width < 8 || sd.v.width < 8)) return false;
         if (L > 1 && !(stride_ok(sd.a.stride_l, sd.a.width) && stride_ok(sd.b.stride_l, sd.a.width) &&
                        stride_ok(sd.v.stride_l, sd.v.width) && stride_ok(sd.out.stride_l, sd.v.width)))
@@ -693,10 +696,10 @@ int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D
     return bytes;
 }
 
-double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L) {
+double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L, bool forced) {
     int nseg = 0, seg_chunks = 0;
     const int64_t chains = std::max<int64_t>(1, N * H), units = chains * nscans * tp_fblocks(F);
-    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, false, 0, true);
+    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, true);
     if (nseg == 0) return 1e30;
     const int64_t rounds = (units * nseg + 255) / 256;
     double longest = 0.0;
@@ -903,7 +906,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     args.group = std::min(args.group, 64);
     while ((pl.nseg + args.group - 1) / args.group > 64) args.group++;
 
-    const bool half_pieces = tp && tph_takes_rows(D);
+    const bool half_pieces = tp && tph_takes_rows(D) && !(odd && forced);
     bool mixed = false;  // rows with bf16 among them
     const bool rows_as_they_are = tp && combo != kFFFF;
     for (int i = 0; i < nscans; i++) {
@@ -943,7 +946,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         else if (half_pieces)
             launch_scan_tph(workspace, args, odd, stream);
         else
-            launch_scan_tp(workspace, args, stream);
+            launch_scan_tp(workspace, args, odd, stream);
     } else if (wg) {
         launch_scan_wg_ffff(D, F, fused != nullptr, workspace, args, stream);
     } else if (dma) {

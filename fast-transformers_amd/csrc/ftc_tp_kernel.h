@@ -146,6 +146,22 @@ struct RowQuad<1> {
     }
 };
 
+// which words of a quad of columns from `col` on are a row's own, of `width` columns (the first one is)
+template <bool ODD>
+struct OwnWords {
+    uint32_t m[3];
+    __device__ __forceinline__ OwnWords(int col, int width) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) m[e] = col + e + 1 < width ? 0xffffffffu : 0u;
+    }
+    template <typename Raw>
+    __device__ __forceinline__ Raw of(const Raw r, bool last_block = true) const {
+        if constexpr (ODD)
+            if (last_block) return Raw{r.x, r.y & m[0], r.z & m[1], r.w & m[2]};
+        return r;
+    }
+};
+
 // which scan (and block of columns and segment: `which`) and which chain a workgroup takes:
 // workgroups of one scan in groups of 8 (one per XCD), the groups of the scans of a launch side by
 // side, so that scans reading the same rows share an L2 (also the segments of a chain, which read the
@@ -184,7 +200,11 @@ constexpr int kTpZBytes = 4 * 2 * 2 * 64;  // z of the four consumers, fused att
 // are stored.
 // PA, PB, PV: pieces of the values of a, b and v: three for fp32 rows, one for bf16 rows, which are
 // multiplied as they are; TO: the type of the result's rows
-template <int ND, int KS2, bool NORM, int PA, int PB, int PV, typename TO>
+// ODD: fp32 rows of any width on 4-byte boundaries, as in ftc_tph_kernel.h: requests of 16 bytes all the
+// same, words that belong to the next row cleared as a quad is cut, quads that straddle the end of a row
+// stored word by word.  A chunk costs what it costs at the next multiple of 4; what is saved are copies
+// (forward, 25 x 33, 99 chains, L=1531 77 -> 33 us, odd_on_three_pieces)
+template <int ND, int KS2, bool NORM, int PA, int PB, int PV, typename TO, bool ODD = false>
 __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, const ScanArgs &p, uint32_t which,
                                              uint32_t chain, lds_char *unit_pc, lds_char *pt_pc,
                                              float (*den_mem)[NORM ? kChunk : 1][2], uint32_t *order_sh) {
@@ -303,6 +323,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
         for (int hb = 0; hb < ND; hb++) ab_in[hb] = 4 * (ptid % QA) + D * hb < Dw;
         const bool v_in = 4 * (ptid % QV) < fw;
+        const OwnWords<ODD> ab_own(4 * (ptid % QA), Dw - D * (ND - 1)), v_own(4 * (ptid % QV), fw);
         uint32_t a_goff[LA], b_goff[LA], v_goff[LV];
         int a_waddr[LA], b_waddr[LA], v_waddr[LV];
 #pragma unroll
@@ -382,14 +403,14 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             lds_char *const pc = unit_pc + buf * kBufBytes;
 #pragma unroll
             for (int q = 0; q < LA; q++) {
-                if (own) QuadA::to_lds(feature_a(r.a[q], hb), pc, kTileA, a_waddr[q]);
+                if (own) QuadA::to_lds(ab_own.of(feature_a(r.a[q], hb), hb == ND - 1), pc, kTileA, a_waddr[q]);
                 if (own || q == 0)
-                    QuadB::to_lds(feature_b(r.b[q], hb, v, q), pc + kOffB, kTileA, b_waddr[q]);
+                    QuadB::to_lds(ab_own.of(feature_b(r.b[q], hb, v, q), hb == ND - 1), pc + kOffB, kTileA, b_waddr[q]);
             }
             if (hb == 0) {
 #pragma unroll
                 for (int q = 0; q < LV; q++)
-                    if (own || q == 0) QuadV::to_lds(r.v[q], pc + kOffV, kTileV, v_waddr[q]);
+                    if (own || q == 0) QuadV::to_lds(v_own.of(r.v[q]), pc + kOffV, kTileV, v_waddr[q]);
             }
             // (a request whose answer is not used would be moved out of the loop: the waits
             // are the same either way)
@@ -504,7 +525,9 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
     for (int x = 0; x < 2; x++)
         o_lane[x] = (uint32_t)(16 * (x ^ ih) + ln) * o_slb + (uint32_t)kOutBytes * (16 * w + 4 * g);
-    const bool o_in = 16 * w + 4 * g < fw;  // (columns beyond the width are not stored)
+    const int o_cols = fw - (16 * w + 4 * g);
+    const bool o_in = o_cols >= (ODD ? 4 : 1);  // (columns beyond the width are not stored)
+    const bool o_straddles = ODD && fw > 0 && fw % 4 != 0 && fw / 16 == w;
 
     f32x4 S[ND][4];  // the slab's rows, block by block
 #pragma unroll
@@ -560,14 +583,28 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     // without it, the workgroup form's short segments are 3e-7; the time is the same.  Not there while
     // chunks are walked for their state alone, nor with two blocks: its registers would spill.  bf16 rows: the state handed
     // out after 1000 positions was 2.7e-7 off without it, 1.0e-7 on the kernels that split L.)
-    constexpr bool kMixed = PA + PB + PV < 9, kApart = (NORM && ND == 1) || kMixed;
+    // ODD: also while chunks are walked for their state (220 -> 237 registers); with two blocks each
+    // chunk's products by themselves, a tile's sum added to the state as soon as it is whole (in the first
+    // walk only where the last block has 32 rows: else 111 registers would spill).  127 x 127 backward,
+    // 15 chains, L=710: 2-norm error 3.6e-7 -> 1.9e-7 at the same time.
+    constexpr bool kMixed = PA + PB + PV < 9, kApart = ((NORM || ODD) && ND == 1) || kMixed,
+                   kFirstApart = kMixed || (ODD && ND == 1), kChunkSums = ODD && ND > 1,
+                   kFirstSums = kChunkSums && KS2 == 1;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 R[ND][4], Zr[ND][2];
-    auto add_product = [&](int hb, int dt, const Frag &x, const Frag &y) {
-        if (kApart)
+    f32x4 chunk_sum[4];
+    auto add_product = [&](int hb, int dt, const Frag &x, const Frag &y, bool first) {
+        if (kChunkSums)
+            chunk_sum[dt] = mfma16(x, y, first ? zero : chunk_sum[dt]);
+        else if (kApart)
             R[hb][dt] = mfma16(x, y, R[hb][dt]);
         else
             S[hb][dt] = mfma16(x, y, S[hb][dt]);
+    };
+    auto add_chunk_sums = [&](int hb, int first, int end) {
+        if (kChunkSums)
+#pragma unroll
+            for (int dt = first; dt < end; dt++) S[hb][dt] += chunk_sum[dt];
     };
     auto state = [&](int hb, int dt, int r) -> float { return kApart ? S[hb][dt][r] + R[hb][dt][r] : S[hb][dt][r]; };
     auto sum_of_keys = [&](int hb, int t, int r) -> float { return Z[hb][t][r] + Zr[hb][t][r]; };
@@ -630,9 +667,17 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     int buf = 0;  // LDS buffer of the chunk at hand
     if (n1 > 0) {
         // ---- the first n1 positions of the walk: state update only ----
-        if (kMixed) clear_apart();
-        auto add_first = [&](int hb, int dt, const Frag &x, const Frag &y) {
-            if (kMixed)
+        if (kFirstApart) clear_apart();
+        // product i of the 24 of a position: tile by tile, or (sums of a chunk by themselves) two tiles after
+        // the other two, whose sums are added meanwhile
+        auto add_first = [&](int hb, int i, const Frag (&btx)[4][PB], const Frag (&vfx)[PV]) {
+            const int dt = kFirstSums ? 2 * (i / 12) + i % 2 : i % 4, m = kFirstSums ? i % 12 / 2 : i / 4;
+            if (kFirstSums && (i == 14 || i == 15)) S[hb][i - 14] += chunk_sum[i - 14];
+            if (dt / 2 >= block_ks(hb) || m >= OfS::count) return;
+            const Frag &x = btx[dt][OfS::x(m)], &y = vfx[OfS::y(m)];
+            if (kFirstSums)
+                chunk_sum[dt] = mfma16(x, y, m == 0 ? zero : chunk_sum[dt]);
+            else if (kFirstApart)
                 R[hb][dt] = mfma16(x, y, R[hb][dt]);
             else
                 S[hb][dt] = mfma16(x, y, S[hb][dt]);
@@ -664,6 +709,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
         for (int hb = 0; hb < ND; hb++) b_in[hb] = 4 * cc4 + D * hb < Dw;
         const bool v_in = 4 * cc4 < fw;
+        const OwnWords<ODD> b_own(4 * cc4, Dw - D * (ND - 1)), v_own(4 * cc4, fw);
         const uint32_t b_goff = (uint32_t)crow * b_slb + 4u * QuadB::bytes * cc4,
                        v_goff = (uint32_t)crow * v_slb + 4u * QuadV::bytes * cc4;
         const int b_waddr = TpSwizzle<RBA>::addr(crow, 2 * b_tile_column(4 * cc4)),
@@ -692,10 +738,10 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 }
                 if (!b_in[v % ND]) x = u32x4{0, 0, 0, 0};
             }
-            QuadB::to_lds(x, unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
+            QuadB::to_lds(b_own.of(x, v % ND == ND - 1), unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
         };
         auto ccut_v = [&](const RawC &r, int bufk) {
-            QuadV::to_lds(r.v, unit_pc + bufk * kBufBytes + kOffV, kTileV, v_waddr);
+            QuadV::to_lds(v_own.of(r.v), unit_pc + bufk * kBufBytes + kOffV, kTileV, v_waddr);
         };
 #pragma unroll
         for (int j = 0; j < PF; j++) cfetch(rawc[j], j, j % ND);
@@ -718,16 +764,13 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 const int hp = (j + ND - 1) % ND;  // block of the position before
 #pragma unroll
                 for (int i = 0; i < 24; i++) {
-                    const bool rows_exist = (i % 4) / 2 < block_ks(hp);
                     if (j % 2 == 0) {
-                        if (rows_exist && i < 4 * OfS::count)
-                            add_first(hp, i % 4, bt2[i % 4][OfS::x(i / 4)], vf2[OfS::y(i / 4)]);
+                        add_first(hp, i, bt2, vf2);
                         if constexpr (NORM)
                             add_keys(hp, i, bt2);
                         tr_frag_into(bt, vf, pc, pcv, i, j % ND);
                     } else {
-                        if (rows_exist && i < 4 * OfS::count)
-                            add_first(hp, i % 4, bt[i % 4][OfS::x(i / 4)], vf[OfS::y(i / 4)]);
+                        add_first(hp, i, bt, vf);
                         if constexpr (NORM)
                             add_keys(hp, i, bt);
                         tr_frag_into(bt2, vf2, pc, pcv, i, j % ND);
@@ -736,24 +779,25 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                     if (i == 19 && cut_next && (j + 1) % ND == 0) ccut_v(rn, bufn);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                if (kFirstSums) add_chunk_sums(hp, 2, 2 * block_ks(hp));
                 cfetch(rawc[(j + 1) % PF], c + j + 1 + PF, (j + 1) % ND);
                 buf = bufn;
                 bufn = next_buf(bufn);
                 wg_barrier();
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (kMixed && c % 8 == 0) add_apart();
+            if (kFirstApart && c % 8 == 0) add_apart();
         }
         // the last of these positions (n1 is even: its fragments are in the second set)
 #pragma unroll
         for (int i = 0; i < 24; i++) {
-            if ((i % 4) / 2 < KS2 && i < 4 * OfS::count)
-                add_first(ND - 1, i % 4, bt2[i % 4][OfS::x(i / 4)], vf2[OfS::y(i / 4)]);
+            add_first(ND - 1, i, bt2, vf2);
             if constexpr (NORM)
                 add_keys(ND - 1, i, bt2);
             rm_frag(unit_pc + buf * kBufBytes, i, 0);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (kFirstSums) add_chunk_sums(ND - 1, 2, 2 * KS2);
     } else {
         wg_barrier();
         FTC_STAMP(13);  // first chunk cut
@@ -770,7 +814,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         StateExchange<DX, 1> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);
-        if (kMixed && n1 > 0) add_apart();
+        if (kFirstApart && n1 > 0) add_apart();
         f32x16 Sx[DX][1], X[DX][1];
         if (NORM) {
             Sx[DX - 1][0] = f32x16{};
@@ -804,7 +848,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         }
         if (!NORM && op.s0) add_caller_state();
     }
-    if (kMixed && n1 > 0 && !exchange) add_apart();
+    if (kFirstApart && n1 > 0 && !exchange) add_apart();
     clear_apart();
     // S_w as pieces in A operand order (slots 0..3 from tile 2 ks, 4..7 from tile 2 ks + 1).
     // Tiles 0 and 1 are final after phase 3 and are cut under phase 4, tiles 2 and 3 after
@@ -835,6 +879,13 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         f32x4 o = O4[x][0] + O4[x][1];
         if (NORM) o *= r_den[x];
         buffer_store_out(o_rs, o_in ? o_off + o_lane[x] : kNoRow, o[0], o[1], o[2], o[3], (TO *)nullptr);
+        if (o_straddles) {
+            const uint32_t first = o_off + o_lane[x];
+#pragma unroll
+            for (int e = 0; e < 3; e++)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[e]), o_rs,
+                                                      o_cols < 4 && o_cols > e ? first + 4u * e : kNoRow, 0, 0);
+        }
     };
     f32x4 Pkeep = {0.f, 0.f, 0.f, 0.f};  // the quadrant summed over the blocks so far
     f32x4 Az = {0.f, 0.f, 0.f, 0.f};     // NORM: phi(a) z of the quadrant's positions
@@ -930,7 +981,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 if (ks < block_ks(hb) && m < OfO::count)
                     O4[x][ks] = mfma16(sf[ks][OfO::x(m)], af[x][ks][OfO::y(m)], O4[x][ks]);
                 if (i < 2 * OfS::count)
-                    add_product(hb, i % 2, bt[i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)]);
+                    add_product(hb, i % 2, bt[i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)], i < 2);
                 if constexpr (NORM)
                     if (i < 6) {
                         f32x4 &sum = kApart ? Zr[hb][i % 2] : Zr[0][i % 2];
@@ -952,6 +1003,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             if (c == c0 + 4) FTC_STAMP(4);
             // All of Pt is in LDS and the next chunk is cut: its row-major fragments are
             // requested under what follows.
+            add_chunk_sums(hb, 0, 2);
             // phase 4: (3) for tiles 2 and 3 in turn with (2a) Ot_w += v_w^T Pt; underneath:
             // tiles 0, 1 of S_w cut into pieces
             const lds_char *pn = unit_pc + buf * kBufBytes;
@@ -979,7 +1031,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 if (block_ks(hb) > 1 && i < 2 * OfS::count)
-                    add_product(hb, 2 + i % 2, bt[2 + i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)]);
+                    add_product(hb, 2 + i % 2, bt[2 + i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)], i < 2);
                 cut_s((hb + 1) % ND, 0, i);
                 rm_frag(pn, i, (hb + 1) % ND);  // (past the last chunk: a buffer of zeros)
                 __builtin_amdgcn_sched_barrier(0);
@@ -988,11 +1040,12 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             for (int i = 0; i < 12; i++) {
                 if (4 + i < 2 * OfS::count && block_ks(hb) > 1) {
                     const int t = 4 + i;
-                    add_product(hb, 2 + t % 2, bt[2 + t % 2][OfS::x(t / 2)], vf[OfS::y(t / 2)]);
+                    add_product(hb, 2 + t % 2, bt[2 + t % 2][OfS::x(t / 2)], vf[OfS::y(t / 2)], false);
                 }
                 const int x = i % 2, m = i / 2;
                 if (last_block && m < OfV::count)
                     O4[x][m % 2] = mfma16(vf[OfV::x(m)], pf[x][OfV::y(m)], O4[x][m % 2]);
+                if (i == 10 && block_ks(hb) > 1) add_chunk_sums(hb, 2, 4);
                 rm_frag(pn, 4 + i, (hb + 1) % ND);
                 if (i < 2) rm_frag(pn, 16 + i, (hb + 1) % ND);
                 __builtin_amdgcn_sched_barrier(0);
@@ -1041,7 +1094,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     }
 }
 
-template <int ND, int KS2, bool NORM>
+template <int ND, int KS2, bool NORM, bool ODD = false>
 __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     __shared__ __align__(16) char pieces_mem[kTpPieceBytes<3, 3, 3>];
     __shared__ __align__(16) char pt_mem[kTpPtBytes + (NORM && ND > 1 ? kTpZBytes : 0)];
@@ -1049,8 +1102,8 @@ __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ 
     __shared__ uint32_t order_sh;
     uint32_t which, chain;
     tp_workgroup(p, which, chain);
-    scan_tp_body<ND, KS2, NORM, 3, 3, 3, float>(ws_ptr, p, which, chain, (lds_char *)pieces_mem, (lds_char *)pt_mem,
-                                                den_mem, &order_sh);
+    scan_tp_body<ND, KS2, NORM, 3, 3, 3, float, ODD>(ws_ptr, p, which, chain, (lds_char *)pieces_mem, (lds_char *)pt_mem,
+                                                     den_mem, &order_sh);
 }
 
 }  // namespace mfma

@@ -140,3 +140,57 @@ def test_small_rows_and_columns_beside_large_ones(small, shape, results):
         for dim in (2, 3):
             if name in results:
                 assert _each(got.cpu(), ex, dim) <= max(4 * _each(ref, ex, dim), 2e-6)
+
+
+THREE_PIECES = [
+    # N, H, L, E, M: states of one and two groups of 32 rows and of one and two blocks of 64; quads that
+    # straddle the width of a first and of a second block by one, two and three words; widths on either
+    # side of a block; one to three blocks of output columns; whole, cut and exchanged chains; scans of a
+    # backward call in one launch and in two
+    (9, 11, 97, 25, 33), (3, 2, 200, 10, 9), (2, 4, 300, 63, 31), (1, 3, 2100, 18, 18), (2, 3, 333, 33, 70),
+    (2, 4, 130, 65, 63), (3, 3, 220, 70, 70), (1, 5, 900, 95, 97), (1, 2, 2600, 99, 101), (2, 2, 260, 127, 127),
+    (1, 4, 150, 110, 150), (5, 8, 33, 75, 11),
+]
+
+
+@pytest.mark.parametrize("shape", THREE_PIECES, ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+def test_odd_widths_in_place_on_three_pieces(shape, monkeypatch):
+    """As above on the kernel of three bf16 pieces, with rows that have NaN beside them and with a state
+    handed in and out."""
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = shape
+    monkeypatch.setenv("FTC_ODD", "2")  # (also where another kernel would take them)
+    cp.reload_tuning()
+    try:
+        Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=950 + L)
+
+        def boxed(t, X, fill):
+            box = torch.full((N, L, H, X + 3), fill, device="cuda")
+            view = box[..., 1:X + 1].permute(0, 2, 1, 3)
+            if t is not None:
+                view.copy_(t)
+            return box, view
+        q, k, v, g = (boxed(t, t.shape[3], float("nan"))[1] for t in (Q, K, V, G))
+        boxes, outs = zip(*(boxed(None, X, 7.0) for X in (M, E, E, M)))
+        cp.causal_dot_product_hip(q, k, v, outs[0])
+        assert b"scan_tp_kernel" in _native.load().ftc_last_kernel()
+        cp.causal_dot_backward_hip(q, k, v, g, *outs[1:])
+        if max(E, M) <= 128:
+            assert b"scan_tp_kernel" in _native.load().ftc_last_kernel()
+        s0 = torch.randn(N, H, E, M, generator=torch.Generator().manual_seed(L))
+        out, s1 = cp.causal_dot_product_with_state(q, k, v, s0.cuda())
+        cp.check_workspaces()
+        for box in boxes:
+            assert (box[..., 0] == 7).all() and (box[..., -2:] == 7).all()
+        want = (oracle.forward(Q, K, V),) + tuple(oracle.backward(Q, K, V, G))
+        d = [t.double() for t in (Q, K, V, G)]
+        exact = (oracle.forward(*d[:3]),) + tuple(oracle.backward(*d))
+        for got, ref, ex in zip(outs, want, exact):
+            assert scale_error(got.cpu(), ex) <= max(4 * scale_error(ref, ex), 2e-6)
+        with_state = exact[0] + d[0] @ s0.double()
+        assert scale_error(out.cpu(), with_state) <= max(4 * scale_error(want[0], exact[0]), 2e-6)
+        assert scale_error(s1.cpu(), s0.double() + d[1].transpose(2, 3) @ d[2]) <= max(4 * scale_error(want[0], exact[0]), 2e-6)
+    finally:
+        monkeypatch.delenv("FTC_ODD")
+        cp.reload_tuning()
