@@ -586,7 +586,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     // ODD: also while chunks are walked for their state (220 -> 237 registers); with two blocks each
     // chunk's products by themselves, a tile's sum added to the state as soon as it is whole (in the first
     // walk only where the last block has 32 rows: else 111 registers would spill).  127 x 127 backward,
-    // 15 chains, L=710: 2-norm error 3.6e-7 -> 1.9e-7 at the same time.
+    // 15 chains, L=710: 2-norm error 3.6e-7 -> 2.7e-7 at the same time.
     constexpr bool kMixed = PA + PB + PV < 9, kApart = ((NORM || ODD) && ND == 1) || kMixed,
                    kFirstApart = kMixed || (ODD && ND == 1), kChunkSums = ODD && ND > 1,
                    kFirstSums = kChunkSums && KS2 == 1;
