@@ -750,6 +750,56 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
     return FTC_OK;
 }
 
+// Whether `units` = chains x scans of at most 64 rows and columns are faster in one launch of the kernel
+// that takes odd widths on three bf16 pieces, where scans of different shapes may stand side by side, than
+// where their widths send them.  `mixed`: scans of several shapes, which are a launch per shape elsewhere;
+// else scans of up to 32 x 32, which are one launch of the kernels that split L.  Measured over 130 calls
+// (us, before / here), backward of two shapes: 32 x 64, 11 chains, L=128 18 / 9; 1 chain, L=1440 51 / 24; 30 chains, L=1280 58 /
+// 37; 80 chains, L=1000 60 / 44; 24 x 48, 20 chains, L=608 34 / 19; 164 chains, L=3968 341 / 326; 190 chains, L=96 24 / 22; but 32 x 64,
+// 32 chains, L=6944 144 / 171, 128 chains, L=4096 (384 workgroups, a round and a half) 244 / 294, 219 chains, L=896 96 / 109.
+// 32 x 32: forward, 16 chains, L=200 11.3 / 9.2, 48 chains, L=400 14.3 / 12.0, 1 chain, L=7552 27 / 20, backward, 22 chains, L=160 11.8 /
+// 8.1; but 7 chains, L=768 16 / 18, 56 chains, L=1920 44 / 51, 360 chains, L=256 forward 17.6 / 21.1.
+bool narrow_rule(int64_t units, int64_t L, bool mixed) {
+    if (tuning().odd >= 0) return tuning().odd == 2;  // tuning aid
+    if (tuning().tp >= 0 || tuning().tph >= 0 || tuning().dma >= 0 || tuning().wg >= 0) return false;
+    const int64_t chunks = (L + 31) / 32;
+    if (!mixed) return (units <= 256 && chunks <= 16) || (units <= 4 && chunks >= 100);
+    if (units <= 256) return chunks <= 128 || units <= 64;
+    return units <= 512 ? chunks <= 8 || (units >= 448 && chunks <= 128) : units <= 768 && chunks <= 4;
+}
+
+// Whether the scans of a call go out that way: fp32 rows that need no copies.  (An exchange that the
+// workspace has no room for leaves them to the other kernels.)
+bool narrow_scans_together(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, const void *workspace,
+                           size_t workspace_bytes) {
+    bool mixed = false;
+    int D = 0, F = 0;
+    for (int i = 0; i < n; i++) {
+        const ScanDesc &sc = scans[i];
+        D = std::max(D, sc.a.width), F = std::max(F, sc.v.width);
+        mixed = mixed || sc.a.width != scans[0].a.width || sc.v.width != scans[0].v.width;
+        if (sc.a.width % 4 || sc.v.width % 4 || sc.out.dtype != FTC_F32) return false;
+        for (const Operand *o : {&sc.a, &sc.b, &sc.v})
+            if (o->dtype != FTC_F32 ||
+                !mfma_operand_in_place(o->ptr, o->stride_n, o->stride_h, o->stride_l, FTC_F32, o->width, L))
+                return false;
+        if (!mfma_operand_in_place(sc.out.ptr, sc.out.stride_n, sc.out.stride_h, sc.out.stride_l, FTC_F32,
+                                   sc.out.width, L))
+            return false;
+    }
+    if (D > (mixed ? 64 : 32) || F > (mixed ? 64 : 32) || !narrow_rule(N * H * n, L, mixed)) return false;
+    const int64_t need = mfma_tp_workspace_bytes(N, H, L, D, F, n, true, true);
+    return (need == 0 || plan_only() || (workspace && (int64_t)workspace_bytes >= need)) &&
+           mfma_tp_takes(scans, n, N, H, L, true, true);
+}
+// ... and the room that it takes
+int64_t narrow_together_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int n) {
+    const bool mixed = n > 1 && D != F;
+    const int64_t w = mixed ? std::max(D, F) : D;
+    if (D % 4 || F % 4 || std::max(D, F) > (mixed ? 64 : 32) || !narrow_rule(N * H * n, L, mixed)) return 0;
+    return mfma_tp_workspace_bytes(N, H, L, w, mixed ? w : F, n, true, true);
+}
+
 // Runs a list of independent scans.  A scan whose shape the MFMA kernels cover is cut into
 // column slices; consecutive slices (of any of the scans) that share widths and element
 // types go out in one launch.  Everything else takes the generic path.
@@ -763,6 +813,8 @@ int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
     // The scans of one shape go to the chain-parallel kernel together where it takes them
     // (whole scans: a column slice made below is never offered to it).
     bool offered[kMfmaMaxScans] = {};
+    if (narrow_scans_together(scans, n, N, H, L, workspace, workspace_bytes))
+        return mfma_scan(scans, n, N, H, L, workspace, workspace_bytes, stream, nullptr, true, true, true);
     for (int i = 0; i < n; i++) {
         if (!wide_shape(scans[i].a.width, scans[i].v.width)) continue;
         const int rc = wide_scan(scans[i], N, H, L, workspace, workspace_bytes, stream);
@@ -886,6 +938,8 @@ int64_t scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t
     if (with_pad && !bf16 && padded_scan_workspace_bytes(N, H, L, D, F) > 0)
         for (int k = 1; k <= kMfmaMaxScans; k++)
             need = std::max(need, mfma_tp_workspace_bytes(N, H, L, D, F, k, false, true));
+    for (int k = 1; k <= 3 && with_pad && !bf16; k++)
+        need = std::max(need, narrow_together_workspace_bytes(N, H, L, D, F, k));
     if (with_pad && split_widths(D, F))
         need = std::max(need, split_scan_workspace_bytes(N, H, L, D, F, nullptr));
     return need;

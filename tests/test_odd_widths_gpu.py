@@ -194,3 +194,40 @@ def test_odd_widths_in_place_on_three_pieces(shape, monkeypatch):
     finally:
         monkeypatch.delenv("FTC_ODD")
         cp.reload_tuning()
+
+
+TOGETHER = [
+    # N, H, L, E, M (widths that need no copies): two state shapes side by side, whole, cut and exchanged
+    # chains, one and two groups of 32 rows, a single chunk, ragged ends; and 32 x 32
+    (2, 3, 70, 32, 64), (1, 1, 32, 64, 32), (5, 4, 300, 24, 48), (2, 4, 2050, 64, 32), (1, 2, 5000, 60, 20),
+    (9, 9, 90, 20, 36), (4, 8, 200, 32, 32), (2, 2, 33, 20, 24), (1, 1, 3500, 32, 32),
+]
+
+
+@pytest.mark.parametrize("shape", TOGETHER, ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+def test_narrow_scans_share_a_launch(shape):
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = shape
+    plan = _native.plan((N, H, L, E), (N, H, L, M), backward=True)
+    assert plan.startswith("scan_tp_kernel") and ": 3 scans" in plan and plan.count("workgroups") == 1
+    Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=970 + L)
+    d = [t.double() for t in (Q, K, V, G)]
+    q, k, v, g = (t.permute(0, 2, 1, 3).contiguous().cuda().permute(0, 2, 1, 3) for t in (Q, K, V, G))
+    outs = [torch.empty_like(t) for t in (v, q, k, v)]
+    cp.causal_dot_product_hip(q, k, v, outs[0])
+    cp.causal_dot_backward_hip(q, k, v, g, *outs[1:])
+    s0 = torch.randn(N, H, E, M, generator=torch.Generator().manual_seed(L))
+    out, s1 = cp.causal_dot_product_with_state(q, k, v, s0.cuda())
+    cp.check_workspaces()
+    want = (oracle.forward(Q, K, V),) + tuple(oracle.backward(Q, K, V, G))
+    exact = (oracle.forward(*d[:3]),) + tuple(oracle.backward(*d))
+    for got, ref, ex in zip(outs, want, exact):
+        assert scale_error(got.cpu(), ex) <= max(4 * scale_error(ref, ex), 2e-6)
+    bound = max(4 * scale_error(want[0], exact[0]), 2e-6)
+    assert scale_error(out.cpu(), exact[0] + d[0] @ s0.double()) <= bound
+    assert scale_error(s1.cpu(), s0.double() + d[1].transpose(2, 3) @ d[2]) <= bound
+    # one gradient by itself is the same to rounding, whatever launch it is in
+    alone = torch.empty_like(q)
+    cp.causal_dot_backward_hip(q, k, v, g, None, alone, None)
+    assert scale_error(alone.cpu(), exact[2]) <= max(4 * scale_error(want[2], exact[2]), 2e-6)
