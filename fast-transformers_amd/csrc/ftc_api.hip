@@ -724,6 +724,10 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
         if (k == ngroups) size[ngroups++] = 0;
         group[k][size[k]++] = scans[i];
     }
+    // (on three pieces: blocks of columns, in which scans may differ)
+    auto blocks = [forced](const ScanDesc *s, int k) {
+        return forced ? (int)column_blocks(s, k) : k;
+    };
     auto room = [&](int d, int f, int k) {
         const int64_t need = mfma_tp_workspace_bytes(N, H, L, d, f, k, forced, true);
         return need == 0 || plan_only() ||
@@ -732,17 +736,17 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
     bool apart_ok = true;
     for (int k = 0; k < ngroups; k++) {
         apart_ok = apart_ok && mfma_tp_takes(group[k], size[k], N, H, L, forced, true) &&
-                   room(group[k][0].a.width, group[k][0].v.width, size[k]);
-        if (apart_ok) apart += mfma_tp_odd_chunks(group[k][0].a.width, group[k][0].v.width, N, H, size[k], L, forced);
+                   room(group[k][0].a.width, group[k][0].v.width, blocks(group[k], size[k]));
+        if (apart_ok) apart += mfma_tp_odd_chunks(group[k][0].a.width, group[k][0].v.width, N, H, blocks(group[k], size[k]), L, forced);
     }
     const bool together_ok = ngroups > 1 && mfma_tp_takes(scans, n, N, H, L, forced, true) &&
-                             room(widest_d, widest_f, n);
+                             room(widest_d, widest_f, blocks(scans, n));
     if (!apart_ok && !together_ok) return FTC_OK;
     auto run = [&](const ScanDesc *s, int k) {
         return mfma_scan(s, k, N, H, L, workspace, workspace_bytes, stream, nullptr, true, forced, true);
     };
     *done = true;
-    if (together_ok && (!apart_ok || mfma_tp_odd_chunks(widest_d, widest_f, N, H, n, L, forced) <= apart)) return run(scans, n);
+    if (together_ok && (!apart_ok || mfma_tp_odd_chunks(widest_d, widest_f, N, H, blocks(scans, n), L, forced) <= apart)) return run(scans, n);
     for (int k = 0; k < ngroups; k++) {
         const int rc = run(group[k], size[k]);
         if (rc) return rc;
@@ -750,7 +754,7 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
     return FTC_OK;
 }
 
-// Whether `units` = chains x scans of at most 64 rows and columns are faster in one launch of the kernel
+// Whether `units` = chains x blocks of 64 columns of the scans of a call are faster in one launch of the kernel
 // that takes odd widths on three bf16 pieces, where scans of different shapes may stand side by side, than
 // where their widths send them.  `mixed`: scans of several shapes, which are a launch per shape elsewhere;
 // else scans of up to 32 x 32, which are one launch of the kernels that split L.  Measured over 130 calls
@@ -759,11 +763,17 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
 // 32 chains, L=6944 144 / 171, 128 chains, L=4096 (384 workgroups, a round and a half) 244 / 294, 219 chains, L=896 96 / 109.
 // 32 x 32: forward, 16 chains, L=200 11.3 / 9.2, 48 chains, L=400 14.3 / 12.0, 1 chain, L=7552 27 / 20, backward, 22 chains, L=160 11.8 /
 // 8.1; but 7 chains, L=768 16 / 18, 56 chains, L=1920 44 / 51, 360 chains, L=256 forward 17.6 / 21.1.
-bool narrow_rule(int64_t units, int64_t L, bool mixed) {
+// `wide`: two shapes of which one has more than 64 rows, so that a chunk of every scan takes as long as one of
+// those; 100 calls, one round of workgroups: 72 x 100, 11 chains, L=128 24 / 13, 36 chains, L=1728 171 / 114; 128 x 64, 20 chains, L=608 47 /
+// 32; 64 x 128, 64 chains, L=64 16 / 10; but 128 x 64, 35 chains, L=3520 172 / 228, 58 chains of 128 x 32, L=96 (290
+// workgroups) 19 / 21.  Fewer workgroups on longer chains would exchange segment sums and win as well (1 chain,
+// L=1440, 64 x 128 57 / 35), but with errors up to a third larger than on the kernels that have them now.
+bool narrow_rule(int64_t units, int64_t L, bool mixed, bool wide) {
     if (tuning().odd >= 0) return tuning().odd == 2;  // tuning aid
     if (tuning().tp >= 0 || tuning().tph >= 0 || tuning().dma >= 0 || tuning().wg >= 0) return false;
     const int64_t chunks = (L + 31) / 32;
     if (!mixed) return (units <= 256 && chunks <= 16) || (units <= 4 && chunks >= 100);
+    if (wide) return mixed && units <= 256 && (chunks <= 16 || (units > 64 && units <= 224 && chunks <= 64));
     if (units <= 256) return chunks <= 128 || units <= 64;
     return units <= 512 ? chunks <= 8 || (units >= 448 && chunks <= 128) : units <= 768 && chunks <= 4;
 }
@@ -787,17 +797,25 @@ bool narrow_scans_together(const ScanDesc *scans, int n, int64_t N, int64_t H, i
                                    sc.out.width, L))
             return false;
     }
-    if (D > (mixed ? 64 : 32) || F > (mixed ? 64 : 32) || !narrow_rule(N * H * n, L, mixed)) return false;
-    const int64_t need = mfma_tp_workspace_bytes(N, H, L, D, F, n, true, true);
+    const int64_t blocks = column_blocks(scans, n);
+    if (D > (mixed ? 128 : 32) || F > (mixed ? 128 : 32) || !narrow_rule(N * H * blocks, L, mixed, D > 64)) return false;
+    const int64_t need = mfma_tp_workspace_bytes(N, H, L, D, F, (int)blocks, true, true);
     return (need == 0 || plan_only() || (workspace && (int64_t)workspace_bytes >= need)) &&
            mfma_tp_takes(scans, n, N, H, L, true, true);
 }
 // ... and the room that it takes
 int64_t narrow_together_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int n) {
     const bool mixed = n > 1 && D != F;
-    const int64_t w = mixed ? std::max(D, F) : D;
-    if (D % 4 || F % 4 || std::max(D, F) > (mixed ? 64 : 32) || !narrow_rule(N * H * n, L, mixed)) return 0;
-    return mfma_tp_workspace_bytes(N, H, L, w, mixed ? w : F, n, true, true);
+    const int64_t w = mixed ? std::max(D, F) : D, most = mixed ? 128 : 32;
+    if (D % 4 || F % 4 || std::max(D, F) > most) return 0;
+    // (two scans of one shape and one of the other, or one of each)
+    int64_t need = 0;
+    for (int two = 0; two < (n == 3 ? 2 : 1); two++) {
+        const int64_t d = (D + 63) / 64, f = (F + 63) / 64, blocks = !mixed ? n * f : n == 2 ? d + f : two ? 2 * d + f : d + 2 * f;
+        if (narrow_rule(N * H * blocks, L, mixed, w > 64))
+            need = std::max(need, mfma_tp_workspace_bytes(N, H, L, w, mixed ? w : F, (int)blocks, true, true));
+    }
+    return need;
 }
 
 // Runs a list of independent scans.  A scan whose shape the MFMA kernels cover is cut into

@@ -146,6 +146,8 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
 // ... and of scans with bf16 rows among them
 int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans);
 // estimated time of such a launch, in chunks walked one after the other
+// blocks of 64 output columns of several scans
+int64_t column_blocks(const ScanDesc *scans, int nscans);
 double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L, bool forced);
 // The fused attention form of a forward scan: a and b go through the feature map
 // elu(x) + 1, rows of b at or beyond key_lengths[n] count as zero, and every output row is

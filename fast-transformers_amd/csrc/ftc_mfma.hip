@@ -625,6 +625,7 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
                                 bool forced, bool odd) {
     int nseg = 0, seg_chunks = 0;
     const int64_t chains = std::max<int64_t>(1, N * H);
+    if (forced && odd) F = 64;  // (`nscans` blocks of columns, see column_blocks)
     tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, odd);
     return seg_chunks > 0 ? tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D) : 0;
 }
@@ -633,6 +634,13 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
 void widest_rows(const ScanDesc *scans, int nscans, int *D, int *F) {
     *D = *F = 0;
     for (int i = 0; i < nscans; i++) *D = std::max(*D, scans[i].a.width), *F = std::max(*F, scans[i].v.width);
+}
+
+// blocks of 64 output columns in all
+int64_t column_blocks(const ScanDesc *scans, int nscans) {
+    int64_t n = 0;
+    for (int i = 0; i < nscans; i++) n += tp_fblocks(scans[i].v.width);
+    return n;
 }
 
 bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L, bool forced,
@@ -650,11 +658,9 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
         if (combo != kFFFF && mixed == 0) mixed = kMixedRows;
         // (rows with bf16 among them: not as parts of wider scans, whose results are added up in fp32)
         if (combo == kNone || (combo != kFFFF && (forced || tuning().tph == 0))) return false;
-        // (odd widths: scans of any widths side by side, as long as they have as many blocks of columns:
-        // one, where pieces are scaled)
-        if ((sd.a.width != D || sd.v.width != F) &&
-            !(odd && (F <= 64 || (forced && tp_fblocks(sd.v.width) == tp_fblocks(F)))))
-            return false;
+        // (odd widths: scans of any widths side by side, where pieces are scaled as long as none has a
+        // second block of columns)
+        if ((sd.a.width != D || sd.v.width != F) && !(odd && (forced || F <= 64))) return false;
         if (odd && (combo != kFFFF || sd.a.width < 8 || sd.v.width < 8)) return false;
         if (L > 1 && !(stride_ok(sd.a.stride_l, sd.a.width) && stride_ok(sd.b.stride_l, sd.a.width) &&
                        stride_ok(sd.v.stride_l, sd.v.width) && stride_ok(sd.out.stride_l, sd.v.width)))
@@ -678,6 +684,8 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     const int64_t chains = std::max<int64_t>(1, N * H);
     if (mixed)
         mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks, &as_before);
+    else if (odd && forced)
+        tp_plan(D, 64, chains, (int)column_blocks(scans, nscans), L, &nseg, &seg_chunks, forced, 0, odd);
     else
         tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, odd);
     return nseg > 0;
@@ -696,8 +704,10 @@ int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D
     return bytes;
 }
 
+// (a chunk of a state of more than 64 rows takes 1.7 times as long)
 double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L, bool forced) {
     int nseg = 0, seg_chunks = 0;
+    if (forced) F = 64;  // (`nscans` blocks of columns)
     const int64_t chains = std::max<int64_t>(1, N * H), units = chains * nscans * tp_fblocks(F);
     tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, true);
     if (nseg == 0) return 1e30;
@@ -711,7 +721,7 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
         for (int s = 0; s < nseg; s++)
             longest = std::max(longest, 0.6 * start[s] + (double)(start[s + 1] - start[s]));
     }
-    return (double)rounds * (longest + 4.0);
+    return (double)rounds * ((D > 64 ? 1.7 : 1.0) * longest + 4.0);
 }
 
 // (rows of 128 values: the chain-parallel kernel alone)
@@ -805,6 +815,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         fused_tp = false, tpx_nseg = tpx_seg_chunks = 0;
     const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd);
     const int64_t fblocks = tp_shape || wide_rows ? tp_fblocks(F) : 1;
+    const int64_t blocks = odd && forced ? column_blocks(scans, nscans) : nscans * fblocks;
     if (fused_tp && tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     if (tp_shape) {
         int any_bf16 = nscans == 1 && combo == kBBFB ? kMixedGradValues : 0;
@@ -812,6 +823,8 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
             if (combo_of(scans[i]) != kFFFF && any_bf16 == 0) any_bf16 = kMixedRows;
         if (any_bf16)
             mixed_plan(D, F, chains, nscans, L, any_bf16, &tpx_nseg, &tpx_seg_chunks, &as_before);
+        else if (odd && forced)
+            tp_plan(D, 64, chains, (int)blocks, L, &tpx_nseg, &tpx_seg_chunks, forced, 0, odd);
         else
             tp_plan(D, F, chains, nscans, L, &tpx_nseg, &tpx_seg_chunks, forced, 0, odd);
         if (tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
@@ -826,7 +839,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         pl.nseg = tpx_nseg;
         pl.seg_len = tpx_seg_chunks * kChunk;
         pl.waves = chains * pl.nseg;
-        pl.workspace_bytes = tp_exchange_workspace_bytes(chains * nscans * fblocks, pl.nseg,
+        pl.workspace_bytes = tp_exchange_workspace_bytes(chains * blocks, pl.nseg,
                                                          fused_tp ? fused_tp_state_rows(D) : D);
     } else if (tp) {  // one workgroup per chain segment, nothing to exchange
         pl.nseg = tp_segment_starts((L + kChunk - 1) / kChunk, tp_nseg, tp_start);
@@ -891,8 +904,9 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     args.tp_seg_chunks = tpx_seg_chunks;
     args.nseg = pl.nseg;
     args.waves_per_scan = (int32_t)pl.waves;
-    args.total_waves = (int32_t)(pl.waves * nscans * fblocks);
+    args.total_waves = (int32_t)(pl.waves * blocks);
     args.tp_d = D, args.tp_fblocks = (int32_t)fblocks;
+    for (int i = 0; i < kMaxScans; i++) args.tp_first[i] = (int32_t)column_blocks(scans, std::min(i, nscans));
     // very short chains: one level (every step adds the sums of all steps before it);
     // otherwise groups of about sqrt(nseg) steps, which moves fewer states per step
     args.group = pl.nseg;

@@ -480,6 +480,8 @@ struct ScanArgs {
     // the widest rows of a and b over the scans (<= 128), and the number of 64-column blocks of v
     // and out, one workgroup each
     int32_t tp_d, tp_fblocks;
+    // (rows of odd widths, where scans may differ in that number: the first block of every scan)
+    int32_t tp_first[kMaxScans];
 };
 
 // Which (scan, chain, L-segment) a wavefront works on.

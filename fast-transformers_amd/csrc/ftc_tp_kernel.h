@@ -155,9 +155,8 @@ struct OwnWords {
         for (int e = 0; e < 3; e++) m[e] = col + e + 1 < width ? 0xffffffffu : 0u;
     }
     template <typename Raw>
-    __device__ __forceinline__ Raw of(const Raw r, bool last_block = true) const {
-        if constexpr (ODD)
-            if (last_block) return Raw{r.x, r.y & m[0], r.z & m[1], r.w & m[2]};
+    __device__ __forceinline__ Raw of(const Raw r) const {
+        if constexpr (ODD) return Raw{r.x, r.y & m[0], r.z & m[1], r.w & m[2]};
         return r;
     }
 };
@@ -237,8 +236,13 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     const uint32_t chains = (uint32_t)p.waves_per_scan / nseg;
     // (a scan with more than 64 output columns counts as two, one per block of columns)
     const uint32_t virt = which / nseg;
-    const uint32_t scan_id = virt / (uint32_t)p.tp_fblocks;
-    const int fb = (int)(virt % (uint32_t)p.tp_fblocks);
+    uint32_t scan_id = ODD ? 0 : virt / (uint32_t)p.tp_fblocks;
+    if (ODD) {
+#pragma unroll
+        for (int i = 1; i < kMaxScans; i++)
+            if ((int)virt >= p.tp_first[i]) scan_id = i;
+    }
+    const int fb = ODD ? (int)virt - p.tp_first[scan_id] : (int)(virt % (uint32_t)p.tp_fblocks);
     const ScanOperands &op = p.scan[scan_id];
     const int Dw = op.d;                        // state rows in all: a and b are this wide
     const int fw = min(F, op.f - F * fb);       // output columns of this block
@@ -323,7 +327,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
         for (int hb = 0; hb < ND; hb++) ab_in[hb] = 4 * (ptid % QA) + D * hb < Dw;
         const bool v_in = 4 * (ptid % QV) < fw;
-        const OwnWords<ODD> ab_own(4 * (ptid % QA), Dw - D * (ND - 1)), v_own(4 * (ptid % QV), fw);
+        const OwnWords<ODD> ab_own[2] = {{4 * (ptid % QA), Dw}, {4 * (ptid % QA) + D, Dw}}, v_own(4 * (ptid % QV), fw);
         uint32_t a_goff[LA], b_goff[LA], v_goff[LV];
         int a_waddr[LA], b_waddr[LA], v_waddr[LV];
 #pragma unroll
@@ -403,9 +407,9 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             lds_char *const pc = unit_pc + buf * kBufBytes;
 #pragma unroll
             for (int q = 0; q < LA; q++) {
-                if (own) QuadA::to_lds(ab_own.of(feature_a(r.a[q], hb), hb == ND - 1), pc, kTileA, a_waddr[q]);
+                if (own) QuadA::to_lds(ab_own[hb].of(feature_a(r.a[q], hb)), pc, kTileA, a_waddr[q]);
                 if (own || q == 0)
-                    QuadB::to_lds(ab_own.of(feature_b(r.b[q], hb, v, q), hb == ND - 1), pc + kOffB, kTileA, b_waddr[q]);
+                    QuadB::to_lds(ab_own[hb].of(feature_b(r.b[q], hb, v, q)), pc + kOffB, kTileA, b_waddr[q]);
             }
             if (hb == 0) {
 #pragma unroll
@@ -709,7 +713,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
         for (int hb = 0; hb < ND; hb++) b_in[hb] = 4 * cc4 + D * hb < Dw;
         const bool v_in = 4 * cc4 < fw;
-        const OwnWords<ODD> b_own(4 * cc4, Dw - D * (ND - 1)), v_own(4 * cc4, fw);
+        const OwnWords<ODD> b_own[2] = {{4 * cc4, Dw}, {4 * cc4 + D, Dw}}, v_own(4 * cc4, fw);
         const uint32_t b_goff = (uint32_t)crow * b_slb + 4u * QuadB::bytes * cc4,
                        v_goff = (uint32_t)crow * v_slb + 4u * QuadV::bytes * cc4;
         const int b_waddr = TpSwizzle<RBA>::addr(crow, 2 * b_tile_column(4 * cc4)),
@@ -738,7 +742,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 }
                 if (!b_in[v % ND]) x = u32x4{0, 0, 0, 0};
             }
-            QuadB::to_lds(b_own.of(x, v % ND == ND - 1), unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
+            QuadB::to_lds(b_own[v % ND].of(x), unit_pc + bufk * kBufBytes + kOffB, kTileA, b_waddr);
         };
         auto ccut_v = [&](const RawC &r, int bufk) {
             QuadV::to_lds(v_own.of(r.v), unit_pc + bufk * kBufBytes + kOffV, kTileV, v_waddr);

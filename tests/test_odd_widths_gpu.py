@@ -149,7 +149,7 @@ THREE_PIECES = [
     # backward call in one launch and in two
     (9, 11, 97, 25, 33), (3, 2, 200, 10, 9), (2, 4, 300, 63, 31), (1, 3, 2100, 18, 18), (2, 3, 333, 33, 70),
     (2, 4, 130, 65, 63), (3, 3, 220, 70, 70), (1, 5, 900, 95, 97), (1, 2, 2600, 99, 101), (2, 2, 260, 127, 127),
-    (1, 4, 150, 110, 150), (5, 8, 33, 75, 11),
+    (1, 4, 150, 110, 150), (5, 8, 33, 75, 11), (2, 4, 100, 35, 77), (1, 6, 90, 127, 63),
 ]
 
 
@@ -198,9 +198,11 @@ def test_odd_widths_in_place_on_three_pieces(shape, monkeypatch):
 
 TOGETHER = [
     # N, H, L, E, M (widths that need no copies): two state shapes side by side, whole, cut and exchanged
-    # chains, one and two groups of 32 rows, a single chunk, ragged ends; and 32 x 32
+    # chains, one and two groups of 32 rows, a single chunk, ragged ends; 32 x 32; and two shapes of which
+    # one has two blocks of rows, with one to three blocks of columns between the scans
     (2, 3, 70, 32, 64), (1, 1, 32, 64, 32), (5, 4, 300, 24, 48), (2, 4, 2050, 64, 32), (1, 2, 5000, 60, 20),
     (9, 9, 90, 20, 36), (4, 8, 200, 32, 32), (2, 2, 33, 20, 24), (1, 1, 3500, 32, 32),
+    (2, 3, 70, 64, 128), (3, 4, 300, 128, 32), (1, 5, 33, 72, 100), (6, 5, 700, 100, 40), (1, 2, 450, 96, 128),
 ]
 
 
