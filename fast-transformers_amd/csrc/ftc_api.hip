@@ -682,9 +682,10 @@ bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64
 // it saves, and faster than the kernels that split L, which narrow ones would go to).  Measured over
 // 170 calls (us, on copies / here): 25 x 33 forward, 99 chains, L=1531 77 / 33, 2000 chains, L=300 255 / 96;
 // 10 x 9, 214 chains, L=197 39 / 11; 70 x 33, 80 chains, L=1688 130 / 65; 127 x 127, 300 chains, L=2000 838 /
-// 446, backward, 24 chains, L=177 42 / 18; 99 x 101 backward, 2 chains, L=5038 71 / 44.  What keeps them:
-// single scans of more than 64 rows on up to three workgroups' worth of chains too short for an exchange
-// there (75 x 10, 1 chain, L=1942 28 / 67), thousands of workgroups with two chunks each (30 x 50 backward,
+// 446, backward, 24 chains, L=177 42 / 18; 99 x 101 backward, 2 chains, L=5038 71 / 44; the scans of two
+// shapes in one launch (odd_scans): 75 x 10 backward, 4 chains, L=789 105 / 32.  What keeps them:
+// single scans of more than 64 rows on up to four workgroups' worth of chains with few segments there
+// (75 x 10, 1 chain, L=1942 28 / 67, 4 chains, L=789 27 / 31), thousands of workgroups with two chunks each (30 x 50 backward,
 // 3000 chains, L=40 161 / 198), and calls of several scans on more than two rounds of workgroups and
 // 128 chunks or more (99 x 101 backward, 128 chains, L=4096 1494 / 922: faster here, but such a call's plan has the
 // copies in its name and size).  Rows of which some fit stay as in odd_in_place, and so does a workspace without room.
@@ -702,7 +703,7 @@ bool odd_on_three_pieces(const ScanDesc *scans, int n, const bool *padded, int64
         widest = std::max(widest, std::max(D, F));
     }
     if (tuning().odd == 2) return true;
-    if (n == 1 && scans[0].a.width > 64 && units <= 3 && chunks > 24 && chunks <= 64) return false;
+    if (n == 1 && scans[0].a.width > 64 && units <= 4 && chunks > 16 && chunks <= 64) return false;
     if (widest <= 64 && chunks <= 2 && units > 4096) return false;
     return n == 1 || units <= 512 || chunks < 128;
 }
