@@ -14,9 +14,9 @@
 // library rounds after every few: against float64 a product of 40960 x 512 by 512 x 512 is off by
 // 1.9e-7 (2-norm) where the library's is by 2.9e-7, of 1024 columns by 2.6e-7 and 4.1e-7.
 //
-// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 86, 512 -> 1536 475 / 220, 512 -> 1024
-// with relu 310 + 51 / 155, 1024 -> 512 with the residual 305 + 37 / 160; 5000 tokens, 256 -> 512 20 / 17;
-// 300 tokens, 128 -> 260 31 / 10.
+// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 85, 512 -> 1536 475 / 226, 512 -> 1024
+// with relu 310 + 51 / 155, 1024 -> 512 with the residual 305 + 37 / 162; 5000 tokens, 256 -> 512 20 / 11;
+// 300 tokens, 128 -> 260 31 / 4.2.  (At the largest sizes the card's power bounds it: on zeros 230 -> 189.)
 //
 // Rows in pieces take the bytes of fp32 rows: block of 32 columns after block, 64 bytes of hi and 64
 // of lo each, one cache line per row and k-step.  Whoever writes rows that only a product reads
