@@ -763,7 +763,8 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
 // 37; 80 chains, L=1000 60 / 44; 24 x 48, 20 chains, L=608 34 / 19; 164 chains, L=3968 341 / 326; 190 chains, L=96 24 / 22; but 32 x 64,
 // 32 chains, L=6944 144 / 171, 128 chains, L=4096 (384 workgroups, a round and a half) 244 / 294, 219 chains, L=896 96 / 109.
 // 32 x 32: forward, 16 chains, L=200 11.3 / 9.2, 48 chains, L=400 14.3 / 12.0, 1 chain, L=7552 27 / 20, backward, 22 chains, L=160 11.8 /
-// 8.1; but 7 chains, L=768 16 / 18, 56 chains, L=1920 44 / 51, 360 chains, L=256 forward 17.6 / 21.1.
+// 8.1; but 7 chains, L=768 16 / 18, 56 chains, L=1920 44 / 51, 360 chains, L=256 forward 17.6 / 21.1,
+// 4 chains, L=16384 forward 31.5 / 35.1.
 // `wide`: two shapes of which one has more than 64 rows, so that a chunk of every scan takes as long as one of
 // those; 100 calls, one round of workgroups: 72 x 100, 11 chains, L=128 24 / 13, 36 chains, L=1728 171 / 114; 128 x 64, 20 chains, L=608 47 /
 // 32; 64 x 128, 64 chains, L=64 16 / 10; but 128 x 64, 35 chains, L=3520 172 / 228, 58 chains of 128 x 32, L=96 (290
@@ -773,7 +774,7 @@ bool narrow_rule(int64_t units, int64_t L, bool mixed, bool wide) {
     if (tuning().odd >= 0) return tuning().odd == 2;  // tuning aid
     if (tuning().tp >= 0 || tuning().tph >= 0 || tuning().dma >= 0 || tuning().wg >= 0) return false;
     const int64_t chunks = (L + 31) / 32;
-    if (!mixed) return (units <= 256 && chunks <= 16) || (units <= 4 && chunks >= 100);
+    if (!mixed) return (units <= 256 && chunks <= 16) || (chunks >= 100 && chunks <= 448 && units * chunks <= 1300);
     if (wide) return mixed && units <= 256 && (chunks <= 16 || (units > 64 && units <= 224 && chunks <= 64));
     if (units <= 256) return chunks <= 128 || units <= 64;
     return units <= 512 ? chunks <= 8 || (units >= 448 && chunks <= 128) : units <= 768 && chunks <= 4;
