@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139228438, "84c8056ce888761b"),
-    "cfg3": (2604773370, "84c8056ce888761b"),
-    "cfg5": (5085015854, "84c8056ce888761b"),
-    "wide": (1877135204, "84c8056ce888761b"),
+    "cfg2": (139265485, "b3f2ab34ccb157de"),
+    "cfg3": (2603261303, "b3f2ab34ccb157de"),
+    "cfg5": (5084373663, "b3f2ab34ccb157de"),
+    "wide": (1877109282, "b3f2ab34ccb157de"),
 }
 
 WORKLOADS = {
