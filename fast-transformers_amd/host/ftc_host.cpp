@@ -435,7 +435,8 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
         const Tensor den = at::empty({q.size(0), q.size(2), q.size(1)}, q.options());
         const Tensor out = run(q, k, v, lengths, eps, den);
         ctx->save_for_backward({q, k, v, out, den});
-        ctx->saved_data["lengths"] = lengths;
+        // (rows of 128: as in the composition, which makes its mask here, the caller may have the lengths back)
+        ctx->saved_data["lengths"] = wide_rows(q, v) ? lengths.clone() : lengths;
         return out;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {

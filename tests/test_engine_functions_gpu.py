@@ -19,14 +19,16 @@ def operator(cp, dtype, seed=0):
     return [torch.rand(2, 3, 70, w, device="cuda", generator=gen).to(dtype) for w in (64, 64, 32)]
 
 
-def attention(seed=0):
+def attention(seed=0, widths=(64, 64, 32)):
     from fast_transformers_amd.attention import CausalLinearAttention
     from fast_transformers_amd.masking import LengthMask, TriangularCausalMask
     gen = torch.Generator(device="cuda").manual_seed(seed)
     lengths = LengthMask(torch.tensor([70, 33], device="cuda"), max_len=70)
-    module, mask = CausalLinearAttention(64), TriangularCausalMask(70, device="cuda")
-    inputs = [torch.randn(2, 70, 3, w, device="cuda", generator=gen) for w in (64, 64, 32)]
-    return inputs, lambda *t: module(*t, mask, lengths, lengths)
+    module, mask = CausalLinearAttention(widths[0]), TriangularCausalMask(70, device="cuda")
+    inputs = [torch.randn(2, 70, 3, w, device="cuda", generator=gen) for w in widths]
+    call = lambda *t: module(*t, mask, lengths, lengths)
+    call.lengths = lengths.lengths
+    return inputs, call
 
 
 def in_engine(out):
@@ -99,3 +101,20 @@ def test_python_errors_in_the_engine_reach_the_caller(cp):
     again = cp.causal_dot_product(q, k, v)
     grads = torch.autograd.grad(again.sum(), (q, k, v))
     assert all(torch.isfinite(g).all() for g in grads)
+
+
+def attention_at_128():
+    inputs, call = attention(widths=(128, 128, 128))
+    t = [x.clone().requires_grad_(True) for x in inputs]
+    out = call(*t)
+    assert in_engine(out)
+    return t, call, torch.autograd.grad(out, t, torch.ones_like(out))
+
+
+def test_lengths_may_change_between_forward_and_backward(cp):
+    """... at rows of 128, as in the composition, whose mask is made in the forward."""
+    t, call, want = attention_at_128()
+    out = call(*t)
+    call.lengths.fill_(5)
+    for a, b in zip(torch.autograd.grad(out, t, torch.ones_like(out)), want):
+        assert torch.equal(a, b)
