@@ -14,6 +14,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -434,9 +435,21 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
                           const Tensor &lengths, double eps) {
         const Tensor den = at::empty({q.size(0), q.size(2), q.size(1)}, q.options());
         const Tensor out = run(q, k, v, lengths, eps, den);
-        ctx->save_for_backward({q, k, v, out, den});
+        if (wide_rows(q, v)) {
+            // The composition does not keep its result, which the caller may then change in place: kept here
+            // as an alias that no check refuses, with a tensor that tells such a change (it shares the
+            // result's version), after which the backward computes the result again.
+            const Tensor version = at::empty({0}, out.options());
+            torch::autograd::impl::set_version_counter(version, torch::autograd::impl::version_counter(out));
+            ctx->saved_data["version"] = version;
+            ctx->saved_data["unchanged"] = (int64_t)out._version();
+            ctx->save_for_backward({q, k, v, out.variable_data(), den});
+        } else {
+            ctx->save_for_backward({q, k, v, out, den});
+        }
         // (rows of 128: as in the composition, which makes its mask here, the caller may have the lengths back)
         ctx->saved_data["lengths"] = wide_rows(q, v) ? lengths.clone() : lengths;
+        ctx->saved_data["eps"] = eps;
         return out;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
@@ -448,9 +461,12 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
             if (ctx->needs_input_grad(i)) out[i] = at::empty_like(saved[i]), to[i] = swapped(out[i]);
         from_engine([&] {
             const bool wide = wide_rows(saved[0], saved[2]);
+            Tensor result = saved[3];
+            if (wide && (int64_t)ctx->saved_data["version"].toTensor()._version() != ctx->saved_data["unchanged"].toInt())
+                result = run(saved[0], saved[1], saved[2], lengths, ctx->saved_data["eps"].toDouble(), std::nullopt);
             const Tensor g = wide && !reads_in_place(grads[0]) ? grads[0].clone(at::MemoryFormat::Contiguous) : grads[0];
             ::fused_attention_backward(swapped(saved[0]), swapped(saved[1]), swapped(saved[2]), lengths,
-                                       swapped(saved[3]), saved[4], swapped(g), to[0], to[1], to[2], wide);
+                                       swapped(result), saved[4], swapped(g), to[0], to[1], to[2], wide);
         });
         return out;
     }

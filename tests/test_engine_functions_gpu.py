@@ -118,3 +118,12 @@ def test_lengths_may_change_between_forward_and_backward(cp):
     call.lengths.fill_(5)
     for a, b in zip(torch.autograd.grad(out, t, torch.ones_like(out)), want):
         assert torch.equal(a, b)
+
+
+def test_a_result_at_128_may_be_changed_in_place(cp):
+    """... before the backward, as the composition's, which does not keep it."""
+    t, call, _ = attention_at_128()
+    want = torch.autograd.grad(call(*t) * 3, t, torch.ones_like(t[0]))
+    out = call(*t).mul_(3)
+    for a, b in zip(torch.autograd.grad(out, t, torch.ones_like(out)), want):
+        assert torch.equal(a, b)
