@@ -443,7 +443,9 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
             torch::autograd::impl::set_version_counter(version, torch::autograd::impl::version_counter(out));
             ctx->saved_data["version"] = version;
             ctx->saved_data["unchanged"] = (int64_t)out._version();
-            ctx->save_for_backward({q, k, v, out.variable_data(), den});
+            // (queries and keys that nothing is derived for: the composition keeps their features, not them)
+            auto own = [](const Tensor &t) { return t.requires_grad() ? t : t.clone(); };
+            ctx->save_for_backward({own(q), own(k), v, out.variable_data(), den});
         } else {
             ctx->save_for_backward({q, k, v, out, den});
         }

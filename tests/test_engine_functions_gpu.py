@@ -127,3 +127,14 @@ def test_a_result_at_128_may_be_changed_in_place(cp):
     out = call(*t).mul_(3)
     for a, b in zip(torch.autograd.grad(out, t, torch.ones_like(out)), want):
         assert torch.equal(a, b)
+
+
+def test_inputs_at_128_without_a_gradient_may_change(cp):
+    """Queries and keys that need no gradient are not watched for changes: the composition keeps their
+    features."""
+    (q, k, v), call, want = attention_at_128()
+    q, k = q.detach().clone(), k.detach().clone()
+    out = call(q, k, v)
+    assert in_engine(out)
+    q.zero_(), k.zero_()
+    assert torch.equal(torch.autograd.grad(out, v, torch.ones_like(out))[0], want[2])
