@@ -121,6 +121,28 @@ def causal_linear(Q, K, V):
     return _CausalLinearNLH.apply(Q, K, V)
 
 
+def _composed(Q, K, values, eps):
+    """Product and normaliser on features (keys masked), as operator calls."""
+    # q_l . cumsum(k)_l  ==  sum_{j<=l} (q_l . k_j) * 1
+    N, L, H, _ = Q.shape
+    denominator = causal_linear(Q, K, _ones_column(N, L, H, Q.device))[..., 0]
+    Z = 1 / (denominator + eps)
+    V = causal_linear(Q, K, values)
+    return V * Z[:, :, :, None]
+
+
+def composed_gradients(queries, keys, values, lengths, eps, grad_out, needed):
+    """Gradients of the composition with the graph behind them that autograd has for it: that of its
+    element-wise parts (the product's own gradients have none).  None where not ``needed``.  The fused
+    backward at rows of 128 calls this when its results are to be differentiated again."""
+    with torch.enable_grad():
+        mask = LengthMask(lengths, max_len=queries.shape[1]).float_matrix
+        out = _composed(_elu_plus_one(queries), _elu_plus_one(keys) * mask[:, :, None, None], values, eps)
+        inputs = [t for t, need in zip((queries, keys, values), needed) if need]
+        grads = iter(torch.autograd.grad(out, inputs, grad_out, create_graph=True))
+    return [next(grads) if need else None for need in needed]
+
+
 class CausalLinearAttention(Module):
     """Causally masked attention with feature maps in O(L D^2) (reference ``:27-104``).
 
@@ -200,9 +222,4 @@ class CausalLinearAttention(Module):
         K = self.feature_map.forward_keys(keys)
         K = K * key_lengths.float_matrix[:, :, None, None]
         K, values = self._make_sizes_compatible(Q, K, values)
-        # q_l . cumsum(k)_l  ==  sum_{j<=l} (q_l . k_j) * 1
-        N, L, H, _ = Q.shape
-        denominator = causal_linear(Q, K, _ones_column(N, L, H, Q.device))[..., 0]
-        Z = 1 / (denominator + self.eps)
-        V = causal_linear(Q, K, values)
-        return V * Z[:, :, :, None]
+        return _composed(Q, K, values, self.eps)

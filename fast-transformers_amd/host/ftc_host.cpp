@@ -459,6 +459,21 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
         const Tensor lengths = ctx->saved_data["lengths"].toTensor();
         variable_list out(5);
         OptTensor to[3];
+        if (wide_rows(saved[0], saved[2]) && at::GradMode::is_enabled()) {
+            // (the caller means to differentiate again: the composition's gradients, whose element-wise parts
+            // can be)
+            from_engine([&] {
+                const py::tuple needed = py::make_tuple(ctx->needs_input_grad(0), ctx->needs_input_grad(1),
+                                                        ctx->needs_input_grad(2));
+                const auto composed = py::module_::import("fast_transformers_amd.attention.causal_linear_attention")
+                                          .attr("composed_gradients")(saved[0], saved[1], saved[2], lengths,
+                                                                      ctx->saved_data["eps"].toDouble(), grads[0], needed)
+                                          .cast<std::vector<OptTensor>>();
+                for (int i = 0; i < 3; i++)
+                    if (composed[i]) out[i] = *composed[i];
+            });
+            return out;
+        }
         for (int i = 0; i < 3; i++)
             if (ctx->needs_input_grad(i)) out[i] = at::empty_like(saved[i]), to[i] = swapped(out[i]);
         from_engine([&] {

@@ -138,3 +138,29 @@ def test_inputs_at_128_without_a_gradient_may_change(cp):
     assert in_engine(out)
     q.zero_(), k.zero_()
     assert torch.equal(torch.autograd.grad(out, v, torch.ones_like(out))[0], want[2])
+
+
+@pytest.mark.parametrize("need", [(1, 1, 1), (0, 1, 0)], ids=str)
+def test_first_derivatives_at_128_are_differentiable_as_the_compositions(cp, need):
+    """create_graph: the composition's element-wise parts can be differentiated again (its products
+    cannot), and a gradient that takes part in them."""
+    inputs, call, _ = attention_at_128()
+    results = []
+    for composed in (False, True):
+        t = [x.detach().clone().requires_grad_(bool(n)) for x, n in zip(inputs, need)]
+        wanted = [x for x in t if x.requires_grad]
+        # (a call with hooks on its saved tensors is composed)
+        same = (lambda x: x) if composed else None
+        with torch.autograd.graph.saved_tensors_hooks(same, same) if composed else torch.enable_grad():
+            out = call(*t)
+            assert in_engine(out) != composed
+            first = torch.autograd.grad(out.square().sum(), wanted, create_graph=True)
+            second = torch.autograd.grad(sum(f.square().sum() for f in first), wanted, allow_unused=True)
+        assert [f.requires_grad for f in first] == [x is not t[2] for x in wanted]
+        results.append(first + second)
+    for a, b in zip(*results):
+        if a is None or b is None:
+            assert a is b
+            continue
+        # (both sides fp32, the last operations the same: what the two forwards differ by)
+        assert ((a - b).norm() / b.norm()).item() <= 5e-6
