@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstdlib>
 #include <map>
 #include <mutex>
@@ -503,7 +504,8 @@ py::object attention_module(py::handle queries, py::handle keys, py::handle valu
         lengths.scalar_type() != at::kLong || !lengths.is_contiguous() || lengths.requires_grad())
         return py::none();
     if (wide_rows(*q, *v)) {  // (what the composition would broadcast or refuse is left to it)
-        if (lengths.dim() != 1 || lengths.size(0) != q->size(0) || mask_length != q->size(1)) return py::none();
+        if (lengths.dim() != 1 || lengths.size(0) != q->size(0) || mask_length != q->size(1) || std::isnan(eps))
+            return py::none();
         for (const Tensor *t : {q, k, v})
             if (!reads_in_place(*t) || t->size(0) != q->size(0) || t->size(2) != q->size(2)) return py::none();
         if (ftc_causal_linear_attention_wide_workspace_bytes(q->size(0), q->size(2), q->size(1), q->size(3), v->size(3),

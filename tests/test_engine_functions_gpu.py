@@ -19,12 +19,12 @@ def operator(cp, dtype, seed=0):
     return [torch.rand(2, 3, 70, w, device="cuda", generator=gen).to(dtype) for w in (64, 64, 32)]
 
 
-def attention(seed=0, widths=(64, 64, 32)):
+def attention(seed=0, widths=(64, 64, 32), **kw):
     from fast_transformers_amd.attention import CausalLinearAttention
     from fast_transformers_amd.masking import LengthMask, TriangularCausalMask
     gen = torch.Generator(device="cuda").manual_seed(seed)
     lengths = LengthMask(torch.tensor([70, 33], device="cuda"), max_len=70)
-    module, mask = CausalLinearAttention(widths[0]), TriangularCausalMask(70, device="cuda")
+    module, mask = CausalLinearAttention(widths[0], **kw), TriangularCausalMask(70, device="cuda")
     inputs = [torch.randn(2, 70, 3, w, device="cuda", generator=gen) for w in widths]
     call = lambda *t: module(*t, mask, lengths, lengths)
     call.lengths = lengths.lengths
@@ -164,3 +164,9 @@ def test_first_derivatives_at_128_are_differentiable_as_the_compositions(cp, nee
             continue
         # (both sides fp32, the last operations the same: what the two forwards differ by)
         assert ((a - b).norm() / b.norm()).item() <= 5e-6
+
+
+def test_an_eps_at_128_that_is_not_a_number(cp):
+    """... makes every row one that is not, as in the composition; the fused kernels refuse it."""
+    inputs, call = attention(widths=(128, 128, 128), eps=float("nan"))
+    assert torch.isnan(call(*inputs)).all()
