@@ -70,6 +70,22 @@ def _elu_plus_one(x):
     return torch.nn.functional.elu(x) + 1
 
 
+def _is_elu_plus_one(fm):
+    """Whether a feature map is elu(x) + 1 and nothing else: no subclass, object or hook that changes what
+    its methods do."""
+    if getattr(fm, "activation_function", None) is not _elu_plus_one:
+        return False
+    cls = type(fm)
+    if cls is not ActivationFunctionFeatureMap and not (
+            issubclass(cls, ActivationFunctionFeatureMap)
+            and all(getattr(cls, m) is getattr(ActivationFunctionFeatureMap, m) for m in _MAP_METHODS)):
+        return False
+    own = fm.__dict__
+    return not (own["_forward_hooks"] or own["_forward_pre_hooks"] or not _MAP_METHODS.isdisjoint(own))
+
+
+_MAP_METHODS = frozenset(("new_feature_map", "forward_queries", "forward_keys", "forward", "__call__"))
+
 # phi(x) = elu(x) + 1 as a feature-map factory (``feature_maps/base.py:71-73``)
 elu_feature_map = ActivationFunctionFeatureMap.factory(_elu_plus_one)
 
@@ -181,9 +197,7 @@ class CausalLinearAttention(Module):
         normaliser) when a fused kernel covers the sizes -- with its own backward (one
         element-wise pass, the three gradient scans, one prefix-sum pass) when something has
         to be differentiated; None otherwise."""
-        fm = self.feature_map
-        if not (isinstance(fm, ActivationFunctionFeatureMap)
-                and fm.activation_function is _elu_plus_one):
+        if not _is_elu_plus_one(self.feature_map):
             return None
         lengths = getattr(key_lengths, "lengths", None)
         if not torch.compiler.is_compiling() and torch.cuda.is_initialized() and _as_defined == (

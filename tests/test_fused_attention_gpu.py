@@ -355,6 +355,33 @@ def test_module_takes_the_fused_path_and_agrees_with_the_composition(lib):
     gate(y_fused.cpu(), q.cpu(), k.cpu(), v.cpu(), torch.tensor([700, 301]), module.eps)
 
 
+@pytest.mark.parametrize("E", [64, 128])
+def test_a_feature_map_with_other_methods_is_not_fused(lib, E):
+    """A subclass, a method set on the object or a hook that changes elu(x) + 1: the composition, which
+    calls it."""
+    from fast_transformers_amd import attention, masking
+    from fast_transformers_amd.attention import causal_linear_attention as cla
+    N, L, H = 2, 70, 3
+    q, k, v = (t.cuda() for t in inputs(N, L, H, E, E, seed=12))
+    full, mask = masking.LengthMask(torch.full((N,), L).cuda(), max_len=L), masking.TriangularCausalMask(L, device="cuda")
+
+    class Doubled(cla.ActivationFunctionFeatureMap):
+        def forward_keys(self, x):
+            return self(2 * x)
+    subclass = attention.CausalLinearAttention(E, feature_map=Doubled.factory(cla._elu_plus_one))
+    method, hook = attention.CausalLinearAttention(E), attention.CausalLinearAttention(E)
+    method.feature_map.forward_keys = lambda x: cla._elu_plus_one(2 * x)
+    hook.feature_map.register_forward_hook(lambda _, args, y: y + 1)
+    plain = attention.CausalLinearAttention(E)
+    with torch.no_grad():
+        want = plain(q, 2 * k, v, mask, full, full)
+        for module in (subclass, method):
+            got = module(q, k, v, mask, full, full)
+            assert scale_error(got.permute(0, 2, 1, 3), want.permute(0, 2, 1, 3)) <= 1e-5
+        unhooked = plain(q, k, v, mask, full, full)
+        assert ((hook(q, k, v, mask, full, full) - unhooked).norm() / unhooked.norm()).item() > 1e-2
+
+
 def _dense_attention(q, k, v, lengths, eps):
     """The closed form of the reference's API test (tests/causal_product/test_causal_product.py:
     34-40) with the feature map and the key-length mask of the module, on (N, L, H, X) tensors
