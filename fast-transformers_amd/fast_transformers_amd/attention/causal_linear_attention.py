@@ -62,7 +62,8 @@ class ActivationFunctionFeatureMap(Module):
         return inner
 
 
-_as_defined = (causal_linear_attention_hip, causal_product.causal_linear_attention_backward_hip,
+# (what the engine's function stands for: with any of them replaced, the Python function runs)
+_as_defined = (fused_attention_covers, causal_linear_attention_hip, causal_product.causal_linear_attention_backward_hip,
                CausalLinearAttentionFunction.forward, CausalLinearAttentionFunction.backward)
 
 
@@ -201,7 +202,7 @@ class CausalLinearAttention(Module):
             return None
         lengths = getattr(key_lengths, "lengths", None)
         if not torch.compiler.is_compiling() and torch.cuda.is_initialized() and _as_defined == (
-                causal_linear_attention_hip, causal_product.causal_linear_attention_backward_hip,
+                fused_attention_covers, causal_linear_attention_hip, causal_product.causal_linear_attention_backward_hip,
                 CausalLinearAttentionFunction.forward, CausalLinearAttentionFunction.backward):
             # plain tensors: the same in the C++ engine, which costs the host less and has the
             # kernels for rows of 128 values (watched calls of those keep the composition)

@@ -356,6 +356,21 @@ def test_module_takes_the_fused_path_and_agrees_with_the_composition(lib):
 
 
 @pytest.mark.parametrize("E", [64, 128])
+def test_a_replaced_size_check_composes(lib, E):
+    """A module whose ``fused_attention_covers`` has been replaced (how the composition is measured beside
+    the fused calls) asks the replacement, in training too."""
+    from fast_transformers_amd import attention, masking
+    from fast_transformers_amd.attention import causal_linear_attention as cla
+    N, L, H = 2, 70, 3
+    q, k, v = (t.cuda().requires_grad_(True) for t in inputs(N, L, H, E, E, seed=13))
+    full, mask = masking.LengthMask(torch.full((N,), L).cuda(), max_len=L), masking.TriangularCausalMask(L, device="cuda")
+    module = attention.CausalLinearAttention(E)
+    assert "CausalAttention" in module(q, k, v, mask, full, full).grad_fn.name()
+    with _composition(cla):
+        assert module(q, k, v, mask, full, full).grad_fn.name() == "MulBackward0"
+
+
+@pytest.mark.parametrize("E", [64, 128])
 def test_a_feature_map_with_other_methods_is_not_fused(lib, E):
     """A subclass, a method set on the object or a hook that changes elu(x) + 1: the composition, which
     calls it."""
