@@ -23,6 +23,7 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/SavedTensorHooks.h>
+#include <ATen/record_function.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -397,6 +398,7 @@ struct CausalDot : torch::autograd::Function<CausalDot> {
         return run(q, k, v);
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        RECORD_FUNCTION("CausalDotProductBackward", std::vector<c10::IValue>());
         const variable_list saved = ctx->get_saved_variables();
         variable_list out;
         for (const Tensor &t : saved) out.push_back(at::empty_like(t, at::MemoryFormat::Contiguous));
@@ -409,6 +411,8 @@ struct CausalDot : torch::autograd::Function<CausalDot> {
 py::object dot(py::handle queries, py::handle keys, py::handle values) {
     const Tensor *q = plain(queries), *k = plain(keys), *v = plain(values);
     if (!q || !k || !v || !nothing_watches()) return py::none();
+    // (a profiler's ranges are those of the Python functions)
+    RECORD_FUNCTION("CausalDotProduct", std::vector<c10::IValue>({*q, *k, *v}));
     return py::cast(differentiated({q, k, v}) ? CausalDot::apply(*q, *k, *v) : CausalDot::run(*q, *k, *v));
 }
 
@@ -434,6 +438,7 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
     }
     static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v,
                           const Tensor &lengths, double eps) {
+        RECORD_FUNCTION("CausalLinearAttentionFunction", std::vector<c10::IValue>({q, k, v}));
         const Tensor den = at::empty({q.size(0), q.size(2), q.size(1)}, q.options());
         const Tensor out = run(q, k, v, lengths, eps, den);
         if (wide_rows(q, v)) {
@@ -456,6 +461,7 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
         return out;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        RECORD_FUNCTION("CausalLinearAttentionFunctionBackward", std::vector<c10::IValue>());
         const variable_list saved = ctx->get_saved_variables();
         const Tensor lengths = ctx->saved_data["lengths"].toTensor();
         variable_list out(5);

@@ -170,3 +170,14 @@ def test_an_eps_at_128_that_is_not_a_number(cp):
     """... makes every row one that is not, as in the composition; the fused kernels refuse it."""
     inputs, call = attention(widths=(128, 128, 128), eps=float("nan"))
     assert torch.isnan(call(*inputs)).all()
+
+
+def test_a_profiler_sees_the_functions_by_name(cp):
+    (inputs, call), operands = attention(), operator(cp, torch.float32)
+    for f, t, name in ((call, inputs, "CausalLinearAttentionFunction"), (cp.causal_dot_product, operands, "CausalDotProduct")):
+        t = [x.clone().requires_grad_(True) for x in t]
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+            out = f(*t)
+            out.sum().backward()
+        names = [event.name for event in prof.events()]
+        assert in_engine(out) and names.count(name) == 1 and names.count(name + "Backward") == 1
