@@ -298,9 +298,9 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #ifdef FTC_TIMELINE
     // tuning aid: 32 time stamps per workgroup behind the pointer that the host passes in
     // p.key_len (FTC_STAMP_PTR), written by lane 0 of consumer 0 (0 .. 15) and of producer 0
-    // (16 .. 31) in chunk 4
+    // (16 .. 31) in chunk 4 (NORM: that is the caller's key lengths, and nothing is stamped)
     typedef __attribute__((address_space(1))) uint64_t gu64;
-    const bool stamp_on = p.key_len != nullptr && w == 0 && lane == 0;
+    const bool stamp_on = !NORM && p.key_len != nullptr && w == 0 && lane == 0;
     gu64 *const stamp_base = (gu64 *)p.key_len + blockIdx.x * 32 + (producer ? 16 : 0);
 #endif
     FTC_STAMP(14);  // workgroup under way
