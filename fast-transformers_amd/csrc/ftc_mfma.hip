@@ -331,7 +331,7 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
 
 // Launches of bf16 rows that the rules above leave to the kernels that split L: on the chain-parallel
 // kernel as well (three pieces for the state and fp32 rows, bf16 rows multiplied as they are,
-// scan_mfma_kernel_tp), in whichever is estimated shorter of whole or cut chains and an exchange of
+// scan_tp_bf16_kernel), in whichever is estimated shorter of whole or cut chains and an exchange of
 // segment sums.  A chunk takes a workgroup 0.63 us (a single scan, a state of up to 64 rows), 0.79 (the
 // scans of a backward call), 1.07 and 1.38 (wider states), a first pass over it about 0.7 of that, the
 // exchange 14 us and half a microsecond for every segment up to 16.  Measured over 1 to 1024 chains of
@@ -498,13 +498,10 @@ void tp_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *n
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
 }
-// (mixed rows: as_before says whether the rules above have taken the launch)
-void mixed_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int mixed, int *nseg, int *seg_chunks,
-                bool *as_before) {
+void mixed_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int mixed, int *nseg, int *seg_chunks) {
     *nseg = *seg_chunks = 0;
     if (D <= 64) tp_plan(D, F, chains, nscans, L, nseg, seg_chunks, false, mixed);
-    *as_before = *nseg > 0;
-    if (*as_before) return;
+    if (*nseg > 0) return;
     static thread_local PlanMemo<TpPlan> memo;
     const int64_t key[8] = {D, F, chains, nscans, L, 0, 0, 0};
     const TpPlan pl = memo.get(key, [&]() {
@@ -680,10 +677,9 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     if ((L + 2 * kChunk) * std::max<int64_t>(widest_stride, std::max(D, F)) * 4 >= 0x7fffffffLL)
         return false;
     int nseg = 0, seg_chunks = 0;
-    bool as_before;
     const int64_t chains = std::max<int64_t>(1, N * H);
     if (mixed)
-        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks, &as_before);
+        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks);
     else if (odd && forced)
         tp_plan(D, 64, chains, (int)column_blocks(scans, nscans), L, &nseg, &seg_chunks, forced, 0, odd);
     else
@@ -696,8 +692,7 @@ int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D
     int64_t bytes = 0;
     for (const int mixed : {kMixedRows, kMixedGradValues}) {
         int nseg = 0, seg_chunks = 0;
-        bool as_before;
-        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks, &as_before);
+        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks);
         if (seg_chunks > 0)
             bytes = std::max(bytes, tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D));
     }
@@ -799,7 +794,6 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for this shape or layout");
     const int64_t chains = std::max<int64_t>(1, N * H);
     int tpx_nseg = 0, tpx_seg_chunks = 0, tp_nseg = 0;
-    bool as_before = true;
     int64_t widest = 0;
     for (int64_t l : {scans[0].a.stride_l, scans[0].b.stride_l, scans[0].v.stride_l, scans[0].out.stride_l})
         widest = std::max(widest, l);
@@ -822,7 +816,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         for (int i = 0; i < nscans; i++)
             if (combo_of(scans[i]) != kFFFF && any_bf16 == 0) any_bf16 = kMixedRows;
         if (any_bf16)
-            mixed_plan(D, F, chains, nscans, L, any_bf16, &tpx_nseg, &tpx_seg_chunks, &as_before);
+            mixed_plan(D, F, chains, nscans, L, any_bf16, &tpx_nseg, &tpx_seg_chunks);
         else if (odd && forced)
             tp_plan(D, 64, chains, (int)blocks, L, &tpx_nseg, &tpx_seg_chunks, forced, 0, odd);
         else
@@ -933,7 +927,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     bool dma = D <= 64 && combo == kFFFF;
     if (tuning().dma >= 0) dma = dma && tuning().dma != 0;  // tuning aid
     note_kernel(fused_tp ? (tpx_seg_chunks > 0 ? "scan_tp_kernel<NORM> (exchange)" : "scan_tp_kernel<NORM>")
-                : rows_as_they_are && !as_before ? (tpx_seg_chunks > 0 ? "scan_mfma_kernel_tp (exchange)" : "scan_mfma_kernel_tp")
+                : rows_as_they_are ? (tpx_seg_chunks > 0 ? "scan_tp_bf16_kernel (exchange)" : "scan_tp_bf16_kernel")
                 : tp ? (half_pieces ? (tpx_seg_chunks > 0 ? "scan_tph_kernel (exchange)" : "scan_tph_kernel")
                                   : (tpx_seg_chunks > 0 ? "scan_tp_kernel (exchange)" : "scan_tp_kernel"))
                 : wg ? (fused ? "scan_wg_kernel<NORM>" : "scan_wg_kernel")
@@ -956,7 +950,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         if (fused)
             launch_scan_tp_norm(workspace, args, stream);
         else if (mixed)
-            launch_scan_tp_mixed(workspace, args, as_before, stream);
+            launch_scan_tp_mixed(workspace, args, stream);
         else if (half_pieces)
             launch_scan_tph(workspace, args, odd, stream);
         else

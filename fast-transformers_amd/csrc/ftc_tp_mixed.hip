@@ -6,8 +6,6 @@
 // matrix instructions per consumer where fp32 rows take 72, and its producers copy instead of cutting:
 // 0.63 us a chunk against 1.1 on the two scaled fp16 pieces that such rows had before, which memory
 // then bounds (256 chains, L=4096, forward 152 -> 131 us, 5.3 TB/s; 80 chains, L=1000, backward 42 -> 34).
-// The launches that the fp16-piece kernel took keep its name (scan_tph_kernel_bf16), those that the
-// kernels which split L took have one of their own.
 #include "ftc_tp_kernel.h"
 
 namespace ftc {
@@ -36,34 +34,29 @@ __device__ __forceinline__ void scan_mixed(uint32_t *__restrict__ ws_ptr, const 
             scan_tp_body<ND, KS2, false, 1, 1, 3, bf16_t>(ws_ptr, p, which, chain, pieces, pt, nullptr, &order_sh);
     }
 }
-template <int KS, bool FORWARD>
-__global__ __launch_bounds__(512, 2) void scan_tph_kernel_bf16(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
-    scan_mixed<1, KS, FORWARD>(ws_ptr, p);
-}
 template <int ND, int KS2, bool FORWARD>
-__global__ __launch_bounds__(512, 2) void scan_mfma_kernel_tp(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
+__global__ __launch_bounds__(512, 2) void scan_tp_bf16_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     scan_mixed<ND, KS2, FORWARD>(ws_ptr, p);
 }
 
 template <bool FORWARD>
-void launch(void *ws, const ScanArgs &args, bool as_tph, hipStream_t stream) {
+void launch(void *ws, const ScanArgs &args, hipStream_t stream) {
     const dim3 grid((unsigned)args.total_waves), block(512);
-#define FTC_LAUNCH(KERNEL) hipLaunchKernelGGL((KERNEL), grid, block, 0, stream, (uint32_t *)ws, args)
-    if (as_tph && args.tp_d <= 32) FTC_LAUNCH((scan_tph_kernel_bf16<1, FORWARD>));
-    else if (as_tph) FTC_LAUNCH((scan_tph_kernel_bf16<2, FORWARD>));
-    else if (args.tp_d <= 32) FTC_LAUNCH((scan_mfma_kernel_tp<1, 1, FORWARD>));
-    else if (args.tp_d <= 64) FTC_LAUNCH((scan_mfma_kernel_tp<1, 2, FORWARD>));
-    else if (args.tp_d <= 96) FTC_LAUNCH((scan_mfma_kernel_tp<2, 1, FORWARD>));
-    else FTC_LAUNCH((scan_mfma_kernel_tp<2, 2, FORWARD>));
+#define FTC_LAUNCH(ND, KS2) \
+    hipLaunchKernelGGL((scan_tp_bf16_kernel<ND, KS2, FORWARD>), grid, block, 0, stream, (uint32_t *)ws, args)
+    if (args.tp_d <= 32) FTC_LAUNCH(1, 1);
+    else if (args.tp_d <= 64) FTC_LAUNCH(1, 2);
+    else if (args.tp_d <= 96) FTC_LAUNCH(2, 1);
+    else FTC_LAUNCH(2, 2);
 #undef FTC_LAUNCH
 }
 }  // namespace
 
-void launch_scan_tp_mixed(void *ws, const ScanArgs &args, bool as_tph, hipStream_t stream) {
+void launch_scan_tp_mixed(void *ws, const ScanArgs &args, hipStream_t stream) {
     if (args.scan[0].pad & kRowsBf16Out)
-        launch<false>(ws, args, as_tph, stream);
+        launch<false>(ws, args, stream);
     else
-        launch<true>(ws, args, as_tph, stream);
+        launch<true>(ws, args, stream);
 }
 
 }  // namespace mfma

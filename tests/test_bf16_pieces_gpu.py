@@ -1,4 +1,4 @@
-"""bf16 rows on the chain-parallel kernel that multiplies them as they are (scan_mfma_kernel_tp):
+"""bf16 rows on the chain-parallel kernel that multiplies them as they are (scan_tp_bf16_kernel):
 states of up to 128 rows, few and many chains, whole, cut and with an exchange of segment sums,
 against float64 as tests/test_bf16_rows_gpu.py does."""
 import ctypes
@@ -12,7 +12,7 @@ from test_bf16_rows_gpu import _check_gradients, _inputs, _last_kernel
 
 pytestmark = pytest.mark.gpu
 
-OURS = (b"scan_mfma_kernel_tp", b"scan_mfma_kernel_tp (exchange)")
+OURS = (b"scan_tp_bf16_kernel", b"scan_tp_bf16_kernel (exchange)")
 
 
 @pytest.fixture(scope="module")
@@ -55,7 +55,7 @@ def test_forward_and_backward(cp, shape):
     cp.causal_dot_backward_hip(q, k, v, G.cuda(), *together)
     used.add(_last_kernel())
     _check_gradients(str(shape), together, Qb, Kb, Vb, G)
-    assert used & set(OURS + (b"scan_tph_kernel", b"scan_tph_kernel (exchange)")), used
+    assert used & set(OURS), used
 
 
 @pytest.mark.parametrize("shape", [(2, 8, 700, 128, 128), (1, 3, 4500, 64, 64), (3, 8, 150, 96, 40)], ids=str)
@@ -128,7 +128,7 @@ def test_without_room_for_an_exchange(cp):
     tensors = [t.cuda() for t in _inputs(N, H, L, E, M, 95)]
     want, got = ([torch.full_like(t, float("nan")) for t in tensors[:3]] for _ in range(2))
     cp.causal_dot_backward_hip(*tensors, *want)
-    assert _last_kernel() == b"scan_mfma_kernel_tp (exchange)"
+    assert _last_kernel() == b"scan_tp_bf16_kernel (exchange)"
     full = lib.ftc_causal_dot_backward_workspace_bytes(N, H, L, E, M, _native.FTC_BF16)
     ws = torch.zeros(full, dtype=torch.uint8, device="cuda")
     d = [_native.describe(t) for t in tensors + got]

@@ -1,10 +1,9 @@
-"""bf16 rows on the chain-parallel kernel's fp16 path (its form that takes rows of either
-element type, scan by scan): the three scans of a backward call over up to 128 chains, a
-forward over at least 256 chains, and widths that the other matrix-core kernels would only
-take as padded copies.
+"""bf16 rows on the chain-parallel kernel that multiplies them as they are: the three scans of a
+backward call over up to 128 chains, a forward over at least 256 chains, and widths that the other
+matrix-core kernels would only take as padded copies.
 
-bf16 values are exact in one fp16 piece after scaling, so the arithmetic is that of fp32 rows
-whose low pieces are zero: the fp32 product must be as close to float64 as the CPU checker's
+bf16 values are one piece each, and the state, the chunk product and the fp32 gradient are in three, so
+the arithmetic is that of fp32 rows whose low pieces are zero: the fp32 product must be as close to float64 as the CPU checker's
 (on the same bf16-rounded inputs), and a bf16 gradient must be the float64 gradient rounded to
 bf16, give or take one unit in the last place where the fp32 value lies near a rounding
 boundary."""
@@ -16,7 +15,7 @@ from parity import scale_error
 
 pytestmark = pytest.mark.gpu
 
-KERNELS = (b"scan_tph_kernel", b"scan_tph_kernel (exchange)")
+KERNELS = (b"scan_tp_bf16_kernel", b"scan_tp_bf16_kernel (exchange)")
 
 
 @pytest.fixture(scope="module")
@@ -127,8 +126,7 @@ def test_bf16_rows_in_interleaved_heads_storage(cp):
 
 
 def test_bf16_rows_far_from_one(cp):
-    """Operands many orders of magnitude away from one, and values that grow along the chain
-    (the running ceilings of b and v rise, the state is rescaled)."""
+    """Operands many orders of magnitude away from one, and values that grow along the chain."""
     N, H, L, E, M = 6, 8, 300, 64, 64
     Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=52)
     ramp = torch.exp2(torch.linspace(-20, 12, L))[None, None, :, None]

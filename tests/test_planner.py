@@ -17,6 +17,11 @@ def lines(q, v, **kw):
     return [l for l in _native.plan(q, v, **kw).split("\n") if l]
 
 
+def kernel(line):
+    """The launch's kernel, with its form: "scan_tp_bf16_kernel (exchange)"."""
+    return line.split(":")[0]
+
+
 def field(line, pattern):
     m = re.search(pattern, line)
     assert m, (pattern, line)
@@ -92,40 +97,31 @@ def test_what_the_chain_parallel_kernel_leaves_to_the_others():
     assert lines((1, 3, 500, 128), (1, 3, 500, 128))[0].startswith("scan_mfma_kernel")
     assert lines((1, 3, 500, 128), (1, 3, 500, 128), backward=True)[0].startswith("scan_tp_kernel: 3 scans")
     assert lines((1, 8, 640, 64), (1, 8, 640, 64))[0].startswith("scan_tph_kernel: 1 scan")
-    # bf16 rows: a single scan stays with the kernels that multiply such rows as they are
-    # until the chain-parallel kernel has workgroups for about half of the CUs, and wherever
-    # it would need an exchange; the three scans of a backward call, and widths that those
-    # kernels would only take as padded copies, go to the chain-parallel kernel
-    bf16 = dict(dtype=_native.FTC_BF16)
-    assert lines((4, 8, 1000, 64), (4, 8, 1000, 64), **bf16)[0].startswith("scan_mfma_kernel")
-    assert lines((1, 8, 2048, 64), (1, 8, 2048, 64), **bf16)[0].startswith("scan_mfma_kernel")
-    assert lines((1, 8, 2048, 64), (1, 8, 2048, 64), backward=True, **bf16)[0] \
-        .startswith("scan_tph_kernel (exchange): 3 scans")
-    whole = lines((1, 64, 16384, 64), (1, 64, 16384, 64), backward=True, **bf16)[0]
-    assert whole.startswith("scan_tph_kernel: 3 scans") and "1 segment of 16384 rows" in whole
-    assert lines((1, 43, 16384, 64), (1, 43, 16384, 64), backward=True, **bf16)[0].startswith("scan_mfma_kernel")
-    assert lines((10, 8, 1000, 64), (10, 8, 1000, 64), **bf16)[0].startswith("scan_mfma_kernel")
-    assert lines((14, 8, 1000, 64), (14, 8, 1000, 64), **bf16)[0].startswith("scan_tph_kernel:")
-    assert lines((16, 8, 1000, 64), (16, 8, 1000, 64), **bf16)[0].startswith("scan_tph_kernel:")
-    assert lines((16, 8, 4096, 64), (16, 8, 4096, 64), **bf16)[0].startswith("scan_mfma_kernel")
-    assert lines((24, 8, 4096, 64), (24, 8, 4096, 64), **bf16)[0].startswith("scan_tph_kernel:")
-    assert lines((16, 16, 1000, 64), (16, 16, 1000, 64), **bf16)[0].startswith("scan_tph_kernel:")
-    # config 5: the dV scan (fp32 values, a state of 32 rows) walks its chains whole, however
-    # long; the forward and the scans with a state of 128 rows stay where they were
-    cfg5 = lines((4, 32, 16384, 32), (4, 32, 16384, 128), backward=True, **bf16)
-    assert len(cfg5) == 3 and sum(l.startswith("scan_mfma_kernel") for l in cfg5) == 2
-    dv = [l for l in cfg5 if l.startswith("scan_tph_kernel:")]
-    assert len(dv) == 1 and "state 32 x 128" in dv[0] and "1 segment of 16384 rows" in dv[0]
-    assert lines((4, 32, 16384, 32), (4, 32, 16384, 128), **bf16)[0].startswith("scan_mfma_kernel")
-    assert all(l.startswith("scan_mfma_kernel")
-               for l in lines((2, 32, 16384, 32), (2, 32, 16384, 128), backward=True, **bf16))
-    assert lines((10, 8, 1000, 64), (10, 8, 1000, 64), backward=True, **bf16)[0] \
-        .startswith("scan_tph_kernel: 3 scans")
-    assert lines((6, 8, 257, 48), (6, 8, 257, 40), **bf16)[0].startswith("scan_tph_kernel:")
-    assert lines((8, 8, 130, 20), (8, 8, 130, 20), **bf16)[0].startswith("scan_tph_kernel:")
-    # (rows of 128 values: no fp16-piece form, and the bf16-piece form takes fp32 rows only)
-    assert lines((10, 8, 1000, 128), (10, 8, 1000, 128), backward=True, **bf16)[0] \
-        .startswith("scan_mfma_kernel")
+    # bf16 rows: the chain-parallel kernel that multiplies them as they are, on whole and cut chains and with
+    # an exchange, but for single scans of few wide chains and the shapes with 32 rows or columns below
+    def bf16(N, H, L, E, M, backward=False):
+        return lines((N, H, L, E), (N, H, L, M), backward=backward, dtype=_native.FTC_BF16)
+    tp, tpx = "scan_tp_bf16_kernel", "scan_tp_bf16_kernel (exchange)"
+    for N, H, L in ((4, 8, 1000), (10, 8, 1000), (14, 8, 1000), (16, 8, 1000), (16, 16, 1000), (16, 8, 4096),
+                    (24, 8, 4096)):
+        assert kernel(bf16(N, H, L, 64, 64)[0]) == tp, (N, H, L)
+    assert kernel(bf16(1, 8, 2048, 64, 64)[0]) == tpx
+    assert bf16(1, 8, 2048, 64, 64, True)[0].startswith(tpx + ": 3 scans")
+    whole = bf16(1, 64, 16384, 64, 64, True)[0]
+    assert whole.startswith(tp + ": 3 scans") and "1 segment of 16384 rows" in whole
+    assert bf16(10, 8, 1000, 64, 64, True)[0].startswith(tp + ": 3 scans")
+    # narrow keys, wide values: the dV scan (fp32 values, a state of 32 rows) walks its chains whole, however
+    # long; the forward and the scans with a state of 128 rows are left to the kernels that split L
+    wide_values = bf16(4, 32, 16384, 32, 128, True)
+    assert [kernel(l) for l in wide_values] == [tp, "scan_mfma_kernel", "scan_mfma_kernel"]
+    assert "state 32 x 128" in wide_values[0] and "1 segment of 16384 rows" in wide_values[0]
+    assert kernel(bf16(4, 32, 16384, 32, 128)[0]) == "scan_mfma_kernel"
+    assert {kernel(l) for l in bf16(2, 32, 16384, 32, 128, True)} == {"scan_mfma_kernel"}
+    # widths that the kernels that split L would only take as padded copies
+    assert kernel(bf16(6, 8, 257, 48, 40)[0]) == tp
+    assert kernel(bf16(8, 8, 130, 20, 20)[0]) == tp
+    # rows of 128 values
+    assert kernel(bf16(10, 8, 1000, 128, 128, True)[0]) == tp
     # odd widths: zero-padded dense copies for the matrix-core kernels when there are enough
     # rows to pay for the extra launches; states of more than 128 rows stay generic
     # (queries and keys are copied, the values and the product stay where they are; in the
@@ -245,9 +241,8 @@ def test_wide_states_on_the_chain_parallel_kernel():
     assert lines((1, 16, 2048, 32), (1, 16, 2048, 96))[0].startswith("scan_tph_kernel:")
     # ... and long ones where whole chains fill three quarters of the CUs
     assert lines((1, 128, 16384, 32), (1, 128, 16384, 128))[0].startswith("scan_tph_kernel: 1 scan")
-    # bf16 rows and widths that are not multiples of 4 go the other ways
-    assert lines((8, 16, 4096, 128), (8, 16, 4096, 128), dtype=_native.FTC_BF16)[0] \
-        .startswith("scan_mfma_kernel")
+    # bf16 rows have a kernel of their own, widths that are not multiples of 4 go another way
+    assert kernel(lines((8, 16, 4096, 128), (8, 16, 4096, 128), dtype=_native.FTC_BF16)[0]) == "scan_tp_bf16_kernel"
     assert lines((8, 16, 4096, 98), (8, 16, 4096, 128))[0].startswith("pad_rows_kernel")
 
 
