@@ -1,6 +1,7 @@
 // Host side of the MFMA scan (kernel: ftc_mfma_kernel.h): which scans qualify, how L is cut
 // into segments, workspace size, and the launch.
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 
@@ -129,7 +130,7 @@ int tp_segment_starts(int64_t chunks, int nseg, int32_t *start) {
 // chain is cut into as many equal segments as fill the GPU (one workgroup each); a workgroup
 // walks its own chunks twice, first for their state alone.  Returns the number of chunks per
 // segment (0: not this way) and the number of segments in *nseg.
-int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg, bool keep_two = false) {
+int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg) {
     const int64_t total_chunks = (L + kChunk - 1) / kChunk;
     *nseg = 0;
     if (tuning().tpx == 0) return 0;  // tuning aid
@@ -180,8 +181,7 @@ int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg, bool ke
     // exchange wins again (backward of 24 chains: 83 against 86; forward of 64: 73 against 88).
     // Wider states the same (64 x 128 forward, 64 chains, L=4096: 116 against 104; 128 x 128
     // backward of 16 chains: 204 against 186).
-    // (`keep_two`: the caller compares with other kernels, not with cut chains)
-    if (!force && !keep_two && want == 2 && total_chunks <= 128) return 0;
+    if (!force && want == 2 && total_chunks <= 128) return 0;
     // segments of at least four chunks (one or two chains, L=4096: 32 segments 21.5 us, 16: 25.1)
     want = std::min<int64_t>(want, total_chunks / 4);
     if (tuning().tpx_segs >= 0) want = std::max(1, tuning().tpx_segs);  // tuning aid
@@ -199,29 +199,14 @@ int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg, bool ke
 // The chain-parallel kernel's plan for `nscans` scans of a D x F state over chains x L rows:
 // *seg_chunks > 0: an exchange with *nseg segments of that many chunks; else *nseg > 0: chains
 // cut into *nseg segments that need no exchange; both 0: another kernel takes the launch.
-// `mixed`: rows with bf16 among them (the fp16-piece form of the kernel takes those; the plans
-// are those of fp32 rows where the kernel is used at all).
-// `mixed`: kMixedRows: rows with bf16 among them; kMixedGradValues: a single scan of bf16 a and b
-// whose values are fp32 (the dV scan of a bf16 backward)
-constexpr int kMixedRows = 1, kMixedGradValues = 2;
+// (fp32 rows; those with bf16 among them have a plan of their own, mixed_plan_compute)
 void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg,
-                     int *seg_chunks, bool forced, int mixed, bool odd) {
+                     int *seg_chunks, bool forced, bool odd) {
     *nseg = *seg_chunks = 0;
     if (!tp_widths(D, F, forced, odd)) return;
     const bool wide = D != 64 || F != 64 || forced || odd;
     const bool others = !forced && !odd && mfma_scan_supported_widths(D, F);
     const int64_t units = chains * nscans * tp_fblocks(F);
-    // A single scan over bf16 rows: the kernels that split L multiply such rows as they are,
-    // one matrix instruction per product, and win while this kernel has workgroups for fewer
-    // than half of the CUs (forward, 64 x 64, L=1000, N*H = 80: 32 against 36 us, 96: 33
-    // against 36, 112: 38 against 36, 128: 42 against 37, 192: 53 against 42) or would need
-    // an exchange (N*H = 128, L=4096: 114 against 132 us; L=8192: 208 against 241; without one,
-    // N*H = 192, L=4096: 160 against 140).  The three scans of a backward call are faster
-    // here for up to 128 chains (L=1000, N*H = 80: 50 against 101 us).
-    const bool lone_mixed = mixed && nscans == 1 && others;
-    if (lone_mixed && units < 112) return;
-    // (N*H = 128, L=1024: 35 against 38 us; L=2048: 61 against 54)
-    if (lone_mixed && units < 192 && L > 48 * kChunk) return;
     // Shapes of the other kernels with 32 rows or columns (a workgroup here has half of its
     // matrix work or half of its consumers to spare for them): measured at N=8, H=16, L=4096,
     // forward + backward, 32 x 128 0.62 against 0.80 ms and 128 x 32 0.76 against 0.78 on whole
@@ -236,12 +221,7 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // against 17, L=512: 22 against 17; 128 x 32 forward, 8 chains, L=512: 27 against 20).
     const int64_t brief_chunks = D <= 64 || (F > 32 && nscans >= 2) ? 23 : 8;
     if (narrow && D <= 32 && F <= 32) return;
-    // A single scan over bf16 rows in blocks of 64 output columns reads a and b once per block:
-    // beyond two rounds of workgroups, or one for a state of 32 rows, the kernels that split L
-    // win (64 x 128, 512 chains, L=512: 92 against 58 us, L=2048: 309 against 272; 256 chains:
-    // 149 against 175.  32 x 128, 256 chains, L=1024: 75 against 58; 128 chains: 40 against 40)
-    if (lone_mixed && units > (narrow ? 256 : 512)) return;
-    // ... and so do thousands of chains of one or two chunks with a state of at most 64 x 64,
+    // Thousands of chains of one or two chunks with a state of at most 64 x 64 go to those kernels too,
     // where a workgroup's start costs more than its chunks (8192 chains, L=64: 32 x 128 1.17
     // against 0.60 ms, 20 x 20 0.63 against 0.46 on padded copies), and 32-wide shapes on more
     // than two rounds of workgroups, as for 64 x 64.
@@ -281,37 +261,9 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // element-wise bound 2.8 times as often as the reference's own order, where twice is the bar.
     // (32-wide states included: 32 x 128 forward, 128 chains, L=16384: 553 against 756; 64 x 32
     // backward, 256 chains, L=12000: 1404 against 1825)
-    // ... and the three scans of a backward call over bf16 rows, whose results are rounded to
-    // bf16 anyway, from 192 workgroups on (64 chains, L=16384: 634 against 783 us; 256 chains:
-    // 1783 against 2430; 43 chains: 512 against 483)
-    const bool mixed_backward = mixed == kMixedRows && nscans == 3;
-    const bool walk_long = (!mixed || mixed_backward) && D <= 64 && !(odd && forced) && L > 256 * kChunk &&
-                           L <= 1024 * kChunk &&
-                           units >= (mixed_backward ? 192 : !wide ? 112 : L > 512 * kChunk ? 128 : 192);
-    if (!narrow && !walk_long) *seg_chunks = tp_exchange_segments(units, L, wide, nseg, lone_mixed);
-    if (lone_mixed && units < 256 && *seg_chunks > 0) {
-        *nseg = *seg_chunks = 0;
-        return;
-    }
-    // ... and so do the three scans of a backward call over bf16 rows where the exchange would
-    // have two segments per chain or more than one round of workgroups (32 chains, L=8192: 232
-    // against 201 us, L=16384: 448 against 364; 16 chains, five segments each: 109 against 168
-    // and 194 against 227)
-    if (mixed == kMixedRows && nscans == 3 && *seg_chunks > 0 && units * 3 > 256) {
-        *nseg = *seg_chunks = 0;
-        return;
-    }
-    // The dV scan of a bf16 backward with a state of at most 32 rows and a workgroup for every
-    // CU is walked whole however long the chain: what the kernels that split L read twice there
-    // is the fp32 gradient, the widest operand by far (N=4, H=32, L=16384, 32 x 128: 0.485
-    // against 0.629 ms; the forward of the same shape, whose wide operand is the fp32 result
-    // that either kernel writes once, loses: 0.656 against 0.495).  bf16 results make the
-    // rounding of a long running fp32 state a non-issue.
-    const bool long_chains = walk_long || (mixed == kMixedGradValues && D <= 32 && units == 256);
-    // The three scans of a backward call over bf16 rows stay here for up to six rounds of
-    // workgroups: the kernels that split L, good at many fp32 chains, multiply bf16 rows as they
-    // are but re-read them in a first pass (backward, us, this kernel / those: 256 chains, L=1024:
-    // 116 / 172; 512 chains, L=2048: 471 / 593; 768 chains, L=512: 227 / 196, L=2048: 701 / 732).
+    const bool walk_long = D <= 64 && !(odd && forced) && L > 256 * kChunk && L <= 1024 * kChunk &&
+                           units >= (!wide ? 112 : L > 512 * kChunk ? 128 : 192);
+    if (!narrow && !walk_long) *seg_chunks = tp_exchange_segments(units, L, wide, nseg);
     // fp32 rows, 64 x 64: any number of chains of 16 chunks or more (the fp16-piece kernel walks
     // them faster than the kernels that split L stream them: backward, 256 chains, L=4096: 528
     // against 694 us; 768 chains, L=2048: 784 against 1013; forward, 1536 chains, L=1024: 309
@@ -320,55 +272,99 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // 136 against 146, of 2048 chains 327 against 295; forward of 768 chains 50 against 50, of
     // 1024 chains 65 against 56), two below that (256 chains, L=128: 31 against 27)
     const int64_t chunks = (L + kChunk - 1) / kChunk;
-    const int64_t most_units = mixed == kMixedRows && nscans == 3 ? 1536
-                               : mixed              ? 512
-                               : chunks >= 16       ? INT64_MAX
-                               : chunks >= 8        ? (nscans == 3 ? 2304 : 768)
-                                                    : 512;
+    const int64_t most_units = chunks >= 16  ? INT64_MAX
+                               : chunks >= 8 ? (nscans == 3 ? 2304 : 768)
+                                             : 512;
     if (*seg_chunks == 0)
-        *nseg = tp_kernel_segments(units, L, wide, others, long_chains, narrow, most_units, brief_chunks);
+        *nseg = tp_kernel_segments(units, L, wide, others, walk_long, narrow, most_units, brief_chunks);
 }
 
-// Launches of bf16 rows that the rules above leave to the kernels that split L: on the chain-parallel
-// kernel as well (three pieces for the state and fp32 rows, bf16 rows multiplied as they are,
-// scan_tp_bf16_kernel), in whichever is estimated shorter of whole or cut chains and an exchange of
-// segment sums.  A chunk takes a workgroup 0.63 us (a single scan, a state of up to 64 rows), 0.79 (the
-// scans of a backward call), 1.07 and 1.38 (wider states), a first pass over it about 0.7 of that, the
-// exchange 14 us and half a microsecond for every segment up to 16.  Measured over 1 to 1024 chains of
-// 64 to 16384 positions (us, before / here): 128 x 128 forward, 128 chains, L=4096 366 / 169, backward
-// 1213 / 629; 80 chains, L=1000 68 + 228 / 40 + 107; 4 chains, L=64, backward 28.6 / 8.1; 64 x 64
-// forward, 80 chains, L=1000 26.6 / 19.1, 128 chains, L=4096 114 / 81; 32 x 32 backward, 16 chains, L=256
-// 30 / 8.8.  What stays: more than a thousand chains of a few chunks (64 x 64 forward, 1024 chains, L=64 12.7 /
-// 18.1, L=256 equal; backward, L=128 63 / 79; 64 x 128 forward, 384 chains, L=128 16 / 20), single scans
-// of wide states on a few chains (128 x 128, 1 chain, L=1000 15.9 / 23.7, 4 chains equal; 96 x 96, 24
-// chains, L=2048 36 / 40), and of narrow ones (32 rows or columns) long chains (32 x 128 forward, 48 chains, L=16384 218 / 251), few chains
-// (128 x 32 forward, 4 chains, L=1000 16.0 / 23.8), many chains (32 x 32 backward, 1024 chains, L=1000
-// 216 / 273; 64 x 32 forward, 384 chains, L=128 9.7 / 12.4) and single scans of 32 x 32 (16 chains, L=4096
-// 20.5 / 26.1).
-void mixed_rest_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg,
-                             int *seg_chunks) {
+// Scans with bf16 rows among them: where the kernels that split L, which multiply such rows as they are
+// too, are faster.  Measured over 4860 launches (the widths 32, 64, 96 and 128, forward, dV alone, dQ with
+// dK, all three; 1 to 2048 chains of 64 to 32768 positions), each in whole and cut chains and with
+// exchanges (us, split L / here):
+//   wide: 64 x 64 forward, 1024 chains, L=64 12.3 / 17.9, L=256 32 / 40, but 512 chains, L=512 49 / 35;
+//   backward, 768 chains, L=128 57 / 67, but 384 chains 45 / 36; 128 x 128 forward, 1 chain, L=1000 18 / 21,
+//   but 4 chains, L=2048 47 / 26;
+//   32 rows or columns, several scans: dQ and dK of 32 x 128, 768 chains, L=128 47 / 60, but 256 chains 32 / 21,
+//   128 chains, L=16384 1118 / 897, 48 chains, L=8192 223 / 264; 32 x 32, 96 chains, L=8192 backward 131 / 179;
+//   single ones: 32 x 32, 16 chains, L=4096 17 / 22, 256 chains, L=1000 43 / 30; 128 x 32, 64 chains,
+//   L=4096 66 / 74, 256 chains 236 / 165; 32 x 128 forward, 128 chains, L=8192 262 / 209, 64 chains 141 / 166
+//   and L=16384 277 / 313, where its fp32 rows have to be exchanged.
+bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunks, bool bf16_results) {
+    // (widths that those kernels take as padded copies only)
+    if (!mfma_scan_supported_widths(D, F)) return D <= 64 && F <= 64 && units > (nscans == 1 ? 512 : 1400) && chunks <= 2;
+    const bool single = nscans == 1;
+    // (a last round of workgroups that is nearly empty)
+    const bool uneven = units > 256 && (units + 255) / 256 * 256 * 7 > units * 10;
+    if (D > 32 && F > 32) {
+        if (D > 64 && F > 64) {
+            if (D <= 96 && ((chunks <= 4 && units >= 320) || (chunks <= 8 && units >= 4096) ||
+                            (single && chunks > 48 && units < 128) || (chunks > 256 && units < 192)))
+                return true;
+        } else if (single ? (chunks <= 4 && units >= 768) || (chunks <= 8 && units >= 1024)
+                          : (chunks <= 2 && units >= 1280) || (chunks <= 8 && units >= 2048)) {
+            return true;
+        }
+        return single && D > 64 &&
+               ((units < 16 && chunks > 8 && chunks < (units < 8 ? 256 : 96)) || (units >= 320 && chunks <= 2));
+    }
+    if (!single) {
+        if (D <= 32 && F <= 32) {
+            if (chunks > 128) return units > 48;
+            return chunks <= 64 && units > (chunks <= 4 ? 1024 : chunks <= 8 ? 1100 : 1536);
+        }
+        if (F <= 32 && chunks >= 192 && ((units > 64 && units < 144) || uneven)) return true;
+        if (F <= 32 && chunks > 512) return units > 16;
+        if (chunks > 64) return false;
+        if (F > 64) return units > (chunks <= 8 ? 1024 : 2048);
+        return chunks <= 2 ? units > 512 : chunks <= 8 ? units > 768 : F <= 32 && units > 1024;
+    }
+    if (F > 64) {  // 32 rows
+        if (chunks <= 64) return units > (chunks <= 2 ? 512 : chunks <= 8 ? 768 : 1024);
+        if (chunks < 192) return false;
+        if (bf16_results) return uneven || (units > 32 && units < 160);
+        return units > 512 || uneven || (units > 32 && (chunks > 256 || units < 192));
+    }
+    if (F > 32) {
+        if (chunks <= 24) return units > (chunks <= 4 ? (bf16_results ? 256 : 384) : chunks <= 8 ? 448 : bf16_results ? 512 : INT64_MAX);
+        return chunks >= 48 && chunks <= 256 && units > 4 && units < (chunks <= 72 ? 48 : bf16_results ? 112 : 64);
+    }
+    // 32 columns
+    if (chunks <= 2) return D <= 64 || units > 256;
+    if (chunks <= 8) return units > (chunks > 4 && !bf16_results ? 320 : 256);
+    if (chunks > 12 && uneven) return true;
+    if (D > 64) {
+        if (chunks <= 48) return units < (chunks <= 16 ? 32 : 16) || (bf16_results && units > 512);
+        if (chunks <= 96) return !((units >= 8 && units <= 32) || units >= 112);
+        return !(units <= (bf16_results && chunks > 256 ? 8 : 16) || (units >= 168 && chunks <= 256) ||
+                 (units >= 112 && units <= 144 && chunks <= 128));
+    }
+    if (chunks <= 24) return units > 512;
+    if (chunks <= 48) return units < 48 || (units > 512 && (bf16_results || D <= 32));
+    if (chunks > 256) return true;
+    if (D <= 32) return units < (chunks <= 72 ? 176 : 224) || (bf16_results && units > 512);
+    return units < (chunks <= 96 ? (bf16_results || chunks > 72 ? 112 : 64) : bf16_results ? 176 : 160) || (bf16_results && units > 512);
+}
+
+// The plan of scans with bf16 rows among them on the chain-parallel kernel (three pieces for the state and
+// fp32 rows, bf16 rows multiplied as they are, scan_tp_bf16_kernel): whichever is estimated shorter of
+// whole or cut chains and an exchange of segment sums.  The estimates are fitted to 15650 launches (within
+// 8 and 6 %): a chunk takes a workgroup 0.48, 0.65, 0.98 or 1.12 us with a state of up to 32, 64, 96 or 128
+// rows, 1.25 times that where one operand is fp32, a round of workgroups 4.7 us besides; both walks of an
+// exchange 1.55 times as long, and the exchange what a round's workgroups wait for each other.
+// Chains are walked whole up to 256 chunks, and up to 1024 where the results are bf16, which makes the
+// rounding of a long running state a non-issue.
+void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, bool bf16_results, int *nseg,
+                        int *seg_chunks) {
     *nseg = *seg_chunks = 0;
     if (!tp_widths(D, F) || tuning().tp == 0) return;
     const int64_t units = chains * nscans * tp_fblocks(F), chunks = (L + kChunk - 1) / kChunk;
-    const bool narrow = D <= 32 || F <= 32, single = nscans == 1;
-    if (narrow) {
-        if ((single && D <= 32 && F <= 32) || chunks > 128 || units > (single ? 768 : 1536) ||
-            (chunks <= 4 && units >= 320) || (chunks <= 8 && units >= (single ? 512 : 1024)) ||
-            (single && (chunks <= 2 || units < (chunks <= 8 ? 1 : chunks <= 32 ? 32 : 128))))
-            return;
-    } else if (D > 64 && F > 64) {
-        if (D <= 96 && ((chunks <= 4 && units >= 320) || (chunks <= 8 && units >= 4096) ||
-                        (single && chunks > 48 && units < 128) || (chunks > 256 && units < 192)))
-            return;
-    } else if ((chunks <= 4 && units >= (single ? 768 : 1024)) || (chunks <= 8 && units >= (single ? 1024 : 2048))) {
-        return;
-    }
-    if (single && D > 64 && ((units < 16 && chunks > 8 && chunks < (units < 8 ? 256 : 96)) || (units >= 320 && chunks <= 2))) return;
-    const double chunk_us = D <= 64 ? (single ? 0.63 : 0.79) : (single ? 1.07 : 1.38);
+    // (FTC_TP=1, FTC_TPX=0: tuning aids)
+    if (tuning().tp < 0 && mixed_splits(D, F, units, nscans, chunks, bf16_results)) return;
+    const double chunk_us = (D <= 32 ? 0.48 : D <= 64 ? 0.65 : D <= 96 ? 0.98 : 1.12) * (bf16_results ? 1.25 : 1.0);
     double least = 1e30;
-    // whole chains, or cut ones whose workgroups rebuild the state before their segment (results in
-    // bf16 make the rounding of a long running state a non-issue)
-    if (chunks <= (single ? 256 : 1024)) {
+    if (chunks <= (bf16_results ? 1024 : 256)) {
         int32_t start[kMaxTpSegments + 1];
         int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), chunks)) : 1;
         n = tp_segment_starts(chunks, n, start);
@@ -377,14 +373,16 @@ void mixed_rest_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, i
             longest = 0;
             for (int i = 0; i < n; i++) longest = std::max(longest, 0.6 * start[i] + (double)(start[i + 1] - start[i]));
         }
-        least = (double)((units * n + 255) / 256) * (longest * chunk_us + 4.0);
+        least = (double)((units * n + 255) / 256) * (longest * chunk_us + 4.7) + 0.5;
         *nseg = n;
     }
-    for (int64_t n = 2; n <= 64 && n <= chunks / 4; n++) {
+    // (not below 24 chunks: 16 of them, 1 chain of 64 x 64 backward 14.4 against 13.5 us cut in four)
+    for (int64_t n = 2; n <= 64 && n <= chunks / 4 && chunks >= 24 && tuning().tpx != 0; n++) {
         const int64_t c = ((chunks + n - 1) / n + kTpAhead - 1) / kTpAhead * kTpAhead, segs = (chunks + c - 1) / c;
         if (c > 256 || segs < 2 || 4 * units * segs > kMaxWaves) continue;
-        const double us = (double)((units * segs + 255) / 256) *
-                          (1.7 * (double)c * chunk_us + 14.0 + 0.5 * (double)std::min<int64_t>(segs, 16));
+        const double filled = std::min(1.0, (double)(units * segs) / 256.0);
+        const double us = (double)((units * segs + 255) / 256) * (1.55 * (double)c * chunk_us + 0.3 + 9.9 * filled) +
+                          5.7 + 0.13 * (double)std::min<int64_t>(segs, 16) + 0.9 * std::sqrt((double)segs);
         if (us < least - 1e-9) least = us, *nseg = (int)segs, *seg_chunks = (int)c;
     }
 }
@@ -488,25 +486,23 @@ struct TpPlan {
     int nseg, seg_chunks;
 };
 void tp_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg, int *seg_chunks,
-             bool forced = false, int mixed = 0, bool odd = false) {
+             bool forced = false, bool odd = false) {
     static thread_local PlanMemo<TpPlan> memo;
-    const int64_t key[8] = {D, F, chains, nscans, L, forced ? 1 : 0, mixed, odd ? 1 : 0};
+    const int64_t key[8] = {D, F, chains, nscans, L, forced ? 1 : 0, odd ? 1 : 0, 0};
     const TpPlan pl = memo.get(key, [&]() {
         TpPlan p;
-        tp_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks, forced, mixed, odd);
+        tp_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks, forced, odd);
         return p;
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
 }
-void mixed_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int mixed, int *nseg, int *seg_chunks) {
-    *nseg = *seg_chunks = 0;
-    if (D <= 64) tp_plan(D, F, chains, nscans, L, nseg, seg_chunks, false, mixed);
-    if (*nseg > 0) return;
+void mixed_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, bool bf16_results, int *nseg,
+                int *seg_chunks) {
     static thread_local PlanMemo<TpPlan> memo;
-    const int64_t key[8] = {D, F, chains, nscans, L, 0, 0, 0};
+    const int64_t key[8] = {D, F, chains, nscans, L, bf16_results ? 1 : 0, 0, 0};
     const TpPlan pl = memo.get(key, [&]() {
         TpPlan p;
-        mixed_rest_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks);
+        mixed_plan_compute(D, F, chains, nscans, L, bf16_results, &p.nseg, &p.seg_chunks);
         return p;
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
@@ -623,7 +619,7 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
     int nseg = 0, seg_chunks = 0;
     const int64_t chains = std::max<int64_t>(1, N * H);
     if (forced && odd) F = 64;  // (`nscans` blocks of columns, see column_blocks)
-    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, odd);
+    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, odd);
     return seg_chunks > 0 ? tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D) : 0;
 }
 
@@ -648,11 +644,11 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     if (!tp_widths(D, F, forced, odd)) return false;
     if (odd && !forced && !tph_takes_rows(D)) return false;
     int64_t widest_stride = 0;
-    int mixed = nscans == 1 && combo_of(scans[0]) == kBBFB ? kMixedGradValues : 0;
+    bool mixed = false;
     for (int i = 0; i < nscans; i++) {
         const ScanDesc &sd = scans[i];
         const Combo combo = combo_of(sd);
-        if (combo != kFFFF && mixed == 0) mixed = kMixedRows;
+        mixed = mixed || combo != kFFFF;
         // (rows with bf16 among them: not as parts of wider scans, whose results are added up in fp32)
         if (combo == kNone || (combo != kFFFF && (forced || tuning().tph == 0))) return false;
         // (odd widths: scans of any widths side by side, where pieces are scaled as long as none has a
@@ -679,20 +675,20 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     int nseg = 0, seg_chunks = 0;
     const int64_t chains = std::max<int64_t>(1, N * H);
     if (mixed)
-        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks);
+        mixed_plan(D, F, chains, nscans, L, scans[0].out.dtype != FTC_F32, &nseg, &seg_chunks);
     else if (odd && forced)
-        tp_plan(D, 64, chains, (int)column_blocks(scans, nscans), L, &nseg, &seg_chunks, forced, 0, odd);
+        tp_plan(D, 64, chains, (int)column_blocks(scans, nscans), L, &nseg, &seg_chunks, forced, odd);
     else
-        tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, odd);
+        tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, odd);
     return nseg > 0;
 }
 
 int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans) {
     const int64_t chains = std::max<int64_t>(1, N * H);
     int64_t bytes = 0;
-    for (const int mixed : {kMixedRows, kMixedGradValues}) {
+    for (const bool bf16_results : {false, true}) {
         int nseg = 0, seg_chunks = 0;
-        mixed_plan(D, F, chains, nscans, L, mixed, &nseg, &seg_chunks);
+        mixed_plan(D, F, chains, nscans, L, bf16_results, &nseg, &seg_chunks);
         if (seg_chunks > 0)
             bytes = std::max(bytes, tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D));
     }
@@ -704,7 +700,7 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
     int nseg = 0, seg_chunks = 0;
     if (forced) F = 64;  // (`nscans` blocks of columns)
     const int64_t chains = std::max<int64_t>(1, N * H), units = chains * nscans * tp_fblocks(F);
-    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, 0, true);
+    tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, true);
     if (nseg == 0) return 1e30;
     const int64_t rounds = (units * nseg + 255) / 256;
     double longest = 0.0;
@@ -812,15 +808,12 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     const int64_t blocks = odd && forced ? column_blocks(scans, nscans) : nscans * fblocks;
     if (fused_tp && tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     if (tp_shape) {
-        int any_bf16 = nscans == 1 && combo == kBBFB ? kMixedGradValues : 0;
-        for (int i = 0; i < nscans; i++)
-            if (combo_of(scans[i]) != kFFFF && any_bf16 == 0) any_bf16 = kMixedRows;
-        if (any_bf16)
-            mixed_plan(D, F, chains, nscans, L, any_bf16, &tpx_nseg, &tpx_seg_chunks);
+        if (combo != kFFFF)
+            mixed_plan(D, F, chains, nscans, L, scans[0].out.dtype != FTC_F32, &tpx_nseg, &tpx_seg_chunks);
         else if (odd && forced)
-            tp_plan(D, 64, chains, (int)blocks, L, &tpx_nseg, &tpx_seg_chunks, forced, 0, odd);
+            tp_plan(D, 64, chains, (int)blocks, L, &tpx_nseg, &tpx_seg_chunks, forced, odd);
         else
-            tp_plan(D, F, chains, nscans, L, &tpx_nseg, &tpx_seg_chunks, forced, 0, odd);
+            tp_plan(D, F, chains, nscans, L, &tpx_nseg, &tpx_seg_chunks, forced, odd);
         if (tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     }
     const bool tp = tp_nseg > 0 || tpx_seg_chunks > 0;

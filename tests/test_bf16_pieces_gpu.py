@@ -21,24 +21,29 @@ def cp():
     return causal_product
 
 
-SHAPES = [
-    # N, H, L, E, M: one and many blocks of state rows and of columns, blocks that are filled to 4, 32
-    # and 64 rows; one position, the ends of chunks; whole chains, cut ones, one and two levels of exchange
-    (1, 3, 1, 128, 128), (2, 4, 33, 128, 128), (4, 4, 600, 128, 128), (1, 4, 4096, 128, 128), (1, 2, 9000, 128, 128),
-    (3, 8, 300, 96, 96), (3, 8, 257, 68, 100), (2, 8, 500, 128, 64), (3, 8, 500, 64, 128), (6, 8, 257, 36, 124),
-    (2, 8, 97, 64, 64), (10, 8, 333, 64, 64), (1, 4, 5000, 64, 64), (3, 8, 300, 32, 128), (6, 8, 300, 128, 32),
-    (2, 8, 200, 32, 32),
-]
+# N, H, L, E, M: one and many blocks of state rows and of columns, blocks that are filled to 4, 32 and 64
+# rows; one position, the ends of chunks; whole chains, cut ones, one and two levels of exchange.  And the
+# launches of the forward, dQ, dK and dV alone and all three (the last one): w: whole or cut chains, x: an
+# exchange, s: the kernels that split L
+SHAPES = {
+    (1, 3, 1, 128, 128): "wwwww", (2, 4, 33, 128, 128): "wwwww", (4, 4, 600, 128, 128): "wwwww",
+    (1, 4, 4096, 128, 128): "xxxxx", (1, 2, 9000, 128, 128): "xxxxx", (3, 8, 300, 96, 96): "wwwww",
+    (3, 8, 257, 68, 100): "wwwww", (2, 8, 500, 128, 64): "wwwww", (3, 8, 500, 64, 128): "wwwww",
+    (6, 8, 257, 36, 124): "wwwww", (2, 8, 97, 64, 64): "wwwww", (10, 8, 333, 64, 64): "wwwww",
+    (1, 4, 5000, 64, 64): "xxxxx", (3, 8, 300, 32, 128): "wssww", (6, 8, 300, 128, 32): "wwwww",
+    (2, 8, 200, 32, 32): "wwwww",
+}
+LAUNCH = dict(zip("wxs", OURS + (b"scan_mfma_kernel",)))
 
 
-@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+@pytest.mark.parametrize("shape", list(SHAPES), ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
 def test_forward_and_backward(cp, shape):
     N, H, L, E, M = shape
     Qb, Kb, Vb, G = _inputs(N, H, L, E, M, 60 + L)
     q, k, v = Qb.cuda(), Kb.cuda(), Vb.cuda()
     out = torch.full((N, H, L, M), float("nan"), device="cuda")
     cp.causal_dot_product_hip(q, k, v, out)
-    used = {_last_kernel()}
+    used = [_last_kernel()]
     exact = oracle.forward(Qb.double(), Kb.double(), Vb.double())
     ref = oracle.forward(Qb.float(), Kb.float(), Vb.float())
     assert torch.isfinite(out).all()
@@ -48,14 +53,14 @@ def test_forward_and_backward(cp, shape):
         alone = [None] * 3
         alone[i] = torch.full_like(grads[i], float("nan"))
         cp.causal_dot_backward_hip(q, k, v, G.cuda(), *alone)
-        used.add(_last_kernel())
+        used.append(_last_kernel())
         grads[i] = alone[i]
     _check_gradients(str(shape), grads, Qb, Kb, Vb, G)
     together = [torch.full_like(g, float("nan")) for g in grads]
     cp.causal_dot_backward_hip(q, k, v, G.cuda(), *together)
-    used.add(_last_kernel())
+    used.append(_last_kernel())
     _check_gradients(str(shape), together, Qb, Kb, Vb, G)
-    assert used & set(OURS), used
+    assert used == [LAUNCH[x] for x in SHAPES[shape]]
 
 
 @pytest.mark.parametrize("shape", [(2, 8, 700, 128, 128), (1, 3, 4500, 64, 64), (3, 8, 150, 96, 40)], ids=str)

@@ -110,13 +110,21 @@ def test_what_the_chain_parallel_kernel_leaves_to_the_others():
     whole = bf16(1, 64, 16384, 64, 64, True)[0]
     assert whole.startswith(tp + ": 3 scans") and "1 segment of 16384 rows" in whole
     assert bf16(10, 8, 1000, 64, 64, True)[0].startswith(tp + ": 3 scans")
-    # narrow keys, wide values: the dV scan (fp32 values, a state of 32 rows) walks its chains whole, however
-    # long; the forward and the scans with a state of 128 rows are left to the kernels that split L
+    # narrow keys, wide values: with a workgroup for every CU the backward's scans (bf16 results) walk their
+    # chains whole, however long; the forward, whose fp32 results would have to be exchanged, and half as
+    # many chains are left to the kernels that split L
     wide_values = bf16(4, 32, 16384, 32, 128, True)
-    assert [kernel(l) for l in wide_values] == [tp, "scan_mfma_kernel", "scan_mfma_kernel"]
-    assert "state 32 x 128" in wide_values[0] and "1 segment of 16384 rows" in wide_values[0]
+    assert [kernel(l) for l in wide_values] == [tp, tp] and all("1 segment of 16384 rows" in l for l in wide_values)
+    assert "2 scans" in wide_values[0] and "state 128 x 32" in wide_values[0] and "state 32 x 128" in wide_values[1]
     assert kernel(bf16(4, 32, 16384, 32, 128)[0]) == "scan_mfma_kernel"
     assert {kernel(l) for l in bf16(2, 32, 16384, 32, 128, True)} == {"scan_mfma_kernel"}
+    # other launches that those kernels are faster at: many short chains, single scans of 32 x 32 on few long
+    # chains, of wide states on fewer than eight workgroups
+    assert kernel(bf16(64, 16, 128, 64, 64)[0]) == kernel(bf16(16, 64, 128, 64, 64, True)[0]) == "scan_mfma_kernel"
+    assert kernel(bf16(64, 16, 512, 64, 64)[0]) == kernel(bf16(16, 64, 512, 64, 64, True)[0]) == tp
+    assert kernel(bf16(1, 16, 4096, 32, 32)[0]) == "scan_mfma_kernel"
+    assert kernel(bf16(1, 16, 4096, 32, 32, True)[0]) == tpx and kernel(bf16(32, 8, 4096, 32, 32)[0]) == tp
+    assert kernel(bf16(1, 1, 1000, 128, 128)[0]) == "scan_mfma_kernel" and kernel(bf16(1, 8, 1000, 128, 128)[0]) == tpx
     # widths that the kernels that split L would only take as padded copies
     assert kernel(bf16(6, 8, 257, 48, 40)[0]) == tp
     assert kernel(bf16(8, 8, 130, 20, 20)[0]) == tp
