@@ -685,10 +685,10 @@ bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64
 // 446, backward, 24 chains, L=177 42 / 18; 99 x 101 backward, 2 chains, L=5038 71 / 44; the scans of two
 // shapes in one launch (odd_scans): 75 x 10 backward, 4 chains, L=789 105 / 32.  What keeps them:
 // single scans of more than 64 rows on up to four workgroups' worth of chains with few segments there
-// (75 x 10, 1 chain, L=1942 28 / 67, 4 chains, L=789 27 / 31), thousands of workgroups with two chunks each (30 x 50 backward,
-// 3000 chains, L=40 161 / 198), and calls of several scans on more than two rounds of workgroups and
-// 128 chunks or more (99 x 101 backward, 128 chains, L=4096 1494 / 922: faster here, but such a call's plan has the
-// copies in its name and size).  Rows of which some fit stay as in odd_in_place, and so does a workspace without room.
+// (75 x 10, 1 chain, L=1942 28 / 67, 4 chains, L=789 27 / 31), and thousands of workgroups with two chunks each
+// (30 x 50 backward, 3000 chains, L=40 161 / 198).  Long chains on many workgroups, 35 calls (2-norm errors
+// a half to a quarter of the copies'): 99 x 101 backward, 128 chains, L=4096 1598 / 1078, 75 x 10, 300 chains,
+// L=5000 2709 / 1294, with an exchange 90 x 90, 128 chains, L=12000 4528 / 3182.  Rows of which some fit stay as in odd_in_place, and so does a workspace without room.
 bool odd_on_three_pieces(const ScanDesc *scans, int n, const bool *padded, int64_t N, int64_t H, int64_t L,
                          size_t workspace_bytes) {
     if (tuning().odd == 0 || tuning().tp == 0) return false;  // tuning aids
@@ -704,8 +704,7 @@ bool odd_on_three_pieces(const ScanDesc *scans, int n, const bool *padded, int64
     }
     if (tuning().odd == 2) return true;
     if (n == 1 && scans[0].a.width > 64 && units <= 4 && chunks > 16 && chunks <= 64) return false;
-    if (widest <= 64 && chunks <= 2 && units > 4096) return false;
-    return n == 1 || units <= 512 || chunks < 128;
+    return !(widest <= 64 && chunks <= 2 && units > 4096);
 }
 
 // Scans for which odd_in_place holds, in one launch or one per shape, whichever is estimated
@@ -740,8 +739,12 @@ int odd_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
                    room(group[k][0].a.width, group[k][0].v.width, blocks(group[k], size[k]));
         if (apart_ok) apart += mfma_tp_odd_chunks(group[k][0].a.width, group[k][0].v.width, N, H, blocks(group[k], size[k]), L, forced);
     }
+    // (an exchange of all of them where one shape has none of its own, its segments being more than there are
+    // flags for: 75 x 10 backward, 200 chains, L=9000 3120 us where the copies take 2730)
     const bool together_ok = ngroups > 1 && mfma_tp_takes(scans, n, N, H, L, forced, true) &&
-                             room(widest_d, widest_f, blocks(scans, n));
+                             room(widest_d, widest_f, blocks(scans, n)) &&
+                             (apart_ok || !forced ||
+                              mfma_tp_workspace_bytes(N, H, L, widest_d, widest_f, blocks(scans, n), forced, true) == 0);
     if (!apart_ok && !together_ok) return FTC_OK;
     auto run = [&](const ScanDesc *s, int k) {
         return mfma_scan(s, k, N, H, L, workspace, workspace_bytes, stream, nullptr, true, forced, true);

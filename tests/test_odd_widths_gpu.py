@@ -196,6 +196,21 @@ def test_odd_widths_in_place_on_three_pieces(shape, monkeypatch):
         cp.reload_tuning()
 
 
+def test_many_long_chains_in_place():
+    """More than two rounds of workgroups on chains of more than 128 chunks: as close to float64 as the
+    fp32 oracle (copies were two to four times as far away)."""
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = 9, 20, 4100, 9, 11
+    Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=961)
+    grads = [torch.full_like(t, float("nan")).cuda() for t in (Q, K, V)]
+    cp.causal_dot_backward_hip(*(t.cuda() for t in (Q, K, V, G)), *grads)
+    assert _native.load().ftc_last_kernel() == b"scan_tp_kernel"
+    exact, ref = oracle.backward(*(t.double() for t in (Q, K, V, G))), oracle.backward(Q, K, V, G)
+    for got, r, ex in zip(grads, ref, exact):
+        assert ((got.cpu() - ex).norm() / ex.norm()).item() <= max(((r - ex).norm() / ex.norm()).item(), 5e-7)
+
+
 TOGETHER = [
     # N, H, L, E, M (widths that need no copies): two state shapes side by side, whole, cut and exchanged
     # chains, one and two groups of 32 rows, a single chunk, ragged ends; 32 x 32; and two shapes of which

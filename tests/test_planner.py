@@ -140,9 +140,12 @@ def test_what_the_chain_parallel_kernel_leaves_to_the_others():
     odd = lines((8, 16, 4096, 25), (8, 16, 4096, 64), backward=True)
     assert odd[0].startswith("pad_rows_kernel: 2 operands") and "2 results" in odd[0]
     assert odd[1].startswith("scan_tph_kernel: 2 scans") and "state 64 x 32" in odd[1]
+    # ... and where every operand would be copied, the kernel that takes odd widths where they lie, on any
+    # number of workgroups; not where one shape has no plan of its own and all of them need an exchange
     wide = lines((8, 16, 4096, 99), (8, 16, 4096, 101), backward=True)
-    assert wide[0].startswith("pad_rows_kernel: 4 operands") and "3 results" in wide[0]
-    assert wide[1].startswith("scan_tp_kernel: 3 scans") and "state 128 x 128" in wide[1]
+    assert len(wide) == 1 and wide[0].startswith("scan_tp_kernel: 3 scans") and "768 workgroups" in wide[0]
+    assert lines((9, 20, 4100, 9), (9, 20, 4100, 11), backward=True)[0].startswith("scan_tp_kernel: 3 scans")
+    assert lines((1, 200, 9000, 75), (1, 200, 9000, 10), backward=True)[0].startswith("pad_rows_kernel: 4 operands")
     assert lines((2, 2, 40, 10), (2, 2, 40, 3))[0].startswith("generic_scan_kernel")
     # (bf16 rows of such a scan are converted into fp32 copies on the way)
     assert lines((1, 2, 8192, 300), (1, 2, 8192, 64), dtype=_native.FTC_BF16)[0] \
