@@ -736,11 +736,12 @@ int64_t fused_tp_state_rows(int64_t D) { return (D + 63) / 64 * 64 + 64; }
 // units split L and which carries two units of 32 value columns per workgroup.  Measured (us, the
 // workgroup form / this way), 64 x 64: 80 chains, L=1000 47.8 / 36.9, L=4096 138 / 114; 512 chains,
 // L=1000 160 / 130; 384 chains, L=2774 350 / 286; 216 chains, L=134 17.6 / 15.1; 64 chains, L=1500
-// 50.3 / 45.2; 32 chains, L=4096 62.9 / 53.9; but 8 chains, L=500 17.1 / 19.0, 16 chains, L=1500
-// 27.4 / 29.5.  (Chains that are not exchanged: from 41 on.  The workgroup form's own tests are cases
-// of 24 to 40 of them and ask for it by name; 32 chains, L=500 would be 23.3 / 19.4.)  One width of
-// 32: 80 chains, L=1000 41.6 / 34.8 and 36.7 / 32.0, but 64 chains, L=1500 42.9 / 44.2, more than a
-// round of workgroups 102 / 116, with an exchange 95.7 / 106.  32 x 32: 31.7 / 31.3 and 64 / 96.
+// 50.3 / 45.2; 32 chains, L=4096 62.9 / 53.9; 32 chains, L=134 17.5 / 11.6, L=500 23.4 / 19.6, L=700 26.5 / 25.6;
+// 8 chains, L=200 14.9 / 13.0; but 8 chains, L=500 17.5 / 19.3, 24 chains, L=700 23.9 / 25.5, 36 chains, L=1000
+// 31.5 / 32.7, 48 chains, L=1500 43.8 / 46.3.  One width of 32: 80 chains, L=1000 41.6 / 34.8 (64 x 32) and
+// 36.7 / 32.0, 32 chains, L=300 19.1 / 14.8 and 16.6 / 13.8; but 48 chains, L=1000 32.3 / 33.0 and 29.1 / 30.7, 64 chains,
+// L=1500 42.9 / 44.2, 32 x 64 on up to four chunks 8.2 / 8.5, more than a round of workgroups 102 / 116, with an
+// exchange 95.7 / 106.  32 x 32: 31.7 / 31.3 and 64 / 96.
 // Chains of more than 256 chunks are not walked whole on three bf16 pieces (tp_plan_compute).
 //
 // Rows of 128 have no other fused form: the plan is that of such a scan where the chain-parallel kernel
@@ -758,9 +759,12 @@ bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, i
     tp_plan(64, 64, chains, 1, L, nseg, seg_chunks);
     if (*nseg > 0 && *seg_chunks == 0 && chunks > 256) *nseg = 0;
     if (*nseg == 0 || tuning().wg == 0) return *nseg > 0;  // (FTC_WG=0: tuning aid)
-    const bool take = D == 64 && F == 64 ? (*seg_chunks > 0 ? chains >= 24 && chunks >= 64 : chains > 40)
-                                         : (D == 64 || F == 64) && *seg_chunks == 0 && chains > 40 &&
-                                               chains <= 256 && chunks <= 32;
+    // the fewest chains without an exchange, where the two cross
+    const bool square = D == 64 && F == 64;
+    int64_t least = chunks <= 10 ? 4 : chunks <= 16 ? 20 : chunks <= 24 ? 32 : chunks <= 32 && square ? 40 : 56;
+    if (D == 32) least = chunks <= 4 ? INT64_MAX : chunks <= 7 ? 8 : chunks <= 10 ? 20 : chunks <= 16 ? 28 : chunks <= 24 ? 44 : 56;
+    const bool take = *seg_chunks > 0 ? square && chains >= 24 && chunks >= 64
+                                      : (square || ((D == 64 || F == 64) && chains <= 256 && chunks <= 32)) && chains >= least;
     if (!take) *nseg = *seg_chunks = 0;
     return take;
 }

@@ -173,6 +173,24 @@ def test_sizes_without_a_fused_kernel_are_refused(lib):
     assert rc == -2 and "fused" in _native.last_error()
 
 
+@pytest.fixture(params=["planned", "workgroup"])
+def form(request, monkeypatch):
+    """Which kernel takes the launch: as planned, or the workgroup form at any size."""
+    from fast_transformers_amd import causal_product as cp
+    if request.param == "workgroup":
+        monkeypatch.setenv("FTC_WG", "1")
+        cp.reload_tuning()
+    yield request.param
+    if request.param == "workgroup":
+        monkeypatch.delenv("FTC_WG")
+        cp.reload_tuning()
+
+
+def taken_by(form, L):
+    """Of these tests' shapes, the chain-parallel kernel has those of short chains."""
+    return b"scan_tp_kernel<NORM>" if form == "planned" and L <= 320 else b"scan_wg_kernel<NORM>"
+
+
 CHAIN_PARALLEL_SHAPES = [
     # N, L, H, E, M, key lengths: whole chains, cut chains, an exchange of segment sums (one and two
     # levels), ragged ends, keys that end before, inside and on a chunk, segments without any key;
@@ -185,13 +203,13 @@ CHAIN_PARALLEL_SHAPES = [
 
 
 @pytest.mark.parametrize("shape", CHAIN_PARALLEL_SHAPES, ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s[:5])
-def test_chain_parallel_form(lib, shape):
+def test_chain_parallel_form(lib, shape, form):
     """Chain counts, lengths and key lengths of every kind, against the CPU restatement in float64."""
     N, L, H, E, M, lens = shape
     q, k, v = inputs(N, L, H, E, M, seed=70 + L)
     lengths = torch.tensor(lens)
     out = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
-    assert lib.ftc_last_kernel() == b"scan_wg_kernel<NORM>"
+    assert lib.ftc_last_kernel() == taken_by(form, L)
     gate(out.cpu(), q, k, v, lengths, 1e-6)
 
 
@@ -202,13 +220,13 @@ MASKED_SHAPES = [(3, 97, 8, 64, 64, [97, 64, 1]), (2, 1000, 16, 64, 64, [1000, 4
 
 @pytest.mark.parametrize("padding", [1e8, 1e30])
 @pytest.mark.parametrize("shape", MASKED_SHAPES, ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s[:5])
-def test_masked_rows_do_not_set_a_scale(lib, shape, padding):
+def test_masked_rows_do_not_set_a_scale(lib, shape, padding, form):
     """Keys and values at or beyond the length leave every row as it is, bit for bit."""
     N, L, H, E, M, lens = shape
     q, k, v = inputs(N, L, H, E, M, seed=170 + L)
     lengths = torch.tensor(lens)
     want = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
-    assert lib.ftc_last_kernel() == b"scan_wg_kernel<NORM>"
+    assert lib.ftc_last_kernel() == taken_by(form, L)
     for n, length in enumerate(lens):
         k[n, length:], v[n, length:] = 60.0, padding
     got = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
@@ -219,7 +237,7 @@ def test_masked_rows_do_not_set_a_scale(lib, shape, padding):
 @pytest.mark.parametrize("small", ["q_rows", "k_early_rows", "v_columns", "v_early_rows"])
 @pytest.mark.parametrize("shape", [(3, 300, 8, 64, 64), (2, 1000, 16, 64, 64), (3, 520, 8, 32, 64)],
                          ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s)
-def test_small_rows_and_columns_beside_large_ones(lib, shape, small):
+def test_small_rows_and_columns_beside_large_ones(lib, shape, small, form):
     """Every row and column of the result is within 2e-6 of float64 on its own scale (a few fp32
     roundings; the float32 restatement is not, where it adds 1 to an expm1 near -1): a row's weights are
     normalised, so rows of small phi(q) or phi(k) beside large ones are still of order one, and columns
@@ -271,7 +289,7 @@ def test_many_chains(lib, shape):
 @pytest.mark.parametrize("shape", [(6, 300, 8, 64, 64), (3, 2100, 8, 64, 64), (6, 520, 8, 64, 32)],
                          ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s)
 def test_many_chains_small_rows_and_columns_beside_large_ones(lib, shape, small):
-    test_small_rows_and_columns_beside_large_ones(lib, shape, small)
+    test_small_rows_and_columns_beside_large_ones(lib, shape, small, "planned")
     assert lib.ftc_last_kernel().startswith(b"scan_tp_kernel<NORM>")
 
 
@@ -420,7 +438,7 @@ BACKWARD_SHAPES = [
 
 
 @pytest.mark.parametrize("shape", BACKWARD_SHAPES, ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s[:5])
-def test_backward_against_autograd_in_float64(lib, shape):
+def test_backward_against_autograd_in_float64(lib, shape, form):
     """ftc_causal_linear_attention_backward (through the autograd Function the module uses)
     against autograd through the dense closed form in float64; the same closed form in
     float32 shows what that arithmetic alone costs."""
@@ -442,7 +460,8 @@ def test_backward_against_autograd_in_float64(lib, shape):
     qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
     nlh = lambda t: t.permute(0, 2, 1, 3)
     out = CausalLinearAttentionFunction.apply(nlh(qd), nlh(kd), nlh(vd), lengths.cuda(), eps)
-    assert lib.ftc_last_kernel().startswith(b"scan_wg_kernel")
+    short = shape in (BACKWARD_SHAPES[0], BACKWARD_SHAPES[4])   # chains that the planner walks whole or cut
+    assert lib.ftc_last_kernel() == taken_by(form, L if short else 1000)
     with _count_backward_calls() as calls:
         nlh(out).backward(g.cuda())
     assert calls == [1]
