@@ -685,15 +685,16 @@ bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64
 // 446, backward, 24 chains, L=177 42 / 18; 99 x 101 backward, 2 chains, L=5038 71 / 44; the scans of two
 // shapes in one launch (odd_scans): 75 x 10 backward, 4 chains, L=789 105 / 32.  What keeps them:
 // single scans of more than 64 rows on up to four workgroups' worth of chains with few segments there
-// (75 x 10, 1 chain, L=1942 28 / 67, 4 chains, L=789 27 / 31), and thousands of workgroups with two chunks each
-// (30 x 50 backward, 3000 chains, L=40 161 / 198).  Long chains on many workgroups, 35 calls (2-norm errors
+// (75 x 10, 1 chain, L=1942 28 / 67, 4 chains, L=789 27 / 31), and many short
+// chains of a width of up to 32 beside any other (18 x 84 backward, 1896 chains, L=16 86 / 138, 18 x 30, 900 chains,
+// L=64 0.9 of the time; wider ones are faster here on any number: 70 x 70, 4000 chains, L=16 1.16 of it).  Long chains on many workgroups, 35 calls (2-norm errors
 // a half to a quarter of the copies'): 99 x 101 backward, 128 chains, L=4096 1598 / 1078, 75 x 10, 300 chains,
 // L=5000 2709 / 1294, with an exchange 90 x 90, 128 chains, L=12000 4528 / 3182.  Rows of which some fit stay as in odd_in_place, and so does a workspace without room.
 bool odd_on_three_pieces(const ScanDesc *scans, int n, const bool *padded, int64_t N, int64_t H, int64_t L,
                          size_t workspace_bytes) {
     if (tuning().odd == 0 || tuning().tp == 0) return false;  // tuning aids
     const int64_t chunks = (L + 31) / 32;
-    int64_t units = 0, widest = 0;
+    int64_t units = 0, widest = 0, least = INT64_MAX;
     for (int i = 0; i < n; i++) {
         const int64_t D = scans[i].a.width, F = scans[i].v.width;
         bool any_fits;
@@ -701,10 +702,15 @@ bool odd_on_three_pieces(const ScanDesc *scans, int n, const bool *padded, int64
         if (!plan_only() && (int64_t)workspace_bytes < padded_scan_workspace_bytes(N, H, L, D, F)) return false;
         units += N * H * ((F + 63) / 64);
         widest = std::max(widest, std::max(D, F));
+        least = std::min(least, std::min(D, F));
     }
     if (tuning().odd == 2) return true;
     if (n == 1 && scans[0].a.width > 64 && units <= 4 && chunks > 16 && chunks <= 64) return false;
-    return !(widest <= 64 && chunks <= 2 && units > 4096);
+    // (measured on 300 to 4000 chains of 16 to 90 positions: where the two cross)
+    if (least > 32 || L > 96) return true;
+    if (widest > 32) return L > 48 || units <= (n == 1 ? (L <= 24 ? 1400 : L <= 32 ? 2200 : 3500) : L <= 32 ? 2600 : 4000);
+    if (n == 1) return L > 64 || units <= (L <= 16 ? 1000 : L <= 32 ? 1300 : L <= 48 ? 2000 : 2200);
+    return units <= (L <= 32 ? 1200 : L <= 64 ? 1900 : 2700);
 }
 
 // Scans for which odd_in_place holds, in one launch or one per shape, whichever is estimated

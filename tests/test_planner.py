@@ -146,6 +146,10 @@ def test_what_the_chain_parallel_kernel_leaves_to_the_others():
     assert len(wide) == 1 and wide[0].startswith("scan_tp_kernel: 3 scans") and "768 workgroups" in wide[0]
     assert lines((9, 20, 4100, 9), (9, 20, 4100, 11), backward=True)[0].startswith("scan_tp_kernel: 3 scans")
     assert lines((1, 200, 9000, 75), (1, 200, 9000, 10), backward=True)[0].startswith("pad_rows_kernel: 4 operands")
+    # ... nor many short chains of up to 32 rows or columns
+    assert lines((1, 1896, 16, 18), (1, 1896, 16, 84), backward=True)[0].startswith("pad_rows_kernel: 4 operands")
+    assert lines((1, 600, 16, 18), (1, 600, 16, 84), backward=True)[0].startswith("scan_tp_kernel: 2 scans")
+    assert lines((1, 4000, 16, 70), (1, 4000, 16, 70), backward=True)[0].startswith("scan_tp_kernel: 3 scans")
     assert lines((2, 2, 40, 10), (2, 2, 40, 3))[0].startswith("generic_scan_kernel")
     # (bf16 rows of such a scan are converted into fp32 copies on the way)
     assert lines((1, 2, 8192, 300), (1, 2, 8192, 64), dtype=_native.FTC_BF16)[0] \
