@@ -291,6 +291,41 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
 //   single ones: 32 x 32, 16 chains, L=4096 17 / 22, 256 chains, L=1000 43 / 30; 128 x 32, 64 chains,
 //   L=4096 66 / 74, 256 chains 236 / 165; 32 x 128 forward, 128 chains, L=8192 262 / 209, 64 chains 141 / 166
 //   and L=16384 277 / 313, where its fp32 rows have to be exchanged.
+// ... of them the short chains of wide states (more than 32 rows and columns): a round of workgroups takes
+// 4.7 us here however short its chains, so those kernels win from some number of workgroups on, which grows
+// with the chunks.  Measured: 128 to 2048 chains of 20 to 512 positions, split L / here: 64 x 64 forward, 684
+// chains, L=126 20 / 26; 512 chains, L=512 49 / 35; 128 x 64, 768 chains, L=64 1.37 of the time here.
+bool short_chains_split(int64_t D, int64_t F, int64_t units, bool single, int64_t chunks) {
+    if (chunks > 16) return false;
+    constexpr int16_t kAny = INT16_MAX;
+    // the most workgroups for chains of 1, 2, 3, 4, 6, 8, 12 and 16 chunks
+    struct Row {
+        int d, f;
+        int16_t most[8];
+    };
+    static constexpr Row kSingle[] = {
+        {64, 64, {256, 256, 256, 256, 416, 512, 512, 512}},    {64, 96, {512, 650, 720, 720, 1024, 1216, 1300, kAny}},
+        {64, 512, {256, 256, 256, 256, 512, 512, 512, 512}},   {96, 64, {256, 256, 256, 256, 800, 800, kAny, kAny}},
+        {96, 96, {256, 256, 256, 256, 256, 256, kAny, kAny}},  {96, 512, {256, 256, 256, 256, kAny, kAny, kAny, kAny}},
+        {128, 512, {256, kAny, kAny, kAny, kAny, kAny, kAny, kAny}}};
+    static constexpr Row kSeveral[] = {
+        {64, 64, {900, 1280, 1600, 1700, 1900, 2000, kAny, kAny}},
+        {64, 96, {1200, 1500, 1700, 2048, 2100, 2400, kAny, kAny}},
+        {64, 512, {600, 800, 880, 1060, 1100, 1160, 1160, kAny}}, {96, 64, {750, kAny, kAny, kAny, kAny, kAny, kAny, kAny}},
+        {96, 96, {1000, 3000, 3300, 3300, 3300, 3300, kAny, kAny}}, {96, 512, {600, 3500, kAny, kAny, kAny, kAny, kAny, kAny}},
+        {128, 64, {kAny, kAny, kAny, kAny, kAny, kAny, kAny, kAny}}, {128, 96, {800, 3500, kAny, kAny, kAny, kAny, kAny, kAny}},
+        {128, 512, {2000, kAny, kAny, kAny, kAny, kAny, kAny, kAny}}};
+    const int bucket = chunks <= 4 ? (int)chunks - 1 : chunks <= 6 ? 4 : chunks <= 8 ? 5 : chunks <= 12 ? 6 : 7;
+    const Row *row = single ? kSingle : kSeveral;
+    while (D > row->d || F > row->f) row++;
+    // (96 x 96, a single scan: a last round less than four fifths full)
+    if (single && D > 64 && D <= 96 && F > 64 && F <= 96 && units > 256 && (units + 255) / 256 * 205 > units) return true;
+    // (many rounds of longer chains: both keep the memory busy)
+    const int64_t again = chunks <= 8 || D > 64 || (F > 64 && F <= 96) ? INT64_MAX
+                          : single ? (F > 64 ? 1100 : chunks <= 12 ? 1200 : 850)
+                                   : 2300;
+    return row->most[bucket] != kAny && units > row->most[bucket] && units < again;
+}
 bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunks, bool bf16_results) {
     // (widths that those kernels take as padded copies only)
     if (!mfma_scan_supported_widths(D, F)) return D <= 64 && F <= 64 && units > (nscans == 1 ? 512 : 1400) && chunks <= 2;
@@ -298,16 +333,10 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     // (a last round of workgroups that is nearly empty)
     const bool uneven = units > 256 && (units + 255) / 256 * 256 * 7 > units * 10;
     if (D > 32 && F > 32) {
-        if (D > 64 && F > 64) {
-            if (D <= 96 && ((chunks <= 4 && units >= 320) || (chunks <= 8 && units >= 4096) ||
-                            (single && chunks > 48 && units < 128) || (chunks > 256 && units < 192)))
-                return true;
-        } else if (single ? (chunks <= 4 && units >= 768) || (chunks <= 8 && units >= 1024)
-                          : (chunks <= 2 && units >= 1280) || (chunks <= 8 && units >= 2048)) {
+        if (short_chains_split(D, F, units, single, chunks)) return true;
+        if (D > 64 && D <= 96 && F > 64 && ((single && chunks > 48 && units < 128) || (chunks > 256 && units < 192)))
             return true;
-        }
-        return single && D > 64 &&
-               ((units < 16 && chunks > 8 && chunks < (units < 8 ? 256 : 96)) || (units >= 320 && chunks <= 2));
+        return single && D > 64 && units < 16 && chunks > 8 && chunks < (units < 8 ? 256 : 96);
     }
     if (!single) {
         if (D <= 32 && F <= 32) {
@@ -317,10 +346,12 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
         if (F <= 32 && chunks >= 192 && ((units > 64 && units < 144) || uneven)) return true;
         if (F <= 32 && chunks > 512) return units > 16;
         if (chunks > 64) return false;
+        if (F > 64 && F <= 96 && chunks <= 12) return units > (chunks == 1 ? 1200 : chunks <= 3 ? 1450 : chunks <= 4 ? 1750 : 2150);
         if (F > 64) return units > (chunks <= 8 ? 1024 : 2048);
         return chunks <= 2 ? units > 512 : chunks <= 8 ? units > 768 : F <= 32 && units > 1024;
     }
     if (F > 64) {  // 32 rows
+        if (F <= 96 && chunks <= 12) return units > (chunks == 1 ? 600 : chunks <= 2 ? 800 : chunks <= 4 ? 900 : 1150);
         if (chunks <= 64) return units > (chunks <= 2 ? 512 : chunks <= 8 ? 768 : 1024);
         if (chunks < 192) return false;
         if (bf16_results) return uneven || (units > 32 && units < 160);
@@ -334,6 +365,7 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     if (chunks <= 2) return D <= 64 || units > 256;
     if (chunks <= 8) return units > (chunks > 4 && !bf16_results ? 320 : 256);
     if (chunks > 12 && uneven) return true;
+    if (D > 64 && D <= 96 && chunks <= 24 && units > 256) return true;
     if (D > 64) {
         if (chunks <= 48) return units < (chunks <= 16 ? 32 : 16) || (bf16_results && units > 512);
         if (chunks <= 96) return !((units >= 8 && units <= 32) || units >= 112);
