@@ -130,24 +130,24 @@ bool mfma_scan_same_launch(const ScanDesc &x, const ScanDesc &y);
 // Workspace for `nscans` scans of one (D, F) run side by side in one launch.
 int64_t mfma_scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F,
                                   int nscans);
-// The chain-parallel kernel: all-fp32 scans of one shape whose state has 16 to 128 rows and
-// columns, widths multiples of 4 (also widths that mfma_scan_supported
+// The chain-parallel kernels: scans of one shape, fp32 rows or rows with bf16 among them, whose state has
+// 16 to 128 rows and up to 512 columns, widths multiples of 4 (also widths that mfma_scan_supported
 // does not list).  True when mfma_scan would run these scans, side by side, on that kernel;
 // its workspace (part of mfma_scan_workspace_bytes where both apply).
 // `forced`: these scans are parts of scans that the caller has split by state rows because
 // only this kernel can take them (any multiple of 4 will do, at any size).
-// `odd`: fp32 rows of any width on any 4-byte boundary, read and written where they lie (states of
-// up to 64 rows; scans of different widths may share the launch where none has more than 64
-// columns).
+// `odd`: fp32 rows of any width on any 4-byte boundary, read and written where they lie: on two fp16
+// pieces states of up to 64 rows, where scans of different widths may share the launch if none has more than
+// 64 columns; with `forced` on three bf16 pieces, states of up to 128 rows and scans of any widths.
 bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
                    bool forced = false, bool odd = false);
 int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans,
                                 bool forced = false, bool odd = false);
 // ... and of scans with bf16 rows among them
 int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans);
-// estimated time of such a launch, in chunks walked one after the other
 // blocks of 64 output columns of several scans
 int64_t column_blocks(const ScanDesc *scans, int nscans);
+// estimated time of an `odd` launch, in chunks walked one after the other
 double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L, bool forced);
 // The fused attention form of a forward scan: a and b go through the feature map
 // elu(x) + 1, rows of b at or beyond key_lengths[n] count as zero, and every output row is

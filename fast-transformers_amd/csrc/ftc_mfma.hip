@@ -31,8 +31,8 @@ bool use_wg_kernel(int64_t D, int64_t F, int nscans, int64_t L, bool all_f32) {
 // widths that are multiples of 4 (a lane's 16 bytes lie wholly inside a row or wholly outside).
 // (`forced`: a part of a scan that the caller has split because only this kernel takes it;
 // then any multiple of 4 will do)
-// `odd`: fp32 rows of any width on 4-byte boundaries, states of up to 64 rows (the fp16-piece
-// kernel reads and writes those where they lie).
+// `odd`: fp32 rows of any width on 4-byte boundaries, which the kernels read and write where they lie: the
+// fp16-piece kernel with states of up to 64 rows, the one on three bf16 pieces (`forced`) of up to 128.
 bool tp_widths(int64_t D, int64_t F, bool forced = false, bool odd = false) {
     if (odd) return D >= 8 && D <= (forced ? 128 : 64) && F >= 8 && F <= 512;
     const int64_t least = forced ? 4 : 16;
@@ -727,7 +727,7 @@ int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D
     return bytes;
 }
 
-// (a chunk of a state of more than 64 rows takes 1.7 times as long)
+// (a chunk of a state of more than 64 rows takes 1.7 times as long; `forced`: on three bf16 pieces, `nscans` blocks)
 double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans, int64_t L, bool forced) {
     int nseg = 0, seg_chunks = 0;
     if (forced) F = 64;  // (`nscans` blocks of columns)

@@ -1,5 +1,5 @@
-// Chain-parallel form of the MFMA causal scan for gfx950, all-fp32 rows, states of up to
-// 128 x 128.  Described for a 64 x 64 state; a state of more rows is walked in two blocks of
+// Chain-parallel form of the MFMA causal scan for gfx950, states of up to 128 x 128, fp32 rows in three
+// bf16 pieces and bf16 rows in one.  Described for fp32 rows and a 64 x 64 state; a state of more rows is walked in two blocks of
 // 64 (ND = 2: two positions of the walk per chunk, each on its own 64 columns of a and b and
 // its own rows of the slabs; their quadrants of Pt are added before the cut, the result rows
 // are stored after the second, and both read one v tile), output columns beyond 64 have a
