@@ -445,7 +445,7 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
             // The composition does not keep its result, which the caller may then change in place: kept here
             // as an alias that no check refuses, with a tensor that tells such a change (it shares the
             // result's version), after which the backward computes the result again.
-            const Tensor version = at::empty({0}, out.options());
+            const Tensor version = at::empty({0});
             torch::autograd::impl::set_version_counter(version, torch::autograd::impl::version_counter(out));
             ctx->saved_data["version"] = version;
             ctx->saved_data["unchanged"] = (int64_t)out._version();
@@ -456,7 +456,8 @@ struct CausalAttention : torch::autograd::Function<CausalAttention> {
             ctx->save_for_backward({q, k, v, out, den});
         }
         // (rows of 128: as in the composition, which makes its mask here, the caller may have the lengths back)
-        ctx->saved_data["lengths"] = wide_rows(q, v) ? lengths.clone() : lengths;
+        const at::AutoDispatchBelowADInplaceOrView below;  // (a plain copy costs the host half as much)
+        ctx->saved_data["lengths"] = wide_rows(q, v) ? at::empty_like(lengths).copy_(lengths) : lengths;
         ctx->saved_data["eps"] = eps;
         return out;
     }
