@@ -285,9 +285,10 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
 // exchanges (us, split L / here):
 //   wide: 64 x 64 forward, 1024 chains, L=64 12.3 / 17.9, L=256 32 / 40, but 512 chains, L=512 49 / 35;
 //   backward, 768 chains, L=128 57 / 67, but 384 chains 45 / 36; 128 x 128 forward, 1 chain, L=1000 18 / 21,
-//   but 4 chains, L=2048 47 / 26;
+//   but 4 chains, L=2048 47 / 26; 96 x 96 forward, 48 chains, L=8192 179 / 194, but 4 chains, L=2048 32 / 21;
 //   32 rows or columns, several scans: dQ and dK of 32 x 128, 768 chains, L=128 47 / 60, but 256 chains 32 / 21,
-//   128 chains, L=16384 1118 / 897, 48 chains, L=8192 223 / 264; 32 x 32, 96 chains, L=8192 backward 131 / 179;
+//   128 chains, L=16384 1118 / 897, 48 chains, L=8192 223 / 264; 32 x 32 backward, 48 chains, L=8192 135 / 157,
+//   but 16 chains 92 / 64 and L=65536 336 / 397;
 //   single ones: 32 x 32, 16 chains, L=4096 17 / 22, 256 chains, L=1000 43 / 30; 128 x 32, 64 chains,
 //   L=4096 66 / 74, 256 chains 236 / 165; 32 x 128 forward, 128 chains, L=8192 262 / 209, 64 chains 141 / 166
 //   and L=16384 277 / 313, where its fp32 rows have to be exchanged.
@@ -334,13 +335,14 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     const bool uneven = units > 256 && (units + 255) / 256 * 256 * 7 > units * 10;
     if (D > 32 && F > 32) {
         if (short_chains_split(D, F, units, single, chunks)) return true;
-        if (D > 64 && D <= 96 && F > 64 && ((single && chunks > 48 && units < 128) || (chunks > 256 && units < 192)))
+        if (!single || D <= 64) return false;
+        if (D <= 96 && F > 64 && F <= 96 && chunks > 48 && units >= (bf16_results ? 12 : 20) && units < (bf16_results ? 176 : 128))
             return true;
-        return single && D > 64 && units < 16 && chunks > 8 && chunks < (units < 8 ? 256 : 96);
+        return chunks > 8 && chunks < (units <= 1 ? 128 : units <= 3 ? 96 : units <= 7 ? 48 : units < 16 ? 28 : 0);
     }
     if (!single) {
         if (D <= 32 && F <= 32) {
-            if (chunks > 128) return units > 48;
+            if (chunks > 128) return units > (chunks > 1024 ? 24 : 48);
             return chunks <= 64 && units > (chunks <= 4 ? 1024 : chunks <= 8 ? 1100 : 1536);
         }
         if (F <= 32 && chunks >= 192 && ((units > 64 && units < 144) || uneven)) return true;
@@ -373,7 +375,7 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
                  (units >= 112 && units <= 144 && chunks <= 128));
     }
     if (chunks <= 24) return units > 512;
-    if (chunks <= 48) return units < 48 || (units > 512 && (bf16_results || D <= 32));
+    if (chunks <= 48) return units < 48 || (units > 512 && (bf16_results || (D <= 32 && units < 900)));
     if (chunks > 256) return true;
     if (D <= 32) return units < (chunks <= 72 ? 176 : 224) || (bf16_results && units > 512);
     return units < (chunks <= 96 ? (bf16_results || chunks > 72 ? 112 : 64) : bf16_results ? 176 : 160) || (bf16_results && units > 512);
@@ -408,8 +410,9 @@ void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_
         least = (double)((units * n + 255) / 256) * (longest * chunk_us + 4.7) + 0.5;
         *nseg = n;
     }
-    // (not below 24 chunks: 16 of them, 1 chain of 64 x 64 backward 14.4 against 13.5 us cut in four)
-    for (int64_t n = 2; n <= 64 && n <= chunks / 4 && chunks >= 24 && tuning().tpx != 0; n++) {
+    // (not below 24 chunks, 28 of wide states: 16 of them, 1 chain of 64 x 64 backward 14.4 us against 13.5 cut in
+    // four; 25, 12 chains of 128 x 64 backward 46 against 42)
+    for (int64_t n = 2; n <= 64 && n <= chunks / 4 && chunks >= (D > 64 ? 28 : 24) && tuning().tpx != 0; n++) {
         const int64_t c = ((chunks + n - 1) / n + kTpAhead - 1) / kTpAhead * kTpAhead, segs = (chunks + c - 1) / c;
         if (c > 256 || segs < 2 || 4 * units * segs > kMaxWaves) continue;
         const double filled = std::min(1.0, (double)(units * segs) / 256.0);
