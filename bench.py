@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139265485, "b3f2ab34ccb157de"),
-    "cfg3": (2603261303, "b3f2ab34ccb157de"),
-    "cfg5": (5084373663, "b3f2ab34ccb157de"),
-    "wide": (1877109282, "b3f2ab34ccb157de"),
+    "cfg2": (139323564, "2470b03351e57230"),
+    "cfg3": (2608551109, "2470b03351e57230"),
+    "cfg5": (4163550728, "2470b03351e57230"),
+    "wide": (1877064671, "2470b03351e57230"),
 }
 
 WORKLOADS = {
