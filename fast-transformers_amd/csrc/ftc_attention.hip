@@ -22,6 +22,8 @@
 // before and after each one, and attn_bwd_finish_kernel, one more pass over dq and dk, adds the
 // prefix sums (those of the other segments, then of the other threads' runs, then its own run)
 // and multiplies by phi'.  Qf and Kf are recomputed there from q and k, which phi' needs anyway.
+// Rows of 64 values on the chain-parallel kernel need none of that (ftc_tph_kernel.h, GRAD: the scans take q, k, v
+// and g as they are and carry the prefix sums along): there attn_bwd_dots_kernel is all that runs beside them.
 #include "ftc_common.h"
 
 namespace ftc {
@@ -121,6 +123,33 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(
         float4 t = part[which][0][c];
         for (int i = 1; i < kRows; i++) t = t + part[which][i][c];
         if (has_e) *(float4 *)(sums + ((chain * nseg + seg) * 2 + which) * E + ce) = t;
+    }
+}
+
+// Only what the scans do not work out for themselves (scan_tph_gradients_kernel): dd and 1 / den of every
+// position, dense.  Two reads of a row and two words out: bound by memory.  Workgroups as above.
+__global__ __launch_bounds__(256) void attn_bwd_dots_kernel(Rows g, Rows out, Rows den, int H, int L, int M, int nseg,
+                                                            float *__restrict__ dd, float *__restrict__ rden) {
+    constexpr int kLanes = 16, kRows = 256 / kLanes;
+    const int h = blockIdx.x % H, seg = (blockIdx.x / H) % nseg, n = blockIdx.x / (H * nseg);
+    const int r = threadIdx.x / kLanes, c = threadIdx.x % kLanes;
+    const bool has_m = 4 * c < M;
+    const int cm = has_m ? 4 * c : 0;
+#pragma unroll
+    for (int p = 0; p < kSegment / kRows; p++) {
+        const int l = seg * kSegment + p * kRows + r;
+        const int lc = l < L ? l : L - 1;
+        const float4 gg = *(const float4 *)(g.ptr + n * g.sn + h * g.sh + lc * g.sl + cm);
+        const float4 o = *(const float4 *)(out.ptr + n * out.sn + h * out.sh + lc * out.sl + cm);
+        const float z = 1.0f / den.ptr[n * den.sn + h * den.sh + lc * den.sl];
+        float dot = has_m ? (gg.x * o.x + gg.y * o.y) + (gg.z * o.z + gg.w * o.w) : 0.f;
+#pragma unroll
+        for (int off = kLanes / 2; off > 0; off >>= 1) dot += __shfl_xor(dot, off, kLanes);
+        if (l < L && c == 0) {
+            const int64_t pos = ((int64_t)n * H + h) * L + l;
+            dd[pos] = -dot * z;
+            rden[pos] = z;
+        }
     }
 }
 
@@ -245,6 +274,13 @@ void launch_attention_backward_prep(const Operand &q, const Operand &k, const Op
     hipLaunchKernelGGL(kernel, dim3((unsigned)(N * H * nseg)), dim3(256), 0, stream,
                        rows_of(q), rows_of(k), rows_of(g), rows_of(out), rows_of(den), key_len, (int)H,
                        (int)L, E, M, nseg, Qf, Kf, gz, dd, sums);
+}
+
+void launch_attention_backward_dots(const Operand &g, const Operand &out, const Operand &den, int64_t N,
+                                    int64_t H, int64_t L, int M, float *dd, float *rden, hipStream_t stream) {
+    const int nseg = (int)attention_backward_segments(L);
+    hipLaunchKernelGGL(attn_bwd_dots_kernel, dim3((unsigned)(N * H * nseg)), dim3(256), 0, stream, rows_of(g),
+                       rows_of(out), rows_of(den), (int)H, (int)L, M, nseg, dd, rden);
 }
 
 void launch_attention_backward_finish(const Operand &q, const Operand &k, const int64_t *key_len,

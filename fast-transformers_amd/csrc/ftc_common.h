@@ -164,13 +164,26 @@ bool fused_attention_supported(const ScanDesc &scan, int64_t L);
 // rows of 128: whether a plan exists for the sizes (no workspace needed: 0 bytes)
 bool fused_attention_wide_covers(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F);
 int64_t fused_attention_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F);
+// The three gradient scans of the fused attention in one launch, straight from its inputs (fp32 rows of
+// 64 values; ftc_tph_kernel.h, GRAD): scans[i] is a scan of `kinds[i]` over the rows of q, k, v and grad_out
+// as the caller has them, `rows[i]` the rows of q (of k) whose phi' multiplies the gradient of q (of k).
+struct AttentionGradients {
+    const int64_t *key_lengths;  // as above
+    const float *dd, *rden;      // -(grad_out . out) / den and 1 / den, one per position
+    int kinds[kMfmaMaxScans];    // 1, 2, 3: the gradient of q, k, v
+    Operand rows[kMfmaMaxScans];
+};
+// Whether they run that way, and the workspace that they need then
+bool attention_gradients_take(const ScanDesc *scans, int nscans, const AttentionGradients &grads, int64_t N,
+                              int64_t H, int64_t L);
+int64_t attention_gradients_workspace_bytes(int64_t N, int64_t H, int64_t L, int nscans);
 // Runs scans[0..nscans) (all of the same row widths) in one launch.  `fused`: a single
 // forward scan in its fused attention form.  `may_chain_parallel` = false keeps the launch
 // off the chain-parallel kernel (column slices of a scan that it has declined as a whole).
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
               void *workspace, size_t workspace_bytes, hipStream_t stream,
               const FusedAttention *fused = nullptr, bool may_chain_parallel = true,
-              bool forced = false, bool odd = false);
+              bool forced = false, bool odd = false, const AttentionGradients *grads = nullptr);
 
 // Chains of a few positions (ftc_short.hip): scans of any widths and element types in one launch,
 // on the vector unit, without a workspace.
@@ -182,7 +195,10 @@ int short_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, h
 // of M floats), dd = -(g . out) / den (one float per position), and per (chain, segment of
 // positions) the totals of Kf and of dd Qf (`sums`: 2 E floats each).  finish: dq and dk, which
 // hold the scans' results, get the prefix sums that the denominator contributes and phi'.
+// dots: only dd and 1 / den, where the scans take the rest upon themselves (AttentionGradients).
 int64_t attention_backward_segments(int64_t L);
+void launch_attention_backward_dots(const Operand &g, const Operand &out, const Operand &den, int64_t N,
+                                    int64_t H, int64_t L, int M, float *dd, float *rden, hipStream_t stream);
 void launch_attention_backward_prep(const Operand &q, const Operand &k, const Operand &g,
                                     const Operand &out, const Operand &den, const int64_t *key_len,
                                     int64_t N, int64_t H, int64_t L, int E, int M, float *Qf,

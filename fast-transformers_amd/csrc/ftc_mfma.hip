@@ -753,6 +753,9 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
 // (rows of 128 values: the chain-parallel kernel alone)
 bool fused_wide(int64_t D, int64_t F) { return D > 64 || F > 64; }
 
+// (the attention's gradients with an exchange: another tile of state for the sums of rows)
+constexpr int64_t kGradStateRows = 128;
+
 bool fused_attention_supported(const ScanDesc &sd, int64_t L) {
     if (combo_of(sd) != kFFFF || sd.reverse || sd.initial.ptr || sd.final_.ptr) return false;
     if (!fused_wide(sd.a.width, sd.v.width))
@@ -818,9 +821,38 @@ bool fused_attention_wide_covers(int64_t N, int64_t H, int64_t L, int64_t D, int
     return fused_tp_plan(D, F, std::max<int64_t>(1, N * H), L, &nseg, &seg_chunks);
 }
 
+bool attention_gradients_take(const ScanDesc *scans, int nscans, const AttentionGradients &grads, int64_t N,
+                              int64_t H, int64_t L) {
+    if (!tph_takes_rows(64) || nscans < 1 || nscans > kMaxScans) return false;
+    // (a whole chain is addressed through one 32-bit descriptor)
+    auto in_place = [&](const void *ptr, int64_t sn, int64_t sh, int64_t sl, int dtype, int width) {
+        return dtype == FTC_F32 && width == 64 && mfma_operand_in_place(ptr, sn, sh, sl, dtype, width, L) &&
+               (L + 2 * kChunk) * std::max<int64_t>(sl, 64) * 4 < 0x7fffffffLL;
+    };
+    for (int i = 0; i < nscans; i++) {
+        for (const Operand *t : {&scans[i].a, &scans[i].b, &scans[i].v, &grads.rows[i]})
+            if (!in_place(t->ptr, t->stride_n, t->stride_h, t->stride_l, t->dtype, t->width)) return false;
+        const OperandOut &o = scans[i].out;
+        if (!in_place(o.ptr, o.stride_n, o.stride_h, o.stride_l, o.dtype, o.width)) return false;
+    }
+    int nseg = 0, seg_chunks = 0;
+    // (where the planner has those scans on the kernels that split L they stay there: they hold every value exactly,
+    // and chains of one to four chunks are faster so, N=32, H=32, L=64, forward and backward 133 us against 168)
+    tp_plan(64, 64, std::max<int64_t>(1, N * H), nscans, L, &nseg, &seg_chunks);
+    return nseg > 0;
+}
+
+int64_t attention_gradients_workspace_bytes(int64_t N, int64_t H, int64_t L, int nscans) {
+    int nseg = 0, seg_chunks = 0;
+    const int64_t chains = std::max<int64_t>(1, N * H);
+    tp_plan(64, 64, chains, nscans, L, &nseg, &seg_chunks);
+    return seg_chunks > 0 ? tp_exchange_workspace_bytes(chains * nscans, nseg, kGradStateRows) : 0;
+}
+
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
               void *workspace, size_t workspace_bytes, hipStream_t stream,
-              const FusedAttention *fused, bool may_chain_parallel, bool forced, bool odd) {
+              const FusedAttention *fused, bool may_chain_parallel, bool forced, bool odd,
+              const AttentionGradients *grads) {
     if (nscans < 1 || nscans > kMaxScans) return fail(FTC_ERR_INVALID, "bad scan count");
     int D, F;
     widest_rows(scans, nscans, &D, &F);
@@ -842,7 +874,9 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     if (fused_tp && !wide_rows && tpx_seg_chunks > 0 && !plan_only() &&
         (int64_t)workspace_bytes < tp_exchange_workspace_bytes(chains, tpx_nseg, fused_tp_state_rows(D)))
         fused_tp = false, tpx_nseg = tpx_seg_chunks = 0;
-    const bool tp_shape = !fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd);
+    if (grads && !attention_gradients_take(scans, nscans, *grads, N, H, L))
+        return fail(FTC_ERR_UNSUPPORTED, "no kernel takes these gradients straight from their inputs");
+    const bool tp_shape = grads || (!fused && may_chain_parallel && mfma_tp_takes(scans, nscans, N, H, L, forced, odd));
     const int64_t fblocks = tp_shape || wide_rows ? tp_fblocks(F) : 1;
     const int64_t blocks = odd && forced ? column_blocks(scans, nscans) : nscans * fblocks;
     if (fused_tp && tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
@@ -866,7 +900,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         pl.seg_len = tpx_seg_chunks * kChunk;
         pl.waves = chains * pl.nseg;
         pl.workspace_bytes = tp_exchange_workspace_bytes(chains * blocks, pl.nseg,
-                                                         fused_tp ? fused_tp_state_rows(D) : D);
+                                                         fused_tp ? fused_tp_state_rows(D) : grads ? kGradStateRows : D);
     } else if (tp) {  // one workgroup per chain segment, nothing to exchange
         pl.nseg = tp_segment_starts((L + kChunk - 1) / kChunk, tp_nseg, tp_start);
         pl.seg_len = (int)L;
@@ -909,6 +943,11 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         o.so_sn = sd.final_.stride_n, o.so_sh = sd.final_.stride_h, o.so_sd = sd.final_.stride_d;
         if (fused && fused->denominators)  // (the fused form has no state to hand out)
             o.s_out = fused->denominators, o.so_sn = fused->den_sn, o.so_sh = fused->den_sh, o.so_sd = 0;
+        if (grads) {  // (nor have these)
+            const Operand &t = grads->rows[i < nscans ? i : 0];
+            o.pad = grads->kinds[i < nscans ? i : 0];
+            o.s0 = (const float *)t.ptr, o.s0_sn = t.stride_n, o.s0_sh = t.stride_h, o.s0_sd = row_stride(t.stride_l, o.f);
+        }
         max_stride = std::max(max_stride, std::max(std::max(sd.a.stride_l, sd.b.stride_l),
                                                    std::max(sd.v.stride_l, sd.out.stride_l)));
     }
@@ -917,9 +956,10 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         return fail(FTC_ERR_UNSUPPORTED, "segment too long for 32-bit offsets");
     args.L = L;
     args.eps = fused ? fused->eps : 0.f;
-    args.key_len = fused ? fused->key_lengths : nullptr;
+    args.key_len = fused ? fused->key_lengths : grads ? grads->key_lengths : nullptr;
+    args.row_dd = grads ? grads->dd : nullptr, args.row_rden = grads ? grads->rden : nullptr;
 #ifdef FTC_TIMELINE
-    if (tp && !fused)  // tuning aid: where the chain-parallel kernel writes its time stamps
+    if (tp && !fused && !grads)  // tuning aid: where the chain-parallel kernel writes its time stamps
         if (const char *env = getenv("FTC_STAMP_PTR"))  // (a build for measurements only)
             args.key_len = (const int64_t *)(uintptr_t)strtoull(env, nullptr, 0);
 #endif
@@ -983,6 +1023,8 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
             launch_scan_tp_norm(workspace, args, stream);
         else if (mixed)
             launch_scan_tp_mixed(workspace, args, stream);
+        else if (grads)
+            launch_scan_tph_gradients(workspace, args, stream);
         else if (half_pieces)
             launch_scan_tph(workspace, args, odd, stream);
         else

@@ -413,10 +413,11 @@ struct ScanOperands {
     int64_t v_sn, v_sh, v_sl;
     int64_t o_sn, o_sh, o_sl;
     int32_t rev;  // 0: j <= l, walk up; 1: j >= l, walk down
-    int32_t pad;  // kRowsBf16* bits (read by the kernel that takes rows of either type scan by scan)
+    int32_t pad;  // kRowsBf16* bits (read by the kernel that takes rows of either type scan by scan) or a GradRole
     int32_t d, f;  // widths of the rows (the chain-parallel kernels): a, b and v, out
     // optional D x F fp32 states per chain (null: none): the state the scan starts from and
     // the state after its last position; strides in elements, unit stride along F
+    // (backward of the fused attention: s0 are the rows of q or k, s0_sd apart, for phi')
     const float *s0;
     float *s_out;
     int64_t s0_sn, s0_sh, s0_sd;
@@ -471,6 +472,8 @@ struct ScanArgs {
     // fused attention form of the workgroup kernel only (ftc_wg_kernel.h, NORM)
     float eps;               // added to the denominator
     const int64_t *key_len;  // keys per batch entry, N values on the device; nullptr: all L
+    // backward of the fused attention only (scan_tph_gradients_kernel): dd and 1 / den, one per position
+    const float *row_dd, *row_rden;
     // chain-parallel kernel only (ftc_tp_kernel.h): segment s of a chain is chunks
     // tp_start[s] .. tp_start[s + 1] - 1 (starts are multiples of kTpAhead)
     int32_t tp_start[kMaxTpSegments + 1];

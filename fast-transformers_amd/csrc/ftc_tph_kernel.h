@@ -171,6 +171,7 @@ __device__ __forceinline__ uint32_t wave_max(float m) {  // (the bits of the lar
 // The running ceilings of a, b and v as one wavefront knows them (wave-uniform).
 struct Ceilings {
     uint32_t Ea, Wb, Wv;
+    uint32_t Ed = 0;  // (gradients of the attention) the biased exponent of the position's largest dd
     __device__ __forceinline__ int Eb() const { return (int)(Wb & 0xffffu); }
     __device__ __forceinline__ int Ev() const { return (int)(Wv & 0xffffu); }
     __device__ __forceinline__ float scale_a() const { return pow2_field(259 - (int)Ea); }
@@ -179,15 +180,23 @@ struct Ceilings {
     // exponent of the state's units, and of a chunk's output units (a x state)
     __device__ __forceinline__ int state_exp() const { return (int)((Wb + Wv) & 0xffffu) - 264; }
     __device__ __forceinline__ int out_exp() const { return (int)(Ea + ((Wb + Wv) & 0xffffu)) - 396; }
+    // dd as weights: the field of the power of two that brings them below 16
+    __device__ __forceinline__ int weight_field() const { return max(1, min(254, 257 - (int)Ed)); }
+    // dd in the units of Pt: 2^up; beyond 2^14 of them the quadrants take units 2^shift as large
+    __device__ __forceinline__ int dd_up() const { return 264 - (int)Ea - Eb(); }
+    __device__ __forceinline__ int dd_shift() const { return Ed == 255u ? 0 : max(0, (int)Ed - 140 + dd_up()); }
 };
 typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
-// The slot of a position is that of its LDS buffer: words (a, b, v, unused).  The words of b
+typedef __attribute__((address_space(3))) f32x4 lds_fvec4;
+// The slot of a position is that of its LDS buffer: words (a, b, v, and dd, tagged as that of a).  The words of b
 // and v hold ceilings that only ever rise (a stale one is harmless: it is below the running
 // ceiling that every wavefront carries).  The word of a holds the ceiling of the rows of that
 // one position, tagged with the position's number in the upper 24 bits, so that what the
 // slot held three positions ago is always smaller and needs no clearing.
+template <bool GRAD = false>
 __device__ __forceinline__ void read_slot(const lds_u32_t *slots, int k, Ceilings &c) {
     const u32x4 s = *(const lds_vec4 *)(slots + 4 * k);
+    if (GRAD) c.Ed = (uint32_t)__builtin_amdgcn_readfirstlane(s.w) & 0xffu;
     c.Ea = max(kExpFloor, (uint32_t)__builtin_amdgcn_readfirstlane(s.x) & 0xffu);
     c.Wb = max(c.Wb, (uint32_t)__builtin_amdgcn_readfirstlane(s.y));
     c.Wv = max(c.Wv, (uint32_t)__builtin_amdgcn_readfirstlane(s.z));
@@ -217,6 +226,21 @@ __device__ __forceinline__ void raise_slot(lds_u32_t *slots, int k, int pos, con
     }
 }
 
+// GRAD: the gradients of the fused attention (equations in ftc_attention.hip) straight from its inputs:
+// a scan's rows become phi(q), phi(k) [j < key_len] and gz = g / den as the producers first touch them, and
+// the normaliser's share of a gradient, whose sums are prefix sums of rows weighted by w = 1 (for dq, which
+// has the factor dd_l outside) or w_l = dd_l (for dk), is part of the walk:
+//  * inside a chunk dd is added to the quadrants of Pt, (gz_l . v_j + dd_l) being the factor of both sums (dd
+//    beyond 2^14 of the quadrant's units is rare, and takes the chunk's result to larger units);
+//  * Z = sum of w_l v_l over the positions before the chunk is kept in fp32, 16 columns a wavefront: one more
+//    product of v^T with the weights in two pieces, three matrix instructions a chunk, and one fma per value
+//    of the result.
+// phi'(q) or phi'(k) multiplies the result on its way out.  A consumer's stream of instructions is what a chunk
+// waits for here, so whatever can be is done by the producers: they leave dd, its pieces and phi' in LDS
+// (N=10, H=8, L=4096, with all of that in the consumers 320 us, this way 228; the dense copies of phi(q),
+// phi(k), gz that the scans read before, the scans and a pass over their results for the rest: 370).
+enum GradRole { kGradQueries = 1, kGradKeys = 2, kGradValues = 3 };
+
 // KS: groups of 32 rows of the state (1: a state of up to 32 rows, which skips the matrix
 // instructions and fragment reads of the empty half).
 // ODD: fp32 rows of any width on 4-byte boundaries.  The requests stay 16 bytes per lane (the
@@ -225,8 +249,9 @@ __device__ __forceinline__ void raise_slot(lds_u32_t *slots, int k, int pos, con
 // look-ahead first touches them, and stores such a quad word by word.  Measured against dense
 // zero-padded copies of the operands and results (8 x 16 chains, L=4096, 50 x 50, forward + backward):
 // 940 -> 387 us; a chunk costs what one of 64 x 64 does.
-template <int KS, bool ODD>
-__global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
+template <int KS, bool ODD, bool GRAD>
+__device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, const ScanArgs &p) {
+    static_assert(!GRAD || (KS == 2 && !ODD), "the gradients' form takes 64 x 64 states");
     constexpr int D = 64, F = 64;              // one block of state rows and of output columns
     constexpr int T = 512;                     // producer lanes (eight wavefronts)
     constexpr int PF = kTpAhead;               // chunks requested ahead
@@ -248,9 +273,16 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     __shared__ __align__(16) char pieces_mem[3 * kBufBytes];
     __shared__ __align__(16) char pt_mem[3 * 2 * kTileP];
     __shared__ __align__(16) uint32_t slot_mem[16];
+    // GRAD, for the rows in each of the three buffers: dd, dd in the units of Pt, the weights' two pieces
+    constexpr int kDdUnits = 4 * kChunk, kWeights = 8 * kChunk, kDdBytes = 12 * kChunk;
+    __shared__ __align__(16) char dd_mem[GRAD ? 3 * kDdBytes : 1];
+    // ... and phi' of the rows of q or k that belong to the result's, piece p of row r in slot p ^ (r mod 16)
+    constexpr int kTileX = kChunk * F * 4;
+    __shared__ __align__(16) char x_mem[GRAD ? 3 * kTileX : 1];
     lds_char *const unit_pc = (lds_char *)pieces_mem;
     lds_char *const pt_pc = (lds_char *)pt_mem;
     lds_u32_t *const slots = (lds_u32_t *)slot_mem;
+    lds_char *const dd_pc = (lds_char *)dd_mem, *const x_pc = (lds_char *)x_mem;
 
     // ---- which chain (as in scan_tp_kernel) ----
     const uint32_t nseg = (uint32_t)p.nseg;
@@ -306,6 +338,11 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     constexpr uint32_t kNoRow = 0x80000000u;  // an offset outside every descriptor
     auto chunk_row0 = [&](int c) -> int { return REV ? rows - kChunk * (c + 1) : kChunk * c; };
     if (tid < 16) slot_mem[tid] = 0;
+    // (what is read before the first position is zero, and so is what the gradient of v reads)
+    if (GRAD && tid < 3 * kDdBytes / 4) *(lds_u32_t *)(dd_pc + 4 * tid) = 0;
+    const int role = op.pad;  // GRAD
+    // (GRAD: rows of k at or beyond the key length count as zero)
+    const int key_rows = GRAD && p.key_len ? (int)max((int64_t)0, min((int64_t)rows, p.key_len[n])) : rows;
     Ceilings ce{kExpFloor, kExpOfZeros, kExpOfZeros};
     // Position k of the walk goes through LDS buffer (B0 + k) % 3 (pieces, Pt and slot), with B0
     // such that the first chunk of the walk proper has buffer 0: the consumers' loop over
@@ -317,7 +354,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     // p.key_len (FTC_STAMP_PTR), written by lane 0 of consumer 0 (0 .. 15) and of producer 0
     // (16 .. 31) in the fifth chunk of the walk proper
     typedef __attribute__((address_space(1))) uint64_t gu64;
-    const bool stamp_on = p.key_len != nullptr && w == 0 && lane == 0;
+    const bool stamp_on = !GRAD && p.key_len != nullptr && w == 0 && lane == 0;
     gu64 *const stamp_base = (gu64 *)p.key_len + blockIdx.x * 32 + (producer ? 16 : 0);
     // ... and behind those, 64 stamps per workgroup: consumer 0 after the barrier of every chunk
     gu64 *const chunk_stamps = (gu64 *)p.key_len + gridDim.x * 32 + blockIdx.x * 64;
@@ -368,7 +405,19 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         };
         struct Raw {
             u32x4 a, b, v;
+            u32x4 x;            // GRAD: q or k
+            uint32_t rden, dd;  // GRAD
         };
+        const uint32_t x_slb = GRAD ? (uint32_t)op.s0_sd * 4 : 0u, x_goff = (uint32_t)prow * x_slb + 16u * pc4;
+        const bool has_x = GRAD && role != kGradValues;
+        const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(has_x ? op.s0 + (int64_t)n * op.s0_sn + (int64_t)h * op.s0_sh : nullptr), 0,
+            has_x ? (rows - 1) * x_slb + Dw * 4 : 0u, kRsrcFlags);
+        // GRAD: 1 / den and dd of the row
+        const __amdgpu_buffer_rsrc_t rden_rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(GRAD ? p.row_rden + (int64_t)chain * rows : nullptr), 0, rows * 4, kRsrcFlags);
+        const __amdgpu_buffer_rsrc_t dd_rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(GRAD ? p.row_dd + (int64_t)chain * rows : nullptr), 0, rows * 4, kRsrcFlags);
         Raw raw[PF];
         // Every request is made every time, whether its rows exist or not (a chunk walked for
         // its state alone needs no rows of a; positions past the end of the walk have no
@@ -382,11 +431,56 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
             r.a = __builtin_amdgcn_raw_buffer_load_b128(a_rs, ab_in ? a_goff + (uint32_t)row0_x * a_slb : kNoRow, 0, 0);
             r.b = __builtin_amdgcn_raw_buffer_load_b128(b_rs, ab_in ? b_goff + (uint32_t)row0 * b_slb : kNoRow, 0, 0);
             r.v = __builtin_amdgcn_raw_buffer_load_b128(v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, 0, 0);
+            if constexpr (GRAD) {
+                r.x = __builtin_amdgcn_raw_buffer_load_b128(x_rs, has_x ? x_goff + (uint32_t)row0_x * x_slb : kNoRow, 0, 0);
+                r.rden = __builtin_amdgcn_raw_buffer_load_b32(rden_rs, 4u * (uint32_t)(prow + row0), 0, 0);
+                r.dd = __builtin_amdgcn_raw_buffer_load_b32(dd_rs, 4u * (uint32_t)(prow + row0), 0, 0);
+            }
+        };
+        // GRAD: the rows as the scan takes them.  phi(0) is one, so rows that are not there are
+        // cleared (a scalar test: most chunks lie wholly inside).
+        auto feature = [&](u32x4 &x, int row0, int limit) {
+            x = feature_quad(x);
+            if (row0 < 0 || row0 + kChunk > limit) {
+                if ((uint32_t)(row0 + prow) >= (uint32_t)limit) x = u32x4{0, 0, 0, 0};
+            }
+        };
+        auto over_den = [](u32x4 &x, uint32_t rden) {
+            const float z = __uint_as_float(rden);
+            x = u32x4{__float_as_uint(z * __uint_as_float(x.x)), __float_as_uint(z * __uint_as_float(x.y)),
+                      __float_as_uint(z * __uint_as_float(x.z)), __float_as_uint(z * __uint_as_float(x.w))};
+        };
+        auto as_taken = [&](Raw &r, int v) {  // v: position of the walk
+            const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
+            if (role == kGradQueries) {
+                over_den(r.a, r.rden);
+                feature(r.v, row0, key_rows);
+            } else if (role == kGradKeys) {
+                over_den(r.b, r.rden);
+                feature(r.v, row0, rows);
+            } else {
+                feature(r.a, v >= n1 ? row0 : -2 * kChunk, key_rows);
+                feature(r.b, row0, rows);
+                over_den(r.v, r.rden);
+            }
         };
         // the largest magnitudes of the rows of a position against the ceilings (rows that
         // were not asked for read as zeros); k: that position's slot
         auto look_ahead = [&](Raw &r, int k, int pos) {
             own_words(r.a, ab_own), own_words(r.b, ab_own), own_words(r.v, v_own);
+            if constexpr (GRAD) {
+                as_taken(r, pos);
+                if (has_x) {  // (rows of 16 lanes share a row of the operands)
+                    const uint32_t d = r.dd & 0x7fffffffu;
+                    const uint32_t m = scalar_max(scalar_max((uint32_t)__builtin_amdgcn_readlane((int)d, 0),
+                                                             (uint32_t)__builtin_amdgcn_readlane((int)d, 16)),
+                                                  scalar_max((uint32_t)__builtin_amdgcn_readlane((int)d, 32),
+                                                             (uint32_t)__builtin_amdgcn_readlane((int)d, 48)));
+                    if (lane == 0)
+                        __hip_atomic_fetch_max(slots + 4 * k + 3, ((uint32_t)(pos + 1) << 8) | m >> 23,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+            }
             raise_slot(slots, k, pos, ce, max_abs4(r.a, 0.f), max_abs4(r.b, 0.f), max_abs4(r.v, 0.f), lane);
         };
         // A position of the walk goes to its LDS buffer through register set (position % PF).
@@ -396,6 +490,28 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
             if (own) cut_quad_to_lds(r.a, ce.scale_a(), pc, kTileA, a_waddr);
             cut_quad_to_lds(r.b, ce.scale_b(), pc + kOffB, kTileA, b_waddr);
             cut_quad_to_lds(r.v, ce.scale_v(), pc + kOffV, kTileV, v_waddr);
+            if constexpr (GRAD) {
+                if (has_x) {
+                    if (own) {
+                        auto slope = [](uint32_t x) -> uint32_t {  // phi'(x); NaN: one (gz is NaN then)
+                            return __float_as_uint(fminf(1.f, __builtin_amdgcn_exp2f(__uint_as_float(x) * 1.44269502f)));
+                        };
+                        *(lds_vec4 *)(x_pc + buf * kTileX + prow * F * 4 + 16 * (pc4 ^ (prow & 15))) =
+                            u32x4{slope(r.x.x), slope(r.x.y), slope(r.x.z), slope(r.x.w)};
+                    }
+                    const float dd = __uint_as_float(r.dd), wt = dd * pow2_field(ce.weight_field());
+                    _Float16 hi = (_Float16)wt, lo = (_Float16)(wt - (float)hi);
+                    if (role == kGradQueries) hi = (_Float16)1.f, lo = (_Float16)0.f;
+                    if (pc4 == 0) {
+                        lds_char *const d = dd_pc + buf * kDdBytes;
+                        *(lds_f32 *)(d + 4 * prow) = dd;
+                        *(lds_f32 *)(d + kDdUnits + 4 * prow) = ce.dd_shift() == 0 ? __builtin_amdgcn_ldexpf(dd, ce.dd_up()) : 0.f;
+                        *(lds_u16 *)(d + kWeights + 2 * prow) = __builtin_bit_cast(uint16_t, hi);
+                        *(lds_u16 *)(d + kWeights + 2 * (kChunk + prow)) = __builtin_bit_cast(uint16_t, lo);
+                    }
+                }
+                if (!own) asm volatile("" ::"v"(r.x));
+            }
             if (!own) asm volatile("" ::"v"(r.a));
         };
 #pragma unroll
@@ -409,7 +525,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         int buf = B0;
         auto step = [&](int v, int j, bool own) {
             if (own && v == n1 + 4) FTC_STAMP(0);
-            read_slot(slots, buf, ce);
+            read_slot<GRAD>(slots, buf, ce);
             look_ahead(raw[(j + 1) % PF], next_buf(buf), v + 1);
             if (own && v == n1 + 4) FTC_STAMP(1);
             cut(raw[j], buf, own);
@@ -434,7 +550,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
 #pragma unroll
         for (int j = 0; j < PF - 1; j++) {
             if (v + j > nwalk) return;
-            read_slot(slots, buf, ce);
+            read_slot<GRAD>(slots, buf, ce);
             look_ahead(raw[(j + 1) % PF], next_buf(buf), v + j + 1);
             cut(raw[j], buf, true);
             buf = buf == 2 ? 0 : buf + 1;
@@ -525,6 +641,37 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         }
     };
 
+    // GRAD: Z, the sum of w_l v_l over the positions before the chunk (w = 1 or dd), in this lane's four
+    // columns of the result
+    const bool sums_rows = GRAD && role != kGradValues;
+    f32x4 Z = {0.f, 0.f, 0.f, 0.f}, Zc = {0.f, 0.f, 0.f, 0.f};  // Zc: the chunk's sum, times 2^-z_exp
+    int z_exp = 0;
+    // the chunk's sum is one more product of v^T, with the weights w in all 16 columns of the second operand
+    auto weights_exp = [&](const Ceilings &c) -> int {  // (the unit of that product)
+        return (role == kGradQueries ? 0 : 127 - c.weight_field()) + c.Ev() - 132;
+    };
+    auto sum_chunk = [&](int b, const Frag (&vfx)[2]) {  // (into Zc; b: the buffer)
+        const lds_char *const at = dd_pc + b * kDdBytes + kWeights + 16 * g;
+        const Frag hi = lds_frag16(at), lo = lds_frag16(at + 2 * kChunk);
+        Zc = mfma16h(vfx[1], hi, f32x4{0.f, 0.f, 0.f, 0.f});
+        Zc = mfma16h(vfx[0], lo, Zc);
+        Zc = mfma16h(vfx[0], hi, Zc);
+    };
+    // dd in the units of Pt (added to a quadrant when the products are summed: a sum that starts from dd is
+    // rounded to dd's last place six times over, and dq came out up to a tenth further from float64)
+    const int dd_addr = kDdUnits + (role == kGradQueries ? 4 * (16 * ih + ln) : 4 * (16 * jh + 4 * g));
+    auto dd_of_quadrant = [&](int b) -> f32x4 {
+        if (role == kGradQueries) {
+            const float d = *(const lds_f32 *)(dd_pc + b * kDdBytes + dd_addr);
+            return f32x4{d, d, d, d};
+        }
+        return *(const lds_fvec4 *)(dd_pc + b * kDdBytes + dd_addr);
+    };
+    auto add_chunk = [&]() {
+#pragma unroll
+        for (int r = 0; r < 4; r++) Z[r] += __builtin_amdgcn_ldexpf(Zc[r], z_exp);
+    };
+
     Frag af[2][2][2], bfr[2][2], bt[4][2], vf[2];
     // row-major fragment number i of a chunk (12: b for the quadrant first, then a)
     auto rm_frag = [&](const lds_char *pc, int i) {
@@ -549,20 +696,26 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     wg_barrier();  // the slots are zero
     wg_barrier();  // the slot of position 0 is complete
     wg_barrier();  // barrier 0: position 0 is cut
-    read_slot(slots, B0, ce);
+    read_slot<GRAD>(slots, B0, ce);
     Ucur = ce.state_exp();
-    if (op.s0 && !exchange) add_caller_state();
+    if (!GRAD && op.s0 && !exchange) add_caller_state();
     if (n1 > 0) {
         // ---- the first n1 positions of the walk: state update only ----
         // The loop is skewed by one position: while the matrix instructions of position k - 1
         // run, the fragments of position k arrive in the other set of registers.
         int U_prev = Ucur;                 // units of the fragments about to be multiplied
         Frag bt2[4][2] = {}, vf2[2] = {};  // (the first round multiplies zeros)
+        // GRAD: the position before, whose dd are in the buffer before (nothing cuts that one now)
+        auto sum_before = [&](int b, const Frag (&vfx)[2]) {
+            sum_chunk(b == 0 ? 2 : b - 1, vfx);
+            add_chunk();
+        };
+        z_exp = 0;  // (zeros)
         for (int c = 0; c < n1; c += PF) {
 #pragma unroll
             for (int j = 0; j < PF; j++) {
                 const lds_char *pc = unit_pc + buf * kBufBytes;
-                read_slot(slots, buf, ce);  // the ceilings of position c + j
+                read_slot<GRAD>(slots, buf, ce);  // the ceilings of position c + j
                 if (U_prev != Ucur) {       // the ceilings rose: the state shrinks
                     scale_state(Ucur - U_prev);
                     Ucur = U_prev;
@@ -578,6 +731,10 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
                         if (i < 10) tr_frag_into(bt2, vf2, pc, i);
                     }
                     __builtin_amdgcn_sched_barrier(0);
+                }
+                if (GRAD && sums_rows) {
+                    sum_before(buf, j % 2 == 0 ? vf2 : vf);
+                    z_exp = weights_exp(ce);
                 }
                 U_prev = ce.state_exp();
                 buf = next_buf(buf);
@@ -596,11 +753,13 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
 #pragma unroll
         for (int i = 0; i < 12; i++) {
             if ((i % 4) / 2 < KS) S[i % 4] = mfma16h(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[i % 4]);
-            rm_frag(unit_pc + buf * kBufBytes, i);  // our own first chunk is cut
+            if (!GRAD) rm_frag(unit_pc + buf * kBufBytes, i);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
-        read_slot(slots, buf, ce);  // the ceilings of our own first chunk
-    } else {
+        if (GRAD && sums_rows) sum_before(buf, vf2);
+        Zc = f32x4{0.f, 0.f, 0.f, 0.f};
+        read_slot<GRAD>(slots, buf, ce);  // the ceilings of our own first chunk
+    } else if (!GRAD) {
 #pragma unroll
         for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
     }
@@ -608,10 +767,16 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         // ---- the sum of this segment's rows goes out, the state before the segment comes in ----
         const uint32_t total_units = (uint32_t)p.total_waves;
         gfloat *const sums = (gfloat *)(hdr + kControlBytes / 4);
-        StateExchange<1, 1> xch(flags, sums, 4u * total_units,
+        constexpr int DX = GRAD ? 2 : 1;  // (Z rides along in a tile of its own)
+        StateExchange<DX, 1> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);
-        f32x16 Sx[1][1], X[1][1];
+        f32x16 Sx[DX][1], X[DX][1];
+        if (GRAD) {
+            Sx[DX - 1][0] = f32x16{};
+#pragma unroll
+            for (int r = 0; r < 4; r++) Sx[DX - 1][0][r] = Z[r];
+        }
 #pragma unroll
         for (int dt = 0; dt < 4; dt++)
 #pragma unroll
@@ -627,7 +792,15 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         for (int dt = 0; dt < NT; dt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) S[dt][r] = __builtin_amdgcn_ldexpf(X[0][0][4 * dt + r], -Ucur);
-        if (op.s0) add_caller_state();
+        if (GRAD) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) Z[r] = X[DX - 1][0][r];
+        }
+        if (!GRAD && op.s0) add_caller_state();
+    }
+    if (GRAD) {  // (not before: two tiles are exchanged, and 48 registers of fragments beside them spilled)
+#pragma unroll
+        for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
     }
     // ---- the walk proper ----
     // `ce` holds the ceilings of the chunk at hand, Ucur the units of S.  dU < 0: the
@@ -681,9 +854,21 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
     for (int x = 0; x < 2; x++) O[x] = f32x4{0.f, 0.f, 0.f, 0.f};
     int Xo = 0;
     uint32_t o_off = 0x80000000u;
+    int o_row0 = 0, o_buf = 0;  // GRAD
     auto store_rows = [&](int x) {
-        const float y0 = __builtin_amdgcn_ldexpf(O[x][0], Xo), y1 = __builtin_amdgcn_ldexpf(O[x][1], Xo),
-                    y2 = __builtin_amdgcn_ldexpf(O[x][2], Xo), y3 = __builtin_amdgcn_ldexpf(O[x][3], Xo);
+        float y0 = __builtin_amdgcn_ldexpf(O[x][0], Xo), y1 = __builtin_amdgcn_ldexpf(O[x][1], Xo),
+              y2 = __builtin_amdgcn_ldexpf(O[x][2], Xo), y3 = __builtin_amdgcn_ldexpf(O[x][3], Xo);
+        if (GRAD && sums_rows) {
+            const int row = 16 * (x ^ ih) + ln;
+            const f32x4 slope = *(const lds_fvec4 *)(x_pc + o_buf * kTileX + row * F * 4 + 16 * ((4 * w + g) ^ ln));
+            const float dd = *(const lds_f32 *)(dd_pc + o_buf * kDdBytes + 4 * row), u = role == kGradQueries ? dd : 1.f;
+            y0 = fmaf(u, Z[0], y0) * slope[0], y1 = fmaf(u, Z[1], y1) * slope[1];
+            y2 = fmaf(u, Z[2], y2) * slope[2], y3 = fmaf(u, Z[3], y3) * slope[3];
+            if (role == kGradKeys && o_row0 + kChunk > key_rows) {  // (rows beyond the key length)
+                const bool live = o_row0 + row < key_rows;
+                y0 = live ? y0 : 0.f, y1 = live ? y1 : 0.f, y2 = live ? y2 : 0.f, y3 = live ? y3 : 0.f;
+            }
+        }
         const uint32_t at = o_in ? o_off + o_lane[x] : kNoRow;
         buffer_store_out(o_rs, at, y0, y1, y2, y3, (float *)nullptr);
         if (o_straddles) {
@@ -695,6 +880,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         }
     };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    int z_exp_next = 0;
     // One chunk, in LDS buffer B (a compile-time number, so that every LDS access of the body
     // has its buffer in the instruction's immediate offset).  Sums that end in one place are
     // chained through one accumulator, with other matrix instructions in between: Ot_w =
@@ -706,6 +892,9 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         lds_char *const ptc = pt_pc + B * (2 * kTileP);
         Frag pf[2][2];
         f32x4 P;  // (cleared by the first matrix instruction of its sum)
+        f32x4 P_dd = zero;  // GRAD
+        const int shift = GRAD && sums_rows ? ce.dd_shift() : 0;
+        if (GRAD && sums_rows) z_exp_next = weights_exp(ce);
         if (c == c0 + 4) FTC_STAMP(0);
         __builtin_amdgcn_sched_barrier(0);
         // phase 1: (1) the quadrant in turn with (2b) Ot_w = S_w^T a^T for rows 0 .. 31 of
@@ -715,12 +904,16 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         for (int i = 0; i < 6; i++) {
             const int m = i % 3, ks = i / 3, x = i % 2, mo = i / 2;
             if (i == 0) store_rows(0);
-            if (i == 1) store_rows(1);
+            if (GRAD && i == 3) P_dd = dd_of_quadrant(B);
+            if (i == 1) {
+                store_rows(1);
+                if (GRAD && sums_rows) add_chunk();  // (the rows before this chunk are all summed)
+            }
             if (ks < KS) P = mfma16h(bfr[ks][kPa[m]], af[0][ks][kPb[m]], i == 0 ? zero : P);
             O[x] = mfma16h(sf[0][kPa[mo]], af[x][0][kPb[mo]], mo == 0 ? zero : O[x]);
             if ((i == 1 || i == 3) && KS > 1) cut_s(1, i / 2, B == 0);
             tr_frag_into(bt, vf, pc, i);
-            if (i < 4) tr_frag_into(bt, vf, pc, 6 + i);
+            if (!GRAD && i < 4) tr_frag_into(bt, vf, pc, 6 + i);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (c == c0 + 4) FTC_STAMP(1);
@@ -743,9 +936,19 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         for (int i = 0; i < 6; i++) {
             const int x = i % 2, m = i / 2;
             if (KS > 1) O[x] = mfma16h(sf[1][kPa[m]], af[x][1][kPb[m]], O[x]);
+            if (GRAD && i >= 2) tr_frag_into(bt, vf, pc, 4 + i);  // (phase 1 has no registers for them)
             S[i % 2] = mfma16h(bt[i % 2][kPa[m]], vf[kPb[m]], S[i % 2]);
             if (i == 1) {
                 uint32_t h0, l0, h1, l1;
+                if (GRAD) P += P_dd;
+                if (GRAD && shift != 0) {  // (that was zero)
+                    const lds_char *const d = dd_pc + B * kDdBytes + dd_addr - kDdUnits;
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        P[r] = __builtin_amdgcn_ldexpf(P[r], -shift) +
+                               __builtin_amdgcn_ldexpf(*(const lds_f32 *)(d + (role == kGradQueries ? 0 : 4 * r)),
+                                                       ce.dd_up() - shift);
+                }
 #pragma unroll
                 for (int r = 0; r < 4; r++) P[r] = keep[r] ? P[r] : 0.f;
                 cut_quad_f16_unscaled(P[0], P[1], P[2], P[3], h0, h1, l0, l1);
@@ -768,12 +971,22 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         for (int x = 0; x < 2; x++)
 #pragma unroll
             for (int k = 0; k < 2; k++) pf[x][k] = lds_frag16(ptc + k * kTileP + pt_raddr[x]);
-        const int Xc = ce.out_exp();
+        const int Xc = ce.out_exp() + shift;
         const u32x4 slot_next = *(const lds_vec4 *)(slots + 4 * BN);
         if (s_cut != 0) {  // (rare: the state has grown beyond 2^14 units)
             const float r_cut = pow2_field(127 + s_cut);
             O[0] *= r_cut;
             O[1] *= r_cut;
+        }
+        if (GRAD && shift != 0) {
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) O[x][r] = __builtin_amdgcn_ldexpf(O[x][r], -shift);
+        }
+        if (GRAD && sums_rows) {
+            sum_chunk(B, vf);
+            z_exp = z_exp_next;
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -788,6 +1001,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
         ce.Ea = max(kExpFloor, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.x) & 0xffu);
         ce.Wb = max(ce.Wb, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.y));
         ce.Wv = max(ce.Wv, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.z));
+        if (GRAD) ce.Ed = (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.w) & 0xffu;
         // (dU > 0: small values after nothing but zeros; the state's units fall, so s rises)
         dU = Ucur - ce.state_exp();
         s += max(dU, 0);
@@ -803,6 +1017,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
             __builtin_amdgcn_sched_barrier(0);
         }
         o_off = (uint32_t)chunk_row0(c) * o_slb;
+        o_row0 = chunk_row0(c), o_buf = B;
         Xo = Xc;
         if (c == c0 + 4) FTC_STAMP(6);
     };
@@ -822,7 +1037,7 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
 #ifdef FTC_TIMELINE
     if (stamp_on) stamp_base[13] = __builtin_amdgcn_s_memtime();
 #endif
-    if (op.s_out && seg == (int)nseg - 1) {
+    if (!GRAD && op.s_out && seg == (int)nseg - 1) {
         float *base =
             op.s_out + (int64_t)n * op.so_sn + (int64_t)h * op.so_sh + F * fb + 16 * w + ln;
 #pragma unroll
@@ -852,6 +1067,11 @@ __global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__
                 __hip_atomic_store(hdr + kHdrDone, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+}
+
+template <int KS, bool ODD>
+__global__ __launch_bounds__(768, 3) void scan_tph_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
+    scan_tph_body<KS, ODD, false>(ws_ptr, p);
 }
 
 }  // namespace mfma

@@ -758,6 +758,8 @@ void launch_scan_tp_norm(void *ws, const ScanArgs &args, hipStream_t stream);
 void launch_scan_tp_mixed(void *ws, const ScanArgs &args, hipStream_t stream);
 // the same on the fp16 matrix path (ftc_tph_kernel.h): states of up to 64 rows
 void launch_scan_tph(void *ws, const ScanArgs &args, bool odd, hipStream_t stream);
+// ... as the gradients of the fused attention (ScanOperands::pad of every scan: its GradRole)
+void launch_scan_tph_gradients(void *ws, const ScanArgs &args, hipStream_t stream);
 
 }  // namespace mfma
 }  // namespace ftc

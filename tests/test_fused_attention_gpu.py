@@ -479,6 +479,59 @@ def test_backward_against_autograd_in_float64(lib, shape, form):
         assert (got[2][n_, len_:] == 0).all()
 
 
+# 64 x 64 rows, whose three scans run straight from the inputs: single positions, one row short of a chunk and
+# one past it, keys that end inside and before a chunk; chains walked whole and cut; segment sums exchanged
+DIRECT_SHAPES = [
+    (2, 1, 3, [1, 0]), (1, 31, 1, [31]), (2, 33, 2, [33, 5]), (3, 129, 8, [129, 0, 64]), (2, 700, 20, [700, 333]),
+    (1, 900, 4, [900]), (1, 2500, 2, [2217]), (15, 97, 8, [97, 32, 0, 65, 96] * 3),
+]
+
+
+@pytest.mark.parametrize("small", [None, "v_late_rows", "g_late_rows"])
+@pytest.mark.parametrize("shape", DIRECT_SHAPES, ids=lambda s: "n%d_l%d_h%d" % s[:3])
+def test_gradients_straight_from_the_inputs(lib, shape, small):
+    """Against autograd through the closed form in float64, eps = 1 (no gradient is a difference of nearly equal
+    numbers then).  Rows of values or of the gradient that are tiny beside the others' leave the normaliser's
+    share of a gradient far beyond the units of the scans' own products."""
+    from fast_transformers_amd import causal_product as cp
+    N, L, H, lens = shape
+    nlh = lambda t: t.permute(0, 2, 1, 3)
+    q, k, v = inputs(N, L, H, 64, 64, seed=81 + L)
+    g = torch.randn(N, L, H, 64, generator=torch.Generator().manual_seed(82 + L))
+    if small:
+        (v if small[0] == "v" else g)[:, (2 * L) // 3:] *= 2.0 ** -40
+    lengths = torch.tensor(lens)
+
+    def grads(dtype):
+        leaves = [t.to(dtype).requires_grad_(True) for t in (q, k, v)]
+        _dense_attention(*leaves, lengths, 1.0).backward(g.to(dtype))
+        return [t.grad for t in leaves]
+    exact, plain = grads(torch.float64), grads(torch.float32)
+    dev = [nlh(t.cuda()) for t in (q, k, v, g)]
+    out, den = nlh(torch.empty(N, L, H, 64, device="cuda")), torch.empty(N, H, L, device="cuda")
+    cp.causal_linear_attention_hip(*dev[:3], lengths.cuda(), 1.0, out, den)
+    got = [nlh(torch.full((N, L, H, 64), float("nan"), device="cuda")) for _ in range(3)]
+    cp.causal_linear_attention_backward_hip(*dev[:3], lengths.cuda(), out, den, dev[3], *got)
+    assert lib.ftc_last_kernel() == b"attention backward: three scans"
+    torch.cuda.synchronize()
+    cp.check_workspaces()
+    for name, a, b, c in zip("qkv", got, plain, exact):
+        a, b, c = a.cpu().double(), nlh(b).double(), nlh(c)
+        e_hip, e_plain = scale_error(a, c), scale_error(b, c)
+        assert torch.isfinite(a).all() and e_hip <= max(4 * e_plain, 2e-6), (name, e_hip, e_plain)
+    # each gradient by itself is the same
+    for i in range(3):
+        alone = [None] * 3
+        alone[i] = torch.empty_like(got[i])
+        cp.causal_linear_attention_backward_hip(*dev[:3], lengths.cuda(), out, den, dev[3], *alone)
+        assert ((alone[i] - got[i]).norm() <= 2e-6 * got[i].norm()).item()
+    # a gradient written over grad_out, which the scans would still read
+    over = dev[3].clone(memory_format=torch.preserve_format)
+    cp.causal_linear_attention_backward_hip(*dev[:3], lengths.cuda(), out, den, over, None, None, over)
+    assert lib.ftc_last_kernel() != b"attention backward: three scans"
+    assert ((over - got[2]).norm() <= 2e-6 * got[2].norm()).item()
+
+
 WIDE_SHAPES = [
     # N, L, H, E, M, key lengths: single positions, ragged ends, keys that end before, inside and on a
     # chunk; cut chains, whole ones of a round and more of workgroups, exchanges of segment sums; one and
