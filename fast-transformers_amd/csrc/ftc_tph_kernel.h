@@ -253,7 +253,7 @@ template <int KS, bool ODD, bool GRAD>
 __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, const ScanArgs &p) {
     static_assert(!GRAD || (KS == 2 && !ODD), "the gradients' form takes 64 x 64 states");
     constexpr int D = 64, F = 64;              // one block of state rows and of output columns
-    constexpr int T = 512;                     // producer lanes (eight wavefronts)
+    constexpr int T = 256;                     // producer lanes at a position (four wavefronts of eight)
     constexpr int PF = kTpAhead;               // chunks requested ahead
     constexpr int RBA = D * 2, RBV = F * 2;    // bytes per row of an fp16 piece tile
     constexpr int kTileA = kChunk * RBA, kTileV = kChunk * RBV;
@@ -367,7 +367,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
 
     if (producer) {
         // =========================== producers ===========================
-        const int ptid = (wave - 4) * 64 + lane;
+        const int ptid = w * 64 + lane;
         const uint32_t a_slb = (uint32_t)op.a_sl * 4, b_slb = (uint32_t)op.b_sl * 4,
                        v_slb = (uint32_t)op.v_sl * 4;
         const char *a_seg = (const char *)op.a + ((int64_t)n * op.a_sn + (int64_t)h * op.a_sh) * 4;
@@ -380,19 +380,22 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             (void *)b_seg, 0, (rows - 1) * b_slb + Dw * 4, kRsrcFlags);
         const __amdgpu_buffer_rsrc_t v_rs = __builtin_amdgcn_make_buffer_rsrc(
             (void *)v_seg, 0, (rows - 1) * v_slb + fw * 4, kRsrcFlags);
-        // One quad (four columns of one row) of every operand per lane and position.  Widths
-        // that do not fill the block: a lane whose four columns lie beyond the width asks
-        // outside the descriptor and cuts zeros (widths are multiples of 4).
-        static_assert(LA == 1 && LV == 1 && QA == QV, "one quad per lane");
+        // Two quads (four columns of one row) of every operand per lane and position, 16 rows
+        // apart.  Widths that do not fill the block: a lane whose four columns lie beyond the width
+        // asks outside the descriptor and cuts zeros (widths are multiples of 4).
+        static_assert(LA == 2 && LV == 2 && QA == QV, "two quads per lane");
         const int prow = ptid / QA, pc4 = ptid % QA;
-        const bool ab_in = 4 * pc4 < Dw;
-        const bool v_in = 4 * pc4 < fw;
+        const bool ab_in = GRAD || 4 * pc4 < Dw;
+        const bool v_in = GRAD || 4 * pc4 < fw;
         const uint32_t a_goff = (uint32_t)prow * a_slb + 16u * pc4,
                        b_goff = (uint32_t)prow * b_slb + 16u * pc4,
                        v_goff = (uint32_t)prow * v_slb + 16u * pc4;
-        const int a_waddr = TpSwizzle<RBA>::addr(prow, 8 * pc4),
-                  b_waddr = TpSwizzle<RBA>::addr(prow, 2 * b_tile_column(4 * pc4)),
-                  v_waddr = TpSwizzle<RBV>::addr(prow, 8 * pc4);
+        int a_waddr[2], b_waddr[2], v_waddr[2];
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+            a_waddr[q] = TpSwizzle<RBA>::addr(prow + 16 * q, 8 * pc4),
+            b_waddr[q] = TpSwizzle<RBA>::addr(prow + 16 * q, 2 * b_tile_column(4 * pc4)),
+            v_waddr[q] = TpSwizzle<RBV>::addr(prow + 16 * q, 8 * pc4);
         // (ODD: which of a quad's words 1 .. 3 are the row's own)
         uint32_t ab_own[3], v_own[3];
 #pragma unroll
@@ -404,9 +407,9 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             if (ODD) r = u32x4{r.x, r.y & m[0], r.z & m[1], r.w & m[2]};
         };
         struct Raw {
-            u32x4 a, b, v;
-            u32x4 x;            // GRAD: q or k
-            uint32_t rden, dd;  // GRAD
+            u32x4 a[2], b[2], v[2];
+            u32x4 x[2];               // GRAD: q or k
+            uint32_t rden[2], dd[2];  // GRAD
         };
         const uint32_t x_slb = GRAD ? (uint32_t)op.s0_sd * 4 : 0u, x_goff = (uint32_t)prow * x_slb + 16u * pc4;
         const bool has_x = GRAD && role != kGradValues;
@@ -418,37 +421,45 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             (void *)(GRAD ? p.row_rden + (int64_t)chain * rows : nullptr), 0, rows * 4, kRsrcFlags);
         const __amdgpu_buffer_rsrc_t dd_rs = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(GRAD ? p.row_dd + (int64_t)chain * rows : nullptr), 0, rows * 4, kRsrcFlags);
-        Raw raw[PF];
         // Every request is made every time, whether its rows exist or not (a chunk walked for
         // its state alone needs no rows of a; positions past the end of the walk have no
         // rows): a request outside the descriptor costs no memory traffic and reads as zero,
         // and with a fixed number of requests per chunk the compiler can wait for the oldest
         // ones only.
         auto fetch = [&](Raw &r, int v) {  // v: position of the walk
-            const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
-            const int row0_x = v >= n1 ? row0 : -2 * kChunk;
-            // (the sums wrap: a chunk that starts before the first row has its later rows in place)
-            r.a = __builtin_amdgcn_raw_buffer_load_b128(a_rs, ab_in ? a_goff + (uint32_t)row0_x * a_slb : kNoRow, 0, 0);
-            r.b = __builtin_amdgcn_raw_buffer_load_b128(b_rs, ab_in ? b_goff + (uint32_t)row0 * b_slb : kNoRow, 0, 0);
-            r.v = __builtin_amdgcn_raw_buffer_load_b128(v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, 0, 0);
-            if constexpr (GRAD) {
-                r.x = __builtin_amdgcn_raw_buffer_load_b128(x_rs, has_x ? x_goff + (uint32_t)row0_x * x_slb : kNoRow, 0, 0);
-                r.rden = __builtin_amdgcn_raw_buffer_load_b32(rden_rs, 4u * (uint32_t)(prow + row0), 0, 0);
-                r.dd = __builtin_amdgcn_raw_buffer_load_b32(dd_rs, 4u * (uint32_t)(prow + row0), 0, 0);
+            const int first = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int row0 = first + 16 * q, row0_x = v >= n1 ? row0 : -2 * kChunk;
+                // (the sums wrap: a chunk that starts before the first row has its later rows in place)
+                r.a[q] = __builtin_amdgcn_raw_buffer_load_b128(a_rs, ab_in ? a_goff + (uint32_t)row0_x * a_slb : kNoRow, 0, 0);
+                r.b[q] = __builtin_amdgcn_raw_buffer_load_b128(b_rs, ab_in ? b_goff + (uint32_t)row0 * b_slb : kNoRow, 0, 0);
+                r.v[q] = __builtin_amdgcn_raw_buffer_load_b128(v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, 0, 0);
+                if constexpr (GRAD) {
+                    r.x[q] = __builtin_amdgcn_raw_buffer_load_b128(x_rs, has_x ? x_goff + (uint32_t)row0_x * x_slb : kNoRow, 0, 0);
+                    r.rden[q] = __builtin_amdgcn_raw_buffer_load_b32(rden_rs, 4u * (uint32_t)(prow + row0), 0, 0);
+                    r.dd[q] = __builtin_amdgcn_raw_buffer_load_b32(dd_rs, 4u * (uint32_t)(prow + row0), 0, 0);
+                }
             }
         };
         // GRAD: the rows as the scan takes them.  phi(0) is one, so rows that are not there are
         // cleared (a scalar test: most chunks lie wholly inside).
-        auto feature = [&](u32x4 &x, int row0, int limit) {
-            x = feature_quad(x);
+        auto feature = [&](u32x4 (&x)[2], int row0, int limit) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) x[q] = feature_quad(x[q]);
             if (row0 < 0 || row0 + kChunk > limit) {
-                if ((uint32_t)(row0 + prow) >= (uint32_t)limit) x = u32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+                    if ((uint32_t)(row0 + 16 * q + prow) >= (uint32_t)limit) x[q] = u32x4{0, 0, 0, 0};
             }
         };
-        auto over_den = [](u32x4 &x, uint32_t rden) {
-            const float z = __uint_as_float(rden);
-            x = u32x4{__float_as_uint(z * __uint_as_float(x.x)), __float_as_uint(z * __uint_as_float(x.y)),
-                      __float_as_uint(z * __uint_as_float(x.z)), __float_as_uint(z * __uint_as_float(x.w))};
+        auto over_den = [](u32x4 (&x)[2], const uint32_t (&rden)[2]) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const float z = __uint_as_float(rden[q]);
+                x[q] = u32x4{__float_as_uint(z * __uint_as_float(x[q].x)), __float_as_uint(z * __uint_as_float(x[q].y)),
+                             __float_as_uint(z * __uint_as_float(x[q].z)), __float_as_uint(z * __uint_as_float(x[q].w))};
+            }
         };
         auto as_taken = [&](Raw &r, int v) {  // v: position of the walk
             const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
@@ -467,11 +478,12 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         // the largest magnitudes of the rows of a position against the ceilings (rows that
         // were not asked for read as zeros); k: that position's slot
         auto look_ahead = [&](Raw &r, int k, int pos) {
-            own_words(r.a, ab_own), own_words(r.b, ab_own), own_words(r.v, v_own);
+#pragma unroll
+            for (int q = 0; q < 2; q++) own_words(r.a[q], ab_own), own_words(r.b[q], ab_own), own_words(r.v[q], v_own);
             if constexpr (GRAD) {
                 as_taken(r, pos);
                 if (has_x) {  // (rows of 16 lanes share a row of the operands)
-                    const uint32_t d = r.dd & 0x7fffffffu;
+                    const uint32_t d = max(r.dd[0] & 0x7fffffffu, r.dd[1] & 0x7fffffffu);
                     const uint32_t m = scalar_max(scalar_max((uint32_t)__builtin_amdgcn_readlane((int)d, 0),
                                                              (uint32_t)__builtin_amdgcn_readlane((int)d, 16)),
                                                   scalar_max((uint32_t)__builtin_amdgcn_readlane((int)d, 32),
@@ -481,82 +493,98 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
             }
-            raise_slot(slots, k, pos, ce, max_abs4(r.a, 0.f), max_abs4(r.b, 0.f), max_abs4(r.v, 0.f), lane);
+            raise_slot(slots, k, pos, ce, max_abs4(r.a[1], max_abs4(r.a[0], 0.f)), max_abs4(r.b[1], max_abs4(r.b[0], 0.f)),
+                       max_abs4(r.v[1], max_abs4(r.v[0], 0.f)), lane);
         };
-        // A position of the walk goes to its LDS buffer through register set (position % PF).
-        // The first n1 positions only feed the state: no piece of a.
+        // A position of the walk goes to its LDS buffer.  The first n1 positions only feed the
+        // state: no piece of a.
         auto cut = [&](const Raw &r, int buf, bool own) {
             lds_char *const pc = unit_pc + buf * kBufBytes;
-            if (own) cut_quad_to_lds(r.a, ce.scale_a(), pc, kTileA, a_waddr);
-            cut_quad_to_lds(r.b, ce.scale_b(), pc + kOffB, kTileA, b_waddr);
-            cut_quad_to_lds(r.v, ce.scale_v(), pc + kOffV, kTileV, v_waddr);
-            if constexpr (GRAD) {
-                if (has_x) {
-                    if (own) {
-                        auto slope = [](uint32_t x) -> uint32_t {  // phi'(x); NaN: one (gz is NaN then)
-                            return __float_as_uint(fminf(1.f, __builtin_amdgcn_exp2f(__uint_as_float(x) * 1.44269502f)));
-                        };
-                        *(lds_vec4 *)(x_pc + buf * kTileX + prow * F * 4 + 16 * (pc4 ^ (prow & 15))) =
-                            u32x4{slope(r.x.x), slope(r.x.y), slope(r.x.z), slope(r.x.w)};
-                    }
-                    const float dd = __uint_as_float(r.dd), wt = dd * pow2_field(ce.weight_field());
-                    _Float16 hi = (_Float16)wt, lo = (_Float16)(wt - (float)hi);
-                    if (role == kGradQueries) hi = (_Float16)1.f, lo = (_Float16)0.f;
-                    if (pc4 == 0) {
-                        lds_char *const d = dd_pc + buf * kDdBytes;
-                        *(lds_f32 *)(d + 4 * prow) = dd;
-                        *(lds_f32 *)(d + kDdUnits + 4 * prow) = ce.dd_shift() == 0 ? __builtin_amdgcn_ldexpf(dd, ce.dd_up()) : 0.f;
-                        *(lds_u16 *)(d + kWeights + 2 * prow) = __builtin_bit_cast(uint16_t, hi);
-                        *(lds_u16 *)(d + kWeights + 2 * (kChunk + prow)) = __builtin_bit_cast(uint16_t, lo);
-                    }
-                }
-                if (!own) asm volatile("" ::"v"(r.x));
-            }
-            if (!own) asm volatile("" ::"v"(r.a));
-        };
 #pragma unroll
-        for (int j = 0; j < PF; j++) fetch(raw[j], j);
-        wg_barrier();  // the slots are zero
-        look_ahead(raw[0], B0, 0);
-        wg_barrier();  // the slot of position 0 is complete
+            for (int q = 0; q < 2; q++) {
+                if (own) cut_quad_to_lds(r.a[q], ce.scale_a(), pc, kTileA, a_waddr[q]);
+                cut_quad_to_lds(r.b[q], ce.scale_b(), pc + kOffB, kTileA, b_waddr[q]);
+                cut_quad_to_lds(r.v[q], ce.scale_v(), pc + kOffV, kTileV, v_waddr[q]);
+            }
+            if (GRAD && has_x) {
+                auto slope = [](uint32_t x) -> uint32_t {  // phi'(x); NaN: one (gz is NaN then)
+                    return __float_as_uint(fminf(1.f, __builtin_amdgcn_exp2f(__uint_as_float(x) * 1.44269502f)));
+                };
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+                    if (own)
+                        *(lds_vec4 *)(x_pc + buf * kTileX + (prow + 16 * q) * F * 4 + 16 * (pc4 ^ prow)) =
+                            u32x4{slope(r.x[q].x), slope(r.x[q].y), slope(r.x[q].z), slope(r.x[q].w)};
+                // (lane 0 of a row's sixteen for the first row, lane 1 for the second)
+                const float dd = __uint_as_float(pc4 == 0 ? r.dd[0] : r.dd[1]), wt = dd * pow2_field(ce.weight_field());
+                const int at = prow + 16 * pc4;
+                _Float16 hi = (_Float16)wt, lo = (_Float16)(wt - (float)hi);
+                if (role == kGradQueries) hi = (_Float16)1.f, lo = (_Float16)0.f;
+                if (pc4 < 2) {
+                    lds_char *const d = dd_pc + buf * kDdBytes;
+                    *(lds_f32 *)(d + 4 * at) = dd;
+                    *(lds_f32 *)(d + kDdUnits + 4 * at) = ce.dd_shift() == 0 ? __builtin_amdgcn_ldexpf(dd, ce.dd_up()) : 0.f;
+                    *(lds_u16 *)(d + kWeights + 2 * at) = __builtin_bit_cast(uint16_t, hi);
+                    *(lds_u16 *)(d + kWeights + 2 * (kChunk + at)) = __builtin_bit_cast(uint16_t, lo);
+                }
+            }
+            if (!own) {
+                asm volatile("" ::"v"(r.a[0]), "v"(r.a[1]));
+                if constexpr (GRAD) asm volatile("" ::"v"(r.x[0]), "v"(r.x[1]));
+            }
+        };
         // Barrier number k (k = 0: before the consumers' first position; k >= 1: in the
         // middle of position k - 1) finds position k cut and the slot of position k + 1
-        // complete.  The last one finds a chunk of zeros.
-        int buf = B0;
-        auto step = [&](int v, int j, bool own) {
-            if (own && v == n1 + 4) FTC_STAMP(0);
-            read_slot<GRAD>(slots, buf, ce);
-            look_ahead(raw[(j + 1) % PF], next_buf(buf), v + 1);
-            if (own && v == n1 + 4) FTC_STAMP(1);
-            cut(raw[j], buf, own);
-            if (own && v == n1 + 4) FTC_STAMP(2);
-            fetch(raw[j], v + PF);
-            buf = buf == 2 ? 0 : buf + 1;
-            if (own && v == n1 + 4) FTC_STAMP(3);
-            wg_barrier();
-            __builtin_amdgcn_sched_barrier(0);  // one chunk at a time, in this order
-            if (own && v == n1 + 4) FTC_STAMP(4);
+        // complete.  The last one finds a chunk of zeros.  The two groups of producers take the
+        // positions in turn: before barrier k group k % 2 cuts position k, which it has looked at
+        // before barrier k - 1, and the other group looks at position k + 1.
+        static_assert(PF == 4, "two positions ahead for each of two groups");
+        auto walk = [&](auto group_number) {
+            constexpr int G = decltype(group_number)::value;
+            Raw raw[2];
+            fetch(raw[0], G), fetch(raw[1], G + 2);
+            wg_barrier();  // the slots are zero
+            if (G == 0) look_ahead(raw[0], B0, 0);
+            wg_barrier();  // the slot of position 0 is complete
+            int buf = B0;
+            auto period = [&](int v, int j, bool own, bool more) {  // v % 4 == j
+                const bool stamped = own && v == n1 + 4;
+                if (stamped) FTC_STAMP(0);
+                read_slot<GRAD>(slots, buf, ce);
+                if (j % 2 == G) {
+                    cut(raw[j / 2], buf, own);
+                    if (stamped) FTC_STAMP(2);
+                    if (more) fetch(raw[j / 2], v + PF);
+                } else {
+                    look_ahead(raw[(j + 1) % 4 / 2], next_buf(buf), v + 1);
+                    if (stamped) FTC_STAMP(1);
+                }
+                buf = next_buf(buf);
+                if (stamped) FTC_STAMP(3);
+                wg_barrier();
+                __builtin_amdgcn_sched_barrier(0);  // one chunk at a time, in this order
+                if (stamped) FTC_STAMP(4);
+            };
+            for (int v = 0; v < n1; v += PF) {
+#pragma unroll
+                for (int j = 0; j < PF; j++) period(v + j, j, false, true);
+            }
+            // (whole trips in the loop, the rest after it)
+            int v = n1;
+            for (; v + PF <= nwalk + 1; v += PF) {
+#pragma unroll
+                for (int j = 0; j < PF; j++) period(v + j, j, true, true);
+            }
+#pragma unroll
+            for (int j = 0; j < PF - 1; j++) {
+                if (v + j > nwalk) return;
+                period(v + j, j, true, false);
+            }
         };
-        for (int v = 0; v < n1; v += PF) {
-#pragma unroll
-            for (int j = 0; j < PF; j++) step(v + j, j, false);
-        }
-        // (whole trips in the loop, the rest after it)
-        int v = n1;
-        for (; v + PF <= nwalk + 1; v += PF) {
-#pragma unroll
-            for (int j = 0; j < PF; j++) step(v + j, j, true);
-        }
-#pragma unroll
-        for (int j = 0; j < PF - 1; j++) {
-            if (v + j > nwalk) return;
-            read_slot<GRAD>(slots, buf, ce);
-            look_ahead(raw[(j + 1) % PF], next_buf(buf), v + j + 1);
-            cut(raw[j], buf, true);
-            buf = buf == 2 ? 0 : buf + 1;
-            wg_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        if (wave < 8)
+            walk(std::integral_constant<int, 0>());
+        else
+            walk(std::integral_constant<int, 1>());
         return;
     }
 
