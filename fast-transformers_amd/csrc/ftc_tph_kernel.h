@@ -257,8 +257,11 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
     constexpr int PF = kTpAhead;               // chunks requested ahead
     constexpr int RBA = D * 2, RBV = F * 2;    // bytes per row of an fp16 piece tile
     constexpr int kTileA = kChunk * RBA, kTileV = kChunk * RBV;
-    constexpr int kOffB = 2 * kTileA, kOffV = 4 * kTileA;
-    constexpr int kBufBytes = 4 * kTileA + 2 * kTileV;
+    // (b's second piece starts 256 bytes further on: 512-byte steps would let the compiler read both pieces' halves
+    // in one instruction and put the fragments together with eight moves a chunk)
+    constexpr int kTileB = kTileA + 256;
+    constexpr int kOffB = 2 * kTileA, kOffV = kOffB + 2 * kTileB;
+    constexpr int kBufBytes = kOffV + 2 * kTileV;
     constexpr int kTileP = kChunk * 64;        // Pt pieces: 32 rows (i) of 32 j
     constexpr int QA = D / 4, QV = F / 4;
     constexpr int LA = kChunk * QA / T, LV = kChunk * QV / T;
@@ -503,7 +506,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
 #pragma unroll
             for (int q = 0; q < 2; q++) {
                 if (own) cut_quad_to_lds(r.a[q], ce.scale_a(), pc, kTileA, a_waddr[q]);
-                cut_quad_to_lds(r.b[q], ce.scale_b(), pc + kOffB, kTileA, b_waddr[q]);
+                cut_quad_to_lds(r.b[q], ce.scale_b(), pc + kOffB, kTileB, b_waddr[q]);
                 cut_quad_to_lds(r.v[q], ce.scale_v(), pc + kOffV, kTileV, v_waddr[q]);
             }
             if (GRAD && has_x) {
@@ -628,16 +631,15 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         const int j = 16 * jh + 4 * g + r, i = 16 * ih + ln;
         keep[r] = REV ? (j >= i) : (j <= i);
     }
-    uint32_t o_lane[2];
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-        o_lane[x] = (uint32_t)(16 * (x ^ ih) + ln) * o_slb + 4u * (16 * w + 4 * g);
     // (columns beyond the width are not stored; ODD: a quad that straddles the width is stored
     // word by word, by the one wavefront that has such a quad)
     const int o_cols = fw - (16 * w + 4 * g);
     const bool o_in = o_cols >= (ODD ? 4 : 1);
     const bool o_straddles = ODD && fw % 4 != 0 && fw / 16 == w;
-
+    uint32_t o_lane[2];
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+        o_lane[x] = (uint32_t)(16 * (x ^ ih) + ln) * o_slb + 4u * (16 * w + 4 * g) + (o_in ? 0u : kNoRow);
     constexpr int NT = 2 * KS;  // state tiles of 16 rows
     f32x4 S[4];                 // the slab, in units of 2^Ucur
 #pragma unroll
@@ -706,7 +708,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         const int k = i % 2, ks = (i / 2) % 2, x = i / 4;
         if (ks >= KS) return;
         if (x == 0)
-            bfr[ks][k] = lds_frag8x2(pc + k * kTileA + b_addr[ks][0], pc + k * kTileA + b_addr[ks][1]);
+            bfr[ks][k] = lds_frag8x2(pc + k * kTileB + b_addr[ks][0], pc + k * kTileB + b_addr[ks][1]);
         else
             af[x - 1][ks][k] = lds_frag16(pc + k * kTileA + a_addr[x - 1][ks]);
     };
@@ -717,7 +719,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             vfx[i] = lds_frag_tr(pc + i * kTileV + vt_addr[0], pc + i * kTileV + vt_addr[1]);
         else {
             const int dt = (i - 2) / 2, k = (i - 2) % 2;
-            btx[dt][k] = lds_frag_tr(pc + k * kTileA + bt_addr[dt][0], pc + k * kTileA + bt_addr[dt][1]);
+            btx[dt][k] = lds_frag_tr(pc + k * kTileB + bt_addr[dt][0], pc + k * kTileB + bt_addr[dt][1]);
         }
     };
     int buf = B0;  // LDS buffer of the chunk at hand
@@ -852,7 +854,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         while (s < 100 && __builtin_amdgcn_ballot_w64(m > pow2_field(127 + 14 + s)) != 0) s++;
     }
     float kappa = pow2_field(127 + dU - s);  // scale of the cut of S
-    bool plain_cut = dU - s == 0;            // ... which is one as a rule: a cheaper cut
     int s_cut = s;                            // ... and the s that went into it
     float mS = 0.f;                           // largest |S| seen while cutting
     Frag sf[2][2];
@@ -865,12 +866,8 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         const f32x4 x = S[2 * ks + u];
         if (track)
             mS = fmaxf(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))), mS);
-        if (plain_cut)
-            cut_quad_f16_unscaled(x[0], x[1], x[2], x[3], sf[ks][0].w[2 * u], sf[ks][0].w[2 * u + 1],
-                                  sf[ks][1].w[2 * u], sf[ks][1].w[2 * u + 1]);
-        else
-            cut_quad_f16(x[0], x[1], x[2], x[3], kappa, sf[ks][0].w[2 * u], sf[ks][0].w[2 * u + 1],
-                         sf[ks][1].w[2 * u], sf[ks][1].w[2 * u + 1]);
+        cut_quad_f16(x[0], x[1], x[2], x[3], kappa, sf[ks][0].w[2 * u], sf[ks][0].w[2 * u + 1], sf[ks][1].w[2 * u],
+                     sf[ks][1].w[2 * u + 1]);
     };
     cut_s(0, 0, true);
     cut_s(0, 1, true);
@@ -881,7 +878,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
 #pragma unroll
     for (int x = 0; x < 2; x++) O[x] = f32x4{0.f, 0.f, 0.f, 0.f};
     int Xo = 0;
-    uint32_t o_off = 0x80000000u;
+    uint32_t o_off = (uint32_t)(rows + kChunk) * o_slb;  // (also beyond the end with kNoRow on top of it)
     int o_row0 = 0, o_buf = 0;  // GRAD
     auto store_rows = [&](int x) {
         float y0 = __builtin_amdgcn_ldexpf(O[x][0], Xo), y1 = __builtin_amdgcn_ldexpf(O[x][1], Xo),
@@ -897,10 +894,9 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
                 y0 = live ? y0 : 0.f, y1 = live ? y1 : 0.f, y2 = live ? y2 : 0.f, y3 = live ? y3 : 0.f;
             }
         }
-        const uint32_t at = o_in ? o_off + o_lane[x] : kNoRow;
-        buffer_store_out(o_rs, at, y0, y1, y2, y3, (float *)nullptr);
+        buffer_store_out(o_rs, o_off + o_lane[x], y0, y1, y2, y3, (float *)nullptr);
         if (o_straddles) {
-            const uint32_t first = o_off + o_lane[x];
+            const uint32_t first = o_off + o_lane[x] - (o_in ? 0u : kNoRow);
             const bool some = o_cols < 4;
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y0), o_rs, some && o_cols > 0 ? first : kNoRow, 0, 0);
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y1), o_rs, some && o_cols > 1 ? first + 4u : kNoRow, 0, 0);
@@ -946,7 +942,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         }
         if (c == c0 + 4) FTC_STAMP(1);
         // all of S is cut: it takes the units of this chunk, and s follows its size
-        if (dU != 0) {
+        if (__builtin_expect(dU != 0, 0)) {
             scale_state(dU);
             mS = __builtin_amdgcn_ldexpf(mS, dU);
             s = max(0, s + min(dU, 0));
@@ -1001,7 +997,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             for (int k = 0; k < 2; k++) pf[x][k] = lds_frag16(ptc + k * kTileP + pt_raddr[x]);
         const int Xc = ce.out_exp() + shift;
         const u32x4 slot_next = *(const lds_vec4 *)(slots + 4 * BN);
-        if (s_cut != 0) {  // (rare: the state has grown beyond 2^14 units)
+        if (__builtin_expect(s_cut != 0, 0)) {  // (rare: the state has grown beyond 2^14 units)
             const float r_cut = pow2_field(127 + s_cut);
             O[0] *= r_cut;
             O[1] *= r_cut;
@@ -1034,7 +1030,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         dU = Ucur - ce.state_exp();
         s += max(dU, 0);
         kappa = pow2_field(127 + dU - s);
-        plain_cut = dU - s == 0;
         s_cut = s;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
