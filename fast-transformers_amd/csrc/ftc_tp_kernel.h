@@ -48,6 +48,8 @@
 //    (2a)) and go on to cut chunk c + 2 into the buffer of chunk c - 1, which nobody has
 //    read since the barrier before.
 #pragma once
+#include <type_traits>
+
 #include "ftc_wg_kernel.h"
 
 namespace ftc {
@@ -97,6 +99,13 @@ __device__ __forceinline__ constexpr int b_tile_column(int d) {
     return 32 * (d / 32) + 16 * ((d / 4) % 2) + 4 * ((d % 32) / 8) + d % 4;
 }
 
+// 1 / x: the estimate and one step of Newton's, half as many instructions as the division, which is left what
+// is special (zero, infinite, NaN, or below 2^-126)
+__device__ __forceinline__ float reciprocal(float x) {
+    const float r = __builtin_amdgcn_rcpf(x), e = fmaf(-x, r, 1.0f);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(e != e) != 0, 0)) return 1.0f / x;
+    return fmaf(e, r, r);
+}
 // sum over the four groups of 16 lanes, in every lane: v_permlane16_swap exchanges the odd groups
 // of its first operand with the even groups of its second, v_permlane32_swap the halves
 __device__ __forceinline__ float sum_of_lane_groups(float x) {
@@ -183,6 +192,11 @@ __device__ __forceinline__ void tp_workgroup(const ScanArgs &p, uint32_t &which,
 template <int PA, int PB, int PV>
 constexpr int kTpPieceBytes = 3 * (PA + PB + PV) * kChunk * 128;
 constexpr int kTpPtBytes = 2 * 3 * kChunk * 64;
+// Whether a kernel's loop over chunks is unrolled three times, with its buffers in the instructions' offsets
+// (and three of Pt): the fused attention, where the vector instructions of a producer and a consumer together fill
+// their SIMD.  535 of them a chunk -> 470 this way, with the quadrant in two sums for four, half a division and
+// its edges on branches: 80 chains, L=1000 36.4 -> 34.7 us, L=4096 137 -> 124.
+constexpr bool tp_unrolled(int ND, bool NORM) { return NORM && ND == 1; }
 constexpr int kTpZBytes = 4 * 2 * 2 * 64;  // z of the four consumers, fused attention with two blocks
 
 // KS2: groups of 32 rows in the state's last block (1: a state of 65 .. 96 rows, whose last
@@ -225,6 +239,9 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     constexpr int QA = D / 4, QV = F / 4;
     constexpr int LA = kChunk * QA / T, LV = kChunk * QV / T;
     static_assert(kChunk == 32 && T % QA == 0 && T % QV == 0, "shape");
+    // (the fused attention's rows have 32, 64 or 128 values)
+    constexpr bool kFullRows = NORM && KS2 == 2;
+    constexpr bool kUnrolled = tp_unrolled(ND, NORM);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -294,6 +311,9 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     // groups of 32 rows of block hb
     auto block_ks = [](int hb) -> int { return hb == ND - 1 ? KS2 : 2; };
     auto chunk_row0 = [&](int c) -> int { return REV ? rows - kChunk * (c + 1) : kChunk * c; };
+    // Position k of the walk goes through LDS buffer (B0 + k) % 3, the first one of the walk proper through
+    // buffer 0, so that a loop over those chunks that is unrolled three times knows its buffers.
+    const int B0 = __builtin_amdgcn_readfirstlane((3 - n1 % 3) % 3);
     __syncthreads();
 #ifdef FTC_TIMELINE
     // tuning aid: 32 time stamps per workgroup behind the pointer that the host passes in
@@ -325,7 +345,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         // of 4).  A lane has the same columns in both of its quads.
         bool ab_in[ND];
 #pragma unroll
-        for (int hb = 0; hb < ND; hb++) ab_in[hb] = 4 * (ptid % QA) + D * hb < Dw;
+        for (int hb = 0; hb < ND; hb++) ab_in[hb] = kFullRows || 4 * (ptid % QA) + D * hb < Dw;
         const bool v_in = 4 * (ptid % QV) < fw;
         const OwnWords<ODD> ab_own[2] = {{4 * (ptid % QA), Dw}, {4 * (ptid % QA) + D, Dw}}, v_own(4 * (ptid % QV), fw);
         uint32_t a_goff[LA], b_goff[LA], v_goff[LV];
@@ -392,6 +412,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 const int row0 = v < nwalk ? chunk_row0(walk_chunk(v)) : -2 * kChunk;
                 // (a scalar test: most chunks lie wholly below the limit)
                 if (row0 < 0 || row0 + kChunk > key_rows) {
+                    asm volatile("" : "+v"(y.x));  // (a branch, not eight selects in every chunk)
                     if ((uint32_t)(row0 + 16 * q + ptid / QA) >= (uint32_t)key_rows) y = u32x4{0, 0, 0, 0};
                 }
                 if (!ab_in[hb]) y = u32x4{0, 0, 0, 0};
@@ -400,7 +421,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 return x;
             }
         };
-        // position k of the walk goes to LDS buffer k % 3 through register set k % PF.  The
+        // position k of the walk goes to its LDS buffer through register set k % PF.  The
         // first n1 positions (a multiple of PF) only feed the state: no piece of a, and the
         // consumers, who have little to do there, cut rows 16 .. 31 of b and v themselves.
         auto cut = [&](const Raw &r, int buf, bool own, int hb, int v) {
@@ -427,7 +448,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         // position k - 1) finds position k cut.  The last one finds a chunk of zeros.
         // Two loops whose bodies are straight-line code, so that the waits inside them count
         // requests instead of draining them.
-        int buf = 0;
+        int buf = B0;
         for (int v = 0; v < n1; v += PF) {
 #pragma unroll
             for (int j = 0; j < PF; j++) {
@@ -583,17 +604,19 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     // The products of up to eight chunks are added up by themselves (R) before they are added to the
     // state, where there are registers for it; the state in use is S + R.  (The sums of the matrix
     // instructions fall short by a part of the last place of the sum each, which keys and weights that
-    // are all positive add up.  NORM: 300 chains of 4000 positions walked whole were 7e-7 from float64
-    // without it, the workgroup form's short segments are 3e-7; the time is the same.  Not there while
-    // chunks are walked for their state alone, nor with two blocks: its registers would spill.  bf16 rows: the state handed
-    // out after 1000 positions was 2.7e-7 off without it, 1.0e-7 on the kernels that split L.)
+    // are all positive add up.  bf16 rows: the state handed out after 1000 positions was 2.7e-7 off
+    // without it, 1.0e-7 on the kernels that split L.)
+    // NORM: each chunk's products by themselves, and z's of up to eight chunks (300 chains of 4000 positions
+    // walked whole were 7e-7 from float64 without either, the workgroup form's short segments are 3e-7; R in place
+    // of the chunk's own sums: 80 chains, L=4096 1.08e-7 against 1.06e-7, and 15 more registers that spilled).  Not
+    // while chunks are walked for their state alone, nor with two blocks: those registers would spill.
     // ODD: also while chunks are walked for their state (220 -> 237 registers); with two blocks each
     // chunk's products by themselves, a tile's sum added to the state as soon as it is whole (in the first
     // walk only where the last block has 32 rows: else 111 registers would spill).  127 x 127 backward,
     // 15 chains, L=710: 2-norm error 3.6e-7 -> 2.7e-7 at the same time.
-    constexpr bool kMixed = PA + PB + PV < 9, kApart = ((NORM || ODD) && ND == 1) || kMixed,
-                   kFirstApart = kMixed || (ODD && ND == 1), kChunkSums = ODD && ND > 1,
-                   kFirstSums = kChunkSums && KS2 == 1;
+    constexpr bool kMixed = PA + PB + PV < 9, kApart = (ODD && ND == 1) || kMixed, kFirstApart = kMixed || (ODD && ND == 1),
+                   kChunkSums = (ODD && ND > 1) || (NORM && ND == 1), kFirstSums = ODD && ND > 1 && KS2 == 1,
+                   kApartZ = NORM && ND == 1;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 R[ND][4], Zr[ND][2];
     f32x4 chunk_sum[4];
@@ -618,17 +641,17 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
             for (int dt = 0; dt < 4; dt++) {
                 if (kApart) R[hb][dt] = zero;
-                if (NORM && kApart) Zr[hb][dt % 2] = zero;
+                if (kApartZ) Zr[hb][dt % 2] = zero;
             }
     };
     auto add_apart = [&]() {
-        if (kApart) {
+        if (kApart || kApartZ) {
 #pragma unroll
             for (int hb = 0; hb < ND; hb++)
 #pragma unroll
                 for (int dt = 0; dt < 4; dt++) {
-                    if (dt / 2 < (hb == ND - 1 ? KS2 : 2)) S[hb][dt] += R[hb][dt];
-                    if (NORM && dt < 2) Z[hb][dt] += Zr[hb][dt];
+                    if (kApart && dt / 2 < (hb == ND - 1 ? KS2 : 2)) S[hb][dt] += R[hb][dt];
+                    if (kApartZ && dt < 2) Z[hb][dt] += Zr[hb][dt];
                 }
             clear_apart();
         }
@@ -668,7 +691,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     auto prev_buf = [](int b) -> int { return b == 0 ? 2 : b - 1; };
 
     auto next_buf = [](int b) -> int { return b == 2 ? 0 : b + 1; };
-    int buf = 0;  // LDS buffer of the chunk at hand
+    int buf = B0;  // LDS buffer of the position at hand
     if (n1 > 0) {
         // ---- the first n1 positions of the walk: state update only ----
         if (kFirstApart) clear_apart();
@@ -711,7 +734,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             (void *)v_seg, 0, (rows - 1) * v_slb + fw * QuadV::bytes, kRsrcFlags);
         bool b_in[ND];
 #pragma unroll
-        for (int hb = 0; hb < ND; hb++) b_in[hb] = 4 * cc4 + D * hb < Dw;
+        for (int hb = 0; hb < ND; hb++) b_in[hb] = kFullRows || 4 * cc4 + D * hb < Dw;
         const bool v_in = 4 * cc4 < fw;
         const OwnWords<ODD> b_own[2] = {{4 * cc4, Dw}, {4 * cc4 + D, Dw}}, v_own(4 * cc4, fw);
         const uint32_t b_goff = (uint32_t)crow * b_slb + 4u * QuadB::bytes * cc4,
@@ -749,13 +772,13 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         };
 #pragma unroll
         for (int j = 0; j < PF; j++) cfetch(rawc[j], j, j % ND);
-        ccut_b(rawc[0], 0, 0);
-        ccut_v(rawc[0], 0);
+        ccut_b(rawc[0], B0, 0);
+        ccut_v(rawc[0], B0);
         cfetch(rawc[0], PF, 0);
         wg_barrier();
         FTC_STAMP(13);  // first chunk cut
         Frag bt2[4][PB] = {}, vf2[PV] = {};  // (the first round multiplies zeros)
-        int bufn = 1;                      // LDS buffer of the chunk after the one at hand
+        int bufn = next_buf(B0);           // LDS buffer of the position after the one at hand
         for (int c = 0; c < n1; c += PF) {
 #pragma unroll
             for (int j = 0; j < PF; j++) {
@@ -891,14 +914,23 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                                                       o_cols < 4 && o_cols > e ? first + 4u * e : kNoRow, 0, 0);
         }
     };
+    const bool den_out = NORM && w == 0 && fb == 0 && op.s_out;
+    const __amdgpu_buffer_rsrc_t den_rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(den_out ? op.s_out + (int64_t)n * op.so_sn + (int64_t)h * op.so_sh : nullptr), 0,
+        den_out ? 4u * (uint32_t)rows : 0u, kRsrcFlags);
+    constexpr int kPSums = NORM && ND == 1 ? 2 : 4;  // sums that the quadrant is added up from
     f32x4 Pkeep = {0.f, 0.f, 0.f, 0.f};  // the quadrant summed over the blocks so far
     f32x4 Az = {0.f, 0.f, 0.f, 0.f};     // NORM: phi(a) z of the quadrant's positions
-    for (int c = c0; c < nchunks; c++) {
+    // (B: the LDS buffer of the chunk's first position, a compile-time number where the loop is unrolled)
+    auto chunk_body = [&](int c, auto buffer_number) {
+        constexpr int B = decltype(buffer_number)::value;
+        const int pt_buf = kUnrolled ? B : c & 1;
 #pragma unroll
         for (int hb = 0; hb < ND; hb++) {  // block hb of the state rows
+            if (kUnrolled) buf = (B + hb) % 3;
             const lds_char *pc = unit_pc + buf * kBufBytes;
             const lds_char *pcv = hb == 0 ? pc : unit_pc + prev_buf(buf) * kBufBytes;
-            lds_char *const ptc = pt_pc + (c & 1) * (3 * kTileP);
+            lds_char *const ptc = pt_pc + pt_buf * (3 * kTileP);
             // The quadrants of a chunk's blocks are added up before they are cut: only the
             // last block of a chunk hands Pt to the others and multiplies it with v.
             const bool last_block = hb == ND - 1;
@@ -917,9 +949,9 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             for (int i = 0; i < 12; i++) {
                 const int ks = i % 2, m = i / 2;
                 if (ks < block_ks(hb) && m < OfP::count)
-                    P4[i % 4] = mfma16(bfr[ks][OfP::x(m)], af[0][ks][OfP::y(m)], i < 4 ? zero : P4[i % 4]);
-                else if (i < 4)
-                    P4[i % 4] = zero;
+                    P4[i % kPSums] = mfma16(bfr[ks][OfP::x(m)], af[0][ks][OfP::y(m)], i < kPSums ? zero : P4[i % kPSums]);
+                else if (i < kPSums)
+                    P4[i % kPSums] = zero;
                 if (i < 4 && block_ks(hb) > 1) cut_s(hb, 1, i);
                 if (NORM && ND > 1 && (i == 5 || i == 7)) Z[0][i / 2 - 2] = z_mem[8 * hb + 4 * (i / 2 - 2)];
                 if (NORM && i >= 8) {  // z in pieces
@@ -952,7 +984,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 if constexpr (NORM)
                     if (i >= 6) Az = mfma16(zf[OfO::x(i - 6)], af[0][0][OfO::y(i - 6)], i == 6 && hb == 0 ? zero : Az);
                 if (i == 4) {
-                    P = (P4[0] + P4[1]) + (P4[2] + P4[3]);
+                    P = kPSums == 2 ? P4[0] + P4[1] : (P4[0] + P4[1]) + (P4[2] + P4[3]);
                     if (hb > 0) P += Pkeep;
                     if (!last_block) Pkeep = P;
                 }
@@ -988,8 +1020,8 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                     add_product(hb, i % 2, bt[i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)], i < 2);
                 if constexpr (NORM)
                     if (i < 6) {
-                        f32x4 &sum = kApart ? Zr[hb][i % 2] : Zr[0][i % 2];
-                        sum = mfma16(bt[i % 2][2 - i / 2], ones, kApart || i >= 2 ? sum : zero);
+                        f32x4 &sum = kApartZ ? Zr[hb][i % 2] : Zr[0][i % 2];
+                        sum = mfma16(bt[i % 2][2 - i / 2], ones, kApartZ || i >= 2 ? sum : zero);
                     }
                 if (NORM && ND > 1) {
                     if (i == 7 || i == 8) Z[0][i - 7] = z_mem[8 * hb + 4 * (i - 7)];
@@ -997,7 +1029,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 }
                 if (NORM && i == 6 && last_block) {
                     P_sum = sum_of_lane_groups(P_sum);
-                    if (g == 0) den_mem[c & 1][16 * ih + ln][w >> 1] = (has_z ? Az[0] : 0.f) + P_sum;
+                    if (g == 0) den_mem[pt_buf][16 * ih + ln][w >> 1] = (has_z ? Az[0] : 0.f) + P_sum;
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1021,13 +1053,14 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 if (last_block) {
 #pragma unroll
                     for (int x = 0; x < 2; x++) {
-                        const float *part = den_mem[c & 1][16 * (x ^ ih) + ln];
+                        const float *part = den_mem[pt_buf][16 * (x ^ ih) + ln];
                         const float den = (part[0] + part[1]) + p.eps;
-                        r_den[x] = 1.0f / den;
+                        r_den[x] = reciprocal(den);
                         // (the caller's copy of the denominators, for the backward)
-                        const int row = chunk_row0(c) + 16 * (x ^ ih) + ln;
-                        if (w == 0 && fb == 0 && op.s_out && g == 0 && row < rows)
-                            op.s_out[(int64_t)n * op.so_sn + (int64_t)h * op.so_sh + row] = den;
+                        if (den_out)
+                            __builtin_amdgcn_raw_buffer_store_b32(
+                                __float_as_uint(den), den_rs,
+                                g == 0 ? 4u * (uint32_t)(chunk_row0(c) + 16 * (x ^ ih) + ln) : kNoRow, 0, 0);
                     }
                 }
             }
@@ -1055,10 +1088,22 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (c == c0 + 4) FTC_STAMP(5);
-            if (kApart && last_block && (c - c0) % 8 == 7) add_apart();
+            if ((kApart || kApartZ) && last_block && (c - c0) % 8 == 7) add_apart();
             o_off = (uint32_t)chunk_row0(c) * o_slb;
             if (c == c0 + 4) FTC_STAMP(6);
         }
+    };
+    if constexpr (kUnrolled) {
+        int c = c0;
+        for (; c + 3 <= nchunks; c += 3) {
+            chunk_body(c, std::integral_constant<int, 0>());
+            chunk_body(c + 1, std::integral_constant<int, ND % 3>());
+            chunk_body(c + 2, std::integral_constant<int, 2 * ND % 3>());
+        }
+        if (c < nchunks) chunk_body(c++, std::integral_constant<int, 0>());
+        if (c < nchunks) chunk_body(c++, std::integral_constant<int, ND % 3>());
+    } else {
+        for (int c = c0; c < nchunks; c++) chunk_body(c, std::integral_constant<int, 0>());
     }
     add_apart();
     store_rows(0);
@@ -1101,8 +1146,8 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 template <int ND, int KS2, bool NORM, bool ODD = false>
 __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     __shared__ __align__(16) char pieces_mem[kTpPieceBytes<3, 3, 3>];
-    __shared__ __align__(16) char pt_mem[kTpPtBytes + (NORM && ND > 1 ? kTpZBytes : 0)];
-    __shared__ __align__(16) float den_mem[NORM ? 2 : 1][NORM ? kChunk : 1][2];
+    __shared__ __align__(16) char pt_mem[kTpPtBytes / 2 * (tp_unrolled(ND, NORM) ? 3 : 2) + (NORM && ND > 1 ? kTpZBytes : 0)];
+    __shared__ __align__(16) float den_mem[NORM ? 3 : 1][NORM ? kChunk : 1][2];
     __shared__ uint32_t order_sh;
     uint32_t which, chain;
     tp_workgroup(p, which, chain);
