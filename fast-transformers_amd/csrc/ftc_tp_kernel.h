@@ -193,10 +193,12 @@ template <int PA, int PB, int PV>
 constexpr int kTpPieceBytes = 3 * (PA + PB + PV) * kChunk * 128;
 constexpr int kTpPtBytes = 2 * 3 * kChunk * 64;
 // Whether a kernel's loop over chunks is unrolled three times, with its buffers in the instructions' offsets
-// (and three of Pt): the fused attention, where the vector instructions of a producer and a consumer together fill
-// their SIMD.  535 of them a chunk -> 470 this way, with the quadrant in two sums for four, half a division and
-// its edges on branches: 80 chains, L=1000 36.4 -> 34.7 us, L=4096 137 -> 124.
-constexpr bool tp_unrolled(int ND, bool NORM) { return NORM && ND == 1; }
+// (and three of Pt).  The fused attention, where the vector instructions of a producer and a consumer together
+// fill their SIMD: 535 of them a chunk -> 470 this way, with the quadrant in two sums for four, half a division and
+// its edges on branches; 80 chains, L=1000 36.4 -> 34.7 us, L=4096 137 -> 124.  bf16 rows, where a consumer's stream
+// is what a chunk waits for: forward, 64 chains, L=2048 32.4 -> 30.5, 80 chains, L=1000 21.4 -> 19.9; 16384 positions of 128
+// chains of 32 x 128, training step 1799 -> 1756.  Not three pieces with two blocks: 108 registers would spill.
+constexpr bool tp_unrolled(int ND, int pieces) { return ND == 1 || pieces < 9; }
 constexpr int kTpZBytes = 4 * 2 * 2 * 64;  // z of the four consumers, fused attention with two blocks
 
 // KS2: groups of 32 rows in the state's last block (1: a state of 65 .. 96 rows, whose last
@@ -241,7 +243,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     static_assert(kChunk == 32 && T % QA == 0 && T % QV == 0, "shape");
     // (the fused attention's rows have 32, 64 or 128 values)
     constexpr bool kFullRows = NORM && KS2 == 2;
-    constexpr bool kUnrolled = tp_unrolled(ND, NORM);
+    constexpr bool kUnrolled = tp_unrolled(ND, PA + PB + PV);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -313,7 +315,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     auto chunk_row0 = [&](int c) -> int { return REV ? rows - kChunk * (c + 1) : kChunk * c; };
     // Position k of the walk goes through LDS buffer (B0 + k) % 3, the first one of the walk proper through
     // buffer 0, so that a loop over those chunks that is unrolled three times knows its buffers.
-    const int B0 = __builtin_amdgcn_readfirstlane((3 - n1 % 3) % 3);
+    const int B0 = kUnrolled ? __builtin_amdgcn_readfirstlane((3 - n1 % 3) % 3) : 0;
     __syncthreads();
 #ifdef FTC_TIMELINE
     // tuning aid: 32 time stamps per workgroup behind the pointer that the host passes in
@@ -918,7 +920,8 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     const __amdgpu_buffer_rsrc_t den_rs = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(den_out ? op.s_out + (int64_t)n * op.so_sn + (int64_t)h * op.so_sh : nullptr), 0,
         den_out ? 4u * (uint32_t)rows : 0u, kRsrcFlags);
-    constexpr int kPSums = NORM && ND == 1 ? 2 : 4;  // sums that the quadrant is added up from
+    // sums that the quadrant is added up from
+    constexpr int kPSums = (NORM && ND == 1) || OfP::count == 1 ? 2 : 4;
     f32x4 Pkeep = {0.f, 0.f, 0.f, 0.f};  // the quadrant summed over the blocks so far
     f32x4 Az = {0.f, 0.f, 0.f, 0.f};     // NORM: phi(a) z of the quadrant's positions
     // (B: the LDS buffer of the chunk's first position, a compile-time number where the loop is unrolled)
@@ -1146,7 +1149,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 template <int ND, int KS2, bool NORM, bool ODD = false>
 __global__ __launch_bounds__(512, 2) void scan_tp_kernel(uint32_t *__restrict__ ws_ptr, ScanArgs p) {
     __shared__ __align__(16) char pieces_mem[kTpPieceBytes<3, 3, 3>];
-    __shared__ __align__(16) char pt_mem[kTpPtBytes / 2 * (tp_unrolled(ND, NORM) ? 3 : 2) + (NORM && ND > 1 ? kTpZBytes : 0)];
+    __shared__ __align__(16) char pt_mem[kTpPtBytes / 2 * (tp_unrolled(ND, 9) ? 3 : 2) + (NORM && ND > 1 ? kTpZBytes : 0)];
     __shared__ __align__(16) float den_mem[NORM ? 3 : 1][NORM ? kChunk : 1][2];
     __shared__ uint32_t order_sh;
     uint32_t which, chain;

@@ -17,7 +17,7 @@ namespace {
 template <int ND, int KS2, bool FORWARD>
 __device__ __forceinline__ void scan_mixed(uint32_t *__restrict__ ws_ptr, const ScanArgs &p) {
     __shared__ __align__(16) char pieces_mem[FORWARD ? kTpPieceBytes<1, 1, 1> : kTpPieceBytes<3, 1, 1>];
-    __shared__ __align__(16) char pt_mem[kTpPtBytes];
+    __shared__ __align__(16) char pt_mem[kTpPtBytes / 2 * 3];
     __shared__ uint32_t order_sh;
     lds_char *const pieces = (lds_char *)pieces_mem, *const pt = (lds_char *)pt_mem;
     uint32_t which, chain;
