@@ -944,18 +944,49 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             // (the first product of a sum adds to a constant)
             if (c == c0 + 4) FTC_STAMP(0);
             __builtin_amdgcn_sched_barrier(0);
-            // phase 1: (1) the quadrant; underneath: tiles 2, 3 of S_w cut into pieces, the
-            // first position-major reads, and the rows of the chunk before go out (their last
-            // matrix instructions have long finished by now; at the end of their own chunk the
-            // wavefront would wait for them)
+            // the quadrant is added up, masked, cut and handed to the others, step by step underneath
+            // the products (bf16 rows: two matrix instructions, and already in phase 1)
+            constexpr bool kEarlyQuadrant = OfP::count == 1;
+            f32x4 P;
+            uint32_t plo[3], phi[3];
+            auto quadrant = [&](int step) {
+                if (step == 1) {
+                    P = kPSums == 2 ? P4[0] + P4[1] : (P4[0] + P4[1]) + (P4[2] + P4[3]);
+                    if (hb > 0) P += Pkeep;
+                    if (!last_block) Pkeep = P;
+                }
+                if (step == 2 && last_block)
+                    split_pair_under_mfma(__uint_as_float(__float_as_uint(P[0]) & keep[0]),
+                                          __uint_as_float(__float_as_uint(P[1]) & keep[1]), plo);
+                if (step == 4 && last_block)
+                    split_pair_under_mfma(__uint_as_float(__float_as_uint(P[2]) & keep[2]),
+                                          __uint_as_float(__float_as_uint(P[3]) & keep[3]), phi);
+                if (step == 6 && last_block) {
+#pragma unroll
+                    for (int k = 0; k < 3; k++) {
+                        const u32x2 xk = {plo[k], phi[k]};
+                        *(lds_vec2 *)(ptc + k * kTileP + pt_waddr) = xk;
+                    }
+                }
+            };
+            // phase 1: (1) the quadrant in turn with (2b) Ot_w = S_w^T a^T for rows 0 .. 31 of the
+            // state; underneath: the rows of the chunk before go out, tiles 2, 3 of S_w are cut into
+            // pieces, the first position-major reads.  (Two matrix instructions to an iteration:
+            // one takes four times what another instruction takes to issue, and with the products
+            // in phases of their own those without vector work beside them ran at the matrix
+            // rate and the others at the rate of issue, twice as long as either.)
 #pragma unroll
             for (int i = 0; i < 12; i++) {
-                const int ks = i % 2, m = i / 2;
+                const int ks = i % 2, m = i / 2, x = i % 2;
+                if (hb == 0 && i < 2) store_rows(i);
                 if (ks < block_ks(hb) && m < OfP::count)
                     P4[i % kPSums] = mfma16(bfr[ks][OfP::x(m)], af[0][ks][OfP::y(m)], i < kPSums ? zero : P4[i % kPSums]);
                 else if (i < kPSums)
                     P4[i % kPSums] = zero;
+                if (m < OfO::count)
+                    O4[x][0] = mfma16(sf[0][OfO::x(m)], af[x][0][OfO::y(m)], i < 2 && hb == 0 ? zero : O4[x][0]);
                 if (i < 4 && block_ks(hb) > 1) cut_s(hb, 1, i);
+                if (kEarlyQuadrant) quadrant(i - 4);
                 if (NORM && ND > 1 && (i == 5 || i == 7)) Z[0][i / 2 - 2] = z_mem[8 * hb + 4 * (i / 2 - 2)];
                 if (NORM && i >= 8) {  // z in pieces
                     uint32_t o[3];
@@ -968,75 +999,44 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                     for (int k = 0; k < 3; k++) zf[k].w[i - 8] = o[k];
                 }
                 tr_frag_into(bt, vf, pc, pcv, i, hb);
-                if (hb == 0 && (i == 5 || i == 7)) store_rows(i == 5 ? 0 : 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (c == c0 + 4) FTC_STAMP(1);
-            // phase 2: first half of (2b) Ot_w = S_w^T a^T; underneath: the last position-major
-            // reads, then the quadrant is added up, masked, cut and handed to the others
-            f32x4 P;
-            uint32_t plo[3], phi[3];
+            // phase 2: (2b) for rows 32 .. 63 in turn with (3) S_w += b^T v_w for tiles 0 and 1;
+            // underneath: the last position-major reads, and the quadrant
 #pragma unroll
             for (int i = 0; i < 12; i++) {
-                const int x = i % 2, ks = (i / 2) % 2, m = i / 4;  // piece products 0..2
-                if (ks < block_ks(hb))
-                    O4[x][ks] = mfma16(sf[ks][OfO::x(m)], af[x][ks][OfO::y(m)], i < 4 && hb == 0 ? zero : O4[x][ks]);
-                else if (i < 4 && hb == 0)
-                    O4[x][ks] = zero;
-                if (i < 3) tr_frag_into(bt, vf, pc, pcv, 12 + i, hb);
-                if constexpr (NORM)
-                    if (i >= 6) Az = mfma16(zf[OfO::x(i - 6)], af[0][0][OfO::y(i - 6)], i == 6 && hb == 0 ? zero : Az);
-                if (i == 4) {
-                    P = kPSums == 2 ? P4[0] + P4[1] : (P4[0] + P4[1]) + (P4[2] + P4[3]);
-                    if (hb > 0) P += Pkeep;
-                    if (!last_block) Pkeep = P;
-                }
-                if (NORM && i == 9 && last_block) {
-                    float m[4];
-#pragma unroll
-                    for (int r = 0; r < 4; r++) m[r] = __uint_as_float(__float_as_uint(P[r]) & keep[r]);
-                    P_sum = (m[0] + m[1]) + (m[2] + m[3]);
-                }
-                if (i == 6 && last_block)
-                    split_pair_under_mfma(__uint_as_float(__float_as_uint(P[0]) & keep[0]),
-                                          __uint_as_float(__float_as_uint(P[1]) & keep[1]), plo);
-                if (i == 8 && last_block)
-                    split_pair_under_mfma(__uint_as_float(__float_as_uint(P[2]) & keep[2]),
-                                          __uint_as_float(__float_as_uint(P[3]) & keep[3]), phi);
-                if (i == 10 && last_block) {
-#pragma unroll
-                    for (int k = 0; k < 3; k++) {
-                        const u32x2 xk = {plo[k], phi[k]};
-                        *(lds_vec2 *)(ptc + k * kTileP + pt_waddr) = xk;
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (c == c0 + 4) FTC_STAMP(2);
-            // phase 3: second half of (2b) in turn with (3) S_w += b^T v_w for tiles 0 and 1
-#pragma unroll
-            for (int i = 0; i < 12; i++) {
-                const int x = i % 2, ks = (i / 2) % 2, m = 3 + i / 4;  // piece products 3..5
-                if (ks < block_ks(hb) && m < OfO::count)
-                    O4[x][ks] = mfma16(sf[ks][OfO::x(m)], af[x][ks][OfO::y(m)], O4[x][ks]);
+                const int x = i % 2, m = i / 2;
+                if (block_ks(hb) > 1 && m < OfO::count)
+                    O4[x][1] = mfma16(sf[1][OfO::x(m)], af[x][1][OfO::y(m)], i < 2 && hb == 0 ? zero : O4[x][1]);
+                else if (i < 2 && hb == 0)
+                    O4[x][1] = zero;
                 if (i < 2 * OfS::count)
                     add_product(hb, i % 2, bt[i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)], i < 2);
-                if constexpr (NORM)
+                if (i < 3) tr_frag_into(bt, vf, pc, pcv, 12 + i, hb);
+                if constexpr (NORM) {
                     if (i < 6) {
+                        Az = mfma16(zf[OfO::x(i)], af[0][0][OfO::y(i)], i == 0 && hb == 0 ? zero : Az);
+                    } else {
                         f32x4 &sum = kApartZ ? Zr[hb][i % 2] : Zr[0][i % 2];
-                        sum = mfma16(bt[i % 2][2 - i / 2], ones, kApartZ || i >= 2 ? sum : zero);
+                        sum = mfma16(bt[i % 2][5 - i / 2], ones, kApartZ || i >= 8 ? sum : zero);
                     }
-                if (NORM && ND > 1) {
-                    if (i == 7 || i == 8) Z[0][i - 7] = z_mem[8 * hb + 4 * (i - 7)];
-                    if (i == 10 || i == 11) z_mem[8 * hb + 4 * (i - 10)] = Z[0][i - 10] + Zr[0][i - 10];
                 }
-                if (NORM && i == 6 && last_block) {
+                if (NORM && ND > 1 && (i == 7 || i == 8)) Z[0][i - 7] = z_mem[8 * hb + 4 * (i - 7)];
+                if (!kEarlyQuadrant) quadrant(i);
+                if (NORM && i == 7 && last_block) {
+                    float m4[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) m4[r] = __uint_as_float(__float_as_uint(P[r]) & keep[r]);
+                    P_sum = (m4[0] + m4[1]) + (m4[2] + m4[3]);
+                }
+                if (NORM && i == 9 && last_block) {
                     P_sum = sum_of_lane_groups(P_sum);
                     if (g == 0) den_mem[pt_buf][16 * ih + ln][w >> 1] = (has_z ? Az[0] : 0.f) + P_sum;
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (c == c0 + 4) FTC_STAMP(3);
+            if (c == c0 + 4) FTC_STAMP(2);
             buf = next_buf(buf);
             wg_barrier();
             if (c == c0 + 4) FTC_STAMP(4);
@@ -1072,6 +1072,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             for (int i = 0; i < 4; i++) {
                 if (block_ks(hb) > 1 && i < 2 * OfS::count)
                     add_product(hb, 2 + i % 2, bt[2 + i % 2][OfS::x(i / 2)], vf[OfS::y(i / 2)], i < 2);
+                if (NORM && ND > 1 && i < 2) z_mem[8 * hb + 4 * i] = Z[0][i] + Zr[0][i];
                 cut_s((hb + 1) % ND, 0, i);
                 rm_frag(pn, i, (hb + 1) % ND);  // (past the last chunk: a buffer of zeros)
                 __builtin_amdgcn_sched_barrier(0);
