@@ -89,19 +89,26 @@ int tp_kernel_segments(int64_t units, int64_t L, bool wide, bool others, bool lo
 
 // Where to cut a chain of `chunks` chunks into (at most) `nseg` segments for the
 // chain-parallel kernel.  The workgroup of a segment first rebuilds the state before its
-// segment from the chunks in front of it (measured: 0.55 to 0.6 of the time of a chunk that
-// also produces rows -- 0.75 against 1.3 us on the fp16-piece kernel with every workgroup
-// streaming rows), so later segments are made shorter until all workgroups finish together:
-// the starts (multiples of kTpAhead chunks, what the producers request ahead) that minimise the
-// longest workgroup.  Returns the number of segments; start[0 .. n] filled (start[n] = chunks).
-int tp_segment_starts(int64_t chunks, int nseg, int32_t *start) {
-    const int groups = (int)((chunks + kTpAhead - 1) / kTpAhead);
+// segment from the chunks in front of it, so later segments are made shorter until all
+// workgroups finish together: the starts (multiples of `step` chunks) that minimise the longest
+// workgroup.  `state_only`: the time of a chunk walked for its state alone, against one that also
+// produces rows: 0.6 on two fp16 pieces (0.75 against 1.3 us with every workgroup streaming rows); on
+// three bf16 pieces 0.45 where a state of 33 to 64 rows writes fp32 results, 0.55 otherwise and for two
+// segments of bf16 rows (128 chains, L=1088, forward 25.2 against 26.0 at 0.45).  Three pieces of fp32
+// rows may start half of what the producers request ahead (kTpAhead) further on (kHalfTrips).  Measured
+// against 0.6 and steps of kTpAhead for all, whose last one counted as whole, 22 shapes drawn for each,
+// geometric means of the time: fused attention of 64 x 64 0.928 (at 0.55: 0.940), odd widths 0.936;
+// 80 chains, L=1000, fused: 38.5 -> 35 us; bf16 rows forward, 64 chains, L=1000: 17.6 -> 16.8, 49,
+// L=1588: 23.7 -> 21.7; backward, 20 chains, L=900: 20.5 -> 19.2, 31, L=407: 15.0 -> 13.0.
+// Returns the number of segments; start[0 .. n] filled (start[n] = chunks).
+int tp_segment_starts(int64_t chunks, int nseg, int32_t *start, int step, double state_only) {
+    const int groups = (int)((chunks + step - 1) / step);
     nseg = std::max(1, std::min(std::min(nseg, groups), kMaxTpSegments));
-    double kStateOnly = 0.6;
-    if (tuning().tp_ratio >= 0) kStateOnly = tuning().tp_ratio;  // tuning aid
+    if (tuning().tp_ratio >= 0) state_only = tuning().tp_ratio;  // tuning aid
+    auto chunk = [&](int g) -> int { return (int)std::min<int64_t>(step * g, chunks); };
     // best[s][g]: smallest achievable longest time of segments s .. nseg-1 when segment s
     // starts at group g (dynamic programme from the last segment back)
-    constexpr int kMaxGroups = 64;  // 256 chunks
+    constexpr int kMaxGroups = 64;
     if (groups > kMaxGroups || nseg == 1) {
         start[0] = 0, start[1] = (int32_t)chunks;
         return 1;
@@ -114,12 +121,14 @@ int tp_segment_starts(int64_t chunks, int nseg, int32_t *start) {
     for (int s = nseg - 1; s >= 0; s--)
         for (int g = s; g < groups; g++)
             for (int e = g + 1; e <= groups - (nseg - 1 - s); e++) {
-                const double t = std::max(kStateOnly * g + (e - g), best[s + 1][e]);
+                const double own = state_only * chunk(g) + (chunk(e) - chunk(g));
+                if (own >= best[s][g]) break;  // (it grows with e)
+                const double t = std::max(own, best[s + 1][e]);
                 if (t < best[s][g]) best[s][g] = t, next[s][g] = e;
             }
     int g = 0;
     for (int s = 0; s < nseg; s++) {
-        start[s] = kTpAhead * g;
+        start[s] = chunk(g);
         g = next[s][g];
     }
     start[nseg] = (int32_t)chunks;
@@ -401,7 +410,7 @@ void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_
     if (chunks <= (bf16_results ? 1024 : 256)) {
         int32_t start[kMaxTpSegments + 1];
         int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), chunks)) : 1;
-        n = tp_segment_starts(chunks, n, start);
+        n = tp_segment_starts(chunks, n, start, kTpAhead, 0.6);
         double longest = (double)chunks;
         if (n > 1) {
             longest = 0;
@@ -743,7 +752,7 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
         longest = 1.6 * seg_chunks + 4.0;
     } else {
         int32_t start[kMaxTpSegments + 1];
-        nseg = tp_segment_starts((L + kChunk - 1) / kChunk, nseg, start);
+        nseg = tp_segment_starts((L + kChunk - 1) / kChunk, nseg, start, kTpAhead, 0.6);
         for (int s = 0; s < nseg; s++)
             longest = std::max(longest, 0.6 * start[s] + (double)(start[s + 1] - start[s]));
     }
@@ -902,7 +911,12 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         pl.workspace_bytes = tp_exchange_workspace_bytes(chains * blocks, pl.nseg,
                                                          fused_tp ? fused_tp_state_rows(D) : grads ? kGradStateRows : D);
     } else if (tp) {  // one workgroup per chain segment, nothing to exchange
-        pl.nseg = tp_segment_starts((L + kChunk - 1) / kChunk, tp_nseg, tp_start);
+        const int64_t chunks = (L + kChunk - 1) / kChunk;
+        if (tph_takes_rows(D) && !(odd && forced) && !fused && combo == kFFFF)  // (scan_tph_kernel)
+            pl.nseg = tp_segment_starts(chunks, tp_nseg, tp_start, kTpAhead, 0.6);
+        else  // (half steps beyond 64 chunks: a longer search for a smaller share of a segment)
+            pl.nseg = tp_segment_starts(chunks, tp_nseg, tp_start, combo == kFFFF && chunks <= 64 ? kTpAhead / 2 : kTpAhead,
+                                        D > 32 && D <= 64 && scans[0].out.dtype == FTC_F32 && (fused || tp_nseg > 2) ? 0.45 : 0.55);
         pl.seg_len = (int)L;
         pl.waves = chains * pl.nseg;
         pl.workspace_bytes = 0;

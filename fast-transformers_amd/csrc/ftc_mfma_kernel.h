@@ -475,7 +475,8 @@ struct ScanArgs {
     // backward of the fused attention only (scan_tph_gradients_kernel): dd and 1 / den, one per position
     const float *row_dd, *row_rden;
     // chain-parallel kernel only (ftc_tp_kernel.h): segment s of a chain is chunks
-    // tp_start[s] .. tp_start[s + 1] - 1 (starts are multiples of kTpAhead)
+    // tp_start[s] .. tp_start[s + 1] - 1 (starts are multiples of kTpAhead; of half of it
+    // on three bf16 pieces of fp32 rows)
     int32_t tp_start[kMaxTpSegments + 1];
     // ... or, with an exchange of segment sums (tp_exchange != 0), nseg segments of
     // tp_seg_chunks chunks (a multiple of kTpAhead), taken in the order of arrival

@@ -244,6 +244,10 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     // (the fused attention's rows have 32, 64 or 128 values)
     constexpr bool kFullRows = NORM && KS2 == 2;
     constexpr bool kUnrolled = tp_unrolled(ND, PA + PB + PV);
+    // Segments may start at half a trip of the first walk (two blocks: a chunk is two positions, so they may
+    // without it).  Not with bf16 rows, whose launches took 0.1 us longer with the code, whole chains too (forward,
+    // 58 chains, L=196 7.98 -> 8.10 us; 38, L=1291 18.4 in half steps, 18.1 in whole ones).
+    constexpr bool kHalfTrips = ND == 1 && PA + PB + PV == 9;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -297,7 +301,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     }
     const int c0 = exchange ? seg * p.tp_seg_chunks : p.tp_start[seg];
     const int nchunks = min(total_chunks, exchange ? c0 + p.tp_seg_chunks : p.tp_start[seg + 1]);
-    // the chunks walked for their state alone: so0 .. so0 + n1 - 1 (n1 a multiple of PF; the
+    // the chunks walked for their state alone: so0 .. so0 + n1 - 1 (n1 a multiple of PF / 2; the
     // last segment of an exchange has no reader for its sum)
     const int so0 = exchange ? c0 : 0;
     const int n1c = exchange ? (seg + 1 < (int)nseg ? nchunks - c0 : 0) : c0;
@@ -424,7 +428,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             }
         };
         // position k of the walk goes to its LDS buffer through register set k % PF.  The
-        // first n1 positions (a multiple of PF) only feed the state: no piece of a, and the
+        // first n1 positions (a multiple of PF / 2) only feed the state: no piece of a, and the
         // consumers, who have little to do there, cut rows 16 .. 31 of b and v themselves.
         auto cut = [&](const Raw &r, int buf, bool own, int hb, int v) {
             lds_char *const pc = unit_pc + buf * kBufBytes;
@@ -444,22 +448,34 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
             if (!own) asm volatile("" ::"v"(r.a[0]), "v"(r.a[1]), "v"(r.b[1]));
             if (!own && hb == 0) asm volatile("" ::"v"(r.v[1]));
         };
-#pragma unroll
-        for (int j = 0; j < PF; j++) fetch(raw[j], j, j % ND);
         // Barrier number k (k = 0: before the first position; k >= 1: in the middle of
         // position k - 1) finds position k cut.  The last one finds a chunk of zeros.
         // Two loops whose bodies are straight-line code, so that the waits inside them count
         // requests instead of draining them.
         int buf = B0;
-        for (int v = 0; v < n1; v += PF) {
+        auto state_only = [&](int v, int j) {  // (v + j: the position, j: its register set)
+            cut(raw[j], buf, false, j % ND, v + j);
+            fetch(raw[j], v + j + PF, j % ND);
+            buf = buf == 2 ? 0 : buf + 1;
+            wg_barrier();
+            __builtin_amdgcn_sched_barrier(0);  // one chunk at a time, in this order
+        };
+        // (half a trip in front where n1 is not a multiple of PF: the sets are requested in the order in which
+        // they are used, and both ways leave them in the order that the loops count on)
+        int first = 0;
+        if (kHalfTrips && n1 % PF != 0) {
+            static_assert(PF == 4, "half a trip: the sets of its second half first");
+            fetch(raw[2], 0, 0), fetch(raw[3], 1, 0), fetch(raw[0], 2, 0), fetch(raw[1], 3, 0);
+            state_only(-2, 2);
+            state_only(-2, 3);
+            first = 2;
+        } else {
 #pragma unroll
-            for (int j = 0; j < PF; j++) {
-                cut(raw[j], buf, false, j % ND, v + j);
-                fetch(raw[j], v + j + PF, j % ND);
-                buf = buf == 2 ? 0 : buf + 1;
-                wg_barrier();
-                __builtin_amdgcn_sched_barrier(0);  // one chunk at a time, in this order
-            }
+            for (int j = 0; j < PF; j++) fetch(raw[j], j, j % ND);
+        }
+        for (int v = first; v < n1; v += PF) {
+#pragma unroll
+            for (int j = 0; j < PF; j++) state_only(v, j);
         }
         // (whole trips in the loop, the rest after it: a way out of the middle of the loop
         // would join the paths at the loop's head and spoil the counting)
@@ -772,50 +788,63 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         auto ccut_v = [&](const RawC &r, int bufk) {
             QuadV::to_lds(v_own.of(r.v), unit_pc + bufk * kBufBytes + kOffV, kTileV, v_waddr);
         };
-#pragma unroll
-        for (int j = 0; j < PF; j++) cfetch(rawc[j], j, j % ND);
-        ccut_b(rawc[0], B0, 0);
-        ccut_v(rawc[0], B0);
-        cfetch(rawc[0], PF, 0);
-        wg_barrier();
-        FTC_STAMP(13);  // first chunk cut
         Frag bt2[4][PB] = {}, vf2[PV] = {};  // (the first round multiplies zeros)
         int bufn = next_buf(B0);           // LDS buffer of the position after the one at hand
-        for (int c = 0; c < n1; c += PF) {
+        auto state_only = [&](int c, int j) {  // (position c + j, in register set j)
+            const lds_char *pc = unit_pc + buf * kBufBytes;
+            const lds_char *pcv = j % ND == 0 ? pc : unit_pc + prev_buf(buf) * kBufBytes;
+            // position c + j + 1 is cut under the matrix instructions of position
+            // c + j - 1 (position n1 is all the producers')
+            const bool cut_next = j < PF - 1 || c + PF < n1;
+            const RawC &rn = rawc[(j + 1) % PF];
+            const int hp = (j + ND - 1) % ND;  // block of the position before
 #pragma unroll
-            for (int j = 0; j < PF; j++) {
-                const lds_char *pc = unit_pc + buf * kBufBytes;
-                const lds_char *pcv = j % ND == 0 ? pc : unit_pc + prev_buf(buf) * kBufBytes;
-                // position c + j + 1 is cut under the matrix instructions of position
-                // c + j - 1 (position n1 is all the producers')
-                const bool cut_next = j < PF - 1 || c + PF < n1;
-                const RawC &rn = rawc[(j + 1) % PF];
-                const int hp = (j + ND - 1) % ND;  // block of the position before
-#pragma unroll
-                for (int i = 0; i < 24; i++) {
-                    if (j % 2 == 0) {
-                        add_first(hp, i, bt2, vf2);
-                        if constexpr (NORM)
-                            add_keys(hp, i, bt2);
-                        tr_frag_into(bt, vf, pc, pcv, i, j % ND);
-                    } else {
-                        add_first(hp, i, bt, vf);
-                        if constexpr (NORM)
-                            add_keys(hp, i, bt);
-                        tr_frag_into(bt2, vf2, pc, pcv, i, j % ND);
-                    }
-                    if (i == 15 && cut_next) ccut_b(rn, bufn, c + j + 1);
-                    if (i == 19 && cut_next && (j + 1) % ND == 0) ccut_v(rn, bufn);
-                    __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < 24; i++) {
+                if (j % 2 == 0) {
+                    add_first(hp, i, bt2, vf2);
+                    if constexpr (NORM)
+                        add_keys(hp, i, bt2);
+                    tr_frag_into(bt, vf, pc, pcv, i, j % ND);
+                } else {
+                    add_first(hp, i, bt, vf);
+                    if constexpr (NORM)
+                        add_keys(hp, i, bt);
+                    tr_frag_into(bt2, vf2, pc, pcv, i, j % ND);
                 }
-                if (kFirstSums) add_chunk_sums(hp, 2, 2 * block_ks(hp));
-                cfetch(rawc[(j + 1) % PF], c + j + 1 + PF, (j + 1) % ND);
-                buf = bufn;
-                bufn = next_buf(bufn);
-                wg_barrier();
+                if (i == 15 && cut_next) ccut_b(rn, bufn, c + j + 1);
+                if (i == 19 && cut_next && (j + 1) % ND == 0) ccut_v(rn, bufn);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (kFirstApart && c % 8 == 0) add_apart();
+            if (kFirstSums) add_chunk_sums(hp, 2, 2 * block_ks(hp));
+            cfetch(rawc[(j + 1) % PF], c + j + 1 + PF, (j + 1) % ND);
+            buf = bufn;
+            bufn = next_buf(bufn);
+            wg_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int first = 0;
+        if (kHalfTrips && n1 % PF != 0) {  // (half a trip in front, as the producers do)
+            cfetch(rawc[2], 0, 0), cfetch(rawc[3], 1, 0), cfetch(rawc[0], 2, 0), cfetch(rawc[1], 3, 0);
+            ccut_b(rawc[2], B0, 0);
+            ccut_v(rawc[2], B0);
+            cfetch(rawc[2], PF, 0);
+            wg_barrier();
+            state_only(-2, 2);
+            state_only(-2, 3);
+            first = 2;
+        } else {
+#pragma unroll
+            for (int j = 0; j < PF; j++) cfetch(rawc[j], j, j % ND);
+            ccut_b(rawc[0], B0, 0);
+            ccut_v(rawc[0], B0);
+            cfetch(rawc[0], PF, 0);
+            wg_barrier();
+        }
+        FTC_STAMP(13);  // first chunk cut
+        for (int c = first; c < n1; c += PF) {
+#pragma unroll
+            for (int j = 0; j < PF; j++) state_only(c, j);
+            if (kFirstApart && c % 8 < PF) add_apart();
         }
         // the last of these positions (n1 is even: its fragments are in the second set)
 #pragma unroll

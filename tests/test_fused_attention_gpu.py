@@ -285,6 +285,18 @@ def test_many_chains(lib, shape):
     assert torch.equal(fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6), out)
 
 
+@pytest.mark.parametrize("shape", [(20, 300, 3, 64, 64), (10, 1000, 6, 64, 64), (64, 900, 2, 64, 32), (25, 129, 2, 32, 64)],
+                         ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s)
+def test_segments_that_start_at_half_a_trip(lib, shape):
+    """Cuts at 2 modulo 4 chunks: the first walk begins with half a trip through its register sets."""
+    N, L, H, E, M = shape
+    q, k, v = inputs(N, L, H, E, M, seed=290 + L)
+    lengths = torch.arange(N) * L // N + 1
+    out = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
+    assert lib.ftc_last_kernel() == b"scan_tp_kernel<NORM>"
+    gate(out.cpu(), q, k, v, lengths, 1e-6)
+
+
 @pytest.mark.parametrize("small", ["q_rows", "k_early_rows", "v_columns", "v_early_rows"])
 @pytest.mark.parametrize("shape", [(6, 300, 8, 64, 64), (3, 2100, 8, 64, 64), (6, 520, 8, 64, 32)],
                          ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s)
