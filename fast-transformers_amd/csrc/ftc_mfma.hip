@@ -785,7 +785,8 @@ int64_t fused_tp_state_rows(int64_t D) { return (D + 63) / 64 * 64 + 64; }
 // L=1000 160 / 130; 384 chains, L=2774 350 / 286; 216 chains, L=134 17.6 / 15.1; 64 chains, L=1500
 // 50.3 / 45.2; 32 chains, L=4096 62.9 / 53.9; 32 chains, L=134 17.5 / 11.6, L=500 23.4 / 19.6, L=700 26.5 / 25.6;
 // 8 chains, L=200 14.9 / 13.0; but 8 chains, L=500 17.5 / 19.3, 24 chains, L=700 23.9 / 25.5, 36 chains, L=1000
-// 31.5 / 32.7, 48 chains, L=1500 43.8 / 46.3.  One width of 32: 80 chains, L=1000 41.6 / 34.8 (64 x 32) and
+// 31.5 / 32.7, 48 chains, L=1500 43.8 / 46.3 (the latter before tp_unrolled and the cuts of tp_segment_starts, which
+// took 0.86 of the time for 80 chains, L=1000, and 0.93 over drawn shapes).  One width of 32: 80 chains, L=1000 41.6 / 34.8 (64 x 32) and
 // 36.7 / 32.0, 32 chains, L=300 19.1 / 14.8 and 16.6 / 13.8; but 48 chains, L=1000 32.3 / 33.0 and 29.1 / 30.7, 64 chains,
 // L=1500 42.9 / 44.2, 32 x 64 on up to four chunks 8.2 / 8.5, more than a round of workgroups 102 / 116, with an
 // exchange 95.7 / 106.  32 x 32: 31.7 / 31.3 and 64 / 96.

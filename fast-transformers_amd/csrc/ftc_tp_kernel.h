@@ -34,6 +34,8 @@
 //           pieces and written to LDS as rows i with j contiguous;
 //      (2b) Ot_w  = S_w^T a^T       16 f x 32 i, contraction over d;
 //      (3)  S_w  += b^T v_w         64 d x 16 f, contraction over the chunk's positions j;
+//           ((2b) of rows 0 .. 31 runs in turn with (1), of rows 32 .. 63 with (3): a sum
+//           waits for its last product while the others go on)
 //      -- barrier: all of Pt is in LDS --
 //      (2a) Ot_w += v_w^T Pt        contraction over j;   Ot_w is stored under (1) of the
 //           next chunk, when its last matrix instructions have long finished.
@@ -43,7 +45,7 @@
 //    stand, the A operand of k-step ks of (2b) with k-slots d = 32 ks + 8 g + t -- the order
 //    of a 16-byte read of a row of a or b, whose fragments serve (1) and (2b) alike.
 //  * One workgroup barrier per chunk, after Pt is written.  The piece tiles rotate through
-//    three LDS buffers and Pt through two: when the barrier of chunk c falls, the producers
+//    three LDS buffers and Pt through two (three where the loop is unrolled, tp_unrolled): when the barrier of chunk c falls, the producers
 //    have cut chunk c + 1 (the consumers request its row-major fragments right away, under
 //    (2a)) and go on to cut chunk c + 2 into the buffer of chunk c - 1, which nobody has
 //    read since the barrier before.

@@ -7,8 +7,8 @@
 // Division of labour, chunking, LDS tiles, swizzles, segments and the exchange of segment
 // sums are those of ftc_tp_kernel.h (one workgroup walks one chain; four consumer wavefronts
 // hold the state as slabs of 16 columns and share the chunk product Pt through LDS; producer
-// wavefronts -- eight here, one quad of every operand per lane and position -- fetch rows
-// four chunks ahead and cut them into piece tiles).  What differs is the arithmetic that
+// wavefronts -- eight here, in two groups of four that take positions in turn, two quads of
+// every operand per lane -- fetch rows four chunks ahead and cut them into piece tiles).  What differs is the arithmetic that
 // stands for an fp32 product:
 //
 //  * Every fp32 value x is scaled by a power of two and cut into TWO fp16 pieces, both rounded
