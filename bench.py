@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139323564, "2470b03351e57230"),
-    "cfg3": (2608551109, "2470b03351e57230"),
-    "cfg5": (4163550728, "2470b03351e57230"),
-    "wide": (1877064671, "2470b03351e57230"),
+    "cfg2": (139921970, "71830fc2a367f114"),
+    "cfg3": (2604889146, "71830fc2a367f114"),
+    "cfg5": (4152541883, "71830fc2a367f114"),
+    "wide": (1877067329, "71830fc2a367f114"),
 }
 
 WORKLOADS = {
