@@ -780,16 +780,17 @@ int64_t fused_tp_state_rows(int64_t D) { return (D + 63) / 64 * 64 + 64; }
 
 // The fused attention launch on the chain-parallel kernel: its plan is that of a single 64 x 64
 // scan whatever the widths (a chunk costs the same).  Returns false: the workgroup form, whose
-// units split L and which carries two units of 32 value columns per workgroup.  Measured (us, the
-// workgroup form / this way), 64 x 64: 80 chains, L=1000 47.8 / 36.9, L=4096 138 / 114; 512 chains,
-// L=1000 160 / 130; 384 chains, L=2774 350 / 286; 216 chains, L=134 17.6 / 15.1; 64 chains, L=1500
-// 50.3 / 45.2; 32 chains, L=4096 62.9 / 53.9; 32 chains, L=134 17.5 / 11.6, L=500 23.4 / 19.6, L=700 26.5 / 25.6;
-// 8 chains, L=200 14.9 / 13.0; but 8 chains, L=500 17.5 / 19.3, 24 chains, L=700 23.9 / 25.5, 36 chains, L=1000
-// 31.5 / 32.7, 48 chains, L=1500 43.8 / 46.3 (the latter before tp_unrolled and the cuts of tp_segment_starts, which
-// took 0.86 of the time for 80 chains, L=1000, and 0.93 over drawn shapes).  One width of 32: 80 chains, L=1000 41.6 / 34.8 (64 x 32) and
-// 36.7 / 32.0, 32 chains, L=300 19.1 / 14.8 and 16.6 / 13.8; but 48 chains, L=1000 32.3 / 33.0 and 29.1 / 30.7, 64 chains,
-// L=1500 42.9 / 44.2, 32 x 64 on up to four chunks 8.2 / 8.5, more than a round of workgroups 102 / 116, with an
-// exchange 95.7 / 106.  32 x 32: 31.7 / 31.3 and 64 / 96.
+// units split L and which carries two units of 32 value columns per workgroup.  The lines are where the
+// two cross; this way / the workgroup form, time, on both sides of them: 64 x 64, 16 chunks, 4 chains 0.98; 21
+// chunks, 20 chains 0.96, 16 chains 1.00; 24 chunks, 20 chains 0.97, 16 chains 1.00; 32 chunks, 36 chains 0.93, 32 (there
+// and below with an exchange) 0.98; 36 chunks, 40 chains 0.92; 42 chunks, 40 chains 0.95, 36 chains 1.00; 48 chunks,
+// 36 chains 0.93, 28 chains 0.97; 64 chunks, 24 chains 0.91, 20 chains 0.98; far from them 64 chains, 10, 24, 42
+// and 64 chunks 0.54, 0.68, 0.80 and 0.85.  64 x 32: 16 chunks, 8 chains 0.89; 24 chunks, 40 chains 0.84; 32 chunks,
+// 40 chains 0.95; 40 chunks, 56 chains 0.90, 48 chains 0.96; 48 chunks, 80 chains 0.89, 64 chains 1.02.  32 x 64: 10
+// chunks, 16 chains 0.94, 8 chains 1.00; 16 chunks, 24 chains 0.96, 16 chains 1.06; 24 chunks, 40 chains 0.91, 32
+// chains 1.11; 32 chunks, 56 chains 0.94, 48 chains 1.00; 40 chunks, 64 chains 0.93; 48 chunks, 80 chains 0.92, 64 chains
+// 1.08.  32 x 32 stays: 1000 positions 31.7 / 31.3 us the other way round.  One width of 32 on more than a round of
+// workgroups, or with an exchange, stays too: 102 / 116 and 95.7 / 106 us.
 // Chains of more than 256 chunks are not walked whole on three bf16 pieces (tp_plan_compute).
 //
 // Rows of 128 have no other fused form: the plan is that of such a scan where the chain-parallel kernel
@@ -809,10 +810,23 @@ bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, i
     if (*nseg == 0 || tuning().wg == 0) return *nseg > 0;  // (FTC_WG=0: tuning aid)
     // the fewest chains without an exchange, where the two cross
     const bool square = D == 64 && F == 64;
-    int64_t least = chunks <= 10 ? 4 : chunks <= 16 ? 20 : chunks <= 24 ? 32 : chunks <= 32 && square ? 40 : 56;
-    if (D == 32) least = chunks <= 4 ? INT64_MAX : chunks <= 7 ? 8 : chunks <= 10 ? 20 : chunks <= 16 ? 28 : chunks <= 24 ? 44 : 56;
-    const bool take = *seg_chunks > 0 ? square && chains >= 24 && chunks >= 64
-                                      : (square || ((D == 64 || F == 64) && chains <= 256 && chunks <= 32)) && chains >= least;
+    int64_t least;
+    if (square)
+        least = chunks <= 16 ? 4 : chunks <= 24 ? 20 : chunks <= 32 ? 36 : 40;
+    else if (D == 64)
+        least = chunks <= 10 ? 4 : chunks <= 16 ? 8 : chunks <= 24 ? 32 : chunks <= 32 ? 40 : chunks <= 44 ? 56 : 80;
+    else
+        least = chunks <= 4    ? INT64_MAX
+                : chunks <= 7  ? 8
+                : chunks <= 10 ? 16
+                : chunks <= 16 ? 24
+                : chunks <= 24 ? 40
+                : chunks <= 28 ? 48
+                : chunks <= 32 ? 56
+                : chunks <= 44 ? 64
+                               : 80;
+    const bool take = *seg_chunks > 0 ? square && chains >= (chunks >= 64 ? 24 : 36) && chunks >= 44
+                                      : (square || ((D == 64 || F == 64) && chains <= 256 && chunks <= 60)) && chains >= least;
     if (!take) *nseg = *seg_chunks = 0;
     return take;
 }

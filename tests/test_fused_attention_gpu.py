@@ -285,6 +285,19 @@ def test_many_chains(lib, shape):
     assert torch.equal(fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6), out)
 
 
+@pytest.mark.parametrize("shape", [(1, 512, 4, 64, 64), (5, 640, 4, 64, 64), (9, 900, 4, 64, 64), (10, 1300, 4, 64, 64),
+                                   (9, 1600, 4, 64, 64), (2, 500, 4, 64, 32), (10, 1000, 4, 64, 32), (14, 1280, 4, 64, 32),
+                                   (20, 1900, 4, 64, 32), (4, 300, 4, 32, 64), (6, 500, 4, 32, 64), (12, 890, 4, 32, 64),
+                                   (16, 1400, 4, 32, 64)], ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s)
+def test_fewest_chains_of_the_chain_parallel_form(lib, shape):
+    """The shapes at the lines between the two forms, on this side of them."""
+    N, L, H, E, M = shape
+    q, k, v = inputs(N, L, H, E, M, seed=310 + L)
+    out = fused(lib, q.cuda(), k.cuda(), v.cuda(), None, 1e-6)
+    assert lib.ftc_last_kernel().startswith(b"scan_tp_kernel<NORM>")
+    gate(out.cpu(), q, k, v, None, 1e-6)
+
+
 @pytest.mark.parametrize("shape", [(20, 300, 3, 64, 64), (10, 1000, 6, 64, 64), (64, 900, 2, 64, 32), (25, 129, 2, 32, 64)],
                          ids=lambda s: "n%d_l%d_h%d_e%d_m%d" % s)
 def test_segments_that_start_at_half_a_trip(lib, shape):
