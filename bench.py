@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139921970, "71830fc2a367f114"),
-    "cfg3": (2604889146, "71830fc2a367f114"),
-    "cfg5": (4152541883, "71830fc2a367f114"),
-    "wide": (1877067329, "71830fc2a367f114"),
+    "cfg2": (139791680, "4c9502e29e4adf1a"),
+    "cfg3": (2616815818, "4c9502e29e4adf1a"),
+    "cfg5": (4154106356, "4c9502e29e4adf1a"),
+    "wide": (1877178962, "4c9502e29e4adf1a"),
 }
 
 WORKLOADS = {
