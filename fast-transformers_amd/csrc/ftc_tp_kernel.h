@@ -101,13 +101,6 @@ __device__ __forceinline__ constexpr int b_tile_column(int d) {
     return 32 * (d / 32) + 16 * ((d / 4) % 2) + 4 * ((d % 32) / 8) + d % 4;
 }
 
-// 1 / x: the estimate and one step of Newton's, half as many instructions as the division, which is left what
-// is special (zero, infinite, NaN, or below 2^-126)
-__device__ __forceinline__ float reciprocal(float x) {
-    const float r = __builtin_amdgcn_rcpf(x), e = fmaf(-x, r, 1.0f);
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(e != e) != 0, 0)) return 1.0f / x;
-    return fmaf(e, r, r);
-}
 // sum over the four groups of 16 lanes, in every lane: v_permlane16_swap exchanges the odd groups
 // of its first operand with the even groups of its second, v_permlane32_swap the halves
 __device__ __forceinline__ float sum_of_lane_groups(float x) {
@@ -196,8 +189,8 @@ constexpr int kTpPieceBytes = 3 * (PA + PB + PV) * kChunk * 128;
 constexpr int kTpPtBytes = 2 * 3 * kChunk * 64;
 // Whether a kernel's loop over chunks is unrolled three times, with its buffers in the instructions' offsets
 // (and three of Pt).  The fused attention, where the vector instructions of a producer and a consumer together
-// fill their SIMD: 535 of them a chunk -> 470 this way, with the quadrant in two sums for four, half a division and
-// its edges on branches; 80 chains, L=1000 36.4 -> 34.7 us, L=4096 137 -> 124.  bf16 rows, where a consumer's stream
+// fill their SIMD: 535 of them a chunk -> 515 this way, with the quadrant in two sums for four and its
+// edges on branches; 80 chains, L=1000 36.4 -> 34.7 us, L=4096 137 -> 124.  bf16 rows, where a consumer's stream
 // is what a chunk waits for: forward, 64 chains, L=2048 32.4 -> 30.5, 80 chains, L=1000 21.4 -> 19.9; 16384 positions of 128
 // chains of 32 x 128, training step 1799 -> 1756.  Not three pieces with two blocks: 108 registers would spill.
 constexpr bool tp_unrolled(int ND, int pieces) { return ND == 1 || pieces < 9; }
@@ -1089,7 +1082,7 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
                     for (int x = 0; x < 2; x++) {
                         const float *part = den_mem[pt_buf][16 * (x ^ ih) + ln];
                         const float den = (part[0] + part[1]) + p.eps;
-                        r_den[x] = reciprocal(den);
+                        r_den[x] = 1.0f / den;
                         // (the caller's copy of the denominators, for the backward)
                         if (den_out)
                             __builtin_amdgcn_raw_buffer_store_b32(

@@ -15,6 +15,7 @@ and an element-wise violation fraction (1e-5 + 1e-4 |want|) no worse than twice 
 float32 CPU restatement shows against float64, plus 6e-4.
 """
 import ctypes
+import math
 import os
 
 import numpy as np
@@ -699,6 +700,39 @@ def test_non_finite_inputs_propagate_as_in_the_composition(lib):
     assert not bad_fused[0, :40, 0].any() and not bad_fused[0, :200, 1].any()
     ok = ~bad_fused
     assert (y_fused[ok] - y_composed[ok]).abs().max() <= 1e-4 * y_composed[ok].abs().max()
+
+
+@pytest.mark.parametrize("E,M", [(64, 64), (64, 32), (32, 64), (128, 128)])
+@pytest.mark.parametrize("what", ["large", "small"])
+def test_denominators_at_the_ends_of_the_range(lib, E, M, what):
+    """Denominators of 3 x 2^126, whose reciprocal is below 2^-126, and of 2^-127 (3 x 2^-122 beside an eps that
+    leaves that much of it): rows are quotients all the same.  One feature counts, of three keys."""
+    from fast_transformers_amd import _native
+    N, L, H = 8, 500, 4
+    v = torch.rand(N, L, H, M, generator=torch.Generator().manual_seed(41))    # (three of them stay below 4)
+    q, k = torch.full((N, L, H, E), -200.0), torch.full((N, L, H, E), -200.0)   # phi is zero
+    k[:, :3, :, 5] = q[..., 5] = 2.0 ** 63 if what == "large" else -61 * math.log(2.0)
+    eps = 0.0 if what == "large" else -(3 * 2.0 ** -122 - 2.0 ** -127)
+    q, k, v, lengths = q.cuda(), k.cuda(), v.cuda(), torch.full((N,), 3).cuda()
+    out, den = torch.empty(N, L, H, M, device="cuda"), torch.empty(N, H, L, 1, device="cuda")
+    nbytes = lib.ftc_causal_linear_attention_wide_workspace_bytes(N, H, L, E, M, _native.FTC_F32)
+    assert nbytes >= 0, _native.last_error()
+    ws = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device="cuda")
+    d = [_native.describe(t.permute(0, 2, 1, 3)) for t in (q, k, v, out)] + [_native.describe(den)]
+    rc = lib.ftc_causal_linear_attention_wide_forward(
+        *(ctypes.byref(x) for x in d[:3]), ctypes.c_void_p(lengths.data_ptr()), ctypes.c_float(eps), ctypes.byref(d[3]),
+        ctypes.byref(d[4]), ctypes.c_void_p(ws.data_ptr()), nbytes, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, _native.last_error()
+    torch.cuda.synchronize()
+    assert lib.ftc_last_kernel().startswith(b"scan_tp_kernel<NORM>")
+    got, d = out.cpu()[:, 2:].double(), den.cpu().permute(0, 2, 1, 3)[:, 2:].double()
+    products = 2.0 ** 126 if what == "large" else 2.0 ** -122
+    assert bool(((d == 3 * products) if what == "large" else (d - 2.0 ** -127).abs() < 2.0 ** -129).all()), d.max().item()
+    want = v.cpu()[:, :3].double().sum(1, keepdim=True) * products / d
+    # (a reciprocal below 2^-126 is rounded to 2^-149, 2^-22 of it; an exponent of 61 ln 2 is rounded twice on its way
+    # into an exp2, which has 2 x 61 ln 2 2^-24 of it for each of two features)
+    error = ((got - want).abs() / want).max().item()
+    assert error <= (2.0 ** -20 if what == "large" else 2e-5), error
 
 
 def test_forward_and_backward_replay_in_a_graph(lib):
