@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <numeric>
 
 #include "ftc_common.h"
 
@@ -1378,14 +1379,23 @@ static int64_t attention_gradients_layout(int64_t N, int64_t H, int64_t L, int n
     return at;
 }
 
-// Whether rows [p, last byte] of two tensors of one shape may share memory (unit stride along a row)
+// Whether rows of two tensors may share memory (unit stride along a row): the ranges from first to last byte
+// meet, and the rows do not lie side by side either, as the parts of a packed buffer's rows do
 static bool may_overlap(const Operand &x, const OperandOut &y, const Dims &d) {
     auto extent = [&](int64_t sn, int64_t sh, int64_t sl, int64_t width) {
         return ((d.N - 1) * sn + (d.H - 1) * sh + (d.L - 1) * sl + width) * 4;
     };
     const char *xp = (const char *)x.ptr, *yp = (const char *)y.ptr;
-    return yp < xp + extent(x.stride_n, x.stride_h, x.stride_l, x.width) &&
-           xp < yp + extent(y.stride_n, y.stride_h, y.stride_l, y.width);
+    if (yp >= xp + extent(x.stride_n, x.stride_h, x.stride_l, x.width) ||
+        xp >= yp + extent(y.stride_n, y.stride_h, y.stride_l, y.width))
+        return false;
+    int64_t pitch = 0;  // every row starts at a multiple of it from its tensor's first
+    if (d.N > 1) pitch = std::gcd(pitch, std::gcd(x.stride_n, y.stride_n));
+    if (d.H > 1) pitch = std::gcd(pitch, std::gcd(x.stride_h, y.stride_h));
+    if (d.L > 1) pitch = std::gcd(pitch, std::gcd(x.stride_l, y.stride_l));
+    if (pitch == 0) return true;
+    const int64_t apart = ((yp - xp) % (pitch * 4) + pitch * 4) % (pitch * 4);
+    return apart < (int64_t)x.width * 4 || apart + (int64_t)y.width * 4 > pitch * 4;
 }
 
 static int64_t attention_backward_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E, int64_t M,
@@ -1450,24 +1460,27 @@ static int attention_backward(const ftc_tensor4 *queries, const ftc_tensor4 *key
                       denominators->stride[2], FTC_F32, 1};
     const Operand q = as_operand(queries), k = as_operand(keys), v = as_operand(values), g = as_operand(grad_out);
     // Rows of 64 values where the three scans share a launch of the chain-parallel kernel: they take q, k,
-    // v and grad_out as they are (N=10, H=8, L=4096: 375 -> 263 us), if no gradient is written
-    // over what they read.
+    // v and grad_out as they are (N=10, H=8, L=4096: 375 -> 263 us), if no gradient is written over what any of
+    // them reads: the workgroups of a cut chain read rows that another one's results belong to.  (The scans
+    // below read copies: grad_values alone may lie over the queries.)
     if (d.E == 64 && d.M == 64) {
         ScanDesc scans[3];
         AttentionGradients grads{key_lengths, nullptr, nullptr, {}, {}};
         int n = 0;
-        bool apart = true;
         auto add = [&](int kind, const Operand &a, const Operand &b, const Operand &x, const ftc_tensor4 *out_rows,
                        const Operand &rows) {
             if (!out_rows) return;
             const OperandOut o = as_operand_out(out_rows);
             grads.kinds[n] = kind, grads.rows[n] = rows;
             scans[n++] = ScanDesc{a, b, x, o, kind != 1};
-            apart = apart && !may_overlap(g, o, d);
         };
         add(1, g, v, k, grad_queries, q);
         add(2, v, g, q, grad_keys, k);
         add(3, k, q, g, grad_values, k);
+        bool apart = true;
+        for (int i = 0; i < n; i++)
+            for (const Operand *t : {&q, &k, &v, &g})
+                if (t != &v || grad_queries || grad_keys) apart = apart && !may_overlap(*t, scans[i].out, d);
         int64_t at[2];
         if (n > 0 && apart && attention_gradients_take(scans, n, grads, d.N, d.H, d.L) &&
             attention_gradients_layout(d.N, d.H, d.L, n, at) <= (int64_t)workspace_bytes) {

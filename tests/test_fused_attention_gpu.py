@@ -558,6 +558,35 @@ def test_gradients_straight_from_the_inputs(lib, shape, small):
     assert ((over - got[2]).norm() <= 2e-6 * got[2].norm()).item()
 
 
+@pytest.mark.parametrize("shape", [(15, 1000, 4), (1, 2500, 2), (2, 700, 20)], ids=lambda s: "n%d_l%d_h%d" % s)
+@pytest.mark.parametrize("over", ["queries", "keys", "inside_a_buffer_of_queries"])
+def test_gradient_of_values_written_over_an_input(lib, shape, over):
+    """grad_values alone may lie over the queries or the keys: chains that are cut or whose segments exchange sums read
+    rows of both in several workgroups, so the scan has to read copies.  Beside them in one buffer is not over them."""
+    from fast_transformers_amd import causal_product as cp
+    N, L, H = shape
+    nlh = lambda t: t.permute(0, 2, 1, 3)
+    q, k, v = (nlh(t.cuda()) for t in inputs(N, L, H, 64, 64, seed=51 + L))
+    g = nlh(torch.randn(N, L, H, 64, generator=torch.Generator().manual_seed(52 + L)).cuda())
+    out, den = nlh(torch.empty(N, L, H, 64, device="cuda")), torch.empty(N, H, L, device="cuda")
+    cp.causal_linear_attention_hip(q, k, v, None, 1e-6, out, den)
+    want = torch.empty_like(v)
+    cp.causal_linear_attention_backward_hip(q, k, v, None, out, den, g, None, None, want)
+    assert lib.ftc_last_kernel() == b"attention backward: three scans"
+    if over == "inside_a_buffer_of_queries":
+        wide = torch.empty(N, L, H, 128, device="cuda")
+        wide[..., :64], q = nlh(q), nlh(wide[..., :64])
+        got = nlh(wide[..., 64:])
+    else:
+        got = (q if over == "queries" else k).clone(memory_format=torch.preserve_format)
+        q, k = (got, k) if over == "queries" else (q, got)
+    cp.causal_linear_attention_backward_hip(q, k, v, None, out, den, g, None, None, got)
+    torch.cuda.synchronize()
+    beside = over == "inside_a_buffer_of_queries"
+    assert (lib.ftc_last_kernel() == b"attention backward: three scans") == beside
+    assert ((got - want).norm() <= 2e-6 * want.norm()).item()
+
+
 WIDE_SHAPES = [
     # N, L, H, E, M, key lengths: single positions, ragged ends, keys that end before, inside and on a
     # chunk; cut chains, whole ones of a round and more of workgroups, exchanges of segment sums; one and
