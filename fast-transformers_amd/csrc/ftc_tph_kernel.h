@@ -171,7 +171,6 @@ __device__ __forceinline__ uint32_t wave_max(float m) {  // (the bits of the lar
 // The running ceilings of a, b and v as one wavefront knows them (wave-uniform).
 struct Ceilings {
     uint32_t Ea, Wb, Wv;
-    uint32_t Ed = 0;  // (gradients of the attention) the biased exponent of the position's largest dd
     __device__ __forceinline__ int Eb() const { return (int)(Wb & 0xffffu); }
     __device__ __forceinline__ int Ev() const { return (int)(Wv & 0xffffu); }
     __device__ __forceinline__ float scale_a() const { return pow2_field(259 - (int)Ea); }
@@ -180,23 +179,16 @@ struct Ceilings {
     // exponent of the state's units, and of a chunk's output units (a x state)
     __device__ __forceinline__ int state_exp() const { return (int)((Wb + Wv) & 0xffffu) - 264; }
     __device__ __forceinline__ int out_exp() const { return (int)(Ea + ((Wb + Wv) & 0xffffu)) - 396; }
-    // dd as weights: the field of the power of two that brings them below 16
-    __device__ __forceinline__ int weight_field() const { return max(1, min(254, 257 - (int)Ed)); }
-    // dd in the units of Pt: 2^up; beyond 2^14 of them the quadrants take units 2^shift as large
-    __device__ __forceinline__ int dd_up() const { return 264 - (int)Ea - Eb(); }
-    __device__ __forceinline__ int dd_shift() const { return Ed == 255u ? 0 : max(0, (int)Ed - 140 + dd_up()); }
 };
 typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
 typedef __attribute__((address_space(3))) f32x4 lds_fvec4;
-// The slot of a position is that of its LDS buffer: words (a, b, v, and dd, tagged as that of a).  The words of b
+// The slot of a position is that of its LDS buffer: words (a, b, v, unused).  The words of b
 // and v hold ceilings that only ever rise (a stale one is harmless: it is below the running
 // ceiling that every wavefront carries).  The word of a holds the ceiling of the rows of that
 // one position, tagged with the position's number in the upper 24 bits, so that what the
 // slot held three positions ago is always smaller and needs no clearing.
-template <bool GRAD = false>
 __device__ __forceinline__ void read_slot(const lds_u32_t *slots, int k, Ceilings &c) {
     const u32x4 s = *(const lds_vec4 *)(slots + 4 * k);
-    if (GRAD) c.Ed = (uint32_t)__builtin_amdgcn_readfirstlane(s.w) & 0xffu;
     c.Ea = max(kExpFloor, (uint32_t)__builtin_amdgcn_readfirstlane(s.x) & 0xffu);
     c.Wb = max(c.Wb, (uint32_t)__builtin_amdgcn_readfirstlane(s.y));
     c.Wv = max(c.Wv, (uint32_t)__builtin_amdgcn_readfirstlane(s.z));
@@ -229,16 +221,15 @@ __device__ __forceinline__ void raise_slot(lds_u32_t *slots, int k, int pos, con
 // GRAD: the gradients of the fused attention (equations in ftc_attention.hip) straight from its inputs:
 // a scan's rows become phi(q), phi(k) [j < key_len] and gz = g / den as the producers first touch them, and
 // the normaliser's share of a gradient, whose sums are prefix sums of rows weighted by w = 1 (for dq, which
-// has the factor dd_l outside) or w_l = dd_l (for dk), is part of the walk:
-//  * inside a chunk dd is added to the quadrants of Pt, (gz_l . v_j + dd_l) being the factor of both sums (dd
-//    beyond 2^14 of the quadrant's units is rare, and takes the chunk's result to larger units);
-//  * Z = sum of w_l v_l over the positions before the chunk is kept in fp32, 16 columns a wavefront: one more
-//    product of v^T with the weights in two pieces, three matrix instructions a chunk, and one fma per value
-//    of the result.
-// phi'(q) or phi'(k) multiplies the result on its way out.  A consumer's stream of instructions is what a chunk
-// waits for here, so whatever can be is done by the producers: they leave dd, its pieces and phi' in LDS
-// (N=10, H=8, L=4096, with all of that in the consumers 320 us, this way 228; the dense copies of phi(q),
-// phi(k), gz that the scans read before, the scans and a pass over their results for the rest: 370).
+// has the factor dd_l outside) or w_l = dd_l (for dk), is part of the walk.  Those are fp32 sums of fp32 rows: in
+// two pieces under the ceiling of all columns, one of features 2^-14 beside the others was up to 1e-4 off, this way
+// 8e-7.  The producers leave the weighted rows of a position in LDS as they look at it; two periods later, while
+// they look at the next one, a lane takes eight rows of one column, adds what the other lanes' rows and the positions
+// before add up to, and puts the sums back in place.  A consumer reads them with the rows that it stores, and
+// the rows of q or k whose phi' multiplies the result.  What bounds a chunk of short chains is the producers' stream
+// of instructions, of long ones the memory (backward, 80 chains, L=4096 / L=1000, us: 244 / 62; with the sums as
+// products of two pieces in the consumers 245 / 60; made where a position is cut, not where the next but one is looked
+// at, 261 / 64; dense copies of phi(q), phi(k), gz, the scans of those and a pass over their results 381 / 87).
 enum GradRole { kGradQueries = 1, kGradKeys = 2, kGradValues = 3 };
 
 // KS: groups of 32 rows of the state (1: a state of up to 32 rows, which skips the matrix
@@ -276,16 +267,22 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
     __shared__ __align__(16) char pieces_mem[3 * kBufBytes];
     __shared__ __align__(16) char pt_mem[3 * 2 * kTileP];
     __shared__ __align__(16) uint32_t slot_mem[16];
-    // GRAD, for the rows in each of the three buffers: dd, dd in the units of Pt, the weights' two pieces
-    constexpr int kDdUnits = 4 * kChunk, kWeights = 8 * kChunk, kDdBytes = 12 * kChunk;
+    // GRAD, for the rows in each of the three buffers: dd, and the rows of q or k that belong to the result's,
+    // quad p of row r in slot p ^ (r mod 16)
+    constexpr int kDdBytes = 4 * kChunk, kTileX = kChunk * F * 4;
     __shared__ __align__(16) char dd_mem[GRAD ? 3 * kDdBytes : 1];
-    // ... and phi' of the rows of q or k that belong to the result's, piece p of row r in slot p ^ (r mod 16)
-    constexpr int kTileX = kChunk * F * 4;
     __shared__ __align__(16) char x_mem[GRAD ? 3 * kTileX : 1];
+    // ... the weighted rows of position k in buffer k % 4 (written before barrier k - 1), then their running sums
+    // (before barrier k + 1, read under the next chunk); quad p of row r in slot p ^ (r mod 16) ^ 4 (r / 16), where neither sixteen rows
+    // of a quad nor sixteen columns of every eighth row meet in a bank
+    __shared__ __align__(16) char sum_mem[GRAD ? 4 * kTileX : 1];
+    auto sum_addr = [](int row, int quad) -> int { return row * F * 4 + 16 * (quad ^ (row % 16) ^ 4 * (row / 16)); };
+    // ... and per column the sum over the positions before position k (k % 2), and over the first walk
+    __shared__ float carry_mem[GRAD ? 2 : 1][GRAD ? F : 1], first_sum[GRAD ? F : 1];
     lds_char *const unit_pc = (lds_char *)pieces_mem;
     lds_char *const pt_pc = (lds_char *)pt_mem;
     lds_u32_t *const slots = (lds_u32_t *)slot_mem;
-    lds_char *const dd_pc = (lds_char *)dd_mem, *const x_pc = (lds_char *)x_mem;
+    lds_char *const dd_pc = (lds_char *)dd_mem, *const x_pc = (lds_char *)x_mem, *const sum_pc = (lds_char *)sum_mem;
 
     // ---- which chain (as in scan_tp_kernel) ----
     const uint32_t nseg = (uint32_t)p.nseg;
@@ -341,9 +338,9 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
     constexpr uint32_t kNoRow = 0x80000000u;  // an offset outside every descriptor
     auto chunk_row0 = [&](int c) -> int { return REV ? rows - kChunk * (c + 1) : kChunk * c; };
     if (tid < 16) slot_mem[tid] = 0;
-    // (what is read before the first position is zero, and so is what the gradient of v reads)
-    if (GRAD && tid < 3 * kDdBytes / 4) *(lds_u32_t *)(dd_pc + 4 * tid) = 0;
+    if (GRAD && tid < F) carry_mem[0][tid] = first_sum[tid] = 0.f;
     const int role = op.pad;  // GRAD
+    const bool sums_rows = GRAD && role != kGradValues;
     // (GRAD: rows of k at or beyond the key length count as zero)
     const int key_rows = GRAD && p.key_len ? (int)max((int64_t)0, min((int64_t)rows, p.key_len[n])) : rows;
     Ceilings ce{kExpFloor, kExpOfZeros, kExpOfZeros};
@@ -415,10 +412,9 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             uint32_t rden[2], dd[2];  // GRAD
         };
         const uint32_t x_slb = GRAD ? (uint32_t)op.s0_sd * 4 : 0u, x_goff = (uint32_t)prow * x_slb + 16u * pc4;
-        const bool has_x = GRAD && role != kGradValues;
         const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void *)(has_x ? op.s0 + (int64_t)n * op.s0_sn + (int64_t)h * op.s0_sh : nullptr), 0,
-            has_x ? (rows - 1) * x_slb + Dw * 4 : 0u, kRsrcFlags);
+            (void *)(sums_rows ? op.s0 + (int64_t)n * op.s0_sn + (int64_t)h * op.s0_sh : nullptr), 0,
+            sums_rows ? (rows - 1) * x_slb + Dw * 4 : 0u, kRsrcFlags);
         // GRAD: 1 / den and dd of the row
         const __amdgpu_buffer_rsrc_t rden_rs = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(GRAD ? p.row_rden + (int64_t)chain * rows : nullptr), 0, rows * 4, kRsrcFlags);
@@ -439,7 +435,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
                 r.b[q] = __builtin_amdgcn_raw_buffer_load_b128(b_rs, ab_in ? b_goff + (uint32_t)row0 * b_slb : kNoRow, 0, 0);
                 r.v[q] = __builtin_amdgcn_raw_buffer_load_b128(v_rs, v_in ? v_goff + (uint32_t)row0 * v_slb : kNoRow, 0, 0);
                 if constexpr (GRAD) {
-                    r.x[q] = __builtin_amdgcn_raw_buffer_load_b128(x_rs, has_x ? x_goff + (uint32_t)row0_x * x_slb : kNoRow, 0, 0);
+                    r.x[q] = __builtin_amdgcn_raw_buffer_load_b128(x_rs, sums_rows ? x_goff + (uint32_t)row0_x * x_slb : kNoRow, 0, 0);
                     r.rden[q] = __builtin_amdgcn_raw_buffer_load_b32(rden_rs, 4u * (uint32_t)(prow + row0), 0, 0);
                     r.dd[q] = __builtin_amdgcn_raw_buffer_load_b32(dd_rs, 4u * (uint32_t)(prow + row0), 0, 0);
                 }
@@ -479,21 +475,20 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             }
         };
         // the largest magnitudes of the rows of a position against the ceilings (rows that
-        // were not asked for read as zeros); k: that position's slot
-        auto look_ahead = [&](Raw &r, int k, int pos) {
+        // were not asked for read as zeros); k: that position's slot; pos % 4 == j
+        auto look_ahead = [&](Raw &r, int k, int pos, int j) {
 #pragma unroll
             for (int q = 0; q < 2; q++) own_words(r.a[q], ab_own), own_words(r.b[q], ab_own), own_words(r.v[q], v_own);
             if constexpr (GRAD) {
                 as_taken(r, pos);
-                if (has_x) {  // (rows of 16 lanes share a row of the operands)
-                    const uint32_t d = max(r.dd[0] & 0x7fffffffu, r.dd[1] & 0x7fffffffu);
-                    const uint32_t m = scalar_max(scalar_max((uint32_t)__builtin_amdgcn_readlane((int)d, 0),
-                                                             (uint32_t)__builtin_amdgcn_readlane((int)d, 16)),
-                                                  scalar_max((uint32_t)__builtin_amdgcn_readlane((int)d, 32),
-                                                             (uint32_t)__builtin_amdgcn_readlane((int)d, 48)));
-                    if (lane == 0)
-                        __hip_atomic_fetch_max(slots + 4 * k + 3, ((uint32_t)(pos + 1) << 8) | m >> 23,
-                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (sums_rows) {
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        const float u = role == kGradQueries ? 1.f : __uint_as_float(r.dd[q]);
+                        *(lds_fvec4 *)(sum_pc + j * kTileX + sum_addr(prow + 16 * q, pc4)) =
+                            f32x4{u * __uint_as_float(r.v[q].x), u * __uint_as_float(r.v[q].y),
+                                  u * __uint_as_float(r.v[q].z), u * __uint_as_float(r.v[q].w)};
+                    }
                 }
             }
             raise_slot(slots, k, pos, ce, max_abs4(r.a[1], max_abs4(r.a[0], 0.f)), max_abs4(r.b[1], max_abs4(r.b[0], 0.f)),
@@ -509,31 +504,50 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
                 cut_quad_to_lds(r.b[q], ce.scale_b(), pc + kOffB, kTileB, b_waddr[q]);
                 cut_quad_to_lds(r.v[q], ce.scale_v(), pc + kOffV, kTileV, v_waddr[q]);
             }
-            if (GRAD && has_x) {
-                auto slope = [](uint32_t x) -> uint32_t {  // phi'(x); NaN: one (gz is NaN then)
-                    return __float_as_uint(fminf(1.f, __builtin_amdgcn_exp2f(__uint_as_float(x) * 1.44269502f)));
-                };
+            if (GRAD && sums_rows) {
 #pragma unroll
                 for (int q = 0; q < 2; q++)
-                    if (own)
-                        *(lds_vec4 *)(x_pc + buf * kTileX + (prow + 16 * q) * F * 4 + 16 * (pc4 ^ prow)) =
-                            u32x4{slope(r.x[q].x), slope(r.x[q].y), slope(r.x[q].z), slope(r.x[q].w)};
+                    if (own) *(lds_vec4 *)(x_pc + buf * kTileX + (prow + 16 * q) * F * 4 + 16 * (pc4 ^ prow)) = r.x[q];
                 // (lane 0 of a row's sixteen for the first row, lane 1 for the second)
-                const float dd = __uint_as_float(pc4 == 0 ? r.dd[0] : r.dd[1]), wt = dd * pow2_field(ce.weight_field());
-                const int at = prow + 16 * pc4;
-                _Float16 hi = (_Float16)wt, lo = (_Float16)(wt - (float)hi);
-                if (role == kGradQueries) hi = (_Float16)1.f, lo = (_Float16)0.f;
-                if (pc4 < 2) {
-                    lds_char *const d = dd_pc + buf * kDdBytes;
-                    *(lds_f32 *)(d + 4 * at) = dd;
-                    *(lds_f32 *)(d + kDdUnits + 4 * at) = ce.dd_shift() == 0 ? __builtin_amdgcn_ldexpf(dd, ce.dd_up()) : 0.f;
-                    *(lds_u16 *)(d + kWeights + 2 * at) = __builtin_bit_cast(uint16_t, hi);
-                    *(lds_u16 *)(d + kWeights + 2 * (kChunk + at)) = __builtin_bit_cast(uint16_t, lo);
-                }
+                if (pc4 < 2) *(lds_u32_t *)(dd_pc + buf * kDdBytes + 4 * (prow + 16 * pc4)) = pc4 == 0 ? r.dd[0] : r.dd[1];
             }
             if (!own) {
                 asm volatile("" ::"v"(r.a[0]), "v"(r.a[1]));
                 if constexpr (GRAD) asm volatile("" ::"v"(r.x[0]), "v"(r.x[1]));
+            }
+        };
+        // GRAD: the running sums of position v in place of its weighted rows.  A wavefront has 16 columns, the
+        // lanes of a column eight rows each, in the order of the walk.
+        int sum_at[8];
+        const int sum_col = 16 * w + lane % 16;
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const int at = 8 * (lane / 16) + t;
+            sum_at[t] = sum_addr(REV ? kChunk - 1 - at : at, sum_col / 4) + 4 * (sum_col % 4);
+        }
+        auto weighted_rows = [&](float (&x)[8], int j) {  // (v % 4 == j)
+#pragma unroll
+            for (int t = 0; t < 8; t++) x[t] = *(const lds_f32 *)(sum_pc + j * kTileX + sum_at[t]);
+        };
+        auto add_rows = [&](float (&x)[8], int v, int j, bool own) {
+            // (an exchange: the second walk starts anew, the consumers add what comes before)
+            const float before = exchange && v == n1 ? 0.f : carry_mem[j % 2][sum_col];
+#pragma unroll
+            for (int t = 1; t < 8; t++) x[t] += x[t - 1];
+            // (the sums of the even and the odd group of 16 lanes of each half, then of the two halves)
+            const uint32_t bits = __float_as_uint(x[7]);
+            const auto pair = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+            const float even = __uint_as_float(pair[0]), both = even + __uint_as_float(pair[1]);
+            const auto half = __builtin_amdgcn_permlane32_swap(__float_as_uint(both), __float_as_uint(both), false, false);
+            const float low = __uint_as_float(half[0]), all = low + __uint_as_float(half[1]);
+            if (own) {
+                const float ahead = before + ((lane & 32 ? low : 0.f) + (lane & 16 ? even : 0.f));
+#pragma unroll
+                for (int t = 0; t < 8; t++) *(lds_f32 *)(sum_pc + j * kTileX + sum_at[t]) = x[t] + ahead;
+            }
+            if (lane < 16) {
+                carry_mem[(j + 1) % 2][sum_col] = before + all;
+                if (v + 1 == n1) first_sum[sum_col] = before + all;
             }
         };
         // Barrier number k (k = 0: before the consumers' first position; k >= 1: in the
@@ -547,19 +561,22 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             Raw raw[2];
             fetch(raw[0], G), fetch(raw[1], G + 2);
             wg_barrier();  // the slots are zero
-            if (G == 0) look_ahead(raw[0], B0, 0);
+            if (G == 0) look_ahead(raw[0], B0, 0, 0);
             wg_barrier();  // the slot of position 0 is complete
             int buf = B0;
             auto period = [&](int v, int j, bool own, bool more) {  // v % 4 == j
                 const bool stamped = own && v == n1 + 4;
                 if (stamped) FTC_STAMP(0);
-                read_slot<GRAD>(slots, buf, ce);
+                read_slot(slots, buf, ce);
                 if (j % 2 == G) {
                     cut(raw[j / 2], buf, own);
                     if (stamped) FTC_STAMP(2);
                     if (more) fetch(raw[j / 2], v + PF);
                 } else {
-                    look_ahead(raw[(j + 1) % 4 / 2], next_buf(buf), v + 1);
+                    float x[8];
+                    if (sums_rows) weighted_rows(x, (j + 3) % 4);  // (they arrive during the look)
+                    look_ahead(raw[(j + 1) % 4 / 2], next_buf(buf), v + 1, (j + 1) % 4);
+                    if (sums_rows && v > 0) add_rows(x, v - 1, (j + 3) % 4, v > n1);
                     if (stamped) FTC_STAMP(1);
                 }
                 buf = next_buf(buf);
@@ -671,37 +688,8 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         }
     };
 
-    // GRAD: Z, the sum of w_l v_l over the positions before the chunk (w = 1 or dd), in this lane's four
-    // columns of the result
-    const bool sums_rows = GRAD && role != kGradValues;
-    f32x4 Z = {0.f, 0.f, 0.f, 0.f}, Zc = {0.f, 0.f, 0.f, 0.f};  // Zc: the chunk's sum, times 2^-z_exp
-    int z_exp = 0;
-    // the chunk's sum is one more product of v^T, with the weights w in all 16 columns of the second operand
-    auto weights_exp = [&](const Ceilings &c) -> int {  // (the unit of that product)
-        return (role == kGradQueries ? 0 : 127 - c.weight_field()) + c.Ev() - 132;
-    };
-    auto sum_chunk = [&](int b, const Frag (&vfx)[2]) {  // (into Zc; b: the buffer)
-        const lds_char *const at = dd_pc + b * kDdBytes + kWeights + 16 * g;
-        const Frag hi = lds_frag16(at), lo = lds_frag16(at + 2 * kChunk);
-        Zc = mfma16h(vfx[1], hi, f32x4{0.f, 0.f, 0.f, 0.f});
-        Zc = mfma16h(vfx[0], lo, Zc);
-        Zc = mfma16h(vfx[0], hi, Zc);
-    };
-    // dd in the units of Pt (added to a quadrant when the products are summed: a sum that starts from dd is
-    // rounded to dd's last place six times over, and dq came out up to a tenth further from float64)
-    const int dd_addr = kDdUnits + (role == kGradQueries ? 4 * (16 * ih + ln) : 4 * (16 * jh + 4 * g));
-    auto dd_of_quadrant = [&](int b) -> f32x4 {
-        if (role == kGradQueries) {
-            const float d = *(const lds_f32 *)(dd_pc + b * kDdBytes + dd_addr);
-            return f32x4{d, d, d, d};
-        }
-        return *(const lds_fvec4 *)(dd_pc + b * kDdBytes + dd_addr);
-    };
-    auto add_chunk = [&]() {
-#pragma unroll
-        for (int r = 0; r < 4; r++) Z[r] += __builtin_amdgcn_ldexpf(Zc[r], z_exp);
-    };
-
+    // GRAD with an exchange: the sums of the weighted rows before the segment, in this lane's four columns
+    f32x4 Z = {0.f, 0.f, 0.f, 0.f};
     Frag af[2][2][2], bfr[2][2], bt[4][2], vf[2];
     // row-major fragment number i of a chunk (12: b for the quadrant first, then a)
     auto rm_frag = [&](const lds_char *pc, int i) {
@@ -726,7 +714,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
     wg_barrier();  // the slots are zero
     wg_barrier();  // the slot of position 0 is complete
     wg_barrier();  // barrier 0: position 0 is cut
-    read_slot<GRAD>(slots, B0, ce);
+    read_slot(slots, B0, ce);
     Ucur = ce.state_exp();
     if (!GRAD && op.s0 && !exchange) add_caller_state();
     if (n1 > 0) {
@@ -735,17 +723,11 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         // run, the fragments of position k arrive in the other set of registers.
         int U_prev = Ucur;                 // units of the fragments about to be multiplied
         Frag bt2[4][2] = {}, vf2[2] = {};  // (the first round multiplies zeros)
-        // GRAD: the position before, whose dd are in the buffer before (nothing cuts that one now)
-        auto sum_before = [&](int b, const Frag (&vfx)[2]) {
-            sum_chunk(b == 0 ? 2 : b - 1, vfx);
-            add_chunk();
-        };
-        z_exp = 0;  // (zeros)
         for (int c = 0; c < n1; c += PF) {
 #pragma unroll
             for (int j = 0; j < PF; j++) {
                 const lds_char *pc = unit_pc + buf * kBufBytes;
-                read_slot<GRAD>(slots, buf, ce);  // the ceilings of position c + j
+                read_slot(slots, buf, ce);  // the ceilings of position c + j
                 if (U_prev != Ucur) {       // the ceilings rose: the state shrinks
                     scale_state(Ucur - U_prev);
                     Ucur = U_prev;
@@ -761,10 +743,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
                         if (i < 10) tr_frag_into(bt2, vf2, pc, i);
                     }
                     __builtin_amdgcn_sched_barrier(0);
-                }
-                if (GRAD && sums_rows) {
-                    sum_before(buf, j % 2 == 0 ? vf2 : vf);
-                    z_exp = weights_exp(ce);
                 }
                 U_prev = ce.state_exp();
                 buf = next_buf(buf);
@@ -786,9 +764,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             if (!GRAD) rm_frag(unit_pc + buf * kBufBytes, i);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (GRAD && sums_rows) sum_before(buf, vf2);
-        Zc = f32x4{0.f, 0.f, 0.f, 0.f};
-        read_slot<GRAD>(slots, buf, ce);  // the ceilings of our own first chunk
+        read_slot(slots, buf, ce);  // the ceilings of our own first chunk
     } else if (!GRAD) {
 #pragma unroll
         for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
@@ -805,7 +781,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         if (GRAD) {
             Sx[DX - 1][0] = f32x16{};
 #pragma unroll
-            for (int r = 0; r < 4; r++) Sx[DX - 1][0][r] = Z[r];
+            for (int r = 0; r < 4; r++) Sx[DX - 1][0][r] = first_sum[16 * w + 4 * g + r];
         }
 #pragma unroll
         for (int dt = 0; dt < 4; dt++)
@@ -879,16 +855,20 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
     for (int x = 0; x < 2; x++) O[x] = f32x4{0.f, 0.f, 0.f, 0.f};
     int Xo = 0;
     uint32_t o_off = (uint32_t)(rows + kChunk) * o_slb;  // (also beyond the end with kNoRow on top of it)
-    int o_row0 = 0, o_buf = 0;  // GRAD
+    int o_row0 = 0, o_buf = 0, o_sum = 0;  // GRAD
     auto store_rows = [&](int x) {
         float y0 = __builtin_amdgcn_ldexpf(O[x][0], Xo), y1 = __builtin_amdgcn_ldexpf(O[x][1], Xo),
               y2 = __builtin_amdgcn_ldexpf(O[x][2], Xo), y3 = __builtin_amdgcn_ldexpf(O[x][3], Xo);
         if (GRAD && sums_rows) {
             const int row = 16 * (x ^ ih) + ln;
-            const f32x4 slope = *(const lds_fvec4 *)(x_pc + o_buf * kTileX + row * F * 4 + 16 * ((4 * w + g) ^ ln));
+            f32x4 slope = *(const lds_fvec4 *)(x_pc + o_buf * kTileX + row * F * 4 + 16 * ((4 * w + g) ^ ln));
+#pragma unroll
+            for (int r = 0; r < 4; r++)  // phi'(x); NaN: one (gz is NaN then)
+                slope[r] = fminf(1.f, __builtin_amdgcn_exp2f(slope[r] * 1.44269502f));
+            const f32x4 sum = *(const lds_fvec4 *)(sum_pc + o_sum + sum_addr(row, 4 * w + g)) + Z;
             const float dd = *(const lds_f32 *)(dd_pc + o_buf * kDdBytes + 4 * row), u = role == kGradQueries ? dd : 1.f;
-            y0 = fmaf(u, Z[0], y0) * slope[0], y1 = fmaf(u, Z[1], y1) * slope[1];
-            y2 = fmaf(u, Z[2], y2) * slope[2], y3 = fmaf(u, Z[3], y3) * slope[3];
+            y0 = fmaf(u, sum[0], y0) * slope[0], y1 = fmaf(u, sum[1], y1) * slope[1];
+            y2 = fmaf(u, sum[2], y2) * slope[2], y3 = fmaf(u, sum[3], y3) * slope[3];
             if (role == kGradKeys && o_row0 + kChunk > key_rows) {  // (rows beyond the key length)
                 const bool live = o_row0 + row < key_rows;
                 y0 = live ? y0 : 0.f, y1 = live ? y1 : 0.f, y2 = live ? y2 : 0.f, y3 = live ? y3 : 0.f;
@@ -904,7 +884,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         }
     };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    int z_exp_next = 0;
     // One chunk, in LDS buffer B (a compile-time number, so that every LDS access of the body
     // has its buffer in the instruction's immediate offset).  Sums that end in one place are
     // chained through one accumulator, with other matrix instructions in between: Ot_w =
@@ -916,9 +895,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         lds_char *const ptc = pt_pc + B * (2 * kTileP);
         Frag pf[2][2];
         f32x4 P;  // (cleared by the first matrix instruction of its sum)
-        f32x4 P_dd = zero;  // GRAD
-        const int shift = GRAD && sums_rows ? ce.dd_shift() : 0;
-        if (GRAD && sums_rows) z_exp_next = weights_exp(ce);
         if (c == c0 + 4) FTC_STAMP(0);
         __builtin_amdgcn_sched_barrier(0);
         // phase 1: (1) the quadrant in turn with (2b) Ot_w = S_w^T a^T for rows 0 .. 31 of
@@ -928,11 +904,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         for (int i = 0; i < 6; i++) {
             const int m = i % 3, ks = i / 3, x = i % 2, mo = i / 2;
             if (i == 0) store_rows(0);
-            if (GRAD && i == 3) P_dd = dd_of_quadrant(B);
-            if (i == 1) {
-                store_rows(1);
-                if (GRAD && sums_rows) add_chunk();  // (the rows before this chunk are all summed)
-            }
+            if (i == 1) store_rows(1);
             if (ks < KS) P = mfma16h(bfr[ks][kPa[m]], af[0][ks][kPb[m]], i == 0 ? zero : P);
             O[x] = mfma16h(sf[0][kPa[mo]], af[x][0][kPb[mo]], mo == 0 ? zero : O[x]);
             if ((i == 1 || i == 3) && KS > 1) cut_s(1, i / 2, B == 0);
@@ -964,15 +936,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             S[i % 2] = mfma16h(bt[i % 2][kPa[m]], vf[kPb[m]], S[i % 2]);
             if (i == 1) {
                 uint32_t h0, l0, h1, l1;
-                if (GRAD) P += P_dd;
-                if (GRAD && shift != 0) {  // (that was zero)
-                    const lds_char *const d = dd_pc + B * kDdBytes + dd_addr - kDdUnits;
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        P[r] = __builtin_amdgcn_ldexpf(P[r], -shift) +
-                               __builtin_amdgcn_ldexpf(*(const lds_f32 *)(d + (role == kGradQueries ? 0 : 4 * r)),
-                                                       ce.dd_up() - shift);
-                }
 #pragma unroll
                 for (int r = 0; r < 4; r++) P[r] = keep[r] ? P[r] : 0.f;
                 cut_quad_f16_unscaled(P[0], P[1], P[2], P[3], h0, h1, l0, l1);
@@ -995,22 +958,12 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         for (int x = 0; x < 2; x++)
 #pragma unroll
             for (int k = 0; k < 2; k++) pf[x][k] = lds_frag16(ptc + k * kTileP + pt_raddr[x]);
-        const int Xc = ce.out_exp() + shift;
+        const int Xc = ce.out_exp();
         const u32x4 slot_next = *(const lds_vec4 *)(slots + 4 * BN);
         if (__builtin_expect(s_cut != 0, 0)) {  // (rare: the state has grown beyond 2^14 units)
             const float r_cut = pow2_field(127 + s_cut);
             O[0] *= r_cut;
             O[1] *= r_cut;
-        }
-        if (GRAD && shift != 0) {
-#pragma unroll
-            for (int x = 0; x < 2; x++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) O[x][r] = __builtin_amdgcn_ldexpf(O[x][r], -shift);
-        }
-        if (GRAD && sums_rows) {
-            sum_chunk(B, vf);
-            z_exp = z_exp_next;
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1025,7 +978,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         ce.Ea = max(kExpFloor, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.x) & 0xffu);
         ce.Wb = max(ce.Wb, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.y));
         ce.Wv = max(ce.Wv, (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.z));
-        if (GRAD) ce.Ed = (uint32_t)__builtin_amdgcn_readfirstlane(slot_next.w) & 0xffu;
         // (dU > 0: small values after nothing but zeros; the state's units fall, so s rises)
         dU = Ucur - ce.state_exp();
         s += max(dU, 0);
@@ -1040,7 +992,7 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
             __builtin_amdgcn_sched_barrier(0);
         }
         o_off = (uint32_t)chunk_row0(c) * o_slb;
-        o_row0 = chunk_row0(c), o_buf = B;
+        o_row0 = chunk_row0(c), o_buf = B, o_sum = (c - c0) % 4 * kTileX;  // (n1 is a multiple of 4)
         Xo = Xc;
         if (c == c0 + 4) FTC_STAMP(6);
     };

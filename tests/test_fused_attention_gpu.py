@@ -587,6 +587,110 @@ def test_gradient_of_values_written_over_an_input(lib, shape, over):
     assert ((got - want).norm() <= 2e-6 * want.norm()).item()
 
 
+@pytest.mark.parametrize("shape", DIRECT_SHAPES[3:7], ids=lambda s: "n%d_l%d_h%d" % s[:3])
+def test_normaliser_sums_of_columns_of_very_different_size(lib, shape):
+    """The normaliser's share of a gradient is a sum of fp32 rows: a column of features 2^-14 beside the others, met
+    where the values are too small to take part, has the relative error of such a sum (2^-24 a term and 14 ln 2 2^-24
+    for the exp2 of each feature, together 1e-6; in two fp16 pieces under the ceiling of all columns 1e-5 to 1e-4)."""
+    from fast_transformers_amd import causal_product as cp
+    N, L, H, lens = shape
+    nlh = lambda t: t.permute(0, 2, 1, 3)
+    q, k, v = inputs(N, L, H, 64, 64, seed=91 + L)
+    g = torch.randn(N, L, H, 64, generator=torch.Generator().manual_seed(92 + L))
+    late = L // 2
+    v[:, late:] *= 2.0 ** -40
+    for t, column in ((k, 5), (q, 9)):      # phi: zero before, 2^-14 and its neighbours from there on
+        t[:, :late, :, column] = -200.0
+        t[:, late:, :, column] = t[:, late:, :, column] / 4 - 9.7
+    lengths = torch.full((N,), L)
+
+    leaves = [t.double().requires_grad_(True) for t in (q, k, v)]
+    _dense_attention(*leaves, lengths, 1.0).backward(g.double())
+    exact = [t.grad for t in leaves]
+    dev = [nlh(t.cuda()) for t in (q, k, v, g)]
+    out, den = nlh(torch.empty(N, L, H, 64, device="cuda")), torch.empty(N, H, L, device="cuda")
+    cp.causal_linear_attention_hip(*dev[:3], lengths.cuda(), 1.0, out, den)
+    got = [nlh(torch.empty(N, L, H, 64, device="cuda")) for _ in range(3)]
+    cp.causal_linear_attention_backward_hip(*dev[:3], lengths.cuda(), out, den, dev[3], *got)
+    assert lib.ftc_last_kernel() == b"attention backward: three scans"
+    for i, column in ((0, 5), (1, 9)):
+        a, c = (x[:, late:, :, column].double() for x in (nlh(got[i]).cpu(), exact[i]))
+        error = ((a - c).norm() / c.norm()).item()
+        print("qk"[i], "column", column, "vs float64: %.3e" % error, flush=True)
+        assert error <= 2e-6, (i, error)
+
+
+@pytest.mark.parametrize("what", ["q_nan", "k_nan", "v_nan", "g_nan", "q_minus_inf", "k_minus_inf", "g_inf", "k_nan_beyond_the_length",
+                                  "tiny_denominator"])
+@pytest.mark.parametrize("shape", [(2, 300, 4), (1, 2500, 2)], ids=lambda s: "n%d_l%d_h%d" % s)
+def test_non_finite_rows_reach_the_same_gradients_on_either_route(lib, shape, what):
+    """The direct route and the launches around dense copies (taken where a gradient lies over grad_out): the same
+    values are finite, and those agree."""
+    from fast_transformers_amd import causal_product as cp
+    N, L, H = shape
+    nlh = lambda t: t.permute(0, 2, 1, 3)
+    q, k, v = inputs(N, L, H, 64, 64, seed=61 + L)
+    g = torch.randn(N, L, H, 64, generator=torch.Generator().manual_seed(62 + L))
+    nan, inf = float("nan"), float("inf")
+    if what == "q_nan":
+        q[0, 40, 0, 3] = nan
+    elif what == "k_nan":
+        k[0, 200, 1, 5] = nan
+    elif what == "v_nan":
+        v[0, 150, 1, 7] = nan
+    elif what == "g_nan":
+        g[0, 77, 0, 9] = nan
+    elif what == "q_minus_inf":
+        q[0, 40, 0, 3] = -inf
+    elif what == "k_minus_inf":
+        k[0, 200, 1, 5] = -inf
+    elif what == "g_inf":
+        g[0, 77, 0, 9] = inf
+    elif what == "k_nan_beyond_the_length":
+        k[0, 290, 0] = nan
+    elif what == "tiny_denominator":   # dd and g / den far beyond those of the other rows
+        q[0, 60, 1] = -40.0
+    q, k, v, g = (nlh(t.cuda()) for t in (q, k, v, g))
+    lengths = torch.full((N,), 280).cuda()
+    out, den = nlh(torch.empty(N, L, H, 64, device="cuda")), torch.empty(N, H, L, device="cuda")
+    cp.causal_linear_attention_hip(q, k, v, lengths, 0.0, out, den)
+    got = [nlh(torch.empty(N, L, H, 64, device="cuda")) for _ in range(3)]
+    cp.causal_linear_attention_backward_hip(q, k, v, lengths, out, den, g, *got)
+    assert lib.ftc_last_kernel() == b"attention backward: three scans"
+    over = g.clone(memory_format=torch.preserve_format)
+    want = [torch.empty_like(got[0]), torch.empty_like(got[1]), over]
+    cp.causal_linear_attention_backward_hip(q, k, v, lengths, out, den, over, *want)
+    assert lib.ftc_last_kernel() != b"attention backward: three scans"
+    torch.cuda.synchronize()
+    cp.check_workspaces()
+    for name, a, b in zip("qkv", got, want):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b)), name
+        a, b = (torch.where(torch.isfinite(b), x, torch.zeros_like(x)) for x in (a, b))
+        for c in range(N * H):          # (each chain at its own scale)
+            x, y = a[c // H, c % H], b[c // H, c % H]
+            assert ((x - y).norm() <= 1e-5 * y.norm()).item(), (name, c)
+
+
+@pytest.mark.parametrize("shape", [(2, 300, 4), (1, 2500, 2)], ids=lambda s: "n%d_l%d_h%d" % s)
+def test_gradients_of_parts_of_one_buffer(lib, shape):
+    """q, k and v as parts of one projection's rows, their gradients as parts of another's."""
+    from fast_transformers_amd import causal_product as cp
+    N, L, H = shape
+    nlh = lambda t: t.permute(0, 2, 1, 3)
+    q, k, v = (t.cuda() for t in inputs(N, L, H, 64, 64, seed=66 + L))
+    g = nlh(torch.randn(N, L, H, 64, generator=torch.Generator().manual_seed(67 + L)).cuda())
+    packed, grads = torch.stack([q, k, v], 2), torch.full((N, L, 3, H, 64), float("nan"), device="cuda")
+    out, den = nlh(torch.empty(N, L, H, 64, device="cuda")), torch.empty(N, H, L, device="cuda")
+    cp.causal_linear_attention_hip(nlh(q), nlh(k), nlh(v), None, 1e-6, out, den)
+    want = [nlh(torch.empty_like(q)) for _ in range(3)]
+    cp.causal_linear_attention_backward_hip(nlh(q), nlh(k), nlh(v), None, out, den, g, *want)
+    got = [nlh(grads[:, :, i]) for i in range(3)]
+    cp.causal_linear_attention_backward_hip(*(nlh(packed[:, :, i]) for i in range(3)), None, out, den, g, *got)
+    assert lib.ftc_last_kernel() == b"attention backward: three scans"
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 WIDE_SHAPES = [
     # N, L, H, E, M, key lengths: single positions, ragged ends, keys that end before, inside and on a
     # chunk; cut chains, whole ones of a round and more of workgroups, exchanges of segment sums; one and
