@@ -87,19 +87,41 @@ int tp_kernel_segments(int64_t units, int64_t L, bool wide, bool others, bool lo
     return (brief || units * nseg >= (long_chains ? 112 : 128)) && units <= most_units ? nseg : 0;
 }
 
+// Plans depend on the sizes alone and a caller repeats the same sizes call after call (the
+// segment search walks up to 4096 candidates for a long sequence): the last plans of every
+// thread are kept, keyed by their arguments and by the generation of the tuning variables.
+template <typename Value>
+struct PlanMemo {
+    static constexpr int kEntries = 32;
+    struct Entry {
+        int64_t key[8];
+        uint64_t generation;
+        Value value;
+    };
+    Entry entry[kEntries] = {};
+    template <typename Compute>
+    Value get(const int64_t (&key)[8], Compute compute) {
+        uint64_t h = 1469598103934665603ull;
+        for (int64_t k : key) h = (h ^ (uint64_t)k) * 1099511628211ull;
+        Entry &e = entry[h % kEntries];
+        const uint64_t generation = tuning().generation;
+        bool hit = e.generation == generation;
+        for (int i = 0; i < 8 && hit; i++) hit = e.key[i] == key[i];
+        if (!hit) {
+            e.value = compute();
+            for (int i = 0; i < 8; i++) e.key[i] = key[i];
+            e.generation = generation;
+        }
+        return e.value;
+    }
+};
+
 // Where to cut a chain of `chunks` chunks into (at most) `nseg` segments for the
 // chain-parallel kernel.  The workgroup of a segment first rebuilds the state before its
 // segment from the chunks in front of it, so later segments are made shorter until all
 // workgroups finish together: the starts (multiples of `step` chunks) that minimise the longest
 // workgroup.  `state_only`: the time of a chunk walked for its state alone, against one that also
-// produces rows: 0.6 on two fp16 pieces (0.75 against 1.3 us with every workgroup streaming rows); on
-// three bf16 pieces 0.45 where a state of 33 to 64 rows writes fp32 results, 0.55 otherwise and for two
-// segments of bf16 rows (128 chains, L=1088, forward 25.2 against 26.0 at 0.45).  Three pieces of fp32
-// rows may start half of what the producers request ahead (kTpAhead) further on (kHalfTrips).  Measured
-// against 0.6 and steps of kTpAhead for all, whose last one counted as whole, 22 shapes drawn for each,
-// geometric means of the time: fused attention of 64 x 64 0.928 (at 0.55: 0.940), odd widths 0.936;
-// 80 chains, L=1000, fused: 38.5 -> 35 us; bf16 rows forward, 64 chains, L=1000: 17.6 -> 16.8, 49,
-// L=1588: 23.7 -> 21.7; backward, 20 chains, L=900: 20.5 -> 19.2, 31, L=407: 15.0 -> 13.0.
+// produces rows.
 // Returns the number of segments; start[0 .. n] filled (start[n] = chunks).
 int tp_segment_starts(int64_t chunks, int nseg, int32_t *start, int step, double state_only) {
     const int groups = (int)((chunks + step - 1) / step);
@@ -133,6 +155,34 @@ int tp_segment_starts(int64_t chunks, int nseg, int32_t *start, int step, double
     }
     start[nseg] = (int32_t)chunks;
     return nseg;
+}
+
+// The cuts of a launch of the chain-parallel kernel with a state of D rows.  `scaled`: on two fp16
+// pieces, where a chunk walked for its state alone takes 0.6 of the others (0.75 against 1.3 us with
+// every workgroup streaming rows); on three bf16 pieces 0.45 where a state of 33 to 64 rows writes fp32
+// results, 0.55 otherwise and for two segments of odd widths or of bf16 rows (128 chains, L=1088, forward
+// 25.2 against 26.0 at 0.45).  Three pieces of fp32 rows may start half of what the producers request
+// ahead (kTpAhead) further on (kHalfTrips; up to 64 chunks, a longer search for a smaller share of a
+// segment beyond).  Measured against 0.6 and steps of kTpAhead for all, whose last one counted as whole, 22
+// shapes drawn for each, geometric means of the time: fused attention of 64 x 64 0.928 (at 0.55: 0.940),
+// odd widths 0.936; 80 chains, L=1000, fused: 38.5 -> 35 us; bf16 rows forward, 64 chains, L=1000: 17.6 ->
+// 16.8, 49, L=1588: 23.7 -> 21.7; backward, 20 chains, L=900: 20.5 -> 19.2, 31, L=407: 15.0 -> 13.0.
+// (Kept like the plans: the search takes the host up to 2 us.)
+struct TpCuts {
+    int nseg;
+    int32_t start[kMaxTpSegments + 1];
+};
+TpCuts tp_cuts(int64_t D, bool scaled, bool fp32_rows, bool fp32_results, bool fused, int nseg, int64_t chunks) {
+    const int step = !scaled && fp32_rows && chunks <= 64 ? kTpAhead / 2 : kTpAhead;
+    const bool light = D > 32 && D <= 64 && fp32_results && (fused || nseg > 2);
+    const int percent = scaled ? 60 : light ? 45 : 55;
+    static thread_local PlanMemo<TpCuts> memo;
+    const int64_t key[8] = {chunks, nseg, step, percent, 0, 0, 0, 0};
+    return memo.get(key, [&]() {
+        TpCuts c = {};
+        c.nseg = tp_segment_starts(chunks, nseg, c.start, step, 0.01 * percent);
+        return c;
+    });
 }
 
 // Longer chains on few CUs: the chain-parallel kernel with an exchange of segment sums.  A
@@ -498,34 +548,6 @@ MfmaPlan make_plan_compute(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F
     return pl;
 }
 
-// Plans depend on the sizes alone and a caller repeats the same sizes call after call (the
-// segment search walks up to 4096 candidates for a long sequence): the last plans of every
-// thread are kept, keyed by their arguments and by the generation of the tuning variables.
-template <typename Value>
-struct PlanMemo {
-    static constexpr int kEntries = 32;
-    struct Entry {
-        int64_t key[8];
-        uint64_t generation;
-        Value value;
-    };
-    Entry entry[kEntries] = {};
-    template <typename Compute>
-    Value get(const int64_t (&key)[8], Compute compute) {
-        uint64_t h = 1469598103934665603ull;
-        for (int64_t k : key) h = (h ^ (uint64_t)k) * 1099511628211ull;
-        Entry &e = entry[h % kEntries];
-        const uint64_t generation = tuning().generation;
-        bool hit = e.generation == generation;
-        for (int i = 0; i < 8 && hit; i++) hit = e.key[i] == key[i];
-        if (!hit) {
-            e.value = compute();
-            for (int i = 0; i < 8; i++) e.key[i] = key[i];
-            e.generation = generation;
-        }
-        return e.value;
-    }
-};
 struct TpPlan {
     int nseg, seg_chunks;
 };
@@ -926,12 +948,11 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         pl.workspace_bytes = tp_exchange_workspace_bytes(chains * blocks, pl.nseg,
                                                          fused_tp ? fused_tp_state_rows(D) : grads ? kGradStateRows : D);
     } else if (tp) {  // one workgroup per chain segment, nothing to exchange
-        const int64_t chunks = (L + kChunk - 1) / kChunk;
-        if (tph_takes_rows(D) && !(odd && forced) && !fused && combo == kFFFF)  // (scan_tph_kernel)
-            pl.nseg = tp_segment_starts(chunks, tp_nseg, tp_start, kTpAhead, 0.6);
-        else  // (half steps beyond 64 chunks: a longer search for a smaller share of a segment)
-            pl.nseg = tp_segment_starts(chunks, tp_nseg, tp_start, combo == kFFFF && chunks <= 64 ? kTpAhead / 2 : kTpAhead,
-                                        D > 32 && D <= 64 && scans[0].out.dtype == FTC_F32 && (fused || tp_nseg > 2) ? 0.45 : 0.55);
+        const bool scaled = tph_takes_rows(D) && !(odd && forced) && !fused && combo == kFFFF;  // (scan_tph_kernel)
+        const TpCuts cuts = tp_cuts(D, scaled, combo == kFFFF, scans[0].out.dtype == FTC_F32, fused != nullptr, tp_nseg,
+                                    (L + kChunk - 1) / kChunk);
+        pl.nseg = cuts.nseg;
+        for (int i = 0; i <= pl.nseg; i++) tp_start[i] = cuts.start[i];
         pl.seg_len = (int)L;
         pl.waves = chains * pl.nseg;
         pl.workspace_bytes = 0;

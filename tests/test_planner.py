@@ -3,7 +3,8 @@ read through ``ftc_causal_dot_plan``: nothing is launched, no GPU is needed.
 
 The figures pinned here are the planner's rules as documented where the planner lives
 (csrc/ftc_mfma.hip): one workgroup per chain segment on up to 256 CUs, chains of up to 64
-chunks cut without an exchange at multiples of four chunks with later segments shorter,
+chunks cut without an exchange at multiples of four chunks (two where fp32 rows are multiplied in
+three bf16 pieces) with later segments shorter,
 longer chains on few CUs with an exchange, everything the MFMA kernels do not cover on the
 generic kernel."""
 import re
@@ -341,3 +342,32 @@ def test_odd_widths_lie_in_place_only_where_their_copies_run_on_the_same_kernel(
     mixed = lines((9, 11, 1531, 25, 33)[:4], (9, 11, 1531, 33), backward=True)
     assert mixed[0].startswith("scan_tph_kernel: 2 scans") and mixed[1].startswith("pad_rows_kernel: 3 operands")
     assert mixed[2].startswith("scan_dma_kernel: 1 scan")
+
+
+def cut_chunks(line):
+    return [int(x) for x in field(line, r"cuts at chunks ([\d,]*\d)").split(",")]
+
+
+def test_cuts_on_three_pieces(monkeypatch):
+    """fp32 rows in three bf16 pieces may start a segment at every second chunk, of chains of up to 64 chunks; bf16
+    rows start at every fourth."""
+    assert cut_chunks(lines((1, 24, 500, 100), (1, 24, 500, 100))[0]) == [0, 2, 10, 14, 16]
+    assert cut_chunks(lines((1, 2, 295, 31), (1, 2, 295, 31))[0]) == [0, 2, 4, 8, 10]     # 32 rows, one position first
+    assert cut_chunks(lines((1, 2, 745, 25), (1, 2, 745, 33))[0]) == [0, 10, 18, 22, 24]  # 64 rows
+    long = lines((1, 60, 4000, 100), (1, 60, 4000, 100))[0]
+    assert long.startswith("scan_tp_kernel: 1 scan") and cut_chunks(long) == [0, 84, 125]
+    bf16 = lines((1, 40, 1000, 64), (1, 40, 1000, 64), dtype=_native.FTC_BF16)[0]
+    assert bf16.startswith("scan_tp_bf16_kernel: 1 scan") and cut_chunks(bf16) == [0, 16, 24, 28, 32]
+    # the fused attention's launches have the cuts of a single scan on that kernel, from three segments on
+    # (tests/test_fused_attention_gpu.py runs these; FTC_TPH=0 keeps two fp16 pieces out)
+    monkeypatch.setenv("FTC_TPH", "0")
+    _native.load().ftc_tuning_reload()
+    try:
+        for (N, L, H, E, M), cuts in [((20, 300, 3, 64, 64), [0, 2, 6, 8, 10]), ((10, 1000, 6, 64, 64), [0, 10, 22, 28, 32]),
+                                      ((25, 129, 2, 32, 64), [0, 2, 4, 5])]:
+            line = lines((N, H, L, E), (N, H, L, M))[0]
+            assert line.startswith("scan_tp_kernel: 1 scan") and cut_chunks(line) == cuts
+    finally:
+        monkeypatch.delenv("FTC_TPH")
+        _native.load().ftc_tuning_reload()
+
