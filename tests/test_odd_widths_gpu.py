@@ -55,6 +55,24 @@ def _odd_widths_in_place(shape, cp, _native):
         assert scale_error(got.cpu(), ex) <= max(4 * scale_error(ref, ex), 2e-6)
 
 
+@pytest.mark.parametrize("shape,cuts", [((1, 2, 295, 31, 31), "0,2,4,8,10"), ((1, 2, 745, 25, 33), "0,10,18,22,24")],
+                         ids=["32_rows", "64_rows"])
+def test_three_pieces_cut_at_half_a_trip(shape, cuts):
+    """Segments that start at 2 modulo 4 chunks, after a first walk of two positions and of more; one and two groups
+    of 32 state rows."""
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = shape
+    line = _native.plan((N, H, L, E), (N, H, L, M))
+    assert line.startswith("scan_tp_kernel: 1 scan") and "cuts at chunks %s," % cuts in line
+    Q, K, V, _ = oracle.make_inputs(N, H, L, E, M, seed=41)
+    out = torch.full((N, H, L, M), float("nan"), device="cuda")
+    cp.causal_dot_product_hip(Q.cuda(), K.cuda(), V.cuda(), out)
+    assert _native.load().ftc_last_kernel() == b"scan_tp_kernel"
+    exact = oracle.forward(Q.double(), K.double(), V.double())
+    assert scale_error(out.cpu(), exact) <= max(4 * scale_error(oracle.forward(Q, K, V), exact), 2e-6)
+
+
 def test_odd_widths_with_no_room_for_an_exchange():
     """A long chain whose segments would exchange their sums, with a workspace that has room for
     the generic kernel only: served as before, and not refused."""
