@@ -1460,7 +1460,7 @@ static int attention_backward(const ftc_tensor4 *queries, const ftc_tensor4 *key
                       denominators->stride[2], FTC_F32, 1};
     const Operand q = as_operand(queries), k = as_operand(keys), v = as_operand(values), g = as_operand(grad_out);
     // Rows of 64 values where the three scans share a launch of the chain-parallel kernel: they take q, k,
-    // v and grad_out as they are (N=10, H=8, L=4096: 375 -> 263 us), if no gradient is written over what any of
+    // v and grad_out as they are (N=10, H=8, L=4096: 381 -> 250 us), if no gradient is written over what any of
     // them reads: the workgroups of a cut chain read rows that another one's results belong to.  (The scans
     // below read copies: grad_values alone may lie over the queries.)
     if (d.E == 64 && d.M == 64) {

@@ -189,10 +189,11 @@ constexpr int kTpPieceBytes = 3 * (PA + PB + PV) * kChunk * 128;
 constexpr int kTpPtBytes = 2 * 3 * kChunk * 64;
 // Whether a kernel's loop over chunks is unrolled three times, with its buffers in the instructions' offsets
 // (and three of Pt).  The fused attention, where the vector instructions of a producer and a consumer together
-// fill their SIMD: 535 of them a chunk -> 515 this way, with the quadrant in two sums for four and its
-// edges on branches; 80 chains, L=1000 36.4 -> 34.7 us, L=4096 137 -> 124.  bf16 rows, where a consumer's stream
-// is what a chunk waits for: forward, 64 chains, L=2048 32.4 -> 30.5, 80 chains, L=1000 21.4 -> 19.9; 16384 positions of 128
-// chains of 32 x 128, training step 1799 -> 1756.  Not three pieces with two blocks: 108 registers would spill.
+// take 58 % of their SIMD's issue (SQ_ACTIVE_INST_VALU, 29 % of a wavefront's life): 535 of them a chunk -> 515 this
+// way, with the quadrant in two sums for four and its edges on branches; 80 chains, L=1000 36.4 -> 34.7 us, L=4096
+// 137 -> 124.  bf16 rows, where a consumer's stream is what a chunk waits for: forward, 64 chains, L=2048 32.4 -> 30.5,
+// 80 chains, L=1000 21.4 -> 19.9; 16384 positions of 128 chains of 32 x 128, training step 1799 -> 1756.  Not three
+// pieces with two blocks: 108 registers would spill.
 constexpr bool tp_unrolled(int ND, int pieces) { return ND == 1 || pieces < 9; }
 constexpr int kTpZBytes = 4 * 2 * 2 * 64;  // z of the four consumers, fused attention with two blocks
 

@@ -253,8 +253,12 @@ int64_t ftc_causal_linear_attention_backward_workspace_bytes(int64_t N, int64_t 
  *
  * out, denominators: what the forward wrote.  All tensors FTC_F32 with 16-byte aligned rows;
  * a gradient that is not wanted may be passed as NULL.  Sizes: E, M in {32, 64}.  The launch
- * sequence: one element-wise pass (feature maps, gz, dd into the workspace), the three scans
- * of ftc_causal_dot_backward on them, and a prefix-sum pass over grad_queries and grad_keys.
+ * sequence where E = M = 64 and the chain-parallel kernel takes the scans: one pass over out and
+ * grad_out (dd and 1 / den into the workspace), then the three scans straight from the inputs, with
+ * the prefix sums and phi' inside.  Otherwise, and where a wanted gradient shares memory with
+ * queries, keys, values or grad_out: one element-wise pass (feature maps, gz, dd into the workspace),
+ * the three scans of ftc_causal_dot_backward on them, and two launches of prefix sums over grad_queries
+ * and grad_keys.
  */
 int ftc_causal_linear_attention_backward(const ftc_tensor4 *queries, const ftc_tensor4 *keys,
                                          const ftc_tensor4 *values, const int64_t *key_lengths,
