@@ -157,8 +157,7 @@ int tp_segment_starts(int64_t chunks, int nseg, int32_t *start, int step, double
     return nseg;
 }
 
-// The cuts of a launch of the chain-parallel kernel with a state of D rows: one rule for the launch and for what is
-// estimated of it.  `scaled`: on two fp16
+// The cuts of a launch of the chain-parallel kernel with a state of D rows.  `scaled`: on two fp16
 // pieces, where a chunk walked for its state alone takes 0.6 of the others (0.75 against 1.3 us with
 // every workgroup streaming rows); on three bf16 pieces 0.45 where a state of 33 to 64 rows writes fp32
 // results, 0.55 otherwise and for two segments of odd widths or of bf16 rows (128 chains, L=1088, forward
@@ -172,13 +171,6 @@ int tp_segment_starts(int64_t chunks, int nseg, int32_t *start, int step, double
 struct TpCuts {
     int nseg;
     int32_t start[kMaxTpSegments + 1];
-    double state_only;
-    // the longest workgroup, in chunks that produce rows, if one walked for its state takes `weight` of those
-    double longest(double weight) const {
-        double most = 0.0;
-        for (int i = 0; i < nseg; i++) most = std::max(most, weight * start[i] + (double)(start[i + 1] - start[i]));
-        return most;
-    }
 };
 TpCuts tp_cuts(int64_t D, bool scaled, bool fp32_rows, bool fp32_results, bool fused, int nseg, int64_t chunks) {
     const int step = !scaled && fp32_rows && chunks <= 64 ? kTpAhead / 2 : kTpAhead;
@@ -188,8 +180,7 @@ TpCuts tp_cuts(int64_t D, bool scaled, bool fp32_rows, bool fp32_results, bool f
     const int64_t key[8] = {chunks, nseg, step, percent, 0, 0, 0, 0};
     return memo.get(key, [&]() {
         TpCuts c = {};
-        c.state_only = 0.01 * percent;
-        c.nseg = tp_segment_starts(chunks, nseg, c.start, step, c.state_only);
+        c.nseg = tp_segment_starts(chunks, nseg, c.start, step, 0.01 * percent);
         return c;
     });
 }
@@ -467,13 +458,16 @@ void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_
     const double chunk_us = (D <= 32 ? 0.48 : D <= 64 ? 0.65 : D <= 96 ? 0.98 : 1.12) * (bf16_results ? 1.25 : 1.0);
     double least = 1e30;
     if (chunks <= (bf16_results ? 1024 : 256)) {
-        const int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), chunks)) : 1;
-        const TpCuts cuts = tp_cuts(D, false, false, !bf16_results, false, n, chunks);
-        // (bf16 results: the estimate is better at 0.6 for a chunk walked for its state.  Backward calls whose
-        // choice between cuts and an exchange moves at 0.55, 153 of 9053: 1.03 times as long; the
-        // forwards whose choice moves from 0.6 to the launch's own rule, 160: 0.95)
-        least = (double)((units * cuts.nseg + 255) / 256) * (cuts.longest(bf16_results ? 0.6 : cuts.state_only) * chunk_us + 4.7) + 0.5;
-        *nseg = cuts.nseg;
+        int32_t start[kMaxTpSegments + 1];
+        int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), chunks)) : 1;
+        n = tp_segment_starts(chunks, n, start, kTpAhead, 0.6);
+        double longest = (double)chunks;
+        if (n > 1) {
+            longest = 0;
+            for (int i = 0; i < n; i++) longest = std::max(longest, 0.6 * start[i] + (double)(start[i + 1] - start[i]));
+        }
+        least = (double)((units * n + 255) / 256) * (longest * chunk_us + 4.7) + 0.5;
+        *nseg = n;
     }
     // (not below 24 chunks, 28 of wide states: 16 of them, 1 chain of 64 x 64 backward 14.4 us against 13.5 cut in
     // four; 25, 12 chains of 128 x 64 backward 46 against 42)
@@ -779,8 +773,10 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
     if (seg_chunks > 0) {
         longest = 1.6 * seg_chunks + 4.0;
     } else {
-        const TpCuts cuts = tp_cuts(D, tph_takes_rows(D) && !forced, true, true, false, nseg, (L + kChunk - 1) / kChunk);
-        longest = cuts.longest(cuts.state_only);
+        int32_t start[kMaxTpSegments + 1];
+        nseg = tp_segment_starts((L + kChunk - 1) / kChunk, nseg, start, kTpAhead, 0.6);
+        for (int s = 0; s < nseg; s++)
+            longest = std::max(longest, 0.6 * start[s] + (double)(start[s + 1] - start[s]));
     }
     return (double)rounds * ((D > 64 ? 1.7 : 1.0) * longest + 4.0);
 }

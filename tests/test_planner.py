@@ -371,11 +371,3 @@ def test_cuts_on_three_pieces(monkeypatch):
         monkeypatch.delenv("FTC_TPH")
         _native.load().ftc_tuning_reload()
 
-
-def test_cuts_and_exchanges_are_priced_as_they_are_launched():
-    """bf16 rows, forward: chains that the launch's cuts make shorter than an exchange of segment sums (us, before /
-    this way: 40 chains, L=1800 27.4 / 23.2; 20 chains of 64 x 128, L=1800 27.4 / 23.5); odd widths: the scans of a backward
-    call side by side or a launch for each (16 chains, L=1000, 33 x 65 56.4 / 38.6)."""
-    for N, H, L, E, M in [(1, 40, 1800, 64, 64), (1, 20, 1800, 64, 128), (1, 4, 1000, 32, 128)]:
-        assert kernel(lines((N, H, L, E), (N, H, L, M), dtype=_native.FTC_BF16)[0]) == "scan_tp_bf16_kernel"
-    assert len(lines((1, 16, 1000, 33), (1, 16, 1000, 65), backward=True)) == 1
