@@ -458,6 +458,10 @@ void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_
     const double chunk_us = (D <= 32 ? 0.48 : D <= 64 ? 0.65 : D <= 96 ? 0.98 : 1.12) * (bf16_results ? 1.25 : 1.0);
     double least = 1e30;
     if (chunks <= (bf16_results ? 1024 : 256)) {
+        // (priced at 0.6 in steps of kTpAhead, as fitted, and not as tp_cuts has them launched: at the launch's price
+        // bf16 forwards of 20 to 60 chunks on few chains would be cut instead of exchanging sums, 160 of 9053
+        // launches in 0.95 of their time, but their sums run over longer segments, 1.08e-7 from float64 for
+        // 1.00e-7; backward calls would take 1.03 times as long)
         int32_t start[kMaxTpSegments + 1];
         int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), chunks)) : 1;
         n = tp_segment_starts(chunks, n, start, kTpAhead, 0.6);
@@ -773,6 +777,8 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
     if (seg_chunks > 0) {
         longest = 1.6 * seg_chunks + 4.0;
     } else {
+        // (at the price of tp_cuts more scans of two shapes would share a launch, 43 calls of 18106 in 0.88 of their
+        // time, but 31 x 120 came out 3.5e-7 from float64 for 2.1e-7 and 75 x 10 2.5e-7 for 1.6e-7)
         int32_t start[kMaxTpSegments + 1];
         nseg = tp_segment_starts((L + kChunk - 1) / kChunk, nseg, start, kTpAhead, 0.6);
         for (int s = 0; s < nseg; s++)
