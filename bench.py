@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139671778, "31f53a40a05884d0"),
-    "cfg3": (2608158152, "31f53a40a05884d0"),
-    "cfg5": (4148561016, "31f53a40a05884d0"),
-    "wide": (1877115208, "31f53a40a05884d0"),
+    "cfg2": (139826373, "c4ea3dca9af73a8a"),
+    "cfg3": (2616595729, "c4ea3dca9af73a8a"),
+    "cfg5": (4148385092, "c4ea3dca9af73a8a"),
+    "wide": (1877122838, "c4ea3dca9af73a8a"),
 }
 
 WORKLOADS = {
