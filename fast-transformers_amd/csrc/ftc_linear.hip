@@ -14,9 +14,9 @@
 // library rounds after every few: against float64 a product of 40960 x 512 by 512 x 512 is off by
 // 1.9e-7 (2-norm) where the library's is by 2.9e-7, of 1024 columns by 2.6e-7 and 4.1e-7.
 //
-// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 85, 512 -> 1536 475 / 226, 512 -> 1024
-// with relu 310 + 51 / 155, 1024 -> 512 with the residual 305 + 37 / 162; 5000 tokens, 256 -> 512 20 / 11;
-// 300 tokens, 128 -> 260 31 / 4.2.  (At the largest sizes the card's power bounds it: on zeros 230 -> 189.)
+// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 74, 512 -> 1536 475 / 189, 512 -> 1024
+// with relu 310 + 51 / 135, 1024 -> 512 with the residual 305 + 37 / 139; 5000 tokens, 256 -> 512 20 / 11;
+// 300 tokens, 128 -> 260 31 / 4.2.  (At the largest sizes the card's power bounds it: on zeros 189 -> 165.)
 //
 // Rows in pieces take the bytes of fp32 rows: block of 32 columns after block, 64 bytes of hi and 64
 // of lo each, one cache line per row and k-step.  Whoever writes rows that only a product reads
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
 #pragma unroll
             for (int j = 0; j < WT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         uint32_t before = 0;
-        for (int s = 0; s < steps; s++) {
+        auto step = [&](int s, auto first, auto last) {
             // The next step's rows have landed (in flight: those of the steps after it and, where
             // these steps were all requested before the rows of the tile before went out, those
             // rows and this tile's scales), and every wavefront has what it needs of this
@@ -430,17 +430,16 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
                     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFlying) : "memory");
             };
             const uint32_t later = after(now);
-            constexpr std::true_type yes{};
-            constexpr std::false_type no{};
-            if (s == 0)
-                compute(tiles + now, tiles + later, now, before, yes, no, wait);
-            else if (s + 1 < steps)
-                compute(tiles + now, tiles + later, now, before, no, no, wait);
-            else
-                compute(tiles + now, tiles + later, now, before, no, yes, wait);
+            compute(tiles + now, tiles + later, now, before, first, last, wait);
             before = now;
             now = later;
-        }
+        };
+        // (The first and the last step stand outside the loop: as one of three bodies inside it each left the
+        // sums in registers of its own, and up to 124 moves a step brought them back together, waiting for the
+        // matrix instructions: 40960 tokens, 512 -> 1536 213 us, 189 this way; 1352, 1024 -> 512 14.8 and 10.2.)
+        step(0, std::true_type{}, std::false_type{});
+        for (int s = 1; s < steps - 1; s++) step(s, std::false_type{}, std::false_type{});
+        step(steps - 1, std::false_type{}, std::true_type{});
         // (this tile's scales: seen to have landed by the steps' waits where there are enough of them)
         if (steps <= STAGES) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // ---- rows out: every store is made, those outside the tensor outside the descriptor, so
@@ -539,19 +538,20 @@ void launch_product(LinearArgs a, hipStream_t stream) {
 // CU: together, and one alone), a tile's rows out the third number, and the launch lasts as long as
 // its busiest XCD of 32 CUs.  Measured (us, 128 x 256 / 64 x 128 / 64 x 64 / 32 x 64; the library's
 // product is none of these):
-//   40960 tokens, 512 -> 1536   230 / 249 / 289 / 385     1352 tokens, 1024 -> 512  46 / 20 / 15 / 15
-//   40960 tokens, 1024 -> 512   166 / 164 / 200 / 263     169 tokens, 1024 -> 256   46 / 19 / 14 / 11
-//   12000 tokens, 256 -> 768     32 /  23 /  24 /  34     169 tokens, 256 -> 768    16 / 7.1 / 5.7 / 4.8
+//   40960 tokens, 512 -> 1536   189 / 225 / 261 / 328     1352 tokens, 1024 -> 512  35 / 13 / 10 / 10
+//   40960 tokens, 512 -> 512     79 /  74 /  84 / 106     169 tokens, 1024 -> 256   34 / 13 / 9.5 / 7.8
+//   40960 tokens, 1024 -> 512   139 / 154 / 184 / 239     169 tokens, 256 -> 768    14 / 5.8 / 4.6 / 4.8
+//   12000 tokens, 256 -> 768     27 /  21 /  22 /  28     2700 tokens, 512 -> 1536  22 / 20 / 19 / 22
 // On few tiles a step is the latency of its barrier, its LDS reads and its matrix instructions one
 // after the other, so the smallest tile has the shortest; on many the large tile reads the least of
-// the L2 and the LDS per matrix instruction (its rate there, 0.83 PFLOP/s of fp16 pieces, rises by a
-// fifth on operands of zeros: the clock under that load is part of the bound).
+// the L2 and the LDS per matrix instruction (its rate there, 1.02 PFLOP/s of fp16 pieces, rises by a
+// seventh on operands of zeros: the clock under that load is part of the bound).
 struct ProductTile {
     int tokens, features, per_cu;
     double step, step_alone, rows;
 };
 constexpr ProductTile kProductTiles[] = {
-    {128, 256, 1, 1.65, 1.65, 3.0}, {64, 128, 2, 0.95, 0.50, 1.5}, {64, 64, 2, 0.57, 0.31, 1.0}, {32, 64, 2, 0.40, 0.21, 0.7}};
+    {128, 256, 1, 1.22, 0.89, 4.8}, {64, 128, 2, 0.78, 0.27, 0.5}, {64, 64, 2, 0.47, 0.18, 0.0}, {32, 64, 2, 0.31, 0.13, 0.0}};
 int product_tile(int64_t tokens, int64_t features, int64_t steps) {
     int best = 0;
     double least = 0;
