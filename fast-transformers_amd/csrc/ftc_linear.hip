@@ -14,9 +14,10 @@
 // library rounds after every few: against float64 a product of 40960 x 512 by 512 x 512 is off by
 // 1.9e-7 (2-norm) where the library's is by 2.9e-7, of 1024 columns by 2.6e-7 and 4.1e-7.
 //
-// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 74, 512 -> 1536 475 / 189, 512 -> 1024
-// with relu 310 + 51 / 135, 1024 -> 512 with the residual 305 + 37 / 139; 5000 tokens, 256 -> 512 20 / 11;
-// 300 tokens, 128 -> 260 31 / 4.2.  (At the largest sizes the card's power bounds it: on zeros 189 -> 165.)
+// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 74, 512 -> 1536 475 / 171, 512 -> 1024
+// with relu 310 + 51 / 123, 1024 -> 512 with the residual 305 + 37 / 132; 5000 tokens, 256 -> 512 20 / 11;
+// 300 tokens, 128 -> 260 31 / 4.2.  (At the largest sizes the card's power and the rows' way out bound it: 512 -> 1536
+// on zeros 189 -> 165, without its stores 148, both before LATER and kStreamed below.)
 //
 // Rows in pieces take the bytes of fp32 rows: block of 32 columns after block, 64 bytes of hi and 64
 // of lo each, one cache line per row and k-step.  Whoever writes rows that only a product reads
@@ -202,7 +203,15 @@ struct LinearArgs {
     float *out_scale;
     int64_t tokens;
     int32_t features, k, feature_tiles;
+    bool streamed;                       // the rows go out past what is worth keeping in the caches
 };
+constexpr int kStreamed = 2;             // (a store's nt bit)
+// Bytes that a product reads and writes from which on its rows are streamed.  Up to the Infinity Cache's 256 MB
+// the next kernel finds them there; beyond, they only push out what both read again.  Streamed rows have to
+// leave in whole lines.  Eight layers at 40960 tokens, d = 512, feed-forward 1024 (us, none / half lines / lines) 6470 /
+// 6266 / 6156; four at 30400 2299 / - / 2277; 1024 -> 512 at 40960 tokens 133 / 142 / 128.  From 140 MB on
+// instead, four layers at 24576 tokens take 2063 us for 1990, and from none on at 20480 1749 for 1682.
+constexpr int64_t kStreamedBytes = (int64_t)176 << 20;
 enum { kPlain = 0, kResidual = 1, kRelu = 2 };
 
 // a raw buffer of `bytes` bytes
@@ -225,6 +234,18 @@ __device__ __forceinline__ void load_dword_to_lds(const u32x4 rs, uint32_t to, u
                  :: "s"(to), "v"(offset), "s"(rs) : "memory", "m0");
 }
 
+// What lanes 8 to 15 of a row of 16 have from lanes 0 to 7 of `other`, the others their own, and the reverse
+// (row_ror:8, written to the lanes of two of its four banks).
+__device__ __forceinline__ uint32_t upper_from_lower(uint32_t own, uint32_t other) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)own, (int)other, 0x128, 0xf, 0xc, false);
+}
+__device__ __forceinline__ uint32_t lower_from_upper(uint32_t own, uint32_t other) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)own, (int)other, 0x128, 0xf, 0x3, false);
+}
+__device__ __forceinline__ uint32_t other_half(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, false);
+}
+
 // A workgroup of four wavefronts takes tiles of TN tokens by TF features one after the other, a
 // wavefront half of either.  v_mfma_f32_16x16x32_f16 with the features as rows of the result, so
 // that a lane has four consecutive features of one token.  A k-step's rows (128 bytes each) go from
@@ -233,19 +254,35 @@ __device__ __forceinline__ void load_dword_to_lds(const u32x4 rs, uint32_t to, u
 // Split: with 64 x 128 results per wavefront a step reads 24 KB of fragments for 96 matrix
 // instructions (1536 cycles); smaller tiles read more of the LDS per instruction, and are there for
 // products of few tiles (product_tile, below, where both are measured).
-template <int TN, int TF, int STAGES, int EPI>
+// Which feature row r of a feature tile's rows in LDS is.  Rows that leave in pieces: a lane has eight
+// consecutive features, 8 g to 8 g + 7 of 32, in two tiles of 16, so that 16 bytes of hi and 16 of lo are one
+// store each, of 64 consecutive bytes of a token (in 8-byte stores of 32: 40960 tokens, 512 -> 1024 135 us for 123).
+template <bool PIECES>
+__device__ __forceinline__ constexpr int feature_of(int r) {
+    return PIECES ? r / 32 * 32 + 8 * (r % 16 / 4) + 4 * (r / 16 % 2) + r % 4 : r;
+}
+// LATER: a tile's rows go out during the next one's steps 1 to 8, four stores a step, the scaling under the
+// matrix instructions (products of at least 10 steps on more than one round of tiles; the tile before waits in
+// the registers that four wavefronts on a CU leave).  Otherwise all workgroups of a round write their rows, 33 MB,
+// at once and compute nothing meanwhile.  With kStreamed, 40960 tokens, 512 -> 1536 178 -> 167 us, 512 -> 1024
+// 119 either way; without, 11536 tokens, 512 -> 1536 65 -> 61; one round of tiles 25.8 -> 27.5.  (Wavefronts that
+// only request rows, two beside the four, which then never wait for their stores to land, gained 1 %, small tiles lost up to 15 %.)
+constexpr int kLaterSteps = 9;           // the first step and eight
+template <int TN, int TF, int STAGES, int EPI, bool LATER = false>
 __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     constexpr int WT = TN / 32, WF = TF / 32;          // tiles of 16 per wavefront
     constexpr int kBuf = (TN + TF) * kRowBytes;
     constexpr int kLoadsX = TN * kRowBytes / 4096, kLoadsW = TF * kRowBytes / 4096;  // per lane
     constexpr int kRequests = kLoadsX + kLoadsW;                                     // of a step
-    constexpr int kStores = (EPI == kRelu ? 2 : 1) * WT * WF;                        // per lane
+    constexpr int kStores = WT * WF;                                                 // per lane
     // scales and bias of a tile's tokens and features, as each wavefront needs them (64 to a request)
     constexpr int kScaleT = TN / 2 < 64 ? 64 : TN / 2, kScaleF = TF / 2 < 64 ? 64 : TF / 2;
     constexpr int kScales = kScaleT + 2 * kScaleF, kScaleLoads = kScales / 64;
+    constexpr int kScaleSets = LATER ? 2 : 1;
+    static_assert(!LATER || (EPI != kResidual && WF > WT && kRequests <= 3 * (WF - WT)), "requests before the stores of a step");
     static_assert(WF % 2 == 0 && TN / 2 <= 64, "the fragments of w in turn; a wavefront's tokens in a request");
     __shared__ __align__(16) char tiles_mem[STAGES * kBuf];
-    __shared__ __align__(16) float scales_mem[4][kScales];
+    __shared__ __align__(16) float scales_mem[kScaleSets][4][kScales];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ln = lane & 15, g = lane >> 4;
@@ -283,11 +320,12 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
 #pragma unroll
     for (int i = 0; i < kLoadsW; i++) {
         const int j = (i * 4 + wave) * 64 + lane, row = j / 8;
-        w_off[i] = (uint32_t)row * row_bytes + 16u * ((j % 8) ^ TpSwizzle<128>::key(row));
+        w_off[i] = (uint32_t)feature_of<EPI == kRelu>(row) * row_bytes + 16u * ((j % 8) ^ TpSwizzle<128>::key(row));
     }
     lds_char *const tiles = (lds_char *)tiles_mem;
     const uint32_t lds0 = (uint32_t)(uintptr_t)tiles + 1024u * wave;
     const uint32_t scales0 = (uint32_t)(uintptr_t)(lds_char *)scales_mem + (uint32_t)(kScales * 4) * wave;
+    constexpr uint32_t kScaleSet = 4 * 4 * kScales;
     // The step whose rows are requested: STAGES steps ahead of the one that is computed, in this
     // tile or in a later one.
     Tile ahead = tile_of(0);
@@ -302,7 +340,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     auto advance = [&]() {
         if (++ahead_step == steps) ahead_step = 0, ahead = tile_of(++ahead_round);
     };
-    auto fetch_scales = [&](const Tile &t) {
+    auto fetch_scales = [&](const Tile &t, uint32_t scales0) {
         const u32x4 xs_rs = descriptor(p.x_scale + t.t0, (uint32_t)t.nt * 4u),
                     ws_rs = descriptor(p.w_scale + t.f0, (uint32_t)t.nf * 4u),
                     b_rs = descriptor(p.bias + t.f0, (uint32_t)t.nf * 4u);
@@ -342,10 +380,10 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     // of a tile's last step all before the rows go out, so that no later wait for them waits for
     // the rows.
     auto compute = [&](const lds_char *buf, const lds_char *next, uint32_t to_now, uint32_t to_before, auto first,
-                       auto last, auto wait) {
+                       auto last, auto wait, auto out) {
         constexpr int kSlots = 3 * WF;
         static_assert(kSlots >= kRequests, "a request per group of matrix instructions");
-        auto slot_of = [](int r) -> int { return r * kSlots / kRequests; };
+        auto slot_of = [](int r) -> int { return LATER ? r : r * kSlots / kRequests; };
         Frag xn[WT];
 #pragma unroll
         for (int i = 0; i < WF; i++) {
@@ -377,6 +415,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
 #pragma unroll
                 for (int j = 0; j < WT; j++)
                     acc[i][j] = mfma16h(w[i % 2][m == 0 ? 1 : 0], m == 1 ? xl[j] : xh[j], acc[i][j]);
+                if (LATER && m == 1 && i >= WF - 4 && i < WF - 1 && (WF - i) % 2 == 0) out((i - (WF - 4)) / 2);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -407,112 +446,239 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     first_frags(tiles);
     uint32_t now = 0;
     auto after = [&](uint32_t buf) -> uint32_t { return buf == (STAGES - 1) * kBuf ? 0u : buf + kBuf; };
+    // ---- rows out: every store is made, those outside the tensor outside the descriptor, so that
+    // their number is known to the waits ----
+    const uint32_t out_row = (uint32_t)p.features * 4u;
+    struct Rows {                        // a tile's
+        __amdgpu_buffer_rsrc_t rs;
+        int f0;
+        const float *scales;
+        float xs[WT], s_out[WT];
+        uint32_t at[WT][2];              // of a pair of feature tiles: either store's 16 bytes
+    };
+    const uint32_t upper = ln / 8;
+    auto token_at = [&](int j) { return (uint32_t)(wt * (TN / 2) + 16 * j + ln) * out_row + 16u * g; };
+    auto rows_of = [&](const Tile &t, const float *scales) -> Rows {
+        Rows r;
+        r.rs = __builtin_amdgcn_make_buffer_rsrc((EPI == kRelu ? (char *)p.out_pieces : (char *)p.out) + t.t0 * out_row, 0,
+                                                 (uint32_t)t.nt * out_row, kRsrcFlags);
+        r.f0 = t.f0 + wf * (TF / 2);
+        r.scales = scales;
+#pragma unroll
+        for (int j = 0; j < WT; j++) {
+            const int tok = 16 * j + ln;
+            r.xs[j] = scales[tok];
+            r.s_out[j] = 0.f;
+            if (EPI == kRelu) {
+                float inverse;
+                const float x_most = 32768.f * r.xs[j], bound = x_most * bound_w + bound_b;
+                scale_of(bound, r.s_out[j], inverse);
+                if (!(bound <= 64.f * (x_most * least_w))) r.s_out[j] = 0.f, inverse = -1.f;  // (in fp32)
+                const int64_t token = t.t0 + wt * (TN / 2) + tok;
+                if (t.f0 == 0 && wf == 0 && g == 0 && token < p.tokens) p.out_scale[token] = inverse;
+            }
+            const uint32_t whole = EPI == kRelu && r.s_out[j] == 0.f, row = (uint32_t)(wt * (TN / 2) + tok) * out_row;
+            const uint32_t whole_other = other_half(whole);
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint32_t half = p.streamed ? upper : u;
+                const bool own = !p.streamed || half == u;
+                const uint32_t wide = own ? whole : whole_other;
+                r.at[j][u] = (own ? row : u ? row + 8 * out_row : row - 8 * out_row) + (16u << wide) * g + (64u >> 2 * wide) * half;
+            }
+        }
+        return r;
+    };
+    struct Features { float4 ws[2], b[2]; };
+    auto features_of = [&](const Rows &r, int pair) -> Features {
+        Features w;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int fl = feature_of<EPI == kRelu>(32 * pair + 16 * u + 4 * g);
+            w.ws[u] = *(const float4 *)(r.scales + kScaleT + fl);
+            w.b[u] = *(const float4 *)(r.scales + kScaleT + kScaleF + fl);
+        }
+        return w;
+    };
+    // two tiles of 16 features of a token: 32 bytes per lane
+    auto pair_out = [&](const Rows &r, const Features &w, int pair, int j, const f32x4 &low, const f32x4 &high,
+                        const u32x4 *res) {
+        float y[2][4];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const f32x4 &sum = u ? high : low;
+            const float xs = r.xs[j];
+            y[u][0] = fmaf(sum[0] * xs, w.ws[u].x, w.b[u].x), y[u][1] = fmaf(sum[1] * xs, w.ws[u].y, w.b[u].y);
+            y[u][2] = fmaf(sum[2] * xs, w.ws[u].z, w.b[u].z), y[u][3] = fmaf(sum[3] * xs, w.ws[u].w, w.b[u].w);
+        }
+        uint32_t half[2][4];
+        bool whole = false;                  // the row in fp32 instead of pieces
+        if (EPI == kRelu) {
+            whole = r.s_out[j] == 0.f;
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) y[u][c] = y[u][c] < 0.f ? 0.f : y[u][c];  // (keeps NaN, as torch's does)
+                cut_quad_f16(y[u][0], y[u][1], y[u][2], y[u][3], r.s_out[j], half[0][2 * u], half[0][2 * u + 1],
+                             half[1][2 * u], half[1][2 * u + 1]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                if (EPI == kResidual) y[u][c] += __uint_as_float(res[u][c]);
+                if (EPI != kRelu || whole) half[u][c] = __float_as_uint(y[u][c]);
+            }
+        }
+        const int f0 = r.f0 + 32 * pair, f = EPI == kRelu ? f0 : f0 + 4 * g;
+        const uint32_t to = 4u * (uint32_t)f0;
+        if (p.streamed) {
+            // Lanes ln and ln ^ 8 change one half each, so that a store has whole lines: of tokens 0 to 7, of 8 to 15.
+            u32x4 low_tokens, high_tokens;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                low_tokens[c] = upper_from_lower(half[0][c], half[1][c]);
+                high_tokens[c] = lower_from_upper(half[1][c], half[0][c]);
+            }
+            const bool there = (EPI == kRelu ? f : f + 16 * (int)upper) < p.features;
+            __builtin_amdgcn_raw_buffer_store_b128(low_tokens, r.rs, there ? r.at[j][0] + to : 0x80000000u, 0, kStreamed);
+            __builtin_amdgcn_raw_buffer_store_b128(high_tokens, r.rs, there ? r.at[j][1] + to : 0x80000000u, 0, kStreamed);
+        } else {
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    u32x4{half[u][0], half[u][1], half[u][2], half[u][3]}, r.rs,
+                    (EPI == kRelu ? f : f + 16 * u) < p.features ? r.at[j][u] + to : 0x80000000u, 0, 0);
+        }
+    };
+    // (the tile before this one, of which the rows are still to go out)
+    f32x4 old[LATER ? WF : 1][LATER ? WT : 1];
+    Rows pending;
+    if (LATER) {
+        pending.rs = __builtin_amdgcn_make_buffer_rsrc((void *)p.x_scale, 0, 0, kRsrcFlags);
+        pending.f0 = 0, pending.scales = scales_mem[0][wave];
+#pragma unroll
+        for (int j = 0; j < WT; j++) pending.xs[j] = pending.s_out[j] = 0.f, pending.at[j][0] = pending.at[j][1] = 0;
+#pragma unroll
+        for (int i = 0; i < WF; i++)
+#pragma unroll
+            for (int j = 0; j < WT; j++) old[LATER ? i : 0][LATER ? j : 0] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     for (int round = 0;; round++) {
         const Tile t = tile_of(round);
         if (!t.there) break;
-        fetch_scales(t);
+        const int set = LATER ? round & 1 : 0;
+        fetch_scales(t, scales0 + set * kScaleSet);
 #pragma unroll
         for (int i = 0; i < WF; i++)
 #pragma unroll
             for (int j = 0; j < WT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         uint32_t before = 0;
-        auto step = [&](int s, auto first, auto last) {
-            // The next step's rows have landed (in flight: those of the steps after it and, where
-            // these steps were all requested before the rows of the tile before went out, those
-            // rows and this tile's scales), and every wavefront has what it needs of this
-            // step's buffer.
-            const bool rows_fly = round > 0 && s < STAGES - 1 && steps >= STAGES;
-            auto wait = [&]() {
-                constexpr int kMore = kFlying + kStores + kScaleLoads < 63 ? kFlying + kStores + kScaleLoads : 63;
-                if (rows_fly)
-                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kMore) : "memory");
-                else
-                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFlying) : "memory");
+        auto none = [](int) {};
+        auto advance_buffers = [&](uint32_t later) { before = now, now = later; };
+        if constexpr (LATER) {
+            // Stores of a step, two tokens' of two tiles of features: behind its requests, so that the waits of
+            // this step and of the next leave them in flight, and those of the one after do not.
+            constexpr int kPut = 4;
+            static_assert(WF == 8 && WT == 4, "eight steps");
+            auto step = [&](auto first, auto last, auto flying, auto out) {
+                const uint32_t later = after(now);
+                compute(tiles + now, tiles + later, now, before, first, last,
+                        [&]() {
+                            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier"
+                                         ::"n"(kFlying + decltype(flying)::value) : "memory");
+                        },
+                        out);
+                advance_buffers(later);
             };
-            const uint32_t later = after(now);
-            compute(tiles + now, tiles + later, now, before, first, last, wait);
-            before = now;
-            now = later;
-        };
-        // (The first and the last step stand outside the loop: as one of three bodies inside it each left the
-        // sums in registers of its own, and up to 124 moves a step brought them back together, waiting for the
-        // matrix instructions: 40960 tokens, 512 -> 1536 213 us, 189 this way; 1352, 1024 -> 512 14.8 and 10.2.)
-        step(0, std::true_type{}, std::false_type{});
-        for (int s = 1; s < steps - 1; s++) step(s, std::false_type{}, std::false_type{});
-        step(steps - 1, std::false_type{}, std::true_type{});
-        // (this tile's scales: seen to have landed by the steps' waits where there are enough of them)
-        if (steps <= STAGES) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        // ---- rows out: every store is made, those outside the tensor outside the descriptor, so
-        // that their number is known to the waits above ----
-        const uint32_t out_row = (uint32_t)p.features * 4u;
-        const __amdgpu_buffer_rsrc_t o_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (EPI == kRelu ? (char *)p.out_pieces : (char *)p.out) + t.t0 * out_row, 0, (uint32_t)t.nt * out_row,
-            kRsrcFlags);
-        const __amdgpu_buffer_rsrc_t r_rs = __builtin_amdgcn_make_buffer_rsrc(
-            (char *)(EPI == kResidual ? p.residual : p.bias) + (EPI == kResidual ? t.t0 * out_row : 0), 0,
-            (uint32_t)t.nt * out_row, kRsrcFlags);
-        const float *const scales = scales_mem[wave];
-        float xs[WT], s_out[WT];
-        uint32_t at[WT];
+            constexpr std::true_type yes{};
+            constexpr std::false_type no{};
+            step(yes, no, std::integral_constant<int, kScaleLoads>{}, none);
+            auto later_step = [&](auto group) {
+                constexpr int k = decltype(group)::value, pair = k / 2, j0 = k % 2 * 2;
+                const Features w = features_of(pending, pair);
+                step(no, no, std::integral_constant<int, kPut + (k == 0 ? kScaleLoads : kPut)>{}, [&](int j) {
+                    pair_out(pending, w, pair, j0 + j, old[2 * pair][j0 + j], old[2 * pair + 1][j0 + j], nullptr);
+                });
+            };
+            later_step(std::integral_constant<int, 0>{});
+            later_step(std::integral_constant<int, 1>{});
+            later_step(std::integral_constant<int, 2>{});
+            later_step(std::integral_constant<int, 3>{});
+            later_step(std::integral_constant<int, 4>{});
+            later_step(std::integral_constant<int, 5>{});
+            later_step(std::integral_constant<int, 6>{});
+            later_step(std::integral_constant<int, 7>{});
+            // (the wait of the step behind them leaves the last one's stores in flight, or waits for them)
+            for (int s = kLaterSteps; s < steps - 1; s++) step(no, no, std::integral_constant<int, 0>{}, none);
+            step(no, yes, std::integral_constant<int, 0>{}, none);
+            pending = rows_of(t, scales_mem[set][wave]);
 #pragma unroll
-        for (int j = 0; j < WT; j++) {
-            const int tok = 16 * j + ln;
-            xs[j] = scales[tok];
-            at[j] = (uint32_t)(wt * (TN / 2) + tok) * out_row;
-            if (EPI == kRelu) {
-                float inverse;
-                const float x_most = 32768.f * xs[j], bound = x_most * bound_w + bound_b;
-                scale_of(bound, s_out[j], inverse);
-                if (!(bound <= 64.f * (x_most * least_w))) s_out[j] = 0.f, inverse = -1.f;  // (in fp32)
-                const int64_t token = t.t0 + wt * (TN / 2) + tok;
-                if (t.f0 == 0 && wf == 0 && g == 0 && token < p.tokens) p.out_scale[token] = inverse;
+            for (int i = 0; i < WF; i++)
+#pragma unroll
+                for (int j = 0; j < WT; j++) old[LATER ? i : 0][LATER ? j : 0] = acc[i][j];
+        } else {
+            auto step = [&](int s, auto first, auto last) {
+                // The next step's rows have landed (in flight: those of the steps after it and, where
+                // these steps were all requested before the rows of the tile before went out, those
+                // rows and this tile's scales), and every wavefront has what it needs of this
+                // step's buffer.
+                const bool rows_fly = round > 0 && s < STAGES - 1 && steps >= STAGES;
+                auto wait = [&]() {
+                    constexpr int kMost = kFlying + (EPI == kResidual && decltype(last)::value ? 2 * WT : 0),
+                                  kMore = kMost + kStores + kScaleLoads < 63 ? kMost + kStores + kScaleLoads : 63;
+                    if (rows_fly)
+                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kMore) : "memory");
+                    else
+                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kMost) : "memory");
+                };
+                const uint32_t later = after(now);
+                compute(tiles + now, tiles + later, now, before, first, last, wait, none);
+                advance_buffers(later);
+            };
+            // (The first and the last step stand outside the loop: as one of three bodies inside it each left the
+            // sums in registers of its own, and up to 124 moves a step brought them back together, waiting for the
+            // matrix instructions: 40960 tokens, 512 -> 1536 213 us, 189 this way; 1352, 1024 -> 512 14.8 and 10.2.)
+            step(0, std::true_type{}, std::false_type{});
+            for (int s = 1; s < steps - 1; s++) step(s, std::false_type{}, std::false_type{});
+            const __amdgpu_buffer_rsrc_t r_rs = __builtin_amdgcn_make_buffer_rsrc(
+                (char *)(EPI == kResidual ? p.residual : p.bias) + (EPI == kResidual ? t.t0 * out_row : 0), 0,
+                (uint32_t)t.nt * out_row, kRsrcFlags);
+            // (residual rows a pair of feature tiles ahead, the first one under the last step: a wait for them then
+            // leaves the stores in flight)
+            u32x4 res[2][WT][2];
+            auto residual = [&](int pair) {
+                const int f = t.f0 + wf * (TF / 2) + 32 * pair;
+#pragma unroll
+                for (int j = 0; j < WT; j++)
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+                        res[pair % 2][j][u] = __builtin_amdgcn_raw_buffer_load_b128(
+                            r_rs, f + 16 * u + 4 * g < p.features ? token_at(j) + 4u * f + 64u * u : 0x80000000u, 0, 0);
+            };
+            if (EPI == kResidual) residual(0);
+            step(steps - 1, std::false_type{}, std::true_type{});
+            // (this tile's scales: seen to have landed by the steps' waits where there are enough of them)
+            if (steps <= STAGES) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const Rows rows = rows_of(t, scales_mem[0][wave]);
+#pragma unroll
+            for (int pair = 0; pair < WF / 2; pair++) {
+                const Features w = features_of(rows, pair);
+                if (EPI == kResidual && pair + 1 < WF / 2) residual(pair + 1);
+#pragma unroll
+                for (int j = 0; j < WT; j++)
+                    pair_out(rows, w, pair, j, acc[2 * pair][j], acc[2 * pair + 1][j], EPI == kResidual ? res[pair % 2][j] : nullptr);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        // (residual rows two feature tiles ahead: a wait for them then leaves the stores in flight)
-        u32x4 res[3][WT];
-        auto residual = [&](int i) {
-            const int f = t.f0 + wf * (TF / 2) + 16 * i + 4 * g;
+    }
+    if constexpr (LATER) {
 #pragma unroll
-            for (int j = 0; j < WT; j++)
-                res[i % 3][j] = __builtin_amdgcn_raw_buffer_load_b128(
-                    r_rs, f < p.features ? at[j] + 4u * f : 0x80000000u, 0, 0);
-        };
-        if (EPI == kResidual) residual(0), residual(1);
+        for (int pair = 0; pair < WF / 2; pair++) {
+            const Features w = features_of(pending, pair);
 #pragma unroll
-        for (int i = 0; i < WF; i++) {
-            const int fl = 16 * i + 4 * g, f = t.f0 + wf * (TF / 2) + fl;
-            const bool f_in = f < p.features;
-            const float4 ws = *(const float4 *)(scales + kScaleT + fl),
-                         b = *(const float4 *)(scales + kScaleT + kScaleF + fl);
-            if (EPI == kResidual && i + 2 < WF) residual(i + 2);
-#pragma unroll
-            for (int j = 0; j < WT; j++) {
-                float y0 = fmaf(acc[i][j][0] * xs[j], ws.x, b.x), y1 = fmaf(acc[i][j][1] * xs[j], ws.y, b.y),
-                      y2 = fmaf(acc[i][j][2] * xs[j], ws.z, b.z), y3 = fmaf(acc[i][j][3] * xs[j], ws.w, b.w);
-                if (EPI == kResidual) {
-                    const u32x4 r = res[i % 3][j];
-                    y0 += __uint_as_float(r.x), y1 += __uint_as_float(r.y);
-                    y2 += __uint_as_float(r.z), y3 += __uint_as_float(r.w);
-                }
-                if (EPI == kRelu) {
-                    uint32_t h0, h1, l0, l1;
-                    auto relu = [](float y) { return y < 0.f ? 0.f : y; };  // (keeps NaN, as torch's does)
-                    y0 = relu(y0), y1 = relu(y1), y2 = relu(y2), y3 = relu(y3);
-                    cut_quad_f16(y0, y1, y2, y3, s_out[j], h0, h1, l0, l1);
-                    const bool whole = s_out[j] == 0.f;  // the row in fp32, both halves of the quad
-                    if (whole) {
-                        h0 = __float_as_uint(y0), h1 = __float_as_uint(y1);
-                        l0 = __float_as_uint(y2), l1 = __float_as_uint(y3);
-                    }
-                    const uint32_t to = !f_in ? 0x80000000u
-                                        : whole ? at[j] + 4u * f
-                                                : at[j] + (uint32_t)(f / kStep * kRowBytes + 2 * (f % kStep));
-                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{h0, h1}, o_rs, to, 0, 0);
-                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{l0, l1}, o_rs, to + (whole ? 8u : 2u * kStep), 0, 0);
-                } else {
-                    buffer_store4(o_rs, f_in ? at[j] + 4u * f : 0x80000000u, y0, y1, y2, y3);
-                }
-            }
+            for (int j = 0; j < WT; j++) pair_out(pending, w, pair, j, old[2 * pair][j], old[2 * pair + 1][j], nullptr);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -526,6 +692,15 @@ void launch_product(LinearArgs a, hipStream_t stream) {
     // (a multiple of the eight XCDs)
     const int64_t tiles = (token_tiles + 7) / 8 * a.feature_tiles;
     const dim3 grid((unsigned)(8 * std::min<int64_t>(tiles, 32 * PER_CU))), block(256);
+    if constexpr (TN == 128) {
+        if (a.k / kStep > kLaterSteps && tiles > 32 && !a.residual) {
+            if (a.out_pieces)
+                hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kRelu, true>), grid, block, 0, stream, a);
+            else
+                hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kPlain, true>), grid, block, 0, stream, a);
+            return;
+        }
+    }
     if (a.out_pieces)
         hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kRelu>), grid, block, 0, stream, a);
     else if (a.residual)
@@ -538,14 +713,14 @@ void launch_product(LinearArgs a, hipStream_t stream) {
 // CU: together, and one alone), a tile's rows out the third number, and the launch lasts as long as
 // its busiest XCD of 32 CUs.  Measured (us, 128 x 256 / 64 x 128 / 64 x 64 / 32 x 64; the library's
 // product is none of these):
-//   40960 tokens, 512 -> 1536   189 / 225 / 261 / 328     1352 tokens, 1024 -> 512  35 / 13 / 10 / 10
-//   40960 tokens, 512 -> 512     79 /  74 /  84 / 106     169 tokens, 1024 -> 256   34 / 13 / 9.5 / 7.8
-//   40960 tokens, 1024 -> 512   139 / 154 / 184 / 239     169 tokens, 256 -> 768    14 / 5.8 / 4.6 / 4.8
-//   12000 tokens, 256 -> 768     27 /  21 /  22 /  28     2700 tokens, 512 -> 1536  22 / 20 / 19 / 22
+//   40960 tokens, 512 -> 1536   171 / 193 / 224 / 291     1352 tokens, 1024 -> 512  35 / 14 / 10 / 10
+//   40960 tokens, 512 -> 512     75 /  73 /  85 / 106     169 tokens, 1024 -> 256   34 / 13 / 9.6 / 8.0
+//   40960 tokens, 1024 -> 512   132 / 152 / 178 / 235     169 tokens, 256 -> 768    14 / 5.8 / 4.6 / 4.4
+//   12000 tokens, 256 -> 768     27 /  22 /  22 /  28     2700 tokens, 512 -> 1536  22 / 20 / 20 / 23
 // On few tiles a step is the latency of its barrier, its LDS reads and its matrix instructions one
 // after the other, so the smallest tile has the shortest; on many the large tile reads the least of
-// the L2 and the LDS per matrix instruction (its rate there, 1.02 PFLOP/s of fp16 pieces, rises by a
-// seventh on operands of zeros: the clock under that load is part of the bound).
+// the L2 and the LDS per matrix instruction (its rate there is 1.13 PFLOP/s of fp16 pieces, what a
+// large library product reaches here: the clock under that load is part of the bound).
 struct ProductTile {
     int tokens, features, per_cu;
     double step, step_alone, rows;
@@ -654,6 +829,7 @@ int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const 
     a.x = (const char *)x, a.w = (const char *)w, a.x_scale = x_scale, a.w_scale = w_scale, a.bias = bias;
     a.w_norm = w_norm, a.residual = residual, a.out = out, a.out_pieces = (char *)relu_pieces;
     a.out_scale = relu_scale, a.tokens = tokens, a.features = (int32_t)features, a.k = (int32_t)k;
+    a.streamed = 4 * tokens * (k + (residual ? 2 : 1) * features) >= kStreamedBytes;
     const hipStream_t on = (hipStream_t)stream;
     switch (product_tile(tokens, features, k / kStep)) {
     case 0: launch_product<128, 256, 3, 1>(a, on); break;

@@ -118,6 +118,47 @@ def test_products_are_the_same_on_every_tile(shape):
         assert not all_rows.isnan().any() and torch.equal(all_rows[T - few:], rows)
 
 
+@pytest.mark.parametrize("shape", [
+    # on the largest tile over more than one round of workgroups, where a tile's rows go out under the next
+    # one's products: the fewest steps that have room for that, rows and features that end inside a tile, and a
+    # product large enough for its rows to be streamed
+    (10237, 320, 1532), (20477, 512, 544), (22600, 512, 1536)], ids=lambda s: "t%d_k%d_f%d" % s)
+def test_rows_that_leave_under_the_next_tile(shape):
+    """Every row is bit for bit what products of a few thousand rows give (other tiles, rows at once)."""
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    T, K, F = shape
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x, w, b = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, K), (F, K), (F,)))
+    # (one bias beside which some rows' features are too small for pieces under one bound, others' not)
+    x *= torch.exp2(torch.randint(-6, 6, (T, 1), device="cuda", generator=gen).float())
+    b[F // 2] = 2.0 ** 10
+    new = lambda *s: torch.full(s, float("nan"), device="cuda")
+    xp, xs, wp, ws, bo, wn = new(T, K), new(T), new(F, K), new(F), new(F), new(F)
+    item = Weight(w.data_ptr(), b.data_ptr(), F, K, wp.data_ptr(), ws.data_ptr(), bo.data_ptr(), wn.data_ptr())
+    assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == 0, _native.last_error()
+    assert lib.ftc_split_rows(ptr(x), ctypes.c_int64(T), ctypes.c_int64(K), ptr(xp), ptr(xs), stream()) == 0
+
+    def run(first, last, relu):
+        out, scale = new(last - first, F), new(last - first)
+        rc = lib.ftc_linear_split(ptr(xp[first:]), ptr(xs[first:]), ctypes.c_int64(last - first), ptr(wp), ptr(ws),
+                                  ptr(bo), ptr(wn), ctypes.c_int64(F), ctypes.c_int64(K), None,
+                                  None if relu else ptr(out), ptr(out) if relu else None,
+                                  ptr(scale) if relu else None, stream())
+        assert rc == 0, _native.last_error()
+        return out, scale
+    for relu in (False, True) if F % 32 == 0 else (False,):
+        rows, scales = run(0, T, relu)
+        for first in range(0, T, 2500):
+            last = min(first + 2500, T)
+            part, part_scales = run(first, last, relu)
+            assert torch.equal(rows[first:last].view(torch.int32), part.view(torch.int32))
+            if relu:
+                assert torch.equal(scales[first:last], part_scales) and (part_scales > 0).all()
+        if not relu:
+            assert not rows.isnan().any()
+
+
 def test_relu_keeps_nan_and_takes_any_bias_below_zero():
     """Features switched off by a bias of the type's lowest value or -inf leave the other features'
     precision alone; NaN in a weight or a bias comes out as NaN, as from torch's relu."""
