@@ -761,20 +761,17 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
 #pragma unroll
         for (int i = 0; i < 12; i++) {
             if ((i % 4) / 2 < KS) S[i % 4] = mfma16h(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[i % 4]);
-            if (!GRAD) rm_frag(unit_pc + buf * kBufBytes, i);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
         read_slot(slots, buf, ce);  // the ceilings of our own first chunk
-    } else if (!GRAD) {
-#pragma unroll
-        for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
     }
+    uint32_t done = 0;  // consumers that have read all they need of the others
     if (exchange) {
         // ---- the sum of this segment's rows goes out, the state before the segment comes in ----
         const uint32_t total_units = (uint32_t)p.total_waves;
         gfloat *const sums = (gfloat *)(hdr + kControlBytes / 4);
         constexpr int DX = GRAD ? 2 : 1;  // (Z rides along in a tile of its own)
-        StateExchange<DX, 1> xch(flags, sums, 4u * total_units,
+        StateExchange<DX, 1, 4 / DX> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);
         f32x16 Sx[DX][1], X[DX][1];
@@ -792,6 +789,8 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         xch.gather(Sx, X);
         if (xch.failed && lane == 0)
             __hip_atomic_store(hdr + kHdrError, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (counted here and looked at in the end: what the others count meanwhile is waited for under the walk)
+        if (lane == 0) done = __hip_atomic_fetch_add(hdr + kHdrDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // the units of the first chunk of the second pass (its ceilings are already known)
         Ucur = ce.state_exp();
 #pragma unroll
@@ -804,10 +803,9 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         }
         if (!GRAD && op.s0) add_caller_state();
     }
-    if (GRAD) {  // (not before: two tiles are exchanged, and 48 registers of fragments beside them spilled)
+    // our own first chunk's (not before: with 48 registers of fragments beside the states that are exchanged, spills)
 #pragma unroll
-        for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
-    }
+    for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
     // ---- the walk proper ----
     // `ce` holds the ceilings of the chunk at hand, Ucur the units of S.  dU < 0: the
     // state's units rise by -dU with this chunk (S is rescaled once all of it has been cut).
@@ -1026,10 +1024,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
     // the last consumer of the launch leaves the control block zeroed
     if (exchange) {
         const uint32_t total_units = (uint32_t)p.total_waves;
-        uint32_t done = 0;
-        if (lane == 0)
-            done = __hip_atomic_fetch_add(hdr + kHdrDone, 1u, __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
         done = __builtin_amdgcn_readfirstlane(done);
         if (done == 4u * total_units - 1) {
             for (uint32_t i = lane; i < 4u * total_units; i += kWave)
