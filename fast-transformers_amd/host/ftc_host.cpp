@@ -539,30 +539,59 @@ struct Layer {
 };
 
 // One weight matrix (or several with the same number of columns, their rows one after the other)
-// in pieces.
+// in pieces, in memory that is handed out from `at` on.
 struct Pieces {
-    Tensor pieces, scale, bias, norm;
+    const float *pieces, *scale, *bias, *norm;
     int64_t rows, cols;
-    Pieces(std::initializer_list<const Linear *> parts, std::vector<ftc_weight> &list) {
+    static int64_t floats(std::initializer_list<const Linear *> parts) {
+        int64_t n = 0;
+        for (const Linear *l : parts) n += l->weight.size(0) * (l->weight.size(1) + 3);
+        return n;
+    }
+    Pieces(std::initializer_list<const Linear *> parts, std::vector<ftc_weight> &list, float *&at) {
         rows = 0, cols = (*parts.begin())->weight.size(1);
         for (const Linear *l : parts) rows += l->weight.size(0);
-        const auto fp32 = (*parts.begin())->weight.options();
-        pieces = at::empty({rows, cols}, fp32);
-        scale = at::empty({rows}, fp32), bias = at::empty({rows}, fp32), norm = at::empty({rows}, fp32);
-        int64_t at_row = 0;
+        float *const p = at, *const s = p + rows * cols, *const b = s + rows, *const n = b + rows;
+        at = n + rows;
+        pieces = p, scale = s, bias = b, norm = n;
+        int64_t row = 0;
         for (const Linear *l : parts) {
             ftc_weight w;
             w.w = l->weight.const_data_ptr<float>();
             w.bias = l->bias ? l->bias->const_data_ptr<float>() : nullptr;
             w.rows = l->weight.size(0), w.cols = cols;
-            w.pieces = pieces.data_ptr<float>() + at_row * cols;
-            w.scale = scale.data_ptr<float>() + at_row, w.bias_out = bias.data_ptr<float>() + at_row;
-            w.norm = norm.data_ptr<float>() + at_row;
+            w.pieces = p + row * cols, w.scale = s + row, w.bias_out = b + row, w.norm = n + row;
             list.push_back(w);
-            at_row += w.rows;
+            row += w.rows;
         }
     }
 };
+// The weights of consecutive layers in pieces, cut in one launch.
+struct LayerPieces {
+    Pieces in, proj, first, second;
+    static int64_t floats(const Layer &l) {
+        return Pieces::floats({&l.query, &l.key, &l.value, &l.out, &l.first, &l.second});
+    }
+    LayerPieces(const Layer &l, std::vector<ftc_weight> &list, float *&at)
+        : in({&l.query, &l.key, &l.value}, list, at), proj({&l.out}, list, at), first({&l.first}, list, at),
+          second({&l.second}, list, at) {}
+};
+// How many layers from `from` on have their weights cut at a time.  Few tokens: all of them, up to eight with
+// pieces of up to 64 MB, since a launch for each (5 to 9 us, much of it latency) is then a tenth of a layer's time.  With
+// more, where the rows of x have twice as many values as a layer's weights, one: the others' pieces
+// would be memory that the modules do not need, for 1 % of the time.
+// Eight layers, 4 x 338 tokens, d = 512 and feed-forward 512: 652 -> 575 us; four, 2 x 966, d = 128: 317 -> 250.
+size_t layers_at_a_time(const std::vector<Layer> &layers, size_t from, int64_t values) {
+    int64_t floats = LayerPieces::floats(layers[from]);
+    if (values > 2 * floats) return 1;
+    size_t n = 1;
+    while (n < 8 && from + n < layers.size()) {
+        floats += LayerPieces::floats(layers[from + n]);
+        if (4 * floats > (int64_t)64 << 20) break;
+        n++;
+    }
+    return n;
+}
 
 // A stack of post-norm encoder layers (attention/encoder.py) with causal linear attention, and the
 // final norm: every product on the fp16 matrix cores in pieces (csrc/ftc_linear.hip), the norms
@@ -607,10 +636,8 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
     // (either the rows themselves or, behind max(., 0), in pieces with a scale)
     auto linear = [&](const float *pieces, const float *pieces_scale, const Pieces &w, const float *residual,
                       float *y, float *relu_pieces, float *relu_scale) {
-        check(ftc_linear_split(pieces, pieces_scale, T, w.pieces.const_data_ptr<float>(),
-                               w.scale.const_data_ptr<float>(), w.bias.const_data_ptr<float>(),
-                               w.norm.const_data_ptr<float>(), w.rows, w.cols, residual, y, relu_pieces,
-                               relu_scale, stream),
+        check(ftc_linear_split(pieces, pieces_scale, T, w.pieces, w.scale, w.bias, w.norm, w.rows, w.cols, residual, y,
+                               relu_pieces, relu_scale, stream),
               "ftc_linear_split");
     };
     auto split = [&](const float *from, int64_t columns, float *pieces, float *pieces_scale) {
@@ -623,23 +650,35 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
     };
     native([&] {
         split(x.const_data_ptr<float>(), d, rows, row_scale);
+        Tensor weights;                  // of layers cut_from, cut_from + 1 ... in pieces
+        std::vector<LayerPieces> cut;
+        size_t cut_from = 0;
         for (size_t i = 0; i < layers.size(); i++) {
             const Layer &l = layers[i];
             const float *const input = i == 0 ? x.const_data_ptr<float>() : to;
-            std::vector<ftc_weight> list;
-            const Pieces in({&l.query, &l.key, &l.value}, list), proj({&l.out}, list), first({&l.first}, list),
-                second({&l.second}, list);
-            check(ftc_split_weights(list.data(), (int32_t)list.size(), stream), "ftc_split_weights");
-            linear(rows, row_scale, in, nullptr, qkv, nullptr, nullptr);
+            if (i == cut_from + cut.size()) {
+                const size_t n = layers_at_a_time(layers, i, T * d);
+                int64_t floats = 0;
+                for (size_t j = i; j < i + n; j++) floats += LayerPieces::floats(layers[j]);
+                cut.clear(), cut_from = i;
+                weights = Tensor();  // (given back first)
+                weights = at::empty({floats}, fp32);
+                float *at = weights.data_ptr<float>();
+                std::vector<ftc_weight> list;
+                for (size_t j = i; j < i + n; j++) cut.emplace_back(layers[j], list, at);
+                check(ftc_split_weights(list.data(), (int32_t)list.size(), stream), "ftc_split_weights");
+            }
+            const LayerPieces &w = cut[i - cut_from];
+            linear(rows, row_scale, w.in, nullptr, qkv, nullptr, nullptr);
             const ftc_tensor4 o = view(rows, 0, H * M, M);
             check(ftc_causal_linear_attention_forward(&q, &k, &v, lengths, (float)l.eps, &o, nullptr, call.ws,
                                                       call.ws_bytes, stream),
                   "ftc_causal_linear_attention_forward");
             split(rows, H * M, qkv, wide_scale);
-            linear(qkv, wide_scale, proj, input, projected, nullptr, nullptr);
+            linear(qkv, wide_scale, w.proj, input, projected, nullptr, nullptr);
             norm(projected, l.norm1, to, rows);
-            linear(rows, row_scale, first, nullptr, nullptr, qkv, wide_scale);
-            linear(qkv, wide_scale, second, to, rows, nullptr, nullptr);
+            linear(rows, row_scale, w.first, nullptr, nullptr, qkv, wide_scale);
+            linear(qkv, wide_scale, w.second, to, rows, nullptr, nullptr);
             if (i + 1 < layers.size()) {
                 norm(rows, l.norm2, to, other);
                 std::swap(rows, other);

@@ -307,7 +307,7 @@ typedef struct ftc_weight {
     float *bias_out;       /* out: bias, or zeros */
     float *norm;           /* out: sum of |w| along each row */
 } ftc_weight;
-/* Up to eight weight matrices into pieces. */
+/* Up to 48 weight matrices into pieces. */
 int ftc_split_weights(const ftc_weight *weights, int32_t count, void *stream);
 /* Dense fp32 rows into pieces. */
 int ftc_split_rows(const float *x, int64_t rows, int64_t cols, void *pieces, float *scale, void *stream);

@@ -377,3 +377,27 @@ def test_encoder_needs_no_more_memory_than_its_modules(ff, final):
     # (a layer's weights in pieces and the scales of the rows come on top)
     weights = 4 * 512 * (4 * 512 + 2 * ff + 16) + 2 * 4 * x.shape[0] * x.shape[1]
     assert native <= modules + 1.1 * weights
+
+
+@pytest.mark.parametrize("count", [1, 47, 48])
+def test_weights_of_many_matrices_are_cut_in_one_launch(count):
+    """Each matrix comes out as in a launch of its own, whatever its number and whatever stands beside it."""
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    gen = torch.Generator(device="cuda").manual_seed(count)
+    kept, items, alone = [], (Weight * count)(), (Weight * 1)()
+    for i in range(count):
+        F, K = 4 * (1 + i % 9), 32 * (1 + i % 5)
+        w, b = torch.randn(F, K, device="cuda", generator=gen), torch.randn(F, device="cuda", generator=gen)
+        outs = [[torch.full(s, float("nan"), device="cuda") for s in ((F, K), (F,), (F,), (F,))] for _ in range(2)]
+        for item, (p, s, bo, n) in ((items[i], outs[0]), (alone[0], outs[1])):
+            item.w, item.bias, item.rows, item.cols = w.data_ptr(), b.data_ptr() if i % 2 else None, F, K
+            item.pieces, item.scale, item.bias_out, item.norm = (t.data_ptr() for t in (p, s, bo, n))
+        assert lib.ftc_split_weights(alone, 1, stream()) == 0
+        kept.append((w, b, outs))
+    assert lib.ftc_split_weights(items, count, stream()) == 0, _native.last_error()
+    for w, b, (together, single) in kept:
+        for x, y in zip(together, single):
+            assert torch.equal(x.view(torch.int32), y.view(torch.int32))
+        assert (whole(*together[:2]) - w.double()).abs().max() <= 2.0 ** -22 * w.abs().max()
+    assert lib.ftc_split_weights((Weight * 49)(), 49, stream()) == -1
