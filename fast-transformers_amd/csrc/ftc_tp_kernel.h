@@ -858,7 +858,6 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
 #pragma unroll
         for (int i = 0; i < kRowFrags; i++) rm_frag(unit_pc, i, 0);
     }
-    uint32_t done = 0;  // consumers that have read all they need of the others
     if (exchange) {
         // ---- the sum of this segment's rows goes out, the state before the segment comes in ----
         const uint32_t total_units = (uint32_t)p.total_waves;
@@ -886,8 +885,6 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         xch.gather(Sx, X);
         if (xch.failed && lane == 0)
             __hip_atomic_store(hdr + kHdrError, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // (counted here and looked at in the end: what the others count meanwhile is waited for under the walk)
-        if (lane == 0) done = __hip_atomic_fetch_add(hdr + kHdrDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
         for (int hb = 0; hb < ND; hb++)
 #pragma unroll
@@ -1157,6 +1154,12 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
     // the last consumer of the launch leaves the control block zeroed (as in ftc_wg_kernel.h)
     if (exchange) {
         const uint32_t total_units = (uint32_t)p.total_waves;
+        // (not where a consumer has gathered, so that others are waited for under the walk: all of them count then while
+        // the last ones look at their flags; attention, 64 chains, L=1600 52.7 -> 54.9 us, 40, L=2000 44.6 -> 46.9)
+        uint32_t done = 0;
+        if (lane == 0)
+            done = __hip_atomic_fetch_add(hdr + kHdrDone, 1u, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
         done = __builtin_amdgcn_readfirstlane(done);
         if (done == 4u * total_units - 1) {
             for (uint32_t i = lane; i < 4u * total_units; i += kWave)

@@ -765,7 +765,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         }
         read_slot(slots, buf, ce);  // the ceilings of our own first chunk
     }
-    uint32_t done = 0;  // consumers that have read all they need of the others
     if (exchange) {
         // ---- the sum of this segment's rows goes out, the state before the segment comes in ----
         const uint32_t total_units = (uint32_t)p.total_waves;
@@ -789,8 +788,6 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         xch.gather(Sx, X);
         if (xch.failed && lane == 0)
             __hip_atomic_store(hdr + kHdrError, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // (counted here and looked at in the end: what the others count meanwhile is waited for under the walk)
-        if (lane == 0) done = __hip_atomic_fetch_add(hdr + kHdrDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // the units of the first chunk of the second pass (its ceilings are already known)
         Ucur = ce.state_exp();
 #pragma unroll
@@ -1024,6 +1021,12 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
     // the last consumer of the launch leaves the control block zeroed
     if (exchange) {
         const uint32_t total_units = (uint32_t)p.total_waves;
+        // (not where a consumer has gathered, so that others are waited for under the walk: all of them count then while
+        // the last ones look at their flags; attention, 64 chains, L=1600 52.7 -> 54.9 us, 40, L=2000 44.6 -> 46.9)
+        uint32_t done = 0;
+        if (lane == 0)
+            done = __hip_atomic_fetch_add(hdr + kHdrDone, 1u, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
         done = __builtin_amdgcn_readfirstlane(done);
         if (done == 4u * total_units - 1) {
             for (uint32_t i = lane; i < 4u * total_units; i += kWave)
