@@ -241,8 +241,13 @@ int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg) {
     // Wider states the same (64 x 128 forward, 64 chains, L=4096: 116 against 104; 128 x 128
     // backward of 16 chains: 204 against 186).
     if (!force && want == 2 && total_chunks <= 128) return 0;
-    // segments of at least four chunks (one or two chains, L=4096: 32 segments 21.5 us, 16: 25.1)
-    want = std::min<int64_t>(want, total_chunks / 4);
+    // segments of at least four chunks (one or two chains, L=4096: 32 segments 21.5 us, 16: 25.1), the last one
+    // of what is left (forward, us, as many segments as there are whole fours of chunks, which makes eight of the four
+    // a segment / this way: 8 chains, L=800 20.7 / 17.9, 1 chain, L=6150 24.8 / 19.9; backward of 4, L=1600 31 / 24).
+    // Not where that were more than 192 workgroups of 64 x 64, which wait for each other longer than
+    // they walk: 101 chunks, 208 of them 25.0 us and 104 24.8, 234 26.5 and 117 25.9, but 156 22.5 and 78 24.1.
+    const int64_t fours = (total_chunks + 3) / 4;
+    want = std::min<int64_t>(want, wide || units * fours <= 192 ? fours : total_chunks / 4);
     if (tuning().tpx_segs >= 0) want = std::max(1, tuning().tpx_segs);  // tuning aid
     if (want < 2) return 0;
     const int64_t seg_chunks = ((total_chunks + want - 1) / want + kTpAhead - 1) / kTpAhead * kTpAhead;

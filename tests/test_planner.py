@@ -371,3 +371,20 @@ def test_cuts_on_three_pieces(monkeypatch):
         monkeypatch.delenv("FTC_TPH")
         _native.load().ftc_tuning_reload()
 
+
+
+@pytest.mark.parametrize("chunks", list(range(24, 60)) + [101, 193])
+@pytest.mark.parametrize("heads", [3, 8])
+def test_segments_of_few_chains_have_four_chunks(chunks, heads):
+    """An exchange on few chains has a segment for every four chunks, the last one what is left, wherever that
+    is at most 192 workgroups; its workspace is what the query answers."""
+    L = 32 * chunks - 5
+    line = lines((1, heads, L, 64), (1, heads, L, 64))[0]
+    assert line.startswith("scan_tph_kernel (exchange): 1 scan")
+    segments, rows = (int(field(line, p)) for p in (r"(\d+) segments of", r"segments of (\d+) rows"))
+    fours = -(-chunks // 4)
+    if heads * fours <= 192:
+        assert (segments, rows) == (fours, 128)
+    assert (segments - 1) * rows < L <= segments * rows
+    need = int(field(line, r"workspace (\d+) bytes"))
+    assert 0 < need <= _native.load().ftc_causal_dot_product_workspace_bytes(1, heads, L, 64, 64, 0)
