@@ -818,7 +818,11 @@ int64_t fused_tp_state_rows(int64_t D) { return (D + 63) / 64 * 64 + 64; }
 // chunks, 20 chains 0.96, 16 chains 1.00; 24 chunks, 20 chains 0.97, 16 chains 1.00; 32 chunks, 36 chains 0.93, 32 (there
 // and below with an exchange) 0.98; 36 chunks, 40 chains 0.92; 42 chunks, 40 chains 0.95, 36 chains 1.00; 48 chunks,
 // 36 chains 0.93, 28 chains 0.97; 64 chunks, 24 chains 0.91, 20 chains 0.98; far from them 64 chains, 10, 24, 42
-// and 64 chunks 0.54, 0.68, 0.80 and 0.85.  64 x 32: 16 chunks, 8 chains 0.89; 24 chunks, 40 chains 0.84; 32 chunks,
+// and 64 chunks 0.54, 0.68, 0.80 and 0.85.  With an exchange up to 6 chains from 28 chunks on, up to 12 from
+// 37, where the workgroup form's segments grow (us, workgroup form / this way: 3 chains, 28 chunks 21.5 / 20.2, 4, 50
+// chunks 27.3 / 21.6, 1, 101 chunks 30.2 / 22.9, 256 chunks 37.6 / 25.4; 8, 37 chunks 25.1 / 21.7, 128 chunks
+// 36.7 / 32.7; 12, 50 chunks 29.9 / 25.1; but 3 to 8 chains, 25 chunks 19.3 / 20.0); 8 chains, 22.5 / 21.1 at 32
+// chunks, and 16, 23.5 / 22.3 at 28 and 41.7 / 39.3 at 128, stay.  64 x 32: 16 chunks, 8 chains 0.89; 24 chunks, 40 chains 0.84; 32 chunks,
 // 40 chains 0.95; 40 chunks, 56 chains 0.90, 48 chains 0.96; 48 chunks, 80 chains 0.89, 64 chains 1.02.  32 x 64: 10
 // chunks, 16 chains 0.94, 8 chains 1.00; 16 chunks, 24 chains 0.96, 16 chains 1.06; 24 chunks, 40 chains 0.91, 32
 // chains 1.11; 32 chunks, 56 chains 0.94, 48 chains 1.00; 40 chunks, 64 chains 0.93; 48 chunks, 80 chains 0.92, 64 chains
@@ -858,7 +862,7 @@ bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, i
                 : chunks <= 32 ? 56
                 : chunks <= 44 ? 64
                                : 80;
-    const bool take = *seg_chunks > 0 ? square && chains >= (chunks >= 64 ? 24 : 36) && chunks >= 44
+    const bool take = *seg_chunks > 0 ? square && (chains <= 6 ? chunks >= 28 : chains <= 12 ? chunks >= 37 : chains >= (chunks >= 64 ? 24 : 36) && chunks >= 44)
                                       : (square || ((D == 64 || F == 64) && chains <= 256 && chunks <= 60)) && chains >= least;
     if (!take) *nseg = *seg_chunks = 0;
     return take;

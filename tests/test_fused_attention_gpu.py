@@ -909,3 +909,21 @@ def test_forward_and_backward_replay_in_a_graph(lib):
         for name, got, ref in zip(("out", "dq", "dk", "dv"), [out] + grads, want):
             assert torch.equal(got, ref), (replay, name)
     assert torch.isfinite(other).all()
+
+
+# few chains in an exchange: the shortest and the first longer ones on either side of its lines, a last segment of one
+# position, segments in which the keys end or that have none
+FEW_CHAINS = [((1, 865, 3, 64, 64, [865]), True), ((2, 1024, 3, 64, 64, [1024, 1]), True), ((1, 1185, 8, 64, 64, [700]), True),
+              ((1, 1000, 7, 64, 64, [1000]), False), ((3, 1590, 4, 64, 64, [1590, 33, 128]), True),
+              ((1, 2049, 1, 64, 64, [2048]), True), ((1, 1590, 13, 64, 64, [1590]), False)]
+
+
+@pytest.mark.parametrize("shape,exchanges", FEW_CHAINS, ids=lambda s: "n%d_l%d_h%d" % s[:3] if isinstance(s, tuple) else "")
+def test_few_chains_exchange_their_segment_sums(lib, shape, exchanges):
+    N, L, H, E, M, lens = shape
+    q, k, v = inputs(N, L, H, E, M, seed=270 + L)
+    lengths = torch.tensor(lens)
+    for _ in range(2):   # (the control block is left as it was found)
+        out = fused(lib, q.cuda(), k.cuda(), v.cuda(), lengths.cuda(), 1e-6)
+        assert lib.ftc_last_kernel() == (b"scan_tp_kernel<NORM> (exchange)" if exchanges else b"scan_wg_kernel<NORM>")
+        gate(out.cpu(), q, k, v, lengths, 1e-6)
