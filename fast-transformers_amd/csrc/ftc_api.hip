@@ -180,6 +180,35 @@ void launch_pad_rows(void *strided, int64_t sn, int64_t sh, int64_t sl, int64_t 
                            (uint16_t *)strided, sn, sh, sl, H, L, Lp, N * H, w, wp, (uint16_t *)dense);
 }
 
+// Several operands into dense rows in one launch, blockIdx.z of them.  Bound by memory (9 x 11 chains, L=1531, rows of 25, 25
+// and 33 into rows of 28, 28 and 36: 106 MB in 18 us); a launch for each leaves the card to its own last workgroups.
+template <typename T>
+struct PadList {
+    struct Item {
+        const T *strided;
+        T *dense;
+        int64_t sn, sh, sl;
+        int32_t w, wp;
+    } item[4 * kMfmaMaxScans];
+};
+template <typename T>
+__global__ __launch_bounds__(256) void pad_rows_of_several_kernel(PadList<T> list, int64_t H, int64_t L, int64_t chains) {
+    constexpr int PER = 16 / sizeof(T);
+    typedef T Vec __attribute__((ext_vector_type(PER)));
+    const typename PadList<T>::Item &o = list.item[blockIdx.z];
+    const uint32_t groups = (uint32_t)o.wp / PER;
+    const uint32_t j = blockIdx.x * 256u + threadIdx.x;
+    if (j >= (uint32_t)L * groups) return;
+    const uint32_t l = j / groups, c0 = (j % groups) * PER;
+    for (int64_t chain = blockIdx.y; chain < chains; chain += gridDim.y) {
+        const T *row = o.strided + (chain / H) * o.sn + (chain % H) * o.sh + (int64_t)l * o.sl;
+        Vec x;
+#pragma unroll
+        for (int e = 0; e < PER; e++) x[e] = (int)(c0 + e) < o.w ? row[c0 + e] : (T)0;
+        *(Vec *)(o.dense + (chain * L + l) * o.wp + c0) = x;
+    }
+}
+
 // The same between bf16 rows of the caller and fp32 dense rows (bf16 operands of a scan that
 // only the fp32 kernels take: exact on the way in, rounded to nearest even on the way out).
 template <bool PAD>
@@ -354,6 +383,61 @@ int64_t padded_scan_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, 
 int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, void *workspace,
               size_t workspace_bytes, hipStream_t stream, bool may_pad);
 
+// Whether rows of two tensors may share memory (unit stride along a row): the ranges from first to last byte
+// meet, and the rows do not lie side by side either, as the parts of a packed buffer's rows do
+bool may_overlap(const Operand &x, const OperandOut &y, const Dims &d) {
+    auto extent = [&](int64_t sn, int64_t sh, int64_t sl, int64_t width) {
+        return ((d.N - 1) * sn + (d.H - 1) * sh + (d.L - 1) * sl + width) * 4;
+    };
+    const char *xp = (const char *)x.ptr, *yp = (const char *)y.ptr;
+    if (yp >= xp + extent(x.stride_n, x.stride_h, x.stride_l, x.width) ||
+        xp >= yp + extent(y.stride_n, y.stride_h, y.stride_l, y.width))
+        return false;
+    int64_t pitch = 0;  // every row starts at a multiple of it from its tensor's first
+    if (d.N > 1) pitch = std::gcd(pitch, std::gcd(x.stride_n, y.stride_n));
+    if (d.H > 1) pitch = std::gcd(pitch, std::gcd(x.stride_h, y.stride_h));
+    if (d.L > 1) pitch = std::gcd(pitch, std::gcd(x.stride_l, y.stride_l));
+    if (pitch == 0) return true;
+    const int64_t apart = ((yp - xp) % (pitch * 4) + pitch * 4) % (pitch * 4);
+    return apart < (int64_t)x.width * 4 || apart + (int64_t)y.width * 4 > pitch * 4;
+}
+
+// Whether the copies of the scans `take` reach to a multiple of four values only, and their results go where they belong
+// at once: fp32 scans of one state shape whose copies would go to scan_dma_kernel, which then clips its
+// tiles (CLIP).  It moves 221 MB where copies of whole tiles and of the result make it 362 (backward, 25 x 33, 99 chains, L=1531,
+// dV with its copies 81 -> 59 us); results are equal bit for bit.  (Not 32 x 32, which may go elsewhere, and with states handed in or
+// out, whose copies are whole.)
+bool clipped_copies(const ScanDesc *scans, int n, const bool *take, int64_t N, int64_t H, int64_t L) {
+    ScanDesc group[kMfmaMaxScans];
+    int ngroup = 0;
+    int64_t D = 0, F = 0;
+    for (int i = 0; i < n; i++) {
+        if (!take[i]) continue;
+        ScanDesc sc = scans[i];
+        if (ngroup == 0) D = padded_rows(sc.a.width), F = round_up(sc.v.width, 32);
+        if (padded_rows(sc.a.width) != D || round_up(sc.v.width, 32) != F || sc.initial.ptr || sc.final_.ptr) return false;
+        // (as copies of whole tiles: what run_scans would do with them)
+        Operand *in[3] = {&sc.a, &sc.b, &sc.v};
+        for (int k = 0; k < 3; k++) {
+            const int64_t w = k == 2 ? F : D;
+            if (in[k]->dtype != FTC_F32) return false;
+            const bool stays = in[k]->width == w && mfma_operand_in_place(in[k]->ptr, in[k]->stride_n, in[k]->stride_h,
+                                                                          in[k]->stride_l, FTC_F32, (int)w, L);
+            for (int j = 0; j < n && stays && !plan_only(); j++)  // (a copy may lie anywhere)
+                if (take[j] && may_overlap(*in[k], scans[j].out, Dims{N, H, L, D, F})) return false;
+            if (!stays) *in[k] = Operand{nullptr, H * L * w, L * w, w, FTC_F32, (int32_t)w};
+        }
+        const OperandOut &o = scans[i].out;
+        if (o.dtype != FTC_F32 || (uintptr_t)o.ptr % 4 || (L > 1 && (o.stride_l < o.width || o.stride_l > (1 << 16))) ||
+            (L + 64) * std::max<int64_t>(o.stride_l, 128) * 4 >= 0x7fffffffLL)
+            return false;
+        sc.out = OperandOut{nullptr, H * L * F, L * F, F, FTC_F32, (int32_t)F};
+        group[ngroup++] = sc;
+    }
+    if (ngroup == 0 || D > 64 || (D == 32 && F == 32) || !mfma_scan_clips(D, F, ngroup, L)) return false;
+    return !short_scans_take(group, ngroup, N, H, L) && !mfma_tp_takes(group, ngroup, N, H, L);
+}
+
 // The scans of a call that the matrix-core kernels do not take as they are, run on padded
 // copies: `take[i]` says which.  An operand that several scans read is copied once; an
 // operand whose rows are fine where they lie is used in place.  Returns with *done = false
@@ -396,6 +480,7 @@ int padded_scans(const ScanDesc *scans, int n, const bool *take, int64_t N, int6
     StateCopy states[2 * kMfmaMaxScans];
     int nstates = 0;
     int which[kMfmaMaxScans][4];
+    const bool clipped = clipped_copies(scans, n, take, N, H, L);
     for (int i = 0; i < n; i++) {
         if (!take[i]) continue;
         const ScanDesc &sc = scans[i];
@@ -421,13 +506,13 @@ int padded_scans(const ScanDesc *scans, int n, const bool *take, int64_t N, int6
                                                             o.dtype, o.width, L)
                                   ? -1
                                   : copy_of(o.ptr, o.stride_n, o.stride_h, o.stride_l, o.dtype, o.width,
-                                            target[k], false, dd);
+                                            clipped ? (int)round_up(o.width, 4) : target[k], false, dd);
         }
         const OperandOut &o = sc.out;
         const int dd = to_f32 ? FTC_F32 : o.dtype;
-        which[nwork][3] = o.width == Fp && dd == o.dtype &&
+        which[nwork][3] = clipped || (o.width == Fp && dd == o.dtype &&
                                   mfma_operand_in_place(o.ptr, o.stride_n, o.stride_h, o.stride_l, o.dtype,
-                                                        o.width, L)
+                                                        o.width, L))
                               ? -1
                               : copy_of(o.ptr, o.stride_n, o.stride_h, o.stride_l, o.dtype, o.width, Fp, true, dd);
         work[nwork++] = sc;
@@ -461,7 +546,8 @@ int padded_scans(const ScanDesc *scans, int n, const bool *take, int64_t N, int6
             if (which[s][k] >= 0) {
                 const Copy &c = copies[which[s][k]];
                 const int64_t w = c.padded;
-                *in[k] = Operand{c.dense, H * L * w, L * w, w, c.dense_dtype, (int32_t)w};
+                // (clipped: the width that the rows have, the one that they lie apart)
+                *in[k] = Operand{c.dense, H * L * w, L * w, w, c.dense_dtype, (int32_t)(clipped ? c.width : w)};
             }
         if (which[s][3] >= 0) {
             const Copy &c = copies[which[s][3]];
@@ -476,17 +562,30 @@ int padded_scans(const ScanDesc *scans, int n, const bool *take, int64_t N, int6
                   "back, workspace %lld bytes", nin, nin == 1 ? "" : "s", nout, nout == 1 ? "" : "s",
                   (long long)need);
     } else {
+        PadList<uint32_t> words;
+        PadList<uint16_t> halves;
+        int nwords = 0, nhalves = 0, most_words = 0, most_halves = 0;
         for (int i = 0; i < ncopies; i++) {
-            if (copies[i].is_output) continue;
-            if (copies[i].dense_dtype != copies[i].dtype)
-                launch_pad_rows_bf16<true>((void *)copies[i].ptr, copies[i].sn, copies[i].sh, copies[i].sl,
-                                           N, H, L, copies[i].width, copies[i].padded, copies[i].dense,
-                                           stream);
+            const Copy &c = copies[i];
+            if (c.is_output) continue;
+            if (c.dense_dtype != c.dtype)
+                launch_pad_rows_bf16<true>((void *)c.ptr, c.sn, c.sh, c.sl, N, H, L, c.width, c.padded, c.dense, stream);
+            else if (esz(c.dtype) == 4)
+                words.item[nwords++] = {(const uint32_t *)c.ptr, (uint32_t *)c.dense, c.sn, c.sh, c.sl, c.width, c.padded},
+                most_words = std::max(most_words, c.padded);
             else
-                launch_pad_rows<true>((void *)copies[i].ptr, copies[i].sn, copies[i].sh, copies[i].sl,
-                                      N, H, L, copies[i].width, copies[i].padded,
-                                      esz(copies[i].dtype), copies[i].dense, stream);
+                halves.item[nhalves++] = {(const uint16_t *)c.ptr, (uint16_t *)c.dense, c.sn, c.sh, c.sl, c.width, c.padded},
+                most_halves = std::max(most_halves, c.padded);
         }
+        auto grid = [&](int most, int per, int count) {
+            return dim3((unsigned)((L * (most / per) + 255) / 256), (unsigned)std::min<int64_t>(N * H, 65535), (unsigned)count);
+        };
+        if (nwords > 0)
+            hipLaunchKernelGGL(pad_rows_of_several_kernel<uint32_t>, grid(most_words, 4, nwords), dim3(256), 0, stream,
+                               words, H, L, N * H);
+        if (nhalves > 0)
+            hipLaunchKernelGGL(pad_rows_of_several_kernel<uint16_t>, grid(most_halves, 8, nhalves), dim3(256), 0, stream,
+                               halves, H, L, N * H);
         for (int i = 0; i < nstates; i++) {
             const StateCopy &st = states[i];
             if (st.is_output) continue;
@@ -497,7 +596,9 @@ int padded_scans(const ScanDesc *scans, int n, const bool *take, int64_t N, int6
                                   N, H, st.D, st.F, st.Fp, 4, st.dense, stream, st.Dp);
         }
     }
-    int rc = run_scans(work, nwork, N, H, L, workspace, (size_t)ws_scan, stream, false);
+    int rc = clipped ? mfma_scan(work, nwork, N, H, L, workspace, (size_t)ws_scan, stream, nullptr, false, false, false,
+                                 nullptr, true)
+                     : run_scans(work, nwork, N, H, L, workspace, (size_t)ws_scan, stream, false);
     if (rc) return rc;
     if (!plan_only()) {
         for (int i = 0; i < ncopies; i++) {
@@ -1377,25 +1478,6 @@ static int64_t attention_gradients_layout(int64_t N, int64_t H, int64_t L, int n
                                    FTC_WORKSPACE_CONTROL_BYTES);
     for (int64_t &o : offset) o = at, at += round_up(N * H * L * 4, 256);
     return at;
-}
-
-// Whether rows of two tensors may share memory (unit stride along a row): the ranges from first to last byte
-// meet, and the rows do not lie side by side either, as the parts of a packed buffer's rows do
-static bool may_overlap(const Operand &x, const OperandOut &y, const Dims &d) {
-    auto extent = [&](int64_t sn, int64_t sh, int64_t sl, int64_t width) {
-        return ((d.N - 1) * sn + (d.H - 1) * sh + (d.L - 1) * sl + width) * 4;
-    };
-    const char *xp = (const char *)x.ptr, *yp = (const char *)y.ptr;
-    if (yp >= xp + extent(x.stride_n, x.stride_h, x.stride_l, x.width) ||
-        xp >= yp + extent(y.stride_n, y.stride_h, y.stride_l, y.width))
-        return false;
-    int64_t pitch = 0;  // every row starts at a multiple of it from its tensor's first
-    if (d.N > 1) pitch = std::gcd(pitch, std::gcd(x.stride_n, y.stride_n));
-    if (d.H > 1) pitch = std::gcd(pitch, std::gcd(x.stride_h, y.stride_h));
-    if (d.L > 1) pitch = std::gcd(pitch, std::gcd(x.stride_l, y.stride_l));
-    if (pitch == 0) return true;
-    const int64_t apart = ((yp - xp) % (pitch * 4) + pitch * 4) % (pitch * 4);
-    return apart < (int64_t)x.width * 4 || apart + (int64_t)y.width * 4 > pitch * 4;
 }
 
 static int64_t attention_backward_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t E, int64_t M,

@@ -183,7 +183,12 @@ int64_t attention_gradients_workspace_bytes(int64_t N, int64_t H, int64_t L, int
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
               void *workspace, size_t workspace_bytes, hipStream_t stream,
               const FusedAttention *fused = nullptr, bool may_chain_parallel = true,
-              bool forced = false, bool odd = false, const AttentionGradients *grads = nullptr);
+              bool forced = false, bool odd = false, const AttentionGradients *grads = nullptr,
+              bool clipped = false);
+// Whether `nscans` fp32 scans of a D x F state (whole tiles) that the chain-parallel kernels leave run on the
+// kernel that takes rows which do not fill the tiles (`clipped`: rows of a, b and v with zeros up to a
+// multiple of four values, of the result of any width on 4-byte boundaries).
+bool mfma_scan_clips(int64_t D, int64_t F, int nscans, int64_t L);
 
 // Chains of a few positions (ftc_short.hip): scans of any widths and element types in one launch,
 // on the vector unit, without a workspace.

@@ -698,6 +698,11 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
     return seg_chunks > 0 ? tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D) : 0;
 }
 
+bool mfma_scan_clips(int64_t D, int64_t F, int nscans, int64_t L) {
+    int widths[kMfmaMaxSlices];
+    return D <= 64 && mfma_slice_widths(D, F, widths) == 1 && tuning().dma != 0 && !use_wg_kernel(D, F, nscans, L, true);
+}
+
 // the widest rows of a launch (they differ between scans only where `odd` allows it)
 void widest_rows(const ScanDesc *scans, int nscans, int *D, int *F) {
     *D = *F = 0;
@@ -913,10 +918,12 @@ int64_t attention_gradients_workspace_bytes(int64_t N, int64_t H, int64_t L, int
 int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L,
               void *workspace, size_t workspace_bytes, hipStream_t stream,
               const FusedAttention *fused, bool may_chain_parallel, bool forced, bool odd,
-              const AttentionGradients *grads) {
+              const AttentionGradients *grads, bool clipped) {
     if (nscans < 1 || nscans > kMaxScans) return fail(FTC_ERR_INVALID, "bad scan count");
     int D, F;
     widest_rows(scans, nscans, &D, &F);
+    auto tiles = [clipped](int width) { return clipped ? (width + 31) / 32 * 32 : width; };
+    D = tiles(D), F = tiles(F);
     const Combo combo = combo_of(scans[0]);
     if (fused && (nscans != 1 || !fused_attention_supported(scans[0], L)))
         return fail(FTC_ERR_UNSUPPORTED, "no fused attention kernel for this shape or layout");
@@ -951,9 +958,9 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
         if (tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     }
     const bool tp = tp_nseg > 0 || tpx_seg_chunks > 0;
-    if (!tp && !mfma_scan_supported(scans[0], L))
+    if (clipped ? tp || !mfma_scan_clips(D, F, nscans, L) : !tp && !mfma_scan_supported(scans[0], L))
         return fail(FTC_ERR_UNSUPPORTED, "no MFMA kernel takes a %d x %d state here", D, F);
-    const bool wg = !fused_tp && (fused || use_wg_kernel(D, F, nscans, L, combo == kFFFF));
+    const bool wg = !fused_tp && !clipped && (fused || use_wg_kernel(D, F, nscans, L, combo == kFFFF));
     MfmaPlan pl = wide_rows ? MfmaPlan{} : make_plan(N, H, L, D, F, nscans, wg, fused != nullptr);
     int32_t tp_start[kMaxTpSegments + 1] = {0};
     if (tpx_seg_chunks > 0) {  // one workgroup per chain segment, segment sums exchanged
@@ -1057,7 +1064,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     for (int i = 0; i < nscans; i++) {
         mixed = mixed || combo_of(scans[i]) != kFFFF;
         if ((!rows_as_they_are && combo_of(scans[i]) != combo) ||
-            (!(tp && odd) && (scans[i].a.width != D || scans[i].v.width != F)))
+            (!(tp && odd) && (tiles(scans[i].a.width) != D || tiles(scans[i].v.width) != F)))
             return fail(FTC_ERR_INVALID, "scans of one launch must share widths and dtypes");
     }
     // fp32 states of up to 64 rows: the kernel that feeds its fragments from LDS tiles
@@ -1097,7 +1104,7 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     } else if (wg) {
         launch_scan_wg_ffff(D, F, fused != nullptr, workspace, args, stream);
     } else if (dma) {
-        launch_scan_dma_ffff(D, F, workspace, args, stream);
+        launch_scan_dma_ffff(D, F, workspace, args, stream, clipped);
     } else switch (combo) {
         case kFFFF: launch_scan_ffff(D, F, workspace, args, stream); break;
         case kBBBF: launch_scan_bbbf(D, F, workspace, args, stream); break;

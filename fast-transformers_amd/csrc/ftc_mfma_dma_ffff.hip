@@ -5,7 +5,8 @@
 namespace ftc {
 namespace mfma {
 #define FTC_INSTANTIATE(DD, FF) \
-    template __global__ void scan_dma_kernel<DD, FF, float, float, float, float>(uint32_t *, ScanArgs)
+    template __global__ void scan_dma_kernel<DD, FF, float, float, float, float, false>(uint32_t *, ScanArgs); \
+    template __global__ void scan_dma_kernel<DD, FF, float, float, float, float, true>(uint32_t *, ScanArgs)
 FTC_INSTANTIATE(64, 64);
 FTC_INSTANTIATE(32, 128);
 FTC_INSTANTIATE(32, 32);
@@ -13,8 +14,9 @@ FTC_INSTANTIATE(32, 64);
 FTC_INSTANTIATE(64, 32);
 #undef FTC_INSTANTIATE
 
-void launch_scan_dma_ffff(int D, int F, void *ws, const ScanArgs &args, hipStream_t stream) {
-    launch_scan_dma<float, float, float, float>(D, F, ws, args, stream);
+void launch_scan_dma_ffff(int D, int F, void *ws, const ScanArgs &args, hipStream_t stream, bool clipped) {
+    if (clipped) launch_scan_dma_clipped<float>(D, F, ws, args, stream);
+    else launch_scan_dma<float, float, float, float>(D, F, ws, args, stream);
 }
 }  // namespace mfma
 }  // namespace ftc

@@ -51,17 +51,18 @@ struct Swizzle {
     }
 };
 
-// Requests for one tile: kLoads instructions, lane offsets prepared once.
+// Requests for one tile: kLoads instructions, lane offsets prepared once.  (`own`: bytes of a row; what of a
+// tile's row lies beyond is asked for outside the descriptor and reads as zero)
 template <int RB>
 struct TileRequest {
     static constexpr int kLoads = kChunk * RB / (kWave * 16);
     uint32_t lane_off[kLoads];
-    __device__ __forceinline__ void prepare(int lane, uint32_t row_stride_bytes) {
+    __device__ __forceinline__ void prepare(int lane, uint32_t row_stride_bytes, uint32_t own = RB) {
 #pragma unroll
         for (int i = 0; i < kLoads; i++) {
             int row, piece;
             Swizzle<RB>::slot(i * kWave + lane, row, piece);
-            lane_off[i] = (uint32_t)row * row_stride_bytes + 16u * (uint32_t)piece;
+            lane_off[i] = (uint32_t)row * row_stride_bytes + (16u * (uint32_t)piece < own ? 16u * (uint32_t)piece : 0x80000000u);
         }
     }
     // rows row0 .. row0 + 31 of the segment -> tile
@@ -105,7 +106,10 @@ __device__ __forceinline__ void lds_column_to_frags(const lds_char *tile, const 
     for (int q = 0; q < 4; q++) f[0].w[q] = x[2 * q] | (x[2 * q + 1] << 16);
 }
 
-template <int D, int F, typename TA, typename TB, typename TV, typename TO>
+// CLIP: fp32 rows that do not fill the tiles: those of a, b and v end on a multiple of four values (of which the
+// last ones are zero), the result's anywhere, on 4-byte boundaries.  Zero columns change nothing, so
+// that a copy of odd rows need not reach to the tile's width, and the result needs none.
+template <int D, int F, typename TA, typename TB, typename TV, typename TO, bool CLIP = false>
 __global__ __launch_bounds__(kWave) void scan_dma_kernel(uint32_t *__restrict__ ws_ptr,
                                                          ScanArgs p) {
     constexpr int NSA = Elem<TA>::kPieces, NSB = Elem<TB>::kPieces, NSV = Elem<TV>::kPieces;
@@ -135,9 +139,12 @@ __global__ __launch_bounds__(kWave) void scan_dma_kernel(uint32_t *__restrict__ 
     TileRequest<RBA> a_req;
     TileRequest<RBB> b_req;
     TileRequest<RBV> v_req;
-    a_req.prepare(lane, a_slb);
-    b_req.prepare(lane, b_slb);
-    v_req.prepare(lane, v_slb);
+    static_assert(!CLIP || (BA == 4 && BB == 4 && BV == 4 && BO == 4), "fp32 rows");
+    const uint32_t own_ab = CLIP ? 16u * (uint32_t)((op.d + 3) / 4) : 0u, own_v = CLIP ? 16u * (uint32_t)((op.f + 3) / 4) : 0u;
+    const uint32_t a_bytes = CLIP ? own_ab : RBA, b_bytes = CLIP ? own_ab : RBB, v_bytes = CLIP ? own_v : RBV;
+    a_req.prepare(lane, a_slb, a_bytes);
+    b_req.prepare(lane, b_slb, b_bytes);
+    v_req.prepare(lane, v_slb, v_bytes);
 
     // per-lane tile addresses
     //  row-major fragments: lane (row = ln, g), k-step ks: elements 16*ks + 4*g + 0..3, + 8
@@ -187,13 +194,13 @@ __global__ __launch_bounds__(kWave) void scan_dma_kernel(uint32_t *__restrict__ 
         (const char *)op.v + ((int64_t)n * op.v_sn + (int64_t)h * op.v_sh + lo * op.v_sl) * BV;
     char *o_seg = (char *)op.out + ((int64_t)n * op.o_sn + (int64_t)h * op.o_sh + lo * op.o_sl) * BO;
     const __amdgpu_buffer_rsrc_t a_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)a_seg, 0, (rows - 1) * a_slb + RBA, kRsrcFlags);
+        (void *)a_seg, 0, (rows - 1) * a_slb + a_bytes, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t b_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)b_seg, 0, (rows - 1) * b_slb + RBB, kRsrcFlags);
+        (void *)b_seg, 0, (rows - 1) * b_slb + b_bytes, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t v_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)v_seg, 0, (rows - 1) * v_slb + RBV, kRsrcFlags);
+        (void *)v_seg, 0, (rows - 1) * v_slb + v_bytes, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t o_rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)o_seg, 0, (rows - 1) * o_slb + F * BO, kRsrcFlags);
+        (void *)o_seg, 0, (rows - 1) * o_slb + (CLIP ? op.f : F) * BO, kRsrcFlags);
     const uint32_t o_lane = ln * o_slb + 4u * BO * g;
 
     auto chunk_row0 = [&](int c) -> int { return REV ? rows - kChunk * (c + 1) : kChunk * c; };
@@ -372,10 +379,21 @@ __global__ __launch_bounds__(kWave) void scan_dma_kernel(uint32_t *__restrict__ 
 #pragma unroll
         for (int ft = 0; ft < FT; ft++)
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                buffer_store_out(o_rs, o_off + (uint32_t)(BO * (32 * ft + 8 * q)), O[ft][4 * q + 0],
-                                 O[ft][4 * q + 1], O[ft][4 * q + 2], O[ft][4 * q + 3],
-                                 (TO *)nullptr);
+            for (int q = 0; q < 4; q++) {
+                const int left = CLIP ? op.f - (32 * ft + 8 * q) : 0;  // columns from this pair of quads on
+                if (CLIP && left <= 0) continue;
+                const uint32_t at = o_off + (uint32_t)(BO * (32 * ft + 8 * q));
+                const bool whole = !CLIP || left >= 4 * g + 4;
+                buffer_store_out(o_rs, whole ? at : 0x80000000u, O[ft][4 * q + 0], O[ft][4 * q + 1], O[ft][4 * q + 2],
+                                 O[ft][4 * q + 3], (TO *)nullptr);
+                if (CLIP && left < 8 && left % 4 != 0) {  // (a quad that ends inside the row, word by word)
+                    const int own = whole ? 0 : left - 4 * g;
+#pragma unroll
+                    for (int e = 0; e < 3; e++)
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(O[ft][4 * q + e]), o_rs,
+                                                              e < own ? at + 4u * e : 0x80000000u, 0, 0);
+                }
+            }
 
         // (3): b by column; this b tile then takes the chunk after next
         Frag bt_frag[DT][2][NSB];
@@ -417,9 +435,24 @@ void launch_scan_dma(int D, int F, void *workspace, const ScanArgs &args, hipStr
 #undef FTC_LAUNCH
 }
 
+// the same with rows that do not fill the tiles (CLIP)
+template <typename T>
+void launch_scan_dma_clipped(int D, int F, void *workspace, const ScanArgs &args, hipStream_t stream) {
+    const dim3 grid((unsigned)args.total_waves), block(kWave);
+#define FTC_LAUNCH(DD, FF)                                                                      \
+    hipLaunchKernelGGL((scan_dma_kernel<DD, FF, T, T, T, T, true>), grid, block, 0, stream,     \
+                       (uint32_t *)workspace, args)
+    if (D == 64 && F == 64) FTC_LAUNCH(64, 64);
+    else if (D == 32 && F == 128) FTC_LAUNCH(32, 128);
+    else if (D == 32 && F == 32) FTC_LAUNCH(32, 32);
+    else if (D == 32 && F == 64) FTC_LAUNCH(32, 64);
+    else FTC_LAUNCH(64, 32);
+#undef FTC_LAUNCH
+}
+
 // Instantiated for all-fp32 scans (ftc_mfma_dma_ffff.hip); with bf16 rows, which need no
 // piece split, the register-fed kernel measured as fast or faster.
-void launch_scan_dma_ffff(int D, int F, void *ws, const ScanArgs &args, hipStream_t stream);
+void launch_scan_dma_ffff(int D, int F, void *ws, const ScanArgs &args, hipStream_t stream, bool clipped);
 
 }  // namespace mfma
 }  // namespace ftc

@@ -268,3 +268,47 @@ def test_narrow_scans_share_a_launch(shape):
     alone = torch.empty_like(q)
     cp.causal_dot_backward_hip(q, k, v, g, None, alone, None)
     assert scale_error(alone.cpu(), exact[2]) <= max(4 * scale_error(want[2], exact[2]), 2e-6)
+
+
+CLIPPED = [
+    # N, H, L, E, M, backward: tiles that rows do not fill, of each state shape; widths one, two and three values into a
+    # quad, on it, and the narrowest; ends of chains inside a chunk, chains of a chunk and some; one launch of
+    # two scans, a call whose other scans run where their rows lie, operands that need no copy
+    (9, 11, 1531, 25, 33, True), (16, 21, 413, 9, 34, True), (3, 20, 1000, 45, 31, True), (2, 3, 97, 27, 63, True),
+    (1, 4, 5000, 33, 32, False), (1, 2, 800, 32, 127, False), (30, 20, 70, 64, 35, False), (1, 3, 2000, 31, 64, False),
+    (30, 20, 70, 62, 64, True),
+]
+
+
+@pytest.mark.parametrize("shape", CLIPPED, ids=lambda s: "n%d_h%d_l%d_e%d_m%d_%s" % (s[:5] + ("bwd" if s[5] else "fwd",)))
+def test_results_of_copies_go_where_they_belong(shape):
+    """Scans on copies whose kernel splits L store odd rows themselves: the oracle's values, and nothing around them."""
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M, backward = shape
+    plan = _native.plan((N, H, L, E), (N, H, L, M), backward=backward)
+    if shape[:2] != (2, 3):   # (rows too few for copies)
+        assert "scan_dma_kernel" in plan and ", 0 results copied back" in plan, plan
+    Q, K, V, G = oracle.make_inputs(N, H, L, E, M, seed=700 + L)
+
+    def boxed(X):   # rows of odd strides, on 4-byte boundaries, among other values
+        box = torch.full((N, H, L + 1, X + 3), 7.0, device="cuda")
+        box[:, :, :L, 1:1 + X] = float("nan")
+        return box, box[:, :, :L, 1:1 + X]
+
+    q, k, v, g = (t.cuda() for t in (Q, K, V, G))
+    if backward:
+        boxes = [boxed(X) for X in (E, E, M)]
+        for _ in range(2):
+            cp.causal_dot_backward_hip(q, k, v, g, *(o for _, o in boxes))
+        exact = oracle.backward(*(t.double() for t in (Q, K, V, G)))
+        ref = oracle.backward(Q, K, V, G)
+    else:
+        boxes = [boxed(M)]
+        for _ in range(2):
+            cp.causal_dot_product_hip(q, k, v, boxes[0][1])
+        exact, ref = [oracle.forward(*(t.double() for t in (Q, K, V)))], [oracle.forward(Q, K, V)]
+    for (box, out), want, plain in zip(boxes, exact, ref):
+        assert scale_error(out.cpu(), want) <= max(4 * scale_error(plain, want), 2e-6)
+        box[:, :, :L, 1:-2] = 7.0
+        assert (box == 7.0).all()
