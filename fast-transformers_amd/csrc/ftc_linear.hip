@@ -110,12 +110,18 @@ __global__ __launch_bounds__(256) void split_weights_kernel(WeightList list) {
 }
 
 // ---- rows: a wavefront per row, which it keeps in registers ------------------------------------
-// NORM: layer norm first (torch's: biased variance, two passes over the row in fp32)
+// a value of a layer norm's row, less the row's mean, r = 1 / sqrt(variance + eps); rounded the same wherever it is made
+__device__ __forceinline__ float normed(float less_mean, float r, float gamma, float beta) {
+    return __builtin_fmaf(less_mean * r, gamma, beta);
+}
+// NORM: layer norm first (torch's: biased variance, two passes over the row in fp32).  Its rows go out, or only what
+// they are made of beside x, (mean, r) of each: who reads them as a residual then makes them again from x.
+// Bound by memory: 40960 rows of 512, pieces and rows 40.3 us, pieces and (mean, r) 29.7.
 constexpr int kMostQuads = 16;           // quads of a row per lane: rows of up to 4096 values
 template <int QUADS, bool NORM>
 __global__ __launch_bounds__(256) void rows_kernel(const float *__restrict__ x, const float *__restrict__ gamma,
                                                    const float *__restrict__ beta, float eps, int64_t rows,
-                                                   int cols, float *__restrict__ out,
+                                                   int cols, float *__restrict__ out, float2 *__restrict__ stats,
                                                    char *__restrict__ pieces, float *__restrict__ scale) {
     const int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
     const int lane = threadIdx.x % 64;
@@ -145,10 +151,11 @@ __global__ __launch_bounds__(256) void rows_kernel(const float *__restrict__ x, 
             if (c >= cols) continue;
             const float4 g = gamma ? *(const float4 *)(gamma + c) : make_float4(1.f, 1.f, 1.f, 1.f);
             const float4 b = beta ? *(const float4 *)(beta + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-            v[i].x = v[i].x * r * g.x + b.x, v[i].y = v[i].y * r * g.y + b.y;
-            v[i].z = v[i].z * r * g.z + b.z, v[i].w = v[i].w * r * g.w + b.w;
-            *(float4 *)(out + row * cols + c) = v[i];
+            v[i].x = normed(v[i].x, r, g.x, b.x), v[i].y = normed(v[i].y, r, g.y, b.y);
+            v[i].z = normed(v[i].z, r, g.z, b.z), v[i].w = normed(v[i].w, r, g.w, b.w);
+            if (out) *(float4 *)(out + row * cols + c) = v[i];
         }
+        if (stats && lane == 0) stats[row] = make_float2(mean, r);
     }
     if (!pieces) return;
     float largest = 0.f;
@@ -197,7 +204,9 @@ __global__ __launch_bounds__(256) void cut_rows_kernel(char *rows, float *scale,
 struct LinearArgs {
     const char *x, *w;                   // rows in pieces
     const float *x_scale, *w_scale, *bias, *w_norm;
-    const float *residual;               // kResidual
+    const float *residual;               // kResidual, kNormed
+    const float2 *stats;                 // kNormed: the residual is the layer norm of those rows
+    const float *gamma, *beta;           // (or nullptr: ones, zeros)
     float *out;                          // kPlain, kResidual
     char *out_pieces;                    // kRelu
     float *out_scale;
@@ -212,7 +221,7 @@ constexpr int kStreamed = 2;             // (a store's nt bit)
 // 6266 / 6156; four at 30400 2299 / - / 2277; 1024 -> 512 at 40960 tokens 133 / 142 / 128.  From 140 MB on
 // instead, four layers at 24576 tokens take 2063 us for 1990, and from none on at 20480 1749 for 1682.
 constexpr int64_t kStreamedBytes = (int64_t)176 << 20;
-enum { kPlain = 0, kResidual = 1, kRelu = 2 };
+enum { kPlain = 0, kResidual = 1, kRelu = 2, kNormed = 3 };
 
 // a raw buffer of `bytes` bytes
 __device__ __forceinline__ u32x4 descriptor(const void *base, uint32_t bytes) {
@@ -279,7 +288,8 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
     constexpr int kScaleT = TN / 2 < 64 ? 64 : TN / 2, kScaleF = TF / 2 < 64 ? 64 : TF / 2;
     constexpr int kScales = kScaleT + 2 * kScaleF, kScaleLoads = kScales / 64;
     constexpr int kScaleSets = LATER ? 2 : 1;
-    static_assert(!LATER || (EPI != kResidual && WF > WT && kRequests <= 3 * (WF - WT)), "requests before the stores of a step");
+    constexpr bool kAdds = EPI == kResidual || EPI == kNormed;
+    static_assert(!LATER || (!kAdds && WF > WT && kRequests <= 3 * (WF - WT)), "requests before the stores of a step");
     static_assert(WF % 2 == 0 && TN / 2 <= 64, "the fragments of w in turn; a wavefront's tokens in a request");
     __shared__ __align__(16) char tiles_mem[STAGES * kBuf];
     __shared__ __align__(16) float scales_mem[kScaleSets][4][kScales];
@@ -527,7 +537,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
         for (int u = 0; u < 2; u++) {
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                if (EPI == kResidual) y[u][c] += __uint_as_float(res[u][c]);
+                if (kAdds) y[u][c] += __uint_as_float(res[u][c]);
                 if (EPI != kRelu || whole) half[u][c] = __float_as_uint(y[u][c]);
             }
         }
@@ -626,7 +636,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
                 // step's buffer.
                 const bool rows_fly = round > 0 && s < STAGES - 1 && steps >= STAGES;
                 auto wait = [&]() {
-                    constexpr int kMost = kFlying + (EPI == kResidual && decltype(last)::value ? 2 * WT : 0),
+                    constexpr int kMost = kFlying + (kAdds && decltype(last)::value ? 2 * WT + (EPI == kNormed ? WT : 0) : 0),
                                   kMore = kMost + kStores + kScaleLoads < 63 ? kMost + kStores + kScaleLoads : 63;
                     if (rows_fly)
                         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kMore) : "memory");
@@ -643,8 +653,13 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
             step(0, std::true_type{}, std::false_type{});
             for (int s = 1; s < steps - 1; s++) step(s, std::false_type{}, std::false_type{});
             const __amdgpu_buffer_rsrc_t r_rs = __builtin_amdgcn_make_buffer_rsrc(
-                (char *)(EPI == kResidual ? p.residual : p.bias) + (EPI == kResidual ? t.t0 * out_row : 0), 0,
+                (char *)(kAdds ? p.residual : p.bias) + (kAdds ? t.t0 * out_row : 0), 0,
                 (uint32_t)t.nt * out_row, kRsrcFlags);
+            const __amdgpu_buffer_rsrc_t stats_rs = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(EPI == kNormed ? (const void *)(p.stats + t.t0) : (const void *)p.bias), 0, EPI == kNormed ? (uint32_t)t.nt * 8u : 0u,
+                kRsrcFlags);
+            typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+            u32x2_t of_row[WT];              // (mean, r)
             // (residual rows a pair of feature tiles ahead, the first one under the last step: a wait for them then
             // leaves the stores in flight)
             u32x4 res[2][WT][2];
@@ -657,7 +672,13 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
                         res[pair % 2][j][u] = __builtin_amdgcn_raw_buffer_load_b128(
                             r_rs, f + 16 * u + 4 * g < p.features ? token_at(j) + 4u * f + 64u * u : 0x80000000u, 0, 0);
             };
-            if (EPI == kResidual) residual(0);
+            if (EPI == kNormed) {
+#pragma unroll
+                for (int j = 0; j < WT; j++)
+                    of_row[j] = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(
+                                                                stats_rs, 8u * (uint32_t)(wt * (TN / 2) + 16 * j + ln), 0, 0));
+            }
+            if (kAdds) residual(0);
             step(steps - 1, std::false_type{}, std::true_type{});
             // (this tile's scales: seen to have landed by the steps' waits where there are enough of them)
             if (steps <= STAGES) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -665,10 +686,28 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(LinearArgs p) {
 #pragma unroll
             for (int pair = 0; pair < WF / 2; pair++) {
                 const Features w = features_of(rows, pair);
-                if (EPI == kResidual && pair + 1 < WF / 2) residual(pair + 1);
+                if (kAdds && pair + 1 < WF / 2) residual(pair + 1);
+                if (EPI == kNormed) {
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        const int f = rows.f0 + 32 * pair + 16 * u + 4 * g;
+                        const int from = f < p.features ? f : 0;
+                        const float4 ga = p.gamma ? *(const float4 *)(p.gamma + from) : make_float4(1.f, 1.f, 1.f, 1.f);
+                        const float4 be = p.beta ? *(const float4 *)(p.beta + from) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                        for (int j = 0; j < WT; j++) {
+                            const float mean = __uint_as_float(of_row[j][0]), r = __uint_as_float(of_row[j][1]);
+                            u32x4 &v = res[pair % 2][j][u];
+                            v = u32x4{__float_as_uint(normed(__uint_as_float(v.x) - mean, r, ga.x, be.x)),
+                                      __float_as_uint(normed(__uint_as_float(v.y) - mean, r, ga.y, be.y)),
+                                      __float_as_uint(normed(__uint_as_float(v.z) - mean, r, ga.z, be.z)),
+                                      __float_as_uint(normed(__uint_as_float(v.w) - mean, r, ga.w, be.w))};
+                        }
+                    }
+                }
 #pragma unroll
                 for (int j = 0; j < WT; j++)
-                    pair_out(rows, w, pair, j, acc[2 * pair][j], acc[2 * pair + 1][j], EPI == kResidual ? res[pair % 2][j] : nullptr);
+                    pair_out(rows, w, pair, j, acc[2 * pair][j], acc[2 * pair + 1][j], kAdds ? res[pair % 2][j] : nullptr);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -703,6 +742,8 @@ void launch_product(LinearArgs a, hipStream_t stream) {
     }
     if (a.out_pieces)
         hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kRelu>), grid, block, 0, stream, a);
+    else if (a.stats)
+        hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kNormed>), grid, block, 0, stream, a);
     else if (a.residual)
         hipLaunchKernelGGL((linear_kernel<TN, TF, STAGES, kResidual>), grid, block, 0, stream, a);
     else
@@ -751,7 +792,7 @@ bool aligned(const void *p) { return (uintptr_t)p % 16 == 0; }
 
 template <bool NORM>
 int launch_rows(const float *x, const float *gamma, const float *beta, float eps, int64_t rows, int64_t cols,
-                float *out, void *pieces, float *scale, hipStream_t stream) {
+                float *out, float *stats, void *pieces, float *scale, hipStream_t stream) {
     if (cols % kStep != 0 || cols > 256 * kMostQuads)
         return fail(FTC_ERR_UNSUPPORTED, "rows of %lld values", (long long)cols);
     if (!aligned(x) || !aligned(gamma) || !aligned(beta) || !aligned(out) || !aligned(pieces))
@@ -761,7 +802,7 @@ int launch_rows(const float *x, const float *gamma, const float *beta, float eps
     const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
 #define FTC_ROWS(Q)                                                                                   \
     hipLaunchKernelGGL((rows_kernel<Q, NORM>), grid, block, 0, stream, x, gamma, beta, eps, rows, (int)cols, out, \
-                       (char *)pieces, scale)
+                       (float2 *)stats, (char *)pieces, scale)
     const int64_t quads = (cols + 255) / 256;
     if (quads <= 1) FTC_ROWS(1);
     else if (quads <= 2) FTC_ROWS(2);
@@ -802,24 +843,32 @@ int ftc_split_weights(const ftc_weight *weights, int32_t count, void *stream) {
 
 int ftc_split_rows(const float *x, int64_t rows, int64_t cols, void *pieces, float *scale, void *stream) {
     if (!x || !pieces || !scale) return fail(FTC_ERR_INVALID, "null pointer");
-    return launch_rows<false>(x, nullptr, nullptr, 0.f, rows, cols, nullptr, pieces, scale, (hipStream_t)stream);
+    return launch_rows<false>(x, nullptr, nullptr, 0.f, rows, cols, nullptr, nullptr, pieces, scale, (hipStream_t)stream);
 }
 
 int ftc_layer_norm_split(const float *x, const float *gamma, const float *beta, float eps, int64_t rows,
                          int64_t cols, float *out, void *pieces, float *scale, void *stream) {
     if (!x || !out || (pieces && !scale)) return fail(FTC_ERR_INVALID, "null pointer");
-    return launch_rows<true>(x, gamma, beta, eps, rows, cols, out, pieces, scale, (hipStream_t)stream);
+    return launch_rows<true>(x, gamma, beta, eps, rows, cols, out, nullptr, pieces, scale, (hipStream_t)stream);
 }
 
-int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
-                     const float *bias, const float *w_norm, int64_t features, int64_t k,
-                     const float *residual, float *out, void *relu_pieces, float *relu_scale, void *stream) {
+int ftc_layer_norm_stats_split(const float *x, const float *gamma, const float *beta, float eps, int64_t rows,
+                               int64_t cols, float *stats, void *pieces, float *scale, void *stream) {
+    if (!x || !stats || !pieces || !scale) return fail(FTC_ERR_INVALID, "null pointer");
+    if (!aligned(stats)) return fail(FTC_ERR_INVALID, "rows must be 16-byte aligned");
+    return launch_rows<true>(x, gamma, beta, eps, rows, cols, nullptr, stats, pieces, scale, (hipStream_t)stream);
+}
+
+static int product(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
+                   const float *bias, const float *w_norm, int64_t features, int64_t k, const float *residual,
+                   const float *stats, const float *gamma, const float *beta, float *out, void *relu_pieces,
+                   float *relu_scale, void *stream) {
     if (!x || !x_scale || !w || !w_scale || !bias || (!out && !relu_pieces))
         return fail(FTC_ERR_INVALID, "null pointer");
     if (relu_pieces && (!relu_scale || !w_norm || residual || out))
         return fail(FTC_ERR_INVALID, "relu rows leave in pieces, with a scale and without a residual");
     if (!aligned(x) || !aligned(w) || !aligned(w_scale) || !aligned(bias) || !aligned(residual) || !aligned(out) ||
-        !aligned(relu_pieces))
+        !aligned(relu_pieces) || !aligned(stats) || !aligned(gamma) || !aligned(beta))
         return fail(FTC_ERR_INVALID, "rows must be 16-byte aligned");
     if (k % kStep != 0 || k < 2 * kStep || k > kMostColumns || features % 4 != 0 || features <= 0 ||
         features > kMostColumns || (relu_pieces && features % kStep != 0))
@@ -827,7 +876,7 @@ int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const 
     if (tokens <= 0) return FTC_OK;
     LinearArgs a;
     a.x = (const char *)x, a.w = (const char *)w, a.x_scale = x_scale, a.w_scale = w_scale, a.bias = bias;
-    a.w_norm = w_norm, a.residual = residual, a.out = out, a.out_pieces = (char *)relu_pieces;
+    a.w_norm = w_norm, a.residual = residual, a.stats = (const float2 *)stats, a.gamma = gamma, a.beta = beta, a.out = out, a.out_pieces = (char *)relu_pieces;
     a.out_scale = relu_scale, a.tokens = tokens, a.features = (int32_t)features, a.k = (int32_t)k;
     a.streamed = 4 * tokens * (k + (residual ? 2 : 1) * features) >= kStreamedBytes;
     const hipStream_t on = (hipStream_t)stream;
@@ -843,6 +892,21 @@ int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const 
                            (int)features);
     }
     return launched("product");
+}
+
+int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
+                     const float *bias, const float *w_norm, int64_t features, int64_t k,
+                     const float *residual, float *out, void *relu_pieces, float *relu_scale, void *stream) {
+    return product(x, x_scale, tokens, w, w_scale, bias, w_norm, features, k, residual, nullptr, nullptr, nullptr, out,
+                   relu_pieces, relu_scale, stream);
+}
+
+int ftc_linear_split_normed(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
+                            const float *bias, int64_t features, int64_t k, const float *rows, const float *stats,
+                            const float *gamma, const float *beta, float *out, void *stream) {
+    if (!rows || !stats || !out) return fail(FTC_ERR_INVALID, "null pointer");
+    return product(x, x_scale, tokens, w, w_scale, bias, nullptr, features, k, rows, stats, gamma, beta, out, nullptr,
+                   nullptr, stream);
 }
 
 }  // extern "C"

@@ -43,7 +43,9 @@ EXPORTED_SYMBOLS = (
     "ftc_split_weights",
     "ftc_split_rows",
     "ftc_layer_norm_split",
+    "ftc_layer_norm_stats_split",
     "ftc_linear_split",
+    "ftc_linear_split_normed",
 )
 
 

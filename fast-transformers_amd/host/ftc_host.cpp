@@ -598,12 +598,11 @@ size_t layers_at_a_time(const std::vector<Layer> &layers, size_t from, int64_t v
 // leaving their rows in pieces as well.  `x`: dense (N, L, d).
 //
 // Memory: rows are kept only as long as they are read, so that the stack needs no more than its
-// modules did (six times x where the feed-forward layer has at most 3 d features: twelve with a
+// modules did (five times x where the feed-forward layer has at most 3 d features: twelve with a
 // buffer for each of them).  `wide` holds a layer's q, k and v; when the attention has read them, its
-// rows in pieces and, behind them, the output projection; then the feed-forward rows.  `rows` begins a
-// layer with x in pieces and has the attention's rows, the first norm's pieces and the second
-// product in turn; the second norm's pieces go to `other`, and the two change places.  `out` has the
-// first norm's rows and then the layer's.
+// rows in pieces; then the feed-forward rows.  `rows` begins a layer with x in pieces and has the attention's
+// rows and either norm's pieces in turn.  `out` has the rows before a norm, to which the next product adds the
+// norm of what was there; norms inside the stack leave their pieces and two numbers a row (stats).
 Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::optional<Norm> &final_norm,
                int64_t H, int64_t E, int64_t M, const OptTensor &key_lengths) {
     const at::NoGradGuard no_grad;
@@ -611,13 +610,13 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
     const auto fp32 = x.options();
     const int64_t *lengths = lengths_ptr(key_lengths, x);
     const int64_t width = H * (2 * E + M), most_rows = std::max(d, H * M);
-    int64_t most_wide = std::max(width, H * M + d);
+    int64_t most_wide = width;
     for (const Layer &l : layers) most_wide = std::max(most_wide, l.first.weight.size(0));
     const Tensor wide = at::empty({T, most_wide}, fp32), scale_of_rows = at::empty({T}, fp32),
                  scale_of_wide = at::empty({T}, fp32), out = at::empty_like(x);
-    Tensor rows_buffer = at::empty({T, most_rows}, fp32), other_buffer = at::empty({T, most_rows}, fp32);
-    float *const qkv = wide.data_ptr<float>(), *const projected = qkv + T * H * M;
-    float *rows = rows_buffer.data_ptr<float>(), *other = other_buffer.data_ptr<float>();
+    const Tensor rows_buffer = at::empty({T, most_rows}, fp32), stats_of_rows = at::empty({T, 2}, fp32);
+    float *const qkv = wide.data_ptr<float>(), *const rows = rows_buffer.data_ptr<float>();
+    float *const stats = stats_of_rows.data_ptr<float>();
     float *const row_scale = scale_of_rows.data_ptr<float>(), *const wide_scale = scale_of_wide.data_ptr<float>();
     float *const to = out.data_ptr<float>();
     auto view = [&](float *base, int64_t column, int64_t row, int64_t X) {
@@ -643,10 +642,19 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
     auto split = [&](const float *from, int64_t columns, float *pieces, float *pieces_scale) {
         check(ftc_split_rows(from, T, columns, pieces, pieces_scale, stream), "ftc_split_rows");
     };
-    auto norm = [&](const float *from, const Norm &n, float *y, float *pieces) {
-        check(ftc_layer_norm_split(from, f(n.weight), f(n.bias), (float)n.eps, T, d, y, pieces,
-                                   pieces ? row_scale : nullptr, stream),
+    auto norm = [&](const float *from, const Norm &n, float *y) {
+        check(ftc_layer_norm_split(from, f(n.weight), f(n.bias), (float)n.eps, T, d, y, nullptr, nullptr, stream),
               "ftc_layer_norm_split");
+    };
+    // the norm of `to` in pieces, and what a product needs to add it to its own rows
+    auto norm_of_rows = [&](const Norm &n) {
+        check(ftc_layer_norm_stats_split(to, f(n.weight), f(n.bias), (float)n.eps, T, d, stats, rows, row_scale, stream),
+              "ftc_layer_norm_stats_split");
+    };
+    auto linear_normed = [&](const Pieces &w, const Norm &n, float *y) {
+        check(ftc_linear_split_normed(qkv, wide_scale, T, w.pieces, w.scale, w.bias, w.rows, w.cols, to, stats,
+                                      f(n.weight), f(n.bias), y, stream),
+              "ftc_linear_split_normed");
     };
     native([&] {
         split(x.const_data_ptr<float>(), d, rows, row_scale);
@@ -655,7 +663,6 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
         size_t cut_from = 0;
         for (size_t i = 0; i < layers.size(); i++) {
             const Layer &l = layers[i];
-            const float *const input = i == 0 ? x.const_data_ptr<float>() : to;
             if (i == cut_from + cut.size()) {
                 const size_t n = layers_at_a_time(layers, i, T * d);
                 int64_t floats = 0;
@@ -675,18 +682,19 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
                                                       call.ws_bytes, stream),
                   "ftc_causal_linear_attention_forward");
             split(rows, H * M, qkv, wide_scale);
-            linear(qkv, wide_scale, w.proj, input, projected, nullptr, nullptr);
-            norm(projected, l.norm1, to, rows);
+            if (i == 0)
+                linear(qkv, wide_scale, w.proj, x.const_data_ptr<float>(), to, nullptr, nullptr);
+            else
+                linear_normed(w.proj, layers[i - 1].norm2, to);
+            norm_of_rows(l.norm1);
             linear(rows, row_scale, w.first, nullptr, nullptr, qkv, wide_scale);
-            linear(qkv, wide_scale, w.second, to, rows, nullptr, nullptr);
             if (i + 1 < layers.size()) {
-                norm(rows, l.norm2, to, other);
-                std::swap(rows, other);
-            } else if (final_norm) {
-                norm(rows, l.norm2, other, nullptr);
-                norm(other, *final_norm, to, nullptr);
+                linear_normed(w.second, l.norm1, to);
+                norm_of_rows(l.norm2);
             } else {
-                norm(rows, l.norm2, to, nullptr);
+                linear_normed(w.second, l.norm1, rows);
+                norm(rows, l.norm2, final_norm ? qkv : to);
+                if (final_norm) norm(qkv, *final_norm, to);
             }
         }
     }, call.turn);

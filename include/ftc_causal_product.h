@@ -314,6 +314,9 @@ int ftc_split_rows(const float *x, int64_t rows, int64_t cols, void *pieces, flo
 /* out = torch.nn.LayerNorm of dense rows (gamma, beta may be NULL), also in pieces unless NULL. */
 int ftc_layer_norm_split(const float *x, const float *gamma, const float *beta, float eps, int64_t rows,
                          int64_t cols, float *out, void *pieces, float *scale, void *stream);
+/* The same rows in pieces alone, and stats[2 r], stats[2 r + 1] = mean and 1 / sqrt(variance + eps) of row r. */
+int ftc_layer_norm_stats_split(const float *x, const float *gamma, const float *beta, float eps, int64_t rows,
+                               int64_t cols, float *stats, void *pieces, float *scale, void *stream);
 /*
  * y[t][f] = sum_k x[t][k] w[f][k] + bias[f] for rows in pieces.  Either out = y (+ residual, dense
  * tokens x features, unless NULL), or max(y, 0) in pieces (relu_pieces, relu_scale; w_norm from
@@ -322,6 +325,13 @@ int ftc_layer_norm_split(const float *x, const float *gamma, const float *beta, 
 int ftc_linear_split(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
                      const float *bias, const float *w_norm, int64_t features, int64_t k,
                      const float *residual, float *out, void *relu_pieces, float *relu_scale, void *stream);
+/*
+ * out = y + the layer norm of `rows` (dense tokens x features; out may be rows), whose stats are those of
+ * ftc_layer_norm_stats_split.
+ */
+int ftc_linear_split_normed(const void *x, const float *x_scale, int64_t tokens, const void *w, const float *w_scale,
+                            const float *bias, int64_t features, int64_t k, const float *rows, const float *stats,
+                            const float *gamma, const float *beta, float *out, void *stream);
 
 #ifdef __cplusplus
 }

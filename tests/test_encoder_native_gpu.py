@@ -401,3 +401,41 @@ def test_weights_of_many_matrices_are_cut_in_one_launch(count):
             assert torch.equal(x.view(torch.int32), y.view(torch.int32))
         assert (whole(*together[:2]) - w.double()).abs().max() <= 2.0 ** -22 * w.abs().max()
     assert lib.ftc_split_weights((Weight * 49)(), 49, stream()) == -1
+
+
+@pytest.mark.parametrize("weights", ["both", "beta", "none"])
+@pytest.mark.parametrize("shape", [
+    # tokens, columns, features: each of the four tiles, rows and features that end inside one, more tiles than
+    # workgroups, steps fewer and more than a tile's buffers
+    (4990, 512, 1536), (9990, 160, 1536), (4100, 160, 288), (70001, 96, 256), (129, 96, 544), (33, 64, 64), (1, 64, 32)],
+    ids=lambda s: "t%d_k%d_f%d" % s)
+def test_a_norm_that_is_added_is_the_norm_that_was_stored(shape, weights):
+    """Products that make a layer norm's rows again from (mean, r) add the same values, bit for bit, as from its rows,
+    also where their own go over the rows before the norm."""
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    T, K, F = shape
+    gen = torch.Generator(device="cuda").manual_seed(T + F)
+    x, w, b, r = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, K), (F, K), (F,), (T, F)))
+    r = r * 3 + 5 * torch.randn(T, 1, device="cuda", generator=gen)
+    gamma = torch.randn(F, device="cuda", generator=gen) if weights == "both" else None
+    beta = torch.randn(F, device="cuda", generator=gen) if weights != "none" else None
+    new = lambda *s: torch.full(s, float("nan"), device="cuda")
+    n = lambda i: ctypes.c_int64(i)
+    xp, xs, wp, ws, bo, wn = new(T, K), new(T), new(F, K), new(F), new(F), new(F)
+    item = Weight(w.data_ptr(), b.data_ptr(), F, K, wp.data_ptr(), ws.data_ptr(), bo.data_ptr(), wn.data_ptr())
+    assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == 0, _native.last_error()
+    assert lib.ftc_split_rows(ptr(x), n(T), n(K), ptr(xp), ptr(xs), stream()) == 0
+    rows, pieces, scale, stats, pieces2, scale2 = new(T, F), new(T, F), new(T), new(T, 2), new(T, F), new(T)
+    eps = ctypes.c_float(1e-5)
+    assert lib.ftc_layer_norm_split(ptr(r), ptr(gamma), ptr(beta), eps, n(T), n(F), ptr(rows), ptr(pieces), ptr(scale), stream()) == 0
+    assert lib.ftc_layer_norm_stats_split(ptr(r), ptr(gamma), ptr(beta), eps, n(T), n(F), ptr(stats), ptr(pieces2),
+                                          ptr(scale2), stream()) == 0, _native.last_error()
+    assert torch.equal(pieces.view(torch.int32), pieces2.view(torch.int32)) and torch.equal(scale, scale2)
+    want, got = new(T, F), new(T, F)
+    assert lib.ftc_linear_split(ptr(xp), ptr(xs), n(T), ptr(wp), ptr(ws), ptr(bo), ptr(wn), n(F), n(K), ptr(rows),
+                                ptr(want), None, None, stream()) == 0
+    for out in (got, r):
+        assert lib.ftc_linear_split_normed(ptr(xp), ptr(xs), n(T), ptr(wp), ptr(ws), ptr(bo), n(F), n(K), ptr(r), ptr(stats),
+                                           ptr(gamma), ptr(beta), ptr(out), stream()) == 0, _native.last_error()
+        assert torch.equal(out, want)
