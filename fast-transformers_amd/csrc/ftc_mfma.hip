@@ -282,8 +282,12 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // walking the chain (64 x 64 forward, 8 chains, L=640: 19 against 27 us; 128 x 128 backward, 4
     // chains, L=512: 29 against 62).  A single scan on the bf16-piece kernel, and its scans with
     // half of the consumers idle, only up to 8 chunks (128 x 128 forward, 2 chains, L=256: 16
-    // against 17, L=512: 22 against 17; 128 x 32 forward, 8 chains, L=512: 27 against 20).
-    const int64_t brief_chunks = D <= 64 || (F > 32 && nscans >= 2) ? 23 : 8;
+    // against 17, L=512: 22 against 17; 128 x 32 forward, 8 chains, L=512: 27 against 20); of that kernel's with
+    // more than 32 columns up to 10, from eight workgroups' worth on up to 13 and from twenty on up to 23 (128 x 128
+    // forward, us, the kernels that split L / this one: 2 chains, L=270 17.2 / 14.4, L=390 18.8 / 18.3; 4, L=390 20.1 / 18.3, L=500
+    // 20.9 / 22.0; 12, L=500 27.3 / 22.0, L=700 30.3 / 27.9; 128 x 64, 20 chains, L=610 29.7 / 25.8; 96 x 96, 12, L=390 20.2 /
+    // 17.2; errors against float64 0.6 to 0.7 of theirs).
+    const int64_t brief_chunks = D <= 64 || (F > 32 && nscans >= 2) ? 23 : F <= 32 ? 8 : units >= 20 ? 23 : units >= 8 ? 13 : 10;
     if (narrow && D <= 32 && F <= 32) return;
     // Thousands of chains of one or two chunks with a state of at most 64 x 64 go to those kernels too,
     // where a workgroup's start costs more than its chunks (8192 chains, L=64: 32 x 128 1.17
@@ -402,7 +406,9 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
         if (!single || D <= 64) return false;
         if (D <= 96 && F > 64 && F <= 96 && chunks > 48 && units >= (bf16_results ? 12 : 20) && units < (bf16_results ? 176 : 128))
             return true;
-        return chunks > 8 && chunks < (units <= 1 ? 128 : units <= 3 ? 96 : units <= 7 ? 48 : units < 16 ? 28 : 0);
+        // (128 x 128, us, split L / here: 3 chains, L=390 15.0 / 13.0, 6, L=610 20.8 / 17.2, L=760 23.3 / 19.3, but 3, L=500 15.0 / 15.2;
+        // errors against float64 half of theirs)
+        return chunks > 13 && chunks < (units <= 1 ? 128 : units <= 3 ? 96 : units <= 7 ? 48 : units < 12 ? 28 : 0);
     }
     if (!single) {
         if (D <= 32 && F <= 32) {
@@ -724,11 +730,12 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     if (!tp_widths(D, F, forced, odd)) return false;
     if (odd && !forced && !tph_takes_rows(D)) return false;
     int64_t widest_stride = 0;
-    bool mixed = false;
+    bool mixed = false, stateful = false;
     for (int i = 0; i < nscans; i++) {
         const ScanDesc &sd = scans[i];
         const Combo combo = combo_of(sd);
         mixed = mixed || combo != kFFFF;
+        stateful = stateful || sd.initial.ptr || sd.final_.ptr;
         // (rows with bf16 among them: not as parts of wider scans, whose results are added up in fp32)
         if (combo == kNone || (combo != kFFFF && (forced || tuning().tph == 0))) return false;
         // (odd widths: scans of any widths side by side, where pieces are scaled as long as none has a
@@ -754,6 +761,15 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
         return false;
     int nseg = 0, seg_chunks = 0;
     const int64_t chains = std::max<int64_t>(1, N * H);
+    // (fp32 states of more than 64 rows that are handed in or out stay with the kernels that split L, whose sums are
+    // shorter, where those have no more than the 9 to 23 chunks of few chains to walk: 128 x 128, 8 chains, L=400 39.0 us
+    // for 22.1, but the state is 1.25e-7 from float64 there and 3.5e-7 here; the rows are 1.9e-7 and 1.3e-7.
+    // Those that are only handed in as well: rows are the same whether the state is asked for or not)
+    const int64_t chunks = (L + kChunk - 1) / kChunk, units = chains * tp_fblocks(F);
+    if (stateful && !mixed && !forced && !odd && nscans == 1 && D > 64 && F > 32 && chunks > 8 && chunks < 24 &&
+        units * std::max<int64_t>(1, std::min<int64_t>(4, 256 / units)) < 128 && tuning().tp < 0 &&
+        mfma_scan_supported_widths(D, F))
+        return false;
     if (mixed)
         mixed_plan(D, F, chains, nscans, L, scans[0].out.dtype != FTC_F32, &nseg, &seg_chunks);
     else if (odd && forced)

@@ -388,3 +388,21 @@ def test_segments_of_few_chains_have_four_chunks(chunks, heads):
     assert (segments - 1) * rows < L <= segments * rows
     need = int(field(line, r"workspace (\d+) bytes"))
     assert 0 < need <= _native.load().ftc_causal_dot_product_workspace_bytes(1, heads, L, 64, 64, 0)
+
+
+def test_short_chains_of_wide_states_on_few_workgroups():
+    """A single scan of more than 64 state rows: up to 10 chunks on any number of workgroups, from eight on up to 13, from
+    twenty on up to where an exchange begins; bf16 rows up to 13, from twelve workgroups on any number."""
+    def fwd(chains, chunks, E=128, M=128, dtype=_native.FTC_F32):
+        s = (1, chains, 32 * chunks - 3)
+        return kernel(lines(s + (E,), s + (M,), dtype=dtype)[0])
+    tp, split = "scan_tp_kernel", "scan_mfma_kernel"
+    for chains, chunks, E, M, want in [(1, 10, 128, 128, tp), (1, 11, 128, 128, split), (3, 13, 128, 128, split),
+                                       (4, 13, 128, 128, tp), (7, 13, 128, 64, split), (8, 13, 128, 64, tp),
+                                       (8, 14, 128, 128, split), (9, 23, 128, 128, split), (10, 14, 128, 128, tp),
+                                       (10, 23, 96, 96, tp), (20, 23, 128, 64, tp), (8, 9, 128, 32, split)]:
+        assert fwd(chains, chunks, E, M) == want, (chains, chunks, E, M)
+    tp = "scan_tp_bf16_kernel"
+    for chains, chunks, M, want in [(1, 13, 128, tp), (1, 14, 128, split), (5, 14, 128, split), (6, 27, 128, tp),
+                                    (11, 27, 64, split), (12, 14, 64, tp)]:
+        assert fwd(chains, chunks, 128, M, _native.FTC_BF16) == want, (chains, chunks, M)

@@ -112,3 +112,25 @@ def test_small_rows_and_columns_beside_large_ones(cp, small, shape):
     for got, ref, ex in zip(outs, refs, exact):
         for dim in (2, 3):
             assert _each(got.cpu(), ex, dim) <= max(4 * _each(ref, ex, dim), 2e-6)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 289, 128, 128), (1, 4, 416, 128, 128), (2, 4, 385, 128, 64), (2, 5, 705, 96, 96),
+                                   (5, 4, 449, 128, 64)], ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_short_chains_of_wide_states(shape, dtype):
+    """Few short chains walked whole or cut where they were split with an exchange: a last chunk of one row, states
+    handed in and out; no further from float64 than the oracle's own order."""
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = shape
+    gen = torch.Generator().manual_seed(L)
+    Q, K = (torch.nn.functional.elu(torch.randn(N, H, L, E, generator=gen)) + 1 for _ in range(2))
+    V, S = torch.randn(N, H, L, M, generator=gen), 5 * torch.randn(N, H, E, M, generator=gen)
+    q, k, v = (t.cuda().to(dtype) for t in (Q, K, V))
+    Q, K, V = (t.float().cpu() for t in (q, k, v))
+    out, state = cp.causal_dot_product_with_state(q, k, v, S.cuda())
+    exact = oracle.forward(Q.double(), K.double(), V.double()) + Q.double() @ S.double()
+    plain = oracle.forward(Q, K, V) + Q @ S
+    assert scale_error(out.cpu(), exact) <= max(4 * scale_error(plain, exact), 2e-6)
+    final = S.double() + K.double().transpose(2, 3).contiguous() @ V.double()
+    assert scale_error(state.cpu(), final) <= 2e-6
+    assert torch.equal(out, cp.causal_dot_product_with_state(q, k, v, S.cuda())[0])
