@@ -309,7 +309,7 @@ struct StateExchange {
 
     // T += the states of `count` slots, `stride` apart, in ascending order.  The states of a batch are
     // in flight together: one after the other each costs a trip past the caches (forward, one chain of 49070
-    // positions 37.6 -> 35.4 us, of 6150 24.3 -> 23.4; 16 chains of 65536, bound by memory, the same).
+    // positions two at a time 36.5 -> 35.0 us; 16 chains of 65536, bound by memory, the same).
     __device__ __forceinline__ void add_states(uint32_t first, uint32_t stride, int count, f32x16 (&T)[DT][FT]) {
         constexpr int kQuads = DT * FT * 4;
         for (int i0 = 0; i0 < count; i0 += kBatch) {

@@ -865,9 +865,9 @@ __device__ __forceinline__ void scan_tp_body(uint32_t *__restrict__ ws_ptr, cons
         // the flag words and state slots of consumer w of the segment with ticket t are those
         // of "ticket" w * total_units + t (as in ftc_wg_kernel.h)
         constexpr int DX = NORM ? ND + 1 : ND;  // (z rides along in a tile of its own)
-        // (bf16 rows keep the registers with which two workgroups share a CU where the state has 32 rows: 114 of them,
-        // 150 with four states at a time; two blocks have none to spare)
-        constexpr int kBatch = ND == 1 && PA + PB + PV == 9 ? 4 / DX : 1;
+        // (bf16 rows keep the registers with which two workgroups share a CU where the state has 32 rows; two blocks have
+        // none to spare)
+        constexpr int kBatch = ND == 1 && PA + PB + PV == 9 ? 2 : 1;
         StateExchange<DX, 1, kBatch> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);

@@ -761,16 +761,22 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
 #pragma unroll
         for (int i = 0; i < 12; i++) {
             if ((i % 4) / 2 < KS) S[i % 4] = mfma16h(bt2[i % 4][kPa[i / 4]], vf2[kPb[i / 4]], S[i % 4]);
+            if (!GRAD) rm_frag(unit_pc + buf * kBufBytes, i);  // our own first chunk is cut
             __builtin_amdgcn_sched_barrier(0);
         }
         read_slot(slots, buf, ce);  // the ceilings of our own first chunk
+    } else if (!GRAD) {
+#pragma unroll
+        for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
     }
     if (exchange) {
         // ---- the sum of this segment's rows goes out, the state before the segment comes in ----
         const uint32_t total_units = (uint32_t)p.total_waves;
         gfloat *const sums = (gfloat *)(hdr + kControlBytes / 4);
         constexpr int DX = GRAD ? 2 : 1;  // (Z rides along in a tile of its own)
-        StateExchange<DX, 1, 4 / DX> xch(flags, sums, 4u * total_units,
+        // (four at a time need the registers of the fragments, and those read behind the exchange: 8 chains, L=512, which
+        // exchange nothing, 15.04 -> 15.14 us)
+        StateExchange<DX, 1, GRAD ? 1 : 2> xch(flags, sums, 4u * total_units,
                                 (uint32_t)w * total_units + chain_id * nseg + (uint32_t)seg, seg,
                                 (int)nseg, p.group, lane);
         f32x16 Sx[DX][1], X[DX][1];
@@ -800,9 +806,10 @@ __device__ __forceinline__ void scan_tph_body(uint32_t *__restrict__ ws_ptr, con
         }
         if (!GRAD && op.s0) add_caller_state();
     }
-    // our own first chunk's (not before: with 48 registers of fragments beside the states that are exchanged, spills)
+    if (GRAD) {  // (not before: two tiles are exchanged, and 48 registers of fragments beside them spilled)
 #pragma unroll
-    for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
+        for (int i = 0; i < 12; i++) rm_frag(unit_pc, i);
+    }
     // ---- the walk proper ----
     // `ce` holds the ceilings of the chunk at hand, Ucur the units of S.  dU < 0: the
     // state's units rise by -dU with this chunk (S is rescaled once all of it has been cut).
