@@ -412,6 +412,13 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     }
     if (!single) {
         if (D <= 32 && F <= 32) {
+            // (bf16 results, rounds of 256 workgroups: two thirds full, or short or few enough for an exchange.  us, split L /
+            // here: 64 chains, L=4128 124 / 86, 85 chains 144 / 91 and L=16384 448 / 305, but 86 chains 469 / 549;
+            // 160 chains, L=8192 417 / 312, 112 chains 302 / 303; 40 chains, L=6000 125 / 110, 20 chains, L=11000
+            // 127 / 106, 32 chains, L=11000 157 / 173)
+            if (bf16_results && chunks > 128 && chunks <= 1024)
+                return units > 48 && units * 3 < (units + 255) / 256 * 512 && !(units <= 256 && chunks <= 192) &&
+                       !(units <= 60 && chunks <= 512) && !(units <= 84 && chunks <= 344);
             if (chunks > 128) return units > (chunks > 1024 ? 24 : 48);
             return chunks <= 64 && units > (chunks <= 4 ? 1024 : chunks <= 8 ? 1100 : 1536);
         }

@@ -406,3 +406,14 @@ def test_short_chains_of_wide_states_on_few_workgroups():
     for chains, chunks, M, want in [(1, 13, 128, tp), (1, 14, 128, split), (5, 14, 128, split), (6, 27, 128, tp),
                                     (11, 27, 64, split), (12, 14, 64, tp)]:
         assert fwd(chains, chunks, 128, M, _native.FTC_BF16) == want, (chains, chunks, M)
+
+
+@pytest.mark.parametrize("chains,L,route", [
+    (64, 4128, "whole"), (85, 16384, "whole"), (85, 32768, "whole"), (172, 8192, "whole"), (20, 11000, "exchange"),
+    (40, 6000, "exchange"), (18, 16384, "exchange"), (86, 16384, None), (32, 11000, None), (112, 8192, None),
+    (64, 32800, None)])
+def test_long_narrow_backward_scans_of_bf16_rows(chains, L, route):
+    """32 x 32: by how full the rounds of workgroups are, or few enough chains for an exchange of sums."""
+    got = lines((1, chains, L, 32), (1, chains, L, 32), backward=True, dtype=_native.FTC_BF16)[0]
+    want = {"whole": "scan_tp_bf16_kernel", "exchange": "scan_tp_bf16_kernel (exchange)", None: "scan_mfma_kernel"}
+    assert kernel(got) == want[route]
