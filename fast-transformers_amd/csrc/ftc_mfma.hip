@@ -412,12 +412,12 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     }
     if (!single) {
         if (D <= 32 && F <= 32) {
-            // (bf16 results, rounds of 256 workgroups: two thirds full, or short or few enough for an exchange.  us, split L /
+            // (bf16 results, rounds of 256 workgroups: seven tenths full, or short or few enough for an exchange.  us, split L /
             // here: 64 chains, L=4128 124 / 86, 85 chains 144 / 91 and L=16384 448 / 305, but 86 chains 469 / 549;
-            // 160 chains, L=8192 417 / 312, 112 chains 302 / 303; 40 chains, L=6000 125 / 110, 20 chains, L=11000
+            // 160 chains, L=8192 417 / 312, but 112 chains 302 / 303; 40 chains, L=6000 125 / 110, 20 chains, L=11000
             // 127 / 106, 32 chains, L=11000 157 / 173)
             if (bf16_results && chunks > 128 && chunks <= 1024)
-                return units > 48 && units * 3 < (units + 255) / 256 * 512 && !(units <= 256 && chunks <= 192) &&
+                return units > 48 && units * 10 < (units + 255) / 256 * 1792 && !(units <= 256 && chunks <= 192) &&
                        !(units <= 60 && chunks <= 512) && !(units <= 84 && chunks <= 344);
             if (chunks > 128) return units > (chunks > 1024 ? 24 : 48);
             return chunks <= 64 && units > (chunks <= 4 ? 1024 : chunks <= 8 ? 1100 : 1536);
@@ -453,9 +453,14 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     }
     if (chunks <= 24) return units > 512;
     if (chunks <= 48) return units < 48 || (units > 512 && (bf16_results || (D <= 32 && units < 900)));
-    if (chunks > 256) return true;
-    if (D <= 32) return units < (chunks <= 72 ? 176 : 224) || (bf16_results && units > 512);
-    return units < (chunks <= 96 ? (bf16_results || chunks > 72 ? 112 : 64) : bf16_results ? 176 : 160) || (bf16_results && units > 512);
+    // (forward, 4 to 512 chains of 1600 to 32768 positions, us with inputs from memory, split L / here.  32 x 32: 96 chains,
+    // L=1600 35.0 / 33.6, but 80 29 / 31; 128, L=2600 57 / 50; 160, L=4128 97 / 78, L=8192 171 / 142, but 120 140 / 142, and 136 84 / 76
+    // and 150 / 136, which is 62 / 68 with inputs left in the caches.  64 x 32: 80 chains, L=2600 57 / 52, but 64 47 / 48; 48, L=6000
+    // 77 / 66; 152, L=8192 241 / 173; 24, L=11000 78 / 64; 448, L=11000 712 / 690.  Errors against float64 0.25 to 0.79 of theirs)
+    if (chunks > 256) return D <= 32 || bf16_results || units < (chunks <= 320 ? 48 : 24) || units > 512;
+    if (bf16_results) return units < (D <= 32 ? (chunks <= 72 ? 176 : 224) : chunks <= 96 ? 112 : 176) || units > 512;
+    if (D <= 32) return units < (chunks <= 56 ? 96 : chunks <= 88 ? 128 : 160);
+    return units < (chunks <= 72 ? 64 : chunks <= 160 ? 80 : 48);
 }
 
 // The plan of scans with bf16 rows among them on the chain-parallel kernel (three pieces for the state and

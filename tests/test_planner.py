@@ -409,7 +409,7 @@ def test_short_chains_of_wide_states_on_few_workgroups():
 
 
 @pytest.mark.parametrize("chains,L,route", [
-    (64, 4128, "whole"), (85, 16384, "whole"), (85, 32768, "whole"), (172, 8192, "whole"), (20, 11000, "exchange"),
+    (64, 4128, "whole"), (85, 16384, "whole"), (85, 32768, "whole"), (180, 8192, "whole"), (20, 11000, "exchange"),
     (40, 6000, "exchange"), (18, 16384, "exchange"), (86, 16384, None), (32, 11000, None), (112, 8192, None),
     (64, 32800, None)])
 def test_long_narrow_backward_scans_of_bf16_rows(chains, L, route):
@@ -417,3 +417,13 @@ def test_long_narrow_backward_scans_of_bf16_rows(chains, L, route):
     got = lines((1, chains, L, 32), (1, chains, L, 32), backward=True, dtype=_native.FTC_BF16)[0]
     want = {"whole": "scan_tp_bf16_kernel", "exchange": "scan_tp_bf16_kernel (exchange)", None: "scan_mfma_kernel"}
     assert kernel(got) == want[route]
+
+
+@pytest.mark.parametrize("chains,L,D,splits", [
+    (95, 1600, 32, True), (96, 1600, 32, False), (127, 2600, 32, True), (128, 2600, 32, False), (159, 8192, 32, True),
+    (160, 8192, 32, False), (160, 8224, 32, True), (79, 3300, 64, True), (80, 3300, 64, False), (47, 6000, 64, True),
+    (48, 6000, 64, False), (47, 8224, 64, True), (48, 8224, 64, False), (23, 11000, 64, True), (24, 11000, 64, False)])
+def test_long_forward_scans_of_bf16_rows_with_32_columns(chains, L, D, splits):
+    got = lines((1, chains, L, D), (1, chains, L, 32), dtype=_native.FTC_BF16)[0]
+    assert (kernel(got) == "scan_mfma_kernel") == splits
+    assert splits or kernel(got).startswith("scan_tp_bf16_kernel")
