@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139913210, "64355113863568e9"),
-    "cfg3": (2618002868, "64355113863568e9"),
-    "cfg5": (4150016208, "64355113863568e9"),
-    "wide": (1877124153, "64355113863568e9"),
+    "cfg2": (139917319, "d18cc6259653fd1e"),
+    "cfg3": (2616000991, "d18cc6259653fd1e"),
+    "cfg5": (4156315083, "d18cc6259653fd1e"),
+    "wide": (1877174347, "d18cc6259653fd1e"),
 }
 
 WORKLOADS = {
