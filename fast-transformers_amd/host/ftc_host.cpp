@@ -632,28 +632,37 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
                                  "ftc_causal_linear_attention_workspace_bytes", N, H, L, E, M, FTC_F32));
     void *const stream = call.stream;
     auto f = [](const OptTensor &t) { return t ? t->const_data_ptr<float>() : nullptr; };
+    // (whoever writes rows of so many values asks first: d, the heads' widths and the feed-forward width are
+    // independent of each other)
+    auto room = [&](float *base, int64_t columns) {
+        const int64_t most = base == qkv ? most_wide : base == rows ? most_rows : d;
+        TORCH_CHECK(columns <= most, "rows of ", columns, " values in a buffer for ", most);
+        return base;
+    };
     // (either the rows themselves or, behind max(., 0), in pieces with a scale)
     auto linear = [&](const float *pieces, const float *pieces_scale, const Pieces &w, const float *residual,
                       float *y, float *relu_pieces, float *relu_scale) {
-        check(ftc_linear_split(pieces, pieces_scale, T, w.pieces, w.scale, w.bias, w.norm, w.rows, w.cols, residual, y,
-                               relu_pieces, relu_scale, stream),
+        check(ftc_linear_split(pieces, pieces_scale, T, w.pieces, w.scale, w.bias, w.norm, w.rows, w.cols, residual,
+                               y ? room(y, w.rows) : y, relu_pieces ? room(relu_pieces, w.rows) : relu_pieces,
+                               relu_scale, stream),
               "ftc_linear_split");
     };
     auto split = [&](const float *from, int64_t columns, float *pieces, float *pieces_scale) {
-        check(ftc_split_rows(from, T, columns, pieces, pieces_scale, stream), "ftc_split_rows");
+        check(ftc_split_rows(from, T, columns, room(pieces, columns), pieces_scale, stream), "ftc_split_rows");
     };
     auto norm = [&](const float *from, const Norm &n, float *y) {
-        check(ftc_layer_norm_split(from, f(n.weight), f(n.bias), (float)n.eps, T, d, y, nullptr, nullptr, stream),
+        check(ftc_layer_norm_split(from, f(n.weight), f(n.bias), (float)n.eps, T, d, room(y, d), nullptr, nullptr, stream),
               "ftc_layer_norm_split");
     };
     // the norm of `to` in pieces, and what a product needs to add it to its own rows
     auto norm_of_rows = [&](const Norm &n) {
-        check(ftc_layer_norm_stats_split(to, f(n.weight), f(n.bias), (float)n.eps, T, d, stats, rows, row_scale, stream),
+        check(ftc_layer_norm_stats_split(to, f(n.weight), f(n.bias), (float)n.eps, T, d, stats, room(rows, d), row_scale,
+                                         stream),
               "ftc_layer_norm_stats_split");
     };
     auto linear_normed = [&](const Pieces &w, const Norm &n, float *y) {
         check(ftc_linear_split_normed(qkv, wide_scale, T, w.pieces, w.scale, w.bias, w.rows, w.cols, to, stats,
-                                      f(n.weight), f(n.bias), y, stream),
+                                      f(n.weight), f(n.bias), room(y, w.rows), stream),
               "ftc_linear_split_normed");
     };
     native([&] {
@@ -677,7 +686,7 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
             }
             const LayerPieces &w = cut[i - cut_from];
             linear(rows, row_scale, w.in, nullptr, qkv, nullptr, nullptr);
-            const ftc_tensor4 o = view(rows, 0, H * M, M);
+            const ftc_tensor4 o = view(room(rows, H * M), 0, H * M, M);
             check(ftc_causal_linear_attention_forward(&q, &k, &v, lengths, (float)l.eps, &o, nullptr, call.ws,
                                                       call.ws_bytes, stream),
                   "ftc_causal_linear_attention_forward");
@@ -692,9 +701,10 @@ Tensor encoder(const Tensor &x, const std::vector<Layer> &layers, const std::opt
                 linear_normed(w.second, l.norm1, to);
                 norm_of_rows(l.norm2);
             } else {
-                linear_normed(w.second, l.norm1, rows);
-                norm(rows, l.norm2, final_norm ? qkv : to);
-                if (final_norm) norm(qkv, *final_norm, to);
+                // (`wide` need not have room for rows of d values; the other two always do)
+                linear_normed(w.second, l.norm1, final_norm ? to : rows);
+                norm(final_norm ? to : rows, l.norm2, final_norm ? rows : to);
+                if (final_norm) norm(rows, *final_norm, to);
             }
         }
     }, call.turn);

@@ -439,3 +439,38 @@ def test_a_norm_that_is_added_is_the_norm_that_was_stored(shape, weights):
         assert lib.ftc_linear_split_normed(ptr(xp), ptr(xs), n(T), ptr(wp), ptr(ws), ptr(bo), n(F), n(K), ptr(r), ptr(stats),
                                            ptr(gamma), ptr(beta), ptr(out), stream()) == 0, _native.last_error()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("final", [True, False], ids=["final_norm", "no_norm"])
+@pytest.mark.parametrize("sizes", [
+    # d, heads, E, M, feed-forward: d beyond the heads' widths and the feed-forward width, by much and by a block;
+    # beyond one of them; heads beyond d and the feed-forward width
+    (512, 2, 32, 32, 128), (224, 2, 32, 32, 64), (512, 2, 64, 64, 1024), (256, 4, 64, 64, 64), (128, 8, 32, 64, 64)],
+    ids=lambda s: "d%d_h%d_e%d_m%d_f%d" % s)
+def test_encoder_whose_width_is_not_that_of_its_heads(sizes, final):
+    """The model's width, the heads' and the feed-forward width are independent of each other: rows of any of them
+    find room, and nothing beside them changes."""
+    from fast_transformers_amd import attention, masking
+    from fast_transformers_amd.attention import encoder as module
+    d, H, E, M, ff = sizes
+    N, L, layers = 3, 130, 2
+    torch.manual_seed(d + H)
+    with torch.device("cuda"):
+        model = attention.TransformerEncoder(
+            [attention.TransformerEncoderLayer(
+                attention.AttentionLayer(attention.CausalLinearAttention(E), d, H, d_keys=E, d_values=M), d, ff)
+             for _ in range(layers)], torch.nn.LayerNorm(d) if final else None).eval().requires_grad_(False)
+    x, mask = torch.rand(N, L, d, device="cuda"), masking.TriangularCausalMask(L, device="cuda")
+    calls, native = [], module.encoder_forward_hip
+    module.encoder_forward_hip = lambda *a: (calls.append(1), native(*a))[1]
+    try:
+        got = model(x, attn_mask=mask)
+        assert calls == [1]
+        handle = model.layers[0].linear1.register_forward_hook(lambda *a: None)
+        want = model(x, attn_mask=mask)
+        handle.remove()
+    finally:
+        module.encoder_forward_hip = native
+    assert calls == [1]
+    # two fp32 evaluations, as above
+    assert (got - want).abs().max() <= 4e-6 * layers * want.abs().max()
