@@ -189,7 +189,8 @@ TpCuts tp_cuts(int64_t D, bool scaled, bool fp32_rows, bool fp32_results, bool f
 // chain is cut into as many equal segments as fill the GPU (one workgroup each); a workgroup
 // walks its own chunks twice, first for their state alone.  Returns the number of chunks per
 // segment (0: not this way) and the number of segments in *nseg.
-int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg) {
+// (`most_fours`: the workgroups up to which a chain has a segment for every four chunks, see below)
+int tp_exchange_segments(int64_t units, int64_t L, bool wide, int64_t most_fours, int *nseg) {
     const int64_t total_chunks = (L + kChunk - 1) / kChunk;
     *nseg = 0;
     if (tuning().tpx == 0) return 0;  // tuning aid
@@ -244,10 +245,15 @@ int tp_exchange_segments(int64_t units, int64_t L, bool wide, int *nseg) {
     // segments of at least four chunks (one or two chains, L=4096: 32 segments 21.5 us, 16: 25.1), the last one
     // of what is left (forward, us, as many segments as there are whole fours of chunks, which makes eight of the four
     // a segment / this way: 8 chains, L=800 20.7 / 17.9, 1 chain, L=6150 24.8 / 19.9; backward of 4, L=1600 31 / 24).
-    // Not where that were more than 192 workgroups of 64 x 64, which wait for each other longer than
-    // they walk: 101 chunks, 208 of them 25.0 us and 104 24.8, 234 26.5 and 117 25.9, but 156 22.5 and 78 24.1.
+    // Not where that were more than `most_fours` workgroups, which wait for each other longer than they walk: a state of
+    // up to 64 rows 192 of them, whichever kernel and widths (eight chunks a segment / four: 64 x 64, 101 chunks, 208
+    // workgroups 24.8 / 25.0, 234 25.9 / 26.5, but 156 24.1 / 22.5; 64 x 128, 10 chains, L=1463 25.2 / 25.7, 4, L=4000 26.7 /
+    // 27.9; 25 x 33, 28 chains, L=1100 23.3 / 25.0; 48 x 48 backward, 9, L=1100 24.1 / 25.3; from 110 calls on either
+    // side of the line 0.88 to 0.97 of the time below it, 1.00 to 1.06 above); several scans of such a state on
+    // three bf16 pieces 240 (32 x 64 backward, 6 chains, L=1600, 234 of them 0.99, 2, L=5154, 246 1.05); wider ones any number
+    // (128 x 128, 8 chains, L=4000 0.89, 245 of 250 calls 0.73 to 0.93).
     const int64_t fours = (total_chunks + 3) / 4;
-    want = std::min<int64_t>(want, wide || units * fours <= 192 ? fours : total_chunks / 4);
+    want = std::min<int64_t>(want, units * fours <= most_fours ? fours : total_chunks / 4);
     if (tuning().tpx_segs >= 0) want = std::max(1, tuning().tpx_segs);  // tuning aid
     if (want < 2) return 0;
     const int64_t seg_chunks = ((total_chunks + want - 1) / want + kTpAhead - 1) / kTpAhead * kTpAhead;
@@ -331,7 +337,8 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // backward, 256 chains, L=12000: 1404 against 1825)
     const bool walk_long = D <= 64 && !(odd && forced) && L > 256 * kChunk && L <= 1024 * kChunk &&
                            units >= (!wide ? 112 : L > 512 * kChunk ? 128 : 192);
-    if (!narrow && !walk_long) *seg_chunks = tp_exchange_segments(units, L, wide, nseg);
+    const int64_t most_fours = D > 64 ? INT64_MAX : forced && nscans > 1 ? 240 : 192;
+    if (!narrow && !walk_long) *seg_chunks = tp_exchange_segments(units, L, wide, most_fours, nseg);
     // fp32 rows, 64 x 64: any number of chains of 16 chunks or more (the fp16-piece kernel walks
     // them faster than the kernels that split L stream them: backward, 256 chains, L=4096: 528
     // against 694 us; 768 chains, L=2048: 784 against 1013; forward, 1536 chains, L=1024: 309

@@ -427,3 +427,16 @@ def test_long_forward_scans_of_bf16_rows_with_32_columns(chains, L, D, splits):
     got = lines((1, chains, L, D), (1, chains, L, 32), dtype=_native.FTC_BF16)[0]
     assert (kernel(got) == "scan_mfma_kernel") == splits
     assert splits or kernel(got).startswith("scan_tp_bf16_kernel")
+
+
+@pytest.mark.parametrize("E,M,chains,L,most", [
+    # (each call's time with segments of four chunks was 1.02 to 1.07 of that with eight)
+    (64, 128, 14, 1100, 192), (64, 128, 4, 4000, 192), (48, 48, 28, 1100, 192), (25, 33, 28, 1100, 192),
+    (27, 63, 8, 4000, 192), (32, 32, 8, 3778, 192)])
+def test_small_states_do_not_exchange_on_too_many_workgroups(E, M, chains, L, most):
+    """Rounding a chain's segments up to one for every four chunks stops where that were more workgroups than gain
+    from it, for every state of up to 64 rows."""
+    chunks = -(-L // 32)
+    assert chunks % 4 and chains * -(-chunks // 4) * -(-M // 64) > most
+    line = lines((1, chains, L, E), (1, chains, L, M))[0]
+    assert "(exchange)" in line and int(field(line, r"segments of (\d+) rows")) == 256, line
