@@ -817,6 +817,16 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
     const int64_t chains = std::max<int64_t>(1, N * H), units = chains * nscans * tp_fblocks(F);
     tp_plan(D, F, chains, nscans, L, &nseg, &seg_chunks, forced, true);
     if (nseg == 0) return 1e30;
+    // (fitted to segments of whole fours of chunks, eight of them where a chain is no multiple of four.  Priced as the four that
+    // are launched, backward calls would be two launches instead of one: 75 x 10, 8 chains, L=989 37.7 -> 49.1 us,
+    // L=2900 61 -> 66, 99 x 101, 4 chains, L=4000 68 -> 85.  Others would gain, 32 chains, L=989, 75 x 10 62 -> 56 and
+    // 120 x 31 70 -> 59, with dQ and dK 1.5 times as far from float64, and 120 x 31, 7 to 20 chains, L=1463 0.87 to 0.92 of
+    // the time, 0.5 to 0.7 times as far)
+    const int64_t chunks = (L + kChunk - 1) / kChunk;
+    if (seg_chunks == kTpAhead && chunks % kTpAhead) {
+        seg_chunks = 2 * kTpAhead;
+        nseg = (int)((chunks + seg_chunks - 1) / seg_chunks);
+    }
     const int64_t rounds = (units * nseg + 255) / 256;
     double longest = 0.0;
     if (seg_chunks > 0) {
@@ -825,7 +835,7 @@ double mfma_tp_odd_chunks(int64_t D, int64_t F, int64_t N, int64_t H, int nscans
         // (at the price of tp_cuts more scans of two shapes would share a launch, 43 calls of 18106 in 0.88 of their
         // time, but 31 x 120 came out 3.5e-7 from float64 for 2.1e-7 and 75 x 10 2.5e-7 for 1.6e-7)
         int32_t start[kMaxTpSegments + 1];
-        nseg = tp_segment_starts((L + kChunk - 1) / kChunk, nseg, start, kTpAhead, 0.6);
+        nseg = tp_segment_starts(chunks, nseg, start, kTpAhead, 0.6);
         for (int s = 0; s < nseg; s++)
             longest = std::max(longest, 0.6 * start[s] + (double)(start[s + 1] - start[s]));
     }

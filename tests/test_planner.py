@@ -440,3 +440,12 @@ def test_small_states_do_not_exchange_on_too_many_workgroups(E, M, chains, L, mo
     assert chunks % 4 and chains * -(-chunks // 4) * -(-M // 64) > most
     line = lines((1, chains, L, E), (1, chains, L, M))[0]
     assert "(exchange)" in line and int(field(line, r"segments of (\d+) rows")) == 256, line
+
+
+@pytest.mark.parametrize("chains,L,E,M", [(8, 989, 75, 10), (9, 1681, 120, 31), (3, 5154, 75, 10), (4, 4000, 99, 101),
+                                          (32, 989, 120, 31)])
+def test_two_odd_shapes_stay_in_one_launch(chains, L, E, M):
+    """The length of an exchange's segments does not decide whether scans of two odd shapes share a launch (two took 1.1
+    to 1.3 times as long, or left dQ and dK 1.5 times as far from float64)."""
+    got = lines((1, chains, L, E), (1, chains, L, M), backward=True)
+    assert len(got) == 1 and kernel(got[0]).startswith("scan_tp_kernel") and "3 scans" in got[0], got
