@@ -419,13 +419,22 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     }
     if (!single) {
         if (D <= 32 && F <= 32) {
-            // (bf16 results, rounds of 256 workgroups: seven tenths full, or short or few enough for an exchange.  us, split L /
-            // here: 64 chains, L=4128 124 / 86, 85 chains 144 / 91 and L=16384 448 / 305, but 86 chains 469 / 549;
-            // 160 chains, L=8192 417 / 312, but 112 chains 302 / 303; 40 chains, L=6000 125 / 110, 20 chains, L=11000
-            // 127 / 106, 32 chains, L=11000 157 / 173)
-            if (bf16_results && chunks > 128 && chunks <= 1024)
-                return units > 48 && units * 10 < (units + 255) / 256 * 1792 && !(units <= 256 && chunks <= 192) &&
-                       !(units <= 60 && chunks <= 512) && !(units <= 84 && chunks <= 344);
+            // (bf16 results: whole chains take a time per round of 256 workgroups, split L a time per chain, so whole ones
+            // where the rounds are 70 to 77 % full on average, or where chains are short or few enough for an exchange.
+            // us, split L / here: 64 chains, L=4128 124 / 86, 85 chains, L=16384 448 / 305, but 86 chains 469 / 549, and 60
+            // chains, L=7000 144 / 127, but L=14385 248 / 254; two rounds: 128 chains, L=4128 163 / 150, L=8192 284 / 287, 120
+            // chains 274 / 288, L=14385 517 / 498; three: 180 chains, L=5154 261 / 271, L=8192 426 / 422, 200 chains 278 /
+            // 273 and 460 / 427; 40 chains, L=6000 113 / 98, 20 chains, L=11000 116 / 92, 32 chains, L=11000 157 / 173)
+            if (bf16_results && chunks > 128 && chunks <= 1024) {
+                const int64_t rounds = (units + 255) / 256;
+                const int64_t least = rounds == 1   ? (chunks > 320 ? 72 : 70)
+                                      : rounds == 2 ? (chunks > 344 ? 70 : 75)
+                                                    : (chunks > 224 ? 70 : 77);
+                const bool full = 100 * units >= rounds * 256 * least;
+                const bool brief = units <= 256 && chunks <= 192;
+                const bool few = units <= 48 || (units <= 60 && chunks <= 512) || (units <= 84 && chunks <= 344);
+                return !full && !brief && !few;
+            }
             if (chunks > 128) return units > (chunks > 1024 ? 24 : 48);
             return chunks <= 64 && units > (chunks <= 4 ? 1024 : chunks <= 8 ? 1100 : 1536);
         }

@@ -449,3 +449,10 @@ def test_two_odd_shapes_stay_in_one_launch(chains, L, E, M):
     to 1.3 times as long, or left dQ and dK 1.5 times as far from float64)."""
     got = lines((1, chains, L, E), (1, chains, L, M), backward=True)
     assert len(got) == 1 and kernel(got[0]).startswith("scan_tp_kernel") and "3 scans" in got[0], got
+
+
+@pytest.mark.parametrize("chains,L", [(120, 8192), (124, 7000), (180, 5154), (186, 4128)])
+def test_narrow_backward_scans_of_bf16_rows_split_where_the_rounds_are_not_full(chains, L):
+    """Rounds of workgroups seven tenths full, which whole chains of this length take 1.02 to 1.05 times as long over."""
+    got = lines((1, chains, L, 32), (1, chains, L, 32), backward=True, dtype=_native.FTC_BF16)
+    assert kernel(got[0]) == "scan_mfma_kernel"
