@@ -469,14 +469,36 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
     }
     if (chunks <= 24) return units > 512;
     if (chunks <= 48) return units < 48 || (units > 512 && (bf16_results || (D <= 32 && units < 900)));
-    // (forward, 4 to 512 chains of 1600 to 32768 positions, us with inputs from memory, split L / here.  32 x 32: 96 chains,
-    // L=1600 35.0 / 33.6, but 80 29 / 31; 128, L=2600 57 / 50; 160, L=4128 97 / 78, L=8192 171 / 142, but 120 140 / 142, and 136 84 / 76
-    // and 150 / 136, which is 62 / 68 with inputs left in the caches.  64 x 32: 80 chains, L=2600 57 / 52, but 64 47 / 48; 48, L=6000
-    // 77 / 66; 152, L=8192 241 / 173; 24, L=11000 78 / 64; 448, L=11000 712 / 690.  Errors against float64 0.25 to 0.79 of theirs)
-    if (chunks > 256) return D <= 32 || bf16_results || units < (chunks <= 320 ? 48 : 24) || units > 512;
-    if (bf16_results) return units < (D <= 32 ? (chunks <= 72 ? 176 : 224) : chunks <= 96 ? 112 : 176) || units > 512;
-    if (D <= 32) return units < (chunks <= 56 ? 96 : chunks <= 88 ? 128 : 160);
-    return units < (chunks <= 72 ? 64 : chunks <= 160 ? 80 : 48);
+    if (bf16_results) return chunks > 256 || units < (D <= 32 ? (chunks <= 72 ? 176 : 224) : chunks <= 96 ? 112 : 176) || units > 512;
+    // Forward, measured on 24 to 512 chains of 1600 to 32768 positions, with inputs from memory and with inputs that the
+    // kernel before left in the caches (us, split L / here, the latter in parentheses).  Where all rows fit the Infinity Cache
+    // split L reads them faster from there, and the lines are where both ways meet; else memory bounds split L.
+    const bool cached = units * chunks * (int64_t)(kChunk * (4 * D + 6 * F)) <= (int64_t)256 << 20;
+    if (D <= 32) {
+        // Two segments a chain on up to 128 chains: 96 chains, L=1600 27.6 / 26.4 (25.1 / 22.7), 128, L=2500 43.9 / 40.4
+        // (35.1 / 32.3).  Whole chains on more: 144, L=1600 34.4 / 29.8 (29.0 / 28.8), but 160, L=2500 51 / 44 (37.8 / 42.9);
+        // 208, L=2900 72 / 50 (49.3 / 48.3), but 192 71 / 55 (46.0 / 48.5).  Beyond the caches 160, L=6000 107 / 96 (98 / 96),
+        // L=8192 133 / 128, 208, L=4700 116 / 79 (106 / 78).  Longer ones are not walked whole.
+        if (chunks > 256) return true;
+        if (units <= 128) return units < (chunks <= 56 ? 96 : chunks <= 88 ? 128 : INT64_MAX);
+        return units < (!cached ? 160 : chunks <= 56 ? 144 : chunks <= 72 ? 176 : 208);
+    }
+    // 64 rows.  Cut up to 128 chunks: 80 chains, L=2500 43.3 / 38.5 (36.4 / 31.5), 128, L=3778 83 / 63 (66 / 54); whole: 152, L=4000
+    // 102 / 82 (93 / 81), but 136, L=3778 88 / 78 (70 / 77).
+    if (chunks <= 72) return units < 64;
+    if (chunks <= 128) return units < 80 || (chunks > 96 && units > 128 && units < 152);
+    // Whole up to 256 chunks, on more than 128 chains: 152, L=5154 122 / 104, 136, L=6000 124 / 120.
+    if (units >= 160 && chunks <= 256) return false;
+    if (units > 128 && chunks <= 256) return cached;
+    // With an exchange where the segments of all chains fill a round of 256 workgroups, two for more than 128 chains, to
+    // seven eighths: 120, L=6000 126 / 113, 64, L=16384 153 / 135, 160, L=11000 254 / 244; but 96, L=9000 134 / 144, 136, L=8224
+    // 165 / 188, 200 233 / 252 (within 1.03 elsewhere: 112, L=20000 322 / 332).  In the caches few long chains gain either way
+    // (28, L=11000 65 / 59 (53 / 52)), five segments on 48 to 51 where rows come from memory, L=6000 59 / 55 (47 / 51); more
+    // stay, 64 71 / 66 (57 / 60), 80 85 / 79 (66 / 73).
+    const int64_t room = units <= 128 ? 256 : 512, groups = units * (room / units);
+    if (units > 512 || 8 * groups < 7 * room) return true;
+    if (!cached) return units < (chunks <= 320 ? 48 : 24);
+    return chunks > 320 ? units < 24 || units > 32 : chunks <= 160 || units < 48 || units > 51;
 }
 
 // The plan of scans with bf16 rows among them on the chain-parallel kernel (three pieces for the state and

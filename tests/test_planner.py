@@ -456,3 +456,12 @@ def test_narrow_backward_scans_of_bf16_rows_split_where_the_rounds_are_not_full(
     """Rounds of workgroups seven tenths full, which whole chains of this length take 1.02 to 1.05 times as long over."""
     got = lines((1, chains, L, 32), (1, chains, L, 32), backward=True, dtype=_native.FTC_BF16)
     assert kernel(got[0]) == "scan_mfma_kernel"
+
+
+@pytest.mark.parametrize("chains,L,D", [(160, 2500, 32), (176, 3200, 32), (192, 3778, 32), (136, 3778, 64), (80, 6000, 64),
+                                        (96, 9000, 64), (136, 8224, 64), (200, 9000, 64)])
+def test_forward_scans_of_bf16_rows_with_32_columns_that_split(chains, L, D):
+    """Where the rows fit the caches and a round of workgroups is not full, or an exchange leaves its rounds a quarter
+    empty: 1.06 to 1.24 times as long on the chain-parallel kernel."""
+    got = lines((1, chains, L, D), (1, chains, L, 32), dtype=_native.FTC_BF16)
+    assert kernel(got[0]) == "scan_mfma_kernel"
