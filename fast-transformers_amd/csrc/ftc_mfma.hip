@@ -251,7 +251,8 @@ int tp_exchange_segments(int64_t units, int64_t L, bool wide, int64_t most_fours
     // 27.9; 25 x 33, 28 chains, L=1100 23.3 / 25.0; 48 x 48 backward, 9, L=1100 24.1 / 25.3; from 110 calls on either
     // side of the line 0.88 to 0.97 of the time below it, 1.00 to 1.06 above); several scans of such a state on
     // three bf16 pieces 240 (32 x 64 backward, 6 chains, L=1600, 234 of them 0.99, 2, L=5154, 246 1.05); wider ones any number
-    // (128 x 128, 8 chains, L=4000 0.89, 245 of 250 calls 0.73 to 0.93).
+    // (128 x 128, 8 chains, L=4000 0.89, 245 of 250 calls 0.73 to 0.93), and fused attention as well, whose chunks take
+    // longer (8 chains, L=3111, 200 of them 31.2 / 28.5, 12, L=2335, 228 32.0 / 29.7).
     const int64_t fours = (total_chunks + 3) / 4;
     want = std::min<int64_t>(want, units * fours <= most_fours ? fours : total_chunks / 4);
     if (tuning().tpx_segs >= 0) want = std::max(1, tuning().tpx_segs);  // tuning aid
@@ -271,7 +272,7 @@ int tp_exchange_segments(int64_t units, int64_t L, bool wide, int64_t most_fours
 // cut into *nseg segments that need no exchange; both 0: another kernel takes the launch.
 // (fp32 rows; those with bf16 among them have a plan of their own, mixed_plan_compute)
 void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg,
-                     int *seg_chunks, bool forced, bool odd) {
+                     int *seg_chunks, bool forced, bool odd, bool normed) {
     *nseg = *seg_chunks = 0;
     if (!tp_widths(D, F, forced, odd)) return;
     const bool wide = D != 64 || F != 64 || forced || odd;
@@ -337,7 +338,7 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // backward, 256 chains, L=12000: 1404 against 1825)
     const bool walk_long = D <= 64 && !(odd && forced) && L > 256 * kChunk && L <= 1024 * kChunk &&
                            units >= (!wide ? 112 : L > 512 * kChunk ? 128 : 192);
-    const int64_t most_fours = D > 64 ? INT64_MAX : forced && nscans > 1 ? 240 : 192;
+    const int64_t most_fours = D > 64 || normed ? INT64_MAX : forced && nscans > 1 ? 240 : 192;
     if (!narrow && !walk_long) *seg_chunks = tp_exchange_segments(units, L, wide, most_fours, nseg);
     // fp32 rows, 64 x 64: any number of chains of 16 chunks or more (the fp16-piece kernel walks
     // them faster than the kernels that split L stream them: backward, 256 chains, L=4096: 528
@@ -617,12 +618,12 @@ struct TpPlan {
     int nseg, seg_chunks;
 };
 void tp_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *nseg, int *seg_chunks,
-             bool forced = false, bool odd = false) {
+             bool forced = false, bool odd = false, bool normed = false) {
     static thread_local PlanMemo<TpPlan> memo;
-    const int64_t key[8] = {D, F, chains, nscans, L, forced ? 1 : 0, odd ? 1 : 0, 0};
+    const int64_t key[8] = {D, F, chains, nscans, L, forced ? 1 : 0, odd ? 1 : 0, normed ? 1 : 0};
     const TpPlan pl = memo.get(key, [&]() {
         TpPlan p;
-        tp_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks, forced, odd);
+        tp_plan_compute(D, F, chains, nscans, L, &p.nseg, &p.seg_chunks, forced, odd, normed);
         return p;
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
@@ -918,12 +919,12 @@ int64_t fused_tp_state_rows(int64_t D) { return (D + 63) / 64 * 64 + 64; }
 bool fused_tp_plan(int64_t D, int64_t F, int64_t chains, int64_t L, int *nseg, int *seg_chunks) {
     *nseg = *seg_chunks = 0;
     if (fused_wide(D, F)) {
-        tp_plan(D, F, chains, 1, L, nseg, seg_chunks, true);
+        tp_plan(D, F, chains, 1, L, nseg, seg_chunks, true, false, true);
         return *nseg > 0;
     }
     if (tuning().wg > 0) return false;
     const int64_t chunks = (L + kChunk - 1) / kChunk;
-    tp_plan(64, 64, chains, 1, L, nseg, seg_chunks);
+    tp_plan(64, 64, chains, 1, L, nseg, seg_chunks, false, false, true);
     if (*nseg > 0 && *seg_chunks == 0 && chunks > 256) *nseg = 0;
     if (*nseg == 0 || tuning().wg == 0) return *nseg > 0;  // (FTC_WG=0: tuning aid)
     // the fewest chains without an exchange, where the two cross

@@ -465,3 +465,13 @@ def test_forward_scans_of_bf16_rows_with_32_columns_that_split(chains, L, D):
     empty: 1.06 to 1.24 times as long on the chain-parallel kernel."""
     got = lines((1, chains, L, D), (1, chains, L, 32), dtype=_native.FTC_BF16)
     assert kernel(got[0]) == "scan_mfma_kernel"
+
+
+@pytest.mark.parametrize("chains,L", [(8, 3140), (10, 2490), (12, 2360), (12, 2650)])
+def test_fused_attention_exchanges_in_segments_of_four_chunks(chains, L):
+    """Up to a whole round of workgroups (the limit of plain scans made them eight: 1.02 to 1.04 times as long as before
+    those chains exchanged at all).  Two states of 128 x 16 values for each of the four consumers of every segment."""
+    fours = -(-L // 128)
+    assert 192 < chains * fours <= 256
+    need = _native.load().ftc_causal_linear_attention_workspace_bytes(1, chains, L, 64, 64, 0)
+    assert need >= 2 * 4 * chains * fours * 128 * 16 * 4
