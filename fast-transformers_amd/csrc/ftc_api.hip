@@ -973,7 +973,8 @@ int run_scans(const ScanDesc *scans, int n, int64_t N, int64_t H, int64_t L, voi
         if (!mfma_tp_takes(group, ngroup, N, H, L)) continue;
         // (bf16 rows: an exchange that the workspace has no room for is left to the other kernels)
         if (group[0].a.dtype != FTC_F32 || group[0].b.dtype != FTC_F32) {
-            const int64_t need = mfma_tp_mixed_workspace_bytes(N, H, L, group[0].a.width, group[0].v.width, ngroup);
+            const int64_t need = mfma_tp_mixed_workspace_bytes(N, H, L, group[0].a.width, group[0].v.width, ngroup,
+                                                               has_state(group, ngroup));
             if (need > 0 && !plan_only() && (int64_t)workspace_bytes < need) continue;
         }
         const int rc = mfma_scan(group, ngroup, N, H, L, workspace, workspace_bytes, stream);

@@ -144,7 +144,10 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
 int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans,
                                 bool forced = false, bool odd = false);
 // ... and of scans with bf16 rows among them
-int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans);
+int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans,
+                                      bool may_have_state = true);
+// whether a state is handed in or out
+bool has_state(const ScanDesc *scans, int nscans);
 // blocks of 64 output columns of several scans
 int64_t column_blocks(const ScanDesc *scans, int nscans);
 // estimated time of an `odd` launch, in chunks walked one after the other

@@ -510,13 +510,24 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
 // exchange 1.55 times as long, and the exchange what a round's workgroups wait for each other.
 // Chains are walked whole up to 256 chunks, and up to 1024 where the results are bf16, which makes the
 // rounding of a long running state a non-issue.
-void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, bool bf16_results, int *nseg,
-                        int *seg_chunks) {
+// `stateful`: a state is handed in or out.
+void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, bool bf16_results, bool stateful,
+                        int *nseg, int *seg_chunks) {
     *nseg = *seg_chunks = 0;
     if (!tp_widths(D, F) || tuning().tp == 0) return;
     const int64_t units = chains * nscans * tp_fblocks(F), chunks = (L + kChunk - 1) / kChunk;
     // (FTC_TP=1, FTC_TPX=0: tuning aids)
     if (tuning().tp < 0 && mixed_splits(D, F, units, nscans, chunks, bf16_results)) return;
+    // A state that a few chains of 9 or 13 chunks hand out: the kernels that split L add it up in sums of a few chunks, a
+    // chain walked whole in one, which leaves it 1.05 times as far from float64 (0.99 at 10 to 12 chunks, where they
+    // have longer sums).  Sums of four chunks, exchanged, leave it 0.96 times as far, and the rows 0.53 times either way.
+    // 128 x 128, us, split L / exchanged / whole: 1 chain, L=270 20.2 / 16.4 / 12.8, 4, L=400 23 / 17.9 / 15.2.
+    if (stateful && nscans == 1 && D > 96 && F > 32 && (chunks == 9 || chunks == 13) && units < 16 && tuning().tp < 0 &&
+        tuning().tpx != 0 && mfma_scan_supported_widths(D, F)) {
+        *seg_chunks = kTpAhead;
+        *nseg = (int)((chunks + kTpAhead - 1) / kTpAhead);
+        return;
+    }
     const double chunk_us = (D <= 32 ? 0.48 : D <= 64 ? 0.65 : D <= 96 ? 0.98 : 1.12) * (bf16_results ? 1.25 : 1.0);
     double least = 1e30;
     if (chunks <= (bf16_results ? 1024 : 256)) {
@@ -628,13 +639,13 @@ void tp_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, int *n
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
 }
-void mixed_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, bool bf16_results, int *nseg,
+void mixed_plan(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L, bool bf16_results, bool stateful, int *nseg,
                 int *seg_chunks) {
     static thread_local PlanMemo<TpPlan> memo;
-    const int64_t key[8] = {D, F, chains, nscans, L, bf16_results ? 1 : 0, 0, 0};
+    const int64_t key[8] = {D, F, chains, nscans, L, bf16_results ? 1 : 0, stateful ? 1 : 0, 0};
     const TpPlan pl = memo.get(key, [&]() {
         TpPlan p;
-        mixed_plan_compute(D, F, chains, nscans, L, bf16_results, &p.nseg, &p.seg_chunks);
+        mixed_plan_compute(D, F, chains, nscans, L, bf16_results, stateful, &p.nseg, &p.seg_chunks);
         return p;
     });
     *nseg = pl.nseg, *seg_chunks = pl.seg_chunks;
@@ -760,6 +771,12 @@ bool mfma_scan_clips(int64_t D, int64_t F, int nscans, int64_t L) {
     return D <= 64 && mfma_slice_widths(D, F, widths) == 1 && tuning().dma != 0 && !use_wg_kernel(D, F, nscans, L, true);
 }
 
+bool has_state(const ScanDesc *scans, int nscans) {
+    for (int i = 0; i < nscans; i++)
+        if (scans[i].initial.ptr || scans[i].final_.ptr) return true;
+    return false;
+}
+
 // the widest rows of a launch (they differ between scans only where `odd` allows it)
 void widest_rows(const ScanDesc *scans, int nscans, int *D, int *F) {
     *D = *F = 0;
@@ -781,12 +798,12 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     if (!tp_widths(D, F, forced, odd)) return false;
     if (odd && !forced && !tph_takes_rows(D)) return false;
     int64_t widest_stride = 0;
-    bool mixed = false, stateful = false;
+    const bool stateful = has_state(scans, nscans);
+    bool mixed = false;
     for (int i = 0; i < nscans; i++) {
         const ScanDesc &sd = scans[i];
         const Combo combo = combo_of(sd);
         mixed = mixed || combo != kFFFF;
-        stateful = stateful || sd.initial.ptr || sd.final_.ptr;
         // (rows with bf16 among them: not as parts of wider scans, whose results are added up in fp32)
         if (combo == kNone || (combo != kFFFF && (forced || tuning().tph == 0))) return false;
         // (odd widths: scans of any widths side by side, where pieces are scaled as long as none has a
@@ -815,14 +832,18 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     // (fp32 states of more than 64 rows that are handed in or out stay with the kernels that split L, whose sums are
     // shorter, where those have no more than the 9 to 23 chunks of few chains to walk: 128 x 128, 8 chains, L=400 39.0 us
     // for 22.1, but the state is 1.25e-7 from float64 there and 3.5e-7 here; the rows are 1.9e-7 and 1.3e-7.
-    // Those that are only handed in as well: rows are the same whether the state is asked for or not)
+    // Those that are only handed in as well: rows are the same whether the state is asked for or not.
+    // So do bf16 rows with 65 to 96 state rows over 9, 12 and 13 chunks: 96 x 96, 1 to 7 chains, 9 and 13 the state 1.05
+    // times as far, 12 13.6 us for 14.7; see mixed_plan_compute)
     const int64_t chunks = (L + kChunk - 1) / kChunk, units = chains * tp_fblocks(F);
-    if (stateful && !mixed && !forced && !odd && nscans == 1 && D > 64 && F > 32 && chunks > 8 && chunks < 24 &&
-        units * std::max<int64_t>(1, std::min<int64_t>(4, 256 / units)) < 128 && tuning().tp < 0 &&
-        mfma_scan_supported_widths(D, F))
-        return false;
+    if (stateful && !forced && !odd && nscans == 1 && D > 64 && F > 32 && chunks > 8 && tuning().tp < 0 &&
+        mfma_scan_supported_widths(D, F)) {
+        if (mixed ? D <= 96 && units < 16 && (chunks == 9 || chunks == 12 || chunks == 13)
+                  : chunks < 24 && units * std::max<int64_t>(1, std::min<int64_t>(4, 256 / units)) < 128)
+            return false;
+    }
     if (mixed)
-        mixed_plan(D, F, chains, nscans, L, scans[0].out.dtype != FTC_F32, &nseg, &seg_chunks);
+        mixed_plan(D, F, chains, nscans, L, scans[0].out.dtype != FTC_F32, stateful, &nseg, &seg_chunks);
     else if (odd && forced)
         tp_plan(D, 64, chains, (int)column_blocks(scans, nscans), L, &nseg, &seg_chunks, forced, odd);
     else
@@ -830,15 +851,17 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     return nseg > 0;
 }
 
-int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans) {
+int64_t mfma_tp_mixed_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int64_t F, int nscans,
+                                      bool may_have_state) {
     const int64_t chains = std::max<int64_t>(1, N * H);
     int64_t bytes = 0;
-    for (const bool bf16_results : {false, true}) {
-        int nseg = 0, seg_chunks = 0;
-        mixed_plan(D, F, chains, nscans, L, bf16_results, &nseg, &seg_chunks);
-        if (seg_chunks > 0)
-            bytes = std::max(bytes, tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D));
-    }
+    for (const bool bf16_results : {false, true})
+        for (const bool stateful : {false, may_have_state}) {
+            int nseg = 0, seg_chunks = 0;
+            mixed_plan(D, F, chains, nscans, L, bf16_results, stateful, &nseg, &seg_chunks);
+            if (seg_chunks > 0)
+                bytes = std::max(bytes, tp_exchange_workspace_bytes(chains * nscans * tp_fblocks(F), nseg, D));
+        }
     return bytes;
 }
 
@@ -1027,7 +1050,8 @@ int mfma_scan(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int64_t L
     if (fused_tp && tpx_seg_chunks == 0) tp_nseg = tpx_nseg, tpx_nseg = 0;
     if (tp_shape) {
         if (combo != kFFFF)
-            mixed_plan(D, F, chains, nscans, L, scans[0].out.dtype != FTC_F32, &tpx_nseg, &tpx_seg_chunks);
+            mixed_plan(D, F, chains, nscans, L, scans[0].out.dtype != FTC_F32, has_state(scans, nscans), &tpx_nseg,
+                       &tpx_seg_chunks);
         else if (odd && forced)
             tp_plan(D, 64, chains, (int)blocks, L, &tpx_nseg, &tpx_seg_chunks, forced, odd);
         else

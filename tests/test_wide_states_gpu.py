@@ -134,3 +134,32 @@ def test_short_chains_of_wide_states(shape, dtype):
     final = S.double() + K.double().transpose(2, 3).contiguous() @ V.double()
     assert scale_error(state.cpu(), final) <= 2e-6
     assert torch.equal(out, cp.causal_dot_product_with_state(q, k, v, S.cuda())[0])
+
+
+@pytest.mark.parametrize("widths", [(128, 128), (128, 64)], ids=lambda s: "e%d_m%d" % s)
+@pytest.mark.parametrize("L", [257, 270, 288, 385, 390, 400])
+def test_states_of_a_short_bf16_prefill(widths, L):
+    """The state that a few chains of 9 or 13 chunks hand out is a sum of sums of four chunks, not one running sum: no
+    further from float64 than such sums, rounded after every 16 products as the matrix instructions add them, come out."""
+    import fast_transformers_amd.causal_product as cp
+    (E, M), C = widths, 6
+    gen = torch.Generator().manual_seed(L)
+    Q, K = ((torch.nn.functional.elu(torch.randn(1, C, L, E, generator=gen)) + 1).bfloat16() for _ in range(2))
+    V = torch.randn(1, C, L, M, generator=gen).bfloat16()
+    S = 20 * torch.randn(1, C, E, M, generator=gen)
+    out, state = cp.causal_dot_product_with_state(Q.cuda(), K.cuda(), V.cuda(), S.cuda())
+    K64, V64 = K.double(), V.double()
+    final = S.double() + K64.transpose(2, 3).contiguous() @ V64
+    total = S.clone()
+    for first in range(0, L, 128):
+        part = torch.zeros_like(total)
+        for at in range(first, min(first + 128, L), 16):
+            k, v = (t[:, :, at:min(at + 16, L)] for t in (K64, V64))
+            part = (part.double() + k.transpose(2, 3).contiguous() @ v).float()
+        total = total + part
+    error = lambda t: ((t.double() - final).norm() / final.norm()).item()
+    # (a running sum: 1.07 times; sums of the same products in another order within 1.02)
+    assert error(state.cpu()) <= 1.05 * error(total)
+    exact = oracle.forward(Q.double(), K64, V64) + Q.double() @ S.double()
+    plain = oracle.forward(Q.float(), K.float(), V.float()) + Q.float() @ S
+    assert scale_error(out.cpu(), exact) <= max(4 * scale_error(plain, exact), 2e-6)
