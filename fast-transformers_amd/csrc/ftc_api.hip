@@ -434,7 +434,7 @@ bool clipped_copies(const ScanDesc *scans, int n, const bool *take, int64_t N, i
         sc.out = OperandOut{nullptr, H * L * F, L * F, F, FTC_F32, (int32_t)F};
         group[ngroup++] = sc;
     }
-    if (ngroup == 0 || D > 64 || (D == 32 && F == 32) || !mfma_scan_clips(D, F, ngroup, L)) return false;
+    if (ngroup == 0 || !mfma_scan_clips(D, F, ngroup, L)) return false;
     return !short_scans_take(group, ngroup, N, H, L) && !mfma_tp_takes(group, ngroup, N, H, L);
 }
 

@@ -768,7 +768,8 @@ int64_t mfma_tp_workspace_bytes(int64_t N, int64_t H, int64_t L, int64_t D, int6
 
 bool mfma_scan_clips(int64_t D, int64_t F, int nscans, int64_t L) {
     int widths[kMfmaMaxSlices];
-    return D <= 64 && mfma_slice_widths(D, F, widths) == 1 && tuning().dma != 0 && !use_wg_kernel(D, F, nscans, L, true);
+    return D <= 64 && !(D == 32 && F == 32) && mfma_slice_widths(D, F, widths) == 1 && tuning().dma != 0 &&
+           !use_wg_kernel(D, F, nscans, L, true);
 }
 
 bool has_state(const ScanDesc *scans, int nscans) {

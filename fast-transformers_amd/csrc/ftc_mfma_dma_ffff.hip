@@ -4,14 +4,17 @@
 
 namespace ftc {
 namespace mfma {
-#define FTC_INSTANTIATE(DD, FF) \
-    template __global__ void scan_dma_kernel<DD, FF, float, float, float, float, false>(uint32_t *, ScanArgs); \
-    template __global__ void scan_dma_kernel<DD, FF, float, float, float, float, true>(uint32_t *, ScanArgs)
-FTC_INSTANTIATE(64, 64);
-FTC_INSTANTIATE(32, 128);
-FTC_INSTANTIATE(32, 32);
-FTC_INSTANTIATE(32, 64);
-FTC_INSTANTIATE(64, 32);
+#define FTC_INSTANTIATE(DD, FF, CLIP) \
+    template __global__ void scan_dma_kernel<DD, FF, float, float, float, float, CLIP>(uint32_t *, ScanArgs)
+FTC_INSTANTIATE(64, 64, false);
+FTC_INSTANTIATE(32, 128, false);
+FTC_INSTANTIATE(32, 32, false);
+FTC_INSTANTIATE(32, 64, false);
+FTC_INSTANTIATE(64, 32, false);
+FTC_INSTANTIATE(64, 64, true);
+FTC_INSTANTIATE(32, 128, true);
+FTC_INSTANTIATE(32, 64, true);
+FTC_INSTANTIATE(64, 32, true);
 #undef FTC_INSTANTIATE
 
 void launch_scan_dma_ffff(int D, int F, void *ws, const ScanArgs &args, hipStream_t stream, bool clipped) {

@@ -435,7 +435,7 @@ void launch_scan_dma(int D, int F, void *workspace, const ScanArgs &args, hipStr
 #undef FTC_LAUNCH
 }
 
-// the same with rows that do not fill the tiles (CLIP)
+// the same with rows that do not fill the tiles (CLIP; the shapes of mfma_scan_clips)
 template <typename T>
 void launch_scan_dma_clipped(int D, int F, void *workspace, const ScanArgs &args, hipStream_t stream) {
     const dim3 grid((unsigned)args.total_waves), block(kWave);
@@ -444,7 +444,6 @@ void launch_scan_dma_clipped(int D, int F, void *workspace, const ScanArgs &args
                        (uint32_t *)workspace, args)
     if (D == 64 && F == 64) FTC_LAUNCH(64, 64);
     else if (D == 32 && F == 128) FTC_LAUNCH(32, 128);
-    else if (D == 32 && F == 32) FTC_LAUNCH(32, 32);
     else if (D == 32 && F == 64) FTC_LAUNCH(32, 64);
     else FTC_LAUNCH(64, 32);
 #undef FTC_LAUNCH
