@@ -46,6 +46,11 @@ bool mfma_scan_supported_widths(int64_t D, int64_t F) {
     return mfma_slice_widths(D, F, widths) > 0;
 }
 
+// segments that a chain may be cut into without an exchange: as many as one round of workgroups has room for, up to four
+int64_t round_segments(int64_t units) { return std::max<int64_t>(1, std::min<int64_t>(4, 256 / units)); }
+// ... which have to fill half the GPU where other kernels take the widths as well
+constexpr int64_t kHalfTheGpu = 128;
+
 // all-fp32 scans can run one workgroup per chain (and block of 64 output columns) with no
 // split of L (ftc_tp_kernel.h).  `units`: chains x scans x column blocks; `wide`: a state
 // other than 64 x 64, for which the kernels that split L are half as fast as for 64 x 64;
@@ -62,7 +67,7 @@ int tp_kernel_segments(int64_t units, int64_t L, bool wide, bool others, bool lo
     // workgroups each rebuild the state before their segment by themselves (a state-only
     // chunk costs a bit more than half of a full one), as long as that fills at least half the GPU.
     const int64_t total_chunks = (L + kChunk - 1) / kChunk;
-    int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), total_chunks));
+    int nseg = (int)std::max<int64_t>(1, std::min(round_segments(units), total_chunks));
     if (tuning().tp_segs >= 0) nseg = std::max(1, std::min(tuning().tp_segs, 16));  // tuning aid
     if (tuning().tp >= 0) return tuning().tp != 0 ? nseg : 0;                       // tuning aid
     // Measured (forward, us, N=10 H=8): cfg2 (L=1000) 30 against 42 for the kernels that split
@@ -81,10 +86,10 @@ int tp_kernel_segments(int64_t units, int64_t L, bool wide, bool others, bool lo
     // H=8, L=2048, 128 x 128 forward: 52 against 91 us.  The VALU kernel loses always.)
     // (chains of up to `brief_chunks` chunks at any number, see tp_plan_compute)
     const bool brief = total_chunks <= brief_chunks;
-    if (wide) return !others || brief || units * nseg >= 128 ? nseg : 0;
+    if (wide) return !others || brief || units * nseg >= kHalfTheGpu ? nseg : 0;
     // Beyond `most_units` workgroups the other kernels win again (short chains: there every
     // chain has its own wavefront, all resident at once, and nothing is split either).
-    return (brief || units * nseg >= (long_chains ? 112 : 128)) && units <= most_units ? nseg : 0;
+    return (brief || units * nseg >= (long_chains ? 112 : kHalfTheGpu)) && units <= most_units ? nseg : 0;
 }
 
 // Plans depend on the sizes alone and a caller repeats the same sizes call after call (the
@@ -536,7 +541,7 @@ void mixed_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_
         // launches in 0.95 of their time, but their sums run over longer segments, 1.08e-7 from float64 for
         // 1.00e-7; backward calls would take 1.03 times as long)
         int32_t start[kMaxTpSegments + 1];
-        int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, 256 / units), chunks)) : 1;
+        int n = chunks <= 128 ? (int)std::max<int64_t>(1, std::min(round_segments(units), chunks)) : 1;
         n = tp_segment_starts(chunks, n, start, kTpAhead, 0.6);
         double longest = (double)chunks;
         if (n > 1) {
@@ -831,7 +836,7 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     int nseg = 0, seg_chunks = 0;
     const int64_t chains = std::max<int64_t>(1, N * H);
     // (fp32 states of more than 64 rows that are handed in or out stay with the kernels that split L, whose sums are
-    // shorter, where those have no more than the 9 to 23 chunks of few chains to walk: 128 x 128, 8 chains, L=400 39.0 us
+    // shorter, over 9 to 23 chunks where the chains' segments do not fill half the GPU: 128 x 128, 8 chains, L=400 39.0 us
     // for 22.1, but the state is 1.25e-7 from float64 there and 3.5e-7 here; the rows are 1.9e-7 and 1.3e-7.
     // Those that are only handed in as well: rows are the same whether the state is asked for or not.
     // So do bf16 rows with 65 to 96 state rows over 9, 12 and 13 chunks: 96 x 96, 1 to 7 chains, 9 and 13 the state 1.05
@@ -840,7 +845,7 @@ bool mfma_tp_takes(const ScanDesc *scans, int nscans, int64_t N, int64_t H, int6
     if (stateful && !forced && !odd && nscans == 1 && D > 64 && F > 32 && chunks > 8 && tuning().tp < 0 &&
         mfma_scan_supported_widths(D, F)) {
         if (mixed ? D <= 96 && units < 16 && (chunks == 9 || chunks == 12 || chunks == 13)
-                  : chunks < 24 && units * std::max<int64_t>(1, std::min<int64_t>(4, 256 / units)) < 128)
+                  : chunks < 24 && units * round_segments(units) < kHalfTheGpu)
             return false;
     }
     if (mixed)
