@@ -474,3 +474,73 @@ def test_encoder_whose_width_is_not_that_of_its_heads(sizes, final):
     assert calls == [1]
     # two fp32 evaluations, as above
     assert (got - want).abs().max() <= 4e-6 * layers * want.abs().max()
+
+
+@pytest.mark.parametrize("kind", ["plain", "residual", "norm", "relu"])
+@pytest.mark.parametrize("shape", [
+    # products of more than 176 MB, whose rows leave in whole lines past the caches: rows that are added on the two
+    # largest tiles, features that end inside a line, too few steps for rows to leave under the next tile
+    (26000, 512, 676), (45003, 512, 512), (60011, 256, 544), (31000, 1024, 352)], ids=lambda s: "t%d_k%d_f%d" % s)
+def test_streamed_rows(shape, kind):
+    """Rows that are streamed are bit for bit those of products too small for it, also over the rows that they add."""
+    from fast_transformers_amd import _native
+    lib = _native.load()
+    T, K, F = shape
+    relu, adds = kind == "relu", kind in ("residual", "norm")
+    if relu:
+        F = F // 32 * 32
+    assert 4 * T * (K + (2 if adds else 1) * F) >= 176 << 20 or not adds
+    gen = torch.Generator(device="cuda").manual_seed(T + F)
+    x, w, b, r = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, K), (F, K), (F,), (T, F)))
+    gamma, beta = torch.randn(F, device="cuda", generator=gen), torch.randn(F, device="cuda", generator=gen)
+    new = lambda *s: torch.full(s, float("nan"), device="cuda")
+    n = lambda i: ctypes.c_int64(i)
+    xp, xs, wp, ws, bo, wn = new(T, K), new(T), new(F, K), new(F), new(F), new(F)
+    item = Weight(w.data_ptr(), b.data_ptr(), F, K, wp.data_ptr(), ws.data_ptr(), bo.data_ptr(), wn.data_ptr())
+    assert lib.ftc_split_weights(ctypes.byref(item), 1, stream()) == 0, _native.last_error()
+    assert lib.ftc_split_rows(ptr(x), n(T), n(K), ptr(xp), ptr(xs), stream()) == 0
+    stats = torch.stack((r.mean(1), 1 / r.std(1)), 1).contiguous()   # (any two numbers a row will do)
+
+    def run(first, last, out, scale):
+        rows, at = n(last - first), slice(first, last)
+        if kind == "norm":
+            rc = lib.ftc_linear_split_normed(ptr(xp[at]), ptr(xs[at]), rows, ptr(wp), ptr(ws), ptr(bo), n(F), n(K),
+                                             ptr(r[at]), ptr(stats[at]), ptr(gamma), ptr(beta), ptr(out), stream())
+        else:
+            rc = lib.ftc_linear_split(ptr(xp[at]), ptr(xs[at]), rows, ptr(wp), ptr(ws), ptr(bo), ptr(wn), n(F), n(K),
+                                      ptr(r[at]) if adds else None, None if relu else ptr(out),
+                                      ptr(out) if relu else None, ptr(scale) if relu else None, stream())
+        assert rc == 0, _native.last_error()
+    want, want_scale, got, got_scale = new(T, F), new(T), new(T, F), new(T)
+    for first in range(0, T, 5000):
+        last = min(first + 5000, T)
+        run(first, last, want[first:last], want_scale[first:last])
+    for out in (got, r) if adds else (got,):
+        run(0, T, out, got_scale)
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+    if relu:
+        assert torch.equal(got_scale, want_scale) and (got_scale > 0).all()
+    else:
+        assert not got.isnan().any()
+
+
+def test_encoder_of_few_tokens_needs_little_more_memory_than_its_modules():
+    """Up to eight layers have their weights in pieces at a time: at most 64 MB of them."""
+    from fast_transformers_amd import attention, masking
+    with torch.device("cuda"):
+        model = attention.build_causal_linear_encoder(12, 8, 64, 64, 1024).eval().requires_grad_(False)
+    x, mask = torch.rand(4, 338, 512, device="cuda"), masking.TriangularCausalMask(338, device="cuda")
+
+    def peak():
+        model(x, attn_mask=mask)     # (workspaces and library handles stay)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        model(x, attn_mask=mask)
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - before
+    native = peak()
+    handle = model.layers[0].linear1.register_forward_hook(lambda *a: None)
+    modules = peak()
+    handle.remove()
+    assert native <= modules + (64 << 20) + 2 * 4 * x.shape[0] * x.shape[1]
