@@ -312,3 +312,25 @@ def test_results_of_copies_go_where_they_belong(shape):
         assert scale_error(out.cpu(), want) <= max(4 * scale_error(plain, want), 2e-6)
         box[:, :, :L, 1:-2] = 7.0
         assert (box == 7.0).all()
+
+
+@pytest.mark.parametrize("offset", [0, 8, 64], ids=["same", "eight_rows_on", "two_chunks_on"])
+@pytest.mark.parametrize("shape", [(30, 20, 70, 64, 35), (2, 5, 1500, 32, 41)], ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+def test_an_odd_result_over_rows_that_are_read_in_place(shape, offset):
+    """Scans on copies of v whose a and b stay where they are, and a result of odd rows that goes over those, from the
+    same row on or from later ones: as if it had gone elsewhere.  (Beside them it goes where it belongs at once.)"""
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = shape
+    plan = _native.plan((N, H, L, E), (N, H, L, M))
+    assert "1 operand copied" in plan and ", 0 results copied back" in plan and "scan_dma_kernel" in plan, plan
+    Q, K, V, _ = oracle.make_inputs(N, H, L, E, M, seed=720 + L)
+    exact, ref = oracle.forward(*(t.double() for t in (Q, K, V))), oracle.forward(Q, K, V)
+    k, v = K.cuda(), V.cuda()
+    room = torch.zeros(N, H, L + 64, E + 64, device="cuda")
+    for first in (E, 0) if M > E else (E, E - M):   # beside the rows of q, over them
+        q, out = room[:, :, :L, :E], room[:, :, offset:offset + L, first:first + M]
+        q.copy_(Q)
+        cp.causal_dot_product_hip(q, k, v, out)
+        assert scale_error(out.cpu(), exact) <= max(4 * scale_error(ref, exact), 2e-6)
+    cp.check_workspaces()
