@@ -145,3 +145,34 @@ def test_without_room_for_an_exchange(cp):
     assert least < full and _last_kernel() == b"scan_mfma_kernel"
     for a, b in zip(got, want):   # (either rounds an fp32 result to bf16)
         assert ((a.float() - b.float()).norm() / b.float().norm()).item() <= 2e-3
+
+
+@pytest.mark.parametrize("shape,kernel", [
+    # long chains of 32 columns: cut, whole beyond the caches, an exchange of five and of ten segments
+    ((1, 128, 2590, 32, 32), OURS[0]), ((1, 160, 5690, 32, 32), OURS[0]), ((8, 19, 4001, 64, 32), OURS[0]),
+    ((3, 16, 5999, 64, 32), OURS[1]), ((2, 12, 11003, 64, 32), OURS[1])], ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s
+    if isinstance(s, tuple) else "")
+def test_long_forward_scans_with_32_columns(cp, shape, kernel):
+    N, H, L, E, M = shape
+    Qb, Kb, Vb, _ = _inputs(N, H, L, E, M, 70 + L)
+    out = torch.full((N, H, L, M), float("nan"), device="cuda")
+    cp.causal_dot_product_hip(Qb.cuda(), Kb.cuda(), Vb.cuda(), out)
+    assert _last_kernel() == kernel
+    exact = oracle.forward(Qb.double(), Kb.double(), Vb.double())
+    ref = oracle.forward(Qb.float(), Kb.float(), Vb.float())
+    assert scale_error(out.cpu(), exact) <= max(2 * scale_error(ref, exact), 1e-6)
+    norm = lambda t: ((t.double() - exact).norm() / exact.norm()).item()
+    assert norm(out.cpu()) <= max(norm(ref), 1e-7)
+
+
+@pytest.mark.parametrize("shape,kernel", [
+    # whole chains of more than 128 chunks, in one round of workgroups and in three; an exchange on few chains
+    ((4, 16, 4127, 32, 32), OURS[0]), ((2, 100, 5153, 32, 32), OURS[0]), ((1, 20, 11003, 32, 32), OURS[1]),
+    ((5, 8, 6001, 32, 32), OURS[1])], ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s if isinstance(s, tuple) else "")
+def test_long_narrow_backward_scans(cp, shape, kernel):
+    N, H, L, E, M = shape
+    Qb, Kb, Vb, G = _inputs(N, H, L, E, M, 80 + L)
+    grads = [torch.full((N, H, L, X), float("nan"), device="cuda", dtype=torch.bfloat16) for X in (E, E, M)]
+    cp.causal_dot_backward_hip(Qb.cuda(), Kb.cuda(), Vb.cuda(), G.cuda(), *grads)
+    assert _last_kernel() == kernel
+    _check_gradients(str(shape), grads, Qb, Kb, Vb, G)

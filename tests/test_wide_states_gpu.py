@@ -163,3 +163,21 @@ def test_states_of_a_short_bf16_prefill(widths, L):
     exact = oracle.forward(Q.double(), K64, V64) + Q.double() @ S.double()
     plain = oracle.forward(Q.float(), K.float(), V.float()) + Q.float() @ S
     assert scale_error(out.cpu(), exact) <= max(4 * scale_error(plain, exact), 2e-6)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 289, 128, 128), (1, 4, 416, 128, 128), (2, 4, 385, 128, 64), (2, 5, 705, 96, 96),
+                                   (5, 4, 449, 128, 64), (2, 5, 736, 128, 128)], ids=lambda s: "n%d_h%d_l%d_e%d_m%d" % s)
+def test_short_chains_of_wide_states_without_a_state(shape):
+    """The same fp32 chains in a plain forward, which walks them whole or cut (those that a state is handed in or out of
+    stay with the kernels that split L): rows no further from float64 than the fp32 oracle's."""
+    from fast_transformers_amd import _native
+    import fast_transformers_amd.causal_product as cp
+    N, H, L, E, M = shape
+    Q, K, V, _ = oracle.make_inputs(N, H, L, E, M, seed=500 + L)
+    out = torch.full((N, H, L, M), float("nan"), device="cuda")
+    cp.causal_dot_product_hip(Q.cuda(), K.cuda(), V.cuda(), out)
+    assert _native.load().ftc_last_kernel() == b"scan_tp_kernel"
+    exact, plain = oracle.forward(*(t.double() for t in (Q, K, V))), oracle.forward(Q, K, V)
+    norm = lambda t: ((t.double() - exact).norm() / exact.norm()).item()
+    assert norm(out.cpu()) <= max(norm(plain), 1.5e-7)
+    assert scale_error(out.cpu(), exact) <= max(4 * scale_error(plain, exact), 2e-6)
