@@ -297,9 +297,9 @@ void tp_plan_compute(int64_t D, int64_t F, int64_t chains, int nscans, int64_t L
     // against 17, L=512: 22 against 17; 128 x 32 forward, 8 chains, L=512: 27 against 20); of that kernel's with
     // more than 32 columns up to 10, from eight workgroups' worth on up to 13 and from twenty on up to 23 (128 x 128
     // forward, us, the kernels that split L / this one: 2 chains, L=270 17.2 / 14.4, L=390 18.8 / 18.3; 4, L=390 20.1 / 18.3, L=500
-    // 20.9 / 22.0; 12, L=500 27.3 / 22.0, L=700 30.3 / 27.9; 128 x 64, 20 chains, L=610 29.7 / 25.8; 96 x 96, 12, L=390 20.2 /
+    // 20.9 / 22.0; 12, L=500 27.3 / 22.0, L=700 30.3 / 27.9; 128 x 96, 10 chains, L=736 28.4 / 30.1, 12 30.7 / 30.0; 128 x 64, 20 chains, L=610 29.7 / 25.8; 96 x 96, 12, L=390 20.2 /
     // 17.2; errors against float64 0.6 to 0.7 of theirs).
-    const int64_t brief_chunks = D <= 64 || (F > 32 && nscans >= 2) ? 23 : F <= 32 ? 8 : units >= 20 ? 23 : units >= 8 ? 13 : 10;
+    const int64_t brief_chunks = D <= 64 || (F > 32 && nscans >= 2) ? 23 : F <= 32 ? 8 : units >= 20 ? (D > 96 && F > 64 && F <= 96 && units < 24 ? 20 : 23) : units >= 8 ? 13 : 10;
     if (narrow && D <= 32 && F <= 32) return;
     // Thousands of chains of one or two chunks with a state of at most 64 x 64 go to those kernels too,
     // where a workgroup's start costs more than its chunks (8192 chains, L=64: 32 x 128 1.17
@@ -420,8 +420,11 @@ bool mixed_splits(int64_t D, int64_t F, int64_t units, int nscans, int64_t chunk
         if (D <= 96 && F > 64 && F <= 96 && chunks > 48 && units >= (bf16_results ? 12 : 20) && units < (bf16_results ? 176 : 128))
             return true;
         // (128 x 128, us, split L / here: 3 chains, L=390 15.0 / 13.0, 6, L=610 20.8 / 17.2, L=760 23.3 / 19.3, but 3, L=500 15.0 / 15.2;
-        // errors against float64 half of theirs)
-        return chunks > 13 && chunks < (units <= 1 ? 128 : units <= 3 ? 96 : units <= 7 ? 48 : units < 12 ? 28 : 0);
+        // errors against float64 half of theirs.  bf16 results, dV of a backward call and the call: 128 x 64, 1 chain, L=416
+        // 25.8 / 26.8, 3, L=380 25.7 / 27.1, but 10, L=410 0.95 of the time; 128 x 96, 7 chains, L=430 0.94, but L=760 46.9 / 49.1)
+        const int64_t brief = bf16_results && units < 8 ? 11 : 13;
+        const int64_t many = bf16_results && F > 64 && F <= 96 && chunks > 16 ? 16 : 12;
+        return chunks > brief && chunks < (units <= 1 ? 128 : units <= 3 ? 96 : units <= 7 ? 48 : units < many ? 28 : 0);
     }
     if (!single) {
         if (D <= 32 && F <= 32) {

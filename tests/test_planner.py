@@ -475,3 +475,13 @@ def test_fused_attention_exchanges_in_segments_of_four_chunks(chains, L):
     assert 192 < chains * fours <= 256
     need = _native.load().ftc_causal_linear_attention_workspace_bytes(1, chains, L, 64, 64, 0)
     assert need >= 2 * 4 * chains * fours * 128 * 16 * 4
+
+
+@pytest.mark.parametrize("chains,L,E,M,backward,dtype", [
+    (1, 416, 128, 64, True, _native.FTC_BF16), (3, 380, 96, 64, True, _native.FTC_BF16),
+    (7, 760, 128, 96, True, _native.FTC_BF16), (6, 860, 128, 96, True, _native.FTC_BF16),
+    (10, 736, 128, 96, False, _native.FTC_F32)])
+def test_short_chains_of_wide_states_that_split(chains, L, E, M, backward, dtype):
+    """1.03 to 1.06 times as long walked whole."""
+    got = lines((1, chains, L, E), (1, chains, L, M), backward=backward, dtype=dtype)
+    assert kernel(got[-1]) == "scan_mfma_kernel", got
