@@ -768,9 +768,10 @@ bool fp32_rows(const ScanDesc &sc, int64_t L, bool *any_fits) {
 // 8 x 16 chains, L=4096, take 500 us on them and 344 here.
 // And a workspace without room for copies means the VALU kernel, here as for any width.
 // (A call of which only some scans run this way has copies for the others.  All of its scans on three bf16
-// pieces (odd_on_three_pieces) would take 0.45 to 0.85 of the time in 90 calls, but the scan that the copies
-// leave to the kernels that split L would be up to 1.3 times as far from float64: 27 x 47, 336 chains,
-// L=413 backward 144 / 84 us, dV 1.3 times.)
+// pieces (odd_on_three_pieces) would be faster in some calls, no rule for which is at hand, and the scan that the copies
+// leave to the kernels that split L then comes out further from float64 in some: backward, us, here / there and the error
+// of dV there, 25 x 33, 99 chains, L=1531 103 / 91, 0.81 times; 27 x 47, 336 chains, L=413 105 / 77, 1.24 times; 50 x 63,
+// 99 chains, L=1531 87 / 109; dQ and dK 0.46 to 0.85 times.)
 bool odd_in_place(const ScanDesc *scans, int n, const bool *padded, int i, int64_t N, int64_t H, int64_t L,
                   size_t workspace_bytes) {
     const ScanDesc &sc = scans[i];

@@ -14,10 +14,10 @@
 // library rounds after every few: against float64 a product of 40960 x 512 by 512 x 512 is off by
 // 1.9e-7 (2-norm) where the library's is by 2.9e-7, of 1024 columns by 2.6e-7 and 4.1e-7.
 //
-// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 74, 512 -> 1536 475 / 171, 512 -> 1024
-// with relu 310 + 51 / 123, 1024 -> 512 with the residual 305 + 37 / 132; 5000 tokens, 256 -> 512 20 / 11;
-// 300 tokens, 128 -> 260 31 / 4.2.  (At the largest sizes the card's power and the rows' way out bound it: 512 -> 1536
-// on zeros 189 -> 165, without its stores 148, both before LATER and kStreamed below.)
+// Measured, 40960 tokens (us, library / here): 512 -> 512 191 / 67, 512 -> 1536 475 / 173, 512 -> 1024
+// with relu 310 + 51 / 123, 1024 -> 512 with the residual 305 + 37 / 122, with a norm made again 128; 5000 tokens,
+// 256 -> 512 20 / 9; 300 tokens, 128 -> 260 31 / 4.2.  (At the largest sizes the card's power bounds it: 512 -> 1536 on
+// zeros 134, 1024 -> 512 100.)
 //
 // Rows in pieces take the bytes of fp32 rows: block of 32 columns after block, 64 bytes of hi and 64
 // of lo each, one cache line per row and k-step.  Whoever writes rows that only a product reads
