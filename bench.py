@@ -44,10 +44,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix, published
 # carries it only while the sources are unchanged, otherwise null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
     # workload: (bytes, kernel source hash at the time of the measurement)
-    "cfg2": (139917319, "d18cc6259653fd1e"),
-    "cfg3": (2616000991, "d18cc6259653fd1e"),
-    "cfg5": (4156315083, "d18cc6259653fd1e"),
-    "wide": (1877174347, "d18cc6259653fd1e"),
+    "cfg2": (139714797, "da8bd2d8a83a24f9"),
+    "cfg3": (2593702343, "da8bd2d8a83a24f9"),
+    "cfg5": (4153230669, "da8bd2d8a83a24f9"),
+    "wide": (1876925346, "da8bd2d8a83a24f9"),
 }
 
 WORKLOADS = {
